@@ -4,152 +4,99 @@
 // weight decay; SAM perturb / sharpness restore helpers).
 //
 // Every entry point covers all tensors with one launch per stage: a tile of
-// 4096 elements is mapped to (tensor, offset) by binary search in a P+1 entry
-// prefix table, so small parameter sets cost a handful of launches instead of
-// several per tensor (the reference launches per tensor and syncs the host for
-// the gradient norm).
-#include <cmath>
-#include <vector>
-
-#include "sg_common.hpp"
-
+// elements is mapped to (tensor, offset) by a search in a prefix table, so
+// small parameter sets cost one or two launches instead of several per tensor
+// (the reference launches per tensor and syncs the host for the gradient norm).
 #include "sg_elemwise.hpp"
 
 namespace sgew {
 namespace {
 
-// ---- Grokfast ------------------------------------------------------------------
-struct GfRec {
-    void* param;
-    void* grad;
-    float* ema;
-    float* ea;
-    float* easq;
-    int64_t numel;
-    int32_t dtype;
-    float step_size, bc2;
-};
-
-template <bool ADAM>
-__global__ __launch_bounds__(THREADS) void k_grokfast(Batch<GfRec> B, float alpha, float lamb, float beta1, float om_beta1,
-                                                       float beta2, float om_beta2, float eps, float decay) {
+// ---- Grokfast (aux: ema) -------------------------------------------------------
+// HBM bound (40 B an element in fp32): four elements per lane and access.
+template <bool ADAM, class BT>
+__global__ __launch_bounds__(THREADS) void k_grokfast(BT B, float alpha, float lamb, float beta1, float om_beta1, float beta2,
+                                                       float om_beta2, float eps, float decay) {
     int start, cnt;
-    const GfRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    const int dtype = R.dtype;
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
     const float om_alpha = 1.0f - alpha;
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const int i = start + k;
-        const float g = sg::load_elem(R.grad, dtype, i);
-        const float e = sg_fma(alpha, R.ema[i], om_alpha * g);
-        R.ema[i] = e;
-        const float amp = sg_fma(lamb, e, g);
-        sg::store_elem(R.grad, dtype, i, amp);
-        if (ADAM) {
-            // AdamW consumes the gradient as stored, i.e. rounded to the tensor's element type
-            const float ga = (dtype == SG_F32) ? amp : sg::load_elem(R.grad, dtype, i);
-            const float ea = sg_fma(beta1, R.ea[i], om_beta1 * ga);
-            const float easq = sg_fma(beta2, R.easq[i], (om_beta2 * ga) * ga);
-            R.ea[i] = ea;
-            R.easq[i] = easq;
-            const float denom = __builtin_sqrtf(easq / R.bc2) + eps;
-            const float p = sg::load_elem(R.param, dtype, i);
-            sg::store_elem(R.param, dtype, i, sg_fma(p, decay, -((R.step_size * ea) / denom)));
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float g[V], e[V];
+        ldt<V>(R.grad, R.dtype, i, g);
+        ldf<V>(R.aux, i, e);
+#pragma unroll
+        for (int c = 0; c < V; c++) {
+            e[c] = sg_fma(alpha, e[c], om_alpha * g[c]);
+            g[c] = rounded(R.dtype, sg_fma(lamb, e[c], g[c]));       // AdamW consumes the gradient as stored
         }
-    }
+        stf<V>(R.aux, i, e);
+        stt<V>(R.grad, R.dtype, i, g);
+        if (ADAM) adam_update<V>(R, i, g, beta1, om_beta1, beta2, om_beta2, eps, decay);
+    });
 }
 
-// ---- SuperGrok v1.5 --------------------------------------------------------------
-struct S15Rec {
-    void* param;
-    void* grad;
-    const void* sharp;
-    float* ea;
-    float* easq;
-    float* mu;
-    int64_t numel;
-    int32_t dtype;
-    float alpha, beta1, bc2, step_size;
-};
-
-template <int GELU>
-__global__ __launch_bounds__(THREADS) void k_sg15(Batch<S15Rec> B, const float* __restrict__ W1, const float* __restrict__ b1,
+// ---- SuperGrok v1.5 (aux: mu, aux2: sharpness) -----------------------------------
+template <int GELU, class BT>
+__global__ __launch_bounds__(THREADS) void k_sg15(BT B, const float* __restrict__ W1, const float* __restrict__ b1,
                                                    const float* __restrict__ W2, const float* __restrict__ b2, int H,
-                                                   float rescale, float lamb_eff, float beta2, float eps, float decay) {
+                                                   float clip_norm, float rescale, float lamb_eff, float beta2, float eps, float decay) {
     __shared__ float sW1[2 * MAX_HIDDEN], sb1[MAX_HIDDEN], sW2[MAX_HIDDEN];
-    for (int k = threadIdx.x; k < 2 * H; k += THREADS) sW1[k] = W1[k];
-    for (int k = threadIdx.x; k < H; k += THREADS) { sb1[k] = b1[k]; sW2[k] = W2[k]; }
-    __syncthreads();
-    const float bias2 = b2[0];
-    const float coef = B.red->coef;
-    const bool clip_on = B.red->clip_on != 0;
+    load_net(W1, b1, W2, H, sW1, sb1, sW2);
+    const Clip clip = global_norm(B, clip_norm);        // (its barriers cover the weights)
+    const MetaNet<GELU> net = {sW1, sb1, sW2, b2[0], H, (const __attribute__((address_space(4))) MetaPoly*)B.table};
 
     int start, cnt;
-    const S15Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    const int dtype = R.dtype;
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
     const float alpha = R.alpha, beta1 = R.beta1;
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const int i = start + k;
-        float g = sg::load_elem(R.grad, dtype, i);
-        if (clip_on) {                       // gradients are rescaled in place, as the reference does
-            sg::store_elem(R.grad, dtype, i, g * coef);
-            g = (dtype == SG_F32) ? g * coef : sg::load_elem(R.grad, dtype, i);
-        }
-        const float s = sg::load_elem(R.sharp, dtype, i);
-        const float mu = sg_fma(alpha, R.mu[i], (1.0f - alpha) * g);
-        R.mu[i] = mu;
-        float acc = 0.0f;
-        for (int h = 0; h < H; h++) {
-            const float z = sg_fma(sW1[2 * h + 1], s, sW1[2 * h] * g) + sb1[h];
-            const float a = (GELU == 0) ? sg_gelu_erf(z) : sg_gelu_sigmoid(z);
-            acc = sg_fma(sW2[h], a, acc);
-        }
-        const float smart = sg_fma(rescale, acc + bias2, g);
-        const float fg = sg_fma(lamb_eff, mu, smart);
-        const float ea = sg_fma(beta1, R.ea[i], (1.0f - beta1) * fg);
-        const float easq = sg_fma(beta2, R.easq[i], ((1.0f - beta2) * fg) * fg);
-        R.ea[i] = ea;
-        R.easq[i] = easq;
-        const float denom = __builtin_sqrtf(easq / R.bc2) + eps;
-        const float p = sg::load_elem(R.param, dtype, i);
-        sg::store_elem(R.param, dtype, i, sg_fma(p, decay, -((R.step_size * ea) / denom)));
-    }
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float g[V], s[V], mu[V];
+        clipped_grad<V>(R, i, clip, g);
+        ldt<V>(R.aux2, R.dtype, i, s);
+        ldf<V>(R.aux, i, mu);
+#pragma unroll
+        for (int c = 0; c < V; c++) mu[c] = sg_fma(alpha, mu[c], (1.0f - alpha) * g[c]);
+        stf<V>(R.aux, i, mu);
+#pragma unroll
+        for (int c = 0; c < V; c++) g[c] = sg_fma(lamb_eff, mu[c], sg_fma(rescale, net(g[c], s[c]), g[c]));
+        adam_update<V>(R, i, g, beta1, 1.0f - beta1, beta2, 1.0f - beta2, eps, decay);
+    });
 }
 
-struct SamRec {
-    void* param;
-    const void* grad;
-    int64_t numel;
-    int32_t dtype;
-};
-__global__ __launch_bounds__(THREADS) void k_sam_perturb(Batch<SamRec> B, float rho) {
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_sam_perturb(BT B, float rho) {
+    const Clip n = global_norm(B, 0.0f);
     int start, cnt;
-    const SamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    const float r = rho / (B.red->norm + 1e-12f);
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const int i = start + k;
-        const float p = sg::load_elem(R.param, R.dtype, i), g = sg::load_elem(R.grad, R.dtype, i);
-        sg::store_elem(R.param, R.dtype, i, sg_fma(r, g, p));
-    }
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+    const float r = rho / (n.norm + 1e-12f);
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float p[V], g[V];
+        ldt<V>(R.param, R.dtype, i, p);
+        ldt<V>(R.grad, R.dtype, i, g);
+#pragma unroll
+        for (int c = 0; c < V; c++) p[c] = sg_fma(r, g[c], p[c]);
+        stt<V>(R.param, R.dtype, i, p);
+    });
 }
 
-struct RestoreRec {
-    void* param;
-    void* sharp;
-    const void* backup;
-    const void* sam_grad;
-    const void* grad;      // the normal gradient
-    int64_t numel;
-    int32_t dtype;
-};
-__global__ __launch_bounds__(THREADS) void k_restore(Batch<RestoreRec> B) {
+// grad: the normal gradient, aux2: the SAM gradient, ea: sharpness, easq: backup (both in the tensor's type)
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_restore(BT B) {
     int start, cnt;
-    const RestoreRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const int i = start + k;
-        const float sgv = sg::load_elem(R.sam_grad, R.dtype, i), ng = sg::load_elem(R.grad, R.dtype, i);
-        sg::store_elem(R.sharp, R.dtype, i, sg_abs(sgv - ng));
-        sg::store_elem(R.param, R.dtype, i, sg::load_elem(R.backup, R.dtype, i));
-    }
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float a[V], b[V], p[V];
+        ldt<V>(R.aux2, R.dtype, i, a);
+        ldt<V>(R.grad, R.dtype, i, b);
+        ldt<V>(R.easq, R.dtype, i, p);
+#pragma unroll
+        for (int c = 0; c < V; c++) a[c] = sg_abs(a[c] - b[c]);
+        stt<V>(R.ea, R.dtype, i, a);
+        stt<V>(R.param, R.dtype, i, p);
+    });
 }
 
 }  // namespace
@@ -169,21 +116,24 @@ int sg_grokfast_ema(int num_tensors, const SgGrokfastTensor* tensors, float alph
     using namespace sgew;
     if (num_tensors <= 0) return 0;
     if (!tensors) return sg::fail("NULL argument");
-    std::vector<GfRec> recs;
+    std::vector<Rec> recs;
+    recs.reserve(num_tensors);
     for (int i = 0; i < num_tensors; i++) {
         const SgGrokfastTensor& t = tensors[i];
         if (t.numel == 0) continue;
         if (!t.grad || !t.ema) return sg::fail("tensor %d: NULL pointer", i);
-        if (check_dtype(i, t.dtype)) return 1;
-        recs.push_back({nullptr, t.grad, t.ema, nullptr, nullptr, t.numel, t.dtype, 0.0f, 1.0f});
+        if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
+        recs.push_back({nullptr, t.grad, nullptr, nullptr, t.ema, nullptr, (int32_t)t.numel, (int16_t)t.dtype,
+                        vec4_ok(t.dtype, bits(t.grad), bits(t.ema)), 0.0f, 1.0f, 0.0f, 0.0f});
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<GfRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    hipLaunchKernelGGL(k_grokfast<false>, dim3(B.tiles), dim3(THREADS), 0, st, B, alpha, lamb, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
-    SG_LAUNCH_CHECK("k_grokfast<ema>");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        hipLaunchKernelGGL((k_grokfast<false, BT>), dim3(B.tiles), dim3(THREADS), 0, st, B, alpha, lamb, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
+        SG_LAUNCH_CHECK("k_grokfast<ema>");
+        return 0;
+    });
 }
 
 int sg_grokfast_adamw_step(int num_tensors, const SgGrokfastAdamTensor* tensors, float alpha, float lamb, double lr,
@@ -192,25 +142,35 @@ int sg_grokfast_adamw_step(int num_tensors, const SgGrokfastAdamTensor* tensors,
     using namespace sgew;
     if (num_tensors <= 0) return 0;
     if (!tensors) return sg::fail("NULL argument");
-    std::vector<GfRec> recs;
+    std::vector<Rec> recs;
+    recs.reserve(num_tensors);
+    int last_step = 0;
+    double bc1 = 1.0, bc2 = 1.0;
     for (int i = 0; i < num_tensors; i++) {
         const SgGrokfastAdamTensor& t = tensors[i];
         if (t.numel == 0) continue;
         if (!t.param || !t.grad || !t.ema || !t.exp_avg || !t.exp_avg_sq) return sg::fail("tensor %d: NULL pointer", i);
-        if (check_dtype(i, t.dtype)) return 1;
+        if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
         if (t.step < 1) return sg::fail("tensor %d: step must be >= 1", i);
-        // bias corrections in double, as the Python helper computes them
-        const double bc1 = 1.0 - std::pow(beta1, (double)t.step), bc2 = 1.0 - std::pow(beta2, (double)t.step);
-        recs.push_back({t.param, t.grad, t.ema, t.exp_avg, t.exp_avg_sq, t.numel, t.dtype, (float)(lr / bc1), (float)bc2});
+        // bias corrections in double, as the Python helper computes them (tensors of a group are nearly always at one step)
+        if (t.step != last_step) {
+            bc1 = 1.0 - std::pow(beta1, (double)t.step);
+            bc2 = 1.0 - std::pow(beta2, (double)t.step);
+            last_step = t.step;
+        }
+        recs.push_back({t.param, t.grad, t.exp_avg, t.exp_avg_sq, t.ema, nullptr, (int32_t)t.numel, (int16_t)t.dtype,
+                        vec4_ok(t.dtype, bits(t.param) | bits(t.grad), bits(t.ema) | bits(t.exp_avg) | bits(t.exp_avg_sq)),
+                        (float)(lr / bc1), (float)bc2, 0.0f, 0.0f});
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<GfRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    hipLaunchKernelGGL(k_grokfast<true>, dim3(B.tiles), dim3(THREADS), 0, st, B, alpha, lamb, (float)beta1,
-                       (float)(1.0 - beta1), (float)beta2, (float)(1.0 - beta2), (float)eps, (float)(1.0 - lr * weight_decay));
-    SG_LAUNCH_CHECK("k_grokfast<adamw>");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        hipLaunchKernelGGL((k_grokfast<true, BT>), dim3(B.tiles), dim3(THREADS), 0, st, B, alpha, lamb, (float)beta1,
+                           (float)(1.0 - beta1), (float)beta2, (float)(1.0 - beta2), (float)eps, (float)(1.0 - lr * weight_decay));
+        SG_LAUNCH_CHECK("k_grokfast<adamw>");
+        return 0;
+    });
 }
 
 int sg15_fused_step(int num_tensors, const Sg15Tensor* tensors, const Sg15Net* net, float lamb_eff, float beta2, float lr,
@@ -220,29 +180,36 @@ int sg15_fused_step(int num_tensors, const Sg15Tensor* tensors, const Sg15Net* n
     if (!tensors || !net || !net->W1 || !net->b1 || !net->W2 || !net->b2) return sg::fail("NULL argument");
     if (net->hidden < 1 || net->hidden > MAX_HIDDEN) return sg::fail("hidden_dim %d outside [1,%d]", net->hidden, MAX_HIDDEN);
     if (net->gelu_mode != 0 && net->gelu_mode != 1) return sg::fail("bad gelu_mode %d", net->gelu_mode);
-    std::vector<S15Rec> recs;
+    std::vector<Rec> recs;
+    recs.reserve(num_tensors);
     for (int i = 0; i < num_tensors; i++) {
         const Sg15Tensor& t = tensors[i];
         if (t.numel == 0) continue;
         if (!t.param || !t.grad || !t.sharpness || !t.exp_avg || !t.exp_avg_sq || !t.mu) return sg::fail("tensor %d: NULL pointer", i);
-        if (check_dtype(i, t.dtype)) return 1;
-        recs.push_back({t.param, t.grad, t.sharpness, t.exp_avg, t.exp_avg_sq, t.mu, t.numel, t.dtype, t.alpha, t.beta1, t.bc2,
-                        lr / t.bc1});
+        if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
+        recs.push_back({t.param, t.grad, t.exp_avg, t.exp_avg_sq, t.mu, t.sharpness, (int32_t)t.numel, (int16_t)t.dtype,
+                        vec4_ok(t.dtype, bits(t.param) | bits(t.grad) | bits(t.sharpness), bits(t.exp_avg) | bits(t.exp_avg_sq) | bits(t.mu)),
+                        lr / t.bc1, t.bc2, t.alpha, t.beta1});
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<S15Rec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    if (reduce_sumsq(recs, B, grad_clip_norm, st)) return 1;
-    const float decay = 1.0f - lr * wd_eff;
-    if (net->gelu_mode == 0)
-        hipLaunchKernelGGL(k_sg15<0>, dim3(B.tiles), dim3(THREADS), 0, st, B, net->W1, net->b1, net->W2, net->b2, net->hidden,
-                           net->rescale, lamb_eff, beta2, eps, decay);
-    else
-        hipLaunchKernelGGL(k_sg15<1>, dim3(B.tiles), dim3(THREADS), 0, st, B, net->W1, net->b1, net->W2, net->b2, net->hidden,
-                           net->rescale, lamb_eff, beta2, eps, decay);
-    SG_LAUNCH_CHECK("k_sg15");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        const float decay = 1.0f - lr * wd_eff;
+        const auto run = [&](auto gelu) {
+            hipLaunchKernelGGL((k_sg15<decltype(gelu)::value, BT>), dim3(B.tiles), dim3(THREADS), 0, st, B, net->W1, net->b1, net->W2,
+                               net->b2, net->hidden, grad_clip_norm, net->rescale, lamb_eff, beta2, eps, decay);
+        };
+        if (net->gelu_mode == 0) {
+            launch_sumsq(B, st, PrepMetaPoly{net->W1, net->b1, net->W2, net->b2, net->hidden});
+            run(std::integral_constant<int, 0>{});
+        } else {
+            launch_sumsq(B, st);
+            run(std::integral_constant<int, 1>{});
+        }
+        SG_LAUNCH_CHECK("k_sg15");
+        return 0;
+    });
 }
 
 int sg15_sam_perturb(int num_tensors, const Sg15SamTensor* tensors, float rho, void* workspace, size_t workspace_bytes,
@@ -250,22 +217,25 @@ int sg15_sam_perturb(int num_tensors, const Sg15SamTensor* tensors, float rho, v
     using namespace sgew;
     if (num_tensors <= 0) return 0;
     if (!tensors) return sg::fail("NULL argument");
-    std::vector<SamRec> recs;
+    std::vector<Rec> recs;
+    recs.reserve(num_tensors);
     for (int i = 0; i < num_tensors; i++) {
         const Sg15SamTensor& t = tensors[i];
         if (t.numel == 0) continue;
         if (!t.param || !t.grad) return sg::fail("tensor %d: NULL pointer", i);
-        if (check_dtype(i, t.dtype)) return 1;
-        recs.push_back({t.param, t.grad, t.numel, t.dtype});
+        if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
+        recs.push_back({t.param, const_cast<void*>(t.grad), nullptr, nullptr, nullptr, nullptr, (int32_t)t.numel, (int16_t)t.dtype,
+                        vec4_ok(t.dtype, bits(t.param) | bits(t.grad), 0), 0.0f, 1.0f, 0.0f, 0.0f});
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<SamRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    if (reduce_sumsq(recs, B, 0.0f, st)) return 1;
-    hipLaunchKernelGGL(k_sam_perturb, dim3(B.tiles), dim3(THREADS), 0, st, B, rho);
-    SG_LAUNCH_CHECK("k_sam_perturb");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        launch_sumsq(B, st);
+        hipLaunchKernelGGL(k_sam_perturb<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B, rho);
+        SG_LAUNCH_CHECK("k_sam_perturb");
+        return 0;
+    });
 }
 
 int sg15_sharpness_restore(int num_tensors, const Sg15RestoreTensor* tensors, void* workspace, size_t workspace_bytes,
@@ -273,21 +243,26 @@ int sg15_sharpness_restore(int num_tensors, const Sg15RestoreTensor* tensors, vo
     using namespace sgew;
     if (num_tensors <= 0) return 0;
     if (!tensors) return sg::fail("NULL argument");
-    std::vector<RestoreRec> recs;
+    std::vector<Rec> recs;
+    recs.reserve(num_tensors);
     for (int i = 0; i < num_tensors; i++) {
         const Sg15RestoreTensor& t = tensors[i];
         if (t.numel == 0) continue;
         if (!t.param || !t.sharpness || !t.backup || !t.sam_grad || !t.normal_grad) return sg::fail("tensor %d: NULL pointer", i);
-        if (check_dtype(i, t.dtype)) return 1;
-        recs.push_back({t.param, t.sharpness, t.backup, t.sam_grad, t.normal_grad, t.numel, t.dtype});
+        if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
+        recs.push_back({t.param, const_cast<void*>(t.normal_grad), static_cast<float*>(t.sharpness),
+                        static_cast<float*>(const_cast<void*>(t.backup)), nullptr, t.sam_grad, (int32_t)t.numel, (int16_t)t.dtype,
+                        vec4_ok(t.dtype, bits(t.param) | bits(t.sharpness) | bits(t.backup) | bits(t.sam_grad) | bits(t.normal_grad), 0),
+                        0.0f, 1.0f, 0.0f, 0.0f});
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<RestoreRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    hipLaunchKernelGGL(k_restore, dim3(B.tiles), dim3(THREADS), 0, st, B);
-    SG_LAUNCH_CHECK("k_restore");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        hipLaunchKernelGGL(k_restore<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
+        SG_LAUNCH_CHECK("k_restore");
+        return 0;
+    });
 }
 
 }  // extern "C"

@@ -5,446 +5,494 @@
 // csrc/ops.cpp:209-656 with their per-optimizer kernels.
 //
 // Same batching as the other elementwise steps: one launch per stage covers
-// every tensor (tile of 4096 elements -> tensor by binary search in a prefix
-// table).  Everything the reference reads back to the host between stages -
+// every tensor.  Everything the reference reads back to the host between stages -
 // the global gradient norm, Prodigy's numerator/denominator, v1.1's cosine
 // gate per tensor, LookSAM's per-tensor norms - is reduced on the device
-// (per-tile partial sums in double, one block per result) and consumed from
-// device memory by the next kernel, so a step enqueues without a host sync.
+// (partial sums in double, added up in a fixed order by the consumer) so a
+// step enqueues without a host sync.
+#include <mutex>
+
 #include "sg_elemwise.hpp"
 
 namespace sgew {
 namespace {
 
-struct FamRec {
-    void* param;
-    void* grad;
-    float* ea;
-    float* easq;
-    float* aux;
-    const void* aux2;
-    float* smart;          // v1.1: this tensor's slice of the smart-gradient scratch
-    int64_t numel;
-    int32_t dtype;
-    float bc1, bc2, alpha, beta1;
-    int32_t vec4;          // fp32 tensor and every pointer 16-byte aligned: four elements per lane and access
+// ---- GrokAdamW (aux: ema, or NULL for plain AdamW) -------------------------------
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_grokadamw(BT B, float clip_norm, float alpha, float lamb, float beta1, float beta2,
+                                                        float eps, float decay) {
+    Clip clip = {0.0f, 1.0f, false};
+    if (clip_norm > 0.0f) clip = global_norm(B, clip_norm);
+    int start, cnt;
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float g[V];
+        clipped_grad<V>(R, i, clip, g);
+        if (R.aux) {
+            float e[V];
+            ldf<V>(R.aux, i, e);
+#pragma unroll
+            for (int c = 0; c < V; c++) {
+                e[c] = sg_fma(alpha, e[c], (1.0f - alpha) * g[c]);
+                g[c] = sg_fma(lamb, e[c], g[c]);
+            }
+            stf<V>(R.aux, i, e);
+        }
+        adam_update<V>(R, i, g, beta1, 1.0f - beta1, beta2, 1.0f - beta2, eps, decay);
+    });
+}
+
+// ---- NeuralGrok ------------------------------------------------------------------
+// The amplifier  sum_h W2 relu(W1 g + b1)  is a straight line  A g + B  between two neighbouring thresholds -b1/W1 of
+// its units.  One block tabulates the lines of all H + 1 intervals per call (in double, while the other blocks of its
+// launch reduce the gradient norm); an element finds its interval by a search of the thresholds in LDS and evaluates
+// one fma.  Evaluating the units one by one is 3 vector instructions and LDS operands for each of 128 units: 332 us
+// for 25 M elements against 140 us for the step's memory traffic.
+constexpr int AMP_SLOTS = 511;         // thresholds, padded with +inf to 2^k - 1 (at most MAX_HIDDEN = 256 real ones)
+struct AmpTable {
+    float t[AMP_SLOTS + 1];
+    float A[MAX_HIDDEN + 1], B[MAX_HIDDEN + 1];
+    float lo, hi;                      // the interval of small gradients: lo < g <= hi
+    int at, direct;                    // its index; direct: non-finite weights, no table
+};
+static_assert(sizeof(AmpTable) <= TABLE_BYTES, "table fits its place in the workspace");
+inline int amp_slots(int H) {          // smallest 2^k - 1 >= H
+    int s = 1;
+    while (s < H) s = 2 * s + 1;
+    return s;
+}
+struct PrepAmp {
+    static constexpr bool any = true;
+    const float *W1, *b1, *W2;
+    int H, slots;
+    template <class BT>
+    __device__ void operator()(const BT& B) const {
+        __shared__ float st[MAX_HIDDEN], sw1[MAX_HIDDEN], sb1[MAX_HIDDEN], sw2[MAX_HIDDEN], sorted[MAX_HIDDEN];
+        __shared__ int srank[MAX_HIDDEN];
+        AmpTable* out = static_cast<AmpTable*>(B.table);
+        const int h = threadIdx.x;
+        bool bad = false;
+        if (h < H) {
+            const float w = W1[h], b = b1[h], u = W2[h];
+            sw1[h] = w;
+            sb1[h] = b;
+            sw2[h] = u;
+            st[h] = w == 0.0f ? __builtin_inff() : -b / w;       // a unit that does not look at g has no threshold
+            bad = !sg_isfinite(w) || !sg_isfinite(b) || !sg_isfinite(u);
+        }
+        bad = __syncthreads_or(bad ? 1 : 0) != 0;
+        if (h < H) {
+            int r = 0;
+            const float t = st[h];
+            for (int k = 0; k < H; k++) r += (st[k] < t || (st[k] == t && k < h)) ? 1 : 0;
+            srank[h] = r & (MAX_HIDDEN - 1);                     // (in range whatever the weights)
+            sorted[r & (MAX_HIDDEN - 1)] = t;
+        }
+        __syncthreads();
+        for (int k = h; k < slots; k += THREADS) out->t[k] = k < H ? sorted[k] : __builtin_inff();
+        for (int k = h; k <= H; k += THREADS) {                  // interval k: thresholds 0 .. k-1 lie below g
+            double a = 0.0, c = 0.0;
+            for (int j = 0; j < H; j++) {
+                const float w = sw1[j];
+                const bool active = w > 0.0f ? srank[j] < k : (w < 0.0f ? srank[j] >= k : sb1[j] > 0.0f);
+                const double u = active ? (double)sw2[j] : 0.0;
+                a += u * (double)w;
+                c += u * (double)sb1[j];
+            }
+            out->A[k] = (float)a;
+            out->B[k] = (float)c;
+        }
+        if (h == 0) {
+            int at = 0;
+            for (int k = 0; k < H; k++) at += sorted[k] < 0.0f ? 1 : 0;
+            out->at = at;
+            out->lo = at > 0 ? sorted[at - 1] : -__builtin_inff();
+            out->hi = at < H ? sorted[at] : __builtin_inff();
+            out->direct = bad ? 1 : 0;
+        }
+    }
 };
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ f32x4 ld4(const void* p, int i) { return *(const SG_GLOBAL f32x4*)(static_cast<const float*>(p) + i); }
-__device__ __forceinline__ void st4(void* p, int i, f32x4 v) { *(SG_GLOBAL f32x4*)(static_cast<float*>(p) + i) = v; }
-
-// Runs body(i) for every element of the tile; when the tensor allows 16-byte accesses, body4(i) handles four
-// consecutive elements per lane and body(i) only the ragged end.
-template <class B1, class B4>
-__device__ __forceinline__ void for_tile(const FamRec& R, int start, int cnt, B1 body, B4 body4) {
-    int done = 0;
-    if (R.vec4) {
-        done = cnt & ~3;
-        for (int k = threadIdx.x * 4; k < done; k += THREADS * 4) body4(start + k);
-    }
-    for (int k = done + threadIdx.x; k < cnt; k += THREADS) body(start + k);
-}
-
-// clipped gradient, written back in place when clipping is active (clip_grad_norms_device_side, csrc/ops.cpp:23-55)
-__device__ __forceinline__ float clipped_grad(const FamRec& R, int i, bool clip_on, float coef) {
-    float g = sg::load_elem(R.grad, R.dtype, i);
-    if (clip_on) {
-        sg::store_elem(R.grad, R.dtype, i, g * coef);
-        g = (R.dtype == SG_F32) ? g * coef : sg::load_elem(R.grad, R.dtype, i);
-    }
-    return g;
-}
-__device__ __forceinline__ f32x4 clipped_grad4(const FamRec& R, int i, bool clip_on, float coef) {
-    f32x4 g = ld4(R.grad, i);
-    if (clip_on) {
-        g = g * coef;
-        st4(R.grad, i, g);
-    }
-    return g;
-}
-
-// decoupled decay, then the Adam step: p*(1 - lr*wd) - (lr/bc1) * ea / (sqrt(easq/bc2) + eps)
-__device__ __forceinline__ float adam_core(float fg, float p, float& ea, float& easq, float beta1, float beta2, float bc2,
-                                           float eps_eff, float decay, float step_size) {
-    ea = sg_fma(beta1, ea, (1.0f - beta1) * fg);
-    easq = sg_fma(beta2, easq, ((1.0f - beta2) * fg) * fg);
-    const float denom = __builtin_sqrtf(easq / bc2) + eps_eff;
-    return sg_fma(p, decay, -((step_size * ea) / denom));
-}
-__device__ __forceinline__ void adam_update(const FamRec& R, int i, float fg, float beta1, float beta2, float eps_eff, float decay,
-                                            float step_size) {
-    float ea = R.ea[i], easq = R.easq[i];
-    const float p = adam_core(fg, sg::load_elem(R.param, R.dtype, i), ea, easq, beta1, beta2, R.bc2, eps_eff, decay, step_size);
-    R.ea[i] = ea;
-    R.easq[i] = easq;
-    sg::store_elem(R.param, R.dtype, i, p);
-}
-__device__ __forceinline__ void adam_update4(const FamRec& R, int i, f32x4 fg, float beta1, float beta2, float eps_eff, float decay,
-                                             float step_size) {
-    f32x4 ea = ld4(R.ea, i), easq = ld4(R.easq, i), p = ld4(R.param, i);
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-        float a = ea[c], q = easq[c];
-        p[c] = adam_core(fg[c], p[c], a, q, beta1, beta2, R.bc2, eps_eff, decay, step_size);
-        ea[c] = a;
-        easq[c] = q;
-    }
-    st4(R.ea, i, ea);
-    st4(R.easq, i, easq);
-    st4(R.param, i, p);
-}
-
-__global__ __launch_bounds__(THREADS) void k_grokadamw(Batch<FamRec> B, float alpha, float lamb, float beta1, float beta2, float lr,
-                                                        float eps, float decay) {
-    int start, cnt;
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    const float coef = B.red->coef;
-    const bool clip_on = B.red->clip_on != 0;
-    const float step_size = lr / R.bc1;
-    for_tile(R, start, cnt,
-        [&](int i) {
-            const float g = clipped_grad(R, i, clip_on, coef);
-            float fg = g;
-            if (R.aux) {        // no EMA buffer: plain AdamW
-                const float e = sg_fma(alpha, R.aux[i], (1.0f - alpha) * g);
-                R.aux[i] = e;
-                fg = sg_fma(lamb, e, g);
-            }
-            adam_update(R, i, fg, beta1, beta2, eps, decay, step_size);
-        },
-        [&](int i) {
-            const f32x4 g = clipped_grad4(R, i, clip_on, coef);
-            f32x4 fg = g;
-            if (R.aux) {
-                f32x4 e = ld4(R.aux, i);
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    e[c] = sg_fma(alpha, e[c], (1.0f - alpha) * g[c]);
-                    fg[c] = sg_fma(lamb, e[c], g[c]);
-                }
-                st4(R.aux, i, e);
-            }
-            adam_update4(R, i, fg, beta1, beta2, eps, decay, step_size);
-        });
-}
-
-__global__ __launch_bounds__(THREADS) void k_neuralgrok(Batch<FamRec> B, const float* __restrict__ W1, const float* __restrict__ b1,
-                                                         const float* __restrict__ W2, const float* __restrict__ b2, int H,
-                                                         float alpha_amp, float beta_amp, float beta1, float beta2, float lr,
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_neuralgrok(BT B, const float* __restrict__ W1, const float* __restrict__ b1,
+                                                         const float* __restrict__ W2, const float* __restrict__ b2, int H, int slots,
+                                                         float clip_norm, float alpha_amp, float beta_amp, float beta1, float beta2,
                                                          float eps, float decay) {
-    __shared__ float sW1[MAX_HIDDEN], sb1[MAX_HIDDEN], sW2[MAX_HIDDEN];
-    for (int k = threadIdx.x; k < H; k += THREADS) { sW1[k] = W1[k]; sb1[k] = b1[k]; sW2[k] = W2[k]; }
-    __syncthreads();
+    __shared__ float st[AMP_SLOTS + 1], sA[MAX_HIDDEN + 1], sB[MAX_HIDDEN + 1];
+    const AmpTable* T = static_cast<const AmpTable*>(B.table);
+    for (int k = threadIdx.x; k < slots; k += THREADS) st[k] = T->t[k];
+    for (int k = threadIdx.x; k <= H; k += THREADS) { sA[k] = T->A[k]; sB[k] = T->B[k]; }
+    const Clip clip = global_norm(B, clip_norm);                 // (its barriers cover the table)
+    const float lo = T->lo, hi = T->hi, A0 = T->A[T->at], B0 = T->B[T->at];
+    const bool direct = T->direct != 0;
     const float bias2 = b2[0];
     int start, cnt;
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    const float coef = B.red->coef;
-    const bool clip_on = B.red->clip_on != 0;
-    const float step_size = lr / R.bc1;
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const int i = start + k;
-        const float g = clipped_grad(R, i, clip_on, coef);
-        float acc = 0.0f;
-        for (int h = 0; h < H; h++) acc = sg_fma(sW2[h], sg_max(sg_fma(sW1[h], g, sb1[h]), 0.0f), acc);
-        const float ag = g * sg_fma(alpha_amp, acc + bias2, beta_amp);
-        adam_update(R, i, ag, beta1, beta2, eps, decay, step_size);
-    }
-}
-
-__device__ __forceinline__ void lion_core(float g, float& m, float& p, float lr, float beta1, float beta2, float wd) {
-    const float interp = sg_fma(beta1, m, (1.0f - beta1) * g);
-    const float s = interp > 0.0f ? 1.0f : (interp < 0.0f ? -1.0f : 0.0f);
-    p = sg_fma(-lr, sg_fma(wd, p, s), p);
-    m = sg_fma(beta2, m, (1.0f - beta2) * g);
-}
-__global__ __launch_bounds__(THREADS) void k_lion(Batch<FamRec> B, float lr, float beta1, float beta2, float wd) {
-    int start, cnt;
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    for_tile(R, start, cnt,
-        [&](int i) {
-            float m = R.ea[i], p = sg::load_elem(R.param, R.dtype, i);
-            lion_core(sg::load_elem(R.grad, R.dtype, i), m, p, lr, beta1, beta2, wd);
-            sg::store_elem(R.param, R.dtype, i, p);
-            R.ea[i] = m;
-        },
-        [&](int i) {
-            const f32x4 g = ld4(R.grad, i);
-            f32x4 m = ld4(R.ea, i), p = ld4(R.param, i);
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+    const auto amplifier = [&](float g) {
+        if (direct || !sg_isfinite(g)) {                         // unit by unit, as written
+            float acc = 0.0f;
+            for (int h = 0; h < H; h++) acc = sg_fma(W2[h], sg_max(sg_fma(W1[h], g, b1[h]), 0.0f), acc);
+            return acc;
+        }
+        if (g > lo && g <= hi) return sg_fma(A0, g, B0);
+        int pos = 0;
+        for (int step = (slots + 1) >> 1; step > 0; step >>= 1)
+            if (g > st[pos + step - 1]) pos += step;
+        return sg_fma(sA[pos], g, sB[pos]);
+    };
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float g[V];
+        clipped_grad<V>(R, i, clip, g);
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                float mc = m[c], pc = p[c];
-                lion_core(g[c], mc, pc, lr, beta1, beta2, wd);
-                m[c] = mc;
-                p[c] = pc;
-            }
-            st4(R.param, i, p);
-            st4(R.ea, i, m);
-        });
+        for (int c = 0; c < V; c++) g[c] = g[c] * sg_fma(alpha_amp, amplifier(g[c]) + bias2, beta_amp);
+        adam_update<V>(R, i, g, beta1, 1.0f - beta1, beta2, 1.0f - beta2, eps, decay);
+    });
 }
 
-// ---- reductions: up to three sums per tile, then one block per tensor (or one for the call) -------------
-__device__ __forceinline__ void tile_sums(const Batch<FamRec>& B, double a, double b, double c) {
-    __shared__ double sm[4];
-    const double ta = block_sum(a, sm), tb = block_sum(b, sm), tc = block_sum(c, sm);
-    if (threadIdx.x == 0) {
-        B.partials[3 * (size_t)blockIdx.x + 0] = ta;
-        B.partials[3 * (size_t)blockIdx.x + 1] = tb;
-        B.partials[3 * (size_t)blockIdx.x + 2] = tc;
-    }
-}
-
-// per_tensor != 0: block t sums the tiles of tensor t into tred[t]; else one block sums every tile into tred[0]
-__global__ __launch_bounds__(THREADS) void k_sum_tiles(Batch<FamRec> B, int per_tensor) {
-    __shared__ double sm[4];
-    const int t = blockIdx.x;
-    const int lo = per_tensor ? B.prefix[t] : 0, hi = per_tensor ? B.prefix[t + 1] : B.tiles;
-    double a = 0.0, b = 0.0, c = 0.0;
-    for (int k = lo + (int)threadIdx.x; k < hi; k += THREADS) {
-        a += B.partials[3 * (size_t)k];
-        b += B.partials[3 * (size_t)k + 1];
-        c += B.partials[3 * (size_t)k + 2];
-    }
-    const double ta = block_sum(a, sm), tb = block_sum(b, sm), tc = block_sum(c, sm);
-    if (threadIdx.x == 0) {
-        B.tred[t].s[0] = ta;
-        B.tred[t].s[1] = tb;
-        B.tred[t].s[2] = tc;
-    }
-}
-
-// ---- Prodigy ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(THREADS) void k_prodigy_partial(Batch<FamRec> B) {
+// ---- Lion ------------------------------------------------------------------------
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_lion(BT B, float lr, float beta1, float beta2, float wd) {
     int start, cnt;
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    const float* p0 = static_cast<const float*>(R.aux2);
-    float num = 0.0f, den = 0.0f;
-    for_tile(R, start, cnt,
-        [&](int i) {
-            num = sg_fma(sg::load_elem(R.grad, R.dtype, i), sg::load_elem(R.param, R.dtype, i) - p0[i], num);
-            den += R.aux[i];
-        },
-        [&](int i) {
-            const f32x4 g = ld4(R.grad, i), p = ld4(R.param, i), q = ld4(p0, i), sv = ld4(R.aux, i);
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float g[V], m[V], p[V];
+        ldt<V>(R.grad, R.dtype, i, g);
+        ldf<V>(R.ea, i, m);
+        ldt<V>(R.param, R.dtype, i, p);
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
+        for (int c = 0; c < V; c++) {
+            const float interp = sg_fma(beta1, m[c], (1.0f - beta1) * g[c]);
+            const float s = interp > 0.0f ? 1.0f : (interp < 0.0f ? -1.0f : 0.0f);
+            p[c] = sg_fma(-lr, sg_fma(wd, p[c], s), p[c]);
+            m[c] = sg_fma(beta2, m[c], (1.0f - beta2) * g[c]);
+        }
+        stt<V>(R.param, R.dtype, i, p);
+        stf<V>(R.ea, i, m);
+    });
+}
+
+// ---- Prodigy (aux: s, aux2: initial parameter, fp32) --------------------------------
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_prodigy_partial(BT B, int blocks) {
+    double nsum = 0.0, dsum = 0.0;
+    for (int tile = blockIdx.x; tile < B.tiles; tile += blocks) {
+        int start, cnt;
+        const Rec& R = tile_rec(B, tile, &start, &cnt);
+        const float* p0 = static_cast<const float*>(R.aux2);
+        float num = 0.0f, den = 0.0f;
+        for_tile(R, start, cnt, [&](auto v, int i) {
+            constexpr int V = decltype(v)::value;
+            float g[V], p[V], q[V], sv[V];
+            ldt<V>(R.grad, R.dtype, i, g);
+            ldt<V>(R.param, R.dtype, i, p);
+            ldf<V>(p0, i, q);
+            ldf<V>(R.aux, i, sv);
+#pragma unroll
+            for (int c = 0; c < V; c++) {
                 num = sg_fma(g[c], p[c] - q[c], num);
                 den += sv[c];
             }
         });
-    tile_sums(B, (double)num, (double)den, 0.0);
+        nsum += (double)num;
+        dsum += (double)den;
+    }
+    tile_sums<2>(B, nsum, dsum);
 }
-
-__global__ void k_prodigy_dlr(Batch<FamRec> B, float d_lr) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const float num = (float)B.tred[0].s[0], den = (float)B.tred[0].s[1];
+// one block: the two sums and this call's d_lr, for the Adam kernel (table) and for the host (pinned, may be NULL)
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_prodigy_dlr(BT B, int blocks, float d_lr, float* host) {
+    double s[2];
+    add_tiles<2>(B, 0, blocks, s);
+    if (threadIdx.x != 0) return;
+    const float num = (float)s[0], den = (float)s[1];
     if (den > 1e-30f) d_lr = sg_max(d_lr, sg_abs(num) / (den + 1e-12f));
-    B.tred[0].d_lr = d_lr;
+    *static_cast<float*>(B.table) = d_lr;
+    if (host) __hip_atomic_store(host, d_lr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-
-__global__ __launch_bounds__(THREADS) void k_prodigy(Batch<FamRec> B, float beta1, float beta2, float lr, float wd, float eps) {
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_prodigy(BT B, float beta1, float beta2, float lr, float wd, float eps) {
     int start, cnt;
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    const float d_lr = B.tred[0].d_lr;
-    const float decay = 1.0f - (lr * d_lr) * wd, step_size = lr / R.bc1, eps_eff = d_lr * eps;
-    for_tile(R, start, cnt,
-        [&](int i) {
-            const float dg = d_lr * sg::load_elem(R.grad, R.dtype, i);
-            R.aux[i] = sg_fma(beta2, R.aux[i], ((1.0f - beta2) * dg) * dg);
-            adam_update(R, i, dg, beta1, beta2, eps_eff, decay, step_size);
-        },
-        [&](int i) {
-            f32x4 dg = ld4(R.grad, i), sv = ld4(R.aux, i);
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+    const float d_lr = *static_cast<const float*>(B.table);
+    const float decay = 1.0f - (lr * d_lr) * wd, eps_eff = d_lr * eps;
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float dg[V], sv[V];
+        ldt<V>(R.grad, R.dtype, i, dg);
+        ldf<V>(R.aux, i, sv);
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                dg[c] = d_lr * dg[c];
-                sv[c] = sg_fma(beta2, sv[c], ((1.0f - beta2) * dg[c]) * dg[c]);
-            }
-            st4(R.aux, i, sv);
-            adam_update4(R, i, dg, beta1, beta2, eps_eff, decay, step_size);
-        });
+        for (int c = 0; c < V; c++) {
+            dg[c] = d_lr * dg[c];
+            sv[c] = sg_fma(beta2, sv[c], ((1.0f - beta2) * dg[c]) * dg[c]);
+        }
+        stf<V>(R.aux, i, sv);
+        adam_update<V>(R, i, dg, beta1, 1.0f - beta1, beta2, 1.0f - beta2, eps_eff, decay);
+    });
 }
 
-// ---- SuperGrok v1.1 -------------------------------------------------------------------------------------
-template <int GELU>
-__global__ __launch_bounds__(THREADS) void k_sg11_smart(Batch<FamRec> B, const float* __restrict__ W1, const float* __restrict__ b1,
+// What a call needs to hand d_lr back to the host: a word of pinned memory that the kernel writes and an event behind
+// it, so that the host waits for the reduction alone while the update runs on.  A copy into the caller's pageable
+// memory would wait for the whole step.  Slots are kept for later calls, at most MAX_SLOTS of them; a call takes one
+// for itself, so threads and streams do not meet.
+struct HostSlot {
+    float* word = nullptr;
+    hipEvent_t done = nullptr;
+    int device = -1;
+};
+constexpr size_t MAX_SLOTS = 16;
+std::mutex g_slot_mutex;
+std::vector<HostSlot> g_slots;
+void drop_slot(HostSlot& s) {
+    if (s.done) (void)hipEventDestroy(s.done);
+    if (s.word) (void)hipHostFree(s.word);
+    s = HostSlot();
+}
+int take_slot(HostSlot* out) {
+    int dev = -1;
+    SG_HIP_CHECK(hipGetDevice(&dev));
+    {
+        std::lock_guard<std::mutex> lock(g_slot_mutex);
+        for (size_t i = 0; i < g_slots.size(); i++)
+            if (g_slots[i].device == dev) {
+                *out = g_slots[i];
+                g_slots.erase(g_slots.begin() + i);
+                return 0;
+            }
+    }
+    HostSlot s;
+    s.device = dev;
+    SG_HIP_CHECK(hipHostMalloc(&s.word, 64, hipHostMallocMapped | hipHostMallocCoherent));
+    if (hipError_t e = hipEventCreateWithFlags(&s.done, hipEventDisableTiming)) {
+        drop_slot(s);
+        return sg::fail("hipEventCreateWithFlags: %s", hipGetErrorString(e));
+    }
+    *out = s;
+    return 0;
+}
+void give_slot(HostSlot s) {
+    std::lock_guard<std::mutex> lock(g_slot_mutex);
+    if (g_slots.size() < MAX_SLOTS) g_slots.push_back(s);
+    else drop_slot(s);
+}
+
+// ---- SuperGrok v1.1 (aux: mu, aux2: sharpness) ------------------------------------------
+// The smart gradient of an element lies in the scratch at its tile's place: tile * B.tile + offset within the tile.
+template <int GELU, class BT>
+__global__ __launch_bounds__(THREADS) void k_sg11_smart(BT B, const float* __restrict__ W1, const float* __restrict__ b1,
                                                          const float* __restrict__ W2, const float* __restrict__ b2, int H,
-                                                         float rescale) {
+                                                         float clip_norm, float rescale, double* norm_partials, float* smart) {
     __shared__ float sW1[2 * MAX_HIDDEN], sb1[MAX_HIDDEN], sW2[MAX_HIDDEN];
-    for (int k = threadIdx.x; k < 2 * H; k += THREADS) sW1[k] = W1[k];
-    for (int k = threadIdx.x; k < H; k += THREADS) { sb1[k] = b1[k]; sW2[k] = W2[k]; }
-    __syncthreads();
-    const float bias2 = b2[0];
+    load_net(W1, b1, W2, H, sW1, sb1, sW2);
+    const Clip clip = global_norm(B, clip_norm);        // (its barriers cover the weights)
+    const MetaNet<GELU> net = {sW1, sb1, sW2, b2[0], H, (const __attribute__((address_space(4))) MetaPoly*)B.table};
     int start, cnt;
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    const float coef = B.red->coef;
-    const bool clip_on = B.red->clip_on != 0;
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+    float* const out = smart + (int64_t)blockIdx.x * B.tile - start;
     const float alpha = R.alpha;
     float dot = 0.0f, ss = 0.0f, mm = 0.0f;
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const int i = start + k;
-        const float g = clipped_grad(R, i, clip_on, coef);
-        const float s = sg::load_elem(R.aux2, R.dtype, i);
-        const float mu = sg_fma(alpha, R.aux[i], (1.0f - alpha) * g);
-        R.aux[i] = mu;
-        float acc = 0.0f;
-        for (int h = 0; h < H; h++) {
-            const float z = sg_fma(sW1[2 * h + 1], s, sW1[2 * h] * g) + sb1[h];
-            acc = sg_fma(sW2[h], (GELU == 0) ? sg_gelu_erf(z) : sg_gelu_sigmoid(z), acc);
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float g[V], s[V], mu[V];
+        clipped_grad<V>(R, i, clip, g);
+        ldt<V>(R.aux2, R.dtype, i, s);
+        ldf<V>(R.aux, i, mu);
+#pragma unroll
+        for (int c = 0; c < V; c++) mu[c] = sg_fma(alpha, mu[c], (1.0f - alpha) * g[c]);
+        stf<V>(R.aux, i, mu);
+#pragma unroll
+        for (int c = 0; c < V; c++) {
+            g[c] = sg_fma(rescale, net(g[c], s[c]), g[c]);
+            dot = sg_fma(g[c], mu[c], dot);
+            ss = sg_fma(g[c], g[c], ss);
+            mm = sg_fma(mu[c], mu[c], mm);
         }
-        const float smart = sg_fma(rescale, acc + bias2, g);
-        R.smart[i] = smart;
-        dot = sg_fma(smart, mu, dot);
-        ss = sg_fma(smart, smart, ss);
-        mm = sg_fma(mu, mu, mm);
-    }
-    tile_sums(B, (double)dot, (double)ss, (double)mm);
+        stf<V>(out, i, g);
+    });
+    BatchCommon C = B;
+    C.partials = norm_partials;
+    tile_sums<3>(C, (double)dot, (double)ss, (double)mm);
 }
 
-__global__ __launch_bounds__(THREADS) void k_sg11_adam(Batch<FamRec> B, float beta2, float lr, float eps, float decay, float lamb,
-                                                        float ramp, float temperature) {
-    int start, cnt;
-    const int ti = sg::upper_seg(B.prefix, B.n, (int)blockIdx.x);
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_sg11_adam(BT B, float beta2, float eps, float decay, float lamb, float ramp,
+                                                        float temperature, const float* smart) {
+    int start, cnt, ti;
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt, &ti);
+    const float* const in = smart + (int64_t)blockIdx.x * B.tile - start;
     // cosine gate of this tensor (compute_cosine_gate_fused; csrc/ops.cpp:272-278)
-    const TRed& T = B.tred[ti];
-    const float cosv = (float)T.s[0] / ((float)sqrt(T.s[1]) * (float)sqrt(T.s[2]) + 1e-8f);
+    double s[3];
+    tensor_sums<3>(B, R, ti, start, s);
+    const float cosv = (float)s[0] / ((float)sqrt(s[1]) * (float)sqrt(s[2]) + 1e-8f);
     const float gate = 1.0f / (1.0f + sg_exp(-temperature * cosv));
     const float lamb_eff = ramp > 0.0f ? (ramp * gate) * lamb : 0.0f;
-    const float step_size = lr / R.bc1;
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const int i = start + k;
-        adam_update(R, i, sg_fma(lamb_eff, R.aux[i], R.smart[i]), R.beta1, beta2, eps, decay, step_size);
-    }
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float fg[V], mu[V];
+        ldf<V>(in, i, fg);
+        ldf<V>(R.aux, i, mu);
+#pragma unroll
+        for (int c = 0; c < V; c++) fg[c] = sg_fma(lamb_eff, mu[c], fg[c]);
+        adam_update<V>(R, i, fg, R.beta1, 1.0f - R.beta1, beta2, 1.0f - beta2, eps, decay);
+    });
 }
 
 // ---- LookSAM ----------------------------------------------------------------------------------------------
-// FamRec roles: restore  param=param, aux2=backup;  directions  aux=v (fp32), grad=sam_grad, aux2=normal_grad;
-//               adjust   grad=grad, aux=v (fp32)
-__global__ __launch_bounds__(THREADS) void k_ls_restore(Batch<FamRec> B) {
+// Rec roles: restore  param=param, aux2=backup;  directions  aux=v (fp32), grad=sam_grad, aux2=normal_grad;
+//            adjust   grad=grad, aux=v (fp32)
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_ls_restore(BT B) {
     int start, cnt;
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    for (int k = threadIdx.x; k < cnt; k += THREADS) sg::store_elem(R.param, R.dtype, start + k, sg::load_elem(R.aux2, R.dtype, start + k));
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float p[V];
+        ldt<V>(R.aux2, R.dtype, i, p);
+        stt<V>(R.param, R.dtype, i, p);
+    });
 }
 
-// difference as the reference forms it: subtracted in the gradients' own type, then widened
-__device__ __forceinline__ float ls_diff(const FamRec& R, int i) {
-    const float d = sg::load_elem(R.grad, R.dtype, i) - sg::load_elem(R.aux2, R.dtype, i);
-    if (R.dtype == SG_F16) return __half2float(__float2half_rn(d));
-    if (R.dtype == SG_BF16) return sg::bf16_bits_to_f(sg::f_to_bf16_bits(d));
-    return d;
-}
-
-__global__ __launch_bounds__(THREADS) void k_ls_diff_sumsq(Batch<FamRec> B) {
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_ls_diff_sumsq(BT B) {
     int start, cnt;
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
     float acc = 0.0f;
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const float d = ls_diff(R, start + k);
-        acc = sg_fma(d, d, acc);
-    }
-    tile_sums(B, (double)acc, 0.0, 0.0);
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float a[V], b[V];
+        ldt<V>(R.grad, R.dtype, i, a);
+        ldt<V>(R.aux2, R.dtype, i, b);
+#pragma unroll
+        for (int c = 0; c < V; c++) {
+            const float d = rounded(R.dtype, a[c] - b[c]);     // as the reference forms it: subtracted in the gradients' own type
+            acc = sg_fma(d, d, acc);
+        }
+    });
+    tile_sums<1>(B, (double)acc);
 }
 
-__global__ __launch_bounds__(THREADS) void k_ls_direction(Batch<FamRec> B) {
-    int start, cnt;
-    const int ti = sg::upper_seg(B.prefix, B.n, (int)blockIdx.x);
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    const float norm = (float)sqrt(B.tred[ti].s[0]);
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_ls_direction(BT B) {
+    int start, cnt, ti;
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt, &ti);
+    double s[1];
+    tensor_sums<1>(B, R, ti, start, s);
+    const float norm = (float)sqrt(s[0]);
     if (!(norm >= 1e-12f)) return;          // that tensor's direction stays as it was
     const float inv = 1.0f / norm;
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const int i = start + k;
-        // the device branch widens both gradients before subtracting (csrc/ops.cpp:621-623)
-        R.aux[i] = (sg::load_elem(R.grad, R.dtype, i) - sg::load_elem(R.aux2, R.dtype, i)) * inv;
-    }
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float a[V], b[V];
+        ldt<V>(R.grad, R.dtype, i, a);
+        ldt<V>(R.aux2, R.dtype, i, b);
+#pragma unroll
+        for (int c = 0; c < V; c++) a[c] = (a[c] - b[c]) * inv;      // the device branch widens both gradients before subtracting (csrc/ops.cpp:621-623)
+        stf<V>(R.aux, i, a);
+    });
 }
 
-__global__ __launch_bounds__(THREADS) void k_ls_grad_sumsq(Batch<FamRec> B) {
+// sum of squares of each tensor's gradient
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_grad_sumsq(BT B) {
     int start, cnt;
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt);
     float acc = 0.0f;
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const float g = sg::load_elem(R.grad, R.dtype, start + k);
-        acc = sg_fma(g, g, acc);
-    }
-    tile_sums(B, (double)acc, 0.0, 0.0);
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float g[V];
+        ldt<V>(R.grad, R.dtype, i, g);
+#pragma unroll
+        for (int c = 0; c < V; c++) acc = sg_fma(g[c], g[c], acc);
+    });
+    tile_sums<1>(B, (double)acc);
 }
 
-__global__ __launch_bounds__(THREADS) void k_ls_adjust(Batch<FamRec> B, float la) {
-    int start, cnt;
-    const int ti = sg::upper_seg(B.prefix, B.n, (int)blockIdx.x);
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
-    const float scale = la * (float)sqrt(B.tred[ti].s[0]);
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const int i = start + k;
-        float v = R.aux[i];                  // the direction is converted to the gradient's type first (csrc/ops.cpp:646)
-        if (R.dtype == SG_F16) v = __half2float(__float2half_rn(v));
-        if (R.dtype == SG_BF16) v = sg::bf16_bits_to_f(sg::f_to_bf16_bits(v));
-        sg::store_elem(R.grad, R.dtype, i, sg_fma(scale, v, sg::load_elem(R.grad, R.dtype, i)));
-    }
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_ls_adjust(BT B, float la) {
+    int start, cnt, ti;
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt, &ti);
+    double s[1];
+    tensor_sums<1>(B, R, ti, start, s);
+    const float scale = la * (float)sqrt(s[0]);
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float d[V], g[V];
+        ldf<V>(R.aux, i, d);
+        ldt<V>(R.grad, R.dtype, i, g);
+#pragma unroll
+        for (int c = 0; c < V; c++) g[c] = sg_fma(scale, rounded(R.dtype, d[c]), g[c]);    // the direction is converted to the gradient's type first (csrc/ops.cpp:646)
+        stt<V>(R.grad, R.dtype, i, g);
+    });
 }
 
 // ---- SuperGrok v2 pre-pass: per-tensor norm clip + non-finite guard ------------------------------------------
-// FamRec roles: grad = input gradient, param = output (a new tensor, as the reference makes one)
-__global__ __launch_bounds__(THREADS) void k_sg2_clip(Batch<FamRec> B, float max_norm) {
-    int start, cnt;
-    const int ti = sg::upper_seg(B.prefix, B.n, (int)blockIdx.x);
-    const FamRec& R = tile_rec(B, blockIdx.x, &start, &cnt);
+// Rec roles: grad = input gradient, param = output (a new tensor, as the reference makes one)
+template <class BT>
+__global__ __launch_bounds__(THREADS) void k_sg2_clip(BT B, float max_norm) {
+    int start, cnt, ti;
+    const Rec& R = tile_rec(B, blockIdx.x, &start, &cnt, &ti);
+    double s[1];
+    tensor_sums<1>(B, R, ti, start, s);
     // a NaN norm compares false (no clip); an infinite one gives scale 0 and the guard below zeroes what 0*inf leaves
-    const float norm = (float)sqrt(B.tred[ti].s[0]);
+    const float norm = (float)sqrt(s[0]);
     const float scale = (norm > max_norm) ? max_norm / (norm + 1e-12f) : 1.0f;
-    for (int k = threadIdx.x; k < cnt; k += THREADS) {
-        const int i = start + k;
-        float g = sg::load_elem(R.grad, R.dtype, i);
-        if (scale != 1.0f) {
-            g = g * scale;
-            if (R.dtype == SG_F16) g = __half2float(__float2half_rn(g));        // the product is a tensor of the gradient's type
-            if (R.dtype == SG_BF16) g = sg::bf16_bits_to_f(sg::f_to_bf16_bits(g));
+    for_tile(R, start, cnt, [&](auto v, int i) {
+        constexpr int V = decltype(v)::value;
+        float g[V];
+        ldt<V>(R.grad, R.dtype, i, g);
+#pragma unroll
+        for (int c = 0; c < V; c++) {
+            if (scale != 1.0f) g[c] = rounded(R.dtype, g[c] * scale);      // the product is a tensor of the gradient's type
+            g[c] = sg::finite_or_zero(g[c]);
         }
-        sg::store_elem(R.param, R.dtype, i, sg::finite_or_zero(g));
-    }
+        stt<V>(R.param, R.dtype, i, g);
+    });
 }
 
 // ---- host side ---------------------------------------------------------------------------------------------
-enum Need { N_PARAM = 1, N_GRAD = 2, N_EA = 4, N_EASQ = 8, N_AUX = 16, N_AUX2 = 32 };
+enum Need { N_PARAM = 1, N_GRAD = 2, N_EA = 4, N_EASQ = 8, N_AUX = 16, N_AUX2 = 32, AUX2_F32 = 64 };
 
-int collect(int n, const SgFamilyTensor* ts, int need, std::vector<FamRec>* recs) {
+int collect(int n, const SgFamilyTensor* ts, int need, float lr, std::vector<Rec>* recs) {
     if (!ts) return sg::fail("NULL argument");
+    recs->reserve(n);
     for (int i = 0; i < n; i++) {
         const SgFamilyTensor& t = ts[i];
         if (t.numel == 0) continue;
         if (((need & N_PARAM) && !t.param) || ((need & N_GRAD) && !t.grad) || ((need & N_EA) && !t.exp_avg) ||
             ((need & N_EASQ) && !t.exp_avg_sq) || ((need & N_AUX) && !t.aux) || ((need & N_AUX2) && !t.aux2))
             return sg::fail("tensor %d: NULL pointer", i);
-        if (check_dtype(i, t.dtype)) return 1;
-        const uintptr_t all = (uintptr_t)t.param | (uintptr_t)t.grad | (uintptr_t)t.exp_avg | (uintptr_t)t.exp_avg_sq | (uintptr_t)t.aux |
-                              (uintptr_t)t.aux2;
-        recs->push_back({t.param, t.grad, t.exp_avg, t.exp_avg_sq, t.aux, t.aux2, nullptr, t.numel, t.dtype, t.bc1, t.bc2, t.alpha, t.beta1,
-                         (t.dtype == SG_F32 && (all & 15u) == 0) ? 1 : 0});
+        if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
+        if ((need & N_EASQ) && (!(t.bc1 > 0.0f) || !(t.bc2 > 0.0f))) return sg::fail("bias corrections must be positive (step >= 1)");
+        const uintptr_t typed = bits(t.param) | bits(t.grad) | ((need & AUX2_F32) ? 0 : bits(t.aux2));
+        const uintptr_t f32 = bits(t.exp_avg) | bits(t.exp_avg_sq) | bits(t.aux) | ((need & AUX2_F32) ? bits(t.aux2) : 0);
+        recs->push_back({t.param, t.grad, t.exp_avg, t.exp_avg_sq, t.aux, t.aux2, (int32_t)t.numel, (int16_t)t.dtype,
+                         vec4_ok(t.dtype, typed, f32), (need & N_EASQ) ? lr / t.bc1 : 0.0f, t.bc2, t.alpha, t.beta1});
     }
     return 0;
 }
 
-int check_bc(const std::vector<FamRec>& recs) {
-    for (size_t i = 0; i < recs.size(); i++)
-        if (!(recs[i].bc1 > 0.0f) || !(recs[i].bc2 > 0.0f)) return sg::fail("bias corrections must be positive (step >= 1)");
-    return 0;
-}
-
-int looksam_collect(int n, const SgLookSamTensor* ts, int mode, std::vector<FamRec>* recs) {
+int looksam_collect(int n, const SgLookSamTensor* ts, int mode, std::vector<Rec>* recs) {
     if (!ts) return sg::fail("NULL argument");
+    recs->reserve(n);
     for (int i = 0; i < n; i++) {
         const SgLookSamTensor& t = ts[i];
         if (t.numel == 0) continue;
         if (!t.a || !t.b || (mode == 1 && !t.c)) return sg::fail("tensor %d: NULL pointer", i);
-        if (check_dtype(i, t.dtype)) return 1;
-        FamRec r = {};
-        r.numel = t.numel;
-        r.dtype = t.dtype;
-        if (mode == 0) { r.param = t.a; r.aux2 = t.b; }
-        if (mode == 1) { r.aux = static_cast<float*>(t.a); r.grad = const_cast<void*>(t.b); r.aux2 = t.c; }
-        if (mode == 2) { r.grad = t.a; r.aux = const_cast<float*>(static_cast<const float*>(t.b)); }
+        if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
+        Rec r = {};
+        r.numel = (int32_t)t.numel;
+        r.dtype = (int16_t)t.dtype;
+        if (mode == 0) { r.param = t.a; r.aux2 = t.b; r.vec4 = vec4_ok(t.dtype, bits(t.a) | bits(t.b), 0); }
+        if (mode == 1) {
+            r.aux = static_cast<float*>(t.a); r.grad = const_cast<void*>(t.b); r.aux2 = t.c;
+            r.vec4 = vec4_ok(t.dtype, bits(t.b) | bits(t.c), bits(t.a));
+        }
+        if (mode == 2) {
+            r.grad = t.a; r.aux = const_cast<float*>(static_cast<const float*>(t.b));
+            r.vec4 = vec4_ok(t.dtype, bits(t.a), bits(t.b));
+        }
         recs->push_back(r);
     }
     return 0;
@@ -459,24 +507,27 @@ size_t sg_family_workspace_bytes(int num_tensors, const int64_t* numels) {
     if (num_tensors < 0 || (num_tensors > 0 && !numels)) return 0;
     sgew::Layout L;
     if (sgew::make_layout(num_tensors, numels, &L)) return 0;
-    return L.bytes + sizeof(float) * (size_t)L.total + 256;
+    // v1.1: smart gradients by tile, and partial sums of the norm apart from those of the cosine gate
+    return L.bytes + sizeof(float) * (size_t)L.tiles * L.tile + sizeof(double) * 3 * (size_t)(L.tiles + 1) + 512;
 }
 
 int sg_grokadamw_step(int num_tensors, const SgFamilyTensor* tensors, float alpha, float lamb, float beta1, float beta2, float lr,
                       float wd, float eps, float grad_clip_norm, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace sgew;
     if (num_tensors <= 0) return 0;
-    std::vector<FamRec> recs;
+    std::vector<Rec> recs;
     // the EMA buffer may be NULL for every tensor when lamb == 0: the step is then plain AdamW
-    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ | (lamb != 0.0f ? N_AUX : 0), &recs) || check_bc(recs)) return 1;
+    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ | (lamb != 0.0f ? N_AUX : 0), lr, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<FamRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    if (reduce_sumsq(recs, B, grad_clip_norm, st)) return 1;
-    hipLaunchKernelGGL(k_grokadamw, dim3(B.tiles), dim3(THREADS), 0, st, B, alpha, lamb, beta1, beta2, lr, eps, 1.0f - lr * wd);
-    SG_LAUNCH_CHECK("k_grokadamw");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        if (grad_clip_norm > 0.0f) launch_sumsq(B, st);
+        hipLaunchKernelGGL(k_grokadamw<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B, grad_clip_norm, alpha, lamb, beta1, beta2, eps,
+                           1.0f - lr * wd);
+        SG_LAUNCH_CHECK("k_grokadamw");
+        return 0;
+    });
 }
 
 int sg_neuralgrok_step(int num_tensors, const SgFamilyTensor* tensors, const SgAmplifier* amp, float alpha_amp, float beta_amp,
@@ -486,17 +537,19 @@ int sg_neuralgrok_step(int num_tensors, const SgFamilyTensor* tensors, const SgA
     if (num_tensors <= 0) return 0;
     if (!amp || !amp->W1 || !amp->b1 || !amp->W2 || !amp->b2) return sg::fail("NULL argument");
     if (amp->hidden < 1 || amp->hidden > MAX_HIDDEN) return sg::fail("hidden_dim %d outside [1,%d]", amp->hidden, MAX_HIDDEN);
-    std::vector<FamRec> recs;
-    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ, &recs) || check_bc(recs)) return 1;
+    std::vector<Rec> recs;
+    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ, lr, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<FamRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    if (reduce_sumsq(recs, B, grad_clip_norm, st)) return 1;
-    hipLaunchKernelGGL(k_neuralgrok, dim3(B.tiles), dim3(THREADS), 0, st, B, amp->W1, amp->b1, amp->W2, amp->b2, amp->hidden, alpha_amp,
-                       beta_amp, beta1, beta2, lr, eps, 1.0f - lr * wd);
-    SG_LAUNCH_CHECK("k_neuralgrok");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        const int slots = amp_slots(amp->hidden);
+        launch_sumsq(B, st, PrepAmp{amp->W1, amp->b1, amp->W2, amp->hidden, slots});
+        hipLaunchKernelGGL(k_neuralgrok<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B, amp->W1, amp->b1, amp->W2, amp->b2, amp->hidden, slots,
+                           grad_clip_norm, alpha_amp, beta_amp, beta1, beta2, eps, 1.0f - lr * wd);
+        SG_LAUNCH_CHECK("k_neuralgrok");
+        return 0;
+    });
 }
 
 int sg_prodigy_step(int num_tensors, const SgFamilyTensor* tensors, float d_lr, float beta1, float beta2, float lr, float wd, float eps,
@@ -504,37 +557,47 @@ int sg_prodigy_step(int num_tensors, const SgFamilyTensor* tensors, float d_lr, 
     using namespace sgew;
     if (d_lr_out) *d_lr_out = d_lr;
     if (num_tensors <= 0) return 0;
-    std::vector<FamRec> recs;
-    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ | N_AUX | N_AUX2, &recs) || check_bc(recs)) return 1;
+    std::vector<Rec> recs;
+    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ | N_AUX | N_AUX2 | AUX2_F32, lr, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<FamRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    hipLaunchKernelGGL(k_prodigy_partial, dim3(B.tiles), dim3(THREADS), 0, st, B);
-    hipLaunchKernelGGL(k_sum_tiles, dim3(1), dim3(THREADS), 0, st, B, 0);
-    hipLaunchKernelGGL(k_prodigy_dlr, dim3(1), dim3(64), 0, st, B, d_lr);
-    hipLaunchKernelGGL(k_prodigy, dim3(B.tiles), dim3(THREADS), 0, st, B, beta1, beta2, lr, wd, eps);
-    SG_LAUNCH_CHECK("k_prodigy");
+    HostSlot slot;
+    if (d_lr_out && take_slot(&slot)) return 1;
+    const int rc = with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        const int blocks = partial_blocks(B.tiles);
+        hipLaunchKernelGGL(k_prodigy_partial<BT>, dim3(blocks), dim3(THREADS), 0, st, B, blocks);
+        hipLaunchKernelGGL(k_prodigy_dlr<BT>, dim3(1), dim3(THREADS), 0, st, B, blocks, d_lr, slot.word);
+        if (d_lr_out) SG_HIP_CHECK(hipEventRecord(slot.done, st));
+        hipLaunchKernelGGL(k_prodigy<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B, beta1, beta2, lr, wd, eps);
+        SG_LAUNCH_CHECK("k_prodigy");
+        if (d_lr_out) {
+            SG_HIP_CHECK(hipEventSynchronize(slot.done));
+            *d_lr_out = *static_cast<volatile float*>(slot.word);
+        }
+        return 0;
+    });
     if (d_lr_out) {
-        SG_HIP_CHECK(hipMemcpyAsync(d_lr_out, &B.tred[0].d_lr, sizeof(float), hipMemcpyDeviceToHost, st));
-        SG_HIP_CHECK(hipStreamSynchronize(st));
+        if (rc == 0) give_slot(slot);
+        else drop_slot(slot);
     }
-    return 0;
+    return rc;
 }
 
 int sg_lion_step(int num_tensors, const SgFamilyTensor* tensors, float lr, float beta1, float beta2, float wd, void* workspace,
                  size_t workspace_bytes, void* stream) {
     using namespace sgew;
     if (num_tensors <= 0) return 0;
-    std::vector<FamRec> recs;
-    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA, &recs)) return 1;
+    std::vector<Rec> recs;
+    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA, lr, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<FamRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    hipLaunchKernelGGL(k_lion, dim3(B.tiles), dim3(THREADS), 0, st, B, lr, beta1, beta2, wd);
-    SG_LAUNCH_CHECK("k_lion");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        hipLaunchKernelGGL(k_lion<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B, lr, beta1, beta2, wd);
+        SG_LAUNCH_CHECK("k_lion");
+        return 0;
+    });
 }
 
 int sg11_fused_step(int num_tensors, const SgFamilyTensor* tensors, const Sg15Net* net, float beta2, float lr, float wd, float eps,
@@ -545,104 +608,121 @@ int sg11_fused_step(int num_tensors, const SgFamilyTensor* tensors, const Sg15Ne
     if (!net || !net->W1 || !net->b1 || !net->W2 || !net->b2) return sg::fail("NULL argument");
     if (net->hidden < 1 || net->hidden > MAX_HIDDEN) return sg::fail("hidden_dim %d outside [1,%d]", net->hidden, MAX_HIDDEN);
     if (net->gelu_mode != 0 && net->gelu_mode != 1) return sg::fail("bad gelu_mode %d", net->gelu_mode);
-    std::vector<FamRec> recs;
-    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ | N_AUX | N_AUX2, &recs) || check_bc(recs)) return 1;
+    std::vector<Rec> recs;
+    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ | N_AUX | N_AUX2, lr, &recs)) return 1;
     if (recs.empty()) return 0;
-    // the smart-gradient scratch follows the bookkeeping region
+    // scratch behind the bookkeeping region: partial sums of the cosine gates, then the smart gradients
     std::vector<int64_t> numels(recs.size());
     for (size_t i = 0; i < recs.size(); i++) numels[i] = recs[i].numel;
     Layout L;
     if (make_layout((int)recs.size(), numels.data(), &L)) return 1;
-    const size_t need = L.bytes + sizeof(float) * (size_t)L.total;
+    const size_t gate_bytes = sg::align_up(sizeof(double) * 3 * (size_t)(L.tiles + 1), 256);
+    const size_t need = L.bytes + gate_bytes + sizeof(float) * (size_t)L.tiles * L.tile;
     if (!workspace || workspace_bytes < need) return sg::fail("workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
-    float* smart = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + L.bytes);
-    for (size_t i = 0; i < recs.size(); i++) { recs[i].smart = smart; smart += recs[i].numel; }
+    double* gates = reinterpret_cast<double*>(static_cast<unsigned char*>(workspace) + L.bytes);
+    float* smart = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + L.bytes + gate_bytes);
     hipStream_t st = (hipStream_t)stream;
-    Batch<FamRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    if (reduce_sumsq(recs, B, grad_clip_norm, st)) return 1;
-    if (net->gelu_mode == 0)
-        hipLaunchKernelGGL(k_sg11_smart<0>, dim3(B.tiles), dim3(THREADS), 0, st, B, net->W1, net->b1, net->W2, net->b2, net->hidden, net->rescale);
-    else
-        hipLaunchKernelGGL(k_sg11_smart<1>, dim3(B.tiles), dim3(THREADS), 0, st, B, net->W1, net->b1, net->W2, net->b2, net->hidden, net->rescale);
-    hipLaunchKernelGGL(k_sum_tiles, dim3(B.n), dim3(THREADS), 0, st, B, 1);
-    hipLaunchKernelGGL(k_sg11_adam, dim3(B.tiles), dim3(THREADS), 0, st, B, beta2, lr, eps, 1.0f - lr * wd, lamb, ramp, gate_temperature);
-    SG_LAUNCH_CHECK("k_sg11");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        const auto run = [&](auto gelu) {
+            hipLaunchKernelGGL((k_sg11_smart<decltype(gelu)::value, BT>), dim3(B.tiles), dim3(THREADS), 0, st, B, net->W1, net->b1, net->W2,
+                               net->b2, net->hidden, grad_clip_norm, net->rescale, gates, smart);
+        };
+        if (net->gelu_mode == 0) {
+            launch_sumsq(B, st, PrepMetaPoly{net->W1, net->b1, net->W2, net->b2, net->hidden});
+            run(std::integral_constant<int, 0>{});
+        } else {
+            launch_sumsq(B, st);
+            run(std::integral_constant<int, 1>{});
+        }
+        BT G = B;
+        G.partials = gates;
+        launch_tensor_sums<3>(G, st);
+        hipLaunchKernelGGL(k_sg11_adam<BT>, dim3(B.tiles), dim3(THREADS), 0, st, G, beta2, eps, 1.0f - lr * wd, lamb, ramp, gate_temperature,
+                           smart);
+        SG_LAUNCH_CHECK("k_sg11");
+        return 0;
+    });
 }
 
 int sg2_clip_grads(int num_tensors, const Sg2ClipTensor* tensors, float max_norm, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace sgew;
     if (num_tensors <= 0) return 0;
     if (!tensors) return sg::fail("NULL argument");
-    std::vector<FamRec> recs;
+    std::vector<Rec> recs;
+    recs.reserve(num_tensors);
     for (int i = 0; i < num_tensors; i++) {
         const Sg2ClipTensor& t = tensors[i];
         if (t.numel == 0) continue;
         if (!t.grad || !t.out) return sg::fail("tensor %d: NULL pointer", i);
-        if (check_dtype(i, t.dtype)) return 1;
-        FamRec r = {};
+        if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
+        Rec r = {};
         r.grad = const_cast<void*>(t.grad);
         r.param = t.out;
-        r.numel = t.numel;
-        r.dtype = t.dtype;
+        r.numel = (int32_t)t.numel;
+        r.dtype = (int16_t)t.dtype;
+        r.vec4 = vec4_ok(t.dtype, bits(t.grad) | bits(t.out), 0);
         recs.push_back(r);
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<FamRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    hipLaunchKernelGGL(k_ls_grad_sumsq, dim3(B.tiles), dim3(THREADS), 0, st, B);
-    hipLaunchKernelGGL(k_sum_tiles, dim3(B.n), dim3(THREADS), 0, st, B, 1);
-    hipLaunchKernelGGL(k_sg2_clip, dim3(B.tiles), dim3(THREADS), 0, st, B, max_norm);
-    SG_LAUNCH_CHECK("k_sg2_clip");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        hipLaunchKernelGGL(k_grad_sumsq<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
+        launch_tensor_sums<1>(B, st);
+        hipLaunchKernelGGL(k_sg2_clip<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B, max_norm);
+        SG_LAUNCH_CHECK("k_sg2_clip");
+        return 0;
+    });
 }
 
 int sg_looksam_restore(int num_tensors, const SgLookSamTensor* tensors, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace sgew;
     if (num_tensors <= 0) return 0;
-    std::vector<FamRec> recs;
+    std::vector<Rec> recs;
     if (looksam_collect(num_tensors, tensors, 0, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<FamRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    hipLaunchKernelGGL(k_ls_restore, dim3(B.tiles), dim3(THREADS), 0, st, B);
-    SG_LAUNCH_CHECK("k_ls_restore");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        hipLaunchKernelGGL(k_ls_restore<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
+        SG_LAUNCH_CHECK("k_ls_restore");
+        return 0;
+    });
 }
 
 int sg_looksam_directions(int num_tensors, const SgLookSamTensor* tensors, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace sgew;
     if (num_tensors <= 0) return 0;
-    std::vector<FamRec> recs;
+    std::vector<Rec> recs;
     if (looksam_collect(num_tensors, tensors, 1, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<FamRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    hipLaunchKernelGGL(k_ls_diff_sumsq, dim3(B.tiles), dim3(THREADS), 0, st, B);
-    hipLaunchKernelGGL(k_sum_tiles, dim3(B.n), dim3(THREADS), 0, st, B, 1);
-    hipLaunchKernelGGL(k_ls_direction, dim3(B.tiles), dim3(THREADS), 0, st, B);
-    SG_LAUNCH_CHECK("k_ls_direction");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        hipLaunchKernelGGL(k_ls_diff_sumsq<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
+        launch_tensor_sums<1>(B, st);
+        hipLaunchKernelGGL(k_ls_direction<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
+        SG_LAUNCH_CHECK("k_ls_direction");
+        return 0;
+    });
 }
 
 int sg_looksam_adjust(int num_tensors, const SgLookSamTensor* tensors, float la, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace sgew;
     if (num_tensors <= 0) return 0;
-    std::vector<FamRec> recs;
+    std::vector<Rec> recs;
     if (looksam_collect(num_tensors, tensors, 2, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    Batch<FamRec> B;
-    if (upload(recs, workspace, workspace_bytes, st, &B)) return 1;
-    hipLaunchKernelGGL(k_ls_grad_sumsq, dim3(B.tiles), dim3(THREADS), 0, st, B);
-    hipLaunchKernelGGL(k_sum_tiles, dim3(B.n), dim3(THREADS), 0, st, B, 1);
-    hipLaunchKernelGGL(k_ls_adjust, dim3(B.tiles), dim3(THREADS), 0, st, B, la);
-    SG_LAUNCH_CHECK("k_ls_adjust");
-    return 0;
+    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+        using BT = std::decay_t<decltype(B)>;
+        hipLaunchKernelGGL(k_grad_sumsq<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
+        launch_tensor_sums<1>(B, st);
+        hipLaunchKernelGGL(k_ls_adjust<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B, la);
+        SG_LAUNCH_CHECK("k_ls_adjust");
+        return 0;
+    });
 }
 
 }  // extern "C"

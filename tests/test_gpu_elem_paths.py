@@ -1,0 +1,89 @@
+"""The elementwise kernels at the edges of their dispatch: amplifier tables of every width class with units that have no
+threshold, gradients on both sides of the meta-net polynomial's reach, tensor counts on both sides of what travels
+as kernel arguments, and pointers that do not allow four elements per access."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import rel_close
+from oracle import family_oracle as fo
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _ops():
+    from grokking_optimizers import _ops
+    return _ops
+
+
+def _dev(arrs, shift=0):
+    """device copies; shift: element offset from an aligned address"""
+    out = []
+    for a in arrs:
+        buf = torch.zeros(a.size + shift, device=DEV)
+        buf[shift:].copy_(torch.from_numpy(a))
+        out.append(buf[shift:])
+    return out
+
+
+def _check(got, want, tag):
+    for k in got:
+        for i, (a, b) in enumerate(zip(got[k], want[k])):
+            ok, worst = rel_close(a.cpu().numpy(), b, 1e-4, 1e-7)
+            assert ok, (tag, k, i, worst)
+
+
+def _state(r, sizes, gstd):
+    f = lambda std: [(r.randn(n) * std).astype(np.float32) for n in sizes]
+    return dict(p=f(0.02), g=f(gstd), ea=f(1e-3), easq=[np.abs(x) * 1e-3 for x in f(1e-3)], aux=f(1e-3), sh=[np.abs(x) for x in f(gstd)])
+
+
+@pytest.mark.parametrize("H", [1, 2, 3, 127, 128, 255, 256])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_amplifier_table(H, shift):
+    r = np.random.RandomState(H)
+    w1, b1, w2, b2 = (r.randn(H, 1)).astype(np.float32), (r.randn(H) * 0.5).astype(np.float32), (r.randn(1, H) * 0.1).astype(np.float32), \
+        np.float32([0.05])
+    w1[::5] = 0.0                      # units that do not look at the gradient
+    b1[::7] = 0.0                      # thresholds at 0
+    st = _state(r, [5000, 3], 0.7)     # gradients on every side of the thresholds
+    st["g"][1][0] = 0.0
+    want = {k: [x.copy() for x in v] for k, v in st.items()}
+    got = {k: _dev(v, shift) for k, v in st.items()}
+    sc = (10.0, 4.0, 0.9, 0.98, 1e-3, 1.0, 1e-8, 0.0)
+    W = [torch.from_numpy(x).to(DEV) for x in (w1, b1, w2, b2)]
+    _ops().neuralgrok_fused_step(got["p"], got["g"], got["ea"], got["easq"], [3, 3], *W, sc[0], sc[1], H, *sc[2:])
+    fo.neuralgrok_step(want["p"], want["g"], want["ea"], want["easq"], [3, 3], w1, b1, w2, b2, *sc)
+    _check({k: got[k] for k in ("p", "g", "ea", "easq")}, want, H)
+
+
+@pytest.mark.parametrize("H", [1, 32, 256])
+@pytest.mark.parametrize("gstd", [1e-3, 0.03, 1.0])
+def test_meta_net_polynomial(H, gstd):
+    r = np.random.RandomState(int(H + 1000 * gstd))
+    W = [(r.randn(H, 2) * 0.5).astype(np.float32), (r.randn(H) * 0.5).astype(np.float32), (r.randn(1, H) * 0.5).astype(np.float32), np.float32([0.1])]
+    st = _state(r, [4099, 700], gstd)
+    want = {k: [x.copy() for x in v] for k, v in st.items()}
+    got = {k: _dev(v) for k, v in st.items()}
+    sc = (0.1, 0.999, 1e-3, 1.0, 1e-8, 5.0, 0.7, 5.0, 1.0)
+    al, be = [0.98, 0.97], [0.9, 0.81]
+    Wd = [torch.from_numpy(x).to(DEV) for x in W]
+    _ops().supergrok11_fused_step(got["p"], got["g"], got["ea"], got["easq"], got["aux"], got["sh"], [4, 4], al, be, *Wd, sc[0], H, *sc[1:])
+    fo.sg11_step(want["p"], want["g"], want["ea"], want["easq"], want["aux"], want["sh"], [4, 4], al, be, *W, *sc)
+    _check({k: got[k] for k in ("p", "g", "ea", "easq", "aux")}, want, (H, gstd))
+
+
+@pytest.mark.parametrize("P", [49, 50, 51, 70])
+def test_tensor_counts(P):
+    r = np.random.RandomState(P)
+    sizes = [1 + 37 * i for i in range(P)]
+    st = _state(r, sizes, 0.05)
+    want = {k: [x.copy() for x in v] for k, v in st.items()}
+    got = {k: _dev(v) for k, v in st.items()}
+    sc = (0.98, 5.0, 0.9, 0.98, 1e-3, 1.0, 1e-8, 1.0)
+    _ops().grokadamw_fused_step(got["p"], got["g"], got["ea"], got["easq"], got["aux"], [2] * P, *sc)
+    fo.grokadamw_step(want["p"], want["g"], want["ea"], want["easq"], want["aux"], [2] * P, *sc)
+    _check({k: got[k] for k in ("p", "g", "ea", "easq", "aux")}, want, P)
+    clipped = _ops().supergrok2_clip_grads(got["sh"], 1e-3)
+    _check({"c": clipped}, {"c": fo.sg2_clip(want["sh"], 1e-3)}, P)
