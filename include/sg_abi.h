@@ -25,6 +25,9 @@ extern "C" {
 
 /* element type of param / grad / sharpness tensors */
 enum { SG_F32 = 0, SG_F16 = 1, SG_BF16 = 2 };
+/* OR-ed into the dtype of a tensor whose sharpness array is fp32 although parameter and gradient are 16-bit: the
+ * kernels round a sharpness value to the tensor's type as they read it (the value a converted copy would hold). */
+#define SG_SHARP_F32 256
 
 /* meta-net dimensions, the trailing ints of
  * launch_mamba3_peer_batched_step (csrc/ops.h:196-229).  The step takes every
@@ -195,6 +198,10 @@ typedef struct SgGrokfastTensor {
     int64_t numel;
     int32_t dtype;
 } SgGrokfastTensor;
+/* Tensors whose records travel as kernel arguments.  With at most this many (non-empty) ones the steps of a single
+ * launch - sg_grokfast_ema, sg_grokfast_adamw_step, sg_lion_step, sg_grokadamw_step without clipping - need no
+ * workspace and take NULL. */
+#define SG_ELEMWISE_ARG_TENSORS 50
 int sg_grokfast_ema(int num_tensors, const SgGrokfastTensor* tensors, float alpha, float lamb,
                     void* workspace, size_t workspace_bytes, void* stream);
 
@@ -229,7 +236,7 @@ int sg_grokfast_adamw_step(int num_tensors, const SgGrokfastAdamTensor* tensors,
 typedef struct Sg15Tensor {
     void* param;            /* [numel] dtype */
     void* grad;             /* [numel] dtype, rescaled in place when clipping is active */
-    const void* sharpness;  /* [numel] dtype */
+    const void* sharpness;  /* [numel] dtype (fp32 with SG_SHARP_F32) */
     float* exp_avg;         /* [numel] fp32 */
     float* exp_avg_sq;      /* [numel] fp32 */
     float* mu;              /* [numel] fp32 */
@@ -414,7 +421,7 @@ typedef struct SgFamilyTensor {
     float* exp_avg;     /* [numel] fp32 */
     float* exp_avg_sq;  /* [numel] fp32 (not Lion) */
     float* aux;         /* [numel] fp32: GrokAdamW ema, Prodigy s, SuperGrok v1.1 mu */
-    const void* aux2;   /* Prodigy: param_init [numel] fp32; SuperGrok v1.1: sharpness [numel] dtype */
+    const void* aux2;   /* Prodigy: param_init [numel] fp32; SuperGrok v1.1: sharpness [numel] dtype (fp32 with SG_SHARP_F32) */
     int64_t numel;
     int32_t dtype;
     float bc1, bc2;     /* 1 - beta1^step, 1 - beta2^step as the caller computed them */

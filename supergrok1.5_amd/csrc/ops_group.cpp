@@ -1,0 +1,430 @@
+// Native bodies of the optimizer classes' step(): one call per parameter group
+// walks the group's parameters, gradients and state and forwards to the C ABI.
+// The lists that the `_ops.*_fused_step` functions take cost a Python loop over
+// the parameters and one reference per tensor and list on the way in, 11 of the
+// 18 us of host time of a Grokfast step on 14 tensors whose kernel takes 5 us.
+//
+// A call that meets anything but the ordinary case (state not created yet, a
+// step counter that is no int) changes nothing and returns False; the class then
+// takes its Python path, which creates the state and calls the list functions.
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <algorithm>
+#include <cmath>
+#include <vector>
+
+#include "ops_common.hpp"
+
+namespace {
+
+struct Member {
+    const at::Tensor *p, *g;
+    const at::Tensor* b[4];
+    PyObject* state;
+    long long step;
+};
+
+PyObject* name_of(const char* s) { return PyUnicode_InternFromString(s); }      // kept for the life of the process
+
+const at::Tensor* as_tensor(PyObject* o) { return o && THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+// Entry of optimizer.state for a parameter, or NULL.  torch's Tensor hashes by identity through a Python-level
+// __hash__; the identity is tried first and the general lookup serves subclasses that hash otherwise.
+PyObject* state_entry(PyObject* state, PyObject* param) {
+    PyObject* e = _PyDict_GetItem_KnownHash(state, param, (Py_hash_t)(uintptr_t)param);
+    if (!e) e = PyDict_GetItemWithError(state, param);
+    if (!e) PyErr_Clear();
+    return e;
+}
+
+// The group's parameters that have a non-empty gradient, with `n` state buffers each; steps counted up when `count`.
+// False (and nothing changed) where the general path has to be taken.
+bool gather(PyObject* params, PyObject* state, PyObject* const* names, int n, bool count, std::vector<Member>* out) {
+    static PyObject* const kStep = name_of("step");
+    if (!PyList_Check(params) || !PyDict_Check(state)) return false;
+    const Py_ssize_t P = PyList_GET_SIZE(params);
+    out->reserve(P);
+    for (Py_ssize_t i = 0; i < P; i++) {
+        PyObject* po = PyList_GET_ITEM(params, i);
+        Member m;
+        m.p = as_tensor(po);
+        if (!m.p) return false;
+        m.g = &m.p->grad();
+        if (!m.g->defined()) continue;
+        m.state = state_entry(state, po);
+        if (!m.state || !PyDict_Check(m.state)) return false;
+        for (int k = 0; k < n; k++) {
+            m.b[k] = as_tensor(PyDict_GetItem(m.state, names[k]));
+            if (!m.b[k]) return false;
+        }
+        m.step = 0;
+        if (count) {
+            PyObject* s = PyDict_GetItem(m.state, kStep);
+            if (!s || !PyLong_CheckExact(s)) return false;
+            m.step = PyLong_AsLongLong(s) + 1;
+        }
+        out->push_back(m);
+    }
+    if (count) {
+        long long shared = -1;
+        PyObject* value = nullptr;       // parameters of a group are nearly always at one step: one int object for all
+        for (Member& m : *out) {
+            if (m.step != shared) {
+                Py_XDECREF(value);
+                value = PyLong_FromLongLong(m.step);
+                shared = m.step;
+            }
+            PyDict_SetItem(m.state, kStep, value);
+        }
+        Py_XDECREF(value);
+    }
+    return true;
+}
+
+void check_pair(const at::Tensor& p, const at::Tensor& g, const char* fn) {
+    check_gpu(p, fn, "param");
+    check_gpu(g, fn, "grad");
+    TORCH_CHECK(p.scalar_type() == g.scalar_type(), fn, ": param/grad dtype mismatch");
+    TORCH_CHECK(p.numel() == g.numel(), fn, ": param/grad size mismatch");
+}
+float* f32_ptr(const at::Tensor& t, int64_t n, const char* fn, const char* what) {
+    check_f32(t, fn, what);
+    TORCH_CHECK(t.numel() == n, fn, ": ", what, " size mismatch");
+    return t.data_ptr<float>();
+}
+
+// per-step bias corrections, computed once for tensors at the same step
+struct FloatCorrections {       // float pow, as the reference computes them (csrc/ops.cpp:333-334)
+    float beta1, beta2, bc1 = 1.0f, bc2 = 1.0f;
+    long long at = -1;
+    void operator()(long long step) {
+        if (step == at) return;
+        at = step;
+        bc1 = 1.0f - std::pow(beta1, static_cast<float>(step));
+        bc2 = 1.0f - std::pow(beta2, static_cast<float>(step));
+    }
+};
+
+struct Family {
+    std::vector<SgFamilyTensor> ts;
+    std::vector<int64_t> numels;
+    const at::Tensor* first = nullptr;
+    torch::Tensor ws;
+    void add(const SgFamilyTensor& t, const at::Tensor* g) {
+        ts.push_back(t);
+        numels.push_back(t.numel);
+        if (!first) first = g;
+    }
+    void make_ws() { ws = make_workspace(sg_family_workspace_bytes((int)ts.size(), numels.data()), *first); }
+    void* stream() const { return current_stream(*first); }
+};
+
+// exp_avg, exp_avg_sq (n >= 2), aux (n >= 3), aux2 in fp32 (n >= 4), in the order the names were given
+Family family_of(const std::vector<Member>& ms, int n, const char* fn) {
+    Family F;
+    F.ts.reserve(ms.size());
+    F.numels.reserve(ms.size());
+    for (const Member& m : ms) {
+        if (m.g->numel() == 0) continue;
+        check_pair(*m.p, *m.g, fn);
+        SgFamilyTensor t = {};
+        t.param = m.p->data_ptr();
+        t.grad = m.g->data_ptr();
+        t.numel = m.g->numel();
+        t.dtype = dtype_code(*m.g, "grad");
+        t.exp_avg = f32_ptr(*m.b[0], t.numel, fn, "exp_avg");
+        if (n > 1) t.exp_avg_sq = f32_ptr(*m.b[1], t.numel, fn, "exp_avg_sq");
+        if (n > 2) t.aux = f32_ptr(*m.b[2], t.numel, fn, "state");
+        if (n > 3) t.aux2 = f32_ptr(*m.b[3], t.numel, fn, "param_init");
+        t.bc1 = t.bc2 = 1.0f;
+        F.add(t, m.g);
+    }
+    return F;
+}
+// (members with an empty gradient are skipped by family_of: the corrections follow the same rule)
+template <class C>
+void correct(Family* F, const std::vector<Member>& ms, C corr) {
+    size_t k = 0;
+    for (const Member& m : ms) {
+        if (m.g->numel() == 0) continue;
+        corr(m.step);
+        F->ts[k].bc1 = corr.bc1;
+        F->ts[k].bc2 = corr.bc2;
+        k++;
+    }
+}
+
+bool grokfast_group_step(py::handle params, py::handle state, float alpha, float lamb, double lr, double beta1, double beta2, double eps,
+                         double weight_decay) {
+    const char* fn = "grokfast_adamw_fused_step";
+    static PyObject* const names[3] = {name_of("ema"), name_of("exp_avg"), name_of("exp_avg_sq")};
+    std::vector<Member> ms;
+    if (!gather(params.ptr(), state.ptr(), names, 3, true, &ms)) return false;
+    std::vector<SgGrokfastAdamTensor> ts;
+    std::vector<int64_t> numels;
+    ts.reserve(ms.size());
+    numels.reserve(ms.size());
+    const at::Tensor* first = nullptr;
+    for (const Member& m : ms) {
+        const int64_t n = m.g->numel();
+        if (n == 0) continue;
+        check_pair(*m.p, *m.g, fn);
+        ts.push_back({m.p->data_ptr(), m.g->data_ptr(), f32_ptr(*m.b[0], n, fn, "ema_buf"), f32_ptr(*m.b[1], n, fn, "exp_avg"),
+                      f32_ptr(*m.b[2], n, fn, "exp_avg_sq"), n, dtype_code(*m.g, "grad"), (int32_t)m.step});
+        numels.push_back(n);
+        if (!first) first = m.g;
+    }
+    if (ts.empty()) return true;
+    torch::Tensor ws;
+    if (ts.size() > SG_ELEMWISE_ARG_TENSORS) ws = make_workspace(sg_elemwise_workspace_bytes((int)ts.size(), numels.data()), *first);
+    check_status(sg_grokfast_adamw_step((int)ts.size(), ts.data(), alpha, lamb, lr, beta1, beta2, eps, weight_decay,
+                                        ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? (size_t)ws.numel() : 0, current_stream(*first)),
+                 fn);
+    return true;
+}
+
+bool lion_group_step(py::handle params, py::handle state, float lr, float beta1, float beta2, float wd) {
+    static PyObject* const names[1] = {name_of("exp_avg")};
+    std::vector<Member> ms;
+    if (!gather(params.ptr(), state.ptr(), names, 1, false, &ms)) return false;
+    Family F = family_of(ms, 1, "lion_fused_step");
+    if (F.ts.empty()) return true;
+    const bool ws = F.ts.size() > SG_ELEMWISE_ARG_TENSORS;
+    if (ws) F.make_ws();
+    check_status(sg_lion_step((int)F.ts.size(), F.ts.data(), lr, beta1, beta2, wd, ws ? F.ws.data_ptr() : nullptr,
+                              ws ? (size_t)F.ws.numel() : 0, F.stream()), "lion_fused_step");
+    return true;
+}
+
+bool grokadamw_group_step(py::handle params, py::handle state, float alpha, float lamb, float beta1, float beta2, float lr, float wd,
+                          float eps, float grad_clip_norm) {
+    static PyObject* const names[3] = {name_of("exp_avg"), name_of("exp_avg_sq"), name_of("ema")};
+    std::vector<Member> ms;
+    if (!gather(params.ptr(), state.ptr(), names, 3, true, &ms)) return false;
+    Family F = family_of(ms, 3, "grokadamw_fused_step");
+    if (F.ts.empty()) return true;
+    correct(&F, ms, FloatCorrections{beta1, beta2});
+    F.make_ws();
+    check_status(sg_grokadamw_step((int)F.ts.size(), F.ts.data(), alpha, lamb, beta1, beta2, lr, wd, eps, grad_clip_norm, F.ws.data_ptr(),
+                                   (size_t)F.ws.numel(), F.stream()), "grokadamw_fused_step");
+    return true;
+}
+
+// AdamW with bias corrections in double (adamw_step of _adamw_helper.py)
+struct DoubleCorrections {
+    double beta1, beta2;
+    float bc1 = 1.0f, bc2 = 1.0f;
+    long long at = -1;
+    void operator()(long long step) {
+        if (step == at) return;
+        at = step;
+        bc1 = (float)(1.0 - std::pow(beta1, (double)step));
+        bc2 = (float)(1.0 - std::pow(beta2, (double)step));
+    }
+};
+bool adamw_group_step(py::handle params, py::handle state, double lr, double beta1, double beta2, double eps, double wd) {
+    static PyObject* const names[2] = {name_of("exp_avg"), name_of("exp_avg_sq")};
+    std::vector<Member> ms;
+    if (!gather(params.ptr(), state.ptr(), names, 2, true, &ms)) return false;
+    Family F = family_of(ms, 2, "adamw_fused_step");
+    if (F.ts.empty()) return true;
+    correct(&F, ms, DoubleCorrections{beta1, beta2});
+    const bool ws = F.ts.size() > SG_ELEMWISE_ARG_TENSORS;
+    if (ws) F.make_ws();
+    check_status(sg_grokadamw_step((int)F.ts.size(), F.ts.data(), 0.0f, 0.0f, (float)beta1, (float)beta2, (float)lr, (float)wd, (float)eps,
+                                   0.0f, ws ? F.ws.data_ptr() : nullptr, ws ? (size_t)F.ws.numel() : 0, F.stream()), "adamw_fused_step");
+    return true;
+}
+
+bool neuralgrok_group_step(py::handle params, py::handle state, const torch::Tensor& W1, const torch::Tensor& b1, const torch::Tensor& W2,
+                           const torch::Tensor& b2, float alpha_amp, float beta_amp, int hidden_dim, float beta1, float beta2, float lr,
+                           float wd, float eps, float grad_clip_norm) {
+    const char* fn = "neuralgrok_fused_step";
+    static PyObject* const names[2] = {name_of("exp_avg"), name_of("exp_avg_sq")};
+    std::vector<Member> ms;
+    if (!gather(params.ptr(), state.ptr(), names, 2, true, &ms)) return false;
+    Family F = family_of(ms, 2, fn);
+    if (F.ts.empty()) return true;
+    correct(&F, ms, FloatCorrections{beta1, beta2});
+    check_f32(W1, fn, "W1"); check_f32(b1, fn, "b1"); check_f32(W2, fn, "W2"); check_f32(b2, fn, "b2");
+    TORCH_CHECK(W1.numel() == hidden_dim && b1.numel() == hidden_dim && W2.numel() == hidden_dim && b2.numel() == 1, fn,
+                ": amplifier weight shapes do not match hidden_dim");
+    SgAmplifier amp = {W1.data_ptr<float>(), b1.data_ptr<float>(), W2.data_ptr<float>(), b2.data_ptr<float>(), hidden_dim};
+    F.make_ws();
+    check_status(sg_neuralgrok_step((int)F.ts.size(), F.ts.data(), &amp, alpha_amp, beta_amp, beta1, beta2, lr, wd, eps, grad_clip_norm,
+                                    F.ws.data_ptr(), (size_t)F.ws.numel(), F.stream()), fn);
+    return true;
+}
+
+// the new d_lr, or None where the general path has to be taken
+py::object prodigy_group_step(py::handle params, py::handle state, float d_lr, float beta1, float beta2, float lr, float wd, float eps) {
+    static PyObject* const names[4] = {name_of("exp_avg"), name_of("exp_avg_sq"), name_of("s"), name_of("param_init")};
+    std::vector<Member> ms;
+    if (!gather(params.ptr(), state.ptr(), names, 4, true, &ms)) return py::none();
+    Family F = family_of(ms, 4, "prodigy_fused_step");
+    if (F.ts.empty()) return py::float_(d_lr);
+    correct(&F, ms, FloatCorrections{beta1, beta2});
+    F.make_ws();
+    float out = d_lr;
+    check_status(sg_prodigy_step((int)F.ts.size(), F.ts.data(), d_lr, beta1, beta2, lr, wd, eps, &out, F.ws.data_ptr(), (size_t)F.ws.numel(),
+                                 F.stream()), "prodigy_fused_step");
+    return py::float_(out);
+}
+
+bool muon_group_step(py::handle params, py::handle state, float momentum, float lr, float wd, int ns_steps) {
+    const char* fn = "muon_fused_step";
+    static PyObject* const names[1] = {name_of("momentum_buffer")};
+    std::vector<Member> ms;
+    if (!gather(params.ptr(), state.ptr(), names, 1, false, &ms)) return false;
+    std::vector<SgMuonMatrix> mats;
+    mats.reserve(ms.size());
+    const at::Tensor* first = nullptr;
+    for (const Member& m : ms) {
+        if (m.g->numel() == 0) continue;
+        check_pair(*m.p, *m.g, fn);
+        TORCH_CHECK(m.p->dim() == 2, fn, ": parameters must be 2-D");
+        mats.push_back({m.p->data_ptr(), m.g->data_ptr(), f32_ptr(*m.b[0], m.p->numel(), fn, "momentum buffer"), m.p->size(0), m.p->size(1),
+                        dtype_code(*m.p, "param")});
+        if (!first) first = m.p;
+    }
+    if (mats.empty()) return true;
+    auto ws = make_workspace(sg_muon_workspace_bytes((int)mats.size(), mats.data()), *first);
+    check_status(sg_muon_step((int)mats.size(), mats.data(), momentum, lr, wd, ns_steps, ws.data_ptr(), (size_t)ws.numel(),
+                              current_stream(*first)), fn);
+    return true;
+}
+
+// ---- SuperGrok v1.5 / v1.1: flat lists, one entry per parameter of the optimizer ---------------
+struct FlatLists {
+    PyObject *params, *data, *ea, *easq, *mu, *sharp, *steps, *factors, *beta1s;
+    Py_ssize_t n;
+    bool ok() const {
+        for (PyObject* l : {params, data, ea, easq, mu, sharp, steps, factors, beta1s})
+            if (!PyList_Check(l) || PyList_GET_SIZE(l) != n) return false;
+        return true;
+    }
+    const at::Tensor& at(PyObject* list, Py_ssize_t i) const {
+        const at::Tensor* t = as_tensor(PyList_GET_ITEM(list, i));
+        TORCH_CHECK(t, "optimizer state list holds a non-tensor");
+        return *t;
+    }
+};
+// sharpness is kept in fp32: the kernel rounds it to the gradient's type as it reads it
+int sharp_code(const at::Tensor& sharp, const at::Tensor& g, const char* fn) {
+    check_gpu(sharp, fn, "sharpness");
+    TORCH_CHECK(sharp.numel() == g.numel(), fn, ": sharpness size mismatch");
+    const int code = dtype_code(g, "grad");
+    if (sharp.scalar_type() == g.scalar_type()) return code;
+    TORCH_CHECK(sharp.scalar_type() == torch::kFloat32, fn, ": sharpness must be float32 or have the gradient's dtype");
+    return code | SG_SHARP_F32;
+}
+struct NetArgs {
+    torch::Tensor t[4];
+    Sg15Net net;
+    NetArgs(const torch::Tensor& W1, const torch::Tensor& b1, const torch::Tensor& W2, const torch::Tensor& b2, int hidden, float rescale,
+            const char* fn) {
+        const torch::Tensor* in[4] = {&W1, &b1, &W2, &b2};
+        for (int k = 0; k < 4; k++) {
+            t[k] = in[k]->to(torch::kFloat32).contiguous();
+            check_f32(t[k], fn, "meta-net weight");
+        }
+        TORCH_CHECK(W1.numel() == 2 * hidden && b1.numel() == hidden && W2.numel() == hidden && b2.numel() == 1, fn,
+                    ": meta-net weight shapes do not match hidden_dim");
+        net = {t[0].data_ptr<float>(), t[1].data_ptr<float>(), t[2].data_ptr<float>(), t[3].data_ptr<float>(), hidden, rescale,
+               g_sg15_gelu_mode};
+    }
+};
+// calls f(i, grad, alpha_i, beta1_i, bc1, bc2) for every parameter with a non-empty gradient
+template <class F>
+void each_flat(const FlatLists& L, double alpha, float beta2, F f) {
+    for (Py_ssize_t i = 0; i < L.n; i++) {
+        const at::Tensor& g = L.at(L.params, i).grad();
+        if (!g.defined() || g.numel() == 0) continue;
+        // the step counters go into the call by value, as in the reference: a call counts its own copy up
+        const float step = static_cast<float>(PyLong_AsLongLong(PyList_GET_ITEM(L.steps, i)) + 1);
+        const double a = std::max(0.0, std::min(1.0, alpha * PyFloat_AsDouble(PyList_GET_ITEM(L.factors, i))));
+        const float b1 = (float)PyFloat_AsDouble(PyList_GET_ITEM(L.beta1s, i));
+        if (PyErr_Occurred()) throw py::error_already_set();
+        f(i, g, (float)a, b1, 1.0f - std::pow(b1, step), 1.0f - std::pow(beta2, step));
+    }
+}
+
+bool supergrok15_flat_step(py::handle params, py::handle data, py::handle eas, py::handle easqs, py::handle mus, py::handle sharps,
+                           py::handle steps, double alpha, py::handle alpha_factors, py::handle beta1s, const torch::Tensor& W1,
+                           const torch::Tensor& b1, const torch::Tensor& W2, const torch::Tensor& b2, float rescale, int hidden, float beta2,
+                           float lr, float wd_eff, float eps, float lamb, float ramp, float gate_signal, float grad_clip_norm) {
+    const char* fn = "supergrok15_fused_step";
+    const FlatLists L = {params.ptr(), data.ptr(), eas.ptr(), easqs.ptr(), mus.ptr(), sharps.ptr(), steps.ptr(), alpha_factors.ptr(),
+                         beta1s.ptr(), PyList_Check(params.ptr()) ? PyList_GET_SIZE(params.ptr()) : -1};
+    if (!L.ok()) return false;
+    std::vector<Sg15Tensor> ts;
+    std::vector<int64_t> numels;
+    ts.reserve(L.n);
+    numels.reserve(L.n);
+    const at::Tensor* first = nullptr;
+    each_flat(L, alpha, beta2, [&](Py_ssize_t i, const at::Tensor& g, float a, float be, float bc1, float bc2) {
+        const at::Tensor& p = L.at(L.data, i);
+        check_pair(p, g, fn);
+        const int64_t n = g.numel();
+        const at::Tensor& s = L.at(L.sharp, i);
+        ts.push_back({p.data_ptr(), g.data_ptr(), s.data_ptr(), f32_ptr(L.at(L.ea, i), n, fn, "exp_avg"),
+                      f32_ptr(L.at(L.easq, i), n, fn, "exp_avg_sq"), f32_ptr(L.at(L.mu, i), n, fn, "mu"), n, sharp_code(s, g, fn), a, be,
+                      bc1, bc2});
+        numels.push_back(n);
+        if (!first) first = &p;
+    });
+    if (ts.empty()) return true;
+    const NetArgs N(W1, b1, W2, b2, hidden, rescale, fn);
+    const float lamb_eff = ramp > 0.0f ? ramp * gate_signal * lamb : 0.0f;
+    auto ws = make_workspace(sg_elemwise_workspace_bytes((int)ts.size(), numels.data()), *first);
+    check_status(sg15_fused_step((int)ts.size(), ts.data(), &N.net, lamb_eff, beta2, lr, wd_eff, eps, grad_clip_norm, ws.data_ptr(),
+                                 (size_t)ws.numel(), current_stream(*first)), fn);
+    return true;
+}
+
+bool supergrok11_flat_step(py::handle params, py::handle data, py::handle eas, py::handle easqs, py::handle mus, py::handle sharps,
+                           py::handle steps, double alpha, py::handle alpha_factors, py::handle beta1s, const torch::Tensor& W1,
+                           const torch::Tensor& b1, const torch::Tensor& W2, const torch::Tensor& b2, float rescale, int hidden, float beta2,
+                           float lr, float wd_eff, float eps, float lamb, float ramp, float gate_temperature, float grad_clip_norm) {
+    const char* fn = "supergrok11_fused_step";
+    const FlatLists L = {params.ptr(), data.ptr(), eas.ptr(), easqs.ptr(), mus.ptr(), sharps.ptr(), steps.ptr(), alpha_factors.ptr(),
+                         beta1s.ptr(), PyList_Check(params.ptr()) ? PyList_GET_SIZE(params.ptr()) : -1};
+    if (!L.ok()) return false;
+    Family F;
+    each_flat(L, alpha, beta2, [&](Py_ssize_t i, const at::Tensor& g, float a, float be, float bc1, float bc2) {
+        const at::Tensor& p = L.at(L.data, i);
+        check_pair(p, g, fn);
+        const at::Tensor& s = L.at(L.sharp, i);
+        SgFamilyTensor t = {};
+        t.numel = g.numel();
+        t.dtype = sharp_code(s, g, fn);
+        t.param = p.data_ptr();
+        t.grad = g.data_ptr();
+        t.aux2 = s.data_ptr();
+        t.exp_avg = f32_ptr(L.at(L.ea, i), t.numel, fn, "exp_avg");
+        t.exp_avg_sq = f32_ptr(L.at(L.easq, i), t.numel, fn, "exp_avg_sq");
+        t.aux = f32_ptr(L.at(L.mu, i), t.numel, fn, "mu");
+        t.bc1 = bc1; t.bc2 = bc2; t.alpha = a; t.beta1 = be;
+        F.add(t, &p);
+    });
+    if (F.ts.empty()) return true;
+    const NetArgs N(W1, b1, W2, b2, hidden, rescale, fn);
+    F.make_ws();
+    check_status(sg11_fused_step((int)F.ts.size(), F.ts.data(), &N.net, beta2, lr, wd_eff, eps, lamb, ramp, gate_temperature, grad_clip_norm,
+                                 F.ws.data_ptr(), (size_t)F.ws.numel(), F.stream()), fn);
+    return true;
+}
+
+}  // namespace
+
+void bind_group_steps(pybind11::module_& m) {
+    m.def("grokfast_group_step", &grokfast_group_step);
+    m.def("lion_group_step", &lion_group_step);
+    m.def("grokadamw_group_step", &grokadamw_group_step);
+    m.def("adamw_group_step", &adamw_group_step);
+    m.def("neuralgrok_group_step", &neuralgrok_group_step);
+    m.def("prodigy_group_step", &prodigy_group_step);
+    m.def("muon_group_step", &muon_group_step);
+    m.def("supergrok15_flat_step", &supergrok15_flat_step);
+    m.def("supergrok11_flat_step", &supergrok11_flat_step);
+}

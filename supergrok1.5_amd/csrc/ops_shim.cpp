@@ -5,51 +5,12 @@
 // function validates its tensors and forwards to the C ABI of libsg_hip.so
 // (include/sg_abi.h) on PyTorch's current HIP stream; scratch memory comes from
 // the caching allocator.  There is no CPU path: non-GPU tensors raise.
-#include <torch/extension.h>
-#include <c10/hip/HIPStream.h>
-
 #include <cmath>
-#include <stdexcept>
-#include <string>
 #include <vector>
 
-#include "../../include/sg_abi.h"
-
-namespace {
-
-void* current_stream(const torch::Tensor& t) {
-    return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream();
-}
-
-int dtype_code(const torch::Tensor& t, const char* what) {
-    switch (t.scalar_type()) {
-        case torch::kFloat32: return SG_F32;
-        case torch::kFloat16: return SG_F16;
-        case torch::kBFloat16: return SG_BF16;
-        default: TORCH_CHECK(false, what, ": unsupported dtype ", t.scalar_type());
-    }
-    return -1;
-}
-
-void check_gpu(const torch::Tensor& t, const char* fn, const char* what) {
-    if (!t.is_cuda()) throw std::runtime_error(std::string(fn) + " requires CUDA tensors (" + what + " is on the CPU).");
-    TORCH_CHECK(t.is_contiguous(), fn, ": ", what, " must be contiguous");
-}
-void check_f32(const torch::Tensor& t, const char* fn, const char* what) {
-    check_gpu(t, fn, what);
-    TORCH_CHECK(t.scalar_type() == torch::kFloat32, fn, ": ", what, " must be float32");
-}
-
-torch::Tensor make_workspace(size_t bytes, const torch::Tensor& like) {
-    return torch::empty({(int64_t)std::max<size_t>(bytes, 256)},
-                        torch::TensorOptions().device(like.device()).dtype(torch::kUInt8));
-}
-
-void check_status(int rc, const char* fn) { TORCH_CHECK(rc == 0, fn, ": ", sg_last_error()); }
+#include "ops_common.hpp"
 
 int g_sg15_gelu_mode = 0;   // 0 exact erf GELU, 1 sigmoid approximation
-
-}  // namespace
 
 // ───────────────────────── Grokfast ─────────────────────────
 void grokfast_fused_step(std::vector<torch::Tensor>& grads, std::vector<torch::Tensor>& ema_bufs, float alpha, float lamb) {
@@ -744,4 +705,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "SuperGrok2 bilevel: batched forward scan with state saving");
     m.def("supergrok2_bilevel_backward_batched", &supergrok2_bilevel_backward_batched, "SuperGrok2 bilevel: batched backward through scan");
     m.def("supergrok2_bilevel_backward", &supergrok2_bilevel_backward, "SuperGrok2 bilevel: full backward through meta-net");
+    bind_group_steps(m);
 }

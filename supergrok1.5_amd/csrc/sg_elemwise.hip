@@ -53,7 +53,7 @@ __global__ __launch_bounds__(THREADS) void k_sg15(BT B, const float* __restrict_
         constexpr int V = decltype(v)::value;
         float g[V], s[V], mu[V];
         clipped_grad<V>(R, i, clip, g);
-        ldt<V>(R.aux2, R.dtype, i, s);
+        ldsharp<V>(R, i, s);
         ldf<V>(R.aux, i, mu);
 #pragma unroll
         for (int c = 0; c < V; c++) mu[c] = sg_fma(alpha, mu[c], (1.0f - alpha) * g[c]);
@@ -124,11 +124,11 @@ int sg_grokfast_ema(int num_tensors, const SgGrokfastTensor* tensors, float alph
         if (!t.grad || !t.ema) return sg::fail("tensor %d: NULL pointer", i);
         if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
         recs.push_back({nullptr, t.grad, nullptr, nullptr, t.ema, nullptr, (int32_t)t.numel, (int16_t)t.dtype,
-                        vec4_ok(t.dtype, bits(t.grad), bits(t.ema)), 0.0f, 1.0f, 0.0f, 0.0f});
+                        vec4_ok(t.dtype, bits(t.grad), bits(t.ema)), 0, 0.0f, 1.0f, 0.0f, 0.0f});
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, false, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         hipLaunchKernelGGL((k_grokfast<false, BT>), dim3(B.tiles), dim3(THREADS), 0, st, B, alpha, lamb, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
         SG_LAUNCH_CHECK("k_grokfast<ema>");
@@ -159,12 +159,12 @@ int sg_grokfast_adamw_step(int num_tensors, const SgGrokfastAdamTensor* tensors,
             last_step = t.step;
         }
         recs.push_back({t.param, t.grad, t.exp_avg, t.exp_avg_sq, t.ema, nullptr, (int32_t)t.numel, (int16_t)t.dtype,
-                        vec4_ok(t.dtype, bits(t.param) | bits(t.grad), bits(t.ema) | bits(t.exp_avg) | bits(t.exp_avg_sq)),
+                        vec4_ok(t.dtype, bits(t.param) | bits(t.grad), bits(t.ema) | bits(t.exp_avg) | bits(t.exp_avg_sq)), 0,
                         (float)(lr / bc1), (float)bc2, 0.0f, 0.0f});
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, false, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         hipLaunchKernelGGL((k_grokfast<true, BT>), dim3(B.tiles), dim3(THREADS), 0, st, B, alpha, lamb, (float)beta1,
                            (float)(1.0 - beta1), (float)beta2, (float)(1.0 - beta2), (float)eps, (float)(1.0 - lr * weight_decay));
@@ -186,14 +186,17 @@ int sg15_fused_step(int num_tensors, const Sg15Tensor* tensors, const Sg15Net* n
         const Sg15Tensor& t = tensors[i];
         if (t.numel == 0) continue;
         if (!t.param || !t.grad || !t.sharpness || !t.exp_avg || !t.exp_avg_sq || !t.mu) return sg::fail("tensor %d: NULL pointer", i);
-        if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
-        recs.push_back({t.param, t.grad, t.exp_avg, t.exp_avg_sq, t.mu, t.sharpness, (int32_t)t.numel, (int16_t)t.dtype,
-                        vec4_ok(t.dtype, bits(t.param) | bits(t.grad) | bits(t.sharpness), bits(t.exp_avg) | bits(t.exp_avg_sq) | bits(t.mu)),
+        const int dtype = t.dtype & ~SG_SHARP_F32;
+        const bool s32 = t.dtype != dtype;
+        if (check_dtype(i, dtype) || check_numel(i, t.numel)) return 1;
+        recs.push_back({t.param, t.grad, t.exp_avg, t.exp_avg_sq, t.mu, t.sharpness, (int32_t)t.numel, (int16_t)dtype,
+                        vec4_ok(dtype, bits(t.param) | bits(t.grad) | (s32 ? 0 : bits(t.sharpness)),
+                                bits(t.exp_avg) | bits(t.exp_avg_sq) | bits(t.mu) | (s32 ? bits(t.sharpness) : 0)), (int8_t)s32,
                         lr / t.bc1, t.bc2, t.alpha, t.beta1});
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, true, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         const float decay = 1.0f - lr * wd_eff;
         const auto run = [&](auto gelu) {
@@ -225,11 +228,11 @@ int sg15_sam_perturb(int num_tensors, const Sg15SamTensor* tensors, float rho, v
         if (!t.param || !t.grad) return sg::fail("tensor %d: NULL pointer", i);
         if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
         recs.push_back({t.param, const_cast<void*>(t.grad), nullptr, nullptr, nullptr, nullptr, (int32_t)t.numel, (int16_t)t.dtype,
-                        vec4_ok(t.dtype, bits(t.param) | bits(t.grad), 0), 0.0f, 1.0f, 0.0f, 0.0f});
+                        vec4_ok(t.dtype, bits(t.param) | bits(t.grad), 0), 0, 0.0f, 1.0f, 0.0f, 0.0f});
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, true, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         launch_sumsq(B, st);
         hipLaunchKernelGGL(k_sam_perturb<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B, rho);
@@ -252,12 +255,12 @@ int sg15_sharpness_restore(int num_tensors, const Sg15RestoreTensor* tensors, vo
         if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
         recs.push_back({t.param, const_cast<void*>(t.normal_grad), static_cast<float*>(t.sharpness),
                         static_cast<float*>(const_cast<void*>(t.backup)), nullptr, t.sam_grad, (int32_t)t.numel, (int16_t)t.dtype,
-                        vec4_ok(t.dtype, bits(t.param) | bits(t.sharpness) | bits(t.backup) | bits(t.sam_grad) | bits(t.normal_grad), 0),
+                        vec4_ok(t.dtype, bits(t.param) | bits(t.sharpness) | bits(t.backup) | bits(t.sam_grad) | bits(t.normal_grad), 0), 0,
                         0.0f, 1.0f, 0.0f, 0.0f});
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, false, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         hipLaunchKernelGGL(k_restore<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
         SG_LAUNCH_CHECK("k_restore");

@@ -31,7 +31,9 @@ struct Rec {
     float* aux;
     const void* aux2;
     int32_t numel;
-    int16_t dtype, vec4;   // vec4: every pointer allows four elements per lane and access
+    int16_t dtype;
+    int8_t vec4;           // every pointer allows four elements per lane and access
+    int8_t sharp32;        // aux2 (sharpness) is fp32, rounded to dtype when read
     float step_size, bc2, alpha, beta1;
 };
 static_assert(sizeof(Rec) == 72, "Rec layout");
@@ -83,7 +85,7 @@ struct BatchCommon {
 // The records of a call as kernel arguments.  A launch of a copy kernel that only carries the table costs 1.6 us of
 // its own and about as much again before the next kernel starts, a third of a Grokfast step on 14 tensors.  CAP: the
 // argument block stays below 4 KB.
-constexpr int CAP = 50;
+constexpr int CAP = SG_ELEMWISE_ARG_TENSORS;
 struct BatchArg : BatchCommon {
     Rec recs[CAP];
     int prefix[CAP];      // first tile of tensor i + 1
@@ -95,15 +97,16 @@ struct BatchPtr : BatchCommon {
     const int* prefix;    // [n + 1]
 };
 
-// Calls f(batch) with the records as kernel arguments where they fit, else uploaded into the workspace.
+// Calls f(batch) with the records as kernel arguments where they fit, else uploaded into the workspace.  scratch:
+// whether the step uses partial sums or a table.
 template <class F>
-int with_batch(const std::vector<Rec>& recs, void* workspace, size_t ws_bytes, hipStream_t st, F&& f) {
+int with_batch(const std::vector<Rec>& recs, void* workspace, size_t ws_bytes, hipStream_t st, bool scratch, F&& f) {
     const int n = (int)recs.size();
     std::vector<int64_t> numels(n);
     for (int i = 0; i < n; i++) numels[i] = recs[i].numel;
     Layout L;
     if (make_layout(n, numels.data(), &L)) return 1;
-    if (!workspace || ws_bytes < L.bytes) return sg::fail("workspace too small: need %zu bytes, got %zu", L.bytes, ws_bytes);
+    if ((scratch || n > CAP) && (!workspace || ws_bytes < L.bytes)) return sg::fail("workspace too small: need %zu bytes, got %zu", L.bytes, ws_bytes);
     if (((uintptr_t)workspace & 255u) != 0) return sg::fail("workspace must be 256-byte aligned");
     unsigned char* ws = static_cast<unsigned char*>(workspace);
     BatchCommon c;
@@ -207,6 +210,15 @@ __device__ __forceinline__ float rounded(int dtype, float v) {
     if (dtype == SG_F16) return __half2float(__float2half_rn(v));
     if (dtype == SG_BF16) return sg::bf16_bits_to_f(sg::f_to_bf16_bits(v));
     return v;
+}
+
+// sharpness of a tensor: in its type, or in fp32 and rounded to it
+template <int V>
+__device__ __forceinline__ void ldsharp(const Rec& R, int i, float (&x)[V]) {
+    if (!R.sharp32) return ldt<V>(R.aux2, R.dtype, i, x);
+    ldf<V>(static_cast<const float*>(R.aux2), i, x);
+#pragma unroll
+    for (int c = 0; c < V; c++) x[c] = rounded(R.dtype, x[c]);
 }
 
 // Runs body(V, i) over the elements of a tile: four consecutive ones per lane where the tensor's pointers allow
@@ -349,7 +361,7 @@ inline int check_numel(int i, int64_t n) {
     return 0;
 }
 // typed: pointers in the tensor's type OR-ed together; f32: fp32 pointers
-inline int16_t vec4_ok(int dtype, uintptr_t typed, uintptr_t f32) {
+inline int8_t vec4_ok(int dtype, uintptr_t typed, uintptr_t f32) {
     return (f32 & 15u) == 0 && (typed & (dtype == SG_F32 ? 15u : 7u)) == 0 ? 1 : 0;
 }
 inline uintptr_t bits(const void* p) { return (uintptr_t)p; }

@@ -297,7 +297,7 @@ __global__ __launch_bounds__(THREADS) void k_sg11_smart(BT B, const float* __res
         constexpr int V = decltype(v)::value;
         float g[V], s[V], mu[V];
         clipped_grad<V>(R, i, clip, g);
-        ldt<V>(R.aux2, R.dtype, i, s);
+        ldsharp<V>(R, i, s);
         ldf<V>(R.aux, i, mu);
 #pragma unroll
         for (int c = 0; c < V; c++) mu[c] = sg_fma(alpha, mu[c], (1.0f - alpha) * g[c]);
@@ -452,7 +452,7 @@ __global__ __launch_bounds__(THREADS) void k_sg2_clip(BT B, float max_norm) {
 }
 
 // ---- host side ---------------------------------------------------------------------------------------------
-enum Need { N_PARAM = 1, N_GRAD = 2, N_EA = 4, N_EASQ = 8, N_AUX = 16, N_AUX2 = 32, AUX2_F32 = 64 };
+enum Need { N_PARAM = 1, N_GRAD = 2, N_EA = 4, N_EASQ = 8, N_AUX = 16, N_AUX2 = 32, AUX2_F32 = 64, SHARP = 128 };      // SHARP: aux2 is a sharpness array
 
 int collect(int n, const SgFamilyTensor* ts, int need, float lr, std::vector<Rec>* recs) {
     if (!ts) return sg::fail("NULL argument");
@@ -463,12 +463,14 @@ int collect(int n, const SgFamilyTensor* ts, int need, float lr, std::vector<Rec
         if (((need & N_PARAM) && !t.param) || ((need & N_GRAD) && !t.grad) || ((need & N_EA) && !t.exp_avg) ||
             ((need & N_EASQ) && !t.exp_avg_sq) || ((need & N_AUX) && !t.aux) || ((need & N_AUX2) && !t.aux2))
             return sg::fail("tensor %d: NULL pointer", i);
-        if (check_dtype(i, t.dtype) || check_numel(i, t.numel)) return 1;
+        const int dtype = (need & SHARP) ? t.dtype & ~SG_SHARP_F32 : t.dtype;
+        const bool s32 = t.dtype != dtype, aux2_f32 = s32 || (need & AUX2_F32);
+        if (check_dtype(i, dtype) || check_numel(i, t.numel)) return 1;
         if ((need & N_EASQ) && (!(t.bc1 > 0.0f) || !(t.bc2 > 0.0f))) return sg::fail("bias corrections must be positive (step >= 1)");
-        const uintptr_t typed = bits(t.param) | bits(t.grad) | ((need & AUX2_F32) ? 0 : bits(t.aux2));
-        const uintptr_t f32 = bits(t.exp_avg) | bits(t.exp_avg_sq) | bits(t.aux) | ((need & AUX2_F32) ? bits(t.aux2) : 0);
-        recs->push_back({t.param, t.grad, t.exp_avg, t.exp_avg_sq, t.aux, t.aux2, (int32_t)t.numel, (int16_t)t.dtype,
-                         vec4_ok(t.dtype, typed, f32), (need & N_EASQ) ? lr / t.bc1 : 0.0f, t.bc2, t.alpha, t.beta1});
+        const uintptr_t typed = bits(t.param) | bits(t.grad) | (aux2_f32 ? 0 : bits(t.aux2));
+        const uintptr_t f32 = bits(t.exp_avg) | bits(t.exp_avg_sq) | bits(t.aux) | (aux2_f32 ? bits(t.aux2) : 0);
+        recs->push_back({t.param, t.grad, t.exp_avg, t.exp_avg_sq, t.aux, t.aux2, (int32_t)t.numel, (int16_t)dtype,
+                         vec4_ok(dtype, typed, f32), (int8_t)s32, (need & N_EASQ) ? lr / t.bc1 : 0.0f, t.bc2, t.alpha, t.beta1});
     }
     return 0;
 }
@@ -520,7 +522,7 @@ int sg_grokadamw_step(int num_tensors, const SgFamilyTensor* tensors, float alph
     if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ | (lamb != 0.0f ? N_AUX : 0), lr, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, grad_clip_norm > 0.0f, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         if (grad_clip_norm > 0.0f) launch_sumsq(B, st);
         hipLaunchKernelGGL(k_grokadamw<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B, grad_clip_norm, alpha, lamb, beta1, beta2, eps,
@@ -541,7 +543,7 @@ int sg_neuralgrok_step(int num_tensors, const SgFamilyTensor* tensors, const SgA
     if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ, lr, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, true, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         const int slots = amp_slots(amp->hidden);
         launch_sumsq(B, st, PrepAmp{amp->W1, amp->b1, amp->W2, amp->hidden, slots});
@@ -563,7 +565,7 @@ int sg_prodigy_step(int num_tensors, const SgFamilyTensor* tensors, float d_lr, 
     hipStream_t st = (hipStream_t)stream;
     HostSlot slot;
     if (d_lr_out && take_slot(&slot)) return 1;
-    const int rc = with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    const int rc = with_batch(recs, workspace, workspace_bytes, st, true, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         const int blocks = partial_blocks(B.tiles);
         hipLaunchKernelGGL(k_prodigy_partial<BT>, dim3(blocks), dim3(THREADS), 0, st, B, blocks);
@@ -592,7 +594,7 @@ int sg_lion_step(int num_tensors, const SgFamilyTensor* tensors, float lr, float
     if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA, lr, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, false, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         hipLaunchKernelGGL(k_lion<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B, lr, beta1, beta2, wd);
         SG_LAUNCH_CHECK("k_lion");
@@ -609,7 +611,7 @@ int sg11_fused_step(int num_tensors, const SgFamilyTensor* tensors, const Sg15Ne
     if (net->hidden < 1 || net->hidden > MAX_HIDDEN) return sg::fail("hidden_dim %d outside [1,%d]", net->hidden, MAX_HIDDEN);
     if (net->gelu_mode != 0 && net->gelu_mode != 1) return sg::fail("bad gelu_mode %d", net->gelu_mode);
     std::vector<Rec> recs;
-    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ | N_AUX | N_AUX2, lr, &recs)) return 1;
+    if (collect(num_tensors, tensors, N_PARAM | N_GRAD | N_EA | N_EASQ | N_AUX | N_AUX2 | SHARP, lr, &recs)) return 1;
     if (recs.empty()) return 0;
     // scratch behind the bookkeeping region: partial sums of the cosine gates, then the smart gradients
     std::vector<int64_t> numels(recs.size());
@@ -622,7 +624,7 @@ int sg11_fused_step(int num_tensors, const SgFamilyTensor* tensors, const Sg15Ne
     double* gates = reinterpret_cast<double*>(static_cast<unsigned char*>(workspace) + L.bytes);
     float* smart = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + L.bytes + gate_bytes);
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, true, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         const auto run = [&](auto gelu) {
             hipLaunchKernelGGL((k_sg11_smart<decltype(gelu)::value, BT>), dim3(B.tiles), dim3(THREADS), 0, st, B, net->W1, net->b1, net->W2,
@@ -666,7 +668,7 @@ int sg2_clip_grads(int num_tensors, const Sg2ClipTensor* tensors, float max_norm
     }
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, true, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         hipLaunchKernelGGL(k_grad_sumsq<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
         launch_tensor_sums<1>(B, st);
@@ -683,7 +685,7 @@ int sg_looksam_restore(int num_tensors, const SgLookSamTensor* tensors, void* wo
     if (looksam_collect(num_tensors, tensors, 0, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, false, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         hipLaunchKernelGGL(k_ls_restore<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
         SG_LAUNCH_CHECK("k_ls_restore");
@@ -698,7 +700,7 @@ int sg_looksam_directions(int num_tensors, const SgLookSamTensor* tensors, void*
     if (looksam_collect(num_tensors, tensors, 1, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, true, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         hipLaunchKernelGGL(k_ls_diff_sumsq<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
         launch_tensor_sums<1>(B, st);
@@ -715,7 +717,7 @@ int sg_looksam_adjust(int num_tensors, const SgLookSamTensor* tensors, float la,
     if (looksam_collect(num_tensors, tensors, 2, &recs)) return 1;
     if (recs.empty()) return 0;
     hipStream_t st = (hipStream_t)stream;
-    return with_batch(recs, workspace, workspace_bytes, st, [&](const auto& B) {
+    return with_batch(recs, workspace, workspace_bytes, st, true, [&](const auto& B) {
         using BT = std::decay_t<decltype(B)>;
         hipLaunchKernelGGL(k_grad_sumsq<BT>, dim3(B.tiles), dim3(THREADS), 0, st, B);
         launch_tensor_sums<1>(B, st);

@@ -24,10 +24,12 @@ class GrokAdamW(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay, alpha=alpha, lamb=lamb,
                                       gamma=gamma, decay=decay, grad_clip=grad_clip))
 
-    @torch.no_grad()
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         for group in self.param_groups:
+            if _ops.grokadamw_group_step(group["params"], self.state, group["alpha"], group["lamb"], group["betas"][0], group["betas"][1],
+                                         group["lr"], group["weight_decay"], group["eps"], group["grad_clip"]):
+                continue
             s = gather(self, group, ("exp_avg", "exp_avg_sq", "ema"))
             if not s["params"]:
                 continue

@@ -4,7 +4,7 @@ Drop-in for the reference class (grokking_optimizers/grokfast.py:30-145):
 same constructor arguments and defaults, same per-parameter state
 (`step`, `ema`, `exp_avg`, `exp_avg_sq`, all fp32), `p.grad` overwritten with
 the amplified gradient.  The whole step is ONE fused kernel launch over all
-parameters (`_ops.grokfast_adamw_fused_step`); `fused=False` keeps the
+parameters (`_ops.grokfast_group_step`); `fused=False` keeps the
 reference's two-phase sequence (`_ops.grokfast_fused_step`, then AdamW).
 """
 from typing import Iterable, Optional, Tuple
@@ -34,13 +34,16 @@ class Grokfast(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay,
                                       grokfast_alpha=grokfast_alpha, grokfast_lamb=grokfast_lamb))
 
-    @torch.no_grad()
     def step(self, closure=None) -> Optional[float]:
         loss = None
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
         for group in self.param_groups:
+            b1, b2 = group["betas"]
+            if self.fused and _ops.grokfast_group_step(group["params"], self.state, group["grokfast_alpha"], group["grokfast_lamb"],
+                                                       group["lr"], b1, b2, group["eps"], group["weight_decay"]):
+                continue
             ps, gs, emas, ms, vs, ts = [], [], [], [], [], []
             for p in group["params"]:
                 if p.grad is None:
@@ -59,7 +62,6 @@ class Grokfast(Optimizer):
                 ts.append(st["step"])
             if not ps:
                 continue
-            b1, b2 = group["betas"]
             if self.fused:
                 _ops.grokfast_adamw_fused_step(ps, gs, emas, ms, vs, ts, group["grokfast_alpha"],
                                                group["grokfast_lamb"], group["lr"], b1, b2, group["eps"],

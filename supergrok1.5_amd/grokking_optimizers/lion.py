@@ -19,10 +19,11 @@ class Lion(Optimizer):
         check_hyper(lr, None, betas)
         super().__init__(params, dict(lr=lr, betas=betas, weight_decay=weight_decay))
 
-    @torch.no_grad()
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         for group in self.param_groups:
+            if _ops.lion_group_step(group["params"], self.state, group["lr"], group["betas"][0], group["betas"][1], group["weight_decay"]):
+                continue
             ps, gs, ms = [], [], []
             for p in group["params"]:
                 if p.grad is None:

@@ -31,11 +31,13 @@ class LookSAM(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay, rho=rho, k=k, alpha=alpha))
         self._global_step: int = 0
 
-    @torch.no_grad()
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         self._global_step += 1
         for group in self.param_groups:
+            if _ops.adamw_group_step(group["params"], self.state, group["lr"], group["betas"][0], group["betas"][1], group["eps"],
+                                     group["weight_decay"]):
+                continue
             s = gather(self, group, self._BUFFERS)
             if s["params"]:
                 adamw_step(s["params"], s["grads"], s["exp_avg"], s["exp_avg_sq"], s["steps"], group["lr"], group["betas"][0],

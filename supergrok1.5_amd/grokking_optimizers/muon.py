@@ -33,7 +33,6 @@ class Muon(Optimizer):
         super().__init__(groups, dict(lr=lr, momentum=momentum, weight_decay=weight_decay, ns_steps=ns_steps,
                                       group_type="muon"))
 
-    @torch.no_grad()
     def step(self, closure=None) -> Optional[float]:
         loss = None
         if closure is not None:
@@ -47,6 +46,8 @@ class Muon(Optimizer):
         return loss
 
     def _step_muon(self, group) -> None:
+        if _ops.muon_group_step(group["params"], self.state, group["momentum"], group["lr"], group["weight_decay"], group["ns_steps"]):
+            return
         ps, gs, bufs = [], [], []
         for p in group["params"]:
             if p.grad is None:
@@ -61,6 +62,9 @@ class Muon(Optimizer):
             _ops.muon_fused_step(ps, gs, bufs, group["momentum"], group["lr"], group["weight_decay"], group["ns_steps"])
 
     def _step_adamw(self, group) -> None:
+        b1, b2 = group.get("betas", (0.9, 0.98))
+        if _ops.adamw_group_step(group["params"], self.state, group["lr"], b1, b2, group.get("eps", 1e-8), group["weight_decay"]):
+            return
         ps, gs, ms, vs, ts = [], [], [], [], []
         for p in group["params"]:
             if p.grad is None:
@@ -77,5 +81,4 @@ class Muon(Optimizer):
             vs.append(st["exp_avg_sq"])
             ts.append(st["step"])
         if ps:
-            b1, b2 = group.get("betas", (0.9, 0.98))
             adamw_step(ps, gs, ms, vs, ts, group["lr"], b1, b2, group.get("eps", 1e-8), group["weight_decay"])

@@ -46,19 +46,37 @@ class NeuralGrok(Optimizer):
                                       inner_steps=inner_steps, grad_clip=grad_clip))
         self._meta_weights_dirty = True
         self._cached_meta_weights = None
+        self._device_weights = {}
 
-    @torch.no_grad()
+    def _weights_on(self, dev):
+        """The amplifier's four tensors on `dev`.  An amplifier that lives elsewhere is copied again when its weights
+        have changed (in-place updates count up a tensor's version, a new extraction makes new tensors)."""
+        weights = self._cached_meta_weights
+        if weights[0].device == dev:
+            return weights
+        key = tuple((id(w), w._version) for w in weights)
+        held = self._device_weights.get(dev)
+        if held is None or held[0] != key:
+            held = self._device_weights[dev] = (key, tuple(w.to(dev) for w in weights))
+        return held[1]
+
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         if self._meta_weights_dirty or self._cached_meta_weights is None:
             self._cached_meta_weights = self.amplifier.get_weights()
+            self._device_weights.clear()
             self._meta_weights_dirty = False
         for group in self.param_groups:
+            dev = next((p.device for p in group["params"] if p.grad is not None), None)
+            if dev is not None and dev.type == "cuda" and _ops.neuralgrok_group_step(
+                    group["params"], self.state, *self._weights_on(dev), group["alpha"], group["beta"], self.amplifier.hidden_dim,
+                    group["betas"][0], group["betas"][1], group["lr"], group["weight_decay"], group["eps"], group["grad_clip"]):
+                continue
             s = gather(self, group, ("exp_avg", "exp_avg_sq"))
             if not s["params"]:
                 continue
             dev = s["params"][0].device
-            W1, b1, W2, b2 = (w.to(dev) for w in self._cached_meta_weights)
+            W1, b1, W2, b2 = self._weights_on(dev)
             _ops.neuralgrok_fused_step(s["params"], s["grads"], s["exp_avg"], s["exp_avg_sq"], s["steps"], W1, b1, W2, b2,
                                        group["alpha"], group["beta"], self.amplifier.hidden_dim, group["betas"][0],
                                        group["betas"][1], group["lr"], group["weight_decay"], group["eps"], group["grad_clip"])

@@ -21,7 +21,6 @@ class Prodigy(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay))
         self._d_lr: float = 1e-6
 
-    @torch.no_grad()
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
 
@@ -29,6 +28,11 @@ class Prodigy(Optimizer):
             st["param_init"] = p.detach().clone().float()
 
         for group in self.param_groups:
+            d_lr = _ops.prodigy_group_step(group["params"], self.state, self._d_lr, group["betas"][0], group["betas"][1], group["lr"],
+                                           group["weight_decay"], group["eps"])
+            if d_lr is not None:
+                self._d_lr = d_lr
+                continue
             s = gather(self, group, ("exp_avg", "exp_avg_sq", "s"), extra_init=keep_init)
             if not s["params"]:
                 continue

@@ -99,7 +99,6 @@ class SuperGrok15(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
             self._flat_sharpness.append(mk())
         self._state_initialized = True
 
-    @torch.no_grad()
     def step(self, closure=None, train_loss=None, val_loss=None, train_acc=None):
         loss = None
         if closure is not None:
@@ -110,24 +109,22 @@ class SuperGrok15(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
         if train_acc is not None:
             self._cached_train_acc = train_acc
         self._maybe_update_alpha(train_loss, val_loss, train_acc)
-        alpha = self._cached_alpha
-        layer_alphas = [max(0.0, min(1.0, alpha * f)) for f in self._flat_layer_alphas]
         group = self.param_groups[0]
-        grads = [p.grad.data if p.grad is not None else torch.Tensor() for p in self._flat_params]
         if self._weights_dirty:
-            self._cached_weights = self.meta_net.get_weights()
+            with torch.no_grad():
+                self._cached_weights = self.meta_net.get_weights()
             self._weights_dirty = False
         W1, b1, W2, b2, rescale = self._cached_weights
-        # sharpness is kept in fp32; hand the kernel the gradient's element type
-        sharp = [s if (g.numel() == 0 or s.dtype == g.dtype) else s.to(g.dtype)
-                 for s, g in zip(self._flat_sharpness, grads)]
         if self.gelu_mode is not None:        # this optimizer's own choice of the meta-net's GELU form, set right before its call
             _ops.supergrok15_set_gelu_mode(self.gelu_mode)
-        _ops.supergrok15_fused_step(
-            self._flat_param_data, grads, self._flat_exp_avgs, self._flat_exp_avg_sqs, self._flat_mus, sharp,
-            self._flat_steps, layer_alphas, self._flat_layer_beta1s, W1, b1, W2, b2, rescale, self.meta_hidden_dim,
-            group["betas"][1], group["lr"], self._get_effective_wd(group["weight_decay"]), group["eps"],
-            self.lamb, self._get_ramp_factor(), self._get_gate_signal(), self.gradient_clipping)
+        # alpha per layer, the gradients and the fp32 sharpness (rounded to the gradient's type by the kernel) are taken from
+        # the lists natively; the work is that of _ops.supergrok15_fused_step
+        if not _ops.supergrok15_flat_step(
+                self._flat_params, self._flat_param_data, self._flat_exp_avgs, self._flat_exp_avg_sqs, self._flat_mus,
+                self._flat_sharpness, self._flat_steps, self._cached_alpha, self._flat_layer_alphas, self._flat_layer_beta1s,
+                W1, b1, W2, b2, rescale, self.meta_hidden_dim, group["betas"][1], group["lr"], self._get_effective_wd(group["weight_decay"]), group["eps"], self.lamb,
+                self._get_ramp_factor(), self._get_gate_signal(), self.gradient_clipping):
+            raise RuntimeError("SuperGrok15: every per-parameter list needs one entry per parameter")
         return loss
 
     # sam_step comes from MetaTraining (supergrok15.py:307-352 of the reference)
