@@ -71,10 +71,15 @@ SG_HD int sg2_contraction_steps(float dt0, float nhA_e, float nhA_o) {
     if (m < 1e-30f) return 1;
     return (int)(69.3147202f / -sg_log(m)) + 1;       /* 100 ln 2 / -ln m */
 }
-/* The largest of those counts over all pairs of both directions (0 if one of them is 0), with an eighth and eight
- * steps of margin, rounded up to whole blocks of eight steps. */
+/* What a summary walk counts as forgotten: every entry of the running 2x2 part below 2^-64.  The state that enters
+ * there is multiplied by less than that, 2^-40 of an fp32 rounding step of a state of the same size; it could only show
+ * where the drive falls by more than 2^38 within the walk. */
+#define SG2_FORGOTTEN 5.421010862427522e-20f
+/* The steps the slowest pair of both directions needs to get there (largest: the largest count to 2^-100, 0 if one of
+ * them is 0), with an eighth and eight steps of margin, rounded up to whole blocks of eight steps. */
 SG_HD int sg2_first_block_steps(int largest, int any_zero) {
     if (any_zero || largest <= 0) return 0;
+    largest = (largest * 16 + 24) / 25;
     return (largest + largest / 8 + 8 + 7) & ~7;
 }
 

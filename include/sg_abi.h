@@ -65,7 +65,7 @@ typedef struct Sg2Weights {
 typedef struct Sg2Tensor {
     void* param;              /* [numel]            updated in place        */
     const void* grad;         /* [numel]            read only               */
-    const void* sharpness;    /* [numel]            read only               */
+    const void* sharpness;    /* [numel]            read only (fp32 with SG_SHARP_F32 in dtype) */
     float* exp_avg;           /* [numel]            updated                 */
     float* exp_avg_sq;        /* [numel]            updated                 */
     float* mu;                /* [numel]            updated                 */
@@ -106,7 +106,7 @@ int sg2_chunk_len_for(int num_tensors, const int64_t* numels);
  * negative value restores the default, SG2_DEFAULT_SCAN_WINDOW).  The recurrence contracts, so a
  * chunk summary is built backwards in blocks of `window` steps and the walk
  * stops as soon as every entry of the 2x2 part of the running summary is below
- * 2^-100 (the chunk summary is then (0, b)); a chunk that never contracts is
+ * 2^-64 (the chunk summary is then (0, b)); a chunk that never contracts is
  * covered completely.  Before that walk one block whose length follows from
  * the weights (the steps the slowest RoPE pair needs to contract at the step
  * size of a zero input) is tried with a bound in place of the 2x2 part; the
@@ -140,6 +140,11 @@ typedef struct Sg2Options {
     int32_t scan_window;
 } Sg2Options;
 size_t sg2_workspace_bytes_opt(const SgDims* dims, int num_tensors, const int64_t* numels, const Sg2Options* options);
+/* sg2_batched_step on gradients clipped per tensor as sg2_clip_grads clips them (g * max_norm/(|g| + 1e-12) where
+ * |g| > max_norm): the factor is applied as the gradients are read, no clipped copies are made.  max_norm > 0. */
+int sg2_clipped_step(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors,
+                     const Sg2Scalars* scalars, float max_norm, int32_t* expert_counts, void* workspace,
+                     size_t workspace_bytes, void* stream);
 int sg2_batched_step_opt(const SgDims* dims, const Sg2Weights* weights, int num_tensors,
                          const Sg2Tensor* tensors, const Sg2Scalars* scalars, int32_t* expert_counts,
                          void* workspace, size_t workspace_bytes, const Sg2Debug* debug,

@@ -52,18 +52,18 @@
  * backwards in blocks of `window` steps.  The last block is summarised from
  * the identity; the recurrence contracts (|A_bar| < 1), so the 2x2 part M of
  * that summary is usually vanishingly small: if every |entry| of M in all
- * (j,p) is below 2^-100 the chunk summary is taken as (0, b) -- whatever state
- * entered the block is multiplied by less than 2^-100, far below fp32
+ * (j,p) is below 2^-64 the chunk summary is taken as (0, b) -- whatever state
+ * entered the block is multiplied by less than 2^-64, far below fp32
  * resolution.  Otherwise the block before it is summarised from the identity
  * and the summary so far is applied on top (M, b) <- (M_late M_early,
  * M_late b_early + b_late), and the test is repeated, until it passes or the
  * chunk start is reached (then the summary is the exact one, re-associated by
  * blocks).  window <= 0 accumulates the whole chunk in one block.
  * Before that walk a windowed summary makes one cheaper attempt: a single block whose length comes from the weights
- * alone (the steps the slowest RoPE pair needs to contract below 2^-100 at the step size of a zero input, plus a
+ * alone (the steps the slowest RoPE pair needs to contract below 2^-64 at the step size of a zero input, plus a
  * margin: sg2_first_block_steps in include/sg2_compose.h), walked with the state part only, while the 2x2 part is
  * bounded by the running product of max(|A_bar_e|, |A_bar_o|) (rotations preserve length).  If the bound is below
- * 2^-100 in every (j,p) the summary is (0, b) with that block's b; otherwise the walk above starts from scratch.
+ * 2^-64 in every (j,p) the summary is (0, b) with that block's b; otherwise the walk above starts from scratch.
  * Step size and gate of a 64-step tile (fp32 policy, as the kernels): when every timestep of the tile has
  * cmax_g |g| + cmax_s |s| < 2^-5 (cmax: the largest |c_g|, |c_s| of the composed dt and gate rows of the
  * direction), softplus(c_0 + d) and silu(c_0' + d') are evaluated as their cubic Taylor polynomials in d around
@@ -500,7 +500,7 @@ void scan_dir(const Dims& d, const DirW<O>& w, const typename O::R* x, const flo
         /* first attempt (windowed summaries only): ONE block of first_block steps -- what the slowest pair needs to
          * contract at the step size of a zero input, sg2_first_block_steps -- walked with the state part alone and,
          * in place of the 2x2 part, the running product of max(|A_bar_e|, |A_bar_o|), which bounds its norm.  Below
-         * 2^-100 in every (j,p): the summary is (0, b).  Otherwise the general walk below starts from scratch. */
+         * 2^-64 in every (j,p): the summary is (0, b).  Otherwise the general walk below starts from scratch. */
         bool lite_done = false;
         if (blk_first > u0 && first_block > 0 && u1 - first_block > u0) {
             std::vector<R> bound(di * hp, (R)1);
@@ -533,7 +533,7 @@ void scan_dir(const Dims& d, const DirW<O>& w, const typename O::R* x, const flo
             }
             lite_done = true;
             for (int i = 0; i < di * hp; i++)
-                if (!(bound[i] < (R)7.888609052210118e-31)) { lite_done = false; break; }
+                if (!(bound[i] < (R)SG2_FORGOTTEN)) { lite_done = false; break; }
         }
         for (; !lite_done;) {
             for (int i = 0; i < di * hp; i++) {
@@ -576,11 +576,11 @@ void scan_dir(const Dims& d, const DirW<O>& w, const typename O::R* x, const flo
                     m[5] = O::fma(L[1], e4, O::fma(L[3], e5, L[5]));
                 }
             if (blk_first == u0) break;
-            bool contracted = true;      /* every |M entry| < 2^-100 (a NaN counts as not contracted) */
+            bool contracted = true;      /* every |M entry| < 2^-64 (a NaN counts as not contracted) */
             for (int i = 0; i < di * hp && contracted; i++)
                 for (int k = 0; k < 4; k++) {
                     const R a = sm[i * 6 + k] < 0 ? -sm[i * 6 + k] : sm[i * 6 + k];
-                    if (!(a < (R)7.888609052210118e-31)) { contracted = false; break; }
+                    if (!(a < (R)SG2_FORGOTTEN)) { contracted = false; break; }
                 }
             if (contracted) {
                 for (int i = 0; i < di * hp; i++)

@@ -41,4 +41,7 @@ inline void check_status(int rc, const char* fn) { TORCH_CHECK(rc == 0, fn, ": "
 
 extern int g_sg15_gelu_mode;   // 0 exact erf GELU, 1 sigmoid approximation
 
+// the 33 meta-net weight tensors of the v2 step: fp32, on the GPU, of the sizes that the dimensions ask for
+void check_sg2_weights(const char* fn, const torch::Tensor* const (&w)[SG2_NUM_WEIGHTS], const SgDims& d, Sg2Weights* W);
+
 void bind_group_steps(pybind11::module_& m);      // ops_group.cpp

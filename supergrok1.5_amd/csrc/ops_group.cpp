@@ -415,6 +415,136 @@ bool supergrok11_flat_step(py::handle params, py::handle data, py::handle eas, p
     return true;
 }
 
+// ---- SuperGrok v2 ------------------------------------------------------------------------------
+// The clip pre-pass and the batched step for every parameter with a gradient, step counters counted up in place.
+// dims: d_model, d_state, d_inner, gru_hidden, num_heads, pk_dim, expert_hidden, num_experts.  Returns how many
+// parameters took part, or -1 (nothing changed) where the general path has to be taken: a Mamba state that is not there
+// yet, a gradient that is not contiguous, parameters elsewhere than on the GPU.
+int64_t supergrok2_flat_step(py::list params, py::list eas, py::list easqs, py::list mus, py::list sharps, py::list grus, py::list mfwd,
+                             py::list mbwd, py::list steps, double alpha, py::list alpha_factors, py::list beta1s, double lamb_eff,
+                             py::list weights, float rescale, double beta2, float lr, float wd_eff, float eps, std::vector<int> dims8,
+                             const torch::Tensor& expert_counts, double max_norm) {
+    const char* fn = "supergrok2_mamba_peer_batched_step";
+    const Py_ssize_t P = PyList_GET_SIZE(params.ptr());
+    for (PyObject* l : {eas.ptr(), easqs.ptr(), mus.ptr(), sharps.ptr(), grus.ptr(), mfwd.ptr(), mbwd.ptr(), steps.ptr(), alpha_factors.ptr(),
+                        beta1s.ptr()})
+        if (PyList_GET_SIZE(l) != P) return -1;
+    if (!(max_norm > 0.0) || dims8.size() != 8 || PyList_GET_SIZE(weights.ptr()) != SG2_NUM_WEIGHTS) return -1;
+    const SgDims dims = {dims8[0], dims8[1], dims8[2], dims8[3], dims8[4], dims8[5], dims8[6], dims8[7]};
+    auto item = [](const py::list& l, Py_ssize_t i) { return as_tensor(PyList_GET_ITEM(l.ptr(), i)); };
+    std::vector<Sg2Tensor> ts;
+    std::vector<int64_t> numels;
+    std::vector<Py_ssize_t> active;
+    ts.reserve(P);
+    numels.reserve(P);
+    active.reserve(P);
+    const at::Tensor* first = nullptr;
+    double bc2 = 1.0;
+    long long bc2_at = -1;
+    for (Py_ssize_t i = 0; i < P; i++) {
+        const at::Tensor* p = item(params, i);
+        if (!p) return -1;
+        const at::Tensor& g = p->grad();
+        if (!g.defined()) continue;
+        const at::Tensor *ea = item(eas, i), *easq = item(easqs, i), *mu = item(mus, i), *s = item(sharps, i), *gru = item(grus, i),
+                         *mf = item(mfwd, i), *mb = item(mbwd, i);
+        PyObject* step = PyList_GET_ITEM(steps.ptr(), i);
+        if (!ea || !easq || !mu || !s || !gru || !mf || !mb || !PyLong_CheckExact(step) || !p->is_cuda() || !g.is_cuda() ||
+            !g.is_contiguous())
+            return -1;
+        active.push_back(i);
+        const int64_t n = g.numel();
+        if (n == 0) continue;
+        const long long t = PyLong_AsLongLong(step) + 1;
+        const double b1 = PyFloat_AsDouble(PyList_GET_ITEM(beta1s.ptr(), i));
+        const double a = std::max(0.0, std::min(1.0, alpha * PyFloat_AsDouble(PyList_GET_ITEM(alpha_factors.ptr(), i))));
+        if (PyErr_Occurred()) throw py::error_already_set();
+        if (t != bc2_at) {
+            bc2 = 1.0 - std::pow(beta2, (double)t);
+            bc2_at = t;
+        }
+        check_pair(*p, g, fn);
+        Sg2Tensor q = {};
+        q.param = p->data_ptr();
+        q.grad = g.data_ptr();
+        q.sharpness = s->data_ptr();
+        q.dtype = sharp_code(*s, g, fn);
+        q.numel = n;
+        q.exp_avg = f32_ptr(*ea, n, fn, "exp_avg");
+        q.exp_avg_sq = f32_ptr(*easq, n, fn, "exp_avg_sq");
+        q.mu = f32_ptr(*mu, n, fn, "mu");
+        q.gru_state = f32_ptr(*gru, n * dims.gru_hidden, fn, "gru_state");
+        q.mamba_fwd_state = f32_ptr(*mf, (int64_t)dims.d_inner * dims.d_state, fn, "mamba_fwd_state");
+        q.mamba_bwd_state = f32_ptr(*mb, (int64_t)dims.d_inner * dims.d_state, fn, "mamba_bwd_state");
+        q.alpha_mu = (float)a;
+        q.lamb_eff = (float)lamb_eff;
+        q.beta1 = (float)b1;
+        q.bc1 = (float)(1.0 - std::pow(b1, (double)t));
+        q.bc2 = (float)bc2;
+        ts.push_back(q);
+        numels.push_back(n);
+        if (!first) first = p;
+    }
+    if (active.empty()) return 0;
+    if (!first) return -1;
+    const torch::Tensor* w[SG2_NUM_WEIGHTS];
+    for (int k = 0; k < SG2_NUM_WEIGHTS; k++) {
+        w[k] = item(weights, k);
+        TORCH_CHECK(w[k], fn, ": meta-net weight ", k, " is no tensor");
+    }
+    Sg2Weights W;
+    check_sg2_weights(fn, w, dims, &W);
+    check_gpu(expert_counts, fn, "expert_counts");
+    TORCH_CHECK(expert_counts.scalar_type() == torch::kInt32 && expert_counts.numel() == dims.num_experts, fn,
+                ": expert_counts must be int32[num_experts]");
+    const size_t bytes = sg2_workspace_bytes(&dims, (int)ts.size(), numels.data());
+    TORCH_CHECK(bytes > 0, fn, ": ", sg_last_error());
+    auto ws = make_workspace(bytes, *first);
+    const Sg2Scalars sc = {rescale, (float)beta2, lr, wd_eff, eps};
+    check_status(sg2_clipped_step(&dims, &W, (int)ts.size(), ts.data(), &sc, (float)max_norm, expert_counts.data_ptr<int32_t>(), ws.data_ptr(),
+                                  (size_t)ws.numel(), current_stream(*first)), fn);
+    for (Py_ssize_t i : active) {
+        PyObject* next = PyLong_FromLongLong(PyLong_AsLongLong(PyList_GET_ITEM(steps.ptr(), i)) + 1);
+        PyList_SetItem(steps.ptr(), i, next);
+    }
+    return (int64_t)active.size();
+}
+
+// The random draws of an expert recycling event, in the order of the reference's loop
+// (grokking_optimizers/mamba3_peer_metanet.py:453-488): per dead expert one N(0,1) draw for each of the four expert
+// tensors into its row of `noise`, then a redraw of its key A row if every expert of that row is dead, then of its key B
+// row.  A row is redrawn once per dead expert that shares it and only the last draw stays: the ones before are not
+// drawn, the generator's offset moves past them (after one of them has shown by how much).
+void recycle_draws(const std::vector<torch::Tensor>& noise, const std::vector<torch::Tensor>& keys_a, const std::vector<torch::Tensor>& keys_b,
+                   const std::vector<int64_t>& dead, const std::vector<bool>& row_dead, const std::vector<bool>& col_dead, int64_t pk,
+                   int64_t experts) {
+    at::NoGradGuard guard;
+    std::vector<std::vector<at::Tensor>> rows;
+    for (const torch::Tensor& t : noise) rows.push_back(t.unbind(0));
+    const bool skip = noise[0].is_cuda();
+    at::Generator gen = at::globalContext().defaultGenerator(noise[0].device());
+    uint64_t stride = 0;       // generator offset of one key row's draw
+    auto redraw = [&](const std::vector<torch::Tensor>& keys, int64_t row, bool stays) {
+        for (const torch::Tensor& k : keys) {
+            if (skip && !stays && stride > 0) {
+                gen.set_offset(gen.get_offset() + stride);
+                continue;
+            }
+            const uint64_t before = skip ? gen.get_offset() : 0;
+            at::Tensor r = k.select(0, row);
+            if (stays) r.normal_().mul_(0.02);
+            else at::empty_like(r).normal_();
+            if (skip) stride = gen.get_offset() - before;
+        }
+    };
+    for (size_t k = 0; k < dead.size(); k++) {
+        const int64_t i = dead[k], a = i / pk, b = i % pk;
+        for (auto& r : rows) r[k].normal_();
+        if (row_dead[a]) redraw(keys_a, a, i == std::min(experts, (a + 1) * pk) - 1);
+        if (col_dead[b]) redraw(keys_b, b, i + pk >= experts);
+    }
+}
+
 }  // namespace
 
 void bind_group_steps(pybind11::module_& m) {
@@ -427,4 +557,6 @@ void bind_group_steps(pybind11::module_& m) {
     m.def("muon_group_step", &muon_group_step);
     m.def("supergrok15_flat_step", &supergrok15_flat_step);
     m.def("supergrok11_flat_step", &supergrok11_flat_step);
+    m.def("supergrok2_flat_step", &supergrok2_flat_step);
+    m.def("recycle_draws", &recycle_draws);
 }

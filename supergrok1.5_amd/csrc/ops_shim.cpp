@@ -200,6 +200,22 @@ void muon_fused_step(std::vector<torch::Tensor>& params, std::vector<torch::Tens
 }
 
 // ───────────────────────── SuperGrok v2 ─────────────────────────
+void check_sg2_weights(const char* fn, const torch::Tensor* const (&w)[SG2_NUM_WEIGHTS], const SgDims& d, Sg2Weights* W) {
+    const int64_t dm = d.d_model, ds = d.d_state, di = d.d_inner, gh = d.gru_hidden, H = d.num_heads, pk = d.pk_dim, E = d.num_experts,
+                  eh = d.expert_hidden;
+    const int64_t gru_row = 2 + 2 * dm + gh, peer_in = gh + 2 * dm + 2, gmat = gh * gru_row;
+    const int64_t mamba[9] = {2 * di * dm, di * di, di, ds * di, ds * di, di * ds, di, di * (ds / 2), dm * di};
+    int64_t want[SG2_NUM_WEIGHTS] = {2 * dm, dm};
+    for (int k = 0; k < 9; k++) want[2 + k] = want[11 + k] = mamba[k];
+    const int64_t tail[13] = {gmat, gh, gmat, gh, gmat, gh, H * dm * peer_in, H * pk * (dm / 2), H * pk * (dm / 2), E * eh, E * eh, E * eh, E};
+    for (int k = 0; k < 13; k++) want[20 + k] = tail[k];
+    for (int k = 0; k < SG2_NUM_WEIGHTS; k++) {
+        check_f32(*w[k], fn, "meta-net weight");
+        TORCH_CHECK(w[k]->numel() == want[k], fn, ": meta-net weight ", k, " has ", w[k]->numel(), " elements, expected ", want[k]);
+        W->w[k] = w[k]->data_ptr<float>();
+    }
+}
+
 void supergrok2_mamba_peer_batched_step(
     std::vector<torch::Tensor> params, std::vector<torch::Tensor> grads, std::vector<torch::Tensor> sharpness_list,
     std::vector<torch::Tensor> exp_avgs, std::vector<torch::Tensor> exp_avg_sqs, std::vector<torch::Tensor> mus,
@@ -225,29 +241,13 @@ void supergrok2_mamba_peer_batched_step(
                     alpha_mus.size() == P && lamb_effs.size() == P && beta1s.size() == P && bc1s.size() == P && bc2s.size() == P,
                 fn, ": per-parameter lists must all have ", P, " entries");
     SgDims dims = {d_model, d_state, d_inner, gru_hidden, num_heads, pk_dim, expert_hidden, num_experts};
-    const int gru_row = 2 + 2 * d_model + gru_hidden, peer_in = gru_hidden + 2 * d_model + 2;
-    torch::Tensor w[SG2_NUM_WEIGHTS] = {
-        input_proj_W, input_proj_b, mamba_fwd_in_proj, mamba_fwd_dt_W, mamba_fwd_dt_b, mamba_fwd_B_proj, mamba_fwd_C_proj,
-        mamba_fwd_A_log, mamba_fwd_D, mamba_fwd_rope, mamba_fwd_out_proj, mamba_bwd_in_proj, mamba_bwd_dt_W, mamba_bwd_dt_b,
-        mamba_bwd_B_proj, mamba_bwd_C_proj, mamba_bwd_A_log, mamba_bwd_D, mamba_bwd_rope, mamba_bwd_out_proj, gru_Wz, gru_bz,
-        gru_Wr, gru_br, gru_Wh, gru_bh, peer_query_Ws, prod_keys_A, prod_keys_B, expert_W1, expert_b1, expert_W2, expert_b2};
-    const int64_t mamba_numel[9] = {2LL * d_inner * d_model, (int64_t)d_inner * d_inner, d_inner, (int64_t)d_state * d_inner,
-                                    (int64_t)d_state * d_inner, (int64_t)d_inner * d_state, d_inner,
-                                    (int64_t)d_inner * (d_state / 2), (int64_t)d_model * d_inner};
-    const int64_t gmat = (int64_t)gru_hidden * gru_row;
-    int64_t want[SG2_NUM_WEIGHTS] = {2LL * d_model, d_model};
-    for (int k = 0; k < 9; k++) want[2 + k] = want[11 + k] = mamba_numel[k];
-    const int64_t tail[13] = {gmat, gru_hidden, gmat, gru_hidden, gmat, gru_hidden, (int64_t)num_heads * d_model * peer_in,
-                              (int64_t)num_heads * pk_dim * (d_model / 2), (int64_t)num_heads * pk_dim * (d_model / 2),
-                              (int64_t)num_experts * expert_hidden, (int64_t)num_experts * expert_hidden,
-                              (int64_t)num_experts * expert_hidden, num_experts};
-    for (int k = 0; k < 13; k++) want[20 + k] = tail[k];
+    const torch::Tensor* const w[SG2_NUM_WEIGHTS] = {
+        &input_proj_W, &input_proj_b, &mamba_fwd_in_proj, &mamba_fwd_dt_W, &mamba_fwd_dt_b, &mamba_fwd_B_proj, &mamba_fwd_C_proj,
+        &mamba_fwd_A_log, &mamba_fwd_D, &mamba_fwd_rope, &mamba_fwd_out_proj, &mamba_bwd_in_proj, &mamba_bwd_dt_W, &mamba_bwd_dt_b,
+        &mamba_bwd_B_proj, &mamba_bwd_C_proj, &mamba_bwd_A_log, &mamba_bwd_D, &mamba_bwd_rope, &mamba_bwd_out_proj, &gru_Wz, &gru_bz,
+        &gru_Wr, &gru_br, &gru_Wh, &gru_bh, &peer_query_Ws, &prod_keys_A, &prod_keys_B, &expert_W1, &expert_b1, &expert_W2, &expert_b2};
     Sg2Weights W;
-    for (int k = 0; k < SG2_NUM_WEIGHTS; k++) {
-        check_f32(w[k], fn, "meta-net weight");
-        TORCH_CHECK(w[k].numel() == want[k], fn, ": meta-net weight ", k, " has ", w[k].numel(), " elements, expected ", want[k]);
-        W.w[k] = w[k].data_ptr<float>();
-    }
+    check_sg2_weights(fn, w, dims, &W);
     check_gpu(expert_counts, fn, "expert_counts");
     TORCH_CHECK(expert_counts.scalar_type() == torch::kInt32 && expert_counts.numel() == num_experts, fn,
                 ": expert_counts must be int32[num_experts]");

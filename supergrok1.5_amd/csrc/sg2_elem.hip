@@ -37,7 +37,7 @@ constexpr int elem_waves() { return G::DM == 8 ? 4 : 2; }
 template <class G, int EH, bool DBG, bool FWD = false>
 __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(elem_waves<G>(), elem_waves<G>()))) void k_elem(Plan pl, int32_t* __restrict__ expert_counts,
                                                        int32_t* __restrict__ dbg_eidx, float* __restrict__ fwd_smart,
-                                                       float* __restrict__ fwd_gru) {
+                                                       float* __restrict__ fwd_gru, int split) {
     constexpr int DM = G::DM, GRL = G::GRL, PIN = G::PIN, EXP_STRIDE = exp_stride<EH>();
     static_assert(EH % 4 == 0, "expert records are read 16 bytes at a time");
     __shared__ float s_exp[NE * EXP_STRIDE];
@@ -81,12 +81,16 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
     const sg::cfloat_p KA0 = sg::as_const(pl.W.w[W_KEYS_A]);
     const sg::cfloat_p KB0 = sg::as_const(pl.W.w[W_KEYS_B]);
 
-    for (int tile = blockIdx.x; tile < pl.elem_tiles; tile += gridDim.x) {
-        const int ti = sg::upper_seg(sg::as_const(pl.elem_tile_prefix), pl.P, tile);
+    // split: parts that a tile is cut into (1 or ELEM_TILE / ELEM_THREADS, see elem_grid)
+    for (int part = blockIdx.x; part < pl.elem_tiles * split; part += gridDim.x) {
+        const int tile = split == 1 ? part : part / split, len = split == 1 ? ELEM_TILE : ELEM_TILE / split;
+        const sg::Seg seg = sg::find_seg(sg::as_const(pl.elem_tile_prefix), pl.P, tile);
+        const int ti = seg.i;
         const TensorDev& T = pl.tensors[ti];
-        const int start = (tile - pl.elem_tile_prefix[ti]) * ELEM_TILE;
-        const int cnt = min(ELEM_TILE, T.numel - start);
+        const int start = (tile - seg.first) * ELEM_TILE + (part - tile * split) * len;
+        const int cnt = min(len, T.numel - start);
         const int dtype = T.dtype;
+        const float gs = grad_scale(pl, ti);
         const bool has_s = pl.sharp_nonzero[ti] != 0;       // set by the sort's key kernel: some sharpness entry of the tensor is not 0
         const float alpha = T.alpha, lamb = T.lamb, beta1 = T.beta1, bc2 = T.bc2, step_size = T.step_size;
         const float beta2 = pl.beta2, eps = pl.eps, rescale = pl.rescale, decay = pl.decay;
@@ -100,8 +104,8 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
             const int zo = sg::opaque_zero();
             const sg::cfloat_p Wz = Wz0 + zo, bz = bz0 + zo, Wr = Wr0 + zo, br = br0 + zo, Wh = Wh0 + zo, bh = bh0 + zo;
             const sg::cfloat_p KA = KA0 + zo, KB = KB0 + zo;
-            const float g = sg::finite_or_zero(sg::load_elem(T.grad, dtype, i));
-            const float s = has_s ? sg::finite_or_zero(sg::load_elem(T.sharp, dtype, i)) : 0.0f;
+            const float g_raw = sg::load_elem(T.grad, dtype, i);        // clipped below, when the loads behind it are on their way
+            float s = has_s ? sharp_raw(T, i) : 0.0f;
             float cf[DM], cb[DM], hold[GH];
             {
                 const SG_GLOBAL vf4* pf = (const SG_GLOBAL vf4*)(pl.ctx + ((size_t)T.off + i) * DM);
@@ -121,6 +125,8 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
                 mu = sg::gptr(T.mu)[i]; ea = sg::gptr(T.ea)[i]; easq = sg::gptr(T.easq)[i];
                 pv = sg::load_elem(T.param, dtype, i);
             }
+            const float g = clipped(g_raw, gs, dtype);
+            s = sharp_value(T, s);
 
             // ---- GRU: chain order = bias, g, s, fwd ctx, bwd ctx, h
             float zg[GH], rg[GH], hnew[GH];
@@ -198,16 +204,20 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
 #pragma unroll
                 for (int hf = 0; hf < 2; hf++) {
                     const sg::cfloat_p keys = (hf ? KB : KA) + hh * PK * (DM / 2);
-                    int bi = 0;
-                    float bs = -1e30f;
+                    // the first of the largest scores: the maximum, then the lowest index that has it.  (A running comparison
+                    // takes two selects per key, each waiting two clocks for the comparison before it.)
+                    float dot[PK], bs = -1e30f;
 #pragma unroll
                     for (int q = 0; q < PK; q++) {
-                        float dot = 0.0f;
+                        dot[q] = 0.0f;
 #pragma unroll
-                        for (int dd = 0; dd < DM / 2; dd++) dot = sg_fma(query[hf * (DM / 2) + dd], keys[q * (DM / 2) + dd], dot);
-                        if (dot > bs) { bs = dot; bi = q; }
+                        for (int dd = 0; dd < DM / 2; dd++) dot[q] = sg_fma(query[hf * (DM / 2) + dd], keys[q * (DM / 2) + dd], dot[q]);
+                        bs = __builtin_fmaxf(bs, dot[q]);
                     }
-                    best[hf] = bi;
+                    int bi = 0;
+#pragma unroll
+                    for (int q = PK - 1; q > 0; q--) bi = dot[q] == bs ? q : bi;
+                    best[hf] = dot[0] == bs ? 0 : bi;
                 }
                 int e = best[0] * PK + best[1];
                 if (e >= NE) e = NE - 1;
@@ -294,13 +304,14 @@ __global__ __launch_bounds__(ELEM_THREADS) void k_elem_any(Plan pl, int ctx_stri
         const int start = (tile - pl.elem_tile_prefix[ti]) * ELEM_TILE;
         const int cnt = min(ELEM_TILE, T.numel - start);
         const int dtype = T.dtype;
+        const float gs = grad_scale(pl, ti);
         const bool has_s = pl.sharp_nonzero[ti] != 0;
         const float alpha = T.alpha, lamb = T.lamb, beta1 = T.beta1, bc2 = T.bc2, step_size = T.step_size;
         const float beta2 = pl.beta2, eps = pl.eps, rescale = pl.rescale, decay = pl.decay;
         for (int k0 = (int)threadIdx.x; k0 < cnt; k0 += ELEM_THREADS) {
             const int i = start + k0;
-            const float g = sg::finite_or_zero(sg::load_elem(T.grad, dtype, i));
-            const float s = has_s ? sg::finite_or_zero(sg::load_elem(T.sharp, dtype, i)) : 0.0f;
+            const float g = grad_of(T, gs, i);
+            const float s = has_s ? sharp_of(T, i) : 0.0f;
             float cf[MAX_DM], cb[MAX_DM], hold[MAX_GH];
             {
                 const SG_GLOBAL float* pf = sg::gptr(pl.ctx) + ((size_t)T.off + i) * ctx_stride;
@@ -454,11 +465,25 @@ __global__ __launch_bounds__(ELEM_THREADS) void k_elem_any(Plan pl, int ctx_stri
 
 }  // namespace
 
+// Workgroups of the per-element kernel, and the parts its tiles are cut into.  Large calls: about five workgroups per
+// resident slot (768 at three per CU): measured 1.38 / 1.35 / 1.33 / 1.33 / 1.37 ms with 768 / 2048 / 4096 / 8192 / 16384
+// workgroups on 24 424 tiles (fewer leave the chip unevenly loaded at the end, more pay the LDS fill too often).  Calls of
+// at most 1024 tiles would leave most of the chip idle while some workgroups run four rounds of 256 elements: they take
+// rounds as units, spread evenly over at most 1024 resident workgroups.
+int elem_grid(const Plan& pl, int* split) {
+    *split = 1;
+    if (pl.elem_tiles > 1024 || pl.elem_kind == ELEM_ANY) return pl.elem_tiles < 4096 ? pl.elem_tiles : 4096;
+    *split = ELEM_TILE / ELEM_THREADS;
+    const int parts = pl.elem_tiles * *split, rounds = (parts + 1023) / 1024;
+    return (parts + rounds - 1) / rounds;
+}
+
 int launch_elem_forward(const Plan& pl, int32_t* expert_counts, float* smart_out, float* gru_out, hipStream_t st) {
     if (pl.total == 0) return 0;
-    const int grid = pl.elem_tiles < 4096 ? pl.elem_tiles : 4096;
+    int split;
+    const int grid = elem_grid(pl, &split);
     int32_t* const no_dbg = nullptr;
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(ELEM_THREADS), 0, st, pl, expert_counts, no_dbg, smart_out, gru_out); };
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(ELEM_THREADS), 0, st, pl, expert_counts, no_dbg, smart_out, gru_out, split); };
     if (pl.elem_kind == ELEM_ANY)
         hipLaunchKernelGGL(k_elem_any<false>, dim3(grid), dim3(ELEM_THREADS), 0, st, pl, geo_info(pl.geo).dm, expert_counts, no_dbg, smart_out, gru_out);
     else if (pl.geo == GEO_LARGE) go(k_elem<GeoLarge, 16, false, true>);
@@ -470,11 +495,10 @@ int launch_elem_forward(const Plan& pl, int32_t* expert_counts, float* smart_out
 
 int launch_elem(const Plan& pl, int32_t* expert_counts, int32_t* dbg_expert_idx, hipStream_t st) {
     if (pl.total == 0) return 0;
-    // about five workgroups per resident slot (768 at three per CU): measured 1.38 / 1.35 / 1.33 / 1.33 / 1.37 ms with 768 / 2048 / 4096 /
-    // 8192 / 16384 workgroups on 24 424 tiles (fewer leave the chip unevenly loaded at the end, more pay the LDS fill too often)
-    const int grid = pl.elem_tiles < 4096 ? pl.elem_tiles : 4096;
+    int split;
+    const int grid = elem_grid(pl, &split);
     float* const none = nullptr;
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(ELEM_THREADS), 0, st, pl, expert_counts, dbg_expert_idx, none, none); };
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(ELEM_THREADS), 0, st, pl, expert_counts, dbg_expert_idx, none, none, split); };
     if (pl.elem_kind == ELEM_ANY) {
         const int stride = geo_info(pl.geo).dm;
         if (dbg_expert_idx) hipLaunchKernelGGL(k_elem_any<true>, dim3(grid), dim3(ELEM_THREADS), 0, st, pl, stride, expert_counts, dbg_expert_idx, none, none);

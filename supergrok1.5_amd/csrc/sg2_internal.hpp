@@ -57,10 +57,9 @@ constexpr int GRL = GeoDefault::GRL;
 constexpr int PIN = GeoDefault::PIN;
 
 constexpr int ELEM_TILE = 1024;        // elements per tile of the elementwise kernels
-#ifndef SG2_SORT_TILE
-#define SG2_SORT_TILE 8192
-#endif
-constexpr int SORT_TILE = SG2_SORT_TILE;   // keys per radix-sort tile (16 per thread)
+constexpr int SORT_TILE = 8192;        // keys per radix-sort tile (16 per thread) ...
+constexpr int SORT_TILE_SMALL = 2048;  // ... and where every tensor is small (4 per thread): see sort_tile_for
+constexpr int SELF_SCAN_TILES = 32;    // tiles of a segment up to which a scatter block adds up the digit counts of its segment itself
 constexpr int SCAN_TT = 64;            // timesteps projected per LDS tile
 constexpr int SCAN_THREADS = GeoDefault::THREADS;
 constexpr int SCAN_BLOCK_ITEMS = 2048; // entries per block of the spine scan
@@ -91,7 +90,8 @@ struct TensorDev {
     int dtype;
     int nchunks;    // scan chunks of this tensor
     float alpha, lamb, beta1, bc2, step_size;
-    int pad_[5];
+    int sharp32;    // sharpness is fp32 whatever dtype says, rounded to dtype when read
+    int pad_[4];
 };
 static_assert(sizeof(TensorDev) == 128, "TensorDev layout");
 
@@ -102,9 +102,16 @@ struct Plan {
     const int* sort_tile_prefix;   // [P+1] tiles of SORT_TILE keys
     const int* chunk_prefix;       // [P+1] scan chunks
     const int* wchunk_prefix;      // [P+1] scan chunks that need a summary (all but the last of a tensor)
+    const int* norm_tile_prefix;   // [P+1] tiles of norm_tile elements (clipping calls)
     int P;
     int total;                     // sum of numel
-    int elem_tiles, sort_tiles, chunks, wchunks;
+    int elem_tiles, sort_tiles, chunks, wchunks, norm_tiles;
+    int sort_tile;                 // SORT_TILE or SORT_TILE_SMALL
+    int sort_widest;               // sort tiles of the largest tensor
+    int norm_tile;
+    double* norm_partials;         // [norm_tiles] sums of squares
+    float* gscale;                 // [P] factor of each tensor's gradients in a clipping call (written by the sort's first kernel); NULL otherwise
+    float max_norm;
     int geo;                       // GEO_*: which instantiation of the scan / elementwise kernels runs
     int elem_kind;                 // ELEM_*: which per-element kernel runs
     int st_di, st_ds;              // the caller's carried Mamba states are [st_di][st_ds] (the true d_inner, d_state;
@@ -137,6 +144,21 @@ struct Plan {
 // records a profiling event (no-op unless profiling is enabled)
 void prof_mark(int idx, hipStream_t st);
 
+// Gradient of an element as every kernel of the step sees it: clipped (gs: the tensor's factor; the product is a value of
+// the gradient's type, as the tensor the reference makes would hold it), non-finite entries zero.
+__device__ __forceinline__ float grad_scale(const Plan& pl, int ti) { return pl.gscale ? sg::as_const(pl.gscale)[ti] : 1.0f; }
+__device__ __forceinline__ float clipped(float g, float gs, int dtype) {
+    g = g * gs;              // (no branch for the usual factor 1: it changes no bit)
+    if (dtype != SG_F32 && gs != 1.0f) g = sg::round_to(dtype, g);
+    return sg::finite_or_zero(g);
+}
+__device__ __forceinline__ float grad_of(const TensorDev& T, float gs, int64_t i) { return clipped(sg::load_elem(T.grad, T.dtype, i), gs, T.dtype); }
+// sharpness of an element: the load, and the value made of it
+__device__ __forceinline__ float sharp_raw(const TensorDev& T, int64_t i) { return sg::load_elem(T.sharp, T.sharp32 ? (int)SG_F32 : T.dtype, i); }
+__device__ __forceinline__ float sharp_value(const TensorDev& T, float v) { return sg::finite_or_zero(T.sharp32 ? sg::round_to(T.dtype, v) : v); }
+__device__ __forceinline__ float sharp_of(const TensorDev& T, int64_t i) { return sharp_value(T, sharp_raw(T, i)); }
+
+int launch_norm(const Plan& pl, hipStream_t st);
 int launch_sort(const Plan& pl, int32_t* dbg_perm, hipStream_t st);
 int launch_scan(const Plan& pl, hipStream_t st);
 // bilevel path: the forward scan keeps the state entering every HT_STEP-th step of a tensor; index of scan step u

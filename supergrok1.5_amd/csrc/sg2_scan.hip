@@ -16,8 +16,8 @@
 //                  recurrence contracts (|A_bar| < 1), so the chunk is walked
 //                  backwards in blocks of `window` steps and the walk stops as
 //                  soon as every |entry| of the running M, in all lanes, is
-//                  below 2^-100: the state entering that block is multiplied
-//                  by less than 2^-100, and the summary is (0, b).  A first
+//                  below 2^-64: the state entering that block is multiplied
+//                  by less than 2^-64, and the summary is (0, b).  A first
 //                  attempt covers one block sized from the weights with the
 //                  state part only and a norm bound instead of M.
 //   k_chunk_prefix start state of each chunk: summaries applied in order to
@@ -26,7 +26,7 @@
 //                  D skip, out_proj, and the 8-float context written straight
 //                  to the element's original position (the "unsort").  The
 //                  last chunk stores the new carried state.
-//   k_compose      runs first: the input of a timestep is two numbers (g, s)
+//   compose_block  (sg2_compose_block.hpp) ran beside the sort's first kernel: the input of a timestep is two numbers (g, s)
 //                  and every projection of the block is linear in their 8-float
 //                  input projection, so input_proj, in_proj, dt_proj, B_proj and
 //                  C_proj are folded into 5 x d_inner coefficient triples per
@@ -176,79 +176,6 @@ __device__ __forceinline__ float pair_tree_max(float f) {
     f = sg_max(f, dpp_half_mirror(f));
     if (HP == 16) f = sg_max(f, dpp_row_mirror(f));
     return f;
-}
-
-// Composed coefficient triples (see sg2_compose.h), one thread per (direction, group, row).
-template <class G>
-__global__ __launch_bounds__(2 * SG2_COMP_GROUPS * G::ROWS) void k_compose(Plan pl) {
-    const int dir = threadIdx.x / (SG2_COMP_GROUPS * G::ROWS), r = threadIdx.x % (SG2_COMP_GROUPS * G::ROWS);
-    const int group = r / G::ROWS, row = r % G::ROWS;
-    const int b = dir ? W_B_INPROJ : W_F_INPROJ;
-    float out[3];
-    sg2_compose_one(group, row, G::DM, G::DI, pl.W.w[W_IN_W], pl.W.w[W_IN_B], pl.W.w[b], pl.W.w[b + 1], pl.W.w[b + 2], pl.W.w[b + 3],
-                    pl.W.w[b + 4], out);
-    float* dst = pl.comp + (size_t)threadIdx.x * 3;
-    dst[0] = out[0];
-    dst[1] = out[1];
-    dst[2] = out[2];
-    // How many steps the first block of a chunk summary should cover: what the slowest pair of either direction needs
-    // to contract below 2^-100 at the step size a zero input gives (sg2_contraction_steps), plus a margin.
-    __shared__ int s_largest, s_zero, s_bad, s_cmax[2][2], s_cdt[2][2], s_amax[2], s_fmax[2], s_slope[2];
-    if (threadIdx.x == 0) {
-        s_largest = 0; s_zero = 0; s_bad = 0;
-        for (int k = 0; k < 2; k++) { s_cmax[k][0] = s_cmax[k][1] = s_cdt[k][0] = s_cdt[k][1] = s_amax[k] = s_fmax[k] = s_slope[k] = 0; }
-    }
-    __syncthreads();
-    // Taylor polynomials of the step size and of the gate around their zero-input arguments (sg2_compose.h), and the
-    // largest |c_g|, |c_s| of those rows (bit patterns of non-negative floats order like integers)
-    if (group == SG2_COMP_DT || group == SG2_COMP_Z) {
-        float t[4];
-        if (group == SG2_COMP_DT) sg2_softplus_taylor(out[2], t);
-        else sg2_silu_taylor(out[2], t);
-        float* tay = pl.comp + 2 * SG2_COMP_GROUPS * G::ROWS * 3 + ((dir * 2 + (group == SG2_COMP_Z ? 1 : 0)) * G::ROWS + row) * 4;
-        tay[0] = t[0]; tay[1] = t[1]; tay[2] = t[2]; tay[3] = t[3];
-        atomicMax(&s_cmax[dir][0], sg_f2i(sg_abs(out[0])));
-        atomicMax(&s_cmax[dir][1], sg_f2i(sg_abs(out[1])));
-        if (group == SG2_COMP_DT) {
-            atomicMax(&s_cdt[dir][0], sg_f2i(sg_abs(out[0])));
-            atomicMax(&s_cdt[dir][1], sg_f2i(sg_abs(out[1])));
-            atomicMax(&s_slope[dir], sg_f2i(sg2_dt_slope(out[2])));       // positive: its bit pattern orders like the value
-        }
-    }
-    if (group == SG2_COMP_DT) {
-        const float dt0 = sg_softplus(out[2]);
-        const float* alog = pl.W.w[dir ? W_B_ALOG : W_F_ALOG] + row * G::DS;
-        for (int p = 0; p < G::HP; p++) {
-            const float a_e = -0.5f * -sg_exp(alog[2 * p]), a_o = -0.5f * -sg_exp(alog[2 * p + 1]);
-            const int n = sg2_contraction_steps(dt0, a_e, a_o);
-            if (n == 0) atomicOr(&s_zero, 1);
-            atomicMax(&s_largest, n);
-            // for sg2_poly_ok: the largest -A/2 and the largest |rotation frequency| of the direction
-            atomicMax(&s_amax[dir], sg_f2i(sg_max(a_e, a_o)));
-            atomicMax(&s_fmax[dir], sg_f2i(sg_abs(pl.W.w[dir ? W_B_ROPE : W_F_ROPE][row * G::HP + p])));
-        }
-    }
-    for (int i = threadIdx.x; i < pl.P; i += blockDim.x)
-        if (pl.state_bad[i] != 0) s_bad = 1;       // plain store: every writer stores the same value
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        pl.contracted[0] = s_bad == 0 ? 1 : 0;      // until a summary kernel finds a chunk that has not contracted; never while a carried state is not finite
-        pl.contracted[2] = s_bad;
-        pl.contracted[1] = sg2_first_block_steps(s_largest, s_zero);
-        float* cmax = pl.comp + 2 * SG2_COMP_GROUPS * G::ROWS * 3 + 2 * 2 * G::ROWS * 4;
-        cmax[0] = sg_i2f(s_cmax[0][0]); cmax[1] = sg_i2f(s_cmax[0][1]);
-        cmax[2] = sg_i2f(s_cmax[1][0]); cmax[3] = sg_i2f(s_cmax[1][1]);
-        for (int k = 0; k < 2; k++) {
-            const float slope = sg_i2f(s_slope[k]);      // how much of a change of its argument the step size follows at most
-            const float kp = sg2_limit_factor(sg_max(128.0f * sg_i2f(s_amax[k]), 256.0f * sg_i2f(s_fmax[k])), slope);
-            cmax[4 + 2 * k] = kp * sg_i2f(s_cdt[k][0]);
-            cmax[5 + 2 * k] = kp * sg_i2f(s_cdt[k][1]);
-            // ... and for the products of the output pass (sg2_pair_products)
-            const float kq = sg2_limit_factor(sg_fma(416.0f, sg_i2f(s_amax[k]), 184.0f * sg_i2f(s_fmax[k])), slope);
-            cmax[8 + 2 * k] = kq * sg_i2f(s_cdt[k][0]);
-            cmax[9 + 2 * k] = kq * sg_i2f(s_cdt[k][1]);
-        }
-    }
 }
 
 // Projections of one timestep from the element's (g, s).  Each wave of the workgroup produces its
@@ -487,8 +414,9 @@ __global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
     const int dir = (int)blockIdx.x >= per_dir ? 1 : 0;
     const int cidx = (int)blockIdx.x - dir * per_dir;
     const sg::cint_p prefix = sg::as_const(OUT ? pl.chunk_prefix : pl.wchunk_prefix);
-    const int ti = sg::upper_seg(prefix, pl.P, cidx);
-    const int c = cidx - prefix[ti];                       // chunk within the tensor
+    const sg::Seg seg = sg::find_seg(prefix, pl.P, cidx);
+    const int ti = seg.i;
+    const int c = cidx - seg.first;                        // chunk within the tensor
     const TensorDev& T = pl.tensors[ti];
     const int N = T.numel, off = T.off;
     const int u0 = c * pl.chunk_len;                       // first scan step of the chunk
@@ -546,6 +474,12 @@ __global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
             const float* sm = pl.summaries + (size_t)(dir * pl.wchunks + pl.wchunk_prefix[ti] + c - 1) * 6 * SCAN_THREADS;
             S.he = sm[4 * SCAN_THREADS + tid];
             S.ho = sm[5 * SCAN_THREADS + tid];
+        } else if (T.nchunks == 1) {       // nothing before it: the carried state itself (no other workgroup writes it)
+            const float* st = dir ? T.mbwd : T.mfwd;
+            if (j < pl.st_di && 2 * p < pl.st_ds) {
+                S.he = st[j * pl.st_ds + 2 * p];
+                S.ho = st[j * pl.st_ds + 2 * p + 1];
+            }
         } else {
             const float* hs = pl.hstart + ((size_t)(dir * pl.chunks + cidx) * 2) * SCAN_THREADS;
             S.he = hs[tid];
@@ -555,12 +489,12 @@ __global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
 
     // Summary pass: the chunk is walked backwards in blocks of `window` steps.  Each block is summarised from the
     // identity and the summary of everything after it (`late`) is applied on top; as soon as the 2x2 part of the
-    // running summary has contracted below 2^-100 the steps before the block cannot matter and the walk stops.
+    // running summary has contracted below 2^-64 the steps before the block cannot matter and the walk stops.
     int blk_end = u1;
     int blk_first = u0;
     if (!OUT && pl.window > 0 && pl.window < pl.chunk_len) blk_first = max(u0, u1 - pl.window);
-    // First attempt: ONE block of as many steps as k_compose expects the slowest pair to need, walked with the state
-    // part only (LITE) and a bound on the 2x2 part in its place.  If the bound is below 2^-100 in every lane the summary
+    // First attempt: ONE block of as many steps as compose_block expects the slowest pair to need, walked with the state
+    // part only (LITE) and a bound on the 2x2 part in its place.  If the bound is below 2^-64 in every lane the summary
     // is (0, b) as below; if not, the walk starts over in its general form.
     bool lite = false;
     if (!OUT && blk_first > u0) {
@@ -757,7 +691,7 @@ __global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
     }
     if (OUT) break;
     if (lite) {          // c0e holds the bound (a NaN counts as "not contracted")
-        if (!__syncthreads_or(!(S.c0e < 7.888609052210118e-31f))) {
+        if (!__syncthreads_or(!(S.c0e < SG2_FORGOTTEN))) {
             S.c0e = S.c0o = S.c1e = S.c1o = 0.0f;
             fully_contracted = true;
             break;
@@ -779,7 +713,7 @@ __global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
     if (blk_first == u0) break;       // the whole chunk is covered
     {   // has the running summary contracted?  (a NaN counts as "no")
         const float mx = sg_max(sg_max(sg_abs(S.c0e), sg_abs(S.c0o)), sg_max(sg_abs(S.c1e), sg_abs(S.c1o)));
-        if (!__syncthreads_or(!(mx < 7.888609052210118e-31f))) {
+        if (!__syncthreads_or(!(mx < SG2_FORGOTTEN))) {
             S.c0e = S.c0o = S.c1e = S.c1o = 0.0f;
             fully_contracted = true;
             break;
@@ -1027,8 +961,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const int dir = (int)blockIdx.x >= per_dir ? 1 : 0;
     const int cidx = (int)blockIdx.x - dir * per_dir;
     const sg::cint_p prefix = sg::as_const(pl.chunk_prefix);
-    const int ti = sg::upper_seg(prefix, pl.P, cidx);
-    const int c = cidx - prefix[ti];
+    const sg::Seg seg = sg::find_seg(prefix, pl.P, cidx);
+    const int ti = seg.i;
+    const int c = cidx - seg.first;
     const TensorDev& T = pl.tensors[ti];
     const int N = T.numel, off = T.off;
     const int u0 = c * pl.chunk_len;
@@ -1083,6 +1018,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             const float* sm = pl.summaries + (size_t)(dir * pl.wchunks + pl.wchunk_prefix[ti] + c - 1) * 6 * LANES;
             S[h].he = sm[4 * LANES + lane];
             S[h].ho = sm[5 * LANES + lane];
+        } else if (T.nchunks == 1) {       // nothing before it: the carried state itself (no other workgroup writes it)
+            const float* st = dir ? T.mbwd : T.mfwd;
+            const int j = jl + 8 * h;
+            if (j < pl.st_di && 2 * p < pl.st_ds) {
+                S[h].he = st[j * pl.st_ds + 2 * p];
+                S[h].ho = st[j * pl.st_ds + 2 * p + 1];
+            }
         } else {
             const float* hs = pl.hstart + ((size_t)(dir * pl.chunks + cidx) * 2) * LANES;
             S[h].he = hs[lane];
@@ -1377,15 +1319,15 @@ __global__ __launch_bounds__(1024) void k_chunk_prefix(Plan pl) {
 
 template <class G>
 int launch_scan_geo(const Plan& pl, hipStream_t st) {
-    hipLaunchKernelGGL(k_compose<G>, dim3(1), dim3(2 * SG2_COMP_GROUPS * G::ROWS), 0, st, pl);
-    SG_LAUNCH_CHECK("k_compose");
     if (pl.wchunks > 0) {
         hipLaunchKernelGGL((k_scan<G, false, false>), dim3(2 * pl.wchunks), dim3(G::THREADS), 0, st, pl);
         SG_LAUNCH_CHECK("k_scan<summary>");
     }
     prof_mark(2, st);
-    hipLaunchKernelGGL(k_chunk_prefix<G>, dim3(2 * pl.P), dim3(1024), 0, st, pl);
-    SG_LAUNCH_CHECK("k_chunk_prefix");
+    if (pl.wchunks > 0) {      // (tensors of one chunk start from their carried state without it)
+        hipLaunchKernelGGL(k_chunk_prefix<G>, dim3(2 * pl.P), dim3(1024), 0, st, pl);
+        SG_LAUNCH_CHECK("k_chunk_prefix");
+    }
     prof_mark(3, st);
     if constexpr (G::PARTS == 2) {
         if (pl.htile != nullptr) {

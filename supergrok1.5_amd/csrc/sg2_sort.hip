@@ -6,48 +6,58 @@
 // cub::DeviceSegmentedRadixSort::SortPairs call (:1860-1879).  Non-negative
 // floats order like their bit patterns, so the keys are sorted as uint32.
 //
-// Four passes of 8 bits over tiles of 8192 keys (512 lanes x 16).  Per pass:
+// Four passes of 8 bits over tiles of 8192 keys (512 lanes x 16), or of 2048 where every tensor is small.  Per pass:
 //   hist     per-tile digit counts -> spine[segment][digit][tile]  (first pass: counted while the keys are made)
-//   scan     exclusive prefix over the whole spine (2 small kernels; one for small models).  Because
+//   scan     exclusive prefix over the whole spine (2 small kernels).  Because
 //            the spine is laid out segment-major, the global prefix of entry
 //            (seg, d, tile) is exactly: keys in earlier segments + keys of this
 //            segment with a smaller digit + keys with digit d in earlier tiles
 //            = destination of the first such key of this tile.
+//            Calls whose tensors have few tiles each have no scan: a scatter
+//            workgroup adds up the counts of its own segment itself.
 //   scatter  stable rank inside the tile (each wave owns a contiguous quarter
 //            of the tile; match-any ballots give the rank among equal digits)
-//            and write to destination.
+//            and write to destination; the last pass of a small call also takes
+//            the sharpness along into sorted order (large ones: a kernel of its own).
+// Calls whose tensors all fit one tile are sorted by one launch, a workgroup per
+// tensor that keeps its keys in LDS for all four passes.
 #include <type_traits>
 
+#include "sg2_compose_block.hpp"
 #include "sg2_internal.hpp"
 
 namespace sg2 {
 namespace {
 
-#ifndef SG2_SORT_THREADS
-#define SG2_SORT_THREADS 512
-#endif
-constexpr int SORT_THREADS = SG2_SORT_THREADS;
-constexpr int ITEMS = SORT_TILE / SORT_THREADS;      // rounds per wave
+constexpr int SORT_THREADS = 512;
 constexpr int WAVES = SORT_THREADS / 64;
-constexpr int WAVE_ITEMS = SORT_TILE / WAVES;        // contiguous keys per wave
-static_assert(SORT_THREADS >= 256 && SORT_THREADS % 64 == 0 && SORT_TILE % SORT_THREADS == 0, "one thread per digit at least");
+static_assert(SORT_THREADS >= 256 && SORT_THREADS % 64 == 0 && SORT_TILE_SMALL % SORT_THREADS == 0, "one thread per digit at least");
 
 struct TileRef {
     int base;        // index of the tile's first key in the packed arrays
     int cnt;         // keys in the tile
     int spine0;      // index of spine entry (digit 0) for this tile
-    int stride;      // spine stride between digits (= tiles of the segment)
+    int stride;      // spine stride between digits
+    int tiles;       // tiles of the segment
+    int seg;         // the segment
+    int tile;        // tile within the segment
+    int seg_off;     // index of the segment's first key
 };
+// SELF: the spine is laid out [segment][tile][digit], else [segment][digit][tile] (see k_scatter)
+template <bool SELF>
 __device__ __forceinline__ TileRef tile_ref(const Plan& pl, int tile) {
-    const int seg = sg::upper_seg(pl.sort_tile_prefix, pl.P, tile);
-    const int t0 = pl.sort_tile_prefix[seg];
-    const int nt = pl.sort_tile_prefix[seg + 1] - t0;
-    const TensorDev& T = pl.tensors[seg];
+    const sg::Seg seg = sg::find_seg(sg::as_const(pl.sort_tile_prefix), pl.P, tile);
+    const int t0 = seg.first, nt = seg.end - seg.first;
+    const TensorDev& T = pl.tensors[seg.i];
     TileRef r;
-    r.base = T.off + (tile - t0) * SORT_TILE;
-    r.cnt = min(SORT_TILE, T.numel - (tile - t0) * SORT_TILE);
-    r.spine0 = 256 * t0 + (tile - t0);
-    r.stride = nt;
+    r.seg = seg.i;
+    r.base = T.off + (tile - t0) * pl.sort_tile;
+    r.cnt = min(pl.sort_tile, T.numel - (tile - t0) * pl.sort_tile);
+    r.spine0 = SELF ? 256 * tile : 256 * t0 + (tile - t0);
+    r.stride = SELF ? 1 : nt;
+    r.tiles = nt;
+    r.tile = tile - t0;
+    r.seg_off = T.off;
     return r;
 }
 
@@ -57,37 +67,76 @@ __device__ __forceinline__ TileRef tile_ref(const Plan& pl, int tile) {
 // forms them again from the gradients (key_of / payload_of) while it moves them.
 // key = |g| bits; the sign rides in bit 31 of the payload so that the sorted (key, payload) pair gives back g
 // exactly and the scan never has to gather gradients from element order
-__device__ __forceinline__ uint32_t key_of(float g) { return (uint32_t)sg_f2i(sg_abs(sg::finite_or_zero(g))); }
-__device__ __forceinline__ int32_t payload_of(float g, int index) { return index | (sg_f2i(sg::finite_or_zero(g)) & (int32_t)0x80000000); }
+__device__ __forceinline__ uint32_t key_of(float g) { return (uint32_t)sg_f2i(sg_abs(g)); }
+__device__ __forceinline__ int32_t payload_of(float g, int index) { return index | (sg_f2i(g) & (int32_t)0x80000000); }
 
+// Without SAM the sharpness of every element is 0 (the optimizer's initial state): remember per tensor whether anything
+// else was seen, so that the gather into sorted order can be skipped for such tensors.  (plain store, and only while the
+// flag still reads 0: every writer stores the same value; called by the whole workgroup)
+__device__ __forceinline__ void note_sharpness(const Plan& pl, int seg, bool nz) {
+    if (__syncthreads_or(nz) && threadIdx.x == 0) {
+        volatile int* flag = pl.sharp_nonzero + seg;
+        if (*flag == 0) *flag = 1;
+    }
+}
+
+// Factor of the tensor's gradients in a clipping call: the workgroup adds up the tensor's norm tiles (k_norm) itself, in
+// the order of a 256-lane reduction; `keep` stores it for the later kernels.
+__device__ __forceinline__ float clip_factor(const Plan& pl, int ti, bool keep) {
+    if (!pl.gscale) return 1.0f;
+    __shared__ double sm[4];
+    double part = 0.0;
+    if (threadIdx.x < 256)
+        for (int k = pl.norm_tile_prefix[ti] + (int)threadIdx.x; k < pl.norm_tile_prefix[ti + 1]; k += 256) part += pl.norm_partials[k];
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) part += __shfl_down(part, d, 64);
+    if (threadIdx.x < 256 && (threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = part;
+    __syncthreads();
+    // a NaN norm compares false (no clip); an infinite one gives factor 0, and what 0 * inf leaves counts as non-finite
+    const float norm = (float)sqrt((sm[0] + sm[1]) + (sm[2] + sm[3]));
+    const float gs = norm > pl.max_norm ? pl.max_norm / (norm + 1e-12f) : 1.0f;
+    if (keep && threadIdx.x == 0) pl.gscale[ti] = gs;
+    return gs;
+}
+
+// Workgroup 0 derives the scan's coefficients (compose_block); workgroup 1 + t counts tile t.
+template <class G, int TILE, bool SELF>
 __global__ __launch_bounds__(SORT_THREADS) void k_keys(Plan pl) {
+    if (blockIdx.x == 0) {
+        compose_block<G>(pl, SORT_THREADS);
+        return;
+    }
+    constexpr int ITEMS = TILE / SORT_THREADS;
     // lane-selected copies of the counters, as in k_hist: gradients that came from a 16-bit format have one value of digit 0
     constexpr int HCOPY = 8, HSTRIDE = 256 + 8;
     __shared__ uint32_t hc[HCOPY * HSTRIDE];
-    const int seg = sg::upper_seg(pl.sort_tile_prefix, pl.P, (int)blockIdx.x);
-    const TileRef tr = tile_ref(pl, blockIdx.x);
+    const int tile = (int)blockIdx.x - 1;
+    const TileRef tr = tile_ref<SELF>(pl, tile);
+    const int seg = tr.seg;
     const TensorDev& T = pl.tensors[seg];
     const int start = tr.base - T.off;
     for (int k = threadIdx.x; k < HCOPY * HSTRIDE; k += SORT_THREADS) hc[k] = 0;
     uint32_t* const h = hc + (threadIdx.x & (HCOPY - 1)) * HSTRIDE;
-    __syncthreads();
     bool nz = false;
     const float* gp = static_cast<const float*>(T.grad) + start;
     const float* sp = static_cast<const float*>(T.sharp) + start;
-    if (T.dtype == SG_F32 && tr.cnt == SORT_TILE && ((((uintptr_t)gp) | ((uintptr_t)sp)) & 15u) == 0) {
-        // whole fp32 tile on a 16-byte boundary: 16 bytes per lane and load, everything requested before the first use
-        constexpr int VR = SORT_TILE / (4 * SORT_THREADS);
+    // everything is requested before the clip factor is waited for
+    if (T.dtype == SG_F32 && tr.cnt == TILE && ((((uintptr_t)gp) | ((uintptr_t)sp)) & 15u) == 0) {
+        // whole fp32 tile on a 16-byte boundary: 16 bytes per lane and load
+        constexpr int VR = TILE / (4 * SORT_THREADS);
         typedef float vf4 __attribute__((ext_vector_type(4)));
         vf4 g[VR], sh[VR];
 #pragma unroll
         for (int r = 0; r < VR; r++) g[r] = ((const SG_GLOBAL vf4*)gp)[r * SORT_THREADS + (int)threadIdx.x];
 #pragma unroll
         for (int r = 0; r < VR; r++) sh[r] = ((const SG_GLOBAL vf4*)sp)[r * SORT_THREADS + (int)threadIdx.x];
+        const float gs = clip_factor(pl, seg, tr.tile == 0);
+        __syncthreads();
 #pragma unroll
         for (int r = 0; r < VR; r++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                atomicAdd(&h[key_of(g[r][e]) & 255u], 1u);
+                atomicAdd(&h[key_of(clipped(g[r][e], gs, SG_F32)) & 255u], 1u);
                 nz = nz || (sg::finite_or_zero(sh[r][e]) != 0.0f);
             }
     } else {
@@ -100,21 +149,17 @@ __global__ __launch_bounds__(SORT_THREADS) void k_keys(Plan pl) {
 #pragma unroll
         for (int r = 0; r < ITEMS; r++) {
             const int k = r * SORT_THREADS + (int)threadIdx.x;
-            if (k < tr.cnt) nz = nz || (sg::finite_or_zero(sg::load_elem(T.sharp, T.dtype, start + k)) != 0.0f);
+            if (k < tr.cnt) nz = nz || (sharp_of(T, start + k) != 0.0f);
         }
+        const float gs = clip_factor(pl, seg, tr.tile == 0);
+        __syncthreads();
 #pragma unroll
         for (int r = 0; r < ITEMS; r++) {
             const int k = r * SORT_THREADS + (int)threadIdx.x;
-            if (k < tr.cnt) atomicAdd(&h[key_of(g[r]) & 255u], 1u);
+            if (k < tr.cnt) atomicAdd(&h[key_of(clipped(g[r], gs, T.dtype)) & 255u], 1u);
         }
     }
-    // Without SAM the sharpness of every element is 0 (the optimizer's initial state): remember per tensor
-    // whether anything else was seen, so that the gather into sorted order can be skipped for such tensors.
-    // (plain store, and only while the flag still reads 0: every writer stores the same value)
-    if (__syncthreads_or(nz) && threadIdx.x == 0) {
-        volatile int* flag = pl.sharp_nonzero + seg;
-        if (*flag == 0) *flag = 1;
-    }
+    note_sharpness(pl, seg, nz);
     if (threadIdx.x < 256) {
         uint32_t tot = 0;
 #pragma unroll
@@ -124,12 +169,13 @@ __global__ __launch_bounds__(SORT_THREADS) void k_keys(Plan pl) {
 }
 
 // ---- per-tile histogram ---------------------------------------------------------
+template <bool SELF>
 __global__ __launch_bounds__(SORT_THREADS) void k_hist(Plan pl, int src, int shift) {
     // HCOPY copies of the counters, chosen by lane: a pass whose digit takes few values (the exponent byte of the
     // magnitudes) would otherwise queue most of a wave's lanes on a dozen counters.  Copies start 8 banks apart.
     constexpr int HCOPY = 8, HSTRIDE = 256 + 8;
     __shared__ uint32_t hc[HCOPY * HSTRIDE];
-    const TileRef tr = tile_ref(pl, blockIdx.x);
+    const TileRef tr = tile_ref<SELF>(pl, blockIdx.x);
     for (int k = threadIdx.x; k < HCOPY * HSTRIDE; k += SORT_THREADS) hc[k] = 0;
     uint32_t* const h = hc + (threadIdx.x & (HCOPY - 1)) * HSTRIDE;
     __syncthreads();
@@ -218,87 +264,22 @@ __global__ __launch_bounds__(256) void k_spine_down(uint32_t* spine, const uint3
     }
 }
 
-// The whole scan in one workgroup, for spines of at most SPINE_SINGLE_MAX entries (a model of up to a million
-// elements): dependent launches of a few microseconds each cost more than the scan itself there.
-constexpr int SPINE_SINGLE_MAX = 32768;
-__global__ __launch_bounds__(1024) void k_spine_single(uint32_t* spine, int n /* a multiple of 256 */) {
-    __shared__ uint32_t sm[16];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t carry = 0;
-    for (int base = 0; base < n; base += 4096) {
-        const int i = base + (int)threadIdx.x * 4;
-        uint4 v = make_uint4(0u, 0u, 0u, 0u);
-        if (i < n) v = *reinterpret_cast<const uint4*>(spine + i);
-        const uint32_t s = (v.x + v.y) + (v.z + v.w);
-        const uint32_t inc = wave_incl_scan(s);
-        if (lane == 63) sm[w] = inc;
-        __syncthreads();
-        uint32_t before = 0, tot = 0;
-#pragma unroll
-        for (int k = 0; k < 16; k++) {
-            const uint32_t t = sm[k];
-            if (k < w) before += t;
-            tot += t;
-        }
-        __syncthreads();
-        const uint32_t run = carry + before + inc - s;
-        if (i < n) *reinterpret_cast<uint4*>(spine + i) = make_uint4(run, run + v.x, run + v.x + v.y, run + v.x + v.y + v.z);
-        carry += tot;
-    }
-}
-
 // ---- stable scatter ---------------------------------------------------------------
-// FIRST: the pass over digit 0 takes its keys and payloads from the tensor's gradients (element order) instead of
-// the key / payload arrays, which nothing has written yet.
-template <bool FIRST>
-__global__ __launch_bounds__(SORT_THREADS) void k_scatter(Plan pl, int src, int shift) {
-    __shared__ uint32_t cnt[WAVES][256];     // running digit counts of each wave; later: destinations
-    __shared__ uint32_t lbase[256], gdelta[256], wsum[4];
-    __shared__ uint32_t skey[SORT_TILE];
-    __shared__ int32_t sval[SORT_TILE];
-    const TileRef tr = tile_ref(pl, blockIdx.x);
+// What a tile's keys are ranked with in LDS, and where its digits' runs start.
+struct RankLds {
+    uint32_t cnt[WAVES][256];     // running digit counts of each wave; later: positions of each wave's first key of a digit
+    uint32_t lbase[256], wsum[4];
+};
+// Stable rank of every key of the tile among the keys of its digit, wave by wave; ROUNDS rounds of 64 keys per wave, wave
+// w holds keys w * ROUNDS * 64 ... .  Returns in rank[r] the number of equal digits before it in its wave's part and leaves
+// the waves' counts in L.cnt.  live(r): whether this lane's key of round r exists.
+template <int ROUNDS, class Live>
+__device__ __forceinline__ void rank_keys(RankLds& L, const uint32_t (&key)[ROUNDS], uint32_t (&rank)[ROUNDS], int shift, Live live) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int k = threadIdx.x; k < WAVES * 256; k += SORT_THREADS) (&cnt[0][0])[k] = 0;
-    __syncthreads();
-
-    // a whole tile (all but the last tile of a tensor) needs no bounds tests: the body exists in both forms
-    auto body = [&](auto full_c) {
-    constexpr bool FULL = decltype(full_c)::value;
-    const uint32_t* __restrict__ keys = pl.keys[src] + tr.base;
-    const int32_t* __restrict__ vals = pl.vals[src] + tr.base;
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-
-    uint32_t key[ITEMS], rank[ITEMS];
-    int32_t val[ITEMS];
-    if (FIRST) {
-        const TensorDev& T = pl.tensors[sg::upper_seg(pl.sort_tile_prefix, pl.P, (int)blockIdx.x)];
-        const int start = tr.base - T.off, dtype = T.dtype;
-        float g[ITEMS];
 #pragma unroll
-        for (int r = 0; r < ITEMS; r++) {
-            const int i = w * WAVE_ITEMS + r * 64 + lane;
-            g[r] = (FULL || i < tr.cnt) ? sg::load_elem(T.grad, dtype, start + i) : 0.0f;
-        }
-#pragma unroll
-        for (int r = 0; r < ITEMS; r++) {
-            const int i = w * WAVE_ITEMS + r * 64 + lane;
-            const bool ok = FULL || i < tr.cnt;
-            key[r] = ok ? key_of(g[r]) : 0u;
-            val[r] = ok ? payload_of(g[r], start + i) : 0;
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < ITEMS; r++) {
-            const int i = w * WAVE_ITEMS + r * 64 + lane;
-            const bool ok = FULL || i < tr.cnt;
-            key[r] = ok ? keys[i] : 0u;
-            val[r] = ok ? vals[i] : 0;
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < ITEMS; r++) {
-        const int i = w * WAVE_ITEMS + r * 64 + lane;
-        const bool ok = FULL || i < tr.cnt;
+    for (int r = 0; r < ROUNDS; r++) {
+        const bool ok = live(r);
         const uint32_t d = (key[r] >> shift) & 255u;       // 0 for a lane past the end (its key reads as 0)
         // lanes of the wave with the same digit: for every bit, keep the lanes whose bit equals this lane's.  With
         // rep = the lane's bit spread over a word, that is m & ~(ballot ^ rep): one three-input bit operation per
@@ -315,52 +296,135 @@ __global__ __launch_bounds__(SORT_THREADS) void k_scatter(Plan pl, int src, int 
         const uint64_t m = ((uint64_t)mhi << 32) | mlo;
         if (ok) {
             const uint32_t before = __popcll(m & lt);
-            const uint32_t prev = cnt[w][d];
+            const uint32_t prev = L.cnt[w][d];
             rank[r] = prev + before;
-            if (before == 0) cnt[w][d] = prev + (uint32_t)__popcll(m);
+            if (before == 0) L.cnt[w][d] = prev + (uint32_t)__popcll(m);
         }
     }
+}
+// Digit d = threadIdx.x: total of the tile, start of the digit in the tile's digit-sorted order (lbase) and position of
+// each wave's first key of it there (cnt).  Called by the whole workgroup after a barrier; ends without one.
+__device__ __forceinline__ void digit_starts(RankLds& L) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int d = threadIdx.x & 255;       // (threads beyond the 256 digits repeat the first ones' work and store nothing)
+    const bool own = threadIdx.x < 256;
+    uint32_t tot = 0;
+#pragma unroll
+    for (int k = 0; k < WAVES; k++) tot += L.cnt[k][d];
+    const uint32_t inc = wave_incl_scan(tot);     // over the 64 digits of this wave, then across the 4 waves
+    if (lane == 63 && own) L.wsum[w] = inc;
     __syncthreads();
-    // digit d = threadIdx.x: position of each wave's first key of digit d inside the tile's digit-sorted order
-    // (cnt[k][d]), start of digit d in that order (lbase[d]) and its distance to the global destination (gdelta[d])
-    {
-        const int d = threadIdx.x & 255;       // (threads beyond the 256 digits repeat the first ones' work and store nothing)
-        const bool own = threadIdx.x < 256;
-        uint32_t tot = 0;
+    uint32_t before = 0;
 #pragma unroll
-        for (int k = 0; k < WAVES; k++) tot += cnt[k][d];
-        uint32_t inc = tot;     // inclusive scan over the 64 digits of this wave, then across the 4 waves
+    for (int k = 0; k < 4; k++) before += (k < (d >> 6)) ? L.wsum[k] : 0u;
+    if (own) {
+        uint32_t run = before + inc - tot;
+        L.lbase[d] = run;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t up = __shfl_up(inc, o, 64);
-            if (lane >= o) inc += up;
+        for (int k = 0; k < WAVES; k++) {
+            const uint32_t c = L.cnt[k][d];
+            L.cnt[k][d] = run;
+            run += c;
         }
-        if (lane == 63 && own) wsum[w] = inc;
+    }
+}
+
+// FIRST: the pass over digit 0 takes its keys and payloads from the tensor's gradients (element order) instead of
+// the key / payload arrays, which nothing has written yet.  LAST (small calls): the sharpness of an element goes with it.  SELF: the
+// spine holds plain counts: digit d of the tile starts after the segment's keys of smaller digits and those of digit d in
+// earlier tiles, added up here (at most SELF_SCAN_TILES counts per digit, two lanes a digit); a scan kernel between the
+// counting and the scatter of each pass costs a small call 5 us and another gap.
+template <int TILE, bool FIRST, bool LAST, bool SELF>
+__global__ __launch_bounds__(SORT_THREADS) void k_scatter(Plan pl, int src, int shift) {
+    constexpr int ITEMS = TILE / SORT_THREADS;      // rounds per wave
+    constexpr int WAVE_ITEMS = TILE / WAVES;        // contiguous keys per wave
+    __shared__ RankLds L;
+    __shared__ uint32_t gdelta[256], wtot[4];
+    __shared__ uint2 half2[SELF ? 256 : 1];
+    __shared__ uint32_t skey[TILE];
+    __shared__ int32_t sval[TILE];
+    const TileRef tr = tile_ref<SELF>(pl, blockIdx.x);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int k = threadIdx.x; k < WAVES * 256; k += SORT_THREADS) (&L.cnt[0][0])[k] = 0;
+    // this tile's start in every digit's run of the segment, before the keys are looked at (its loads pass under theirs)
+    uint32_t seg_total = 0, seg_before = 0;
+    if (SELF) {
+        // lanes 0-255 take the even tiles of their digit, lanes 256-511 the odd ones: coalesced rows of 256 counts
+        static_assert(SORT_THREADS == 512, "two lanes per digit");
+        const uint32_t* col = pl.spine + (tr.spine0 - 256 * tr.tile) + (threadIdx.x & 255);
+#pragma unroll 4
+        for (int k = threadIdx.x >> 8; k < tr.tiles; k += 2) {
+            const uint32_t c = col[256 * k];
+            seg_total += c;
+            seg_before += k < tr.tile ? c : 0u;
+        }
+        if (threadIdx.x >= 256) { half2[threadIdx.x & 255] = make_uint2(seg_total, seg_before); }
+    }
+    __syncthreads();
+
+    // a whole tile (all but the last tile of a tensor) needs no bounds tests: the body exists in both forms
+    auto body = [&](auto full_c) {
+    constexpr bool FULL = decltype(full_c)::value;
+    const uint32_t* __restrict__ keys = pl.keys[src] + tr.base;
+    const int32_t* __restrict__ vals = pl.vals[src] + tr.base;
+    const int seg = tr.seg;
+
+    uint32_t key[ITEMS], rank[ITEMS];
+    int32_t val[ITEMS];
+    if (FIRST) {
+        const TensorDev& T = pl.tensors[seg];
+        const int start = tr.base - T.off, dtype = T.dtype;
+        const float gs = grad_scale(pl, seg);
+        float g[ITEMS];
+#pragma unroll
+        for (int r = 0; r < ITEMS; r++) {
+            const int i = w * WAVE_ITEMS + r * 64 + lane;
+            g[r] = (FULL || i < tr.cnt) ? sg::load_elem(T.grad, dtype, start + i) : 0.0f;
+        }
+#pragma unroll
+        for (int r = 0; r < ITEMS; r++) {
+            const int i = w * WAVE_ITEMS + r * 64 + lane;
+            const bool ok = FULL || i < tr.cnt;
+            const float v = clipped(g[r], gs, dtype);
+            key[r] = ok ? key_of(v) : 0u;
+            val[r] = ok ? payload_of(v, start + i) : 0;
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < ITEMS; r++) {
+            const int i = w * WAVE_ITEMS + r * 64 + lane;
+            const bool ok = FULL || i < tr.cnt;
+            key[r] = ok ? keys[i] : 0u;
+            val[r] = ok ? vals[i] : 0;
+        }
+    }
+    rank_keys<ITEMS>(L, key, rank, shift, [&](int r) { return FULL || w * WAVE_ITEMS + r * 64 + lane < tr.cnt; });
+    __syncthreads();
+    digit_starts(L);
+    __syncthreads();
+    if (SELF) {
+        // exclusive scan of the segment's totals over the digits (lanes beyond the 256 digits store nothing)
+        const int d = threadIdx.x & 255;
+        const uint2 odd = half2[d];
+        seg_total += odd.x;
+        seg_before += odd.y;
+        const uint32_t inc = wave_incl_scan(seg_total);
+        if (lane == 63 && w < 4) wtot[w] = inc;
         __syncthreads();
-        uint32_t before = 0;
+        uint32_t smaller = 0;
 #pragma unroll
-        for (int k = 0; k < 4; k++) before += (k < (d >> 6)) ? wsum[k] : 0u;
-        const uint32_t lb = before + inc - tot;
-        if (own) {
-            lbase[d] = lb;
-            gdelta[d] = pl.spine[tr.spine0 + d * tr.stride] - lb;     // global destination = gdelta[d] + local position (mod 2^32)
-            uint32_t run = lb;
-#pragma unroll
-            for (int k = 0; k < WAVES; k++) {
-                const uint32_t c = cnt[k][d];
-                cnt[k][d] = run;
-                run += c;
-            }
-        }
+        for (int k = 0; k < 4; k++) smaller += k < (d >> 6) ? wtot[k] : 0u;
+        if (threadIdx.x < 256) gdelta[d] = tr.seg_off + smaller + inc - seg_total + seg_before - L.lbase[d];
+    } else if (threadIdx.x < 256) {
+        gdelta[threadIdx.x] = pl.spine[tr.spine0 + (int)threadIdx.x * tr.stride] - L.lbase[threadIdx.x];     // global destination = gdelta[d] + local position (mod 2^32)
     }
-    __syncthreads();
     // reorder through LDS so that global stores go out in digit-sorted order: consecutive lanes then write
     // consecutive addresses within each digit's run instead of 4-byte pieces all over the tile's 256 runs
 #pragma unroll
     for (int r = 0; r < ITEMS; r++) {
         const int i = w * WAVE_ITEMS + r * 64 + lane;
         if (FULL || i < tr.cnt) {
-            const uint32_t lp = cnt[w][(key[r] >> shift) & 255u] + rank[r];
+            const uint32_t lp = L.cnt[w][(key[r] >> shift) & 255u] + rank[r];
             skey[lp] = key[r];
             sval[lp] = val[r];
         }
@@ -368,64 +432,173 @@ __global__ __launch_bounds__(SORT_THREADS) void k_scatter(Plan pl, int src, int 
     __syncthreads();
     uint32_t* __restrict__ kout = pl.keys[src ^ 1];
     int32_t* __restrict__ vout = pl.vals[src ^ 1];
+    const bool gather = LAST && SELF && pl.sharp_nonzero[seg] != 0;      // all-zero sharpness: no sorted copy is made, every reader tests the same flag
+    const TensorDev& T = pl.tensors[seg];
 #pragma unroll
     for (int r = 0; r < ITEMS; r++) {
         const int lp = r * SORT_THREADS + threadIdx.x;
         if (FULL || lp < tr.cnt) {
             const uint32_t kk = skey[lp];
+            const int32_t v = sval[lp];
             const uint32_t dst = gdelta[(kk >> shift) & 255u] + (uint32_t)lp;
             kout[dst] = kk;
-            vout[dst] = sval[lp];
+            vout[dst] = v;
+            if (LAST && SELF && gather) pl.ssorted[dst] = sharp_of(T, v & 0x7fffffff);
         }
     }
     };
-    if (tr.cnt == SORT_TILE) body(std::true_type{});
+    if (tr.cnt == TILE) body(std::true_type{});
     else body(std::false_type{});
 }
 
-// After the sort: sharpness gathered into sorted order (one random read per element, once, instead of
-// one per scan pass and direction), and optionally the plain permutation for inspection.
-__global__ __launch_bounds__(256) void k_gather_sorted(Plan pl, int32_t* __restrict__ dbg_perm) {
+// ---- every tensor fits one tile: keys, four passes and the sharpness in one launch ----------------------------------
+// Workgroup 0 derives the scan's coefficients; workgroup 1 + i sorts tensor i.  The keys stay in LDS between the passes:
+// the launches of the general sort (12 for 8 tensors of at most 255 elements, 48 us) carry next to no work there.
+template <class G>
+__global__ __launch_bounds__(SORT_THREADS) void k_sort_tile(Plan pl) {
+    if (blockIdx.x == 0) {
+        compose_block<G>(pl, SORT_THREADS);
+        return;
+    }
+    constexpr int ITEMS = SORT_TILE / SORT_THREADS;
+    __shared__ RankLds L;
+    __shared__ uint32_t skey[SORT_TILE];
+    __shared__ int32_t sval[SORT_TILE];
+    const int seg = (int)blockIdx.x - 1, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const TensorDev& T = pl.tensors[seg];
+    const int n = T.numel, dtype = T.dtype;
+    if (n == 0) return;
+    const float gs = clip_factor(pl, seg, true);
+    bool nz = false;
+    for (int i = threadIdx.x; i < n; i += SORT_THREADS) {
+        const float v = clipped(sg::load_elem(T.grad, dtype, i), gs, dtype);
+        skey[i] = key_of(v);
+        sval[i] = payload_of(v, i);
+        nz = nz || (sharp_of(T, i) != 0.0f);
+    }
+    note_sharpness(pl, seg, nz);
+    const bool gather = __syncthreads_or(nz);
+    // rounds per wave, so that the waves' parts cover the tensor: 1, 2, 4, 8 or 16
+    auto passes = [&](auto rounds_c) {
+        constexpr int ROUNDS = decltype(rounds_c)::value;
+        uint32_t key[ROUNDS], rank[ROUNDS];
+        int32_t val[ROUNDS];
+        auto at = [&](int r) { return (w * ROUNDS + r) * 64 + lane; };
+        for (int shift = 0; shift < 32; shift += 8) {
+            for (int k = threadIdx.x; k < WAVES * 256; k += SORT_THREADS) (&L.cnt[0][0])[k] = 0;
+#pragma unroll
+            for (int r = 0; r < ROUNDS; r++) {
+                key[r] = at(r) < n ? skey[at(r)] : 0u;
+                val[r] = at(r) < n ? sval[at(r)] : 0;
+            }
+            __syncthreads();
+            rank_keys<ROUNDS>(L, key, rank, shift, [&](int r) { return at(r) < n; });
+            __syncthreads();
+            digit_starts(L);
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < ROUNDS; r++)
+                if (at(r) < n) {
+                    const uint32_t lp = L.cnt[w][(key[r] >> shift) & 255u] + rank[r];
+                    skey[lp] = key[r];
+                    sval[lp] = val[r];
+                }
+            __syncthreads();
+        }
+    };
+    const int rounds = (n + SORT_THREADS - 1) / SORT_THREADS;
+    if (rounds <= 1) passes(std::integral_constant<int, 1>{});
+    else if (rounds <= 4) passes(std::integral_constant<int, 4>{});
+    else passes(std::integral_constant<int, ITEMS>{});
+    for (int i = threadIdx.x; i < n; i += SORT_THREADS) {
+        const int32_t v = sval[i];
+        pl.keys[0][T.off + i] = skey[i];
+        pl.vals[0][T.off + i] = v;
+        if (gather) pl.ssorted[T.off + i] = sharp_of(T, v & 0x7fffffff);
+    }
+}
+
+// Sharpness into sorted order for large calls (one random read per element, once, instead of one per scan pass and
+// direction).  In the last scatter these reads have two workgroups per CU to hide behind (3.1 M elements: 37 us more
+// there, 17 us here); small calls save the launch instead.
+constexpr int GATHER_PARTS = 4;      // workgroups per sort tile
+__global__ __launch_bounds__(SORT_THREADS) void k_gather_sharpness(Plan pl) {
+    constexpr int ITEMS = SORT_TILE / SORT_THREADS / GATHER_PARTS;
+    const TileRef tr = tile_ref<false>(pl, blockIdx.x / GATHER_PARTS);
+    if (pl.sharp_nonzero[tr.seg] == 0) return;          // nothing to gather: every reader tests the same flag
+    const TensorDev& T = pl.tensors[tr.seg];
+    const int k0 = (blockIdx.x % GATHER_PARTS) * (SORT_TILE / GATHER_PARTS) + (int)threadIdx.x;
+    float s[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const int k = k0 + r * SORT_THREADS;
+        s[r] = k < tr.cnt ? sharp_raw(T, pl.vals[0][tr.base + k] & 0x7fffffff) : 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const int k = k0 + r * SORT_THREADS;
+        if (k < tr.cnt) pl.ssorted[tr.base + k] = sharp_value(T, s[r]);
+    }
+}
+
+// the plain permutation, for inspection
+__global__ __launch_bounds__(256) void k_permutation(Plan pl, int32_t* __restrict__ dbg_perm) {
     const int tile = blockIdx.x;
     const int ti = sg::upper_seg(sg::as_const(pl.elem_tile_prefix), pl.P, tile);
     const TensorDev& T = pl.tensors[ti];
     const int start = (tile - pl.elem_tile_prefix[ti]) * ELEM_TILE;
     const int cnt = min(ELEM_TILE, T.numel - start);
-    const bool gather = pl.sharp_nonzero[ti] != 0;      // all-zero sharpness: nothing to gather, no sorted copy is made
-    if (!gather && !dbg_perm) return;                   // every reader tests the same flag before it touches ssorted
-    for (int k = threadIdx.x; k < cnt; k += 256) {
-        const int t = T.off + start + k;
-        int idx = pl.vals[0][t] & 0x7fffffff;
-        idx = ((unsigned)idx < (unsigned)T.numel) ? idx : 0;       // never index outside the tensor
-        if (gather) pl.ssorted[t] = sg::finite_or_zero(sg::load_elem(T.sharp, T.dtype, idx));
-        if (dbg_perm) dbg_perm[t] = idx;
+    for (int k = threadIdx.x; k < cnt; k += 256) dbg_perm[T.off + start + k] = pl.vals[0][T.off + start + k] & 0x7fffffff;
+}
+
+template <class G, int TILE, bool SELF>
+int launch_passes(const Plan& pl, hipStream_t st) {
+    hipLaunchKernelGGL((k_keys<G, TILE, SELF>), dim3(1 + pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl);
+    SG_LAUNCH_CHECK("k_keys");
+    const int n = 256 * pl.sort_tiles;
+    const int nb = (n + SCAN_BLOCK_ITEMS - 1) / SCAN_BLOCK_ITEMS;
+    for (int pass = 0; pass < 4; pass++) {
+        const int src = pass & 1, shift = 8 * pass;
+        if (pass > 0) hipLaunchKernelGGL(k_hist<SELF>, dim3(pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl, src, shift);     // the first pass's counts come from k_keys
+        if (!SELF) {
+            hipLaunchKernelGGL(k_spine_reduce, dim3(nb), dim3(256), 0, st, pl.spine, pl.blocksums, n);
+            hipLaunchKernelGGL(k_spine_down, dim3(nb), dim3(256), 0, st, pl.spine, pl.blocksums, n);
+        }
+        const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl, src, shift); };
+        if (pass == 0) go(k_scatter<TILE, true, false, SELF>);
+        else if (pass == 3 && SELF) go(k_scatter<TILE, false, SELF, SELF>);
+        else go(k_scatter<TILE, false, false, SELF>);
+        SG_LAUNCH_CHECK("radix pass");
     }
+    if (!SELF) {
+        hipLaunchKernelGGL(k_gather_sharpness, dim3(GATHER_PARTS * pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl);
+        SG_LAUNCH_CHECK("k_gather_sharpness");
+    }
+    return 0;
+}
+
+template <class G>
+int launch_sort_geo(const Plan& pl, hipStream_t st) {
+    if (pl.sort_tile == SORT_TILE_SMALL) return launch_passes<G, SORT_TILE_SMALL, true>(pl, st);
+    if (pl.sort_widest <= 1) {
+        hipLaunchKernelGGL(k_sort_tile<G>, dim3(1 + pl.P), dim3(SORT_THREADS), 0, st, pl);
+        SG_LAUNCH_CHECK("k_sort_tile");
+        return 0;
+    }
+    if (pl.sort_widest <= SELF_SCAN_TILES) return launch_passes<G, SORT_TILE, true>(pl, st);
+    return launch_passes<G, SORT_TILE, false>(pl, st);
 }
 
 }  // namespace
 
 int launch_sort(const Plan& pl, int32_t* dbg_perm, hipStream_t st) {
     if (pl.total == 0) return 0;
-    hipLaunchKernelGGL(k_keys, dim3(pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl);
-    SG_LAUNCH_CHECK("k_keys");
-    const int n = 256 * pl.sort_tiles;
-    const int nb = (n + SCAN_BLOCK_ITEMS - 1) / SCAN_BLOCK_ITEMS;
-    for (int pass = 0; pass < 4; pass++) {
-        const int src = pass & 1, shift = 8 * pass;
-        if (pass > 0) hipLaunchKernelGGL(k_hist, dim3(pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl, src, shift);     // the first pass's counts come from k_keys
-        if (n <= SPINE_SINGLE_MAX) {
-            hipLaunchKernelGGL(k_spine_single, dim3(1), dim3(1024), 0, st, pl.spine, n);
-        } else {
-            hipLaunchKernelGGL(k_spine_reduce, dim3(nb), dim3(256), 0, st, pl.spine, pl.blocksums, n);
-            hipLaunchKernelGGL(k_spine_down, dim3(nb), dim3(256), 0, st, pl.spine, pl.blocksums, n);
-        }
-        if (pass == 0) hipLaunchKernelGGL(k_scatter<true>, dim3(pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl, src, shift);
-        else hipLaunchKernelGGL(k_scatter<false>, dim3(pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl, src, shift);
-        SG_LAUNCH_CHECK("radix pass");
+    if (pl.geo == GEO_LARGE ? launch_sort_geo<GeoLarge>(pl, st) : launch_sort_geo<GeoDefault>(pl, st)) return 1;
+    // result in keys[0] / vals[0]
+    if (dbg_perm) {
+        hipLaunchKernelGGL(k_permutation, dim3(pl.elem_tiles), dim3(256), 0, st, pl, dbg_perm);
+        SG_LAUNCH_CHECK("k_permutation");
     }
-    // result is back in keys[0] / vals[0]
-    hipLaunchKernelGGL(k_gather_sorted, dim3(pl.elem_tiles), dim3(256), 0, st, pl, dbg_perm);
-    SG_LAUNCH_CHECK("k_gather_sorted");
     return 0;
 }
 

@@ -1,6 +1,6 @@
 // C-ABI entry points of the SuperGrok v2 batched step: validation, workspace
 // carving, the small per-call table upload and the launch sequence
-//   keys -> 4 radix passes -> sharpness gather -> coefficient composition
+//   [gradient norms ->] keys and coefficient composition -> 4 radix passes
 //   -> chunk summaries -> chunk prefix -> scan output
 //   -> per-element GRU/PEER/expert/Adam,
 // and of the scan part of the bilevel pass (the same sort + scan with the
@@ -64,9 +64,10 @@ struct Prof {
     std::vector<hipEvent_t> ev;     // [SG2_PROF_MAX_CALLS][PROF_MARKS], created on first enable
 } g_prof;
 
+constexpr int PREFIXES = 5;     // prefix tables: tiles of the elementwise kernels, sort tiles, scan chunks, chunks with a summary, norm tiles
 struct Layout {
-    int P, total, elem_tiles, sort_tiles, chunks, wchunks, nb;
-    size_t off_tables, off_keys[2], off_vals[2], off_ssorted, off_spine, off_blocksums, off_summ, off_hstart, off_comp, off_flags, off_padw, off_ctx, off_htile, off_adj_summ, off_adj_lam, off_adj_part, off_adj_blk, bytes;
+    int P, total, elem_tiles, sort_tiles, chunks, wchunks, nb, sort_tile, sort_widest, norm_tile, norm_tiles;
+    size_t off_norm, off_gscale, off_tables, off_keys[2], off_vals[2], off_ssorted, off_spine, off_blocksums, off_summ, off_hstart, off_comp, off_flags, off_padw, off_ctx, off_htile, off_adj_summ, off_adj_lam, off_adj_part, off_adj_blk, bytes;
     size_t tables_bytes;
 };
 
@@ -124,27 +125,44 @@ __global__ __launch_bounds__(256) void k_pad_weights(PadArgs a) {
     }
 }
 
+// Keys per sort tile.  A scatter of 8192 keys is 16 rounds in series per wave whatever the call's size; tensors of at
+// most 65 536 elements take tiles of 2048 (the 14-tensor set: 212 workgroups instead of 57, 6 us per pass instead of 11), at
+// which they have no more than SELF_SCAN_TILES.  Tensors of one large tile each are sorted in LDS by one launch.
+inline int sort_tile_for(int64_t widest) {
+    return widest > SORT_TILE && widest <= (int64_t)SELF_SCAN_TILES * SORT_TILE_SMALL ? SORT_TILE_SMALL : SORT_TILE;
+}
+// Elements per workgroup of the norm reduction: as the other steps' tiles (many short ones for small calls).
+inline int norm_tile_for(int64_t total) { return total >= (8 << 20) ? 4096 : (total >= (1 << 20) ? 1024 : 256); }
+
 int make_layout(int geo, int P, Numels numels, int chunk_len, Layout* L, bool bilevel = false) {
     const GeoInfo gi = geo_info(geo);
-    int64_t total = 0, et = 0, stl = 0, ch = 0, wch = 0;
+    int64_t total = 0, et = 0, stl = 0, ch = 0, wch = 0, nt = 0, widest = 0;
     for (int i = 0; i < P; i++) {
         const int64_t n = numels[i];
         if (n < 0) return sg::fail("tensor %d: negative numel", i);
         if (n > 0x7fffffff) return sg::fail("tensor %d: numel %lld exceeds 2^31-1", i, (long long)n);
         total += n;
+        widest = n > widest ? n : widest;
+    }
+    L->sort_tile = sort_tile_for(widest);
+    L->sort_widest = (int)((widest + L->sort_tile - 1) / L->sort_tile);
+    L->norm_tile = norm_tile_for(total);
+    for (int i = 0; i < P; i++) {
+        const int64_t n = numels[i];
         et += (n + ELEM_TILE - 1) / ELEM_TILE;
-        stl += (n + SORT_TILE - 1) / SORT_TILE;
+        stl += (n + L->sort_tile - 1) / L->sort_tile;
+        nt += (n + L->norm_tile - 1) / L->norm_tile;
         const int64_t nc = (n + chunk_len - 1) / chunk_len;
         ch += nc;
         wch += nc > 0 ? nc - 1 : 0;
     }
     if (total > 0x7ffffff0) return sg::fail("total element count %lld exceeds the 2^31 indexing limit", (long long)total);
     L->P = P; L->total = (int)total; L->elem_tiles = (int)et; L->sort_tiles = (int)stl;
-    L->chunks = (int)ch; L->wchunks = (int)wch;
+    L->chunks = (int)ch; L->wchunks = (int)wch; L->norm_tiles = (int)nt;
     L->nb = (int)((256 * stl + SCAN_BLOCK_ITEMS - 1) / SCAN_BLOCK_ITEMS);
     size_t o = 0;
     auto take = [&](size_t bytes) { size_t r = o; o = sg::align_up(o + bytes, 256); return r; };
-    L->tables_bytes = sizeof(TensorDev) * (size_t)P + 4 * sizeof(int) * (size_t)(P + 1);
+    L->tables_bytes = sizeof(TensorDev) * (size_t)P + PREFIXES * sizeof(int) * (size_t)(P + 1);
     L->off_tables = take(L->tables_bytes);
     for (int k = 0; k < 2; k++) L->off_keys[k] = take(4 * (size_t)total);
     for (int k = 0; k < 2; k++) L->off_vals[k] = take(4 * (size_t)total);
@@ -154,6 +172,8 @@ int make_layout(int geo, int P, Numels numels, int chunk_len, Layout* L, bool bi
     L->off_summ = take(4 * 2 * (size_t)wch * 6 * gi.threads);
     L->off_hstart = take(4 * 2 * (size_t)ch * 2 * gi.threads);
     L->off_comp = take(4 * (2 * 5 * (size_t)gi.rows * 3 + 2 * 2 * (size_t)gi.rows * 4 + 12));      // composed triples, Taylor polynomials, coefficient maxima and polynomial limits
+    L->off_norm = take(8 * (size_t)nt);
+    L->off_gscale = take(4 * (size_t)P);
     L->off_flags = take(4 * (2 * (size_t)P + 3));    // apart from the tensor records: it is written while those are being read
     L->off_padw = take(4 * (size_t)padded_weight_floats(gi));   // scan weights embedded in the kernel geometry (used when the caller's block is smaller)
     L->off_ctx = take(4 * 2 * (size_t)total * gi.dm);
@@ -168,19 +188,18 @@ int make_layout(int geo, int P, Numels numels, int chunk_len, Layout* L, bool bi
 }
 
 
-// Per-call tables travel as kernel arguments: UPLOAD_RECS tensor records and their entries of the four prefix
-// tables (tiles of the elementwise kernels, sort tiles, scan chunks, chunks with a summary) per launch.
+// Per-call tables travel as kernel arguments: UPLOAD_RECS tensor records and their entries of the prefix tables per launch.
 constexpr int UPLOAD_RECS = 24;
 struct TableChunk {
     TensorDev rec[UPLOAD_RECS];
-    int pre[4][UPLOAD_RECS];       // prefix table q, entries i0+1 .. i0+cnt
+    int pre[PREFIXES][UPLOAD_RECS];       // prefix table q, entries i0+1 .. i0+cnt
     TensorDev* dst_rec;
-    int* dst_pre;                  // four tables of P+1 ints, back to back
+    int* dst_pre;                  // PREFIXES tables of P+1 ints, back to back
     int* flags;                    // per-tensor "sharpness is not all zero" flags to clear, or NULL to keep them
     int* state_bad;                // with flags: per tensor, 1 when one of its carried Mamba states holds a non-finite entry
     int i0, cnt, P, state_floats;  // state_floats: d_inner * d_state of the caller's states
 };
-static_assert(sizeof(TableChunk) <= 3600, "kernel arguments stay well below 4 KB");
+static_assert(sizeof(TableChunk) <= 3700, "kernel arguments stay well below 4 KB");
 
 // Workgroup 0 writes the records and tables; workgroup 1 + k looks at the carried states of tensor i0 + k.
 __global__ __launch_bounds__(256) void k_tables(TableChunk c) {
@@ -202,16 +221,48 @@ __global__ __launch_bounds__(256) void k_tables(TableChunk c) {
     const int* src = reinterpret_cast<const int*>(c.rec);
     int* dst = reinterpret_cast<int*>(c.dst_rec + c.i0);
     for (int w = threadIdx.x; w < c.cnt * WORDS; w += 256) dst[w] = src[w];
-    for (int w = threadIdx.x; w < 4 * c.cnt; w += 256) {
+    for (int w = threadIdx.x; w < PREFIXES * c.cnt; w += 256) {
         const int q = w / c.cnt, k = w % c.cnt;
         c.dst_pre[q * (c.P + 1) + c.i0 + 1 + k] = c.pre[q][k];
     }
-    if (c.i0 == 0 && threadIdx.x < 4) c.dst_pre[threadIdx.x * (c.P + 1)] = 0;
+    if (c.i0 == 0 && threadIdx.x < PREFIXES) c.dst_pre[threadIdx.x * (c.P + 1)] = 0;
     if (c.flags != nullptr)
         for (int k = threadIdx.x; k < c.cnt; k += 256) c.flags[c.i0 + k] = 0;
 }
 
+// Pre-pass of a clipping call (supergrok2.py:316-321 of the reference): sums of squares of every tensor's gradient, one per
+// tile; the sort's first kernel adds them up (clip_factor) and every kernel applies the factor to a gradient as it reads
+// it.  HBM bound (one read of the gradients); writing clipped copies and reading those instead cost a second pass (38 us
+// for 25 M elements) and three launches.  (The tile that finishes a tensor could add them up here, but an atomic counter
+// with release order per workgroup took 38 us where the plain stores take 5: each one writes back its L2.)
+__global__ __launch_bounds__(256) void k_norm(Plan pl) {
+    __shared__ double sm[4];
+    const int tile = blockIdx.x;
+    const sg::Seg seg = sg::find_seg(sg::as_const(pl.norm_tile_prefix), pl.P, tile);
+    const TensorDev& T = pl.tensors[seg.i];
+    const int start = (tile - seg.first) * pl.norm_tile, cnt = min(pl.norm_tile, T.numel - start);
+    float acc = 0.0f;
+    for (int k0 = 0; k0 < cnt; k0 += 8 * 256) {       // eight loads on their way at a time, added in order
+        float g[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const int k = k0 + r * 256 + (int)threadIdx.x;
+            g[r] = k < cnt ? sg::load_elem(T.grad, T.dtype, start + k) : 0.0f;
+        }
+#pragma unroll
+        for (int r = 0; r < 8; r++) acc = sg_fma(g[r], g[r], acc);
+    }
+    const double sum = sg::block_sum((double)acc, sm);
+    if (threadIdx.x == 0) pl.norm_partials[tile] = sum;
+}
+
 }  // namespace
+
+int launch_norm(const Plan& pl, hipStream_t st) {
+    hipLaunchKernelGGL(k_norm, dim3(pl.norm_tiles), dim3(256), 0, st, pl);
+    SG_LAUNCH_CHECK("k_norm");
+    return 0;
+}
 
 int geo_of(const SgDims* d) {
     if (!d) return sg::fail("dims is NULL"), -1;
@@ -369,7 +420,8 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
         if (t.numel > 0) {
             if (!t.grad || !t.sharpness || !t.mamba_fwd_state || !t.mamba_bwd_state) return sg::fail("tensor %d: NULL pointer", i);
             if (full_step && (!t.param || !t.exp_avg || !t.exp_avg_sq || !t.mu || !t.gru_state)) return sg::fail("tensor %d: NULL pointer", i);
-            if (t.dtype != SG_F32 && t.dtype != SG_F16 && t.dtype != SG_BF16) return sg::fail("tensor %d: bad dtype %d", i, t.dtype);
+            const int dtype = t.dtype & ~SG_SHARP_F32;
+            if (dtype != SG_F32 && dtype != SG_F16 && dtype != SG_BF16) return sg::fail("tensor %d: bad dtype %d", i, t.dtype);
             if (full_step && ((uintptr_t)t.gru_state & 15u) != 0) return sg::fail("tensor %d: gru_state must be 16-byte aligned", i);
         }
     }
@@ -387,7 +439,7 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
         TensorDev* d_rec = reinterpret_cast<TensorDev*>(ws + L.off_tables);
         int* d_pre = reinterpret_cast<int*>(ws + L.off_tables + sizeof(TensorDev) * (size_t)P);
         int* d_flags = keep_flags ? nullptr : reinterpret_cast<int*>(ws + L.off_flags);
-        int off = 0, run[4] = {0, 0, 0, 0};
+        int off = 0, run[PREFIXES] = {};
         for (int i0 = 0; i0 < P; i0 += UPLOAD_RECS) {
             TableChunk c;
             c.dst_rec = d_rec; c.dst_pre = d_pre; c.flags = d_flags;
@@ -402,16 +454,18 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
                 d.param = t.param; d.grad = t.grad; d.sharp = t.sharpness;
                 d.ea = t.exp_avg; d.easq = t.exp_avg_sq; d.mu = t.mu; d.gru = t.gru_state;
                 d.mfwd = t.mamba_fwd_state; d.mbwd = t.mamba_bwd_state;
-                d.off = off; d.numel = n; d.dtype = t.dtype; d.nchunks = nc;
+                d.off = off; d.numel = n; d.dtype = t.dtype & ~SG_SHARP_F32; d.nchunks = nc;
+                d.sharp32 = t.dtype != d.dtype && d.dtype != SG_F32 ? 1 : 0;
                 d.alpha = t.alpha_mu; d.lamb = t.lamb_eff; d.beta1 = t.beta1; d.bc2 = t.bc2;
                 d.step_size = full_step ? scalars->lr / t.bc1 : 0.0f;
-                for (int q = 0; q < 5; q++) d.pad_[q] = 0;
+                for (int q = 0; q < 4; q++) d.pad_[q] = 0;
                 off += n;
                 run[0] += (n + ELEM_TILE - 1) / ELEM_TILE;
-                run[1] += (n + SORT_TILE - 1) / SORT_TILE;
+                run[1] += (int)(((int64_t)n + L.sort_tile - 1) / L.sort_tile);
                 run[2] += nc;
                 run[3] += nc > 0 ? nc - 1 : 0;
-                for (int q = 0; q < 4; q++) c.pre[q][k] = run[q];
+                run[4] += (int)(((int64_t)n + L.norm_tile - 1) / L.norm_tile);
+                for (int q = 0; q < PREFIXES; q++) c.pre[q][k] = run[q];
             }
             hipLaunchKernelGGL(k_tables, dim3(d_flags ? 1 + c.cnt : 1), dim3(256), 0, st, c);
             SG_LAUNCH_CHECK("k_tables");
@@ -424,6 +478,12 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
     pl.sort_tile_prefix = dpre + (P + 1);
     pl.chunk_prefix = dpre + 2 * (P + 1);
     pl.wchunk_prefix = dpre + 3 * (P + 1);
+    pl.norm_tile_prefix = dpre + 4 * (P + 1);
+    pl.sort_tile = L.sort_tile; pl.sort_widest = L.sort_widest;
+    pl.norm_tile = L.norm_tile; pl.norm_tiles = L.norm_tiles;
+    pl.norm_partials = reinterpret_cast<double*>(ws + L.off_norm);
+    pl.gscale = nullptr;
+    pl.max_norm = 0.0f;
     pl.P = P; pl.total = L.total; pl.elem_tiles = L.elem_tiles; pl.sort_tiles = L.sort_tiles;
     pl.chunks = L.chunks; pl.wchunks = L.wchunks; pl.chunk_len = chunk_len; pl.window = window_override >= 0 ? window_override : g_window.load();
     for (int k = 0; k < 2; k++) {
@@ -484,7 +544,7 @@ int resolve_options(const Sg2Options* o, int P, Numels numels, int* chunk_len, i
 
 int run_step(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, const Sg2Scalars* scalars,
              int32_t* expert_counts, void* workspace, size_t workspace_bytes, const Sg2Debug* debug, hipStream_t st,
-             const Sg2Options* options = nullptr) {
+             const Sg2Options* options = nullptr, float clip_norm = 0.0f) {
     Plan pl;
     Layout L;
     int chunk_override = 0, window_override = -1;
@@ -494,6 +554,11 @@ int run_step(const SgDims* dims, const Sg2Weights* weights, int num_tensors, con
         return 1;
     if (pl.total == 0) return 0;
     prof_mark(0, st);
+    if (clip_norm > 0.0f) {
+        pl.gscale = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + L.off_gscale);
+        pl.max_norm = clip_norm;
+        if (launch_norm(pl, st)) return 1;
+    }
     if (launch_sort(pl, debug ? debug->perm : nullptr, st)) return 1;
     prof_mark(1, st);
     if (launch_scan(pl, st)) return 1;
@@ -540,6 +605,13 @@ int sg2_batched_step(const SgDims* dims, const Sg2Weights* weights, int num_tens
                      const Sg2Debug* debug, void* stream) {
     return sg2::run_step(dims, weights, num_tensors, tensors, scalars, expert_counts, workspace, workspace_bytes, debug,
                          (hipStream_t)stream);
+}
+
+int sg2_clipped_step(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, const Sg2Scalars* scalars,
+                     float max_norm, int32_t* expert_counts, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!(max_norm > 0.0f)) return sg::fail("sg2_clipped_step: max_norm must be positive");
+    return sg2::run_step(dims, weights, num_tensors, tensors, scalars, expert_counts, workspace, workspace_bytes, nullptr, (hipStream_t)stream,
+                         nullptr, max_norm);
 }
 
 size_t sg2_workspace_bytes_opt(const SgDims* dims, int num_tensors, const int64_t* numels, const Sg2Options* options) {

@@ -63,6 +63,22 @@ __device__ __forceinline__ void store_elem(void* p, int dtype, int64_t i, float 
     else ((SG_GLOBAL uint16_t*)p)[i] = f_to_bf16_bits(v);
 }
 __device__ __forceinline__ float finite_or_zero(float v) { return sg_isfinite(v) ? v : 0.0f; }
+// v as it reads back after being stored in the type
+__device__ __forceinline__ float round_to(int dtype, float v) {
+    if (dtype == SG_F16) return __half2float(__float2half_rn(v));
+    if (dtype == SG_BF16) return bf16_bits_to_f(f_to_bf16_bits(v));
+    return v;
+}
+// sum over the 256 threads of a block (waves in order), for every thread; sm: 4 doubles of LDS
+__device__ __forceinline__ double block_sum(double v, double* sm) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_down(v, d, 64);
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
+    __syncthreads();
+    const double r = (sm[0] + sm[1]) + (sm[2] + sm[3]);
+    __syncthreads();
+    return r;
+}
 
 // Read-only tables and weights are read through the constant address space: a
 // wave-uniform index then becomes a scalar load (s_load_dword*), which the
@@ -91,6 +107,27 @@ __device__ __forceinline__ int upper_seg(P prefix, int n, int x) {
         if (prefix[mid] <= x) lo = mid; else hi = mid;
     }
     return lo;
+}
+
+// The segment of a prefix table that holds x, its first entry and its end.  Called by whole waves with one x: for up to
+// 64 segments a lane loads the end of each and a ballot counts those not above x, one memory latency where the binary
+// search waits for six dependent ones (and the table's neighbours come along).
+struct Seg { int i, first, end; };
+template <class P>
+__device__ __forceinline__ Seg find_seg(P prefix, int n, int x) {
+    Seg s;
+    if (n <= 64) {
+        const int lane = threadIdx.x & 63;
+        const int end = lane < n ? prefix[lane + 1] : 0x7fffffff;
+        s.i = __popcll(__ballot(end <= x));
+        s.first = s.i > 0 ? __builtin_amdgcn_readlane(end, s.i - 1) : 0;
+        s.end = __builtin_amdgcn_readlane(end, s.i);
+    } else {
+        s.i = upper_seg(prefix, n, x);
+        s.first = prefix[s.i];
+        s.end = prefix[s.i + 1];
+    }
+    return s;
 }
 
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }

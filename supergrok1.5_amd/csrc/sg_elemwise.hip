@@ -28,7 +28,7 @@ __global__ __launch_bounds__(THREADS) void k_grokfast(BT B, float alpha, float l
 #pragma unroll
         for (int c = 0; c < V; c++) {
             e[c] = sg_fma(alpha, e[c], om_alpha * g[c]);
-            g[c] = rounded(R.dtype, sg_fma(lamb, e[c], g[c]));       // AdamW consumes the gradient as stored
+            g[c] = sg::round_to(R.dtype, sg_fma(lamb, e[c], g[c]));       // AdamW consumes the gradient as stored
         }
         stf<V>(R.aux, i, e);
         stt<V>(R.grad, R.dtype, i, g);

@@ -205,20 +205,13 @@ __device__ __forceinline__ void stt(void* p, int dtype, int i, const float (&x)[
         sg::store_elem(p, dtype, i, x[0]);
     }
 }
-// v as it reads back after being stored in the tensor's type
-__device__ __forceinline__ float rounded(int dtype, float v) {
-    if (dtype == SG_F16) return __half2float(__float2half_rn(v));
-    if (dtype == SG_BF16) return sg::bf16_bits_to_f(sg::f_to_bf16_bits(v));
-    return v;
-}
-
 // sharpness of a tensor: in its type, or in fp32 and rounded to it
 template <int V>
 __device__ __forceinline__ void ldsharp(const Rec& R, int i, float (&x)[V]) {
     if (!R.sharp32) return ldt<V>(R.aux2, R.dtype, i, x);
     ldf<V>(static_cast<const float*>(R.aux2), i, x);
 #pragma unroll
-    for (int c = 0; c < V; c++) x[c] = rounded(R.dtype, x[c]);
+    for (int c = 0; c < V; c++) x[c] = sg::round_to(R.dtype, x[c]);
 }
 
 // Runs body(V, i) over the elements of a tile: four consecutive ones per lane where the tensor's pointers allow
@@ -234,16 +227,6 @@ __device__ __forceinline__ void for_tile(const Rec& R, int start, int cnt, B bod
 }
 
 // ---- deterministic sums -------------------------------------------
-__device__ __forceinline__ double block_sum(double v, double* sm /*[4]*/) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v += __shfl_down(v, d, 64);
-    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
-    __syncthreads();
-    const double r = (sm[0] + sm[1]) + (sm[2] + sm[3]);
-    __syncthreads();
-    return r;
-}
-
 // blocks of a whole-call reduction over `tiles` tiles
 inline int partial_blocks(int tiles) { return tiles < MAX_PARTIALS ? tiles : MAX_PARTIALS; }
 
@@ -275,7 +258,7 @@ __global__ __launch_bounds__(THREADS) void k_sumsq(BT B, int blocks, Extra extra
         sum += (double)acc;
         acc = 0.0f;
     }
-    const double tot = block_sum(sum, sm);
+    const double tot = sg::block_sum(sum, sm);
     if (threadIdx.x == 0) B.partials[blockIdx.x] = tot;
 }
 template <class BT, class Extra = NoExtra>
@@ -296,7 +279,7 @@ __device__ __forceinline__ Clip global_norm(const BT& B, float clip_norm) {
     double acc = 0.0;
     for (int k = threadIdx.x; k < blocks; k += THREADS) acc += B.partials[k];
     Clip c;
-    c.norm = (float)sqrt(block_sum(acc, sm));
+    c.norm = (float)sqrt(sg::block_sum(acc, sm));
     c.on = clip_norm > 0.0f && c.norm > clip_norm;
     c.coef = c.on ? clip_norm / (c.norm + 1e-6f) : 1.0f;
     return c;
@@ -309,7 +292,7 @@ __device__ __forceinline__ void tile_sums(const BT& B, double a, double b = 0.0,
     const double v[3] = {a, b, c};
 #pragma unroll
     for (int s = 0; s < S; s++) {
-        const double t = block_sum(v[s], sm);
+        const double t = sg::block_sum(v[s], sm);
         if (threadIdx.x == 0) B.partials[3 * (size_t)blockIdx.x + s] = t;
     }
 }
@@ -321,7 +304,7 @@ __device__ __forceinline__ void add_tiles(const BT& B, int lo, int hi, double (&
 #pragma unroll
         for (int s = 0; s < S; s++) acc[s] += B.partials[3 * (size_t)k + s];
 #pragma unroll
-    for (int s = 0; s < S; s++) out[s] = block_sum(acc[s], sm);
+    for (int s = 0; s < S; s++) out[s] = sg::block_sum(acc[s], sm);
 }
 // block t: sums of tensor t's tiles into tred[t]
 template <int S, class BT>
@@ -372,7 +355,7 @@ __device__ __forceinline__ void clipped_grad(const Rec& R, int i, const Clip& cl
     ldt<V>(R.grad, R.dtype, i, g);
     if (clip.on) {
 #pragma unroll
-        for (int c = 0; c < V; c++) g[c] = rounded(R.dtype, g[c] * clip.coef);
+        for (int c = 0; c < V; c++) g[c] = sg::round_to(R.dtype, g[c] * clip.coef);
         stt<V>(R.grad, R.dtype, i, g);
     }
 }

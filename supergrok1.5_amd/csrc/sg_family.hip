@@ -366,7 +366,7 @@ __global__ __launch_bounds__(THREADS) void k_ls_diff_sumsq(BT B) {
         ldt<V>(R.aux2, R.dtype, i, b);
 #pragma unroll
         for (int c = 0; c < V; c++) {
-            const float d = rounded(R.dtype, a[c] - b[c]);     // as the reference forms it: subtracted in the gradients' own type
+            const float d = sg::round_to(R.dtype, a[c] - b[c]);     // as the reference forms it: subtracted in the gradients' own type
             acc = sg_fma(d, d, acc);
         }
     });
@@ -422,7 +422,7 @@ __global__ __launch_bounds__(THREADS) void k_ls_adjust(BT B, float la) {
         ldf<V>(R.aux, i, d);
         ldt<V>(R.grad, R.dtype, i, g);
 #pragma unroll
-        for (int c = 0; c < V; c++) g[c] = sg_fma(scale, rounded(R.dtype, d[c]), g[c]);    // the direction is converted to the gradient's type first (csrc/ops.cpp:646)
+        for (int c = 0; c < V; c++) g[c] = sg_fma(scale, sg::round_to(R.dtype, d[c]), g[c]);    // the direction is converted to the gradient's type first (csrc/ops.cpp:646)
         stt<V>(R.grad, R.dtype, i, g);
     });
 }
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(THREADS) void k_sg2_clip(BT B, float max_norm) {
         ldt<V>(R.grad, R.dtype, i, g);
 #pragma unroll
         for (int c = 0; c < V; c++) {
-            if (scale != 1.0f) g[c] = rounded(R.dtype, g[c] * scale);      // the product is a tensor of the gradient's type
+            if (scale != 1.0f) g[c] = sg::round_to(R.dtype, g[c] * scale);      // the product is a tensor of the gradient's type
             g[c] = sg::finite_or_zero(g[c]);
         }
         stt<V>(R.param, R.dtype, i, g);

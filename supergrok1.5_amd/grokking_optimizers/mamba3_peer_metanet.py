@@ -241,28 +241,28 @@ class Mamba3PEERMetaNet(nn.Module):
         sharing it is dead.  Returns True if anything changed.  Random draws, in order: one multinomial,
         then per dead expert (ascending index) W1, b1, W2, b2 noise, then key A redraws per head, then
         key B redraws per head -- the sequence of the reference (mamba3_peer_metanet.py:453-488)."""
+        from grokking_optimizers import _ops
         total = self.expert_counts.sum().item()
         if total == 0:
             return False
-        dead = (self.expert_counts.float() / total) < self.recycle_threshold
+        dead = ((self.expert_counts.float() / total) < self.recycle_threshold).cpu()
         if not dead.any():
             self.expert_counts.zero_()
             return False
         top = torch.multinomial(self.expert_counts.float(), 1).item()
-        pk, H = self.pk_dim, self.num_peer_heads
-        for i in dead.nonzero(as_tuple=True)[0].tolist():
-            for name in ("expert_W1", "expert_b1", "expert_W2", "expert_b2"):
-                t = getattr(self, name).data
-                t[i] = t[top] + 0.01 * torch.randn_like(t[i])
-            a, b = divmod(i, pk)
-            if dead[a * pk:(a + 1) * pk].all():
-                for h in range(H):
-                    row = self.product_keys_A[h].data[a]
-                    self.product_keys_A[h].data[a] = torch.randn_like(row) * 0.02
-            cols = torch.arange(0, self.num_experts, pk, device=dead.device) + b
-            if dead[cols[cols < self.num_experts]].all():
-                for h in range(H):
-                    row = self.product_keys_B[h].data[b]
-                    self.product_keys_B[h].data[b] = torch.randn_like(row) * 0.02
+        pk, E = self.pk_dim, self.num_experts
+        flags, where = dead.tolist(), dead.nonzero(as_tuple=True)[0]
+        indices = where.tolist()
+        tensors = [getattr(self, name).data for name in ("expert_W1", "expert_b1", "expert_W2", "expert_b2")]
+        noise = [torch.empty((len(indices),) + tuple(t.shape[1:]), dtype=t.dtype, device=t.device) for t in tensors]
+        _ops.recycle_draws(noise, [k.data for k in self.product_keys_A], [k.data for k in self.product_keys_B], indices,
+                           [all(flags[a * pk:(a + 1) * pk]) for a in range(pk)], [all(flags[b:E:pk]) for b in range(pk)], pk, E)
+        where = where.to(self.expert_counts.device)
+        for t, z in zip(tensors, noise):
+            rows = t[top] + 0.01 * z
+            if flags[top]:      # the sampled expert is itself dead: the experts after it clone its new values
+                k = indices.index(top)
+                rows[k + 1:] = rows[k] + 0.01 * z[k + 1:]
+            t[where] = rows
         self.expert_counts.zero_()
         return True

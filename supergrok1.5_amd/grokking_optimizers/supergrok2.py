@@ -107,7 +107,6 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
         three launches for all tensors, norms reduced on the device, no host syncs."""
         return _ops.supergrok2_clip_grads([g.contiguous() for g in grads], float(self.gradient_clipping))
 
-    @torch.no_grad()
     def step(self, closure=None, train_loss=None, val_loss=None, train_acc=None):
         loss = None
         if closure is not None:
@@ -124,9 +123,36 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
         wd_eff = self._get_effective_wd(group["weight_decay"])
         lamb_eff = self.lamb * self._get_ramp_factor() * self._get_gate_signal()
 
+        mn = self.meta_net
+        if self._weights_dirty:
+            self._cached_weights = mn.flat_weights()
+            self._weights_dirty = False
+        # clip, scalars and lists natively (the work of _ops.supergrok2_clip_grads and supergrok2_mamba_peer_batched_step)
+        active = _ops.supergrok2_flat_step(
+            self._flat_params, self._flat_exp_avgs, self._flat_exp_avg_sqs, self._flat_mus, self._flat_sharpness, self._flat_gru_states,
+            self._flat_mamba_fwd_states, self._flat_mamba_bwd_states, self._flat_steps, self._cached_alpha, self._flat_layer_alphas,
+            self._flat_layer_beta1s, float(lamb_eff), self._cached_weights, float(mn.rescale), float(beta2), float(lr), float(wd_eff),
+            float(eps),
+            (mn.d_model, mn.d_state, mn.mamba_fwd.d_inner, mn.gru_hidden, mn.num_peer_heads, mn.pk_dim, mn.expert_hidden, mn.num_experts),
+            mn.expert_counts, float(self.gradient_clipping))
+        if active < 0:
+            with torch.no_grad():
+                active = self._step_lists(lr, beta2, eps, wd_eff, lamb_eff)
+        if active == 0:
+            return loss
+        self._step_counter += 1
+        if mn.recycle_interval > 0 and self._step_counter % mn.recycle_interval == 0:
+            if mn._recycle_dead_experts():
+                self._weights_dirty = True
+        return loss
+
+    def _step_lists(self, lr, beta2, eps, wd_eff, lamb_eff):
+        """The step through the list functions, for what the native walk leaves to it: Mamba states that are created on
+        first use, gradients that are not contiguous, a clip threshold that is not positive.  Returns the number of
+        parameters with a gradient."""
         active = [i for i, p in enumerate(self._flat_params) if p.grad is not None]
         if not active:
-            return loss
+            return 0
         mn = self.meta_net
         if not self._flat_params[active[0]].is_cuda:
             raise RuntimeError("SuperGrok2 on MI355X needs GPU parameters: the fused step has no CPU path")
@@ -146,9 +172,6 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
                 self._flat_mamba_bwd_states[i] = torch.zeros(*shape, dtype=torch.float32, device=p.device)
         grads = self._clip([self._flat_params[i].grad.data for i in active])
         grads = [g.contiguous() for g in grads]
-        if self._weights_dirty:
-            self._cached_weights = mn.flat_weights()
-            self._weights_dirty = False
         sharp = [self._flat_sharpness[i].to(g.dtype) for i, g in zip(active, grads)]
         pick = lambda lst: [lst[i] for i in active]
         _ops.supergrok2_mamba_peer_batched_step(
@@ -158,11 +181,7 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
             alphas, lambs, beta1s, bc1s, bc2s, float(mn.rescale), float(beta2), float(lr), float(wd_eff), float(eps),
             mn.d_model, mn.d_state, mn.mamba_fwd.d_inner, mn.gru_hidden, mn.num_peer_heads, mn.pk_dim,
             mn.expert_hidden, mn.num_experts, mn.expert_counts)
-        self._step_counter += 1
-        if mn.recycle_interval > 0 and self._step_counter % mn.recycle_interval == 0:
-            if mn._recycle_dead_experts():
-                self._weights_dirty = True
-        return loss
+        return len(active)
 
     # sam_step comes from MetaTraining (supergrok2.py:474-514 of the reference); sam_meta_step, step_full and the
     # getters from ScheduledTraining.
