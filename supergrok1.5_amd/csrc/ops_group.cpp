@@ -510,6 +510,98 @@ int64_t supergrok2_flat_step(py::list params, py::list eas, py::list easqs, py::
     return (int64_t)active.size();
 }
 
+// The bilevel pass over tensors that stay where they are (sg2_bilevel_pass): (smart gradients or None, gradients of the
+// per-element weights, gradients of the scan weights), flat.  exact: fp32 sharpness next to 16-bit gradients is used as it
+// is.  None where the general path has to be taken (other sizes of the net, tensors that would have to be converted).
+py::object supergrok2_bilevel_pass(py::list grads, py::list sharps, py::list grus, py::list mfwd, py::list mbwd, py::list cots,
+                                   py::list weights, float rescale, bool normalise, bool exact, bool want_smart, std::vector<int> dims8) {
+    const char* fn = "supergrok2_bilevel_pass";
+    const Py_ssize_t P = PyList_GET_SIZE(grads.ptr());
+    for (PyObject* l : {sharps.ptr(), grus.ptr(), mfwd.ptr(), mbwd.ptr(), cots.ptr()})
+        if (PyList_GET_SIZE(l) != P) return py::none();
+    if (P == 0 || dims8.size() != 8 || PyList_GET_SIZE(weights.ptr()) != SG2_NUM_WEIGHTS) return py::none();
+    const SgDims dims = {dims8[0], dims8[1], dims8[2], dims8[3], dims8[4], dims8[5], dims8[6], dims8[7]};
+    auto item = [](const py::list& l, Py_ssize_t i) { return as_tensor(PyList_GET_ITEM(l.ptr(), i)); };
+    std::vector<Sg2Tensor> ts;
+    std::vector<int64_t> numels;
+    std::vector<at::Tensor> held;        // cotangents that had to be made contiguous
+    held.reserve(P);
+    int64_t total = 0;
+    const at::Tensor* first = nullptr;
+    for (Py_ssize_t i = 0; i < P; i++) {
+        const at::Tensor *g = item(grads, i), *s = item(sharps, i), *gru = item(grus, i), *mf = item(mfwd, i), *mb = item(mbwd, i),
+                         *c = item(cots, i);
+        if (!g || !s || !gru || !mf || !mb || !c) return py::none();
+        const int64_t n = g->numel();
+        if (n == 0) continue;
+        if (!g->is_cuda() || !g->is_contiguous() || g->scalar_type() != c->scalar_type() || c->numel() != n || s->numel() != n) return py::none();
+        for (const at::Tensor* t : {s, gru, mf, mb})
+            if (!t->is_cuda() || !t->is_contiguous()) return py::none();
+        for (const at::Tensor* t : {gru, mf, mb})
+            if (t->scalar_type() != torch::kFloat32) return py::none();
+        if (gru->numel() != n * dims.gru_hidden || mf->numel() != (int64_t)dims.d_inner * dims.d_state || mb->numel() != mf->numel()) return py::none();
+        if (((uintptr_t)gru->data_ptr() & 15u) != 0 || !c->is_cuda()) return py::none();
+        if (!c->is_contiguous()) {
+            held.push_back(c->contiguous());
+            c = &held.back();
+        }
+        Sg2Tensor q = {};
+        q.dtype = dtype_code(*g, "grad");
+        if (s->scalar_type() != g->scalar_type()) {
+            if (!exact || s->scalar_type() != torch::kFloat32) return py::none();
+            q.dtype |= SG_SHARP_F32 | SG_SHARP_EXACT;
+        }
+        q.param = c->data_ptr();
+        q.grad = g->data_ptr();
+        q.sharpness = s->data_ptr();
+        q.gru_state = gru->data_ptr<float>();
+        q.mamba_fwd_state = mf->data_ptr<float>();
+        q.mamba_bwd_state = mb->data_ptr<float>();
+        q.numel = n;
+        ts.push_back(q);
+        numels.push_back(n);
+        total += n;
+        if (!first) first = g;
+    }
+    if (!first) return py::none();
+    const torch::Tensor* w[SG2_NUM_WEIGHTS];
+    for (int k = 0; k < SG2_NUM_WEIGHTS; k++) {
+        w[k] = item(weights, k);
+        if (!w[k]) return py::none();
+    }
+    Sg2Weights W;
+    check_sg2_weights(fn, w, dims, &W);
+    const size_t bytes = sg2_bilevel_pass_workspace_bytes(&dims, (int)ts.size(), numels.data());
+    TORCH_CHECK(bytes > 0, fn, ": ", sg_last_error());
+    auto ws = make_workspace(bytes, *first);
+    const auto opt = torch::TensorOptions().device(first->device()).dtype(torch::kFloat32);
+    auto elem = torch::empty({(SG2_ELEM_GRAD_FLOATS - dims.num_experts * 49) + dims.num_experts * (3 * dims.expert_hidden + 1)}, opt);
+    auto scan = torch::empty({SG2_SCAN_GRAD_FLOATS}, opt);
+    torch::Tensor smart;
+    if (want_smart) smart = torch::empty({total}, opt);
+    check_status(sg2_bilevel_pass(&dims, &W, (int)ts.size(), ts.data(), rescale, normalise ? 1 : 0, want_smart ? smart.data_ptr<float>() : nullptr,
+                                  elem.data_ptr<float>(), scan.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), current_stream(*first)), fn);
+    return py::make_tuple(want_smart ? py::cast(smart) : py::object(py::none()), elem, scan);
+}
+
+// p.grad (+)= its slice of `flat`, parameter after parameter; one without a gradient gets a view of the flat tensor.
+void add_flat_grads(const std::vector<torch::Tensor>& params, const torch::Tensor& flat) {
+    at::NoGradGuard guard;
+    int64_t o = 0;
+    for (const torch::Tensor& p : params) {
+        const int64_t n = p.numel();
+        TORCH_CHECK(o + n <= flat.numel(), "add_flat_grads: parameters and gradients do not match");
+        if (p.requires_grad()) {
+            at::Tensor g = flat.narrow(0, o, n).view(p.sizes());
+            if (g.scalar_type() != p.scalar_type()) g = g.to(p.scalar_type());
+            at::Tensor& mine = const_cast<torch::Tensor&>(p).mutable_grad();
+            mine = mine.defined() ? mine + g : g;
+        }
+        o += n;
+    }
+    TORCH_CHECK(o == flat.numel(), "add_flat_grads: parameters and gradients do not match");
+}
+
 // The random draws of an expert recycling event, in the order of the reference's loop
 // (grokking_optimizers/mamba3_peer_metanet.py:453-488): per dead expert one N(0,1) draw for each of the four expert
 // tensors into its row of `noise`, then a redraw of its key A row if every expert of that row is dead, then of its key B
@@ -558,5 +650,7 @@ void bind_group_steps(pybind11::module_& m) {
     m.def("supergrok15_flat_step", &supergrok15_flat_step);
     m.def("supergrok11_flat_step", &supergrok11_flat_step);
     m.def("supergrok2_flat_step", &supergrok2_flat_step);
+    m.def("supergrok2_bilevel_pass", &supergrok2_bilevel_pass);
+    m.def("add_flat_grads", &add_flat_grads);
     m.def("recycle_draws", &recycle_draws);
 }

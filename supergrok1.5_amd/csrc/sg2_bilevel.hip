@@ -84,7 +84,7 @@ __device__ __forceinline__ float pair_sum(float v) {             // sum over the
 // What a (chunk, direction) needs to find its steps.
 struct ChunkRef {
     int ti, N, off, ustart, uend;
-    bool has_s;
+    bool has_s, own_order;
     const uint32_t* skey;
     const int32_t* sval;
     const float* ssrt;
@@ -100,6 +100,7 @@ __device__ __forceinline__ ChunkRef chunk_ref(const Plan& pl, int chunk, int dir
     c.ustart = (chunk - pl.chunk_prefix[c.ti]) * pl.chunk_len;
     c.uend = min(c.N, c.ustart + pl.chunk_len);
     c.has_s = pl.sharp_nonzero[c.ti] != 0;        // all-zero sharpness is never gathered into sorted order
+    c.own_order = pl.own_order;
     c.skey = pl.keys[0] + c.off;
     c.sval = pl.vals[0] + c.off;
     c.ssrt = pl.ssorted + c.off;
@@ -114,7 +115,7 @@ __device__ __forceinline__ void load_step(const ChunkRef& c, int dir, int u, boo
         const int t = dir ? (c.N - 1 - u) : u;
         const int32_t v = c.sval[t];
         int o = v & 0x7fffffff;
-        *orig = ((unsigned)o < (unsigned)c.N) ? o : 0;
+        *orig = c.own_order ? t : ((unsigned)o < (unsigned)c.N) ? o : 0;
         *g = sg_i2f((int32_t)c.skey[t] | (v & (int32_t)0x80000000));
         *s = c.has_s ? c.ssrt[t] : 0.0f;
     }

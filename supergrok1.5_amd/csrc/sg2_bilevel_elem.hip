@@ -8,73 +8,85 @@
 // grokking_optimizers/supergrok2.py:516-1330); the arithmetic is that of Mamba3PEERMetaNet.forward_for_bilevel
 // (grokking_optimizers/mamba3_peer_metanet.py:395-436) and its autograd derivative.
 //
-// One lane per element, persistent grid over tiles of 256 elements, one 256-lane workgroup per CU.  Nothing is kept
-// between forward and backward: a lane holds its element's activations in registers, and the routing of a head is
-// differentiated before the next head is evaluated.  Weight gradients are sums over elements:
+// One wave per tile of 64 elements, one lane per element, every wave on its own: its tiles are a contiguous range, its
+// staging rows are its own part of LDS, and nothing in the tile loop waits for another wave.  20 KB of LDS and at most
+// 256 registers per wave: eight waves, two per SIMD, share a CU.  Nothing is kept between forward and backward: a
+// lane holds its element's activations in registers, and the routing of a head is differentiated before the next head
+// is evaluated.  Weight gradients are sums over elements, formed by fp32 matrix instructions from rows that the lanes
+// leave in LDS (64 elements are the contraction):
 //   * experts (16 per element and head, chosen per element).  An expert's hidden unit m is active where
 //     W1[m] g + b1[m] > 0, i.e. on one side of the threshold -b1[m] / W1[m], so between two neighbouring thresholds of
-//     its 16 units the expert is a straight line  out = A g + B.  Each workgroup sorts the thresholds of every expert
-//     once and tabulates (A, B) for the 17 intervals; an element then finds its interval with five LDS reads and
-//     evaluates the expert with one fma, instead of reading the expert's 49 weights.  The gradients of expert e need,
-//     per unit, S0 = sum w [unit active] and S1 = sum w g [unit active] over the elements routed to e (w: routing
-//     weight times d loss / d head), i.e. sums of (w, w g) per interval.  Small gradients lie in the interval next to
-//     g = 0 on their side of it for every expert; for those the sums over elements are outer products (first sub-key
-//     weights) (x) (second sub-key weights), which every wave accumulates for its 64 elements with fp32 matrix
-//     instructions in registers (16 x 16 x 4: four elements a step), separately for g > 0 and g <= 0.  An element in
-//     any other interval of one of its experts moves its (w, w g) there with LDS float atomics (about 3 clocks a lane,
-//     which is why they are kept for the exceptions).  S0, S1 of a unit are the sums of the bins on the unit's active
-//     side, formed once when the workgroup is done.
+//     its 16 units the expert is a straight line  out = A g + B.  k_expert_tables sorts the thresholds of every expert
+//     and tabulates (A, B) for the 17 intervals.  The gradients of expert e need, per unit, S0 = sum w [unit active] and
+//     S1 = sum w g [unit active] over the elements routed to e (w: routing weight times d loss / d head), i.e. sums of
+//     (w, w g) per interval.  A wave holds, for +x and for -x of a reference magnitude x, the line of every expert and
+//     the borders of the interval it holds on: an element whose g lies there for all of its experts costs one 16-byte
+//     LDS read and a fma per expert, and the sums over such elements are outer products (first sub-key weights) (x)
+//     (second sub-key weights), 16 x 16 x 4 instructions, separately for g > 0 and g <= 0.  The positive elements of a
+//     tile take the first rows and the others the rows after them, so that each step is of one sign.
+//     The bilevel pass hands the elements over in the order of the scan, by |g|: x is then the |g| of the tile's middle
+//     element and almost every element of a large tensor lies in the interval of x for every expert.  When x moves past a
+//     threshold of an expert, the lane that holds that expert's sums adds them to the interval's bin (a row of this
+//     workgroup in memory) and starts again.  In element order x stays next to zero.  The exceptions - elements in
+//     another interval of one of their experts - look the interval up in the tables and move their (w, w g) to its bin
+//     with atomics, one expert per lane at a time.  (With all of a trained net's exceptions taken by LDS atomics, in
+//     element order, they were half of the pass.)
 //     (An element exactly on a threshold counts the unit as inactive on both sides; forward value and gradient use
 //     the same interval, so they stay consistent.)
-//   * GRU and query matrices (dense outer products d (x) x): every lane leaves its x (31 values) and, per head
-//     and once more for the GRU, its d (8 / 12 values) in LDS; each lane of the workgroup owns one entry of the
-//     head's query matrix and up to two of the GRU matrices and sums their products over the tile's elements;
-//   * product keys (rows chosen per element): the same, with d score scattered into a 12-vector per sub-key.
-// Each workgroup writes its sums to its own row of a partials buffer; a second kernel adds the rows in a fixed
-// order.  The dense, key and near-zero expert sums are formed in a fixed order; the other expert bins are filled by
-// atomics of four waves, so where gradients reach beyond the intervals next to zero the last bits of the expert
-// gradients can differ from run to run (as with the reference's atomicAdd).
+//   * GRU and query matrices: d (x) x, 16 x 16 x 4 steps over 27 columns of x;
+//   * product keys (rows chosen per element): d score as two 12-vectors with four non-zeros each (x) the query's halves,
+//     in 4 x 4 x 1 blocks, two elements a step.
+// Each workgroup writes its sums to its own row of a partials buffer and k_elem_finish adds the rows in a fixed order
+// and turns the bins into the experts' gradients.  The dense and key sums are formed in a fixed order; the bins are
+// filled by atomics of four waves, so the last bits of the expert gradients can differ from run to run (as with the
+// reference's atomicAdd).
+//
+// Bound by the vector ALU (about 5000 instructions per wave and tile, two thirds of them the fixed multiply-adds of the
+// net and its derivative).  Measured on 25 M elements with module-initialised experts after some meta steps: 9.3 ms, 47 ms
+// as one lane per element of a 256-lane workgroup that summed the outer products lane by lane from LDS; on 0.42 M elements
+// 0.34 ms instead of 1.1.
 #include "sg2_internal.hpp"
 
 namespace sg2 {
 namespace {
 
-constexpr int BE_THREADS = 256;         // four waves; the LDS tables leave room for one workgroup per CU
-constexpr int BE_WAVES = BE_THREADS / 64;
+constexpr int BE_WAVES = 4;
+constexpr int BE_THREADS = 64 * BE_WAVES;
 constexpr int TOPK = 4;
-constexpr int RH = 16;                  // a staged 12-vector is padded to 16 entries (zeros): one operand row of a 16 x 16 x 4 matrix instruction
-constexpr int RW = 2 * RH + 1;          // staged row of a head: first-index vector at 0, second-index vector at RH (odd stride: consecutive rows hit all banks)
-static_assert(PK <= RH, "a sub-key vector fits its padded half row");
 typedef float be_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int NBIN = EH + 1;            // intervals between an expert's sorted unit thresholds
-static_assert(EH == 16, "the interval search takes steps of 8, 4, 2, 1 and one more");
-constexpr int XW = 31, DW = 13;         // row strides of the staged x and d vectors (odd: lane-consecutive rows hit all banks)
-// x row: g, s, fwd ctx[8], bwd ctx[8], h_old[4], r*h_old[4], h_new[4], 1
-constexpr int X_G = 0, X_S = 1, X_CF = 2, X_CB = 10, X_H = 18, X_RH = 22, X_HN = 26, X_ONE = 30;
-// d row, reused: d query[8] of the current head, then d pre_z[4], d pre_r[4], d pre_h[4] of the GRU
-constexpr int D_Z = 0, D_R = 4, D_H = 8;
-constexpr int N_GRU = 3 * (GH * GRL + GH), N_QHEAD = DM * PIN;     // 276 GRU entries, 176 query entries per head
-constexpr int N_DENSE = N_GRU + NH * N_QHEAD;                      // 276 + 704
-constexpr int OFF_KA = N_DENSE, OFF_KB = OFF_KA + NH * PK * (DM / 2);
-constexpr int OFF_W1 = OFF_KB + NH * PK * (DM / 2), OFF_B1 = OFF_W1 + NE * EH, OFF_W2 = OFF_B1 + NE * EH, OFF_B2 = OFF_W2 + NE * EH;
-constexpr int N_GRADS = OFF_B2 + NE;
-static_assert(N_GRADS == SG2_ELEM_GRAD_FLOATS, "gradient layout");
-constexpr int GRU_PER_LANE = (N_GRU + BE_THREADS - 1) / BE_THREADS, Q_PER_LANE = (N_QHEAD + BE_THREADS - 1) / BE_THREADS;
+static_assert(EH == 16 && PK == 12 && NE == PK * PK && NH == 4 && DM == 8 && GH == 4, "row layouts and lane roles below");
+// x row: h_new[4] (r * h_old[4] once the heads are done), fwd ctx[8], bwd ctx[8], g, s, 1, h_old[4]; the first 22 are the query's input
+constexpr int X_HN = 0, X_CF = 4, X_CB = 12, X_G = 20, X_S = 21, X_ONE = 22, X_H = 23;
+constexpr int XW = 27;
+// rows of the second staging area, by turns:
+constexpr int CW = 25;                  // routing weights of a head: first sub-key[12], second sub-key[12], g
+constexpr int C_ROWS = 80;              // 64 elements, those of either sign padded to whole pairs of steps
+constexpr int KW = 33;                  // d score of a head: first[12], second[12], query[8]
+constexpr int DW = 17;                  // d query of two heads [16], or d pre_z[4], d pre_r[4], d pre_h[4] of the GRU
+constexpr int R_FLOATS = 64 * KW;
+static_assert(C_ROWS * CW <= R_FLOATS && XW % 2 == 1 && CW % 2 == 1 && KW % 2 == 1 && DW % 2 == 1, "odd strides: lane-consecutive rows hit all banks");
+constexpr int WAVE_FLOATS = 64 * XW + R_FLOATS + 2 * NE * 4;       // ... and the lines (A, B, low border, high border) of every expert at +x and -x
+constexpr int KEY_FLOATS = 2 * NH * PK * (DM / 2);
+constexpr int BE_LDS_BYTES = 4 * (KEY_FLOATS + BE_WAVES * WAVE_FLOATS);
+static_assert(2 * BE_LDS_BYTES <= 160 * 1024 && (64 * XW + R_FLOATS) % 4 == 0 && WAVE_FLOATS % 4 == 0 && KEY_FLOATS % 4 == 0, "two workgroups per CU, aligned tables");
 
-// (column of d, column of x) whose products make up GRU gradient entry o, in the order
+constexpr int N_GRU = 3 * (GH * GRL + GH), N_QHEAD = DM * PIN;     // 276 GRU entries, 176 query entries per head
+constexpr int N_DENSE = N_GRU + NH * N_QHEAD + KEY_FLOATS;         // 276 + 704 + 384
+constexpr int N_BINS = NE * NBIN * 2;                              // sums of w and w g over the elements of each interval
+constexpr int ROW_FLOATS = (N_BINS + N_DENSE + 31) / 32 * 32;      // a workgroup's row: bins, then the dense sums
+constexpr int TABLE_FLOATS = NE * EH + NE * NBIN * 2;              // thresholds ascending [NE][EH], lines [NE][NBIN][2]
+static_assert(TABLE_FLOATS % 32 == 0 && N_DENSE + 3 * NE * EH + NE == SG2_ELEM_GRAD_FLOATS, "gradient layout, aligned rows");
+constexpr int BE_MAX_GROUPS = 512;       // two resident workgroups on each of the 256 CUs: one round, every wave walks the same number of tiles (+-1)
+
+// (row of d, column of x) whose product sums make up GRU gradient entry o, in the order
 // W_z[4][22] b_z[4] W_r[4][22] b_r[4] W_h[4][22] b_h[4]
-__device__ __forceinline__ void gru_entry(int o, int* dcol, int* xcol) {
+__device__ __forceinline__ void gru_entry(int o, int* drow, int* xcol) {
     const int gate = o / (GH * GRL + GH), q = o % (GH * GRL + GH);
-    if (q >= GH * GRL) { *dcol = gate * GH + (q - GH * GRL); *xcol = X_ONE; return; }
+    if (q >= GH * GRL) { *drow = gate * GH + (q - GH * GRL); *xcol = X_ONE; return; }
     const int j = q / GRL, c = q % GRL;
-    *dcol = gate * GH + j;
-    *xcol = (gate == 2 && c >= 2 + 2 * DM) ? X_RH + (c - 2 - 2 * DM) : c;     // the candidate sees r*h in place of h
-}
-// same for entry o = r*22 + c of a head's query matrix [8][22]; query input = h_new, fwd ctx, bwd ctx, g, s
-__device__ __forceinline__ void query_entry(int o, int* dcol, int* xcol) {
-    const int c = o % PIN;
-    *dcol = o / PIN;
-    *xcol = c < GH ? X_HN + c : (c < GH + 2 * DM ? X_CF + (c - GH) : (c == GH + 2 * DM ? X_G : X_S));
+    *drow = gate * GH + j;
+    *xcol = c < 2 ? X_G + c : c < 2 + 2 * DM ? X_CF + (c - 2) : (gate == 2 ? X_HN : X_H) + (c - 2 - 2 * DM);     // the candidate sees r*h in place of h
 }
 
 // Is the hidden unit (w1, b1), whose threshold is the rank-th lowest of its expert, active on interval k (the k lowest
@@ -82,72 +94,146 @@ __device__ __forceinline__ void query_entry(int o, int* dcol, int* xcol) {
 __device__ __forceinline__ bool unit_active(float w1, float b1, int rank, int k) {
     return w1 > 0.0f ? rank < k : (w1 < 0.0f ? rank >= k : b1 > 0.0f);
 }
+// Threshold of unit m of an expert of width eh and its rank among the 16 (ties by unit index); a unit with W1 = 0, or beyond
+// eh, has none (+inf, never passed): it is active or not by the sign of b1 alone.  Called by 16 lanes, one per unit.
+struct Unit { float w1, b1, thr; int rank; };
+__device__ __forceinline__ Unit unit_of(const float* __restrict__ W1, const float* __restrict__ B1, int e, int eh, int m) {
+    Unit u;
+    u.w1 = m < eh ? W1[e * eh + m] : 0.0f;
+    u.b1 = m < eh ? B1[e * eh + m] : 0.0f;
+    u.thr = u.w1 != 0.0f ? -u.b1 / u.w1 : __builtin_inff();
+    u.rank = 0;
+#pragma unroll
+    for (int j = 0; j < EH; j++) {
+        const float tj = __shfl(u.thr, j, EH);
+        u.rank += (tj < u.thr || (tj == u.thr && j < m)) ? 1 : 0;
+    }
+    return u;
+}
 
+// One expert per wave.
+__global__ __launch_bounds__(64) void k_expert_tables(Sg2Weights W, int eh, float* __restrict__ tables) {
+    const int e = blockIdx.x, lane = threadIdx.x, m = lane & (EH - 1);
+    const Unit u = unit_of(W.w[W_EXP_W1], W.w[W_EXP_B1], e, eh, m);
+    const float w2 = m < eh ? W.w[W_EXP_W2][e * eh + m] : 0.0f;
+    if (lane < EH) tables[e * EH + u.rank] = u.thr;
+    float A = 0.0f, B = W.w[W_EXP_B2][e];
+#pragma unroll
+    for (int j = 0; j < EH; j++) {
+        const float w1j = __shfl(u.w1, j, EH), b1j = __shfl(u.b1, j, EH), w2j = __shfl(w2, j, EH);
+        const int rj = __shfl(u.rank, j, EH);
+        if (unit_active(w1j, b1j, rj, lane)) {        // interval = lane
+            A = sg_fma(w2j, w1j, A);
+            B = sg_fma(w2j, b1j, B);
+        }
+    }
+    if (lane < NBIN) {
+        tables[NE * EH + (e * NBIN + lane) * 2] = A;
+        tables[NE * EH + (e * NBIN + lane) * 2 + 1] = B;
+    }
+}
+
+// Where the elements come from: flat arrays in element order, or (FLAT false) the sorted order a bilevel forward pass left
+// in its workspace (ctx and d_ctx in sorted order too; gradients and sharpness from the sort's arrays, GRU state and
+// cotangent gathered).
 struct ElemArgs {
-    const float *g, *s, *ctx, *gru, *cot;
+    const float *g, *s, *gru, *cot;       // flat only
+    const float* ctx;
     float *smart, *d_ctx, *partials, *gru_out;
+    const float* tables;
     int total;
+    bool normalise;                       // sorted only: the cotangent is -v / |v|, |v| over the tensor (v itself, negated, where |v| <= 1e-12)
     float rescale;
     Sg2Weights W;
 };
 
-__global__ __launch_bounds__(BE_THREADS) void k_bilevel_elem(ElemArgs a) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
-    float* s_ths = lds;                                   // [NE][EH] unit thresholds of every expert, ascending
-    float* s_ab = s_ths + NE * EH;                        // [NE][NBIN][2] the expert as a line A g + B on each interval
-    float* s_bin = s_ab + NE * NBIN * 2;                  // [NE][NBIN][2] sums of w and w g over the elements of each interval
-    float* s_gkey = s_bin + NE * NBIN * 2;                // [2][NH][PK][DM/2]
-    float* s_x = s_gkey + 2 * NH * PK * (DM / 2);         // [256][XW]
-    float* s_d = s_x + BE_THREADS * XW;                   // [256][DW]
-    float* s_rt = s_d + BE_THREADS * DW;                  // [256][RW]
-    float* s_gq = s_rt + BE_THREADS * RW;                 // [NH][8][22] query-matrix gradients of this workgroup
-    unsigned char* s_rank = reinterpret_cast<unsigned char*>(s_gq + NH * N_QHEAD);      // [NE][EH] position of a unit's threshold among its expert's
-    unsigned char* s_kz = s_rank + NE * EH;               // [NE][2] the interval just below / just above g = 0: thresholds < 0, thresholds <= 0
+// LDS accesses of a wave execute in order; this keeps the compiler from moving them across each other where lanes
+// exchange data.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// (the row belongs to this workgroup alone: workgroup scope lets the add run in the L2 next to it)
+__device__ __forceinline__ void bin_add(float* p, float v) { __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 
-    const int tid = threadIdx.x;
-    {
-        const float* __restrict__ W1 = a.W.w[W_EXP_W1];
-        const float* __restrict__ B1 = a.W.w[W_EXP_B1];
-        const float* __restrict__ W2 = a.W.w[W_EXP_W2];
-        const float* __restrict__ B2 = a.W.w[W_EXP_B2];
-        for (int i = tid; i < 2 * NH * PK * (DM / 2); i += BE_THREADS) s_gkey[i] = 0.0f;
-        for (int i = tid; i < NH * N_QHEAD; i += BE_THREADS) s_gq[i] = 0.0f;
-        for (int i = tid; i < NE * NBIN * 2; i += BE_THREADS) s_bin[i] = 0.0f;
-        for (int i = tid; i < BE_THREADS * RW; i += BE_THREADS) s_rt[i] = 0.0f;      // the padding entries stay zero
-        // one lane per expert: thresholds ranked by counting (ties by unit index), then the line of every interval.
-        // A unit with W1 = 0 has no threshold (+inf, never passed): it is active or not by the sign of b1 alone.
-        for (int e = tid; e < NE; e += BE_THREADS) {
-            const float* w1 = W1 + e * EH;
-            const float* b1 = B1 + e * EH;
-            const float* w2 = W2 + e * EH;
-            auto thr = [&](int m) { return w1[m] != 0.0f ? -b1[m] / w1[m] : __builtin_inff(); };
-            int below = 0, upto = 0;
-            for (int m = 0; m < EH; m++) {
-                const float tm = thr(m);
-                below += tm < 0.0f ? 1 : 0;
-                upto += tm <= 0.0f ? 1 : 0;
-                int r = 0;
-                for (int j = 0; j < EH; j++) {
-                    const float tj = thr(j);
-                    r += (tj < tm || (tj == tm && j < m)) ? 1 : 0;
-                }
-                s_rank[e * EH + m] = (unsigned char)r;
-                s_ths[e * EH + r] = tm;
-            }
-            s_kz[2 * e] = (unsigned char)below;
-            s_kz[2 * e + 1] = (unsigned char)upto;
-            for (int k = 0; k < NBIN; k++) {        // interval k: the k lowest thresholds lie below g
-                float A = 0.0f, B = B2[e];
-                for (int m = 0; m < EH; m++) {
-                    if (!unit_active(w1[m], b1[m], (int)s_rank[e * EH + m], k)) continue;
-                    A = sg_fma(w2[m], w1[m], A);
-                    B = sg_fma(w2[m], b1[m], B);
-                }
-                s_ab[(e * NBIN + k) * 2] = A;
-                s_ab[(e * NBIN + k) * 2 + 1] = B;
-            }
-        }
+// how many of an expert's thresholds lie below g
+__device__ __forceinline__ int interval_of(const float* __restrict__ ths, int e, float g) {
+    const float4* t4 = reinterpret_cast<const float4*>(ths + e * EH);
+    int k = 0;
+#pragma unroll
+    for (int q = 0; q < EH / 4; q++) {
+        const float4 t = t4[q];
+        k += (t.x < g ? 1 : 0) + (t.y < g ? 1 : 0) + (t.z < g ? 1 : 0) + (t.w < g ? 1 : 0);
     }
+    return k;
+}
+
+__device__ __forceinline__ void order(float& a, float& b) {
+    const float hi = __builtin_fmaxf(a, b), lo = __builtin_fminf(a, b);
+    a = hi;
+    b = lo;
+}
+// The four best of twelve scores, ties to the lower index, in index order, with the softmax of 10 x score over them.  A
+// selection network gives the fourth best value and with it the set; scratch (12 floats of the lane's own) turns an index
+// into its score.
+__device__ __forceinline__ void best_four(const float (&sc)[PK], float* scratch, int (&idx)[TOPK], float (&wgt)[TOPK]) {
+    float v[PK];
+#pragma unroll
+    for (int q = 0; q < PK; q++) { v[q] = sc[q]; scratch[q] = sc[q]; }
+#pragma unroll
+    for (int b = 0; b < PK; b += 4) {
+        order(v[b], v[b + 1]); order(v[b + 2], v[b + 3]);
+        order(v[b], v[b + 2]); order(v[b + 1], v[b + 3]);
+        order(v[b + 1], v[b + 2]);
+    }
+    const float best = __builtin_fmaxf(__builtin_fmaxf(v[0], v[4]), v[8]);
+    float c[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) c[k] = __builtin_fmaxf(v[k], v[7 - k]);
+    order(c[0], c[2]); order(c[1], c[3]); order(c[0], c[1]); order(c[2], c[3]);
+    float fourth = __builtin_fmaxf(c[0], v[11]);
+#pragma unroll
+    for (int k = 1; k < 4; k++) fourth = __builtin_fminf(fourth, __builtin_fmaxf(c[k], v[11 - k]));
+    unsigned set = 0u;                       // bit PK-1-q: score q is among them
+#pragma unroll
+    for (int q = 0; q < PK; q++) set = set + set + (sc[q] >= fourth ? 1u : 0u);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(__popc(set) != TOPK) != 0, 0)) {
+        // ties at the border go to the lower indices; scores that do not compare (NaN) leave the set short
+        for (int q = PK - 1; q >= 0 && __popc(set) > TOPK; q--)
+            if (scratch[q] == fourth) set &= ~(1u << (PK - 1 - q));
+        for (int q = 0; q < PK && __popc(set) < TOPK; q++) set |= 1u << (PK - 1 - q);
+    }
+    float den = 0.0f;
+#pragma unroll
+    for (int k = 0; k < TOPK; k++) {
+        const int lead = __builtin_clz(set);          // set is never empty here
+        idx[k] = lead - (32 - PK);
+        set &= ~(0x80000000u >> lead);
+        wgt[k] = sg_exp(10.0f * (scratch[idx[k]] - best));
+        den += wgt[k];
+    }
+    const float inv = 1.0f / den;
+#pragma unroll
+    for (int k = 0; k < TOPK; k++) wgt[k] *= inv;
+}
+
+template <bool FLAT>
+__global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_bilevel_elem(ElemArgs a, Plan pl) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float* const s_keys = lds;                                        // [2][NH][PK][DM/2]
+    float* const s_x = lds + KEY_FLOATS + wave * WAVE_FLOATS;         // [64][XW]
+    float* const s_r = s_x + 64 * XW;
+    float4* const s_tab = reinterpret_cast<float4*>(s_r + R_FLOATS);  // [2][NE]: g > 0, g <= 0
+    float* const bins = a.partials + (size_t)blockIdx.x * ROW_FLOATS;
+    const float* __restrict__ ths = a.tables;
+    const float* __restrict__ lines = a.tables + NE * EH;
+
+    for (int i = tid; i < N_BINS; i += BE_THREADS) bins[i] = 0.0f;
+    for (int i = tid; i < KEY_FLOATS; i += BE_THREADS) s_keys[i] = i < KEY_FLOATS / 2 ? a.W.w[W_KEYS_A][i] : a.W.w[W_KEYS_B][i - KEY_FLOATS / 2];
+    for (int i = lane; i < 64 * XW + R_FLOATS; i += 64) s_x[i] = 0.0f;     // rows are read whole: no NaN may lie in what was never written
+    for (int i = lane; i < 2 * NE; i += 64) s_tab[i] = make_float4(0.0f, 0.0f, __builtin_inff(), -__builtin_inff());
     __syncthreads();
 
     const sg::cfloat_p Wz = sg::as_const(a.W.w[W_GRU_WZ]), bz = sg::as_const(a.W.w[W_GRU_BZ]);
@@ -156,53 +242,138 @@ __global__ __launch_bounds__(BE_THREADS) void k_bilevel_elem(ElemArgs a) {
     const sg::cfloat_p Wq = sg::as_const(a.W.w[W_PEER_Q]);
     const sg::cfloat_p KA = sg::as_const(a.W.w[W_KEYS_A]), KB = sg::as_const(a.W.w[W_KEYS_B]);
 
-    // the lane's entries of the GRU gradients (sums kept in registers) and of a head's query matrix (summed per
-    // tile and head, then added to s_gq)
-    int gdcol[GRU_PER_LANE], gxcol[GRU_PER_LANE], qdcol[Q_PER_LANE], qxcol[Q_PER_LANE];
-    float gsum[GRU_PER_LANE];
-#pragma unroll
-    for (int q = 0; q < GRU_PER_LANE; q++) {
-        gdcol[q] = 0; gxcol[q] = 0; gsum[q] = 0.0f;
-        if (tid + q * BE_THREADS < N_GRU) gru_entry(tid + q * BE_THREADS, &gdcol[q], &gxcol[q]);
-    }
-#pragma unroll
-    for (int q = 0; q < Q_PER_LANE; q++) {
-        qdcol[q] = 0; qxcol[q] = 0;
-        if (tid + q * BE_THREADS < N_QHEAD) query_entry(tid + q * BE_THREADS, &qdcol[q], &qxcol[q]);
-    }
+    const int li = lane & 15, lk = lane >> 4;             // operand roles of the 16 x 16 x 4 instructions: row / column, element of the step
+    // accumulators.  Register v of a 16 x 16 one: row 4 (lane / 16) + v, column lane % 16; of a 4 x 4 x 16 one: block lane / 4, row v, column lane % 4
+    const be_f32x4 zero4 = be_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    be_f32x4 cen[4] = {zero4, zero4, zero4, zero4};       // outer products of the routing weights: w for g > 0, w for g <= 0, w g for g > 0, for g <= 0
+    be_f32x4 qacc[2][2] = {{zero4, zero4}, {zero4, zero4}};       // d query of two heads (x) x: columns 0..15, 16..31
+    be_f32x4 gacc[2] = {zero4, zero4};
+    be_f32x4 kacc[NH] = {zero4, zero4, zero4, zero4};     // blocks 0..5 (even elements) and 6..11 (odd): first sub-key rows 0-3, 4-7, 8-11, second
+    const int kb = (lane >> 2) % 12, kb6 = kb % 6;
+    const int key_a = (kb / 6) * KW + kb6 * 4 + (lane & 3), key_b = (kb / 6) * KW + 24 + (kb6 / 3) * 4 + (lane & 3);
 
-    // near-zero expert sums of this wave (the heads share the experts): sum of w for g > 0, for g <= 0, sum of w g for
-    // g > 0, for g <= 0, each a 16 x 16 (first index x second index) accumulator of the matrix instruction
-    be_f32x4 cen[4];
+    // the four experts whose sums this lane holds in cen: first index 4 lk + v, second index li
+    const bool owner = lane < 48 && li < PK;
+    float x_held = -1.0f;                                 // reference magnitude of the lines in s_tab (< 0: none yet)
+    auto reference = [](float x, int neg) { return neg ? -x : __builtin_fmaxf(x, 1.40129846e-45f); };      // (+0 stands for the interval just above zero)
+    auto flush = [&](int v, int neg) {
+        const int e = (4 * lk + v) * PK + li;
+        float* b = bins + 2 * (e * NBIN + interval_of(ths, e, reference(x_held, neg)));
+        bin_add(b, cen[neg][v]);
+        bin_add(b + 1, cen[2 + neg][v]);
+        cen[neg][v] = 0.0f;
+        cen[2 + neg][v] = 0.0f;
+    };
+    auto move_reference = [&](float x) {
+        bool stale = false;
+        if (owner) {
 #pragma unroll
-    for (int q = 0; q < 4; q++) cen[q] = be_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int tiles = (a.total + BE_THREADS - 1) / BE_THREADS;
-    const float kscale = a.rescale / (float)NH;
-    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        // every lane runs the element code (the passes over the tile need whole workgroups): lanes past the end redo
-        // the last element with a zero cotangent, which zeroes everything they add, and store nothing
-        const bool valid = tile * BE_THREADS + tid < a.total;
-        const int i = valid ? tile * BE_THREADS + tid : a.total - 1;
-        float* xrow = s_x + tid * XW;
-        float* drow = s_d + tid * DW;
-        float* rtrow = s_rt + tid * RW;
-        {
-            const float g = a.g[i], s = a.s[i], cot = valid ? a.cot[i] : 0.0f;
-            float cf[DM], cb[DM], h[GH];
-            {
-                const float4* pf = reinterpret_cast<const float4*>(a.ctx + (size_t)i * DM);
-                const float4* pb = reinterpret_cast<const float4*>(a.ctx + ((size_t)a.total + i) * DM);
-                const float4 a0 = pf[0], a1 = pf[1], b0 = pb[0], b1 = pb[1];
-                cf[0] = a0.x; cf[1] = a0.y; cf[2] = a0.z; cf[3] = a0.w; cf[4] = a1.x; cf[5] = a1.y; cf[6] = a1.z; cf[7] = a1.w;
-                cb[0] = b0.x; cb[1] = b0.y; cb[2] = b0.z; cb[3] = b0.w; cb[4] = b1.x; cb[5] = b1.y; cb[6] = b1.z; cb[7] = b1.w;
-                const float4 h4 = reinterpret_cast<const float4*>(a.gru)[i];
-                h[0] = h4.x; h[1] = h4.y; h[2] = h4.z; h[3] = h4.w;
+            for (int q = 0; q < 8; q++) {
+                const float4 t = s_tab[(q & 1) * NE + (4 * lk + (q >> 1)) * PK + li];
+                const float r = reference(x, q & 1);
+                stale = stale || !(t.z < r && r <= t.w);
             }
-            // (a zero the compiler cannot see through where the wave-uniform weights are used keeps their scalar loads there;
-            //  held across the whole element they are spilled into vector-register lanes and read back, 3000 instructions)
-            const int zo_gf = sg::opaque_zero();
-            // ---- GRU forward
-            float zg[GH], rg[GH], cand[GH], hn[GH];
+        }
+        if (__builtin_amdgcn_ballot_w64(stale) != 0) {
+            if (stale) {
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    const int e = (4 * lk + (q >> 1)) * PK + li;
+                    float4* rec = s_tab + (q & 1) * NE + e;
+                    const float r = reference(x, q & 1);
+                    const float4 t = *rec;
+                    if (t.z < r && r <= t.w) continue;
+                    if (x_held >= 0.0f) flush(q >> 1, q & 1);
+                    const int k = interval_of(ths, e, r);
+                    const float2 ab = reinterpret_cast<const float2*>(lines)[e * NBIN + k];
+                    *rec = make_float4(ab.x, ab.y, k > 0 ? ths[e * EH + k - 1] : -__builtin_inff(), k < EH ? ths[e * EH + k] : __builtin_inff());
+                }
+            }
+        }
+        x_held = x;
+        wave_sync();
+    };
+
+    const int ntiles = FLAT ? (a.total + 63) / 64 : pl.elem_tiles * (ELEM_TILE / 64);
+    const int nwaves = (int)gridDim.x * BE_WAVES, wv = (int)blockIdx.x * BE_WAVES + wave;
+    const int tile0 = (int)((int64_t)ntiles * wv / nwaves), tile1 = (int)((int64_t)ntiles * (wv + 1) / nwaves);
+    const float kscale = a.rescale / (float)NH;
+    sg::Seg seg = {-1, 0, 0};
+    float cot_norm = 0.0f;
+    for (int tile = tile0; tile < tile1; tile++) {
+        // every lane runs the element code (the wave works on whole tiles): lanes past the end redo the last element with a
+        // zero cotangent, which zeroes everything they add, and store nothing
+        bool valid;
+        int at;                              // where ctx and d_ctx rows lie
+        int out_at;                          // where smart goes
+        float g, s, cot;
+        float4 h4;
+        if (FLAT) {
+            valid = tile * 64 + lane < a.total;
+            at = out_at = valid ? tile * 64 + lane : a.total - 1;
+            g = a.g[at]; s = a.s[at]; cot = valid ? a.cot[at] : 0.0f;
+            h4 = reinterpret_cast<const float4*>(a.gru)[at];
+            if (x_held < 0.0f) move_reference(0.0f);
+        } else {
+            const int et = tile / (ELEM_TILE / 64);
+            if (et >= seg.end) {
+                seg = sg::find_seg(sg::as_const(pl.elem_tile_prefix), pl.P, et);
+                if (a.normalise) {           // |v| of the tensor from its norm tiles
+                    double part = 0.0;
+                    for (int k = pl.norm_tile_prefix[seg.i] + lane; k < pl.norm_tile_prefix[seg.i + 1]; k += 64) part += pl.norm_partials[k];
+#pragma unroll
+                    for (int d = 32; d >= 1; d >>= 1) part += __shfl_xor(part, d, 64);
+                    cot_norm = (float)sqrt(part);
+                }
+            }
+            const TensorDev& T = pl.tensors[seg.i];
+            const int start = (et - seg.first) * ELEM_TILE + (tile % (ELEM_TILE / 64)) * 64;
+            const int cnt = T.numel - start;
+            if (cnt <= 0) continue;          // an empty rest of a tensor's last tile
+            valid = lane < cnt;
+            at = T.off + start + (valid ? lane : cnt - 1);
+            const int32_t val = pl.vals[0][at];
+            const uint32_t key = pl.keys[0][at];
+            const int orig = min(val & 0x7fffffff, T.numel - 1);
+            out_at = T.off + orig;
+            // the sort's values, except where it put 0 for an entry that is not finite: those stay what they are
+            g = sg_i2f((int32_t)key | (val & (int32_t)0x80000000));
+            if (key == 0u) g = sg::load_elem(T.grad, T.dtype, orig);
+            s = 0.0f;
+            if (pl.sharp_nonzero[seg.i] != 0) {
+                s = pl.ssorted[at];
+                if (s == 0.0f) s = sharp_rounded(T, orig);
+            }
+            cot = sg::load_elem(T.param, T.dtype, orig);
+            if (a.normalise) cot = -(cot_norm > 1e-12f ? cot / cot_norm : cot);
+            cot = valid ? cot : 0.0f;
+            const be_f32x4 hv = ((const SG_GLOBAL be_f32x4*)T.gru)[orig];
+            h4 = make_float4(hv[0], hv[1], hv[2], hv[3]);
+            move_reference(__shfl(sg_abs(g), min(cnt - 1, 32), 64));
+        }
+        float* const xrow = s_x + lane * XW;
+        // rows of the routing weights: positive elements first, padded to whole pairs of steps (eight rows), then the others
+        const unsigned long long pos = __builtin_amdgcn_ballot_w64(g > 0.0f);
+        const int npos = __popcll(pos), npos8 = (npos + 7) >> 3, nneg8 = (64 - npos + 7) >> 3;
+        const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(pos >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)pos, 0u));      // positive elements in lower lanes
+        const int slot = g > 0.0f ? before : 8 * npos8 + (lane - before);
+        // ... of which lane 0..7 / 8..15 clears one
+        const int pad = (lane < 8 ? npos : 8 * npos8 + (64 - npos) - 8) + lane, pad_end = lane < 8 ? 8 * npos8 : lane < 16 ? 8 * (npos8 + nneg8) : 0;
+
+        float cf[DM], cb[DM], h[GH] = {h4.x, h4.y, h4.z, h4.w};
+        {
+            const float4* pf = reinterpret_cast<const float4*>(a.ctx + (size_t)at * DM);
+            const float4* pb = reinterpret_cast<const float4*>(a.ctx + ((size_t)a.total + at) * DM);
+            const float4 a0 = pf[0], a1 = pf[1], b0 = pb[0], b1 = pb[1];
+            cf[0] = a0.x; cf[1] = a0.y; cf[2] = a0.z; cf[3] = a0.w; cf[4] = a1.x; cf[5] = a1.y; cf[6] = a1.z; cf[7] = a1.w;
+            cb[0] = b0.x; cb[1] = b0.y; cb[2] = b0.z; cb[3] = b0.w; cb[4] = b1.x; cb[5] = b1.y; cb[6] = b1.z; cb[7] = b1.w;
+        }
+        // (a zero the compiler cannot see through where the wave-uniform weights are used keeps their scalar loads there;
+        //  held across the whole element they are spilled into vector-register lanes and read back, 3000 instructions)
+        const int zo_gf = sg::opaque_zero();
+        // ---- GRU forward
+        float zg[GH], rg[GH], cand[GH], hn[GH];
+        {
 #pragma unroll
             for (int j = 0; j < GH; j++) {
                 const sg::cfloat_p wz = Wz + j * GRL + zo_gf, wr = Wr + j * GRL + zo_gf;
@@ -232,344 +403,414 @@ __global__ __launch_bounds__(BE_THREADS) void k_bilevel_elem(ElemArgs a) {
                 cand[j] = sg_tanh(v);
                 hn[j] = sg_fma(zg[j], cand[j], (1.0f - zg[j]) * h[j]);
             }
-            if (valid && a.gru_out != nullptr) reinterpret_cast<float4*>(a.gru_out)[i] = make_float4(hn[0], hn[1], hn[2], hn[3]);
-            xrow[X_G] = g; xrow[X_S] = s; xrow[X_ONE] = 1.0f;
+        }
+        if (FLAT && valid && a.gru_out != nullptr) reinterpret_cast<float4*>(a.gru_out)[at] = make_float4(hn[0], hn[1], hn[2], hn[3]);
+        xrow[X_G] = g; xrow[X_S] = s; xrow[X_ONE] = 1.0f;
 #pragma unroll
-            for (int q = 0; q < DM; q++) { xrow[X_CF + q] = cf[q]; xrow[X_CB + q] = cb[q]; }
+        for (int q = 0; q < DM; q++) { xrow[X_CF + q] = cf[q]; xrow[X_CB + q] = cb[q]; }
 #pragma unroll
-            for (int q = 0; q < GH; q++) { xrow[X_H + q] = h[q]; xrow[X_RH + q] = rg[q] * h[q]; xrow[X_HN + q] = hn[q]; }
+        for (int q = 0; q < GH; q++) { xrow[X_H + q] = h[q]; xrow[X_HN + q] = hn[q]; }
 
-            // ---- heads: forward, then at once the head's backward
-            float total = 0.0f;
-            float dhn[GH] = {0.f, 0.f, 0.f, 0.f}, dcf[DM], dcb[DM];
+        // ---- heads: forward, then at once the head's backward
+        float total = 0.0f;
+        float dhn[GH] = {0.f, 0.f, 0.f, 0.f}, dcf[DM], dcb[DM], dq_even[DM];
 #pragma unroll
-            for (int q = 0; q < DM; q++) { dcf[q] = 0.0f; dcb[q] = 0.0f; }
-            const float kk = cot * kscale;                 // d loss / d head output
+        for (int q = 0; q < DM; q++) { dcf[q] = 0.0f; dcb[q] = 0.0f; dq_even[q] = 0.0f; }
+        const float kk = cot * kscale;                 // d loss / d head output
+        const int side = g > 0.0f ? 0 : NE;
 #pragma unroll 1
-            for (int hh = 0; hh < NH; hh++) {
-                const int zo_q = sg::opaque_zero();
-                float query[DM];
+        for (int hh = 0; hh < NH; hh++) {
+            const int zo_q = sg::opaque_zero();
+            float query[DM];
 #pragma unroll
-                for (int dd = 0; dd < DM; dd++) {
-                    const sg::cfloat_p qr = Wq + (hh * DM + dd) * PIN + zo_q;
-                    float v = 0.0f;
+            for (int dd = 0; dd < DM; dd++) {
+                const sg::cfloat_p qr = Wq + (hh * DM + dd) * PIN + zo_q;
+                float v = 0.0f;
 #pragma unroll
-                    for (int q = 0; q < GH; q++) v = sg_fma(qr[q], hn[q], v);
+                for (int q = 0; q < GH; q++) v = sg_fma(qr[q], hn[q], v);
 #pragma unroll
-                    for (int q = 0; q < DM; q++) v = sg_fma(qr[GH + q], cf[q], v);
+                for (int q = 0; q < DM; q++) v = sg_fma(qr[GH + q], cf[q], v);
 #pragma unroll
-                    for (int q = 0; q < DM; q++) v = sg_fma(qr[GH + DM + q], cb[q], v);
-                    v = sg_fma(qr[GH + 2 * DM], g, v);
-                    v = sg_fma(qr[GH + 2 * DM + 1], s, v);
-                    query[dd] = v;
+                for (int q = 0; q < DM; q++) v = sg_fma(qr[GH + DM + q], cb[q], v);
+                v = sg_fma(qr[GH + 2 * DM], g, v);
+                v = sg_fma(qr[GH + 2 * DM + 1], s, v);
+                query[dd] = v;
+            }
+            int idx[2][TOPK];
+            float wgt[2][TOPK];
+#pragma unroll
+            for (int hf = 0; hf < 2; hf++) {
+                const sg::cfloat_p keys = (hf ? KB : KA) + hh * PK * (DM / 2) + zo_q;
+                float sc[PK];
+#pragma unroll
+                for (int q = 0; q < PK; q++) {
+                    float dot = 0.0f;
+#pragma unroll
+                    for (int dd = 0; dd < DM / 2; dd++) dot = sg_fma(query[hf * (DM / 2) + dd], keys[q * (DM / 2) + dd], dot);
+                    sc[q] = dot;
                 }
-                int idx[2][TOPK];
-                float wgt[2][TOPK];
+                best_four(sc, s_r + lane * CW + hf * PK, idx[hf], wgt[hf]);
+            }
+            wave_sync();
+            // ---- experts: the line of each at this element's side of zero, where its interval holds g
+            float ra[TOPK] = {0.f, 0.f, 0.f, 0.f}, rb[TOPK] = {0.f, 0.f, 0.f, 0.f};
+            unsigned other = 0u;                     // picks whose interval is another one
 #pragma unroll
-                for (int hf = 0; hf < 2; hf++) {
-                    const sg::cfloat_p keys = (hf ? KB : KA) + hh * PK * (DM / 2) + zo_q;
-                    float sc[PK];
+            for (int ia = 0; ia < TOPK; ia++) {
+                const float4* ta = s_tab + side + idx[0][ia] * PK;
 #pragma unroll
-                    for (int q = 0; q < PK; q++) {
-                        float dot = 0.0f;
-#pragma unroll
-                        for (int dd = 0; dd < DM / 2; dd++) dot = sg_fma(query[hf * (DM / 2) + dd], keys[q * (DM / 2) + dd], dot);
-                        sc[q] = dot;
-                    }
-                    // four best scores, ties to the lower index; softmax of 10 x score over them
-                    float val[TOPK];
-                    unsigned taken = 0u;
-#pragma unroll
-                    for (int k = 0; k < TOPK; k++) {
-                        int bi = 0;
-                        float bs = -3.0e38f;
-#pragma unroll
-                        for (int q = 0; q < PK; q++) {
-                            const bool free_ = ((taken >> q) & 1u) == 0u;
-                            if (free_ && sc[q] > bs) { bs = sc[q]; bi = q; }
-                        }
-                        taken |= 1u << bi;
-                        idx[hf][k] = bi;
-                        val[k] = bs;
-                    }
-                    float den = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < TOPK; k++) { wgt[hf][k] = sg_exp(10.0f * (val[k] - val[0])); den += wgt[hf][k]; }
-                    const float inv = 1.0f / den;
-#pragma unroll
-                    for (int k = 0; k < TOPK; k++) wgt[hf][k] *= inv;
+                for (int ib = 0; ib < TOPK; ib++) {
+                    const float4 t = ta[idx[1][ib]];
+                    const bool in = t.z < g && g <= t.w;
+                    const float out = in ? sg_fma(t.x, g, t.y) : 0.0f;
+                    other |= in ? 0u : 1u << (ia * TOPK + ib);
+                    ra[ia] = sg_fma(wgt[1][ib], out, ra[ia]);
+                    rb[ib] = sg_fma(wgt[0][ia], out, rb[ib]);
                 }
-                // experts: outputs per lane; each expert's bin of this element's activation pattern takes (w, w g)
-                float ra[TOPK] = {0.f, 0.f, 0.f, 0.f}, rb[TOPK] = {0.f, 0.f, 0.f, 0.f};
-                float head_out = 0.0f;
-#pragma unroll 1
-                for (int ia = 0; ia < TOPK; ia++) {
-                    // the unrolled selects keep idx/wgt in registers (a dynamic index would send them to scratch); the four
-                    // second indices are unrolled, so that the record reads of four experts are in flight together
+            }
+            if (!valid) other = 0u;
+            while (__builtin_amdgcn_ballot_w64(other != 0u) != 0) {
+                if (other != 0u) {
+                    const int pick = __builtin_ctz(other), ia = pick / TOPK, ib = pick % TOPK;
+                    other &= other - 1u;
+                    // (selects keep idx and wgt in registers: a dynamic index would send them to scratch)
                     const int ea = ia == 0 ? idx[0][0] : ia == 1 ? idx[0][1] : ia == 2 ? idx[0][2] : idx[0][3];
+                    const int eb = ib == 0 ? idx[1][0] : ib == 1 ? idx[1][1] : ib == 2 ? idx[1][2] : idx[1][3];
                     const float wa = ia == 0 ? wgt[0][0] : ia == 1 ? wgt[0][1] : ia == 2 ? wgt[0][2] : wgt[0][3];
-                    float ra_sum = 0.0f;
-                    int xbin[TOPK], xcen[TOPK];         // a pick outside the interval next to zero: its bin and that interval's, else -1
-                    float xw[TOPK];
-#pragma unroll
-                    for (int ib = 0; ib < TOPK; ib++) {
-                        const float wb = wgt[1][ib];
-                        int e = ea * PK + idx[1][ib];
-                        if (e >= NE) e = NE - 1;
-                        const float* th = s_ths + e * EH;
-                        int k = th[7] < g ? 8 : 0;              // how many of the expert's thresholds lie below g
-                        k += th[k + 3] < g ? 4 : 0;
-                        k += th[k + 1] < g ? 2 : 0;
-                        k += th[k] < g ? 1 : 0;
-                        k += th[k] < g ? 1 : 0;
-                        const int bin = e * NBIN + k;
-                        const float out = sg_fma(s_ab[2 * bin], g, s_ab[2 * bin + 1]);
-                        const int kc = g > 0.0f ? s_kz[2 * e + 1] : s_kz[2 * e];
-                        xbin[ib] = k != kc ? bin : -1;
-                        xcen[ib] = e * NBIN + kc;
-                        xw[ib] = (kk * wa) * wb;
-                        head_out = sg_fma(wa * wb, out, head_out);
-                        ra_sum = sg_fma(wb, out, ra_sum);
-                        rb[ib] = sg_fma(wa, out, rb[ib]);
-                    }
-                    ra[0] += ia == 0 ? ra_sum : 0.0f; ra[1] += ia == 1 ? ra_sum : 0.0f; ra[2] += ia == 2 ? ra_sum : 0.0f; ra[3] += ia == 3 ? ra_sum : 0.0f;
-                    // picks outside the interval next to zero move their share from there to their own bin; the wave skips
-                    // this when none of its lanes has one (so the four interval searches above stay one straight block)
-                    if (__builtin_amdgcn_ballot_w64(((xbin[0] & xbin[1]) & (xbin[2] & xbin[3])) >= 0) != 0) {
-#pragma unroll
-                        for (int ib = 0; ib < TOPK; ib++) {
-                            if (xbin[ib] < 0) continue;
-                            atomicAdd(&s_bin[2 * xbin[ib]], xw[ib]);
-                            atomicAdd(&s_bin[2 * xbin[ib] + 1], xw[ib] * g);
-                            atomicAdd(&s_bin[2 * xcen[ib]], -xw[ib]);
-                            atomicAdd(&s_bin[2 * xcen[ib] + 1], -(xw[ib] * g));
-                        }
-                    }
+                    const float wb = ib == 0 ? wgt[1][0] : ib == 1 ? wgt[1][1] : ib == 2 ? wgt[1][2] : wgt[1][3];
+                    const int e = ea * PK + eb;
+                    const int k = interval_of(ths, e, g), kr = interval_of(ths, e, reference(x_held, side != 0));
+                    const float2 ab = reinterpret_cast<const float2*>(lines)[e * NBIN + k];
+                    const float out = sg_fma(ab.x, g, ab.y);
+                    const float pa = wb * out, pb = wa * out;
+                    ra[0] += ia == 0 ? pa : 0.0f; ra[1] += ia == 1 ? pa : 0.0f; ra[2] += ia == 2 ? pa : 0.0f; ra[3] += ia == 3 ? pa : 0.0f;
+                    rb[0] += ib == 0 ? pb : 0.0f; rb[1] += ib == 1 ? pb : 0.0f; rb[2] += ib == 2 ? pb : 0.0f; rb[3] += ib == 3 ? pb : 0.0f;
+                    const float w = (kk * wa) * wb;
+                    float* b = bins + 2 * e * NBIN;
+                    bin_add(b + 2 * k, w);
+                    bin_add(b + 2 * k + 1, w * g);
+                    bin_add(b + 2 * kr, -w);
+                    bin_add(b + 2 * kr + 1, -(w * g));
                 }
-                // near-zero expert sums: this wave's 64 elements, four a step
+            }
+            float head_out = 0.0f;
 #pragma unroll
-                for (int k = 0; k < PK; k++) { rtrow[k] = 0.0f; rtrow[RH + k] = 0.0f; }
+            for (int ia = 0; ia < TOPK; ia++) head_out = sg_fma(wgt[0][ia], ra[ia], head_out);
+            total += head_out;
+            // ---- sums of the routing weights over this tile's elements, four a step
+            {
+                float* const crow = s_r + slot * CW;
+#pragma unroll
+                for (int k = 0; k < 2 * PK; k++) crow[k] = 0.0f;
+                crow[2 * PK] = g;
+                if (pad < pad_end) {
+#pragma unroll
+                    for (int k = 0; k < CW; k++) s_r[pad * CW + k] = 0.0f;
+                }
 #pragma unroll
                 for (int k = 0; k < TOPK; k++) {
-                    rtrow[idx[0][k]] = kk * wgt[0][k];
-                    rtrow[RH + idx[1][k]] = wgt[1][k];
+                    crow[idx[0][k]] = kk * wgt[0][k];
+                    crow[PK + idx[1][k]] = wgt[1][k];
                 }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                {
-                    const int li = tid & 15, el0 = (tid & ~63) + ((tid & 63) >> 4);
+                wave_sync();
+                // two steps at a time, the next two on their way
+                const float* row = s_r + lk * CW;
+                float av[2], bv[2], gv[2];
+                auto fetch = [&]() {
+#pragma unroll
+                    for (int u = 0; u < 2; u++) { av[u] = row[4 * u * CW + li]; bv[u] = row[4 * u * CW + PK + li]; gv[u] = row[4 * u * CW + 2 * PK]; }
+                    row += 8 * CW;
+                };
+                auto sums = [&](int steps, be_f32x4& acc, be_f32x4& acc_g) {
+                    for (int t = 0; t < steps; t++) {
+                        const float a0 = av[0], b0 = bv[0], g0 = gv[0], a1 = av[1], b1 = bv[1], g1 = gv[1];
+                        fetch();
+                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b0, acc, 0, 0, 0);
+                        acc_g = __builtin_amdgcn_mfma_f32_16x16x4f32(a0 * g0, b0, acc_g, 0, 0, 0);
+                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, acc, 0, 0, 0);
+                        acc_g = __builtin_amdgcn_mfma_f32_16x16x4f32(a1 * g1, b1, acc_g, 0, 0, 0);
+                    }
+                };
+                fetch();
+                sums(npos8, cen[0], cen[2]);
+                sums(nneg8, cen[1], cen[3]);
+                wave_sync();
+            }
+            // ---- routing backward: softmax, scores, query
+            float dq[DM], dv[2][TOPK];
+#pragma unroll
+            for (int hf = 0; hf < 2; hf++) {
+                const float4* keys = reinterpret_cast<const float4*>(s_keys) + (hf * NH + hh) * PK;
+                float mean = 0.0f;
+#pragma unroll
+                for (int k = 0; k < TOPK; k++) mean = sg_fma(wgt[hf][k], kk * (hf ? rb[k] : ra[k]), mean);
+                float d0 = 0.0f, d1 = 0.0f, d2 = 0.0f, d3 = 0.0f;
+#pragma unroll
+                for (int k = 0; k < TOPK; k++) {
+                    const float4 key = keys[idx[hf][k]];
+                    dv[hf][k] = 10.0f * wgt[hf][k] * (kk * (hf ? rb[k] : ra[k]) - mean);
+                    d0 = sg_fma(dv[hf][k], key.x, d0);
+                    d1 = sg_fma(dv[hf][k], key.y, d1);
+                    d2 = sg_fma(dv[hf][k], key.z, d2);
+                    d3 = sg_fma(dv[hf][k], key.w, d3);
+                }
+                dq[4 * hf] = d0; dq[4 * hf + 1] = d1; dq[4 * hf + 2] = d2; dq[4 * hf + 3] = d3;
+            }
+            const int zo_rb = sg::opaque_zero();
+#pragma unroll
+            for (int dd = 0; dd < DM; dd++) {
+                const sg::cfloat_p qr = Wq + (hh * DM + dd) * PIN + zo_rb;
+#pragma unroll
+                for (int q = 0; q < GH; q++) dhn[q] = sg_fma(qr[q], dq[dd], dhn[q]);
+#pragma unroll
+                for (int q = 0; q < DM; q++) dcf[q] = sg_fma(qr[GH + q], dq[dd], dcf[q]);
+#pragma unroll
+                for (int q = 0; q < DM; q++) dcb[q] = sg_fma(qr[GH + DM + q], dq[dd], dcb[q]);
+            }
+            // ---- product-key gradients, d score (x) query half, two elements a step
+            {
+                float* const krow = s_r + lane * KW;
+#pragma unroll
+                for (int k = 0; k < 2 * PK; k++) krow[k] = 0.0f;
+#pragma unroll
+                for (int k = 0; k < TOPK; k++) {
+                    krow[idx[0][k]] = dv[0][k];
+                    krow[PK + idx[1][k]] = dv[1][k];
+                }
+#pragma unroll
+                for (int dd = 0; dd < DM; dd++) krow[2 * PK + dd] = query[dd];
+                wave_sync();
+                auto key_sums = [&](be_f32x4& acc) {
+#pragma unroll 8
+                    for (int t = 0; t < 32; t++)
+                        acc = __builtin_amdgcn_mfma_f32_4x4x1f32(s_r[2 * t * KW + key_a], s_r[2 * t * KW + key_b], acc, 0, 0, 0);
+                };
+                if (hh == 0) key_sums(kacc[0]);
+                else if (hh == 1) key_sums(kacc[1]);
+                else if (hh == 2) key_sums(kacc[2]);
+                else key_sums(kacc[3]);
+                wave_sync();
+            }
+            // ---- query-matrix gradients, d query (x) query input, two heads at a time
+            if ((hh & 1) == 0) {
+#pragma unroll
+                for (int dd = 0; dd < DM; dd++) dq_even[dd] = dq[dd];
+            } else {
+                float* const drow = s_r + lane * DW;
+#pragma unroll
+                for (int dd = 0; dd < DM; dd++) { drow[dd] = dq_even[dd]; drow[DM + dd] = dq[dd]; }
+                wave_sync();
+                auto query_sums = [&](be_f32x4 (&acc)[2]) {
 #pragma unroll 4
                     for (int t = 0; t < 16; t++) {
-                        const int el = el0 + 4 * t;
-                        const float av = s_rt[el * RW + li], bv = s_rt[el * RW + RH + li], gv = s_x[el * XW + X_G];
-                        const float ap = gv > 0.0f ? av : 0.0f, an = gv > 0.0f ? 0.0f : av;
-                        cen[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ap, bv, cen[0], 0, 0, 0);
-                        cen[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(an, bv, cen[1], 0, 0, 0);
-                        cen[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(ap * gv, bv, cen[2], 0, 0, 0);
-                        cen[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(an * gv, bv, cen[3], 0, 0, 0);
+                        const float av = s_r[(4 * t + lk) * DW + li];
+                        const float* xr = s_x + (4 * t + lk) * XW + li;
+                        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, xr[0], acc[0], 0, 0, 0);
+                        acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, xr[16], acc[1], 0, 0, 0);
                     }
-                }
-                total += head_out;
-                const int zo_rb = sg::opaque_zero();
-                // routing backward: softmax, scores, query (the product keys' own gradients: see the end of the head)
-                float dq[DM], dv[2][TOPK];
-#pragma unroll
-                for (int hf = 0; hf < 2; hf++) {
-                    const sg::cfloat_p keys = (hf ? KB : KA) + hh * PK * (DM / 2) + zo_rb;
-                    float mean = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < TOPK; k++) mean = sg_fma(wgt[hf][k], kk * (hf ? rb[k] : ra[k]), mean);
-#pragma unroll
-                    for (int dd = 0; dd < DM / 2; dd++) dq[hf * (DM / 2) + dd] = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < TOPK; k++) {
-                        dv[hf][k] = 10.0f * wgt[hf][k] * (kk * (hf ? rb[k] : ra[k]) - mean);
-                        const int row = idx[hf][k];
-#pragma unroll
-                        for (int dd = 0; dd < DM / 2; dd++)
-                            dq[hf * (DM / 2) + dd] = sg_fma(dv[hf][k], keys[row * (DM / 2) + dd], dq[hf * (DM / 2) + dd]);
-                    }
-                }
-#pragma unroll
-                for (int dd = 0; dd < DM; dd++) {
-                    drow[dd] = dq[dd];
-                    const sg::cfloat_p qr = Wq + (hh * DM + dd) * PIN + zo_rb;
-#pragma unroll
-                    for (int q = 0; q < GH; q++) dhn[q] = sg_fma(qr[q], dq[dd], dhn[q]);
-#pragma unroll
-                    for (int q = 0; q < DM; q++) dcf[q] = sg_fma(qr[GH + q], dq[dd], dcf[q]);
-#pragma unroll
-                    for (int q = 0; q < DM; q++) dcb[q] = sg_fma(qr[GH + DM + q], dq[dd], dcb[q]);
-                }
-                __syncthreads();
-                // this head's query-matrix gradients: d query (x) query input over the tile's elements
-                {
-                    float qs[Q_PER_LANE];
-#pragma unroll
-                    for (int q = 0; q < Q_PER_LANE; q++) qs[q] = 0.0f;
-#pragma unroll 16
-                    for (int e = 0; e < BE_THREADS; e++) {      // (unrolled: the LDS reads of 16 elements are in flight together)
-#pragma unroll
-                        for (int q = 0; q < Q_PER_LANE; q++) qs[q] = sg_fma(s_d[e * DW + qdcol[q]], s_x[e * XW + qxcol[q]], qs[q]);
-                    }
-#pragma unroll
-                    for (int q = 0; q < Q_PER_LANE; q++)
-                        if (tid + q * BE_THREADS < N_QHEAD) s_gq[hh * N_QHEAD + tid + q * BE_THREADS] += qs[q];      // one owner per entry
-                }
-                __syncthreads();
-                // product-key gradients, d score (x) query half, the same way: the staged rows are free now, so each
-                // lane leaves d score as two 12-vectors (four non-zeros each) and its query; 96 lanes own one entry each
-#pragma unroll
-                for (int k = 0; k < PK; k++) { rtrow[k] = 0.0f; rtrow[RH + k] = 0.0f; }
-#pragma unroll
-                for (int k = 0; k < TOPK; k++) {
-                    rtrow[idx[0][k]] = dv[0][k];
-                    rtrow[RH + idx[1][k]] = dv[1][k];
-                }
-#pragma unroll
-                for (int dd = 0; dd < DM; dd++) drow[dd] = query[dd];
-                __syncthreads();
-                if (tid < 2 * PK * (DM / 2)) {
-                    const int hf = tid / (PK * (DM / 2)), row = (tid / (DM / 2)) % PK, dd = tid % (DM / 2);
-                    float acc = 0.0f;
-#pragma unroll 16
-                    for (int e = 0; e < BE_THREADS; e++) acc = sg_fma(s_rt[e * RW + hf * RH + row], s_d[e * DW + hf * (DM / 2) + dd], acc);
-                    s_gkey[(hf * NH + hh) * PK * (DM / 2) + row * (DM / 2) + dd] += acc;
-                }
-                __syncthreads();
-            }
-            if (valid && a.smart != nullptr) a.smart[i] = sg_fma(a.rescale, total / (float)NH, g);
-
-            const int zo_gb = sg::opaque_zero();
-            // ---- GRU backward
-            float dpz[GH], dpr[GH], dph[GH], drh[GH] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < GH; j++) {
-                dpz[j] = (dhn[j] * (cand[j] - h[j])) * (zg[j] * (1.0f - zg[j]));
-                dph[j] = (dhn[j] * zg[j]) * (1.0f - cand[j] * cand[j]);
-            }
-#pragma unroll
-            for (int j = 0; j < GH; j++) {
-                const sg::cfloat_p wh = Wh + j * GRL + zo_gb;
-#pragma unroll
-                for (int q = 0; q < DM; q++) { dcf[q] = sg_fma(wh[2 + q], dph[j], dcf[q]); dcb[q] = sg_fma(wh[2 + DM + q], dph[j], dcb[q]); }
-#pragma unroll
-                for (int q = 0; q < GH; q++) drh[q] = sg_fma(wh[2 + 2 * DM + q], dph[j], drh[q]);
-            }
-#pragma unroll
-            for (int j = 0; j < GH; j++) dpr[j] = (drh[j] * h[j]) * (rg[j] * (1.0f - rg[j]));
-#pragma unroll
-            for (int j = 0; j < GH; j++) {
-                const sg::cfloat_p wz = Wz + j * GRL + zo_gb, wr = Wr + j * GRL + zo_gb;
-#pragma unroll
-                for (int q = 0; q < DM; q++) {
-                    dcf[q] = sg_fma(wz[2 + q], dpz[j], dcf[q]); dcf[q] = sg_fma(wr[2 + q], dpr[j], dcf[q]);
-                    dcb[q] = sg_fma(wz[2 + DM + q], dpz[j], dcb[q]); dcb[q] = sg_fma(wr[2 + DM + q], dpr[j], dcb[q]);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < GH; j++) { drow[D_Z + j] = dpz[j]; drow[D_R + j] = dpr[j]; drow[D_H + j] = dph[j]; }
-            if (valid) {
-                float4* of = reinterpret_cast<float4*>(a.d_ctx + (size_t)i * DM);
-                float4* ob = reinterpret_cast<float4*>(a.d_ctx + ((size_t)a.total + i) * DM);
-                of[0] = make_float4(dcf[0], dcf[1], dcf[2], dcf[3]); of[1] = make_float4(dcf[4], dcf[5], dcf[6], dcf[7]);
-                ob[0] = make_float4(dcb[0], dcb[1], dcb[2], dcb[3]); ob[1] = make_float4(dcb[4], dcb[5], dcb[6], dcb[7]);
+                };
+                if (hh == 1) query_sums(qacc[0]);
+                else query_sums(qacc[1]);
+                wave_sync();
             }
         }
-        __syncthreads();
-        // ---- GRU gradients: each lane's entries, summed over the tile's elements
-#pragma unroll 16
-        for (int e = 0; e < BE_THREADS; e++) {
+        if (valid && a.smart != nullptr) a.smart[out_at] = sg_fma(a.rescale, total / (float)NH, g);
+
+        const int zo_gb = sg::opaque_zero();
+        // ---- GRU backward
+        float dpz[GH], dpr[GH], dph[GH], drh[GH] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int q = 0; q < GRU_PER_LANE; q++) gsum[q] = sg_fma(s_d[e * DW + gdcol[q]], s_x[e * XW + gxcol[q]], gsum[q]);
+        for (int j = 0; j < GH; j++) {
+            dpz[j] = (dhn[j] * (cand[j] - h[j])) * (zg[j] * (1.0f - zg[j]));
+            dph[j] = (dhn[j] * zg[j]) * (1.0f - cand[j] * cand[j]);
         }
-        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < GH; j++) {
+            const sg::cfloat_p wh = Wh + j * GRL + zo_gb;
+#pragma unroll
+            for (int q = 0; q < DM; q++) { dcf[q] = sg_fma(wh[2 + q], dph[j], dcf[q]); dcb[q] = sg_fma(wh[2 + DM + q], dph[j], dcb[q]); }
+#pragma unroll
+            for (int q = 0; q < GH; q++) drh[q] = sg_fma(wh[2 + 2 * DM + q], dph[j], drh[q]);
+        }
+#pragma unroll
+        for (int j = 0; j < GH; j++) dpr[j] = (drh[j] * h[j]) * (rg[j] * (1.0f - rg[j]));
+#pragma unroll
+        for (int j = 0; j < GH; j++) {
+            const sg::cfloat_p wz = Wz + j * GRL + zo_gb, wr = Wr + j * GRL + zo_gb;
+#pragma unroll
+            for (int q = 0; q < DM; q++) {
+                dcf[q] = sg_fma(wz[2 + q], dpz[j], dcf[q]); dcf[q] = sg_fma(wr[2 + q], dpr[j], dcf[q]);
+                dcb[q] = sg_fma(wz[2 + DM + q], dpz[j], dcb[q]); dcb[q] = sg_fma(wr[2 + DM + q], dpr[j], dcb[q]);
+            }
+        }
+        if (valid) {
+            float4* of = reinterpret_cast<float4*>(a.d_ctx + (size_t)at * DM);
+            float4* ob = reinterpret_cast<float4*>(a.d_ctx + ((size_t)a.total + at) * DM);
+            of[0] = make_float4(dcf[0], dcf[1], dcf[2], dcf[3]); of[1] = make_float4(dcf[4], dcf[5], dcf[6], dcf[7]);
+            ob[0] = make_float4(dcb[0], dcb[1], dcb[2], dcb[3]); ob[1] = make_float4(dcb[4], dcb[5], dcb[6], dcb[7]);
+        }
+        // ---- GRU gradients
+        {
+            float* const drow = s_r + lane * DW;
+#pragma unroll
+            for (int j = 0; j < GH; j++) { drow[j] = dpz[j]; drow[GH + j] = dpr[j]; drow[2 * GH + j] = dph[j]; xrow[X_HN + j] = rg[j] * h[j]; }
+            wave_sync();
+#pragma unroll 4
+            for (int t = 0; t < 16; t++) {
+                const float av = s_r[(4 * t + lk) * DW + li];
+                const float* xr = s_x + (4 * t + lk) * XW + li;
+                gacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, xr[0], gacc[0], 0, 0, 0);
+                gacc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, xr[16], gacc[1], 0, 0, 0);
+            }
+            wave_sync();
+        }
     }
 
-    // ---- this workgroup's sums -> its row of the partials buffer
-    float* out = a.partials + (size_t)blockIdx.x * N_GRADS;
-#pragma unroll
-    for (int q = 0; q < GRU_PER_LANE; q++) {
-        const int o = tid + q * BE_THREADS;
-        if (o < N_GRU) out[o] = gsum[q];
-    }
-    __syncthreads();
-    for (int i = tid; i < NH * N_QHEAD; i += BE_THREADS) out[N_GRU + i] = s_gq[i];
-    for (int i = tid; i < 2 * NH * PK * (DM / 2); i += BE_THREADS) out[OFF_KA + i] = s_gkey[i];
-    // the waves' near-zero sums into the bins of those intervals, one wave after the other (a fixed order).  Register v
-    // of an accumulator holds first index 4 (lane / 16) + v, second index lane % 16.
+    // ---- this workgroup's sums -> its row of the partials buffer.  The waves' held expert sums into their bins, one wave
+    // after the other; the dense sums through LDS.
     for (int w = 0; w < BE_WAVES; w++) {
         __syncthreads();
-        if ((tid >> 6) != w) continue;
+        if (wave != w || x_held < 0.0f || !owner) continue;
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int ia = 4 * ((tid & 63) >> 4) + v, ib = tid & 15;
-            if (ia >= PK || ib >= PK) continue;
-            int e = ia * PK + ib;
-            if (e >= NE) e = NE - 1;
-            const int bp = e * NBIN + s_kz[2 * e + 1], bn = e * NBIN + s_kz[2 * e];
-            s_bin[2 * bp] += cen[0][v];
-            s_bin[2 * bn] += cen[1][v];
-            s_bin[2 * bp + 1] += cen[2][v];
-            s_bin[2 * bn + 1] += cen[3][v];
+        for (int q = 0; q < 8; q++) flush(q >> 1, q & 1);
+    }
+    constexpr int M_Q = 16 * 32, M_K = M_Q + 32 * 32, M_FLOATS = M_K + NH * 256;       // GRU [16][32], query [32][32], keys [NH][16 blocks][4][4]
+    static_assert(M_FLOATS <= 64 * XW + R_FLOATS, "the sums fit the wave's staging rows");
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int row = 4 * lk + v;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            s_x[row * 32 + 16 * c + li] = gacc[c][v];
+#pragma unroll
+            for (int p = 0; p < 2; p++) s_x[M_Q + (16 * p + row) * 32 + 16 * c + li] = qacc[p][c][v];
         }
+#pragma unroll
+        for (int hd = 0; hd < NH; hd++) s_x[M_K + hd * 256 + (lane >> 2) * 16 + v * 4 + (lane & 3)] = kacc[hd][v];
     }
     __syncthreads();
-    // expert gradients from the bins: d b1 = W2 * S0, d W1 = W2 * S1, d W2 = sum w relu(pre) = W1 * S1 + b1 * S0, d b2 = sum w
-    for (int i = tid; i < NE * EH; i += BE_THREADS) {
-        const int e = i / EH;
-        const float w1 = a.W.w[W_EXP_W1][i], b1 = a.W.w[W_EXP_B1][i], w2 = a.W.w[W_EXP_W2][i];
-        const int rank = s_rank[i];
-        float S0 = 0.0f, S1 = 0.0f;
-        for (int k = 0; k < NBIN; k++) {
-            if (!unit_active(w1, b1, rank, k)) continue;
-            S0 += s_bin[2 * (e * NBIN + k)];
-            S1 += s_bin[2 * (e * NBIN + k) + 1];
+    const float* const m0 = lds + KEY_FLOATS;
+    auto waves_sum = [&](int i) { return ((m0[i] + m0[i + WAVE_FLOATS]) + m0[i + 2 * WAVE_FLOATS]) + m0[i + 3 * WAVE_FLOATS]; };
+    static_assert(BE_WAVES == 4, "waves_sum");
+    float* const out = bins + N_BINS;
+    for (int o = tid; o < N_DENSE; o += BE_THREADS) {
+        float v;
+        if (o < N_GRU) {
+            int drow, xcol;
+            gru_entry(o, &drow, &xcol);
+            v = waves_sum(drow * 32 + xcol);
+        } else if (o < N_GRU + NH * N_QHEAD) {
+            const int q = o - N_GRU;
+            v = waves_sum(M_Q + (q / PIN) * 32 + q % PIN);
+        } else {        // [half][head][row][entry]
+            const int q = o - N_GRU - NH * N_QHEAD, hf = q / (KEY_FLOATS / 2), hd = q / (PK * (DM / 2)) % NH, row = q / (DM / 2) % PK, dd = q % (DM / 2);
+            const int i = M_K + hd * 256 + (hf * 3 + row / 4) * 16 + (row % 4) * 4 + dd;
+            v = waves_sum(i) + waves_sum(i + 6 * 16);
         }
-        out[OFF_W1 + i] = w2 * S1;
-        out[OFF_B1 + i] = w2 * S0;
-        out[OFF_W2 + i] = sg_fma(w1, S1, b1 * S0);
-    }
-    for (int e = tid; e < NE; e += BE_THREADS) {
-        float sd = 0.0f;
-        for (int k = 0; k < NBIN; k++) sd += s_bin[2 * (e * NBIN + k)];
-        out[OFF_B2 + e] = sd;
+        out[o] = v;
     }
 }
 
-// Rows of the partials buffer added in a fixed order: 64 entries per workgroup, four lanes per entry each taking
-// every fourth row, then the four partial sums in order.
-__global__ __launch_bounds__(256) void k_sum_partials(const float* __restrict__ partials, int rows, float* __restrict__ out) {
-    __shared__ float s_part[4][64];
+// Rows of the partials buffer added in a fixed order, eight slices of rows per column.  The first workgroups take 64 columns
+// of the dense sums each; each of the others takes the bins of one expert and forms its gradients from them: with S0, S1 of
+// a unit the sums of the bins on its active side, d b1 = W2 S0, d W1 = W2 S1, d W2 = sum w relu(pre) = W1 S1 + b1 S0,
+// d b2 = sum w.
+constexpr int FIN_SLICES = 8;
+constexpr int FIN_DENSE = (N_DENSE + 63) / 64;
+__global__ __launch_bounds__(64 * FIN_SLICES) void k_elem_finish(const float* __restrict__ partials, int rows, Sg2Weights W, int eh,
+                                                                 float* __restrict__ out) {
+    __shared__ float s_part[FIN_SLICES][64];
     const int col = threadIdx.x & 63, slice = threadIdx.x >> 6;
-    const int o = blockIdx.x * 64 + col;
+    const bool dense = blockIdx.x < FIN_DENSE;
+    const int e = (int)blockIdx.x - FIN_DENSE;
+    const int o = dense ? (int)blockIdx.x * 64 + col : col;
+    const bool live = dense ? o < N_DENSE : col < 2 * NBIN;
+    const float* src = partials + (dense ? N_BINS + o : e * NBIN * 2 + o);
     float acc = 0.0f;
-    if (o < N_GRADS) {
-#pragma unroll 4
-        for (int r = slice; r < rows; r += 4) acc += partials[(size_t)r * N_GRADS + o];
+    if (live) {
+#pragma unroll 8
+        for (int r = slice; r < rows; r += FIN_SLICES) acc += src[(size_t)r * ROW_FLOATS];
     }
     s_part[slice][col] = acc;
     __syncthreads();
-    if (slice == 0 && o < N_GRADS) out[o] = ((s_part[0][col] + s_part[1][col]) + s_part[2][col]) + s_part[3][col];
+    if (slice != 0) return;
+#pragma unroll
+    for (int q = 1; q < FIN_SLICES; q++) acc += s_part[q][col];
+    if (dense) {
+        if (live) out[o] = acc;
+        return;
+    }
+    s_part[0][col] = acc;
+    wave_sync();
+    const int m = col & (EH - 1);
+    const Unit u = unit_of(W.w[W_EXP_W1], W.w[W_EXP_B1], e, eh, m);
+    const float* bin = s_part[0];
+    float S0 = 0.0f, S1 = 0.0f, sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NBIN; k++) {
+        sum += bin[2 * k];
+        if (!unit_active(u.w1, u.b1, u.rank, k)) continue;
+        S0 += bin[2 * k];
+        S1 += bin[2 * k + 1];
+    }
+    float* const dst = out + N_DENSE;
+    if (col < eh) {
+        const float w2 = W.w[W_EXP_W2][e * eh + m];
+        dst[e * eh + m] = w2 * S1;
+        dst[NE * eh + e * eh + m] = w2 * S0;
+        dst[2 * NE * eh + e * eh + m] = sg_fma(u.w1, S1, u.b1 * S0);
+    }
+    if (col == 0) dst[3 * NE * eh + e] = sum;
 }
 
-constexpr int BE_LDS_BYTES = 4 * (NE * EH + NE * NBIN * 4 + 2 * NH * PK * (DM / 2) + BE_THREADS * (XW + DW + RW) + NH * N_QHEAD) + NE * EH + NE * 2;
-static_assert(BE_LDS_BYTES <= 160 * 1024, "one workgroup of k_bilevel_elem per CU");
-constexpr int BE_MAX_GROUPS = 256;       // one resident workgroup on each of the 256 CUs: one round, every workgroup walks the same number of tiles (+-1)
+int elem_groups(int64_t tiles) {
+    const int64_t groups = (tiles + BE_WAVES - 1) / BE_WAVES;
+    return (int)(groups < BE_MAX_GROUPS ? (groups > 0 ? groups : 1) : BE_MAX_GROUPS);
+}
 
-int elem_groups(int64_t total) {
-    const int64_t tiles = (total + BE_THREADS - 1) / BE_THREADS;
-    return (int)(tiles < BE_MAX_GROUPS ? (tiles > 0 ? tiles : 1) : BE_MAX_GROUPS);
+size_t elem_workspace(int groups) { return sizeof(float) * (TABLE_FLOATS + (size_t)groups * ROW_FLOATS); }
+
+// a.tables and a.partials are set here, from the workspace
+template <bool FLAT>
+int run_elem(ElemArgs& a, const Plan& pl, int groups, int eh, void* workspace, float* grads_out, hipStream_t st) {
+    {
+        static bool raised[64] = {};
+        int dev = 0;
+        SG_HIP_CHECK(hipGetDevice(&dev));
+        if (dev < 0 || dev >= 64) return sg::fail("device index %d out of range", dev);
+        if (!raised[dev]) {
+            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_bilevel_elem<FLAT>), hipFuncAttributeMaxDynamicSharedMemorySize, BE_LDS_BYTES));
+            raised[dev] = true;
+        }
+    }
+    float* tables = static_cast<float*>(workspace);
+    a.tables = tables;
+    a.partials = tables + TABLE_FLOATS;
+    hipLaunchKernelGGL(k_expert_tables, dim3(NE), dim3(64), 0, st, a.W, eh, tables);
+    SG_LAUNCH_CHECK("k_expert_tables");
+    hipLaunchKernelGGL(k_bilevel_elem<FLAT>, dim3(groups), dim3(BE_THREADS), BE_LDS_BYTES, st, a, pl);
+    SG_LAUNCH_CHECK("k_bilevel_elem");
+    hipLaunchKernelGGL(k_elem_finish, dim3(FIN_DENSE + NE), dim3(64 * FIN_SLICES), 0, st, a.partials, groups, a.W, eh, grads_out);
+    SG_LAUNCH_CHECK("k_elem_finish");
+    return 0;
 }
 
 }  // namespace
+
+size_t bilevel_elem_workspace(int elem_tiles) { return elem_workspace(elem_groups((int64_t)elem_tiles * (ELEM_TILE / 64))); }
+int launch_bilevel_elem(const Plan& pl, bool normalise, int eh, float* smart_out, float* d_ctx, float* grads_out, void* workspace, hipStream_t st) {
+    ElemArgs a = {};
+    a.ctx = pl.ctx; a.smart = smart_out; a.d_ctx = d_ctx;
+    a.total = pl.total; a.normalise = normalise; a.rescale = pl.rescale; a.W = pl.W;
+    return run_elem<false>(a, pl, elem_groups((int64_t)pl.elem_tiles * (ELEM_TILE / 64)), eh, workspace, grads_out, st);
+}
 }  // namespace sg2
 
 extern "C" {
 
 size_t sg2_bilevel_elem_workspace_bytes(int64_t total) {
     if (total < 0) return 0;
-    return sizeof(float) * (size_t)sg2::elem_groups(total) * sg2::N_GRADS;
+    return sg2::elem_workspace(sg2::elem_groups((total + 63) / 64));
 }
 
 int sg2_bilevel_elem(const SgDims* dims, const Sg2Weights* weights, int64_t total, const float* grad, const float* sharpness,
@@ -589,33 +830,20 @@ int sg2_bilevel_elem_ex(const SgDims* dims, const Sg2Weights* weights, int64_t t
     if (total < 0 || total > 0x7fffffffLL - BE_THREADS) return sg::fail("element count %lld out of range", (long long)total);
     for (int k = W_GRU_WZ; k < SG2_NUM_WEIGHTS; k++)
         if (!weights->w[k]) return sg::fail("weight pointer %d is NULL", k);
-    const int groups = elem_groups(total);
-    if (!workspace || workspace_bytes < sizeof(float) * (size_t)groups * N_GRADS)
-        return sg::fail("workspace too small: need %zu bytes, got %zu", sizeof(float) * (size_t)groups * N_GRADS, workspace_bytes);
+    const int groups = elem_groups((total + 63) / 64);
+    if (!workspace || workspace_bytes < elem_workspace(groups))
+        return sg::fail("workspace too small: need %zu bytes, got %zu", elem_workspace(groups), workspace_bytes);
+    if (((uintptr_t)workspace & 127u) != 0) return sg::fail("workspace must be 128-byte aligned");
     if (total > 0) {
         if (!grad || !sharpness || !ctx || !gru_state || !cotangent || !d_ctx) return sg::fail("NULL argument");
         if ((((uintptr_t)ctx | (uintptr_t)gru_state | (uintptr_t)d_ctx | (uintptr_t)gru_out) & 15u) != 0)
             return sg::fail("ctx, gru_state, gru_out and d_ctx must be 16-byte aligned");
     }
-    {
-        static bool raised[64] = {};
-        int dev = 0;
-        SG_HIP_CHECK(hipGetDevice(&dev));
-        if (dev < 0 || dev >= 64) return sg::fail("device index %d out of range", dev);
-        if (!raised[dev]) {
-            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_bilevel_elem), hipFuncAttributeMaxDynamicSharedMemorySize, BE_LDS_BYTES));
-            raised[dev] = true;
-        }
-    }
-    ElemArgs a;
+    ElemArgs a = {};
     a.g = grad; a.s = sharpness; a.ctx = ctx; a.gru = gru_state; a.cot = cotangent;
-    a.smart = smart_out; a.d_ctx = d_ctx; a.partials = static_cast<float*>(workspace); a.gru_out = gru_out;
+    a.smart = smart_out; a.d_ctx = d_ctx; a.gru_out = gru_out;
     a.total = (int)total; a.rescale = rescale; a.W = *weights;
-    hipLaunchKernelGGL(k_bilevel_elem, dim3(groups), dim3(BE_THREADS), BE_LDS_BYTES, st, a);
-    SG_LAUNCH_CHECK("k_bilevel_elem");
-    hipLaunchKernelGGL(k_sum_partials, dim3((N_GRADS + 63) / 64), dim3(256), 0, st, a.partials, groups, grads_out);
-    SG_LAUNCH_CHECK("k_sum_partials");
-    return 0;
+    return run_elem<true>(a, Plan{}, groups, EH, workspace, grads_out, st);
 }
 
 }  // extern "C"

@@ -391,11 +391,9 @@ __device__ __forceinline__ void block_steps(LaneState& S, const float (&dt)[UB],
     }
 }
 
-// KEEP (bilevel pass, OUT only): also store the state entering every HT_STEP-th step for the adjoint kernels.
-template <class G, bool OUT, bool KEEP = false>
+template <class G, bool OUT>
 __global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
     constexpr int DM = G::DM, DS = G::DS, DI = G::DI, HP = G::HP, SCAN_THREADS = G::THREADS, PARTS = G::PARTS;
-    static_assert(!KEEP || PARTS == 2, "the bilevel pass exists for the default geometry only");
     __shared__ __attribute__((aligned(16))) float s_dt[DI * LDS_STRIDE];
     __shared__ __attribute__((aligned(16))) float s_ux[DI * LDS_STRIDE];       // dt * x-branch
     __shared__ __attribute__((aligned(16))) float s_B[DS * LDS_STRIDE];
@@ -578,12 +576,6 @@ __global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
         };
         const unsigned long long large = uniform64(s_large[half]), nottiny = uniform64(s_nottiny[half]);
 
-        auto keep_state = [&](int u) {
-            float* ht = pl.htile + ((size_t)dir * htile_count(pl.total, pl.P) + htile_index(off, ti, u)) * 2 * SCAN_THREADS;
-            ht[tid] = S.he;
-            ht[SCAN_THREADS + tid] = S.ho;
-        };
-        if (KEEP) keep_state(tile0);
         // ---------------- phase B: the recurrence over the tile, lane = (j,p)
         const float* __restrict__ r_dt = s_dt + j * LDS_STRIDE;
         const float* __restrict__ r_ux = s_ux + j * LDS_STRIDE;
@@ -593,7 +585,6 @@ __global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
         const float* __restrict__ r_Co = s_C + (OUT ? (2 * p + 1) * LDS_STRIDE : 0);
         int k0 = 0;
         for (; k0 + UB <= cnt; k0 += UB) {
-            if (KEEP && k0 == HT_STEP) keep_state(tile0 + HT_STEP);
             float dt[UB], xv[UB], Be[UB], Bo[UB], Ce[UB], Co[UB], y[UB];
 #pragma unroll
             for (int q = 0; q < UB; q += 4) {
@@ -632,7 +623,6 @@ __global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
                     *reinterpret_cast<float2*>(&s_y[j * LDS_STRIDE + k0 + 2 * (p >> 2)]) = make_float2(y[0], y[1]);
             }
         }
-        if (KEEP && k0 == HT_STEP && cnt > HT_STEP) keep_state(tile0 + HT_STEP);      // the ragged end starts right there
         for (; k0 < cnt; k0++) {       // ragged end of the last tile of a tensor
             const float dt = r_dt[k0], ux = r_ux[k0];
             float ae, ao, sn, cs;
@@ -677,14 +667,6 @@ __global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
                     *reinterpret_cast<float4*>(dst) = make_float4(cx[0], cx[1], cx[2], cx[3]);
                 else
                     *reinterpret_cast<float2*>(dst) = make_float2(cx[0], cx[1]);
-                if constexpr (KEEP) {
-                    if (pl.scan_out[dir] != nullptr) {
-                        // the gated scan output itself (before out_proj), at the step's position in scan order; this half's 8 columns
-                        float4* so = reinterpret_cast<float4*>(pl.scan_out[dir] + ((size_t)off + tile0 + tu) * DI) + 2 * half;
-                        so[0] = half ? make_float4(o[8], o[9], o[10], o[11]) : make_float4(o[0], o[1], o[2], o[3]);
-                        so[1] = half ? make_float4(o[12], o[13], o[14], o[15]) : make_float4(o[4], o[5], o[6], o[7]);
-                    }
-                }
             }
             __syncthreads();
         }
@@ -941,7 +923,9 @@ __device__ __forceinline__ void block_steps_pair(LaneState (&S)[2], const float 
 // its element's row.  Row owner (the usual tile, on the polynomials throughout): lane (column, quarter of the tile)
 // forms that column's projections before the recurrence and gates its outputs after it (project_rows, gate_rows);
 // other tiles keep the timestep-per-lane projections (project_all, gates_all).
-template <class G>
+// KEEP (bilevel pass): also store the state entering every HT_STEP-th step for the adjoint kernels, and the gated outputs
+// where they are asked for.  (5.9 ms for 25 M elements; 7.1 as a variant of the two-wave kernel.)
+template <class G, bool KEEP>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_replay(Plan pl) {
     constexpr int DM = G::DM, DS = G::DS, DI = G::DI, HP = G::HP, LANES = G::THREADS;
     static_assert(G::PARTS == 2 && LANES == 128 && HP == 8, "two columns per lane of one wave");
@@ -1097,6 +1081,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         }
         __syncthreads();      // one wave: no s_barrier is issued, the LDS writes above are ordered before the reads below
 
+        auto keep_state = [&](int u) {
+            float* ht = pl.htile + ((size_t)dir * htile_count(pl.total, pl.P) + htile_index(off, ti, u)) * 2 * LANES;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                ht[tid + 64 * h] = S[h].he;
+                ht[LANES + tid + 64 * h] = S[h].ho;
+            }
+        };
+        if (KEEP) keep_state(tile0);
+
         // ---------------- phase B: the recurrences of this lane's two columns over the tile
         const float* __restrict__ r_Be = s_B + (2 * p) * LDS_STRIDE;
         const float* __restrict__ r_Bo = s_B + (2 * p + 1) * LDS_STRIDE;
@@ -1135,11 +1129,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             };
 #pragma unroll 1
             for (; k0 < SCAN_TT; k0 += UB) {
+                if (KEEP && k0 == HT_STEP) keep_state(tile0 + HT_STEP);
                 fetch(k0, Be, Bo, Ce, Co, dt, xv);
                 compute(k0, Be, Bo, Ce, Co, dt, xv);
             }
         }
         for (; k0 + UB <= cnt; k0 += UB) {
+            if (KEEP && k0 == HT_STEP) keep_state(tile0 + HT_STEP);
             float Be[UB], Bo[UB], Ce[UB], Co[UB];
 #pragma unroll
             for (int q = 0; q < UB; q += 4) {
@@ -1175,6 +1171,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                     *reinterpret_cast<f32x4*>(&s_y[j * LDS_STRIDE + k0 + 4 * (p >> 2)]) = f32x4{y[0], y[1], y[2], y[3]};
             }
         }
+        if (KEEP && k0 == HT_STEP && cnt > HT_STEP) keep_state(tile0 + HT_STEP);      // the ragged end starts right there
         for (; k0 < cnt; k0++) {       // ragged end of the last tile of a tensor
 #pragma unroll
             for (int h = 0; h < 2; h++) {
@@ -1223,14 +1220,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                 }
             }
             const float cx[DM] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            held_dst = valid ? reinterpret_cast<float4*>(pl.ctx + ((size_t)dir * pl.total + off + orig) * DM) : nullptr;
+            const int at = KEEP && pl.own_order ? (dir ? N - 1 - (tile0 + tu) : tile0 + tu) : orig;
+            held_dst = valid ? reinterpret_cast<float4*>(pl.ctx + ((size_t)dir * pl.total + off + at) * DM) : nullptr;
             held[0] = make_float4(cx[0], cx[1], cx[2], cx[3]);
             held[1] = make_float4(cx[4], cx[5], cx[6], cx[7]);
+            if constexpr (KEEP) {
+                if (pl.scan_out[dir] != nullptr && valid) {        // the gated scan output itself (before out_proj), in scan order
+                    float4* so = reinterpret_cast<float4*>(pl.scan_out[dir] + ((size_t)off + tile0 + tu) * DI);
+#pragma unroll
+                    for (int m = 0; m < DI; m += 4) so[m / 4] = make_float4(o[m], o[m + 1], o[m + 2], o[m + 3]);
+                }
+            }
         }
         __syncthreads();
     }
     flush();
-    if (u1 == N) {   // last chunk in scan order: new carried state of the tensor
+    if (u1 == N && !(KEEP && pl.own_order)) {   // last chunk in scan order: new carried state of the tensor
         float* st = dir ? T.mbwd : T.mfwd;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -1320,7 +1325,7 @@ __global__ __launch_bounds__(1024) void k_chunk_prefix(Plan pl) {
 template <class G>
 int launch_scan_geo(const Plan& pl, hipStream_t st) {
     if (pl.wchunks > 0) {
-        hipLaunchKernelGGL((k_scan<G, false, false>), dim3(2 * pl.wchunks), dim3(G::THREADS), 0, st, pl);
+        hipLaunchKernelGGL((k_scan<G, false>), dim3(2 * pl.wchunks), dim3(G::THREADS), 0, st, pl);
         SG_LAUNCH_CHECK("k_scan<summary>");
     }
     prof_mark(2, st);
@@ -1329,20 +1334,13 @@ int launch_scan_geo(const Plan& pl, hipStream_t st) {
         SG_LAUNCH_CHECK("k_chunk_prefix");
     }
     prof_mark(3, st);
-    if constexpr (G::PARTS == 2) {
-        if (pl.htile != nullptr) {
-            hipLaunchKernelGGL((k_scan<G, true, true>), dim3(2 * pl.chunks), dim3(G::THREADS), 0, st, pl);
-            SG_LAUNCH_CHECK("k_scan<out, keep>");
-            prof_mark(4, st);
-            return 0;
-        }
-    }
-    if (pl.htile != nullptr) return sg::fail("the bilevel pass is built for the default meta-net dimensions only");
+    if (pl.htile != nullptr && G::PARTS != 2) return sg::fail("the bilevel pass is built for the default meta-net dimensions only");
     if constexpr (G::PARTS == 2) {          // one wave per chunk, two columns per lane
-        hipLaunchKernelGGL(k_replay<G>, dim3(2 * pl.chunks), dim3(64), 0, st, pl);
+        if (pl.htile != nullptr) hipLaunchKernelGGL((k_replay<G, true>), dim3(2 * pl.chunks), dim3(64), 0, st, pl);
+        else hipLaunchKernelGGL((k_replay<G, false>), dim3(2 * pl.chunks), dim3(64), 0, st, pl);
         SG_LAUNCH_CHECK("k_replay");
     } else {
-        hipLaunchKernelGGL((k_scan<G, true, false>), dim3(2 * pl.chunks), dim3(G::THREADS), 0, st, pl);
+        hipLaunchKernelGGL((k_scan<G, true>), dim3(2 * pl.chunks), dim3(G::THREADS), 0, st, pl);
         SG_LAUNCH_CHECK("k_scan<out>");
     }
     prof_mark(4, st);

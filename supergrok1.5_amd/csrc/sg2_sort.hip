@@ -137,7 +137,7 @@ __global__ __launch_bounds__(SORT_THREADS) void k_keys(Plan pl) {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 atomicAdd(&h[key_of(clipped(g[r][e], gs, SG_F32)) & 255u], 1u);
-                nz = nz || (sg::finite_or_zero(sh[r][e]) != 0.0f);
+                nz = nz || sh[r][e] != 0.0f;
             }
     } else {
         float g[ITEMS];
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(SORT_THREADS) void k_keys(Plan pl) {
 #pragma unroll
         for (int r = 0; r < ITEMS; r++) {
             const int k = r * SORT_THREADS + (int)threadIdx.x;
-            if (k < tr.cnt) nz = nz || (sharp_of(T, start + k) != 0.0f);
+            if (k < tr.cnt) nz = nz || sharp_rounded(T, start + k) != 0.0f;
         }
         const float gs = clip_factor(pl, seg, tr.tile == 0);
         __syncthreads();
@@ -474,7 +474,7 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort_tile(Plan pl) {
         const float v = clipped(sg::load_elem(T.grad, dtype, i), gs, dtype);
         skey[i] = key_of(v);
         sval[i] = payload_of(v, i);
-        nz = nz || (sharp_of(T, i) != 0.0f);
+        nz = nz || sharp_rounded(T, i) != 0.0f;
     }
     note_sharpness(pl, seg, nz);
     const bool gather = __syncthreads_or(nz);

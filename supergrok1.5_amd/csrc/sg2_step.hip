@@ -67,7 +67,7 @@ struct Prof {
 constexpr int PREFIXES = 5;     // prefix tables: tiles of the elementwise kernels, sort tiles, scan chunks, chunks with a summary, norm tiles
 struct Layout {
     int P, total, elem_tiles, sort_tiles, chunks, wchunks, nb, sort_tile, sort_widest, norm_tile, norm_tiles;
-    size_t off_norm, off_gscale, off_tables, off_keys[2], off_vals[2], off_ssorted, off_spine, off_blocksums, off_summ, off_hstart, off_comp, off_flags, off_padw, off_ctx, off_htile, off_adj_summ, off_adj_lam, off_adj_part, off_adj_blk, bytes;
+    size_t off_norm, off_gscale, off_tables, off_keys[2], off_vals[2], off_ssorted, off_spine, off_blocksums, off_summ, off_hstart, off_comp, off_flags, off_padw, off_ctx, off_htile, off_adj_summ, off_adj_lam, off_adj_part, off_adj_blk, off_dctx, off_elem, bytes;
     size_t tables_bytes;
 };
 
@@ -134,7 +134,8 @@ inline int sort_tile_for(int64_t widest) {
 // Elements per workgroup of the norm reduction: as the other steps' tiles (many short ones for small calls).
 inline int norm_tile_for(int64_t total) { return total >= (8 << 20) ? 4096 : (total >= (1 << 20) ? 1024 : 256); }
 
-int make_layout(int geo, int P, Numels numels, int chunk_len, Layout* L, bool bilevel = false) {
+// bilevel: with what the adjoint needs; whole_pass: and the per-element part of the bilevel pass
+int make_layout(int geo, int P, Numels numels, int chunk_len, Layout* L, bool bilevel = false, bool whole_pass = false) {
     const GeoInfo gi = geo_info(geo);
     int64_t total = 0, et = 0, stl = 0, ch = 0, wch = 0, nt = 0, widest = 0;
     for (int i = 0; i < P; i++) {
@@ -183,6 +184,8 @@ int make_layout(int geo, int P, Numels numels, int chunk_len, Layout* L, bool bi
     L->off_adj_lam = take(bilevel ? 4 * 2 * (size_t)L->chunks * SCAN_THREADS * 2 : 0);
     L->off_adj_part = take(bilevel ? 4 * 2 * (size_t)ADJ_GROUPS * SG2_BWD_STRIDE : 0);
     L->off_adj_blk = take(bilevel ? 4 * 2 * (size_t)SG2_BWD_STRIDE : 0);
+    L->off_dctx = take(whole_pass ? 4 * 2 * (size_t)total * gi.dm : 0);
+    L->off_elem = take(whole_pass ? bilevel_elem_workspace(L->elem_tiles) : 0);
     L->bytes = o;
     return 0;
 }
@@ -235,19 +238,20 @@ __global__ __launch_bounds__(256) void k_tables(TableChunk c) {
 // it.  HBM bound (one read of the gradients); writing clipped copies and reading those instead cost a second pass (38 us
 // for 25 M elements) and three launches.  (The tile that finishes a tensor could add them up here, but an atomic counter
 // with release order per workgroup took 38 us where the plain stores take 5: each one writes back its L2.)
-__global__ __launch_bounds__(256) void k_norm(Plan pl) {
+__global__ __launch_bounds__(256) void k_norm(Plan pl, bool of_param) {
     __shared__ double sm[4];
     const int tile = blockIdx.x;
     const sg::Seg seg = sg::find_seg(sg::as_const(pl.norm_tile_prefix), pl.P, tile);
     const TensorDev& T = pl.tensors[seg.i];
     const int start = (tile - seg.first) * pl.norm_tile, cnt = min(pl.norm_tile, T.numel - start);
+    const void* const src = of_param ? T.param : T.grad;
     float acc = 0.0f;
     for (int k0 = 0; k0 < cnt; k0 += 8 * 256) {       // eight loads on their way at a time, added in order
         float g[8];
 #pragma unroll
         for (int r = 0; r < 8; r++) {
             const int k = k0 + r * 256 + (int)threadIdx.x;
-            g[r] = k < cnt ? sg::load_elem(T.grad, T.dtype, start + k) : 0.0f;
+            g[r] = k < cnt ? sg::load_elem(src, T.dtype, start + k) : 0.0f;
         }
 #pragma unroll
         for (int r = 0; r < 8; r++) acc = sg_fma(g[r], g[r], acc);
@@ -258,8 +262,8 @@ __global__ __launch_bounds__(256) void k_norm(Plan pl) {
 
 }  // namespace
 
-int launch_norm(const Plan& pl, hipStream_t st) {
-    hipLaunchKernelGGL(k_norm, dim3(pl.norm_tiles), dim3(256), 0, st, pl);
+int launch_norm(const Plan& pl, bool of_param, hipStream_t st) {
+    hipLaunchKernelGGL(k_norm, dim3(pl.norm_tiles), dim3(256), 0, st, pl, of_param);
     SG_LAUNCH_CHECK("k_norm");
     return 0;
 }
@@ -397,7 +401,7 @@ namespace sg2 {
 // states (bilevel forward/backward).  Returns 0 with pl->total == 0 when there is nothing to do.
 int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, const Sg2Scalars* scalars,
                void* workspace, size_t workspace_bytes, bool full_step, bool bilevel, bool keep_flags, hipStream_t st, Plan* plp, Layout* Lp,
-               int chunk_override = 0, int window_override = -1) {
+               int chunk_override = 0, int window_override = -1, bool whole_pass = false) {
     Plan& pl = *plp;
     Layout& L = *Lp;
     pl.total = 0;
@@ -420,13 +424,13 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
         if (t.numel > 0) {
             if (!t.grad || !t.sharpness || !t.mamba_fwd_state || !t.mamba_bwd_state) return sg::fail("tensor %d: NULL pointer", i);
             if (full_step && (!t.param || !t.exp_avg || !t.exp_avg_sq || !t.mu || !t.gru_state)) return sg::fail("tensor %d: NULL pointer", i);
-            const int dtype = t.dtype & ~SG_SHARP_F32;
+            const int dtype = t.dtype & ~(SG_SHARP_F32 | SG_SHARP_EXACT);
             if (dtype != SG_F32 && dtype != SG_F16 && dtype != SG_BF16) return sg::fail("tensor %d: bad dtype %d", i, t.dtype);
             if (full_step && ((uintptr_t)t.gru_state & 15u) != 0) return sg::fail("tensor %d: gru_state must be 16-byte aligned", i);
         }
     }
     const int chunk_len = chunk_override > 0 ? chunk_override : effective_chunk_len(P, numels);
-    if (make_layout(geo, P, numels, chunk_len, &L, bilevel)) return 1;
+    if (make_layout(geo, P, numels, chunk_len, &L, bilevel, whole_pass)) return 1;
     if (L.total == 0) return 0;
     if (!workspace || workspace_bytes < L.bytes)
         return sg::fail("workspace too small: need %zu bytes, got %zu", L.bytes, workspace_bytes);
@@ -454,8 +458,8 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
                 d.param = t.param; d.grad = t.grad; d.sharp = t.sharpness;
                 d.ea = t.exp_avg; d.easq = t.exp_avg_sq; d.mu = t.mu; d.gru = t.gru_state;
                 d.mfwd = t.mamba_fwd_state; d.mbwd = t.mamba_bwd_state;
-                d.off = off; d.numel = n; d.dtype = t.dtype & ~SG_SHARP_F32; d.nchunks = nc;
-                d.sharp32 = t.dtype != d.dtype && d.dtype != SG_F32 ? 1 : 0;
+                d.off = off; d.numel = n; d.dtype = t.dtype & ~(SG_SHARP_F32 | SG_SHARP_EXACT); d.nchunks = nc;
+                d.sharp32 = t.dtype == d.dtype || d.dtype == SG_F32 ? 0 : (t.dtype & SG_SHARP_EXACT) != 0 ? 2 : 1;
                 d.alpha = t.alpha_mu; d.lamb = t.lamb_eff; d.beta1 = t.beta1; d.bc2 = t.bc2;
                 d.step_size = full_step ? scalars->lr / t.bc1 : 0.0f;
                 for (int q = 0; q < 4; q++) d.pad_[q] = 0;
@@ -484,6 +488,7 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
     pl.norm_partials = reinterpret_cast<double*>(ws + L.off_norm);
     pl.gscale = nullptr;
     pl.max_norm = 0.0f;
+    pl.own_order = whole_pass;
     pl.P = P; pl.total = L.total; pl.elem_tiles = L.elem_tiles; pl.sort_tiles = L.sort_tiles;
     pl.chunks = L.chunks; pl.wchunks = L.wchunks; pl.chunk_len = chunk_len; pl.window = window_override >= 0 ? window_override : g_window.load();
     for (int k = 0; k < 2; k++) {
@@ -557,7 +562,7 @@ int run_step(const SgDims* dims, const Sg2Weights* weights, int num_tensors, con
     if (clip_norm > 0.0f) {
         pl.gscale = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + L.off_gscale);
         pl.max_norm = clip_norm;
-        if (launch_norm(pl, st)) return 1;
+        if (launch_norm(pl, false, st)) return 1;
     }
     if (launch_sort(pl, debug ? debug->perm : nullptr, st)) return 1;
     prof_mark(1, st);
@@ -750,6 +755,45 @@ int sg2_bilevel_backward_ex(const SgDims* dims, const Sg2Weights* weights, int n
                         GeoDefault::DS, GeoDefault::DI);
     const float* const d_scan[2] = {d_scan_out_fwd, d_scan_out_bwd};
     return launch_bilevel_backward(pl, d_ctx, d_scan, row_dx, dx_out, grads_out, st);
+}
+
+size_t sg2_bilevel_pass_workspace_bytes(const SgDims* dims, int num_tensors, const int64_t* numels) {
+    if (sg2::check_dims(dims) || num_tensors < 0 || (num_tensors > 0 && !numels)) return 0;
+    sg2::Layout L;
+    const sg2::Numels n = {numels, nullptr};
+    if (sg2::make_layout(sg2::GEO_DEFAULT, num_tensors, n, sg2::effective_chunk_len(num_tensors, n), &L, true, true)) return 0;
+    return L.bytes;
+}
+
+int sg2_bilevel_pass(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, float rescale, int normalise,
+                     float* smart_out, float* elem_grads_out, float* scan_grads_out, void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace sg2;
+    hipStream_t st = (hipStream_t)stream;
+    Plan pl;
+    Layout L;
+    const Sg2Scalars none = {rescale, 0.0f, 0.0f, 0.0f, 0.0f};
+    if (!elem_grads_out || !scan_grads_out) return sg::fail("NULL argument");
+    if (num_tensors <= 0 || !tensors) return sg::fail("sg2_bilevel_pass: no tensors");
+    const int geo = geo_of(dims);
+    if (geo < 0) return 1;
+    SgDims routing = *dims;
+    routing.expert_hidden = EH;          // narrower experts are read at their own width
+    if (check_dims(&routing, true)) return 1;
+    if (!scan_exact(dims, geo) || dims->expert_hidden > EH)
+        return sg::fail("sg2_bilevel_pass is built for d_model=%d d_state=%d d_inner=%d and expert_hidden up to %d", GeoDefault::DM, GeoDefault::DS,
+                        GeoDefault::DI, EH);
+    for (int i = 0; i < num_tensors; i++)
+        if (tensors[i].numel > 0 && (!tensors[i].gru_state || !tensors[i].param || ((uintptr_t)tensors[i].gru_state & 15u) != 0))
+            return sg::fail("tensor %d: gru_state (16-byte aligned) and param (the cotangent) are needed", i);
+    if (build_plan(dims, weights, num_tensors, tensors, &none, workspace, workspace_bytes, false, true, false, st, &pl, &L, 0, -1, true)) return 1;
+    if (pl.total == 0) return sg::fail("sg2_bilevel_pass: no elements");
+    unsigned char* ws = static_cast<unsigned char*>(workspace);
+    float* d_ctx = reinterpret_cast<float*>(ws + L.off_dctx);
+    if (normalise && launch_norm(pl, true, st)) return 1;
+    if (launch_sort(pl, nullptr, st)) return 1;
+    if (launch_scan(pl, st)) return 1;
+    if (launch_bilevel_elem(pl, normalise != 0, dims->expert_hidden, smart_out, d_ctx, elem_grads_out, ws + L.off_elem, st)) return 1;
+    return launch_bilevel_backward(pl, d_ctx, nullptr, nullptr, nullptr, scan_grads_out, st);
 }
 
 int sg2_bilevel_backward(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, const float* d_ctx,

@@ -20,7 +20,7 @@ take the scan blocks' own torch forward (chunked, on the GPU) under autograd.
 """
 import torch
 
-from grokking_optimizers import _cabi
+from grokking_optimizers import _cabi, _ops
 
 def split_flat(flat, params):
     """Views of one flat gradient tensor, one per parameter, in order (no copies, no kernels)."""
@@ -139,6 +139,13 @@ def elem_kernel_fits(mn):
             and d["gru_hidden"] <= _cabi.BILEVEL_GRU_HIDDEN and d["expert_hidden"] <= _cabi.BILEVEL_EXPERT_WIDTH)
 
 
+def _pass_fits(mn):
+    """Whether sg2_bilevel_pass can run this net: the scan block, GRU and routing sizes as built, experts up to its width."""
+    d = meta_dims(mn)
+    return ((d["d_model"], d["d_state"], d["d_inner"]) == _cabi.BILEVEL_SCAN_BLOCK and d["gru_hidden"] == _cabi.BILEVEL_GRU_HIDDEN
+            and elem_kernel_fits(mn))
+
+
 def scan_kernels_fit(mn):
     """Whether the scan kernels of the bilevel pass can run this net's scan block (up to d_model 8, d_state 16,
     d_inner 16; smaller ones run embedded)."""
@@ -220,18 +227,24 @@ def elem_parameters(mn):
     return out + [mn.expert_W1, mn.expert_b1, mn.expert_W2, mn.expert_b2]
 
 
-def _add_grads(params, flat):
-    """p.grad (+)= its slice of `flat`; a parameter without a gradient gets a view of the flat tensor."""
-    for p, gr in zip(params, split_flat(flat, params)):
-        if p.requires_grad:
-            gr = gr if gr.dtype == p.dtype else gr.to(p.dtype)
-            p.grad = gr if p.grad is None else p.grad + gr
-
-
-def accumulate_meta_gradients(mn, grads, sharps, gru_states, mamba_fwd, mamba_bwd, cotangents):
+def accumulate_meta_gradients(mn, grads, sharps, gru_states, mamba_fwd, mamba_bwd, cotangents, validation=False, want_smart=True):
     """Adds the gradient of  sum_p <smart_grad_p, cotangent_p>  with respect to every parameter of `mn` to its
-    .grad, for a list of tensors at once, all in HIP: scan forward (sg2_bilevel_forward), per-element forward and
-    backward (sg2_bilevel_elem), scan adjoint (sg2_bilevel_backward).  Returns the smart gradients (flat, packed)."""
+    .grad, for a list of tensors at once, all in HIP: scan forward, per-element forward and backward, scan adjoint
+    (sg2_bilevel_pass; for nets smaller than its sizes sg2_bilevel_forward, sg2_bilevel_elem and sg2_bilevel_backward on
+    packed copies).  validation: `cotangents` are validation gradients v and the cotangent is -v / |v| (-v where |v| is
+    0); sharpness is then used at its own precision whatever the gradients' type.  Returns the smart gradients (flat,
+    packed), or None without want_smart where they cost extra."""
+    if _pass_fits(mn) and None not in mamba_fwd and None not in mamba_bwd:
+        got = _ops.supergrok2_bilevel_pass(grads, sharps, gru_states, mamba_fwd, mamba_bwd, cotangents, mn.flat_weights(), float(mn.rescale),
+                                           validation, validation, want_smart, list(meta_dims(mn).values()))
+        if got is not None:
+            _ops.add_flat_grads(elem_parameters(mn), got[1])
+            _ops.add_flat_grads(scan_parameters(mn), got[2])
+            return got[0]
+    if validation:
+        grads, sharps = [g.float() for g in grads], [s.float() for s in sharps]
+        norms = [(v, v.norm()) for v in (c.float() for c in cotangents)]
+        cotangents = [-torch.where(norm > 1e-12, v / norm, v) for v, norm in norms]
     if not scan_kernels_fit(mn):
         # a scan block larger than the bilevel kernels are built for: tensor by tensor through the autograd form
         params = [p for p in mn.parameters() if p.requires_grad]
@@ -263,8 +276,8 @@ def accumulate_meta_gradients(mn, grads, sharps, gru_states, mamba_fwd, mamba_bw
         return smart.detach()
     ctx = plan.forward()
     smart, d_ctx, blk = _cabi.bilevel_elem(plan.weights, g_all, s_all, ctx, h_all, c_all, float(mn.rescale), meta_dims(mn))
-    _add_grads(elem_parameters(mn), blk)
-    _add_grads(scan_parameters(mn), plan.backward(d_ctx))
+    _ops.add_flat_grads(elem_parameters(mn), blk)
+    _ops.add_flat_grads(scan_parameters(mn), plan.backward(d_ctx))
     return smart
 
 

@@ -195,30 +195,25 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
         from grokking_optimizers import _bilevel
         self._ensure_state()
         named = list(model.named_parameters())
-        saved = {n: p.grad.detach().clone() for n, p in named if p.grad is not None}
+        saved = {n: p.grad for n, p in named if p.grad is not None}
         picked = [(n, p, self._param_to_idx[id(p)]) for n, p in named
                   if n in saved and id(p) in self._param_to_idx and saved[n].numel() > 0]
         if not picked:
             return 0.0
+        for _, p in named:
+            p.grad = None              # the training gradients step aside, whatever zero_grad would do to them
         model.zero_grad()
         with torch.enable_grad():
             val_loss = criterion(model(val_x), val_y)
             val_loss.backward()
         meta_optimizer.zero_grad()
-        grads, sharps, grus, mf, mb, cots = [], [], [], [], [], []
-        for n, p, i in picked:
-            if p.grad is None:
-                continue
-            vg = p.grad.detach().float()
-            norm = vg.norm()
-            grads.append(saved[n].reshape(-1).float().contiguous())
-            sharps.append(self._flat_sharpness[i].reshape(-1).float().contiguous())
-            grus.append(self._flat_gru_states[i])
-            mf.append(self._flat_mamba_fwd_states[i])
-            mb.append(self._flat_mamba_bwd_states[i])
-            cots.append(-torch.where(norm > 1e-12, vg / norm, vg).reshape(-1))
-        if grads:
-            _bilevel.accumulate_meta_gradients(self.meta_net, grads, sharps, grus, mf, mb, cots)
+        picked = [(saved[n].detach(), p.grad.detach(), i) for n, p, i in picked if p.grad is not None]
+        if picked:
+            at = [i for _, _, i in picked]
+            state = [[kept[i] for i in at] for kept in (self._flat_sharpness, self._flat_gru_states, self._flat_mamba_fwd_states,
+                                                        self._flat_mamba_bwd_states)]
+            _bilevel.accumulate_meta_gradients(self.meta_net, [g for g, _, _ in picked], *state, [v for _, v, _ in picked],
+                                               validation=True, want_smart=False)
             meta_optimizer.step()
             self._weights_dirty = True
         for n, p in named:
