@@ -9,30 +9,36 @@
 // the state entering every 32nd step; the per-element part of the meta-net (GRU, soft top-4 PEER routing,
 // experts) is differentiated by torch autograd on the caller's side.
 //
-// The adjoint state lambda obeys a linear recurrence over the scan steps in reverse, so a tensor is cut into the
-// chunks of the forward pass and handled in three launches, like the forward scan:
+// The adjoint state lambda obeys a linear recurrence over the scan steps in reverse.  Its transfer map contracts like
+// the forward recurrence's, so it is not handed from chunk to chunk: k_adjoint gives every wave a range of steps of equal
+// length, and the wave starts its walk behind the end of its range, at lambda = 0, as many steps as it takes for the
+// map from there to fall below 2^-64 (the bound the forward summaries use; checked by the product of the steps' norms, and
+// exact where the walk starts at the tensor's end).  Where the forward pass found a chunk whose map does not contract
+// (Plan::contracted is 0) the ranges are the forward pass's chunks, and two more launches hand lambda over exactly:
 //   k_adj_summary  per (chunk, direction): the affine map lambda_end-of-chunk -> lambda_start-of-chunk
 //                  (a 2x2 matrix and an offset per lane), which needs only d y of every step, not the states;
 //   k_adj_prefix   per (tensor, direction): composes the maps from the last chunk to the first, leaving the adjoint
-//                  state that arrives at the end of every chunk;
-//   k_bilevel_backward  per (chunk, direction), exact from that arriving state.  A 128-lane workgroup walks the
-//                  chunk's 32-step tiles from the last to the first, lane (j,p) owning column j and RoPE pair p
-//                  as in the forward kernels.  Per tile:
-//   1  projections of the 32 steps from (g, s) and the composed coefficients, with the derivatives of softplus
-//      and SiLU, and the incoming context gradients gathered from element order;
-//   2  the forward recurrence from the saved tile-start state, keeping the state after every step in LDS;
-//   3  per step and column: out, d out = out_proj^T d ctx, d y, d z, the D-skip part of d x-branch;
-//   4  the adjoint recurrence over the steps in reverse: lambda <- R(theta)^T diag(A_bar) (lambda + d y C), with
-//      the gradients of dt, x-branch, B and C per step (reduced over pairs / columns) and of A_log and the RoPE
-//      frequencies per lane;
-//   5  sums over the tile's steps: composed-coefficient gradients d v (x) (g, s, 1) of x-branch, z and dt (those of B
-//      and C are summed per lane during 4 and reduced over columns once per workgroup), d D, d out_proj.
-// Nothing is truncated: the result is the exact adjoint.  Gradients of the composed coefficients are carried back
-// to input_proj / in_proj / dt_proj / B_proj / C_proj by a last one-workgroup kernel (k_compose_backward, the
-// transpose of the composition).  Every workgroup keeps its sums in registers over the chunks it handles and writes them to its own
-// row of a partials buffer, which k_adj_sum_rows adds in a fixed order: the result is reproducible run to run.
+//                  state that arrives at the end of every chunk.
+// (They return at once in the usual case: handing lambda over that way cost 0.15 ms of the pass on 0.42 M elements.)
+//
+// A range is walked in tiles of 16 steps from the last to the first.  Per tile:
+//   1  projections of the 16 steps from (g, s) and the composed coefficients, the incoming context gradients and
+//      d out = out_proj^T d ctx, d y;
+//   2  from the kept state at the tile's start, in blocks of four steps, last block first: the forward recurrence once more,
+//      then the adjoint  lambda <- R(theta)^T diag(A_bar) (lambda + d y C)  with the gradients of dt, x-branch, B and C
+//      per step (reduced over pairs / columns) and of A_log and the RoPE frequencies per lane;
+//   3  per step and column: out, d z and the rest of d x-branch and d dt, and the sums over the tile's steps:
+//      composed-coefficient gradients d v (x) (g, s, 1), d D, d out_proj.
+// Gradients of the composed coefficients are carried back to input_proj / in_proj / dt_proj / B_proj / C_proj by a last
+// one-workgroup kernel (k_compose_backward, the transpose of the composition).  Every wave keeps its sums in registers
+// over the steps it handles and writes them to its own row of a partials buffer, which k_adj_sum_rows adds in a fixed
+// order: the result is reproducible run to run.
+// k_bilevel_backward is the form with the gradient of the input projection as a second output, chunk by chunk.
+#include <algorithm>
+
 #include "sg2_internal.hpp"
 #include "../../include/sg2_compose.h"
+#include "sg2_pair_sums.hpp"
 
 namespace sg2 {
 namespace {
@@ -41,9 +47,9 @@ constexpr int BST = SCAN_TT + 4;                 // row stride of the [16][64] L
 constexpr int ROWS = 16;
 // LDS arrays of ROWS x BST floats
 enum { A_DT, A_DSP, A_XB, A_B, A_C, A_GATE, A_DGATE, A_Y, A_DY, A_DZ, A_DXB, A_DDT, A_COUNT };
-// The gradient kernel works on tiles of BT = HT_STEP steps (half a forward tile), which keeps its LDS below half
+// k_bilevel_backward works on tiles of BT steps (half a forward tile), which keeps its LDS below half
 // a CU's so that two workgroups share a CU.
-constexpr int BT = HT_STEP;
+constexpr int BT = 2 * HT_STEP;
 constexpr int BBST = BT + 1;                     // row stride of its [16][BT] arrays (odd: the 16 rows a step reads hit 16 banks)
 constexpr int LDS_ROWS_FLOATS = A_COUNT * ROWS * BBST;
 constexpr int LDS_H_FLOATS = BT * SCAN_THREADS * 2;               // state after every step of the tile
@@ -143,9 +149,9 @@ __device__ __forceinline__ void adj_apply(float ae, float ao, float sn, float cs
     *xo = sg_fma(dro, cs, -(dre * sn));
 }
 
-// ---- launch 1: affine map of the adjoint state across every chunk
+// ---- affine map of the adjoint state across every chunk
 constexpr int SUMM_ROWS = 4;                     // LDS arrays of the summary kernel: dt, C, gate, d y
-__global__ __launch_bounds__(SCAN_THREADS) void k_adj_summary(Plan pl, AdjIO io) {
+__global__ __launch_bounds__(SCAN_THREADS) void k_adj_summary(Plan pl, AdjIO io, bool use_flag) {
     __shared__ float rows[SUMM_ROWS * ROWS * BST];
     __shared__ __attribute__((aligned(16))) float s_dctx[SCAN_TT * DM];
     __shared__ float s_fmax[DI];
@@ -162,6 +168,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_adj_summary(Plan pl, AdjIO io)
     const int j = tid >> 3, p = tid & 7;
     const float a_e = 0.5f * sg_exp(Alog[j * DS + 2 * p]), a_o = 0.5f * sg_exp(Alog[j * DS + 2 * p + 1]);
     const float freq = rope[j * HP + p];
+    if (use_flag && *pl.contracted != 0) return;   // nobody reads the maps
     if (chunk == pl.chunk_prefix[c.ti]) return;    // nothing lies before a tensor's first chunk: its map is never applied
     fill_fmax(s_fmax, rope);
     float u1e, u1o, u2e, u2o, ve, vo;
@@ -241,8 +248,9 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_adj_summary(Plan pl, AdjIO io)
     out[0] = u1e; out[1] = u1o; out[2] = u2e; out[3] = u2o; out[4] = ve; out[5] = vo;
 }
 
-// ---- launch 2: adjoint state arriving at the end of every chunk, last chunk of a tensor first
-__global__ __launch_bounds__(SCAN_THREADS) void k_adj_prefix(Plan pl) {
+// ---- adjoint state arriving at the end of every chunk, last chunk of a tensor first
+__global__ __launch_bounds__(SCAN_THREADS) void k_adj_prefix(Plan pl, bool use_flag) {
+    if (use_flag && *pl.contracted != 0) return;
     const int ti = blockIdx.x, dir = blockIdx.y, tid = threadIdx.x;
     const int base = pl.chunk_prefix[ti], nc = pl.chunk_prefix[ti + 1] - base;
     float le = 0.0f, lo = 0.0f;
@@ -259,9 +267,556 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_adj_prefix(Plan pl) {
     }
 }
 
-// ---- launch 3: the gradients, chunk by chunk
-template <bool DX>
+// ---- the gradients, range by range
+// One wave per (range, direction); eight per CU.  Lane roles within a tile: step st = lane % 16 with rows 4 (lane / 16) .. + 3
+// of every 16-row group (projections, part 3), and column jl = lane / 8 and jl + 8 with RoPE pair p = lane % 8 (recurrence):
+// the two columns share their B and C, the gradients of B and C add up over both before they go anywhere, and their
+// sums against (g, s, 1) are 4 x 4 x 1 matrix instructions, one per step and entry.
+// A tile of 16 whole steps whose inputs are small enough takes polynomials: softplus, SiLU and their derivatives as cubics
+// around the constant of their row (sg2_taylor_ok), A_bar as a cubic, sin and cos as quadratics in d = dt - dt0 (remainders
+// below 5e-8 while a d < 1/80, f d < 1/256; limits from compose_block).  Other tiles, and the ragged last one of a tensor, take the functions
+// themselves.
+// Bound by the vector ALU: 160 instructions per step (for its 256 states), 78 % of the time one is issued.  18.9 ms on 25 M
+// elements, 0.40 ms on 0.42 M; 53.5 and 1.14 as one 128-lane workgroup per chunk with one wave per SIMD, the exact functions
+// at every step and all states of a tile in LDS.
+constexpr int AT = HT_STEP;             // steps per tile
+constexpr int AB = 4;                   // steps per block
+constexpr int FLUSH_TILES = 64;         // tiles between two writes of the sums
+constexpr int ADJ_STRIDE = 4 * DI + 4;  // per step: (dt, dt - dt0, dt * x-branch, d y) of the 16 columns; later (d x-branch, d dt, d z, out)
+constexpr int BC_STRIDE = 4 * HP + 4;   // per step: (B even, B odd, C even, C odd) of the 8 pairs
+constexpr int SUM_STRIDE = AT + 4;      // per column: sums over the pairs of every step
+constexpr int IN_STRIDE = 17;           // per step: g, s, 1, d ctx[8]
+typedef float adj_f32x4 __attribute__((ext_vector_type(4)));
+
+// sigmoid and the derivative of SiLU as cubics around c (as sg2_softplus_taylor, sg2_silu_taylor)
+__device__ __forceinline__ void sigmoid_taylor(float c, float t[4]) {
+    const float s = sg_sigmoid(c), q = s * (1.0f - s), r = 1.0f - (s + s);
+    t[0] = s;
+    t[1] = q;
+    t[2] = 0.5f * (q * r);
+    t[3] = (q * sg_fma(r, r, -(q + q))) * 0.166666672f;
+}
+__device__ __forceinline__ void dsilu_taylor(float c, float t[4]) {
+    const float s = sg_sigmoid(c), q = s * (1.0f - s), r = 1.0f - (s + s);
+    const float a = sg_fma(r, sg_fma(c, r, 3.0f), -((c + c) * q));          // third derivative of SiLU over q
+    t[0] = sg_fma(c, q, s);
+    t[1] = q * sg_fma(c, r, 2.0f);
+    t[2] = 0.5f * (q * a);
+    t[3] = (q * (sg_fma(r, a, sg_fma(r, r, -8.0f * q)) - 6.0f * (c * q) * r)) * 0.166666672f;
+}
+__device__ __forceinline__ float cubic(const adj_f32x4 t, float d) { return sg_fma(sg_fma(sg_fma(t[3], d, t[2]), d, t[1]), d, t[0]); }
+
+template <bool SCAN_GRADS>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adjoint(Plan pl, AdjIO io) {      // SCAN_GRADS: the gradient of the gated outputs comes in instead of that of the contexts
+    static_assert(AT == 16 && DI == 16 && DS == 16 && HP == 8 && DM == 8 && AB == 4, "lane roles");
+    __shared__ __attribute__((aligned(16))) float s_a[AT * ADJ_STRIDE];
+    __shared__ __attribute__((aligned(16))) float s_b[AT * BC_STRIDE];
+    __shared__ __attribute__((aligned(16))) float s_y[DI * SUM_STRIDE], s_q[DI * SUM_STRIDE], s_d[DI * SUM_STRIDE];     // y, d / d (dt * x-branch), d dt but for that
+    __shared__ __attribute__((aligned(16))) float s_in[AT * IN_STRIDE], s_gt[4 * SUM_STRIDE];      // inputs per step; g, s, 1 per row
+    __shared__ __attribute__((aligned(16))) float s_h[(AT / AB) * 64 * 4];        // the lanes' states at the starts of the blocks
+    __shared__ __attribute__((aligned(16))) float s_k[2 * 64 * 4];                // gate and d out of the lanes' steps and rows, for part 3
+    __shared__ __attribute__((aligned(16))) float s_coef[SG2_COMP_GROUPS * DI * 4];   // composed triples, D beside the x-branch's
+    __shared__ __attribute__((aligned(16))) float s_tay[4 * DI * 4];              // dt, its derivative, gate, its derivative
+
+    const int lane = threadIdx.x, dir = blockIdx.y;
+    const int st = lane & 15, rg = lane >> 4;
+    const int jl = lane >> 3, p = lane & 7;
+    const int b = dir ? W_B_INPROJ : W_F_INPROJ;
+    const float* __restrict__ Wout = pl.W.w[b + 8];
+
+    // ---- tables and the lane's constants
+    {
+        const float* comp = pl.comp + dir * (SG2_COMP_GROUPS * DI * 3);
+        const float* tay = pl.comp + 2 * SG2_COMP_GROUPS * DI * 3 + dir * 2 * DI * 4;
+        const float* Dw = pl.W.w[b + 6];
+        for (int i = lane; i < SG2_COMP_GROUPS * DI; i += 64) {
+            const float* t = comp + i * 3;
+            *reinterpret_cast<adj_f32x4*>(s_coef + i * 4) = adj_f32x4{t[0], t[1], t[2], i / DI == SG2_COMP_XB ? Dw[i % DI] : 0.0f};
+        }
+        // (the forward pass's own polynomials for dt and gate)
+        s_tay[lane] = tay[lane];
+        s_tay[2 * DI * 4 + lane] = tay[DI * 4 + lane];
+        if (lane < DI) {
+            float t[4];
+            sigmoid_taylor(comp[(SG2_COMP_DT * DI + lane) * 3 + 2], t);
+            *reinterpret_cast<adj_f32x4*>(s_tay + (DI + lane) * 4) = adj_f32x4{t[0], t[1], t[2], t[3]};
+            dsilu_taylor(comp[(SG2_COMP_Z * DI + lane) * 3 + 2], t);
+            *reinterpret_cast<adj_f32x4*>(s_tay + (3 * DI + lane) * 4) = adj_f32x4{t[0], t[1], t[2], t[3]};
+        }
+        for (int i = lane; i < AT * IN_STRIDE; i += 64) s_in[i] = 0.0f;
+        for (int i = lane; i < 4 * SUM_STRIDE; i += 64) s_gt[i] = 0.0f;
+        __syncthreads();
+    }
+    float pe[2][4], po[2][4], qs[2][3], qc[2][3];       // A_bar even / odd, sin, cos of the lane's two pairs as polynomials in dt - dt0
+    float se[2], so[2], freq[2];                        // -a/2 of the two poles (a = -A/2), rotation frequency
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int j = jl + 8 * h;
+        const float dt0 = s_tay[j * 4];
+        const float a_e = 0.5f * sg_exp(pl.W.w[b + 5][j * DS + 2 * p]), a_o = 0.5f * sg_exp(pl.W.w[b + 5][j * DS + 2 * p + 1]);
+        freq[h] = pl.W.w[b + 7][j * HP + p];
+        se[h] = -0.5f * a_e;
+        so[h] = -0.5f * a_o;
+        sg2_abar_poly(dt0, a_e, pe[h]);
+        sg2_abar_poly(dt0, a_o, po[h]);
+        sg2_sincos_poly(dt0, freq[h], qs[h], qc[h]);
+    }
+    const float wo0 = Wout[rg * DI + st], wo1 = Wout[(4 + rg) * DI + st];      // operand of d out = out_proj^T d ctx
+    const sg::cfloat_p lim = sg::as_const(pl.comp) + 2 * SG2_COMP_GROUPS * DI * 3 + 2 * 2 * DI * 4;
+    const float cmax_g = lim[2 * dir], cmax_s = lim[2 * dir + 1], kcub_g = lim[12 + 2 * dir], kcub_s = lim[13 + 2 * dir];
+
+    // ---- sums
+    const adj_f32x4 zero4 = adj_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    float al_e[2] = {0.0f, 0.0f}, al_o[2] = {0.0f, 0.0f}, rope[2] = {0.0f, 0.0f};
+    adj_f32x4 aBe = zero4, aBo = zero4, aCe = zero4, aCo = zero4;
+    adj_f32x4 a16[4] = {zero4, zero4, zero4, zero4};     // rows x (g, s, 1, d ctx): d x-branch, d dt, d z, out
+    float accD[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+
+    // this wave's sums -> its row of the partials buffer, every FLUSH_TILES tiles: one chain of additions over all of a
+    // wave's steps would lose two digits of the sums of B and C where these nearly cancel (an entry is always the same lane's)
+    float* const row = pl.adj_part + ((size_t)dir * gridDim.x + blockIdx.x) * SG2_BWD_STRIDE;
+    for (int i = lane; i < SG2_BWD_STRIDE; i += 64) row[i] = 0.0f;
+    __syncthreads();
+    int unflushed = 0;
+    auto flush = [&]() {
+        float* const g_comp = row;
+        float* const g_alog = g_comp + SG2_COMP_GROUPS * DI * 3;
+        float* const g_rope = g_alog + DI * DS;
+        float* const g_D = g_rope + DI * HP;
+        float* const g_wout = g_D + DI;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int j = jl + 8 * h;
+            g_alog[j * DS + 2 * p] += al_e[h] * se[h];
+            g_alog[j * DS + 2 * p + 1] += al_o[h] * so[h];
+            g_rope[j * HP + p] += rope[h];
+            al_e[h] = al_o[h] = rope[h] = 0.0f;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            // 16 x 16: rows 4 rg + v, column st
+            if (st < 3) {
+                g_comp[(SG2_COMP_XB * DI + 4 * rg + v) * 3 + st] += a16[0][v];
+                g_comp[(SG2_COMP_DT * DI + 4 * rg + v) * 3 + st] += a16[1][v];
+                g_comp[(SG2_COMP_Z * DI + 4 * rg + v) * 3 + st] += a16[2][v];
+            } else if (st < 3 + DM) {
+                g_wout[(st - 3) * DI + 4 * rg + v] += a16[3][v];
+            }
+            // 4 x 4: the pair of lane 4 (lane / 4) + v against column lane % 4; added over the columns jl
+            auto over_columns = [](float x) {
+                x += __shfl_xor(x, 8, 64);
+                x += __shfl_xor(x, 16, 64);
+                return x + __shfl_xor(x, 32, 64);
+            };
+            const float sums[4] = {over_columns(aBe[v]), over_columns(aBo[v]), over_columns(aCe[v]), over_columns(aCo[v])};
+            if (lane < 8 && (lane & 3) < 3) {
+                const int pr = (lane & 4) + v;
+#pragma unroll
+                for (int q = 0; q < 4; q++) g_comp[((q < 2 ? SG2_COMP_B : SG2_COMP_C) * DI + 2 * pr + (q & 1)) * 3 + (lane & 3)] += sums[q];
+            }
+            float d = accD[v];
+#pragma unroll
+            for (int m = 8; m >= 1; m >>= 1) d += __shfl_xor(d, m, 64);
+            if (st == 0) g_D[4 * rg + v] += d;
+        }
+        aBe = aBo = aCe = aCo = zero4;
+#pragma unroll
+        for (int q = 0; q < 4; q++) { a16[q] = zero4; accD[q] = 0.0f; }
+        unflushed = 0;
+    };
+
+    // ---- the tensor at hand
+    int ti = 0, N = 0, off = 0;
+    bool has_s = false;
+    float le[2] = {0.0f, 0.0f}, lo[2] = {0.0f, 0.0f};
+    const float* dctx = nullptr;
+    const float* dscan = nullptr;
+
+    // what a tile reads from memory, requested one tile ahead
+    struct Inputs { uint32_t key; int32_t val; float s, d0, d1; adj_f32x4 ds, h; };
+    auto request = [&](int u0, bool with_state) {
+        Inputs in = {0, 0, 0.0f, 0.0f, 0.0f, zero4, zero4};
+        const int u = u0 + st;
+        if (u < N) {
+            const int t = dir ? N - 1 - u : u;
+            in.key = pl.keys[0][off + t];
+            in.val = pl.vals[0][off + t];
+            if (has_s) in.s = pl.ssorted[off + t];
+            if (SCAN_GRADS) {
+                in.ds = *reinterpret_cast<const adj_f32x4*>(dscan + (size_t)u * DI + 4 * rg);
+            } else {
+                const int at = pl.own_order ? t : min(in.val & 0x7fffffff, N - 1);
+                in.d0 = dctx[(size_t)at * DM + rg];
+                in.d1 = dctx[(size_t)at * DM + 4 + rg];
+            }
+        }
+        if (with_state) {
+            const float* ht = pl.htile + ((size_t)dir * htile_count(pl.total, pl.P) + htile_index(off, ti, u0)) * 2 * SCAN_THREADS;
+            in.h = adj_f32x4{ht[lane], ht[SCAN_THREADS + lane], ht[64 + lane], ht[SCAN_THREADS + 64 + lane]};
+        }
+        return in;
+    };
+
+    // A_bar, sin, cos of the lane's pair h
+    auto coefficients = [&](auto fast_c, int h, float dt, float d, float& ae, float& ao, float& sn, float& cs) {
+        if (decltype(fast_c)::value) {
+            ae = sg2_poly3(pe[h], d);
+            ao = sg2_poly3(po[h], d);
+            sn = sg2_poly2(qs[h], d);
+            cs = sg2_poly2(qc[h], d);
+        } else {
+            sg_abar_pair(dt, -2.0f * se[h], -2.0f * so[h], &ae, &ao);
+            sg_sincos(dt * freq[h], &sn, &cs);
+        }
+    };
+
+    // operands of a step of the recurrence: its two columns, its B and C.  They are fetched one step ahead, and fetched_here()
+    // keeps the compiler from moving a fetch down to where it is used (with registers scarce it does, and waits each time).
+    struct Step { adj_f32x4 a[2], bc; };
+    auto step_at = [&](int k) {
+        Step o;
+        o.a[0] = *reinterpret_cast<const adj_f32x4*>(s_a + k * ADJ_STRIDE + 4 * jl);
+        o.a[1] = *reinterpret_cast<const adj_f32x4*>(s_a + k * ADJ_STRIDE + 4 * jl + 32);
+        o.bc = *reinterpret_cast<const adj_f32x4*>(s_b + k * BC_STRIDE + 4 * p);
+        return o;
+    };
+    auto fetched_here = []() { asm volatile("" ::: "memory"); };
+
+    // part 1 -> s_a, s_b, s_in, s_gt; gate and d out of the lane's step and rows -> s_k
+    struct Rows { float g, s; bool valid; };
+    auto project = [&](auto fast_c, const Inputs& in, int cnt, float g, float s) {
+        constexpr bool FAST = decltype(fast_c)::value;
+        Rows R;
+        R.g = g; R.s = s; R.valid = st < cnt;
+        adj_f32x4 dout = in.ds;
+        if (!SCAN_GRADS) {
+            dout = __builtin_amdgcn_mfma_f32_16x16x4f32(wo0, in.d0, zero4, 0, 0, 0);
+            dout = __builtin_amdgcn_mfma_f32_16x16x4f32(wo1, in.d1, dout, 0, 0, 0);
+        }
+        if (rg == 0) {
+            s_gt[st] = g; s_gt[SUM_STRIDE + st] = s; s_gt[2 * SUM_STRIDE + st] = R.valid ? 1.0f : 0.0f;
+            s_in[st * IN_STRIDE] = g; s_in[st * IN_STRIDE + 1] = s; s_in[st * IN_STRIDE + 2] = R.valid ? 1.0f : 0.0f;
+        }
+        s_in[st * IN_STRIDE + 3 + rg] = in.d0;
+        s_in[st * IN_STRIDE + 7 + rg] = in.d1;
+        float B[4], C[4];
+        adj_f32x4 gate;
+        auto eval = [&](const adj_f32x4 c) { return sg_fma(c[0], g, sg_fma(c[1], s, c[2])); };
+#pragma unroll
+        for (int v0 = 0; v0 < 4; v0 += 2) {
+            adj_f32x4 c[2][SG2_COMP_GROUPS], td[2], tg[2];
+#pragma unroll
+            for (int v = 0; v < 2; v++) {
+                const int row = 4 * rg + v0 + v;
+#pragma unroll
+                for (int q = 0; q < SG2_COMP_GROUPS; q++) c[v][q] = *reinterpret_cast<const adj_f32x4*>(s_coef + (q * DI + row) * 4);
+                td[v] = *reinterpret_cast<const adj_f32x4*>(s_tay + row * 4);
+                tg[v] = *reinterpret_cast<const adj_f32x4*>(s_tay + (2 * DI + row) * 4);
+            }
+            fetched_here();
+#pragma unroll
+            for (int v = v0; v < v0 + 2; v++) {
+                const adj_f32x4 (&cv)[SG2_COMP_GROUPS] = c[v - v0];
+                const adj_f32x4 cd = cv[SG2_COMP_DT], cz = cv[SG2_COMP_Z];
+                float dt;
+                if (FAST) {
+                    dt = cubic(td[v - v0], sg_fma(cd[0], g, cd[1] * s));
+                    gate[v] = cubic(tg[v - v0], sg_fma(cz[0], g, cz[1] * s));
+                } else {
+                    dt = R.valid ? sg_softplus(eval(cd)) : 0.0f;
+                    const float z = eval(cz);
+                    gate[v] = z * sg_sigmoid(z);
+                    if (!R.valid) dout[v] = 0.0f;
+                }
+                const float xb = FAST || R.valid ? eval(cv[SG2_COMP_XB]) : 0.0f;
+                B[v] = eval(cv[SG2_COMP_B]);
+                C[v] = eval(cv[SG2_COMP_C]);
+                *reinterpret_cast<adj_f32x4*>(s_a + st * ADJ_STRIDE + 4 * (4 * rg + v)) = adj_f32x4{dt, FAST ? dt - td[v - v0][0] : dt, dt * xb, dout[v] * gate[v]};
+            }
+        }
+        reinterpret_cast<adj_f32x4*>(s_k)[lane] = gate;
+        reinterpret_cast<adj_f32x4*>(s_k)[64 + lane] = dout;
+        *reinterpret_cast<adj_f32x4*>(s_b + st * BC_STRIDE + 8 * rg) = adj_f32x4{B[0], B[1], C[0], C[1]};
+        *reinterpret_cast<adj_f32x4*>(s_b + st * BC_STRIDE + 8 * rg + 4) = adj_f32x4{B[2], B[3], C[2], C[3]};
+        __syncthreads();       // one wave: no s_barrier is issued, the LDS writes above are ordered before the reads below
+        return R;
+    };
+    // (g, s) of the lane's step, and whether the whole tile may take the polynomials
+    auto unpack = [&](const Inputs& in, int cnt, float& g, float& s) {
+        const bool valid = st < cnt;
+        g = valid ? sg_i2f((int32_t)in.key | (in.val & (int32_t)0x80000000)) : 0.0f;
+        s = valid ? in.s : 0.0f;
+        return cnt == AT && __builtin_amdgcn_ballot_w64(!(sg2_taylor_ok(cmax_g, cmax_s, g, s) && sg2_poly_ok(kcub_g, kcub_s, g, s))) == 0;
+    };
+
+    // lambda alone, from step v_end (0 there) to u_end; bound: product of the norms of the steps' maps
+    auto approach = [&](int v_end, int u_end, float& bound) {
+        float bd[2] = {1.0f, 1.0f};
+        le[0] = le[1] = lo[0] = lo[1] = 0.0f;
+        const int first = u_end, last = first + ((v_end - first - 1) / AT) * AT;
+        Inputs next = request(last, false);
+        for (int u0 = last; u0 >= first; u0 -= AT) {
+            const Inputs in = next;
+            if (u0 > first) next = request(u0 - AT, false);
+            const int cnt = min(AT, v_end - u0);
+            float g, s;
+            const bool fast = unpack(in, cnt, g, s);
+            auto walk = [&](auto fast_c) {
+                project(fast_c, in, cnt, g, s);
+                Step o = step_at(cnt - 1);
+#pragma unroll 2
+                for (int k = cnt - 1; k >= 0; k--) {
+                    const Step now = o;
+                    o = step_at(max(k - 1, 0));
+                    fetched_here();
+                    const adj_f32x4 bc = now.bc;
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const adj_f32x4 a = now.a[h];
+                        float ae, ao, sn, cs;
+                        coefficients(fast_c, h, a[0], a[1], ae, ao, sn, cs);
+                        const float dre = sg_fma(a[3], bc[2], le[h]) * ae, dro = sg_fma(a[3], bc[3], lo[h]) * ao;
+                        le[h] = sg_fma(dre, cs, dro * sn);
+                        lo[h] = sg_fma(dro, cs, -(dre * sn));
+                        bd[h] *= sg_max(sg_abs(ae), sg_abs(ao));
+                    }
+                }
+            };
+            if (fast) walk(std::true_type{});
+            else walk(std::false_type{});
+            __syncthreads();
+        }
+        bound = sg_max(bd[0], bd[1]);
+    };
+
+    // the gradients of steps [u_lo, u_hi), lambda behind them given; u_lo is a multiple of AT
+    auto range = [&](int u_lo, int u_hi) {
+        const int last = u_lo + ((u_hi - u_lo - 1) / AT) * AT;
+        Inputs next = request(last, true);
+        for (int u0 = last; u0 >= u_lo; u0 -= AT) {
+            const Inputs in = next;
+            if (u0 > u_lo) next = request(u0 - AT, true);
+            const int cnt = min(AT, u_hi - u0);
+            float g, s;
+            const bool fast = unpack(in, cnt, g, s);
+            auto walk = [&](auto fast_c) {
+                constexpr bool FAST = decltype(fast_c)::value;
+                const Rows R = project(fast_c, in, cnt, g, s);
+                // ---- 2: states at the starts of the blocks
+                adj_f32x4* const sh = reinterpret_cast<adj_f32x4*>(s_h) + lane;
+                {
+                    adj_f32x4 hh = in.h;
+                    sh[0] = hh;
+                    Step o = step_at(0);
+#pragma unroll 1
+                    for (int k0 = 0; k0 < AT - AB; k0 += AB) {
+#pragma unroll
+                        for (int u = 0; u < AB; u++) {
+                            const Step now = o;
+                            o = step_at(k0 + u + 1);
+                            fetched_here();
+                            const adj_f32x4 bc = now.bc;
+#pragma unroll
+                            for (int h = 0; h < 2; h++) {
+                                const adj_f32x4 a = now.a[h];
+                                float ae, ao, sn, cs;
+                                coefficients(fast_c, h, a[0], a[1], ae, ao, sn, cs);
+                                const float re = sg_fma(hh[2 * h], cs, -(hh[2 * h + 1] * sn)), ro = sg_fma(hh[2 * h + 1], cs, hh[2 * h] * sn);
+                                hh[2 * h] = sg_fma(ae, re, a[2] * bc[0]);
+                                hh[2 * h + 1] = sg_fma(ao, ro, a[2] * bc[1]);
+                            }
+                        }
+                        sh[(k0 / AB + 1) * 64] = hh;
+                    }
+                }
+                // ---- the blocks, last first (a ragged tile: its steps past the end leave lambda alone and add nothing, their
+                // dt, x-branch and d y being 0)
+                Step o = step_at(AT - AB);
+                adj_f32x4 h_next = sh[(AT / AB - 1) * 64];
+#pragma unroll 1
+                for (int k0 = AT - AB; k0 >= 0; k0 -= AB) {
+                    const adj_f32x4 h0 = h_next;
+                    float ae[2][AB], ao[2][AB], sn[2][AB], cs[2][AB], re[2][AB], ro[2][AB], he[2][AB + 1], ho[2][AB + 1];
+                    float y[8];
+                    he[0][0] = h0[0]; ho[0][0] = h0[1]; he[1][0] = h0[2]; ho[1][0] = h0[3];
+#pragma unroll
+                    for (int u = 0; u < AB; u++) {
+                        const Step now = o;
+                        if (u < AB - 1) {
+                            o = step_at(k0 + u + 1);
+                            fetched_here();
+                        }
+                        const adj_f32x4 bc = now.bc;
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            const adj_f32x4 a = now.a[h];
+                            coefficients(fast_c, h, a[0], a[1], ae[h][u], ao[h][u], sn[h][u], cs[h][u]);
+                            re[h][u] = sg_fma(he[h][u], cs[h][u], -(ho[h][u] * sn[h][u]));
+                            ro[h][u] = sg_fma(ho[h][u], cs[h][u], he[h][u] * sn[h][u]);
+                            he[h][u + 1] = sg_fma(ae[h][u], re[h][u], a[2] * bc[0]);
+                            ho[h][u + 1] = sg_fma(ao[h][u], ro[h][u], a[2] * bc[1]);
+                            y[4 * h + u] = sg_fma(ho[h][u + 1], bc[3], he[h][u + 1] * bc[2]);
+                        }
+                    }
+                    // (the operands of the four steps are fetched again below, from the last, still at hand, down: held they would spill)
+                    const adj_f32x4 gt = *reinterpret_cast<const adj_f32x4*>(s_gt + (lane & 3) * SUM_STRIDE + k0);
+                    fetched_here();
+                    block_pair_sums<HP>(y);
+                    float q[8], dd[8];
+#pragma unroll
+                    for (int u = AB - 1; u >= 0; u--) {
+                        float tBe = 0.0f, tBo = 0.0f, tCe = 0.0f, tCo = 0.0f;
+                        const Step now = o;
+                        o = step_at(max(u > 0 ? k0 + u - 1 : k0 - AB, 0));
+                        if (u == 0) h_next = sh[max(k0 / AB - 1, 0) * 64];
+                        fetched_here();
+                        const adj_f32x4 bc = now.bc;
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            const adj_f32x4 a = now.a[h];
+                            const float dt = a[0], ux = a[2], dy = a[3];
+                            // y = sum h C
+                            const float l_e = sg_fma(dy, bc[2], le[h]), l_o = sg_fma(dy, bc[3], lo[h]);
+                            tCe = sg_fma(dy, he[h][u + 1], tCe);
+                            tCo = sg_fma(dy, ho[h][u + 1], tCo);
+                            // h' = A_bar * rot(h) + dt * xb * B
+                            tBe = sg_fma(l_e, ux, tBe);
+                            tBo = sg_fma(l_o, ux, tBo);
+                            q[4 * h + u] = sg_fma(l_e, bc[0], l_o * bc[1]);
+                            // A_bar = 2/(1 + a dt) - 1: dA_bar/d dt = -a/2 (A_bar + 1)^2
+                            const float ve = ae[h][u] + 1.0f, vo = ao[h][u] + 1.0f;
+                            const float te = (l_e * re[h][u]) * (ve * ve), to = (l_o * ro[h][u]) * (vo * vo);
+                            al_e[h] = sg_fma(te, dt, al_e[h]);
+                            al_o[h] = sg_fma(to, dt, al_o[h]);
+                            // lambda for the previous step; d theta = d ro * re - d re * ro
+                            const float dre = l_e * ae[h][u], dro = l_o * ao[h][u];
+                            const float dth = sg_fma(dro, re[h][u], -(dre * ro[h][u]));
+                            rope[h] = sg_fma(dth, dt, rope[h]);
+                            dd[4 * h + u] = sg_fma(dth, freq[h], sg_fma(te, se[h], to * so[h]));
+                            const float n_e = sg_fma(dre, cs[h][u], dro * sn[h][u]), n_o = sg_fma(dro, cs[h][u], -(dre * sn[h][u]));
+                            le[h] = FAST || k0 + u < cnt ? n_e : le[h];
+                            lo[h] = FAST || k0 + u < cnt ? n_o : lo[h];
+                        }
+                        aBe = __builtin_amdgcn_mfma_f32_4x4x1f32(tBe, gt[u], aBe, 0, 0, 0);
+                        aBo = __builtin_amdgcn_mfma_f32_4x4x1f32(tBo, gt[u], aBo, 0, 0, 0);
+                        aCe = __builtin_amdgcn_mfma_f32_4x4x1f32(tCe, gt[u], aCe, 0, 0, 0);
+                        aCo = __builtin_amdgcn_mfma_f32_4x4x1f32(tCo, gt[u], aCo, 0, 0, 0);
+                    }
+                    block_pair_sums<HP>(q);
+                    block_pair_sums<HP>(dd);
+                    if ((p & 3) == 0) {      // lanes p = 0 hold the sums of column jl, p = 4 those of column jl + 8
+                        const int at = (jl + 2 * p) * SUM_STRIDE + k0;
+                        *reinterpret_cast<adj_f32x4*>(s_y + at) = adj_f32x4{y[0], y[1], y[2], y[3]};
+                        *reinterpret_cast<adj_f32x4*>(s_q + at) = adj_f32x4{q[0], q[1], q[2], q[3]};
+                        *reinterpret_cast<adj_f32x4*>(s_d + at) = adj_f32x4{dd[0], dd[1], dd[2], dd[3]};
+                    }
+                }
+                __syncthreads();
+                // ---- 3
+                const adj_f32x4 gate = reinterpret_cast<adj_f32x4*>(s_k)[lane], dout = reinterpret_cast<adj_f32x4*>(s_k)[64 + lane];
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int row = 4 * rg + v;
+                    const float yv = s_y[row * SUM_STRIDE + st], qb = s_q[row * SUM_STRIDE + st], ddr = s_d[row * SUM_STRIDE + st];
+                    const float dt = s_a[st * ADJ_STRIDE + 4 * row];
+                    const adj_f32x4 cd = *reinterpret_cast<const adj_f32x4*>(s_coef + (SG2_COMP_DT * DI + row) * 4);
+                    const adj_f32x4 cz = *reinterpret_cast<const adj_f32x4*>(s_coef + (SG2_COMP_Z * DI + row) * 4);
+                    const adj_f32x4 cx = *reinterpret_cast<const adj_f32x4*>(s_coef + (SG2_COMP_XB * DI + row) * 4);
+                    const adj_f32x4 td = *reinterpret_cast<const adj_f32x4*>(s_tay + (DI + row) * 4);
+                    const adj_f32x4 tg = *reinterpret_cast<const adj_f32x4*>(s_tay + (3 * DI + row) * 4);
+                    fetched_here();
+                    const float D = cx[3], xb = FAST || R.valid ? sg_fma(cx[0], R.g, sg_fma(cx[1], R.s, cx[2])) : 0.0f;
+                    float dsp, dgate;
+                    if (FAST) {
+                        dsp = cubic(td, sg_fma(cd[0], R.g, cd[1] * R.s));
+                        dgate = cubic(tg, sg_fma(cz[0], R.g, cz[1] * R.s));
+                    } else {
+                        const float raw = sg_fma(cd[0], R.g, sg_fma(cd[1], R.s, cd[2])), z = sg_fma(cz[0], R.g, sg_fma(cz[1], R.s, cz[2]));
+                        const float sz = sg_sigmoid(z);
+                        dsp = raw > 20.0f ? 1.0f : sg_sigmoid(raw);
+                        dgate = sz * sg_fma(z, 1.0f - sz, 1.0f);
+                    }
+                    accD[v] = sg_fma(dout[v], xb, accD[v]);
+                    adj_f32x4 out = adj_f32x4{sg_fma(qb, dt, dout[v] * D), sg_fma(qb, xb, ddr) * dsp, (dout[v] * yv) * dgate,
+                                              sg_fma(yv, gate[v], D * xb)};
+                    if (!FAST && !R.valid) out = zero4;
+                    *reinterpret_cast<adj_f32x4*>(s_a + st * ADJ_STRIDE + 4 * row) = out;
+                }
+                __syncthreads();
+#pragma unroll
+                for (int t = 0; t < AT / 4; t++) {
+                    const adj_f32x4 d = *reinterpret_cast<const adj_f32x4*>(s_a + (4 * t + rg) * ADJ_STRIDE + 4 * st);      // step 4 t + rg, row st
+                    const float in16 = s_in[(4 * t + rg) * IN_STRIDE + st];
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; q4++) a16[q4] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[q4], in16, a16[q4], 0, 0, 0);
+                }
+                __syncthreads();
+            };
+            if (fast) walk(std::true_type{});
+            else walk(std::false_type{});
+            if (++unflushed == FLUSH_TILES) flush();
+        }
+    };
+
+    auto set_tensor = [&](int i) {
+        ti = i;
+        const TensorDev& T = pl.tensors[i];
+        N = T.numel;
+        off = T.off;
+        has_s = __builtin_amdgcn_readfirstlane(pl.sharp_nonzero[i]) != 0;
+        dctx = io.d_ctx ? io.d_ctx + ((size_t)dir * pl.total + off) * DM : nullptr;
+        dscan = io.d_scan[dir] ? io.d_scan[dir] + (size_t)off * DI : nullptr;
+    };
+    // Usual case: the tiles of all tensors in one row (a tensor takes whole elementwise tiles of it), an equal part to every
+    // wave.  Else the chunks of the forward pass, every gridDim.x-th.
+    constexpr int PER = ELEM_TILE / AT;
+    const bool parts = __builtin_amdgcn_readfirstlane(pl.contracted[0]) != 0;
+    const int first_block = __builtin_amdgcn_readfirstlane(pl.contracted[1]);
+    const int64_t tiles = (int64_t)pl.elem_tiles * PER;
+    int at = parts ? (int)(tiles * blockIdx.x / gridDim.x) : (int)blockIdx.x;
+    const int end = parts ? (int)(tiles * (blockIdx.x + 1) / gridDim.x) : pl.chunks;
+    while (at < end) {
+        int u_lo, u_hi;
+        const sg::Seg seg = sg::find_seg(sg::as_const(parts ? pl.elem_tile_prefix : pl.chunk_prefix), pl.P, parts ? at / PER : at);
+        set_tensor(seg.i);
+        le[0] = le[1] = lo[0] = lo[1] = 0.0f;
+        int from, far;                     // where the walk to u_hi starts, and where it starts if that was not far enough
+        if (parts) {
+            const int stop = min(end, seg.end * PER);
+            u_lo = (at - seg.first * PER) * AT;
+            u_hi = min((stop - seg.first * PER) * AT, N);
+            at = stop;
+            // two chunk lengths hold a whole chunk of the forward pass, whose map is known to contract
+            far = min(N, u_hi + 2 * pl.chunk_len);
+            from = first_block > 0 ? min(far, u_hi + (first_block + AT - 1) / AT * AT) : far;
+        } else {
+            u_lo = (at - seg.first) * pl.chunk_len;
+            u_hi = min(N, u_lo + pl.chunk_len);
+            from = far = u_hi;
+            const float* lam = pl.adj_lam + ((size_t)dir * pl.chunks + at) * SCAN_THREADS * 2;
+            if (u_hi < N) {
+#pragma unroll
+                for (int h = 0; h < 2; h++) { le[h] = lam[(lane + 64 * h) * 2]; lo[h] = lam[(lane + 64 * h) * 2 + 1]; }
+            }
+            at += (int)gridDim.x;
+        }
+        if (u_lo >= u_hi) continue;        // an empty rest of a tensor's last elementwise tile
+        while (from > u_hi) {
+            float bound;
+            approach(from, u_hi, bound);
+            if (from == far || __builtin_amdgcn_ballot_w64(!(bound < SG2_FORGOTTEN)) == 0) break;
+            from = far;
+        }
+        range(u_lo, u_hi);
+    }
+
+    flush();
+}
+
+// ---- the gradients with the gradient of the input projection, chunk by chunk: one 128-lane workgroup per (chunk,
+// direction), lane (j,p) owning column j and RoPE pair p as in k_scan
 __global__ __launch_bounds__(SCAN_THREADS) void k_bilevel_backward(Plan pl, AdjIO io) {
+    constexpr bool DX = true;
     extern __shared__ __attribute__((aligned(16))) float lds[];
     float* rows = lds;
     float* sH = lds + LDS_ROWS_FLOATS;
@@ -605,22 +1160,26 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_bilevel_backward(Plan pl, AdjI
     g_wout[tid] = acc_wout;
 }
 
-// ---- launch 4: rows of the partials buffer added in a fixed order (64 entries per workgroup, four lanes per entry
-// each taking every fourth row, then the four partial sums in order)
-__global__ __launch_bounds__(256) void k_adj_sum_rows(const float* __restrict__ part, int rows_per_dir, float* __restrict__ out) {
-    __shared__ float s_part[4][64];
+// ---- rows of the partials buffer added in a fixed order (64 entries per workgroup, ROW_SLICES lanes per entry each taking
+// every ROW_SLICES-th row, then the partial sums in order)
+constexpr int ROW_SLICES = 16;
+__global__ __launch_bounds__(64 * ROW_SLICES) void k_adj_sum_rows(const float* __restrict__ part, int rows_per_dir, float* __restrict__ out) {
+    __shared__ float s_part[ROW_SLICES][64];
     const int col = threadIdx.x & 63, slice = threadIdx.x >> 6;
     const int o = blockIdx.x * 64 + col;          // 2 * SG2_BWD_STRIDE is a multiple of 64
     const int dir = o / SG2_BWD_STRIDE, e = o % SG2_BWD_STRIDE;
     float acc = 0.0f;
-#pragma unroll 4
-    for (int r = slice; r < rows_per_dir; r += 4) acc += part[((size_t)dir * rows_per_dir + r) * SG2_BWD_STRIDE + e];
+#pragma unroll 8
+    for (int r = slice; r < rows_per_dir; r += ROW_SLICES) acc += part[((size_t)dir * rows_per_dir + r) * SG2_BWD_STRIDE + e];
     s_part[slice][col] = acc;
     __syncthreads();
-    if (slice == 0) out[o] = ((s_part[0][col] + s_part[1][col]) + s_part[2][col]) + s_part[3][col];
+    if (slice != 0) return;
+#pragma unroll
+    for (int q = 1; q < ROW_SLICES; q++) acc += s_part[q][col];
+    out[o] = acc;
 }
 
-// ---- launch 5: from the gradients of the composed coefficients to those of the weights they were composed from
+// ---- from the gradients of the composed coefficients to those of the weights they were composed from
 // (the transpose of sg2_compose_one), and the final layout: input_proj W [8][2], b [8]; then per direction in_proj
 // [32][8], dt_proj W [16][16], b [16], B_proj [16][16], C_proj [16][16], A_log [16][16], D [16], rope_freq [16][8],
 // out_proj [8][16].  One workgroup; blk is k_adj_sum_rows' output ([2][SG2_BWD_STRIDE]).
@@ -742,9 +1301,9 @@ struct SavedOut {
     int interval;
 };
 __global__ __launch_bounds__(SCAN_THREADS) void k_saved_fill(Plan pl, SavedOut out) {
-    constexpr int ST = HT_STEP + 1;
+    constexpr int STEPS = 2 * HT_STEP, ST = STEPS + 1;
     __shared__ float s_dt[DI * ST], s_xb[DI * ST], s_B[DS * ST];
-    static_assert(SCAN_THREADS == 4 * HT_STEP && DI == 16 && DS == 16, "four row groups of four rows per step");
+    static_assert(SCAN_THREADS == 4 * STEPS && DI == 16 && DS == 16, "four row groups of four rows per step");
     const int chunk = blockIdx.x, dir = blockIdx.y, tid = threadIdx.x;
     const AdjIO none = {nullptr, {nullptr, nullptr}, nullptr, nullptr};
     const ChunkRef c = chunk_ref(pl, chunk, dir, none);
@@ -752,7 +1311,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_saved_fill(Plan pl, SavedOut o
     const float* __restrict__ Alog = pl.W.w[b + 5];
     const float* __restrict__ rope = pl.W.w[b + 7];
     const float* __restrict__ comp = pl.comp + dir * (SG2_COMP_GROUPS * 16 * 3);
-    const int tu = tid & (HT_STEP - 1), quarter = tid >> 5;
+    const int tu = tid & (STEPS - 1), quarter = tid >> 5;
     const int j = tid >> 3, p = tid & 7;
     const float a_e = 0.5f * sg_exp(Alog[j * DS + 2 * p]), a_o = 0.5f * sg_exp(Alog[j * DS + 2 * p + 1]);
     const float freq = rope[j * HP + p];
@@ -761,8 +1320,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_saved_fill(Plan pl, SavedOut o
         row0 = 0;
         for (int i = 0; i < c.ti; i++) row0 += (pl.tensors[i].numel + out.interval - 1) / out.interval;
     }
-    for (int u0 = c.ustart; u0 < c.uend; u0 += HT_STEP) {
-        const int cnt = min(HT_STEP, c.uend - u0);
+    for (int u0 = c.ustart; u0 < c.uend; u0 += STEPS) {
+        const int cnt = min(STEPS, c.uend - u0);
         {
             const bool valid = tu < cnt;
             float g, s;
@@ -838,37 +1397,43 @@ int launch_bilevel_backward(const Plan& pl, const float* d_ctx, const float* con
                             hipStream_t st) {
     static_assert(DM * DI == SCAN_THREADS, "one thread per out_proj entry");
     static_assert(SG2_BWD_STRIDE == SG2_COMP_GROUPS * 16 * 3 + DI * DS + DI * HP + DI + DM * DI, "layout of the per-direction sums");
-    {
-        static bool raised[64] = {};
-        int dev = 0;
-        SG_HIP_CHECK(hipGetDevice(&dev));
-        if (dev < 0 || dev >= 64) return sg::fail("device index %d out of range", dev);
-        if (!raised[dev]) {
-            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_bilevel_backward<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             BILEVEL_LDS_BYTES));
-            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_bilevel_backward<true>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             BILEVEL_DX_LDS_BYTES));
-            raised[dev] = true;
-        }
-    }
     if (pl.total == 0) {
         hipLaunchKernelGGL(k_fill_zero, dim3(8), dim3(256), 0, st, grads_out, SG2_SCAN_GRAD_FLOATS);
         SG_LAUNCH_CHECK("k_fill_zero");
         return 0;
     }
     const AdjIO io = {d_ctx, {d_scan ? d_scan[0] : nullptr, d_scan ? d_scan[1] : nullptr}, rx, dx};
-    const int groups = pl.chunks < ADJ_GROUPS ? pl.chunks : ADJ_GROUPS;
-    hipLaunchKernelGGL(k_adj_summary, dim3(pl.chunks, 2), dim3(SCAN_THREADS), 0, st, pl, io);
-    SG_LAUNCH_CHECK("k_adj_summary");
-    hipLaunchKernelGGL(k_adj_prefix, dim3(pl.P, 2), dim3(SCAN_THREADS), 0, st, pl);
-    SG_LAUNCH_CHECK("k_adj_prefix");
-    if (dx != nullptr)
-        hipLaunchKernelGGL(k_bilevel_backward<true>, dim3(groups, 2), dim3(SCAN_THREADS), BILEVEL_DX_LDS_BYTES, st, pl, io);
-    else
-        hipLaunchKernelGGL(k_bilevel_backward<false>, dim3(groups, 2), dim3(SCAN_THREADS), BILEVEL_LDS_BYTES, st, pl, io);
-    SG_LAUNCH_CHECK("k_bilevel_backward");
+    // at least four tiles per wave: below that the steps behind the range outweigh it
+    const int64_t tiles = (int64_t)pl.elem_tiles * (ELEM_TILE / AT);
+    const int64_t waves = std::max<int64_t>((tiles + 3) / 4, pl.chunks);
+    const int groups = dx != nullptr ? std::min(pl.chunks, 512) : (int)std::min<int64_t>(waves, ADJ_GROUPS);
+    if (pl.wchunks > 0) {
+        hipLaunchKernelGGL(k_adj_summary, dim3(pl.chunks, 2), dim3(SCAN_THREADS), 0, st, pl, io, dx == nullptr);
+        SG_LAUNCH_CHECK("k_adj_summary");
+    }
+    if (pl.wchunks > 0 || dx != nullptr) {
+        hipLaunchKernelGGL(k_adj_prefix, dim3(pl.P, 2), dim3(SCAN_THREADS), 0, st, pl, dx == nullptr);
+        SG_LAUNCH_CHECK("k_adj_prefix");
+    }
+    if (dx != nullptr) {
+        static bool raised[64] = {};
+        int dev = 0;
+        SG_HIP_CHECK(hipGetDevice(&dev));
+        if (dev < 0 || dev >= 64) return sg::fail("device index %d out of range", dev);
+        if (!raised[dev]) {
+            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_bilevel_backward), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             BILEVEL_DX_LDS_BYTES));
+            raised[dev] = true;
+        }
+        hipLaunchKernelGGL(k_bilevel_backward, dim3(groups, 2), dim3(SCAN_THREADS), BILEVEL_DX_LDS_BYTES, st, pl, io);
+        SG_LAUNCH_CHECK("k_bilevel_backward");
+    } else {
+        if (d_ctx != nullptr) hipLaunchKernelGGL(k_adjoint<false>, dim3(groups, 2), dim3(64), 0, st, pl, io);
+        else hipLaunchKernelGGL(k_adjoint<true>, dim3(groups, 2), dim3(64), 0, st, pl, io);
+        SG_LAUNCH_CHECK("k_adjoint");
+    }
     static_assert((2 * SG2_BWD_STRIDE) % 64 == 0, "k_adj_sum_rows: whole workgroups");
-    hipLaunchKernelGGL(k_adj_sum_rows, dim3(2 * SG2_BWD_STRIDE / 64), dim3(256), 0, st, pl.adj_part, groups, pl.adj_blk);
+    hipLaunchKernelGGL(k_adj_sum_rows, dim3(2 * SG2_BWD_STRIDE / 64), dim3(64 * ROW_SLICES), 0, st, pl.adj_part, groups, pl.adj_blk);
     SG_LAUNCH_CHECK("k_adj_sum_rows");
     hipLaunchKernelGGL(k_compose_backward, dim3(1), dim3(256), 0, st, pl, pl.adj_blk, grads_out);
     SG_LAUNCH_CHECK("k_compose_backward");

@@ -29,7 +29,7 @@
 //     threshold of an expert, the lane that holds that expert's sums adds them to the interval's bin (a row of this
 //     workgroup in memory) and starts again.  In element order x stays next to zero.  The exceptions - elements in
 //     another interval of one of their experts - look the interval up in the tables and move their (w, w g) to its bin
-//     with atomics, one expert per lane at a time.  (With all of a trained net's exceptions taken by LDS atomics, in
+//     with atomics, one expert per lane at a time (four at a time cost more registers than they saved time).  (With all of a trained net's exceptions taken by LDS atomics, in
 //     element order, they were half of the pass.)
 //     (An element exactly on a threshold counts the unit as inactive on both sides; forward value and gradient use
 //     the same interval, so they stay consistent.)
@@ -42,9 +42,10 @@
 // reference's atomicAdd).
 //
 // Bound by the vector ALU (about 5000 instructions per wave and tile, two thirds of them the fixed multiply-adds of the
-// net and its derivative).  Measured on 25 M elements with module-initialised experts after some meta steps: 9.3 ms, 47 ms
+// net and its derivative).  Measured on 25 M elements with module-initialised experts after some meta steps: 8.4 ms, 47 ms
 // as one lane per element of a 256-lane workgroup that summed the outer products lane by lane from LDS; on 0.42 M elements
-// 0.34 ms instead of 1.1.
+// 0.33 ms instead of 1.1.  (The net's products as 4 x 4 x 1 matrix instructions with the weights in LDS or in memory took as
+// long, with the bins in LDS longer on large calls: registers are what there is least of.)
 #include "sg2_internal.hpp"
 
 namespace sg2 {
@@ -157,18 +158,33 @@ __device__ __forceinline__ void wave_sync() {
 // (the row belongs to this workgroup alone: workgroup scope lets the add run in the L2 next to it)
 __device__ __forceinline__ void bin_add(float* p, float v) { __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 
-// how many of an expert's thresholds lie below g
-__device__ __forceinline__ int interval_of(const float* __restrict__ ths, int e, float g) {
-    const float4* t4 = reinterpret_cast<const float4*>(ths + e * EH);
-    int k = 0;
+// The thresholds of an expert, read together.
+struct Thresholds {
+    float t[EH];
+    __device__ __forceinline__ Thresholds(const float* __restrict__ ths, int e) {
+        const float4* t4 = reinterpret_cast<const float4*>(ths + e * EH);
 #pragma unroll
-    for (int q = 0; q < EH / 4; q++) {
-        const float4 t = t4[q];
-        k += (t.x < g ? 1 : 0) + (t.y < g ? 1 : 0) + (t.z < g ? 1 : 0) + (t.w < g ? 1 : 0);
+        for (int q = 0; q < EH / 4; q++) { const float4 v = t4[q]; t[4 * q] = v.x; t[4 * q + 1] = v.y; t[4 * q + 2] = v.z; t[4 * q + 3] = v.w; }
     }
-    return k;
-}
-
+    __device__ __forceinline__ int below(float g) const {      // how many lie below g
+        int k = 0;
+#pragma unroll
+        for (int q = 0; q < EH; q++) k += t[q] < g ? 1 : 0;
+        return k;
+    }
+    __device__ __forceinline__ float low(float g) const {      // the last below g, the first not below it
+        float v = -__builtin_inff();
+#pragma unroll
+        for (int q = 0; q < EH; q++) v = t[q] < g ? t[q] : v;
+        return v;
+    }
+    __device__ __forceinline__ float high(float g) const {
+        float v = __builtin_inff();
+#pragma unroll
+        for (int q = EH - 1; q >= 0; q--) v = t[q] < g ? v : t[q];
+        return v;
+    }
+};
 __device__ __forceinline__ void order(float& a, float& b) {
     const float hi = __builtin_fmaxf(a, b), lo = __builtin_fminf(a, b);
     a = hi;
@@ -233,7 +249,6 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     for (int i = tid; i < N_BINS; i += BE_THREADS) bins[i] = 0.0f;
     for (int i = tid; i < KEY_FLOATS; i += BE_THREADS) s_keys[i] = i < KEY_FLOATS / 2 ? a.W.w[W_KEYS_A][i] : a.W.w[W_KEYS_B][i - KEY_FLOATS / 2];
     for (int i = lane; i < 64 * XW + R_FLOATS; i += 64) s_x[i] = 0.0f;     // rows are read whole: no NaN may lie in what was never written
-    for (int i = lane; i < 2 * NE; i += 64) s_tab[i] = make_float4(0.0f, 0.0f, __builtin_inff(), -__builtin_inff());
     __syncthreads();
 
     const sg::cfloat_p Wz = sg::as_const(a.W.w[W_GRU_WZ]), bz = sg::as_const(a.W.w[W_GRU_BZ]);
@@ -256,37 +271,45 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     const bool owner = lane < 48 && li < PK;
     float x_held = -1.0f;                                 // reference magnitude of the lines in s_tab (< 0: none yet)
     auto reference = [](float x, int neg) { return neg ? -x : __builtin_fmaxf(x, 1.40129846e-45f); };      // (+0 stands for the interval just above zero)
-    auto flush = [&](int v, int neg) {
-        const int e = (4 * lk + v) * PK + li;
-        float* b = bins + 2 * (e * NBIN + interval_of(ths, e, reference(x_held, neg)));
-        bin_add(b, cen[neg][v]);
-        bin_add(b + 1, cen[2 + neg][v]);
-        cen[neg][v] = 0.0f;
-        cen[2 + neg][v] = 0.0f;
+    auto line_at = [&](const Thresholds& th, int e, float r) {       // the expert's line at r and the borders of its interval
+        const float2 ab = reinterpret_cast<const float2*>(lines)[e * NBIN + th.below(r)];
+        return make_float4(ab.x, ab.y, th.low(r), th.high(r));
     };
     auto move_reference = [&](float x) {
-        bool stale = false;
-        if (owner) {
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const float4 t = s_tab[(q & 1) * NE + (4 * lk + (q >> 1)) * PK + li];
-                const float r = reference(x, q & 1);
-                stale = stale || !(t.z < r && r <= t.w);
+        if (x_held < 0.0f) {
+#pragma unroll 1
+            for (int t = lane; t < 2 * NE; t += 64) {
+                const int neg = t >= NE ? 1 : 0, e = t - neg * NE;
+                s_tab[t] = line_at(Thresholds(ths, e), e, reference(x, neg));
             }
-        }
-        if (__builtin_amdgcn_ballot_w64(stale) != 0) {
-            if (stale) {
+        } else if (!FLAT) {
+            unsigned stale = 0u;             // bit 2 v + neg: x lies in another interval of expert v on that side
+            if (owner) {
 #pragma unroll
                 for (int q = 0; q < 8; q++) {
-                    const int e = (4 * lk + (q >> 1)) * PK + li;
-                    float4* rec = s_tab + (q & 1) * NE + e;
+                    const float4 t = s_tab[(q & 1) * NE + (4 * lk + (q >> 1)) * PK + li];
                     const float r = reference(x, q & 1);
-                    const float4 t = *rec;
-                    if (t.z < r && r <= t.w) continue;
-                    if (x_held >= 0.0f) flush(q >> 1, q & 1);
-                    const int k = interval_of(ths, e, r);
-                    const float2 ab = reinterpret_cast<const float2*>(lines)[e * NBIN + k];
-                    *rec = make_float4(ab.x, ab.y, k > 0 ? ths[e * EH + k - 1] : -__builtin_inff(), k < EH ? ths[e * EH + k] : __builtin_inff());
+                    stale |= t.z < r && r <= t.w ? 0u : 1u << q;
+                }
+            }
+            while (__builtin_amdgcn_ballot_w64(stale != 0u) != 0) {       // one per lane at a time: a tile passes a few thresholds
+                if (stale != 0u) {
+                    const int q = __builtin_ctz(stale), v = q >> 1, neg = q & 1, e = (4 * lk + v) * PK + li;
+                    stale &= stale - 1u;
+                    const Thresholds th(ths, e);
+                    float w = 0.0f, wg = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {      // (selects: a dynamic index would send the sums to scratch)
+                        const bool it = k == q;
+                        w = it ? cen[k & 1][k >> 1] : w;
+                        wg = it ? cen[2 + (k & 1)][k >> 1] : wg;
+                        cen[k & 1][k >> 1] = it ? 0.0f : cen[k & 1][k >> 1];
+                        cen[2 + (k & 1)][k >> 1] = it ? 0.0f : cen[2 + (k & 1)][k >> 1];
+                    }
+                    s_tab[neg * NE + e] = line_at(th, e, reference(x, neg));
+                    float* b = bins + 2 * (e * NBIN + th.below(reference(x_held, neg)));
+                    bin_add(b, w);
+                    bin_add(b + 1, wg);
                 }
             }
         }
@@ -479,7 +502,8 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                     const float wa = ia == 0 ? wgt[0][0] : ia == 1 ? wgt[0][1] : ia == 2 ? wgt[0][2] : wgt[0][3];
                     const float wb = ib == 0 ? wgt[1][0] : ib == 1 ? wgt[1][1] : ib == 2 ? wgt[1][2] : wgt[1][3];
                     const int e = ea * PK + eb;
-                    const int k = interval_of(ths, e, g), kr = interval_of(ths, e, reference(x_held, side != 0));
+                    const Thresholds th(ths, e);
+                    const int k = th.below(g), kr = th.below(reference(x_held, side != 0));
                     const float2 ab = reinterpret_cast<const float2*>(lines)[e * NBIN + k];
                     const float out = sg_fma(ab.x, g, ab.y);
                     const float pa = wb * out, pb = wa * out;
@@ -666,14 +690,33 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
         }
     }
 
-    // ---- this workgroup's sums -> its row of the partials buffer.  The waves' held expert sums into their bins, one wave
-    // after the other; the dense sums through LDS.
-    for (int w = 0; w < BE_WAVES; w++) {
-        __syncthreads();
-        if (wave != w || x_held < 0.0f || !owner) continue;
+    // ---- this workgroup's sums -> its row of the partials buffer, through LDS: the waves' held expert sums with the
+    // intervals they belong to (wave after wave: a fixed order), then the dense sums
+    static_assert(6 * NE <= 64 * XW + R_FLOATS, "the held sums fit the wave's staging rows");
+    if (owner) {
 #pragma unroll
-        for (int q = 0; q < 8; q++) flush(q >> 1, q & 1);
+        for (int v = 0; v < 4; v++) {
+            const int e = (4 * lk + v) * PK + li;
+            const Thresholds th(ths, e);
+#pragma unroll
+            for (int neg = 0; neg < 2; neg++) {
+                float* t = s_x + (neg * NE + e) * 3;
+                t[0] = cen[neg][v];
+                t[1] = cen[2 + neg][v];
+                t[2] = (float)(x_held < 0.0f ? 0 : th.below(reference(x_held, neg)));      // (a wave without a tile holds zeros)
+            }
+        }
     }
+    __syncthreads();
+    for (int t = tid; t < 2 * NE; t += BE_THREADS) {
+        for (int w = 0; w < BE_WAVES; w++) {
+            const float* held = lds + KEY_FLOATS + w * WAVE_FLOATS + t * 3;
+            float* b = bins + 2 * ((t % NE) * NBIN + (int)held[2]);
+            bin_add(b, held[0]);
+            bin_add(b + 1, held[1]);
+        }
+    }
+    __syncthreads();
     constexpr int M_Q = 16 * 32, M_K = M_Q + 32 * 32, M_FLOATS = M_K + NH * 256;       // GRU [16][32], query [32][32], keys [NH][16 blocks][4][4]
     static_assert(M_FLOATS <= 64 * XW + R_FLOATS, "the sums fit the wave's staging rows");
 #pragma unroll

@@ -114,6 +114,10 @@ __device__ __forceinline__ void compose_block(const Plan& pl, int threads) {
             const float kq = sg2_limit_factor(sg_fma(416.0f, sg_i2f(s_amax[k]), 184.0f * sg_i2f(s_fmax[k])), slope);
             cmax[8 + 2 * k] = kq * sg_i2f(s_cdt[k][0]);
             cmax[9 + 2 * k] = kq * sg_i2f(s_cdt[k][1]);
+            // ... and for the polynomials of the adjoint (sg2_bilevel.hip)
+            const float kc = sg2_limit_factor(sg_max(80.0f * sg_i2f(s_amax[k]), 256.0f * sg_i2f(s_fmax[k])), slope);
+            cmax[12 + 2 * k] = kc * sg_i2f(s_cdt[k][0]);
+            cmax[13 + 2 * k] = kc * sg_i2f(s_cdt[k][1]);
         }
     }
 }

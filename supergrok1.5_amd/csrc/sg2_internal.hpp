@@ -166,12 +166,12 @@ int launch_sort(const Plan& pl, int32_t* dbg_perm, hipStream_t st);
 int launch_scan(const Plan& pl, hipStream_t st);
 // bilevel path: the forward scan keeps the state entering every HT_STEP-th step of a tensor; index of scan step u
 // (a multiple of HT_STEP) of tensor ti (element offset off) in that array, and the array's length
-constexpr int HT_STEP = 32;
+constexpr int HT_STEP = 16;
 __host__ __device__ inline int htile_index(int off, int ti, int u) { return off / HT_STEP + ti + u / HT_STEP; }
 __host__ __device__ inline int htile_count(int total, int P) { return total / HT_STEP + P + 1; }
 // floats per direction of the adjoint kernels' sums: composed coefficients [5][16][3], A_log [16][16], rope_freq [16][8], D [16], out_proj [8][16]
 constexpr int SG2_BWD_STRIDE = 768;
-constexpr int ADJ_GROUPS = 512;    // workgroups per direction of the adjoint replay (upper bound)
+constexpr int ADJ_GROUPS = 1024;   // workgroups per direction of the adjoint (upper bound)
 // GEO_* of the smallest compiled geometry that holds these dimensions, or -1 with the error set
 int geo_of(const SgDims* d);
 // whether (d_model, d_state, d_inner) are exactly that geometry's (else the scan weights are embedded in it)

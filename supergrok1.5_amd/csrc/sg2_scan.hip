@@ -58,6 +58,7 @@
 // 32nd step (Plan::htile), which the adjoint kernels restart from.
 #include <type_traits>
 #include "sg2_internal.hpp"
+#include "sg2_pair_sums.hpp"
 #include "../../include/sg2_compose.h"
 
 namespace sg2 {
@@ -71,7 +72,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #endif
 constexpr int UB = SG2_SCAN_UB;           // timesteps per unrolled block of the recurrence
 static_assert(UB % 4 == 0 && SCAN_TT % UB == 0 && SCAN_TT == 64, "blocks are fetched 4 timesteps per LDS read; one ballot covers a tile");
-static_assert(HT_STEP % UB == 0 && SCAN_TT % HT_STEP == 0 && SCAN_TT / HT_STEP <= 2, "kept states fall on block borders: tile start and at most one more");
+static_assert(HT_STEP % UB == 0 && SCAN_TT % HT_STEP == 0, "kept states fall on block borders");
 // Three waves per SIMD (168 VGPRs) is where the default geometry's kernels stop gaining from occupancy; keep the
 // register allocation from drifting just past that boundary.  The large geometry's workgroup is two waves per SIMD by itself,
 // and at 128 VGPRs (two workgroups per CU) the recurrence spills: one workgroup per CU, up to 256 VGPRs.
@@ -82,93 +83,6 @@ template <class G>
 constexpr int scan_waves() { return G::PARTS == 2 ? SG2_SCAN_WAVES : 2; }
 #define SG2_SCAN_ATTR __attribute__((amdgpu_waves_per_eu(scan_waves<G>(), scan_waves<G>())))
 
-__device__ __forceinline__ float dpp_quad_swap1(float v) {   // lane ^ 1
-    return sg_i2f(__builtin_amdgcn_update_dpp(0, sg_f2i(v), 0xB1, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float dpp_quad_swap2(float v) {   // lane ^ 2
-    return sg_i2f(__builtin_amdgcn_update_dpp(0, sg_f2i(v), 0x4E, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float dpp_half_mirror(float v) {  // lane -> 7 - lane within each group of 8
-    return sg_i2f(__builtin_amdgcn_update_dpp(0, sg_f2i(v), 0x141, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float dpp_row_mirror(float v) {   // lane -> 15 - lane within each group of 16
-    return sg_i2f(__builtin_amdgcn_update_dpp(0, sg_f2i(v), 0x140, 0xF, 0xF, true));
-}
-// sum over the HP lanes of a (column) group.  The tree folds the group in halves, mirrored, until four sums are left:
-// HP = 8: s_i = y_i + y_(7-i), total = (s_0 + s_1) + (s_2 + s_3); HP = 16: r_i = y_i + y_(15-i) first, then the same on r.
-// (Mirrored folds first, because a fold across DPP banks can be written to some banks only: see block_pair_sums.)
-template <int HP>
-__device__ __forceinline__ float pair_tree_sum(float y) {
-    if (HP == 16) y = y + dpp_row_mirror(y);
-    y = y + dpp_half_mirror(y);
-    y = y + dpp_quad_swap1(y);
-    y = y + dpp_quad_swap2(y);
-    return y;
-}
-// The same sums for the 8 steps of a block in 16 instructions instead of 24 (32 for HP = 16).  A DPP instruction can
-// be restricted to some banks (groups of four lanes) of every row of 16, leaving the destination's other lanes as
-// they were.  After a mirrored fold both halves of the folded group hold the same sums, so two steps' folds are
-// written into ONE register - step u into the first half's lanes, step u + 4 into the second half's - and the rest
-// of the tree runs on half as many registers.  Additions commute bit for bit, so every lane that ends up holding a
-// step's total holds pair_tree_sum's value.  On return, for HP = 8, y[k] (k < 4) is the total of step k + 4 (p >> 2)
-// in lane (j, p); for HP = 16, y[m] (m < 2) that of step m + 2 (p >> 2).
-// (Inline assembly: the compiler has no form for a bank-masked DPP addition that keeps the other lanes, and it does
-// not see a hazard between instructions inside the block - a DPP operand must not be read within two instructions of the
-// vector instruction that wrote it, hence the order of the instructions and the s_nop.)
-template <int HP>
-__device__ __forceinline__ void block_pair_sums(float (&y)[8]) {
-    float z0, z1, z2, z3;
-    if (HP == 8) {
-        asm volatile(
-            "s_nop 1\n\t"
-            "v_add_f32_dpp %0, %4, %4 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
-            "v_add_f32_dpp %0, %8, %8 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
-            "v_add_f32_dpp %1, %5, %5 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
-            "v_add_f32_dpp %1, %9, %9 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
-            "v_add_f32_dpp %2, %6, %6 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
-            "v_add_f32_dpp %2, %10, %10 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
-            "v_add_f32_dpp %3, %7, %7 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
-            "v_add_f32_dpp %3, %11, %11 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
-            "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "v_add_f32_dpp %1, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "v_add_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "v_add_f32_dpp %3, %3, %3 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-            "v_add_f32_dpp %1, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-            "v_add_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-            "v_add_f32_dpp %3, %3, %3 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-            "s_nop 1"
-            : "=&v"(z0), "=&v"(z1), "=&v"(z2), "=&v"(z3)
-            : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(y[4]), "v"(y[5]), "v"(y[6]), "v"(y[7]));
-        y[0] = z0; y[1] = z1; y[2] = z2; y[3] = z3;
-    } else {
-        asm volatile(
-            "s_nop 1\n\t"
-            "v_add_f32_dpp %0, %4, %4 row_mirror row_mask:0xf bank_mask:0x3\n\t"
-            "v_add_f32_dpp %0, %8, %8 row_mirror row_mask:0xf bank_mask:0xc\n\t"
-            "v_add_f32_dpp %1, %5, %5 row_mirror row_mask:0xf bank_mask:0x3\n\t"
-            "v_add_f32_dpp %1, %9, %9 row_mirror row_mask:0xf bank_mask:0xc\n\t"
-            "v_add_f32_dpp %2, %6, %6 row_mirror row_mask:0xf bank_mask:0x3\n\t"
-            "v_add_f32_dpp %2, %10, %10 row_mirror row_mask:0xf bank_mask:0xc\n\t"
-            "v_add_f32_dpp %3, %7, %7 row_mirror row_mask:0xf bank_mask:0x3\n\t"
-            "v_add_f32_dpp %3, %11, %11 row_mirror row_mask:0xf bank_mask:0xc\n\t"
-            "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
-            "v_add_f32_dpp %1, %1, %1 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
-            "s_nop 0\n\t"
-            "v_add_f32_dpp %0, %2, %2 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
-            "v_add_f32_dpp %1, %3, %3 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
-            "s_nop 1\n\t"
-            "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "v_add_f32_dpp %1, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "s_nop 1\n\t"
-            "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-            "v_add_f32_dpp %1, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-            "s_nop 1"
-            : "=&v"(z0), "=&v"(z1), "=&v"(z2), "=&v"(z3)
-            : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(y[4]), "v"(y[5]), "v"(y[6]), "v"(y[7]));
-        y[0] = z0; y[1] = z1;
-    }
-}
 template <int HP>
 __device__ __forceinline__ float pair_tree_max(float f) {
     f = sg_max(f, dpp_quad_swap1(f));
@@ -1089,7 +1003,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                 ht[LANES + tid + 64 * h] = S[h].ho;
             }
         };
-        if (KEEP) keep_state(tile0);
 
         // ---------------- phase B: the recurrences of this lane's two columns over the tile
         const float* __restrict__ r_Be = s_B + (2 * p) * LDS_STRIDE;
@@ -1129,13 +1042,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             };
 #pragma unroll 1
             for (; k0 < SCAN_TT; k0 += UB) {
-                if (KEEP && k0 == HT_STEP) keep_state(tile0 + HT_STEP);
+                if (KEEP && k0 % HT_STEP == 0) keep_state(tile0 + k0);
                 fetch(k0, Be, Bo, Ce, Co, dt, xv);
                 compute(k0, Be, Bo, Ce, Co, dt, xv);
             }
         }
         for (; k0 + UB <= cnt; k0 += UB) {
-            if (KEEP && k0 == HT_STEP) keep_state(tile0 + HT_STEP);
+            if (KEEP && k0 % HT_STEP == 0) keep_state(tile0 + k0);
             float Be[UB], Bo[UB], Ce[UB], Co[UB];
 #pragma unroll
             for (int q = 0; q < UB; q += 4) {
@@ -1171,7 +1084,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                     *reinterpret_cast<f32x4*>(&s_y[j * LDS_STRIDE + k0 + 4 * (p >> 2)]) = f32x4{y[0], y[1], y[2], y[3]};
             }
         }
-        if (KEEP && k0 == HT_STEP && cnt > HT_STEP) keep_state(tile0 + HT_STEP);      // the ragged end starts right there
+        if (KEEP && k0 % HT_STEP == 0 && k0 < cnt) keep_state(tile0 + k0);      // the ragged end starts right there
         for (; k0 < cnt; k0++) {       // ragged end of the last tile of a tensor
 #pragma unroll
             for (int h = 0; h < 2; h++) {
