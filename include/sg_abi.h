@@ -408,17 +408,17 @@ int sg2_bilevel_elem_ex(const SgDims* dims, const Sg2Weights* weights, int64_t t
 
 /* The whole bilevel pass in one call: sg2_bilevel_forward, sg2_bilevel_elem and sg2_bilevel_backward on tensors that
  * stay where they are.  Of a record only grad, sharpness, gru_state, the two Mamba states (all read only), param - the
- * cotangent, in the tensor's dtype -, numel and dtype (SG_SHARP_F32, SG_SHARP_EXACT) are used.  normalise != 0: element
- * i's cotangent is -v_i / |v|, |v| the 2-norm of the tensor's v (-v_i where |v| <= 1e-12), as the bilevel update takes it from
- * the validation gradient; else v_i.
+ * cotangent, in the tensor's dtype -, numel and dtype (SG_SHARP_F32, SG_SHARP_EXACT) are used.  norms (device memory, one
+ * per tensor, or NULL): tensor t's element i then has the cotangent -v_i / norms[t] (-v_i where norms[t] <= 1e-12), as the
+ * bilevel update takes it from the validation gradient v and its 2-norm; else v_i.
  *   smart_out [sum numel]  smart gradients, packed in call order (may be NULL)
  *   elem_grads_out         as grads_out of sg2_bilevel_elem, the expert tensors at the caller's own expert_hidden
  *                          (1364 + 144 * (3 * expert_hidden + 1) floats)
  *   scan_grads_out [SG2_SCAN_GRAD_FLOATS]
  * Built for d_model 8, d_state 16, d_inner 16, gru_hidden 4, 4 heads, 12 keys, 144 experts of width <= 16.  Contexts and
- * their gradients travel between the three parts in the order of the sort, in the workspace. */
+ * their gradients travel between the three parts in the workspace. */
 size_t sg2_bilevel_pass_workspace_bytes(const SgDims* dims, int num_tensors, const int64_t* numels);
-int sg2_bilevel_pass(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, float rescale, int normalise,
+int sg2_bilevel_pass(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, float rescale, const float* norms,
                      float* smart_out, float* elem_grads_out, float* scan_grads_out, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The meta-net's own forward with the step's hard top-1 routing, for callers that use the net outside the fused

@@ -511,7 +511,7 @@ int64_t supergrok2_flat_step(py::list params, py::list eas, py::list easqs, py::
 }
 
 // The bilevel pass over tensors that stay where they are (sg2_bilevel_pass): (smart gradients or None, gradients of the
-// per-element weights, gradients of the scan weights), flat.  exact: fp32 sharpness next to 16-bit gradients is used as it
+// per-element weights, gradients of the scan weights), flat.  normalise: the cotangent is -v / |v|.  exact: fp32 sharpness next to 16-bit gradients is used as it
 // is.  None where the general path has to be taken (other sizes of the net, tensors that would have to be converted).
 py::object supergrok2_bilevel_pass(py::list grads, py::list sharps, py::list grus, py::list mfwd, py::list mbwd, py::list cots,
                                    py::list weights, float rescale, bool normalise, bool exact, bool want_smart, std::vector<int> dims8) {
@@ -525,6 +525,7 @@ py::object supergrok2_bilevel_pass(py::list grads, py::list sharps, py::list gru
     std::vector<Sg2Tensor> ts;
     std::vector<int64_t> numels;
     std::vector<at::Tensor> held;        // cotangents that had to be made contiguous
+    std::vector<const at::Tensor*> active;
     held.reserve(P);
     int64_t total = 0;
     const at::Tensor* first = nullptr;
@@ -560,6 +561,7 @@ py::object supergrok2_bilevel_pass(py::list grads, py::list sharps, py::list gru
         q.numel = n;
         ts.push_back(q);
         numels.push_back(n);
+        active.push_back(c);
         total += n;
         if (!first) first = g;
     }
@@ -577,9 +579,18 @@ py::object supergrok2_bilevel_pass(py::list grads, py::list sharps, py::list gru
     const auto opt = torch::TensorOptions().device(first->device()).dtype(torch::kFloat32);
     auto elem = torch::empty({(SG2_ELEM_GRAD_FLOATS - dims.num_experts * 49) + dims.num_experts * (3 * dims.expert_hidden + 1)}, opt);
     auto scan = torch::empty({SG2_SCAN_GRAD_FLOATS}, opt);
+    torch::Tensor norms;
+    if (normalise) {
+        at::NoGradGuard guard;
+        norms = torch::empty({(int64_t)ts.size()}, opt);
+        for (size_t i = 0; i < ts.size(); i++) {
+            at::Tensor out = norms.select(0, i);
+            at::linalg_vector_norm_out(out, active[i]->scalar_type() == torch::kFloat32 ? *active[i] : active[i]->to(torch::kFloat32), 2);
+        }
+    }
     torch::Tensor smart;
     if (want_smart) smart = torch::empty({total}, opt);
-    check_status(sg2_bilevel_pass(&dims, &W, (int)ts.size(), ts.data(), rescale, normalise ? 1 : 0, want_smart ? smart.data_ptr<float>() : nullptr,
+    check_status(sg2_bilevel_pass(&dims, &W, (int)ts.size(), ts.data(), rescale, normalise ? norms.data_ptr<float>() : nullptr, want_smart ? smart.data_ptr<float>() : nullptr,
                                   elem.data_ptr<float>(), scan.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), current_stream(*first)), fn);
     return py::make_tuple(want_smart ? py::cast(smart) : py::object(py::none()), elem, scan);
 }

@@ -90,7 +90,7 @@ __device__ __forceinline__ float pair_sum(float v) {             // sum over the
 // What a (chunk, direction) needs to find its steps.
 struct ChunkRef {
     int ti, N, off, ustart, uend;
-    bool has_s, own_order;
+    bool has_s;
     const uint32_t* skey;
     const int32_t* sval;
     const float* ssrt;
@@ -106,7 +106,6 @@ __device__ __forceinline__ ChunkRef chunk_ref(const Plan& pl, int chunk, int dir
     c.ustart = (chunk - pl.chunk_prefix[c.ti]) * pl.chunk_len;
     c.uend = min(c.N, c.ustart + pl.chunk_len);
     c.has_s = pl.sharp_nonzero[c.ti] != 0;        // all-zero sharpness is never gathered into sorted order
-    c.own_order = pl.own_order;
     c.skey = pl.keys[0] + c.off;
     c.sval = pl.vals[0] + c.off;
     c.ssrt = pl.ssorted + c.off;
@@ -121,7 +120,7 @@ __device__ __forceinline__ void load_step(const ChunkRef& c, int dir, int u, boo
         const int t = dir ? (c.N - 1 - u) : u;
         const int32_t v = c.sval[t];
         int o = v & 0x7fffffff;
-        *orig = c.own_order ? t : ((unsigned)o < (unsigned)c.N) ? o : 0;
+        *orig = ((unsigned)o < (unsigned)c.N) ? o : 0;
         *g = sg_i2f((int32_t)c.skey[t] | (v & (int32_t)0x80000000));
         *s = c.has_s ? c.ssrt[t] : 0.0f;
     }
@@ -169,6 +168,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_adj_summary(Plan pl, AdjIO io,
     const float a_e = 0.5f * sg_exp(Alog[j * DS + 2 * p]), a_o = 0.5f * sg_exp(Alog[j * DS + 2 * p + 1]);
     const float freq = rope[j * HP + p];
     if (use_flag && *pl.contracted != 0) return;   // nobody reads the maps
+    const bool in_order = sorted_rows(pl);
     if (chunk == pl.chunk_prefix[c.ti]) return;    // nothing lies before a tensor's first chunk: its map is never applied
     fill_fmax(s_fmax, rope);
     float u1e, u1o, u2e, u2o, ve, vo;
@@ -193,7 +193,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_adj_summary(Plan pl, AdjIO io,
             int orig;
             load_step(c, dir, u0 + tu, valid, &g, &s, &orig);
             if (c.dctx != nullptr) {
-                const float4 dv = valid ? reinterpret_cast<const float4*>(c.dctx + (size_t)orig * DM)[half] : make_float4(0.f, 0.f, 0.f, 0.f);
+                const int at = in_order ? (dir ? c.N - 1 - (u0 + tu) : u0 + tu) : orig;
+                const float4 dv = valid ? reinterpret_cast<const float4*>(c.dctx + (size_t)at * DM)[half] : make_float4(0.f, 0.f, 0.f, 0.f);
                 reinterpret_cast<float4*>(s_dctx + tu * DM)[half] = dv;
             }
             for (int q = 0; q < ROWS / 2; q++) {
@@ -432,6 +433,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const float* dctx = nullptr;
     const float* dscan = nullptr;
 
+    const bool in_order = sorted_rows(pl);
     // what a tile reads from memory, requested one tile ahead
     struct Inputs { uint32_t key; int32_t val; float s, d0, d1; adj_f32x4 ds, h; };
     auto request = [&](int u0, bool with_state) {
@@ -445,7 +447,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             if (SCAN_GRADS) {
                 in.ds = *reinterpret_cast<const adj_f32x4*>(dscan + (size_t)u * DI + 4 * rg);
             } else {
-                const int at = pl.own_order ? t : min(in.val & 0x7fffffff, N - 1);
+                const int at = in_order ? t : min(in.val & 0x7fffffff, N - 1);
                 in.d0 = dctx[(size_t)at * DM + rg];
                 in.d1 = dctx[(size_t)at * DM + 4 + rg];
             }

@@ -112,12 +112,14 @@ __device__ __forceinline__ Unit unit_of(const float* __restrict__ W1, const floa
     return u;
 }
 
-// One expert per wave.
-__global__ __launch_bounds__(64) void k_expert_tables(Sg2Weights W, int eh, float* __restrict__ tables) {
+// One expert per wave; clears *all_zero where a threshold is not 0.
+__global__ __launch_bounds__(64) void k_expert_tables(Sg2Weights W, int eh, float* __restrict__ tables, int* all_zero) {
     const int e = blockIdx.x, lane = threadIdx.x, m = lane & (EH - 1);
     const Unit u = unit_of(W.w[W_EXP_W1], W.w[W_EXP_B1], e, eh, m);
     const float w2 = m < eh ? W.w[W_EXP_W2][e * eh + m] : 0.0f;
     if (lane < EH) tables[e * EH + u.rank] = u.thr;
+    // (plain store: every writer stores the same value)
+    if (all_zero != nullptr && __builtin_amdgcn_ballot_w64(u.w1 != 0.0f ? u.thr != 0.0f : u.b1 > 0.0f) != 0 && lane == 0) *all_zero = 0;
     float A = 0.0f, B = W.w[W_EXP_B2][e];
 #pragma unroll
     for (int j = 0; j < EH; j++) {
@@ -134,16 +136,23 @@ __global__ __launch_bounds__(64) void k_expert_tables(Sg2Weights W, int eh, floa
     }
 }
 
-// Where the elements come from: flat arrays in element order, or (FLAT false) the sorted order a bilevel forward pass left
-// in its workspace (ctx and d_ctx in sorted order too; gradients and sharpness from the sort's arrays, GRU state and
-// cotangent gathered).
+// Where the elements come from: flat arrays in element order, or (FLAT false) the tensors of a bilevel pass, in the sorted
+// order that its forward scan left in the workspace (ctx and d_ctx in sorted order too; gradients and sharpness from the
+// sort's arrays, GRU state and cotangent gathered).
+// While every unit threshold is 0 - the state a meta-net is made in - the pass goes through the elements as they lie, and
+// the experts' sums are formed in one order that depends on nothing but the number of elements: PLAIN_GROUPS workgroups take
+// tiles of 256 elements in turns, the four elements of a step of either sign.  No element is an exception then, and the
+// first step of an optimizer that divides a gradient by its own size (Adam) makes the thresholds of these sums: of one that
+// nearly cancels, the order it was added up in decides a good part, and with it what every later pass computes.
+constexpr int PLAIN_GROUPS = 256, PLAIN_TILE = 256;
+__device__ __forceinline__ int plain_groups(int total) { return min(PLAIN_GROUPS, (total + PLAIN_TILE - 1) / PLAIN_TILE); }
 struct ElemArgs {
     const float *g, *s, *gru, *cot;       // flat only
     const float* ctx;
     float *smart, *d_ctx, *partials, *gru_out;
     const float* tables;
     int total;
-    bool normalise;                       // sorted only: the cotangent is -v / |v|, |v| over the tensor (v itself, negated, where |v| <= 1e-12)
+    const float* norms;                   // not flat, or NULL: the cotangent is -v / norms[tensor] (-v where that is <= 1e-12)
     float rescale;
     Sg2Weights W;
 };
@@ -220,16 +229,17 @@ __device__ __forceinline__ void best_four(const float (&sc)[PK], float* scratch,
             if (scratch[q] == fourth) set &= ~(1u << (PK - 1 - q));
         for (int q = 0; q < PK && __popc(set) < TOPK; q++) set |= 1u << (PK - 1 - q);
     }
-    float den = 0.0f;
+    float ex[TOPK];
 #pragma unroll
     for (int k = 0; k < TOPK; k++) {
         const int lead = __builtin_clz(set);          // set is never empty here
         idx[k] = lead - (32 - PK);
         set &= ~(0x80000000u >> lead);
-        wgt[k] = sg_exp(10.0f * (scratch[idx[k]] - best));
-        den += wgt[k];
+        ex[k] = wgt[k] = sg_exp(10.0f * (scratch[idx[k]] - best));
     }
-    const float inv = 1.0f / den;
+    // added from the best score down
+    order(ex[0], ex[1]); order(ex[2], ex[3]); order(ex[0], ex[2]); order(ex[1], ex[3]); order(ex[1], ex[2]);
+    const float inv = 1.0f / (((ex[0] + ex[1]) + ex[2]) + ex[3]);
 #pragma unroll
     for (int k = 0; k < TOPK; k++) wgt[k] *= inv;
 }
@@ -319,11 +329,18 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 
     const int ntiles = FLAT ? (a.total + 63) / 64 : pl.elem_tiles * (ELEM_TILE / 64);
     const int nwaves = (int)gridDim.x * BE_WAVES, wv = (int)blockIdx.x * BE_WAVES + wave;
-    const int tile0 = (int)((int64_t)ntiles * wv / nwaves), tile1 = (int)((int64_t)ntiles * (wv + 1) / nwaves);
+    int tile0 = (int)((int64_t)ntiles * wv / nwaves), tile1 = (int)((int64_t)ntiles * (wv + 1) / nwaves), step = 1;
+    const bool plain = !FLAT && !sorted_rows(pl);
+    if (plain) {
+        static_assert(PLAIN_TILE == 64 * BE_WAVES, "a tile of 64 per wave");
+        tile0 = wv;
+        tile1 = (int)blockIdx.x < plain_groups(a.total) ? (a.total + 63) / 64 : 0;
+        step = plain_groups(a.total) * BE_WAVES;
+    }
     const float kscale = a.rescale / (float)NH;
     sg::Seg seg = {-1, 0, 0};
     float cot_norm = 0.0f;
-    for (int tile = tile0; tile < tile1; tile++) {
+    for (int tile = tile0; tile < tile1; tile += step) {
         // every lane runs the element code (the wave works on whole tiles): lanes past the end redo the last element with a
         // zero cotangent, which zeroes everything they add, and store nothing
         bool valid;
@@ -337,17 +354,30 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             g = a.g[at]; s = a.s[at]; cot = valid ? a.cot[at] : 0.0f;
             h4 = reinterpret_cast<const float4*>(a.gru)[at];
             if (x_held < 0.0f) move_reference(0.0f);
+        } else if (plain) {
+            valid = tile * 64 + lane < a.total;
+            at = out_at = valid ? tile * 64 + lane : a.total - 1;
+            int ti = 0;                      // the lane's tensor: the last one that starts no later
+            for (int n = pl.P; n > 1;) {
+                const int half = n / 2;
+                if (pl.tensors[ti + half].off <= at) ti += half;
+                n -= half;
+            }
+            const TensorDev& T = pl.tensors[ti];
+            const int orig = at - T.off;
+            g = sg::load_elem(T.grad, T.dtype, orig);
+            s = sharp_rounded(T, orig);
+            cot = sg::load_elem(T.param, T.dtype, orig);
+            if (a.norms) { const float norm = a.norms[ti]; cot = -(norm > 1e-12f ? cot / norm : cot); }
+            cot = valid ? cot : 0.0f;
+            const be_f32x4 hv = ((const SG_GLOBAL be_f32x4*)T.gru)[orig];
+            h4 = make_float4(hv[0], hv[1], hv[2], hv[3]);
+            if (x_held < 0.0f) move_reference(0.0f);
         } else {
             const int et = tile / (ELEM_TILE / 64);
             if (et >= seg.end) {
                 seg = sg::find_seg(sg::as_const(pl.elem_tile_prefix), pl.P, et);
-                if (a.normalise) {           // |v| of the tensor from its norm tiles
-                    double part = 0.0;
-                    for (int k = pl.norm_tile_prefix[seg.i] + lane; k < pl.norm_tile_prefix[seg.i + 1]; k += 64) part += pl.norm_partials[k];
-#pragma unroll
-                    for (int d = 32; d >= 1; d >>= 1) part += __shfl_xor(part, d, 64);
-                    cot_norm = (float)sqrt(part);
-                }
+                cot_norm = a.norms ? a.norms[seg.i] : 0.0f;
             }
             const TensorDev& T = pl.tensors[seg.i];
             const int start = (et - seg.first) * ELEM_TILE + (tile % (ELEM_TILE / 64)) * 64;
@@ -368,7 +398,7 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                 if (s == 0.0f) s = sharp_rounded(T, orig);
             }
             cot = sg::load_elem(T.param, T.dtype, orig);
-            if (a.normalise) cot = -(cot_norm > 1e-12f ? cot / cot_norm : cot);
+            if (a.norms) cot = -(cot_norm > 1e-12f ? cot / cot_norm : cot);
             cot = valid ? cot : 0.0f;
             const be_f32x4 hv = ((const SG_GLOBAL be_f32x4*)T.gru)[orig];
             h4 = make_float4(hv[0], hv[1], hv[2], hv[3]);
@@ -379,9 +409,9 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
         const unsigned long long pos = __builtin_amdgcn_ballot_w64(g > 0.0f);
         const int npos = __popcll(pos), npos8 = (npos + 7) >> 3, nneg8 = (64 - npos + 7) >> 3;
         const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(pos >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)pos, 0u));      // positive elements in lower lanes
-        const int slot = g > 0.0f ? before : 8 * npos8 + (lane - before);
+        const int slot = plain ? lane : g > 0.0f ? before : 8 * npos8 + (lane - before);
         // ... of which lane 0..7 / 8..15 clears one
-        const int pad = (lane < 8 ? npos : 8 * npos8 + (64 - npos) - 8) + lane, pad_end = lane < 8 ? 8 * npos8 : lane < 16 ? 8 * (npos8 + nneg8) : 0;
+        const int pad = (lane < 8 ? npos : 8 * npos8 + (64 - npos) - 8) + lane, pad_end = plain ? 0 : lane < 8 ? 8 * npos8 : lane < 16 ? 8 * (npos8 + nneg8) : 0;
 
         float cf[DM], cb[DM], h[GH] = {h4.x, h4.y, h4.z, h4.w};
         {
@@ -555,9 +585,21 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                         acc_g = __builtin_amdgcn_mfma_f32_16x16x4f32(a1 * g1, b1, acc_g, 0, 0, 0);
                     }
                 };
-                fetch();
-                sums(npos8, cen[0], cen[2]);
-                sums(nneg8, cen[1], cen[3]);
+                if (!plain) {
+                    fetch();
+                    sums(npos8, cen[0], cen[2]);
+                    sums(nneg8, cen[1], cen[3]);
+                } else {
+#pragma unroll 1
+                    for (int t = 0; t < 16; t++, row += 4 * CW) {
+                        const float a4 = row[li], b4 = row[PK + li], g4 = row[2 * PK];
+                        const float ap = g4 > 0.0f ? a4 : 0.0f, an = g4 > 0.0f ? 0.0f : a4;
+                        cen[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ap, b4, cen[0], 0, 0, 0);
+                        cen[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(an, b4, cen[1], 0, 0, 0);
+                        cen[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(ap * g4, b4, cen[2], 0, 0, 0);
+                        cen[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(an * g4, b4, cen[3], 0, 0, 0);
+                    }
+                }
                 wave_sync();
             }
             // ---- routing backward: softmax, scores, query
@@ -760,8 +802,10 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 // d b2 = sum w.
 constexpr int FIN_SLICES = 8;
 constexpr int FIN_DENSE = (N_DENSE + 63) / 64;
+// (All thresholds 0 in the bilevel pass: the gradients are formed per row and then added, in four slices, for the one order of
+// k_bilevel_elem's sums.)
 __global__ __launch_bounds__(64 * FIN_SLICES) void k_elem_finish(const float* __restrict__ partials, int rows, Sg2Weights W, int eh,
-                                                                 float* __restrict__ out) {
+                                                                 float* __restrict__ out, Plan pl) {
     __shared__ float s_part[FIN_SLICES][64];
     const int col = threadIdx.x & 63, slice = threadIdx.x >> 6;
     const bool dense = blockIdx.x < FIN_DENSE;
@@ -770,6 +814,32 @@ __global__ __launch_bounds__(64 * FIN_SLICES) void k_elem_finish(const float* __
     const bool live = dense ? o < N_DENSE : col < 2 * NBIN;
     const float* src = partials + (dense ? N_BINS + o : e * NBIN * 2 + o);
     float acc = 0.0f;
+    if (!dense && pl.whole_pass && !sorted_rows(pl)) {
+        // columns: d W1[16], d b1[16], d W2[16], d b2; of a unit's active side only the bin next to zero is not empty
+        const int kind = col / EH, m = col % EH, mw = min(m, eh - 1);
+        const float w1 = W.w[W_EXP_W1][e * eh + mw], b1 = W.w[W_EXP_B1][e * eh + mw], w2 = W.w[W_EXP_W2][e * eh + mw];
+        int above = 0;
+        for (int q = 0; q < eh; q++) above += W.w[W_EXP_W1][e * eh + q] != 0.0f ? 1 : 0;
+        const float* bin = partials + e * NBIN * 2;
+        rows = plain_groups(pl.total);
+        if (slice < 4) {
+#pragma unroll 4
+            for (int r = slice; r < rows; r += 4) {
+                const float* at = bin + (size_t)r * ROW_FLOATS + (w1 > 0.0f ? 2 * above : 0);
+                const float S0 = w1 != 0.0f ? at[0] : 0.0f, S1 = w1 != 0.0f ? at[1] : 0.0f;
+                acc += kind == 0 ? w2 * S1 : kind == 1 ? w2 * S0 : kind == 2 ? sg_fma(w1, S1, b1 * S0)
+                                 : above > 0 ? bin[(size_t)r * ROW_FLOATS] + bin[(size_t)r * ROW_FLOATS + 2 * above] : bin[(size_t)r * ROW_FLOATS];
+            }
+        }
+        s_part[slice][col] = acc;
+        __syncthreads();
+        if (slice != 0) return;
+        acc = ((s_part[0][col] + s_part[1][col]) + s_part[2][col]) + s_part[3][col];
+        float* const dst = out + N_DENSE;
+        if (kind < 3 && m < eh) dst[kind * NE * eh + e * eh + m] = acc;
+        if (col == 3 * EH) dst[3 * NE * eh + e] = acc;
+        return;
+    }
     if (live) {
 #pragma unroll 8
         for (int r = slice; r < rows; r += FIN_SLICES) acc += src[(size_t)r * ROW_FLOATS];
@@ -813,7 +883,13 @@ int elem_groups(int64_t tiles) {
 
 size_t elem_workspace(int groups) { return sizeof(float) * (TABLE_FLOATS + (size_t)groups * ROW_FLOATS); }
 
-// a.tables and a.partials are set here, from the workspace
+int run_tables(const Sg2Weights& W, int eh, float* tables, int* all_zero, hipStream_t st) {
+    hipLaunchKernelGGL(k_expert_tables, dim3(NE), dim3(64), 0, st, W, eh, tables, all_zero);
+    SG_LAUNCH_CHECK("k_expert_tables");
+    return 0;
+}
+
+// a.tables and a.partials are set here, from the workspace; the tables are there
 template <bool FLAT>
 int run_elem(ElemArgs& a, const Plan& pl, int groups, int eh, void* workspace, float* grads_out, hipStream_t st) {
     {
@@ -829,11 +905,9 @@ int run_elem(ElemArgs& a, const Plan& pl, int groups, int eh, void* workspace, f
     float* tables = static_cast<float*>(workspace);
     a.tables = tables;
     a.partials = tables + TABLE_FLOATS;
-    hipLaunchKernelGGL(k_expert_tables, dim3(NE), dim3(64), 0, st, a.W, eh, tables);
-    SG_LAUNCH_CHECK("k_expert_tables");
     hipLaunchKernelGGL(k_bilevel_elem<FLAT>, dim3(groups), dim3(BE_THREADS), BE_LDS_BYTES, st, a, pl);
     SG_LAUNCH_CHECK("k_bilevel_elem");
-    hipLaunchKernelGGL(k_elem_finish, dim3(FIN_DENSE + NE), dim3(64 * FIN_SLICES), 0, st, a.partials, groups, a.W, eh, grads_out);
+    hipLaunchKernelGGL(k_elem_finish, dim3(FIN_DENSE + NE), dim3(64 * FIN_SLICES), 0, st, a.partials, groups, a.W, eh, grads_out, pl);
     SG_LAUNCH_CHECK("k_elem_finish");
     return 0;
 }
@@ -841,10 +915,13 @@ int run_elem(ElemArgs& a, const Plan& pl, int groups, int eh, void* workspace, f
 }  // namespace
 
 size_t bilevel_elem_workspace(int elem_tiles) { return elem_workspace(elem_groups((int64_t)elem_tiles * (ELEM_TILE / 64))); }
-int launch_bilevel_elem(const Plan& pl, bool normalise, int eh, float* smart_out, float* d_ctx, float* grads_out, void* workspace, hipStream_t st) {
+int launch_expert_tables(const Plan& pl, int eh, void* workspace, hipStream_t st) {
+    return run_tables(pl.W, eh, static_cast<float*>(workspace), pl.contracted + 3, st);
+}
+int launch_bilevel_elem(const Plan& pl, const float* norms, int eh, float* smart_out, float* d_ctx, float* grads_out, void* workspace, hipStream_t st) {
     ElemArgs a = {};
     a.ctx = pl.ctx; a.smart = smart_out; a.d_ctx = d_ctx;
-    a.total = pl.total; a.normalise = normalise; a.rescale = pl.rescale; a.W = pl.W;
+    a.total = pl.total; a.norms = norms; a.rescale = pl.rescale; a.W = pl.W;
     return run_elem<false>(a, pl, elem_groups((int64_t)pl.elem_tiles * (ELEM_TILE / 64)), eh, workspace, grads_out, st);
 }
 }  // namespace sg2
@@ -886,6 +963,7 @@ int sg2_bilevel_elem_ex(const SgDims* dims, const Sg2Weights* weights, int64_t t
     a.g = grad; a.s = sharpness; a.ctx = ctx; a.gru = gru_state; a.cot = cotangent;
     a.smart = smart_out; a.d_ctx = d_ctx; a.gru_out = gru_out;
     a.total = (int)total; a.rescale = rescale; a.W = *weights;
+    if (run_tables(a.W, EH, static_cast<float*>(workspace), nullptr, st)) return 1;
     return run_elem<true>(a, Plan{}, groups, EH, workspace, grads_out, st);
 }
 

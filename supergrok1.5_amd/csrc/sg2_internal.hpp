@@ -133,11 +133,11 @@ struct Plan {
     float* adj_lam;                // bilevel: [2][chunks][128][2] adjoint state arriving at the end of every chunk
     float* adj_blk;                // bilevel: [2][SG2_BWD_STRIDE] sums of adj_part's rows
     float* adj_part;               // bilevel: [2][ADJ_GROUPS][SG2_BWD_STRIDE] per-workgroup gradient sums
-    int* contracted;               // [0] set by k_compose (1 while every carried state of the call is finite), cleared by any summary whose 2x2 part is not exactly zero; [1] steps of a summary's first block (k_compose); [2] k_compose: some carried state is not finite
+    int* contracted;               // [3] bilevel pass: every unit threshold of the experts is 0 (set by k_tables, cleared by k_expert_tables); [0] set by k_compose (1 while every carried state of the call is finite), cleared by any summary whose 2x2 part is not exactly zero; [1] steps of a summary's first block (k_compose); [2] k_compose: some carried state is not finite
     int* state_bad;                // [P] set by k_tables: a carried Mamba state of the tensor holds a non-finite entry
     int* sharp_nonzero;            // [P] uploaded as 0; set by k_keys when some sharpness entry of the tensor is not 0
     float* ctx;                    // [2][total][d_model]
-    bool own_order;                // bilevel pass in one call: ctx and its gradient lie in the order of the sort, and the carried states are only read
+    bool whole_pass;               // bilevel pass in one call: the carried states are only read, and ctx and its gradient lie in sorted order (see sorted_rows)
     float decay, beta2, eps, rescale;
     Sg2Weights W;
 };
@@ -160,8 +160,7 @@ __device__ __forceinline__ float sharp_value(const TensorDev& T, float v) { retu
 __device__ __forceinline__ float sharp_rounded(const TensorDev& T, int64_t i) { const float v = sharp_raw(T, i); return T.sharp32 == 1 ? sg::round_to(T.dtype, v) : v; }      // not finite stays so
 __device__ __forceinline__ float sharp_of(const TensorDev& T, int64_t i) { return sharp_value(T, sharp_raw(T, i)); }
 
-// sums of squares per norm tile of the gradients, or of the tensors `param` points to
-int launch_norm(const Plan& pl, bool of_param, hipStream_t st);
+int launch_norm(const Plan& pl, hipStream_t st);
 int launch_sort(const Plan& pl, int32_t* dbg_perm, hipStream_t st);
 int launch_scan(const Plan& pl, hipStream_t st);
 // bilevel path: the forward scan keeps the state entering every HT_STEP-th step of a tensor; index of scan step u
@@ -184,9 +183,13 @@ int check_dims(const SgDims* d, bool per_element = false);
 // exactly one of d_ctx (element order, after out_proj) / d_scan (scan order, before out_proj) is given; dx (with rx) is optional
 int launch_bilevel_backward(const Plan& pl, const float* d_ctx, const float* const d_scan[2], const float* rx, float* dx, float* grads_out,
                             hipStream_t st);
-// the per-element part of the bilevel pass on the elements as the forward scan left them (own_order); eh: the experts' true width
+// Whether the rows of ctx and of its gradient lie in the order of the sort: in the whole pass, unless every unit threshold of
+// the experts is 0 (see k_bilevel_elem).
+__device__ __forceinline__ bool sorted_rows(const Plan& pl) { return pl.whole_pass && __builtin_amdgcn_readfirstlane(pl.contracted[3]) == 0; }
+// the per-element part of the whole pass; eh: the experts' true width.  launch_expert_tables goes before the forward scan.
 size_t bilevel_elem_workspace(int elem_tiles);
-int launch_bilevel_elem(const Plan& pl, bool normalise, int eh, float* smart_out, float* d_ctx, float* grads_out, void* workspace, hipStream_t st);
+int launch_expert_tables(const Plan& pl, int eh, void* workspace, hipStream_t st);
+int launch_bilevel_elem(const Plan& pl, const float* norms, int eh, float* smart_out, float* d_ctx, float* grads_out, void* workspace, hipStream_t st);
 int launch_saved_intermediates(const Plan& pl, const Sg2BilevelExtra& ex, hipStream_t st);
 int launch_x_sorted(const Plan& pl, float* x_out, hipStream_t st);
 int launch_elem(const Plan& pl, int32_t* expert_counts, int32_t* dbg_expert_idx, hipStream_t st);

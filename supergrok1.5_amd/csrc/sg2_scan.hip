@@ -930,6 +930,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         }
     }
 
+    const bool in_order = KEEP && sorted_rows(pl);
     uint32_t nx_key = 0;
     int32_t nx_val = 0;
     float nx_sh = 0.0f;
@@ -1133,7 +1134,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                 }
             }
             const float cx[DM] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            const int at = KEEP && pl.own_order ? (dir ? N - 1 - (tile0 + tu) : tile0 + tu) : orig;
+            const int at = KEEP && in_order ? (dir ? N - 1 - (tile0 + tu) : tile0 + tu) : orig;
             held_dst = valid ? reinterpret_cast<float4*>(pl.ctx + ((size_t)dir * pl.total + off + at) * DM) : nullptr;
             held[0] = make_float4(cx[0], cx[1], cx[2], cx[3]);
             held[1] = make_float4(cx[4], cx[5], cx[6], cx[7]);
@@ -1148,7 +1149,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         __syncthreads();
     }
     flush();
-    if (u1 == N && !(KEEP && pl.own_order)) {   // last chunk in scan order: new carried state of the tensor
+    if (u1 == N && !(KEEP && pl.whole_pass)) {   // last chunk in scan order: new carried state of the tensor
         float* st = dir ? T.mbwd : T.mfwd;
 #pragma unroll
         for (int h = 0; h < 2; h++) {

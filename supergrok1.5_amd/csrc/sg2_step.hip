@@ -175,7 +175,7 @@ int make_layout(int geo, int P, Numels numels, int chunk_len, Layout* L, bool bi
     L->off_comp = take(4 * (2 * 5 * (size_t)gi.rows * 3 + 2 * 2 * (size_t)gi.rows * 4 + 16));      // composed triples, Taylor polynomials, coefficient maxima and polynomial limits
     L->off_norm = take(8 * (size_t)nt);
     L->off_gscale = take(4 * (size_t)P);
-    L->off_flags = take(4 * (2 * (size_t)P + 3));    // apart from the tensor records: it is written while those are being read
+    L->off_flags = take(4 * (2 * (size_t)P + 4));    // apart from the tensor records: it is written while those are being read
     L->off_padw = take(4 * (size_t)padded_weight_floats(gi));   // scan weights embedded in the kernel geometry (used when the caller's block is smaller)
     L->off_ctx = take(4 * 2 * (size_t)total * gi.dm);
     // bilevel only: state entering every HT_STEP-th step, both directions
@@ -231,6 +231,7 @@ __global__ __launch_bounds__(256) void k_tables(TableChunk c) {
     if (c.i0 == 0 && threadIdx.x < PREFIXES) c.dst_pre[threadIdx.x * (c.P + 1)] = 0;
     if (c.flags != nullptr)
         for (int k = threadIdx.x; k < c.cnt; k += 256) c.flags[c.i0 + k] = 0;
+    if (c.flags != nullptr && c.i0 == 0 && threadIdx.x == 0) c.flags[c.P + 3] = 1;
 }
 
 // Pre-pass of a clipping call (supergrok2.py:316-321 of the reference): sums of squares of every tensor's gradient, one per
@@ -238,20 +239,19 @@ __global__ __launch_bounds__(256) void k_tables(TableChunk c) {
 // it.  HBM bound (one read of the gradients); writing clipped copies and reading those instead cost a second pass (38 us
 // for 25 M elements) and three launches.  (The tile that finishes a tensor could add them up here, but an atomic counter
 // with release order per workgroup took 38 us where the plain stores take 5: each one writes back its L2.)
-__global__ __launch_bounds__(256) void k_norm(Plan pl, bool of_param) {
+__global__ __launch_bounds__(256) void k_norm(Plan pl) {
     __shared__ double sm[4];
     const int tile = blockIdx.x;
     const sg::Seg seg = sg::find_seg(sg::as_const(pl.norm_tile_prefix), pl.P, tile);
     const TensorDev& T = pl.tensors[seg.i];
     const int start = (tile - seg.first) * pl.norm_tile, cnt = min(pl.norm_tile, T.numel - start);
-    const void* const src = of_param ? T.param : T.grad;
     float acc = 0.0f;
     for (int k0 = 0; k0 < cnt; k0 += 8 * 256) {       // eight loads on their way at a time, added in order
         float g[8];
 #pragma unroll
         for (int r = 0; r < 8; r++) {
             const int k = k0 + r * 256 + (int)threadIdx.x;
-            g[r] = k < cnt ? sg::load_elem(src, T.dtype, start + k) : 0.0f;
+            g[r] = k < cnt ? sg::load_elem(T.grad, T.dtype, start + k) : 0.0f;
         }
 #pragma unroll
         for (int r = 0; r < 8; r++) acc = sg_fma(g[r], g[r], acc);
@@ -262,8 +262,8 @@ __global__ __launch_bounds__(256) void k_norm(Plan pl, bool of_param) {
 
 }  // namespace
 
-int launch_norm(const Plan& pl, bool of_param, hipStream_t st) {
-    hipLaunchKernelGGL(k_norm, dim3(pl.norm_tiles), dim3(256), 0, st, pl, of_param);
+int launch_norm(const Plan& pl, hipStream_t st) {
+    hipLaunchKernelGGL(k_norm, dim3(pl.norm_tiles), dim3(256), 0, st, pl);
     SG_LAUNCH_CHECK("k_norm");
     return 0;
 }
@@ -447,7 +447,7 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
         for (int i0 = 0; i0 < P; i0 += UPLOAD_RECS) {
             TableChunk c;
             c.dst_rec = d_rec; c.dst_pre = d_pre; c.flags = d_flags;
-            c.state_bad = reinterpret_cast<int*>(ws + L.off_flags) + P + 3;
+            c.state_bad = reinterpret_cast<int*>(ws + L.off_flags) + P + 4;
             c.state_floats = dims->d_inner * dims->d_state;
             c.i0 = i0; c.cnt = P - i0 < UPLOAD_RECS ? P - i0 : UPLOAD_RECS; c.P = P;
             for (int k = 0; k < c.cnt; k++) {
@@ -488,7 +488,7 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
     pl.norm_partials = reinterpret_cast<double*>(ws + L.off_norm);
     pl.gscale = nullptr;
     pl.max_norm = 0.0f;
-    pl.own_order = whole_pass;
+    pl.whole_pass = whole_pass;
     pl.P = P; pl.total = L.total; pl.elem_tiles = L.elem_tiles; pl.sort_tiles = L.sort_tiles;
     pl.chunks = L.chunks; pl.wchunks = L.wchunks; pl.chunk_len = chunk_len; pl.window = window_override >= 0 ? window_override : g_window.load();
     for (int k = 0; k < 2; k++) {
@@ -503,7 +503,7 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
     pl.comp = reinterpret_cast<float*>(ws + L.off_comp);
     pl.sharp_nonzero = reinterpret_cast<int*>(ws + L.off_flags);
     pl.contracted = pl.sharp_nonzero + P;
-    pl.state_bad = pl.contracted + 3;
+    pl.state_bad = pl.contracted + 4;
     pl.ctx = reinterpret_cast<float*>(ws + L.off_ctx);
     pl.decay = 1.0f - scalars->lr * scalars->wd_eff;
     pl.beta2 = scalars->beta2; pl.eps = scalars->eps; pl.rescale = scalars->rescale;
@@ -562,7 +562,7 @@ int run_step(const SgDims* dims, const Sg2Weights* weights, int num_tensors, con
     if (clip_norm > 0.0f) {
         pl.gscale = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + L.off_gscale);
         pl.max_norm = clip_norm;
-        if (launch_norm(pl, false, st)) return 1;
+        if (launch_norm(pl, st)) return 1;
     }
     if (launch_sort(pl, debug ? debug->perm : nullptr, st)) return 1;
     prof_mark(1, st);
@@ -765,7 +765,7 @@ size_t sg2_bilevel_pass_workspace_bytes(const SgDims* dims, int num_tensors, con
     return L.bytes;
 }
 
-int sg2_bilevel_pass(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, float rescale, int normalise,
+int sg2_bilevel_pass(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, float rescale, const float* norms,
                      float* smart_out, float* elem_grads_out, float* scan_grads_out, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace sg2;
     hipStream_t st = (hipStream_t)stream;
@@ -789,10 +789,10 @@ int sg2_bilevel_pass(const SgDims* dims, const Sg2Weights* weights, int num_tens
     if (pl.total == 0) return sg::fail("sg2_bilevel_pass: no elements");
     unsigned char* ws = static_cast<unsigned char*>(workspace);
     float* d_ctx = reinterpret_cast<float*>(ws + L.off_dctx);
-    if (normalise && launch_norm(pl, true, st)) return 1;
+    if (launch_expert_tables(pl, dims->expert_hidden, ws + L.off_elem, st)) return 1;
     if (launch_sort(pl, nullptr, st)) return 1;
     if (launch_scan(pl, st)) return 1;
-    if (launch_bilevel_elem(pl, normalise != 0, dims->expert_hidden, smart_out, d_ctx, elem_grads_out, ws + L.off_elem, st)) return 1;
+    if (launch_bilevel_elem(pl, norms, dims->expert_hidden, smart_out, d_ctx, elem_grads_out, ws + L.off_elem, st)) return 1;
     return launch_bilevel_backward(pl, d_ctx, nullptr, nullptr, nullptr, scan_grads_out, st);
 }
 
