@@ -406,11 +406,13 @@ int sg2_bilevel_elem_ex(const SgDims* dims, const Sg2Weights* weights, int64_t t
                         const float* ctx, const float* gru_state, const float* cotangent, float rescale, float* smart_out,
                         float* gru_out, float* d_ctx, float* grads_out, void* workspace, size_t workspace_bytes, void* stream);
 
-/* The whole bilevel pass in one call: sg2_bilevel_forward, sg2_bilevel_elem and sg2_bilevel_backward on tensors that
- * stay where they are.  Of a record only grad, sharpness, gru_state, the two Mamba states (all read only), param - the
- * cotangent, in the tensor's dtype -, numel and dtype (SG_SHARP_F32, SG_SHARP_EXACT) are used.  norms (device memory, one
- * per tensor, or NULL): tensor t's element i then has the cotangent -v_i / norms[t] (-v_i where norms[t] <= 1e-12), as the
- * bilevel update takes it from the validation gradient v and its 2-norm; else v_i.
+/* The whole bilevel pass on tensors that stay where they are: sg2_bilevel_forward, sg2_bilevel_elem and
+ * sg2_bilevel_backward in two calls on one workspace, the first of which needs no cotangent: it can run while the caller
+ * still computes the validation gradient.  Of a record grad, sharpness, gru_state, the two Mamba states (all read
+ * only), numel and dtype (SG_SHARP_F32, SG_SHARP_EXACT) are used, by the second call also param: the cotangent, in
+ * the tensor's dtype.  norms (device memory, one per tensor, or NULL): tensor t's element i then has the cotangent
+ * -v_i / norms[t] (-v_i where norms[t] <= 1e-12), as the bilevel update takes it from the validation gradient v and its
+ * 2-norm; else v_i.
  *   smart_out [sum numel]  smart gradients, packed in call order (may be NULL)
  *   elem_grads_out         as grads_out of sg2_bilevel_elem, the expert tensors at the caller's own expert_hidden
  *                          (1364 + 144 * (3 * expert_hidden + 1) floats)
@@ -418,8 +420,11 @@ int sg2_bilevel_elem_ex(const SgDims* dims, const Sg2Weights* weights, int64_t t
  * Built for d_model 8, d_state 16, d_inner 16, gru_hidden 4, 4 heads, 12 keys, 144 experts of width <= 16.  Contexts and
  * their gradients travel between the three parts in the workspace. */
 size_t sg2_bilevel_pass_workspace_bytes(const SgDims* dims, int num_tensors, const int64_t* numels);
-int sg2_bilevel_pass(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, float rescale, const float* norms,
-                     float* smart_out, float* elem_grads_out, float* scan_grads_out, void* workspace, size_t workspace_bytes, void* stream);
+int sg2_bilevel_pass_begin(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, void* workspace,
+                           size_t workspace_bytes, void* stream);
+int sg2_bilevel_pass_finish(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, float rescale,
+                            const float* norms, float* smart_out, float* elem_grads_out, float* scan_grads_out, void* workspace,
+                            size_t workspace_bytes, void* stream);
 
 /* The meta-net's own forward with the step's hard top-1 routing, for callers that use the net outside the fused
  * step: Mamba3PEERMetaNet.forward (grokking_optimizers/mamba3_peer_metanet.py:275-370 of the reference).  Sort,

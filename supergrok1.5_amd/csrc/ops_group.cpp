@@ -510,88 +510,111 @@ int64_t supergrok2_flat_step(py::list params, py::list eas, py::list easqs, py::
     return (int64_t)active.size();
 }
 
-// The bilevel pass over tensors that stay where they are (sg2_bilevel_pass): (smart gradients or None, gradients of the
-// per-element weights, gradients of the scan weights), flat.  normalise: the cotangent is -v / |v|.  exact: fp32 sharpness next to 16-bit gradients is used as it
-// is.  None where the general path has to be taken (other sizes of the net, tensors that would have to be converted).
-py::object supergrok2_bilevel_pass(py::list grads, py::list sharps, py::list grus, py::list mfwd, py::list mbwd, py::list cots,
-                                   py::list weights, float rescale, bool normalise, bool exact, bool want_smart, std::vector<int> dims8) {
-    const char* fn = "supergrok2_bilevel_pass";
+// The bilevel pass over tensors that stay where they are.  begin (sort and scan) returns what finish needs, or None where the
+// general path has to be taken (other sizes of the net, tensors that would have to be converted).
+struct BilevelPass {
+    SgDims dims;
+    Sg2Weights W;
+    std::vector<Sg2Tensor> ts;
+    std::vector<Py_ssize_t> at;            // the lists' index of each
+    std::vector<at::Tensor> kept;          // whatever the records point to
+    torch::Tensor ws;
+    int64_t total = 0;
+};
+
+// exact: fp32 sharpness next to 16-bit gradients is used as it is
+py::object supergrok2_bilevel_begin(py::list grads, py::list sharps, py::list grus, py::list mfwd, py::list mbwd, py::list weights, bool exact,
+                                    std::vector<int> dims8) {
+    const char* fn = "supergrok2_bilevel_begin";
     const Py_ssize_t P = PyList_GET_SIZE(grads.ptr());
-    for (PyObject* l : {sharps.ptr(), grus.ptr(), mfwd.ptr(), mbwd.ptr(), cots.ptr()})
+    for (PyObject* l : {sharps.ptr(), grus.ptr(), mfwd.ptr(), mbwd.ptr()})
         if (PyList_GET_SIZE(l) != P) return py::none();
     if (P == 0 || dims8.size() != 8 || PyList_GET_SIZE(weights.ptr()) != SG2_NUM_WEIGHTS) return py::none();
+    auto pass = std::make_unique<BilevelPass>();
     const SgDims dims = {dims8[0], dims8[1], dims8[2], dims8[3], dims8[4], dims8[5], dims8[6], dims8[7]};
+    pass->dims = dims;
     auto item = [](const py::list& l, Py_ssize_t i) { return as_tensor(PyList_GET_ITEM(l.ptr(), i)); };
-    std::vector<Sg2Tensor> ts;
     std::vector<int64_t> numels;
-    std::vector<at::Tensor> held;        // cotangents that had to be made contiguous
-    std::vector<const at::Tensor*> active;
-    held.reserve(P);
-    int64_t total = 0;
-    const at::Tensor* first = nullptr;
+    pass->kept.reserve(5 * P + SG2_NUM_WEIGHTS);
     for (Py_ssize_t i = 0; i < P; i++) {
-        const at::Tensor *g = item(grads, i), *s = item(sharps, i), *gru = item(grus, i), *mf = item(mfwd, i), *mb = item(mbwd, i),
-                         *c = item(cots, i);
-        if (!g || !s || !gru || !mf || !mb || !c) return py::none();
+        const at::Tensor *g = item(grads, i), *s = item(sharps, i), *gru = item(grus, i), *mf = item(mfwd, i), *mb = item(mbwd, i);
+        if (!g || !s || !gru || !mf || !mb) return py::none();
         const int64_t n = g->numel();
         if (n == 0) continue;
-        if (!g->is_cuda() || !g->is_contiguous() || g->scalar_type() != c->scalar_type() || c->numel() != n || s->numel() != n) return py::none();
-        for (const at::Tensor* t : {s, gru, mf, mb})
+        if (s->numel() != n || gru->numel() != n * dims.gru_hidden || mf->numel() != (int64_t)dims.d_inner * dims.d_state ||
+            mb->numel() != mf->numel())
+            return py::none();
+        for (const at::Tensor* t : {g, s, gru, mf, mb}) {
             if (!t->is_cuda() || !t->is_contiguous()) return py::none();
+            pass->kept.push_back(*t);
+        }
         for (const at::Tensor* t : {gru, mf, mb})
             if (t->scalar_type() != torch::kFloat32) return py::none();
-        if (gru->numel() != n * dims.gru_hidden || mf->numel() != (int64_t)dims.d_inner * dims.d_state || mb->numel() != mf->numel()) return py::none();
-        if (((uintptr_t)gru->data_ptr() & 15u) != 0 || !c->is_cuda()) return py::none();
-        if (!c->is_contiguous()) {
-            held.push_back(c->contiguous());
-            c = &held.back();
-        }
+        if (((uintptr_t)gru->data_ptr() & 15u) != 0) return py::none();
         Sg2Tensor q = {};
         q.dtype = dtype_code(*g, "grad");
         if (s->scalar_type() != g->scalar_type()) {
             if (!exact || s->scalar_type() != torch::kFloat32) return py::none();
             q.dtype |= SG_SHARP_F32 | SG_SHARP_EXACT;
         }
-        q.param = c->data_ptr();
         q.grad = g->data_ptr();
         q.sharpness = s->data_ptr();
         q.gru_state = gru->data_ptr<float>();
         q.mamba_fwd_state = mf->data_ptr<float>();
         q.mamba_bwd_state = mb->data_ptr<float>();
         q.numel = n;
-        ts.push_back(q);
+        pass->ts.push_back(q);
+        pass->at.push_back(i);
         numels.push_back(n);
-        active.push_back(c);
-        total += n;
-        if (!first) first = g;
+        pass->total += n;
     }
-    if (!first) return py::none();
+    if (pass->ts.empty()) return py::none();
+    const at::Tensor like = pass->kept[0];
     const torch::Tensor* w[SG2_NUM_WEIGHTS];
     for (int k = 0; k < SG2_NUM_WEIGHTS; k++) {
         w[k] = item(weights, k);
         if (!w[k]) return py::none();
+        pass->kept.push_back(*w[k]);
     }
-    Sg2Weights W;
-    check_sg2_weights(fn, w, dims, &W);
-    const size_t bytes = sg2_bilevel_pass_workspace_bytes(&dims, (int)ts.size(), numels.data());
+    check_sg2_weights(fn, w, dims, &pass->W);
+    const size_t bytes = sg2_bilevel_pass_workspace_bytes(&dims, (int)pass->ts.size(), numels.data());
     TORCH_CHECK(bytes > 0, fn, ": ", sg_last_error());
-    auto ws = make_workspace(bytes, *first);
-    const auto opt = torch::TensorOptions().device(first->device()).dtype(torch::kFloat32);
-    auto elem = torch::empty({(SG2_ELEM_GRAD_FLOATS - dims.num_experts * 49) + dims.num_experts * (3 * dims.expert_hidden + 1)}, opt);
-    auto scan = torch::empty({SG2_SCAN_GRAD_FLOATS}, opt);
+    pass->ws = make_workspace(bytes, like);
+    check_status(sg2_bilevel_pass_begin(&dims, &pass->W, (int)pass->ts.size(), pass->ts.data(), pass->ws.data_ptr(), (size_t)pass->ws.numel(),
+                                        current_stream(like)), fn);
+    return py::cast(std::move(pass));
+}
+
+// (smart gradients or None, gradients of the per-element weights, gradients of the scan weights), flat; normalise: the
+// cotangent is -v / |v|.  None where a cotangent is not of its gradient's size and type.
+py::object supergrok2_bilevel_finish(BilevelPass& pass, py::list cots, float rescale, bool normalise, bool want_smart) {
+    const char* fn = "supergrok2_bilevel_finish";
+    at::NoGradGuard guard;
+    const Py_ssize_t given = PyList_GET_SIZE(cots.ptr());
+    std::vector<at::Tensor> v;
+    for (size_t k = 0; k < pass.ts.size(); k++) {
+        const at::Tensor* c = pass.at[k] < given ? as_tensor(PyList_GET_ITEM(cots.ptr(), pass.at[k])) : nullptr;
+        if (!c || !c->is_cuda() || c->numel() != pass.ts[k].numel || dtype_code(*c, "cotangent") != (pass.ts[k].dtype & ~(SG_SHARP_F32 | SG_SHARP_EXACT)))
+            return py::none();
+        v.push_back(c->contiguous());
+        pass.ts[k].param = v.back().data_ptr();
+    }
+    const auto opt = torch::TensorOptions().device(pass.ws.device()).dtype(torch::kFloat32);
     torch::Tensor norms;
     if (normalise) {
-        at::NoGradGuard guard;
-        norms = torch::empty({(int64_t)ts.size()}, opt);
-        for (size_t i = 0; i < ts.size(); i++) {
+        norms = torch::empty({(int64_t)v.size()}, opt);
+        for (size_t i = 0; i < v.size(); i++) {
             at::Tensor out = norms.select(0, i);
-            at::linalg_vector_norm_out(out, active[i]->scalar_type() == torch::kFloat32 ? *active[i] : active[i]->to(torch::kFloat32), 2);
+            at::linalg_vector_norm_out(out, v[i].scalar_type() == torch::kFloat32 ? v[i] : v[i].to(torch::kFloat32), 2);
         }
     }
+    auto elem = torch::empty({(SG2_ELEM_GRAD_FLOATS - pass.dims.num_experts * 49) + pass.dims.num_experts * (3 * pass.dims.expert_hidden + 1)}, opt);
+    auto scan = torch::empty({SG2_SCAN_GRAD_FLOATS}, opt);
     torch::Tensor smart;
-    if (want_smart) smart = torch::empty({total}, opt);
-    check_status(sg2_bilevel_pass(&dims, &W, (int)ts.size(), ts.data(), rescale, normalise ? norms.data_ptr<float>() : nullptr, want_smart ? smart.data_ptr<float>() : nullptr,
-                                  elem.data_ptr<float>(), scan.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), current_stream(*first)), fn);
+    if (want_smart) smart = torch::empty({pass.total}, opt);
+    check_status(sg2_bilevel_pass_finish(&pass.dims, &pass.W, (int)pass.ts.size(), pass.ts.data(), rescale, normalise ? norms.data_ptr<float>() : nullptr,
+                                         want_smart ? smart.data_ptr<float>() : nullptr, elem.data_ptr<float>(), scan.data_ptr<float>(),
+                                         pass.ws.data_ptr(), (size_t)pass.ws.numel(), current_stream(pass.ws)), fn);
     return py::make_tuple(want_smart ? py::cast(smart) : py::object(py::none()), elem, scan);
 }
 
@@ -661,7 +684,9 @@ void bind_group_steps(pybind11::module_& m) {
     m.def("supergrok15_flat_step", &supergrok15_flat_step);
     m.def("supergrok11_flat_step", &supergrok11_flat_step);
     m.def("supergrok2_flat_step", &supergrok2_flat_step);
-    m.def("supergrok2_bilevel_pass", &supergrok2_bilevel_pass);
+    py::class_<BilevelPass>(m, "BilevelPass");
+    m.def("supergrok2_bilevel_begin", &supergrok2_bilevel_begin);
+    m.def("supergrok2_bilevel_finish", &supergrok2_bilevel_finish);
     m.def("add_flat_grads", &add_flat_grads);
     m.def("recycle_draws", &recycle_draws);
 }

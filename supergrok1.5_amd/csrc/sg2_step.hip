@@ -580,6 +580,26 @@ int run_step(const SgDims* dims, const Sg2Weights* weights, int num_tensors, con
     return 0;
 }
 
+void remember_forward(const void* workspace, const Plan& pl, int num_tensors) {
+    std::lock_guard<std::mutex> lock(g_bilevel_mutex);
+    // bounded memory: a workspace whose forward call is the oldest on record is forgotten first (a live pair of
+    // forward and backward calls is only ever separated by the calls of other workspaces still in use)
+    while (g_bilevel_records.size() >= MAX_BILEVEL_RECORDS && g_bilevel_records.find(workspace) == g_bilevel_records.end()) {
+        auto oldest = g_bilevel_records.begin();
+        for (auto it = g_bilevel_records.begin(); it != g_bilevel_records.end(); ++it)
+            if (it->second.seq < oldest->second.seq) oldest = it;
+        g_bilevel_records.erase(oldest);
+    }
+    g_bilevel_records[workspace] = BilevelRecord{pl.total > 0 ? pl.chunk_len : 0, pl.total > 0 ? pl.window : 0, num_tensors, pl.total, ++g_bilevel_seq};
+}
+int recall_forward(const void* workspace, const char* fn, BilevelRecord* rec) {
+    std::lock_guard<std::mutex> lock(g_bilevel_mutex);
+    const auto it = g_bilevel_records.find(workspace);
+    if (it == g_bilevel_records.end()) return sg::fail("%s: no forward call has been made on this workspace", fn);
+    *rec = it->second;
+    return 0;
+}
+
 // Scratch of sg2_batched_step_static: one array per GPU the library runs on, held until the process ends.  The
 // array's name is only a handle in host code; its device address is looked up once per device.
 static __device__ __align__(256) unsigned char scratch[SG2_STATIC_SCRATCH_BYTES];
@@ -691,18 +711,7 @@ int sg2_bilevel_forward_ex(const SgDims* dims, const Sg2Weights* weights, int nu
     Layout L;
     const Sg2Scalars none = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if (build_plan(dims, weights, num_tensors, tensors, &none, workspace, workspace_bytes, false, true, false, st, &pl, &L)) return 1;
-    {
-        std::lock_guard<std::mutex> lock(g_bilevel_mutex);
-        // bounded memory: a workspace whose forward call is the oldest on record is forgotten first (a live pair of
-        // forward and backward calls is only ever separated by the calls of other workspaces still in use)
-        while (g_bilevel_records.size() >= MAX_BILEVEL_RECORDS && g_bilevel_records.find(workspace) == g_bilevel_records.end()) {
-            auto oldest = g_bilevel_records.begin();
-            for (auto it = g_bilevel_records.begin(); it != g_bilevel_records.end(); ++it)
-                if (it->second.seq < oldest->second.seq) oldest = it;
-            g_bilevel_records.erase(oldest);
-        }
-        g_bilevel_records[workspace] = BilevelRecord{pl.total > 0 ? pl.chunk_len : 0, pl.total > 0 ? pl.window : 0, num_tensors, pl.total, ++g_bilevel_seq};
-    }
+    remember_forward(workspace, pl, num_tensors);
     if (pl.total == 0) return 0;
     if (extra && !scan_exact(dims, pl.geo))
         return sg::fail("sg2_bilevel_forward_ex: the extra outputs are laid out for d_model=%d d_state=%d d_inner=%d only", GeoDefault::DM,
@@ -732,13 +741,7 @@ int sg2_bilevel_backward_ex(const SgDims* dims, const Sg2Weights* weights, int n
     const Sg2Scalars none = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if (!grads_out) return sg::fail("grads_out is NULL");
     BilevelRecord rec;
-    {
-        std::lock_guard<std::mutex> lock(g_bilevel_mutex);
-        const auto it = g_bilevel_records.find(workspace);
-        if (it == g_bilevel_records.end())
-            return sg::fail("sg2_bilevel_backward: no forward call has been made on this workspace");
-        rec = it->second;
-    }
+    if (recall_forward(workspace, "sg2_bilevel_backward", &rec)) return 1;
     // the layout of the forward call (its chunk length and window, whatever the settings are now): sorted keys /
     // payloads / sharpness, the sharpness flags, coefficients and tile states are still in place
     if (build_plan(dims, weights, num_tensors, tensors, &none, workspace, workspace_bytes, false, true, true, st, &pl, &L, rec.chunk_len,
@@ -765,33 +768,52 @@ size_t sg2_bilevel_pass_workspace_bytes(const SgDims* dims, int num_tensors, con
     return L.bytes;
 }
 
-int sg2_bilevel_pass(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, float rescale, const float* norms,
-                     float* smart_out, float* elem_grads_out, float* scan_grads_out, void* workspace, size_t workspace_bytes, void* stream) {
+int sg2_bilevel_pass_begin(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, void* workspace,
+                           size_t workspace_bytes, void* stream) {
     using namespace sg2;
     hipStream_t st = (hipStream_t)stream;
     Plan pl;
     Layout L;
-    const Sg2Scalars none = {rescale, 0.0f, 0.0f, 0.0f, 0.0f};
-    if (!elem_grads_out || !scan_grads_out) return sg::fail("NULL argument");
-    if (num_tensors <= 0 || !tensors) return sg::fail("sg2_bilevel_pass: no tensors");
+    const Sg2Scalars none = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    if (num_tensors <= 0 || !tensors) return sg::fail("sg2_bilevel_pass_begin: no tensors");
     const int geo = geo_of(dims);
     if (geo < 0) return 1;
     SgDims routing = *dims;
     routing.expert_hidden = EH;          // narrower experts are read at their own width
     if (check_dims(&routing, true)) return 1;
     if (!scan_exact(dims, geo) || dims->expert_hidden > EH)
-        return sg::fail("sg2_bilevel_pass is built for d_model=%d d_state=%d d_inner=%d and expert_hidden up to %d", GeoDefault::DM, GeoDefault::DS,
-                        GeoDefault::DI, EH);
-    for (int i = 0; i < num_tensors; i++)
+        return sg::fail("the bilevel pass in two calls is built for d_model=%d d_state=%d d_inner=%d and expert_hidden up to %d", GeoDefault::DM,
+                        GeoDefault::DS, GeoDefault::DI, EH);
+    if (build_plan(dims, weights, num_tensors, tensors, &none, workspace, workspace_bytes, false, true, false, st, &pl, &L, 0, -1, true)) return 1;
+    if (pl.total == 0) return sg::fail("sg2_bilevel_pass_begin: no elements");
+    remember_forward(workspace, pl, num_tensors);
+    if (launch_expert_tables(pl, dims->expert_hidden, static_cast<unsigned char*>(workspace) + L.off_elem, st)) return 1;
+    if (launch_sort(pl, nullptr, st)) return 1;
+    return launch_scan(pl, st);
+}
+
+int sg2_bilevel_pass_finish(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, float rescale,
+                            const float* norms, float* smart_out, float* elem_grads_out, float* scan_grads_out, void* workspace,
+                            size_t workspace_bytes, void* stream) {
+    using namespace sg2;
+    hipStream_t st = (hipStream_t)stream;
+    Plan pl;
+    Layout L;
+    const Sg2Scalars none = {rescale, 0.0f, 0.0f, 0.0f, 0.0f};
+    if (!elem_grads_out || !scan_grads_out) return sg::fail("NULL argument");
+    BilevelRecord rec;
+    if (recall_forward(workspace, "sg2_bilevel_pass_finish", &rec)) return 1;
+    for (int i = 0; i < num_tensors && tensors; i++)
         if (tensors[i].numel > 0 && (!tensors[i].gru_state || !tensors[i].param || ((uintptr_t)tensors[i].gru_state & 15u) != 0))
             return sg::fail("tensor %d: gru_state (16-byte aligned) and param (the cotangent) are needed", i);
-    if (build_plan(dims, weights, num_tensors, tensors, &none, workspace, workspace_bytes, false, true, false, st, &pl, &L, 0, -1, true)) return 1;
-    if (pl.total == 0) return sg::fail("sg2_bilevel_pass: no elements");
+    if (build_plan(dims, weights, num_tensors, tensors, &none, workspace, workspace_bytes, false, true, true, st, &pl, &L, rec.chunk_len,
+                   rec.window, true))
+        return 1;
+    if (num_tensors != rec.P || pl.total != rec.total)
+        return sg::fail("sg2_bilevel_pass_finish: %d tensors / %d elements, but the first call on this workspace had %d / %d", num_tensors, pl.total,
+                        rec.P, rec.total);
     unsigned char* ws = static_cast<unsigned char*>(workspace);
     float* d_ctx = reinterpret_cast<float*>(ws + L.off_dctx);
-    if (launch_expert_tables(pl, dims->expert_hidden, ws + L.off_elem, st)) return 1;
-    if (launch_sort(pl, nullptr, st)) return 1;
-    if (launch_scan(pl, st)) return 1;
     if (launch_bilevel_elem(pl, norms, dims->expert_hidden, smart_out, d_ctx, elem_grads_out, ws + L.off_elem, st)) return 1;
     return launch_bilevel_backward(pl, d_ctx, nullptr, nullptr, nullptr, scan_grads_out, st);
 }

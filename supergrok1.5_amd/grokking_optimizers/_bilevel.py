@@ -227,16 +227,27 @@ def elem_parameters(mn):
     return out + [mn.expert_W1, mn.expert_b1, mn.expert_W2, mn.expert_b2]
 
 
-def accumulate_meta_gradients(mn, grads, sharps, gru_states, mamba_fwd, mamba_bwd, cotangents, validation=False, want_smart=True):
+def begin_pass(mn, grads, sharps, gru_states, mamba_fwd, mamba_bwd, exact_sharpness=False):
+    """The part of accumulate_meta_gradients that needs no cotangents (sort and scan: sg2_bilevel_pass_begin), enqueued on
+    the current stream: what its `begun` takes, or None for nets and tensors that the pass is not built for."""
+    if not (_pass_fits(mn) and all(m is not None for m in mamba_fwd) and all(m is not None for m in mamba_bwd)):
+        return None
+    return _ops.supergrok2_bilevel_begin(grads, sharps, gru_states, mamba_fwd, mamba_bwd, mn.flat_weights(), exact_sharpness,
+                                         list(meta_dims(mn).values()))
+
+
+def accumulate_meta_gradients(mn, grads, sharps, gru_states, mamba_fwd, mamba_bwd, cotangents, validation=False, want_smart=True, begun=None):
     """Adds the gradient of  sum_p <smart_grad_p, cotangent_p>  with respect to every parameter of `mn` to its
     .grad, for a list of tensors at once, all in HIP: scan forward, per-element forward and backward, scan adjoint
-    (sg2_bilevel_pass; for nets smaller than its sizes sg2_bilevel_forward, sg2_bilevel_elem and sg2_bilevel_backward on
-    packed copies).  validation: `cotangents` are validation gradients v and the cotangent is -v / |v| (-v where |v| is
-    0); sharpness is then used at its own precision whatever the gradients' type.  Returns the smart gradients (flat,
-    packed), or None without want_smart where they cost extra."""
-    if _pass_fits(mn) and None not in mamba_fwd and None not in mamba_bwd:
-        got = _ops.supergrok2_bilevel_pass(grads, sharps, gru_states, mamba_fwd, mamba_bwd, cotangents, mn.flat_weights(), float(mn.rescale),
-                                           validation, validation, want_smart, list(meta_dims(mn).values()))
+    (sg2_bilevel_pass_begin / _finish; for nets smaller than their sizes sg2_bilevel_forward, sg2_bilevel_elem and
+    sg2_bilevel_backward on packed copies).  validation: `cotangents` are validation gradients v and the cotangent is
+    -v / |v| (-v where |v| is 0); sharpness is then used at its own precision whatever the gradients' type.  begun: what
+    begin_pass returned for the same tensors and weights.  Returns the smart gradients (flat, packed), or None without
+    want_smart where they cost extra."""
+    if begun is None:
+        begun = begin_pass(mn, grads, sharps, gru_states, mamba_fwd, mamba_bwd, validation)
+    if begun is not None:
+        got = _ops.supergrok2_bilevel_finish(begun, cotangents, float(mn.rescale), validation, want_smart)
         if got is not None:
             _ops.add_flat_grads(elem_parameters(mn), got[1])
             _ops.add_flat_grads(scan_parameters(mn), got[2])

@@ -200,6 +200,11 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
                   if n in saved and id(p) in self._param_to_idx and saved[n].numel() > 0]
         if not picked:
             return 0.0
+        grads = [saved[n].detach() for n, _, _ in picked]
+        state = [[kept[i] for _, _, i in picked] for kept in (self._flat_sharpness, self._flat_gru_states, self._flat_mamba_fwd_states,
+                                                              self._flat_mamba_bwd_states)]
+        # sort and scan need the training gradients only: the GPU has them to do while the validation pass is being enqueued
+        begun = _bilevel.begin_pass(self.meta_net, grads, *state, exact_sharpness=True)
         for _, p in named:
             p.grad = None              # the training gradients step aside, whatever zero_grad would do to them
         model.zero_grad()
@@ -207,13 +212,12 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
             val_loss = criterion(model(val_x), val_y)
             val_loss.backward()
         meta_optimizer.zero_grad()
-        picked = [(saved[n].detach(), p.grad.detach(), i) for n, p, i in picked if p.grad is not None]
-        if picked:
-            at = [i for _, _, i in picked]
-            state = [[kept[i] for i in at] for kept in (self._flat_sharpness, self._flat_gru_states, self._flat_mamba_fwd_states,
-                                                        self._flat_mamba_bwd_states)]
-            _bilevel.accumulate_meta_gradients(self.meta_net, [g for g, _, _ in picked], *state, [v for _, v, _ in picked],
-                                               validation=True, want_smart=False)
+        reached = [k for k, (_, p, _) in enumerate(picked) if p.grad is not None]
+        if len(reached) < len(picked):           # the validation loss does not depend on all of them
+            begun, grads, state = None, [grads[k] for k in reached], [[kept[k] for k in reached] for kept in state]
+        if reached:
+            _bilevel.accumulate_meta_gradients(self.meta_net, grads, *state, [picked[k][1].grad.detach() for k in reached], validation=True,
+                                               want_smart=False, begun=begun)
             meta_optimizer.step()
             self._weights_dirty = True
         for n, p in named:
