@@ -22,8 +22,10 @@
 // operand by other workgroups).  A tall parameter enters and leaves the wide
 // orientation in the momentum and update kernels, which transpose 64x64 tiles
 // through LDS.
-// Work buffers are zero-padded to multiples of 256 so the GEMM needs no edge
+// Work buffers are padded with zeros to multiples of 256 (written by the momentum kernel) so the GEMM needs no edge
 // handling (zero rows/columns stay zero through the iteration).
+// A call whose matrices all fit the LDS of a CU (k_newton_schulz) takes one launch for the whole iteration instead of
+// three products a step.
 //
 // GEMM: 256x256 output tile per 512-thread workgroup, 8 waves as 2x4, each
 // wave 128x64 = 4x2 MFMA 32x32x16 bf16 tiles (128 fp32 accumulators per
@@ -36,7 +38,9 @@
 // from L2; the symmetric products (G and G*G) compute only the tiles on or above
 // the diagonal.  Tile index -> XCD-contiguous order so that the workgroups
 // sharing operand panels share an L2.
+#include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "sg_common.hpp"
@@ -545,6 +549,159 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int i
     }
 }
 
+// ---- all iterations of one matrix in one workgroup: Y [mp x np] (mp 64 or 128) and G, then H in its place, stay in LDS.
+// Eight waves.  G and G G: 32x32 tiles, one row of tiles to a pair of waves; apply: strips of 32 columns, whose Y' replaces
+// their Y (a strip is read by its own wave only).  Same roundings as the GEMM path: G, H and Y are bf16 between the
+// products, the first step carries 1/norm^2 and 1/norm.
+// Rows lie 16-byte chunk by chunk, chunk c of row r at c ^ swizzle(r): consecutive rows' chunks fall on different banks.
+// Bound by LDS operand fetches (1.25 to 1.5 per MFMA) and the barriers between the products: 50 us for five iterations of
+// 128 x 512, the largest, where fifteen launches of k_gemm_nt took 180.
+constexpr int NS_THREADS = 512;
+constexpr int NS_Y_ELEMS = 128 * 512;          // Y: 128 KB ...
+constexpr int NS_LDS_BYTES = 2 * (NS_Y_ELEMS + 128 * 128);      // ... and G: 32 KB, all of a CU's 160 KB
+inline bool fits_lds(int mp, int np) { return mp <= 128 && mp * np <= NS_Y_ELEMS; }
+__device__ __forceinline__ int ns_swizzle(int row, int width) { return (width & 64) ? (row >> 1) & 7 : row & 15; }
+
+template <int MT>       // mp / 32
+__device__ __forceinline__ void newton_schulz(const Mat& M, float inv, int steps, bf16_t* __restrict__ sY, bf16_t* __restrict__ sG) {
+    constexpr int mp = 32 * MT, TPW = MT == 4 ? 2 : 1;       // tiles of a row of tiles per wave
+    const int np = M.np, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r32 = lane & 31, kh = lane >> 5;
+    {
+        const int chunks = np / 8;
+        const u32x4* __restrict__ src = reinterpret_cast<const u32x4*>(M.Y);
+        for (int i = tid; i < mp * chunks; i += NS_THREADS) {
+            const int r = i / chunks, c = i % chunks;
+            *reinterpret_cast<u32x4*>(sY + (size_t)r * np + (c ^ ns_swizzle(r, np)) * 8) = *(gvec_p)(src + i);
+        }
+    }
+    __syncthreads();
+    // eight consecutive k of row r of a [rows x width] array
+    auto chunk = [](const bf16_t* s, int width, int r, int c) {
+        return *reinterpret_cast<const bf16x8*>(s + (size_t)r * width + (c ^ ns_swizzle(r, width)) * 8);
+    };
+    // four consecutive columns c .. c + 3 (c a multiple of 4) of row r
+    auto at = [](int width, int r, int c) { return (size_t)r * width + (((c >> 3) ^ ns_swizzle(r, width)) << 3) + (c & 4); };
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    const bool active = wave < MT * MT / TPW;
+    const int rt = active ? wave / (MT / TPW) : 0, ct = active ? (wave % (MT / TPW)) * TPW : 0;
+    for (int it = 0; it < steps; it++) {
+        const float g_scale = it == 0 ? inv * inv : 1.0f, y_scale = it == 0 ? inv : 1.0f;
+        f32x16 acc[TPW];
+        // the wave's tiles of S S^T, S [mp x width]
+        auto gram = [&](const bf16_t* s, int width) {
+#pragma unroll
+            for (int j = 0; j < TPW; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[j][e] = 0.0f;
+            // two k steps at a time (width is a multiple of 64), the operands of the next two on their way
+            const int nk = width / 16;
+            bf16x8 a[2], b[2][TPW];
+            auto fetch = [&](int k) {
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    a[u] = chunk(s, width, 32 * rt + r32, 2 * (k + u) + kh);
+#pragma unroll
+                    for (int j = 0; j < TPW; j++) b[u][j] = chunk(s, width, 32 * (ct + j) + r32, 2 * (k + u) + kh);
+                }
+            };
+            fetch(0);
+#pragma unroll 1
+            for (int k = 0; k < nk; k += 2) {
+                bf16x8 a0[2], b0[2][TPW];
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    a0[u] = a[u];
+#pragma unroll
+                    for (int j = 0; j < TPW; j++) b0[u][j] = b[u][j];
+                }
+                fetch(min(k + 2, nk - 2));
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int j = 0; j < TPW; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b0[u][j], a0[u], acc[j], 0, 0, 0);
+            }
+        };
+        // (the operands change places, so that a lane holds, of its row of the result, four times four consecutive columns)
+        auto put = [&](auto value) {
+#pragma unroll
+            for (int j = 0; j < TPW; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int c = 32 * (ct + j) + 8 * q + 4 * kh;
+                    u32x2* p = reinterpret_cast<u32x2*>(sG + at(mp, 32 * rt + r32, c));
+                    *p = value(j, q, c, p);
+                }
+        };
+        if (active) {
+            gram(sY, np);
+            put([&](int j, int q, int, const u32x2*) {
+                return u32x2{bf16r2(acc[j][4 * q] * g_scale, acc[j][4 * q + 1] * g_scale), bf16r2(acc[j][4 * q + 2] * g_scale, acc[j][4 * q + 3] * g_scale)};
+            });
+        }
+        __syncthreads();
+        if (active) gram(sG, mp);            // G is symmetric
+        __syncthreads();
+        if (active)
+            put([&](int j, int q, int c, const u32x2* p) {       // H = a I + b G + c G G in place of G
+                const u32x2 w = *p;
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float x = sg_i2f((int32_t)((e & 1) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16)));
+                    v[e] = sg_fma(NS_C, acc[j][4 * q + e], NS_B * x) + (32 * rt + r32 == c + e ? NS_A : 0.0f);
+                }
+                return u32x2{bf16r2(v[0], v[1]), bf16r2(v[2], v[3])};
+            });
+        __syncthreads();
+        // transposing read (see k_gemm_nt): lane -> k row 8 (lane / 32) + (lane % 16) / 4, columns 16 ((lane / 16) % 2) + 4 (lane % 4)
+        for (int strip = wave; strip < np / 32; strip += NS_THREADS / 64) {
+            f32x16 y[MT];
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) y[i][e] = 0.0f;
+            const int col = 32 * strip + 16 * ((lane >> 4) & 1) + 4 * (lane & 3), row0 = 8 * kh + ((lane & 15) >> 2);
+#pragma unroll 2
+            for (int k = 0; k < mp / 16; k++) {
+                const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_p)(sY + at(np, 16 * k + row0, col)));
+                const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_p)(sY + at(np, 16 * k + row0 + 4, col)));
+                const bf16x8 b = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+                    y[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, chunk(sG, mp, 32 * i + r32, 2 * k + kh), y[i], 0, 0, 0);
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    *reinterpret_cast<u32x2*>(sY + at(np, 32 * i + r32, 32 * strip + 8 * q + 4 * kh)) =
+                        u32x2{bf16r2(y[i][4 * q] * y_scale, y[i][4 * q + 1] * y_scale), bf16r2(y[i][4 * q + 2] * y_scale, y[i][4 * q + 3] * y_scale)};
+        }
+        __syncthreads();
+    }
+    const int chunks = np / 8;
+    u32x4* dst = reinterpret_cast<u32x4*>(steps & 1 ? M.Y2 : M.Y);
+    for (int i = tid; i < mp * chunks; i += NS_THREADS) {
+        const int r = i / chunks, c = i % chunks;
+        *(gvec_w)(dst + i) = *reinterpret_cast<const u32x4*>(sY + (size_t)r * np + (c ^ ns_swizzle(r, np)) * 8);
+    }
+}
+
+__global__ __launch_bounds__(NS_THREADS) void k_newton_schulz(Batch B, int steps) {
+    extern __shared__ __attribute__((aligned(16))) bf16_t smem[];
+    const int mi = blockIdx.x;
+    const Mat& M = B.mats[mi];
+    // the norm, from the momentum kernel's tiles (a matrix has at most 16 of them)
+    double part = 0.0;
+    for (int k = B.ttile_prefix[mi]; k < B.ttile_prefix[mi + 1]; k++) part += B.partials[k];
+    const float inv = 1.0f / ((float)sqrt(part) + 1e-7f);
+    bf16_t* const sG = smem + M.mp * M.np;
+    if (M.mp == 128) newton_schulz<4>(M, inv, steps, smem, sG);
+    else newton_schulz<2>(M, inv, steps, smem, sG);
+}
+
 // p = (p - 0.2*lr*X) * (1 - lr*wd).  X lies in the wide orientation; one 64x64 tile of the parameter's own
 // orientation per workgroup (the grid of k_momentum), a tall parameter's tile of X is transposed through LDS.
 // scale_inv: no iteration ran, X is still the unnormalised momentum
@@ -611,17 +768,14 @@ __global__ __launch_bounds__(256) void k_update(Batch B, float lr, float decay, 
     }
 }
 
-__global__ __launch_bounds__(256) void k_zero(uint4* p, size_t n16) {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) p[i] = make_uint4(0, 0, 0, 0);
-}
-
 inline int round_up(int x, int a) { return (x + a - 1) / a * a; }
 
 struct Layout {
     int P;
     std::vector<Mat> mats;
+    bool small;                    // every matrix fits k_newton_schulz
     std::vector<int> pre_g[3], pre_t;
-    size_t off_mats, off_pre_g[3], off_pre_t, off_partials, off_inv, off_buffers, bytes;
+    size_t off_mats, off_pre, off_partials, off_inv, bytes;
 };
 
 int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
@@ -632,8 +786,16 @@ int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
     size_t o = 0;
     auto take = [&](size_t b) { size_t r = o; o = sg::align_up(o + b, 256); return r; };
     L->off_mats = take(sizeof(Mat) * (size_t)P);
-    for (int k = 0; k < 3; k++) L->off_pre_g[k] = take(sizeof(int) * (size_t)(P + 1));
-    L->off_pre_t = take(sizeof(int) * (size_t)(P + 1));
+    L->off_pre = L->off_mats + sizeof(Mat) * (size_t)P;      // right behind the records: one upload
+    o = sg::align_up(L->off_pre + 4 * sizeof(int) * (size_t)(P + 1), 256);
+    // One workgroup per matrix does its five iterations in 50 us at most (128 x 512), fifteen products of small matrices take
+    // ten to fourteen each; next to matrices that need the products anyway the small ones come along in their launches.
+    L->small = true;
+    for (int i = 0; i < P; i++) {
+        const int64_t m = std::min(in[i].rows, in[i].cols), n = std::max(in[i].rows, in[i].cols);
+        L->small = L->small && m > 0 && m <= 128 && n <= NS_Y_ELEMS && fits_lds(round_up((int)m, 64), round_up((int)n, 64));
+    }
+    const int pad = L->small ? 64 : BT;
     for (int i = 0; i < P; i++) {
         const SgMuonMatrix& s = in[i];
         if (s.rows <= 0 || s.cols <= 0 || s.rows * s.cols > 0x7fffffff) return sg::fail("matrix %d: bad shape %lld x %lld", i, (long long)s.rows, (long long)s.cols);
@@ -644,23 +806,25 @@ int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
         M.wide = s.rows <= s.cols;
         M.vec8 = (s.cols % 8 == 0) && ((((uintptr_t)s.param | (uintptr_t)s.grad | (uintptr_t)s.buf) & 15u) == 0);
         M.m = (int)std::min(s.rows, s.cols); M.n = (int)std::max(s.rows, s.cols);
-        M.mp = round_up(M.m, BT); M.np = round_up(M.n, BT);
-        const int nt = M.mp / BT, tri = nt * (nt + 1) / 2;      // symmetric products: tiles on or above the diagonal
+        M.mp = round_up(M.m, pad); M.np = round_up(M.n, pad);
+
+        const int nt = L->small ? 0 : M.mp / BT, tri = nt * (nt + 1) / 2;      // symmetric products: tiles on or above the diagonal
         L->pre_g[EPI_GRAM][i + 1] = L->pre_g[EPI_GRAM][i] + tri;
         L->pre_g[EPI_POLY][i + 1] = L->pre_g[EPI_POLY][i] + tri;
-        L->pre_g[EPI_APPLY][i + 1] = L->pre_g[EPI_APPLY][i] + (M.mp / BT) * (M.np / BT);
+        L->pre_g[EPI_APPLY][i + 1] = L->pre_g[EPI_APPLY][i] + nt * (M.np / BT);
         L->pre_t[i + 1] = L->pre_t[i] + (M.mp / 64) * (M.np / 64);
     }
     int64_t ttiles = 0;
     for (int i = 0; i < P; i++) ttiles += (int64_t)(L->mats[i].mp / 64) * (L->mats[i].np / 64);
     L->off_partials = take(sizeof(double) * (size_t)(ttiles + 1));
     L->off_inv = take(sizeof(float) * (size_t)P);
-    L->off_buffers = o;
     for (int i = 0; i < P; i++) {
         Mat& M = L->mats[i];
         // offsets for now; turned into pointers once the workspace base is known
         M.Y = (bf16_t*)take(2 * (size_t)M.mp * M.np);
         M.Y2 = (bf16_t*)take(2 * (size_t)M.mp * M.np);
+        M.G = M.H = nullptr;
+        if (L->small) continue;
         M.G = (bf16_t*)take(2 * (size_t)M.mp * M.mp);
         M.H = (bf16_t*)take(2 * (size_t)M.mp * M.mp);
     }
@@ -699,15 +863,21 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
         M.Y = (bf16_t*)(ws + (size_t)M.Y); M.Y2 = (bf16_t*)(ws + (size_t)M.Y2);
         M.G = (bf16_t*)(ws + (size_t)M.G); M.H = (bf16_t*)(ws + (size_t)M.H);
     }
-    // per-call tables: through kernel arguments (no host-to-device copy, nothing blocks the host)
-    if (sg::upload_words(ws + L.off_mats, L.mats.data(), sizeof(Mat) * (size_t)P, st)) return 1;
-    for (int k = 0; k < 3; k++)
-        if (sg::upload_words(ws + L.off_pre_g[k], L.pre_g[k].data(), sizeof(int) * (size_t)(P + 1), st)) return 1;
-    if (sg::upload_words(ws + L.off_pre_t, L.pre_t.data(), sizeof(int) * (size_t)(P + 1), st)) return 1;
+    // per-call tables: through kernel arguments (no host-to-device copy, nothing blocks the host), records and tile prefixes
+    // one after the other
     Batch B;
+    {
+        std::vector<uint32_t> w((sizeof(Mat) * (size_t)P) / 4 + 4 * (size_t)(P + 1));
+        memcpy(w.data(), L.mats.data(), sizeof(Mat) * (size_t)P);
+        uint32_t* pre = w.data() + sizeof(Mat) * (size_t)P / 4;
+        static_assert(sizeof(Mat) % 4 == 0, "records in words");
+        for (int k = 0; k < 4; k++) memcpy(pre + (size_t)k * (P + 1), (k < 3 ? L.pre_g[k] : L.pre_t).data(), sizeof(int) * (size_t)(P + 1));
+        if (sg::upload_words(ws + L.off_mats, w.data(), 4 * w.size(), st)) return 1;
+    }
     B.mats = reinterpret_cast<const Mat*>(ws + L.off_mats);
-    for (int k = 0; k < 3; k++) B.gtile_prefix[k] = reinterpret_cast<const int*>(ws + L.off_pre_g[k]);
-    B.ttile_prefix = reinterpret_cast<const int*>(ws + L.off_pre_t);
+    const int* pre = reinterpret_cast<const int*>(ws + L.off_pre);
+    for (int k = 0; k < 3; k++) B.gtile_prefix[k] = pre + (size_t)k * (P + 1);
+    B.ttile_prefix = pre + 3 * (size_t)(P + 1);
     B.P = P;
     for (int k = 0; k < 3; k++) B.gtiles[k] = L.pre_g[k][P];
     B.ttiles = L.pre_t[P];
@@ -724,23 +894,21 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
             SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_nt<EPI_GRAM>), hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS_BYTES));
             SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_nt<EPI_POLY>), hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS_BYTES));
             SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_nt<EPI_APPLY>), hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS_BYTES));
+            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_newton_schulz), hipFuncAttributeMaxDynamicSharedMemorySize, NS_LDS_BYTES));
             raised[dev] = true;
         }
     }
 
-    // padded work buffers start from zero (a fill kernel, not a memset node, so the call stays capturable)
-    bool any_pad = false;
-    for (const auto& M : L.mats) any_pad = any_pad || M.mp != M.m || M.np != M.n;
-    if (any_pad) {
-        const size_t n16 = (L.bytes - L.off_buffers) / 16;
-        hipLaunchKernelGGL(k_zero, dim3((unsigned)std::min<size_t>((n16 + 255) / 256, 65535)), dim3(256), 0, st,
-                           reinterpret_cast<uint4*>(ws + L.off_buffers), n16);
-    }
-
     hipLaunchKernelGGL(k_momentum, dim3(B.ttiles), dim3(256), 0, st, B, momentum);
-    hipLaunchKernelGGL(k_norm, dim3(P), dim3(256), 0, st, B);
+    if (!L.small || ns_steps == 0) hipLaunchKernelGGL(k_norm, dim3(P), dim3(256), 0, st, B);
     SG_LAUNCH_CHECK("muon prologue");
-    for (int it = 0; it < ns_steps; it++) {
+    if (L.small && ns_steps > 0) {
+        size_t lds = 0;
+        for (const auto& M : L.mats) lds = std::max(lds, 2 * ((size_t)M.mp * M.np + (size_t)M.mp * M.mp));
+        hipLaunchKernelGGL(k_newton_schulz, dim3(P), dim3(NS_THREADS), lds, st, B, ns_steps);
+        SG_LAUNCH_CHECK("k_newton_schulz");
+    }
+    for (int it = 0; it < (L.small ? 0 : ns_steps); it++) {
         const int sel = it & 1, last = it == 0 ? 2 : 0;     // iter_flags
         hipLaunchKernelGGL(k_gemm_nt<EPI_GRAM>, dim3(B.gtiles[EPI_GRAM]), dim3(GTHREADS), GEMM_LDS_BYTES, st, B, sel, last);
         hipLaunchKernelGGL(k_gemm_nt<EPI_POLY>, dim3(B.gtiles[EPI_POLY]), dim3(GTHREADS), GEMM_LDS_BYTES, st, B, sel, last);
