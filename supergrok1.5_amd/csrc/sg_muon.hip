@@ -13,7 +13,7 @@
 // (for a tall parameter X this is X^T X and X (bG + cG^2): the reference's
 // X X^T form re-associated, 6 m^2 n instead of 6 n^2 m flops per iteration).
 // The Gram and polynomial products are "NT" GEMMs (both operands K-contiguous).
-// The apply step is an "NN" one: its B operand is Y itself, whose K axis is
+// The apply step is (on 256x256 tiles) an "NN" one: its B operand is Y itself, whose K axis is
 // the slow one.  Its tiles are staged in LDS as they lie in memory
 // ([k][n], n contiguous) and the MFMA operand (8 consecutive k per lane) is
 // fetched with gfx950's transposing LDS read (ds_read_b64_tr_b16), so no
@@ -22,10 +22,10 @@
 // operand by other workgroups).  A tall parameter enters and leaves the wide
 // orientation in the momentum and update kernels, which transpose 64x64 tiles
 // through LDS.
-// Work buffers are padded with zeros to multiples of 256 (written by the momentum kernel) so the GEMM needs no edge
-// handling (zero rows/columns stay zero through the iteration).
+// Work buffers are padded with zeros to multiples of 256 (64 where no product takes 256x256 tiles), written by the momentum
+// kernel, so the products need no edge handling (zero rows/columns stay zero through the iteration).
 // A call whose matrices all fit the LDS of a CU (k_newton_schulz) takes one launch for the whole iteration instead of
-// three products a step.
+// three products a step; products that would leave most of the chip idle go to 64x64 tiles (k_gemm_64, choose_tiles).
 //
 // GEMM: 256x256 output tile per 512-thread workgroup, 8 waves as 2x4, each
 // wave 128x64 = 4x2 MFMA 32x32x16 bf16 tiles (128 fp32 accumulators per
@@ -68,6 +68,7 @@ struct Mat {
     const void* grad;
     float* buf;
     bf16_t *Y, *Y2, *G, *H;       // [mp x np] twice (an iteration reads one and writes the other), [mp x mp], [mp x mp]
+    bf16_t *T, *T2;                // the transposes of Y and Y2 [np x mp], or NULL (kept for k_gemm_64's apply step)
     int rows, cols, dtype;
     int m, n, mp, np;              // min / max dim and their padded sizes
     int wide;                      // rows <= cols
@@ -141,12 +142,12 @@ __global__ __launch_bounds__(256) void k_momentum(Batch B, float momentum) {
     __shared__ double sm[4];
     const int mi = sg::upper_seg(B.ttile_prefix, B.P, blockIdx.x);
     const Mat& M = B.mats[mi];
-    bf16_t* own = M.Y;                            // wide: [R x C] in the parameter's orientation, padded
-    bf16_t* other = M.Y;                          // tall: [C x R]
+    bf16_t* own = M.wide ? M.Y : M.T;             // [R x C] in the parameter's orientation, padded
+    bf16_t* other = M.wide ? M.T : M.Y;           // [C x R]
     const int R = M.wide ? M.mp : M.np, C = M.wide ? M.np : M.mp;
     const int tile = (int)blockIdx.x - B.ttile_prefix[mi];
     const int tc = C / 64, tr0 = (tile / tc) * 64, tc0 = (tile % tc) * 64;
-    const bool w_own = M.wide, w_other = !M.wide;               // uniform over the workgroup
+    const bool w_own = own != nullptr, w_other = other != nullptr;               // uniform over the workgroup
     const bool full = tr0 + 64 <= M.rows && tc0 + 64 <= M.cols && M.vec8;
     double acc = 0.0;
     if (full) {
@@ -549,6 +550,199 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int i
     }
 }
 
+// ---- the same products on 64x64 output tiles, for calls whose 256x256 tiles leave most of the chip idle
+// Four waves share a tile by splitting K: chunk c of 32 k goes to wave c % 4, which multiplies the whole tile and stages
+// its operands in LDS of its own, one chunk ahead; the four partial tiles are added up through LDS.  So there is no barrier
+// in the K loop and a chain of a quarter of K, and two workgroups fit a CU (one's epilogue under the other's products: eight
+// waves on a tile were 0 to 5 % faster for calls of few tiles and 10 to 40 % slower for the rest; operands straight from
+// memory into registers, 16 bytes a row, took up to twice as long).
+// The apply step reads the transpose T of Y, which its own epilogue (and the momentum kernel) leaves beside Y: with it all
+// three products have both operands K-contiguous.
+// Bound by latency for few tiles (the operands come through memory, where other XCDs wrote them: 5 to 8 us a product, of
+// which 4 are the launch), for many by what a CU gets from L2 (32 flop per byte: 0.6 PFLOP/s).
+// Step over bf16 matrices, with k_gemm_nt alone and with choose_tiles between the two: 1 of 200 x 800 232 -> 112 us,
+// 24 of 64 x 3000 493 -> 180, 1 of 1024 x 1024 410 -> 147, 2 of 1024 x 4096 691 -> 365, 24 of 512 x 2048 642 -> 498.
+constexpr int NT64 = 64;
+constexpr int KS_WAVES = 4, KS_THREADS = 64 * KS_WAVES;
+constexpr int KS_ROW = NT64 + 4;                                                // floats per row of a partial tile
+constexpr int KS_LDS_BYTES = KS_WAVES * NT64 * KS_ROW * 4;                      // 69,632 bytes
+constexpr int KS_STAGE = 2 * NT64 * 32 * 2, KS_WAVE = 2 * KS_STAGE;             // two stages of 8 KB per wave
+static_assert(KS_WAVES * KS_WAVE <= KS_LDS_BYTES, "the waves' stages fit where their partial tiles go");
+
+// y_sel: as for k_gemm_nt; iter_flags: bit 1 = first iteration, bit 2 = last (no product reads T any more)
+template <int EPI>
+__global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, int y_sel, int iter_flags) {
+    constexpr int W = KS_WAVES;
+    extern __shared__ __attribute__((aligned(16))) float part[];
+    __shared__ double sm[W];
+    const int nblk = gridDim.x;
+    int lb = blockIdx.x;
+    if (nblk % 8 == 0) lb = (blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8;      // XCD-contiguous, as in k_gemm_nt
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const sg::cint_p prefix = sg::as_const(Bt.gtile_prefix[EPI]);
+    const int mi = sg::upper_seg(prefix, Bt.P, lb);
+    const Mat& Mt = Bt.mats[mi];
+    int tile = lb - prefix[mi];
+    const bool first = (iter_flags & 2) != 0, last = (iter_flags & 4) != 0;      // uniform over the grid
+
+    const bf16_t *A, *B;
+    bf16_t *C, *CT;         // CT: where the transposed tile goes (NULL: nowhere)
+    int K, ldc, ldct, tm, tn;
+    if (EPI == EPI_APPLY) {
+        A = Mt.H; B = y_sel ? Mt.T2 : Mt.T; C = y_sel ? Mt.Y : Mt.Y2; K = Mt.mp; ldc = Mt.np;
+        CT = last ? nullptr : (y_sel ? Mt.T : Mt.T2); ldct = Mt.mp;
+        const int ntm = Mt.mp / NT64;
+        tm = tile % ntm;
+        tn = tile / ntm;
+    } else {
+        if (EPI == EPI_GRAM) { A = B = y_sel ? Mt.Y2 : Mt.Y; C = Mt.G; K = Mt.np; }
+        else { A = B = Mt.G; C = Mt.H; K = Mt.mp; }
+        ldc = ldct = Mt.mp;
+        const int nt = Mt.mp / NT64;
+        tm = 0;
+        while (tile >= nt - tm) { tile -= nt - tm; tm++; }
+        tn = tm + tile;
+        CT = tm != tn ? C : nullptr;
+    }
+    const int r32 = lane & 31, kh = lane >> 5;
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+    // a wave's stage: {A, B} rows of 32 k, in blocks of 16 rows with the swizzle of k_gemm_nt's [256 x 32 k] tiles
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) float*)part + (uint32_t)wave * KS_WAVE;
+    const unsigned char* const mine = reinterpret_cast<const unsigned char*>(part) + wave * KS_WAVE;
+    const uint32_t lane_off = (uint32_t)(((lane >> 2) * K + (((lane & 3) ^ ((lane >> 4) & 3)) * 8)) * 2);
+    const char* const pa = reinterpret_cast<const char*>(A + (size_t)tm * NT64 * K);            // every operand's row stride is K
+    const char* const pb = reinterpret_cast<const char*>(B + (size_t)tn * NT64 * K);
+    auto fetch = [&](int s, int c) {
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const char* base = (q < 4 ? pa : pb) + ((size_t)(q & 3) * 16 * K + (size_t)c * 32) * 2;
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n"
+                         : : "v"(lane_off), "s"(base), "s"(lds0 + (uint32_t)(s * KS_STAGE + q * 1024)) : "memory");
+        }
+    };
+    // (the operands change places, so that a lane holds, of its row of the result, four times four consecutive columns)
+    auto multiply = [&](int s, auto refill) {
+        bf16x8 a[2][2], b[2][2];
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int r = 32 * i + r32, at = s * KS_STAGE + (r >> 4) * 1024 + (r & 15) * 64 + (((2 * u + kh) ^ ((r >> 2) & 3)) * 16);
+                a[u][i] = *reinterpret_cast<const bf16x8*>(mine + at);
+                b[u][i] = *reinterpret_cast<const bf16x8*>(mine + at + 4096);
+            }
+        refill();
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[u][j], a[u][i], acc[i][j], 0, 0, 0);
+    };
+    const int nk = K / 32;
+    int c = wave, s = 0;
+    if (c < nk) {
+        fetch(0, c);
+        if (c + W < nk) fetch(1, c + W);
+#pragma unroll 1
+        for (; c + W < nk; c += W) {
+            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");            // this chunk has landed, the next may be on its way
+            multiply(s, [&] {
+                if (c + 2 * W < nk) {
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage has been read
+                    fetch(s, c + 2 * W);
+                }
+            });
+            s ^= 1;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        multiply(s, [] {});
+    }
+    __syncthreads();                                            // the partial tiles overlay the stages
+    constexpr int NR = 8 / W;                                   // eight elements each in this many rows of the tile per thread
+    const int row0 = tid >> 3, c8 = tid & 7;
+    u32x4 g[NR];
+    if (EPI == EPI_POLY) {
+#pragma unroll
+        for (int h = 0; h < NR; h++) g[h] = *(gvec_p)(Mt.G + (size_t)(tm * NT64 + row0 + 8 * W * h) * ldc + tn * NT64 + 8 * c8);
+    }
+    // first iteration: Y is the unnormalised momentum, see k_momentum; the norm is added up from its tiles here
+    float scale = 1.0f;
+    if (EPI != EPI_POLY && first) {
+        double sq = 0.0;
+        for (int k = Bt.ttile_prefix[mi] + tid; k < Bt.ttile_prefix[mi + 1]; k += 64 * W) sq += Bt.partials[k];
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) sq += __shfl_down(sq, d, 64);
+        if (lane == 0) sm[wave] = sq;
+    }
+    const int waves = min(nk, W);                               // those that have a partial tile
+    if (wave < waves) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    *reinterpret_cast<f32x4*>(part + (wave * NT64 + 32 * i + r32) * KS_ROW + 32 * j + 8 * q + 4 * kh) =
+                        f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+    }
+    __syncthreads();
+    if (EPI != EPI_POLY && first) {
+        const double tot = (sm[0] + sm[1]) + (sm[2] + sm[3]);
+        const float inv = 1.0f / ((float)sqrt(tot) + 1e-7f);
+        scale = EPI == EPI_GRAM ? inv * inv : inv;
+    }
+    u32x4 out[NR];
+#pragma unroll
+    for (int h = 0; h < NR; h++) {
+        const int row = row0 + 8 * W * h;
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = 0.0f;
+        for (int w = 0; w < waves; w++) {
+            const f32x4* src = reinterpret_cast<const f32x4*>(part + (w * NT64 + row) * KS_ROW + 8 * c8);
+            const f32x4 lo = src[0], hi = src[1];
+#pragma unroll
+            for (int k = 0; k < 4; k++) { v[k] += lo[k]; v[4 + k] += hi[k]; }
+        }
+        if (EPI == EPI_POLY) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const float x = sg_i2f((int32_t)((k & 1) ? (g[h][k >> 1] & 0xffff0000u) : (g[h][k >> 1] << 16)));
+                v[k] = sg_fma(NS_C, v[k], NS_B * x) + (tm == tn && row == 8 * c8 + k ? NS_A : 0.0f);
+            }
+        } else if (first) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] *= scale;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) out[h][k] = bf16r2(v[2 * k], v[2 * k + 1]);
+        *(gvec_w)(C + (size_t)(tm * NT64 + row) * ldc + tn * NT64 + 8 * c8) = out[h];
+    }
+    if (CT) {       // uniform over the workgroup
+        constexpr int TR = NT64 + 8;
+        bf16_t* t = reinterpret_cast<bf16_t*>(part);
+        __syncthreads();                                        // the partial tiles have been read
+#pragma unroll
+        for (int h = 0; h < NR; h++) *reinterpret_cast<u32x4*>(t + (row0 + 8 * W * h) * TR + 8 * c8) = out[h];
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < NR; h++) {
+            const int row = row0 + 8 * W * h;
+            u32x4 o;
+#pragma unroll
+            for (int k = 0; k < 4; k++) o[k] = (uint32_t)t[(8 * c8 + 2 * k) * TR + row] | ((uint32_t)t[(8 * c8 + 2 * k + 1) * TR + row] << 16);
+            *(gvec_w)(CT + (size_t)(tn * NT64 + row) * ldct + tm * NT64 + 8 * c8) = o;
+        }
+    }
+}
+
 // ---- all iterations of one matrix in one workgroup: Y [mp x np] (mp 64 or 128) and G, then H in its place, stay in LDS.
 // Eight waves.  G and G G: 32x32 tiles, one row of tiles to a pair of waves; apply: strips of 32 columns, whose Y' replaces
 // their Y (a strip is read by its own wave only).  Same roundings as the GEMM path: G, H and Y are bf16 between the
@@ -774,9 +968,36 @@ struct Layout {
     int P;
     std::vector<Mat> mats;
     bool small;                    // every matrix fits k_newton_schulz
+    bool fine[3];                  // products that go to k_gemm_64
     std::vector<int> pre_g[3], pre_t;
     size_t off_mats, off_pre, off_partials, off_inv, bytes;
 };
+
+// Which products of a call take 64x64 tiles (k_gemm_64): those that a fit to the measured times says are faster so.  A product
+// on 256x256 tiles takes, in microseconds, 7 + 0.0165 K for each round of 256 tiles (one per CU); on 64x64 tiles 5, and the
+// longer of the chain of one tile (0.003 K) and what all tiles take together (3 ns and 14 ps per k each).  Over 18 sets from
+// 1 x 200 x 800 to 6 x 1024 x 4096 the choice so made was within 8 % of the best.
+// fine_pad: what the matrices would be padded to for k_gemm_64 (64, or 256 where another product keeps its large tiles)
+void choose_tiles(int P, const SgMuonMatrix* in, int fine_pad, bool fine[3]) {
+    double tiles[3] = {}, each[3] = {}, chain[3] = {}, k_max[3] = {};
+    for (int i = 0; i < P; i++) {
+        const double m = (double)std::min(in[i].rows, in[i].cols), n = (double)std::max(in[i].rows, in[i].cols);
+        auto up = [](double x, int a) { return std::ceil(x / a) * a; };
+        for (int e = 0; e < 3; e++) {
+            auto count = [&](int pad, int size) {
+                const double tm = up(m, pad) / size, tn = up(n, pad) / size;
+                return e == EPI_APPLY ? tm * tn : tm * (tm + 1) / 2;
+            };
+            tiles[e] += count(BT, BT);
+            k_max[e] = std::max(k_max[e], up(e == EPI_GRAM ? n : m, BT));
+            const double k = up(e == EPI_GRAM ? n : m, fine_pad);
+            each[e] += count(fine_pad, NT64) * (0.003 + 14e-6 * k);
+            chain[e] = std::max(chain[e], 0.003 * k);
+        }
+    }
+    for (int e = 0; e < 3; e++)
+        fine[e] = 5.0 + std::max(chain[e], each[e]) < std::ceil(tiles[e] / 256.0) * (7.0 + 0.0165 * k_max[e]);
+}
 
 int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
     L->P = P;
@@ -795,7 +1016,10 @@ int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
         const int64_t m = std::min(in[i].rows, in[i].cols), n = std::max(in[i].rows, in[i].cols);
         L->small = L->small && m > 0 && m <= 128 && n <= NS_Y_ELEMS && fits_lds(round_up((int)m, 64), round_up((int)n, 64));
     }
-    const int pad = L->small ? 64 : BT;
+    auto all_fine = [&] { return L->fine[EPI_GRAM] && L->fine[EPI_POLY] && L->fine[EPI_APPLY]; };
+    choose_tiles(P, in, NT64, L->fine);
+    if (!all_fine()) choose_tiles(P, in, BT, L->fine);
+    const int pad = L->small || all_fine() ? 64 : BT;
     for (int i = 0; i < P; i++) {
         const SgMuonMatrix& s = in[i];
         if (s.rows <= 0 || s.cols <= 0 || s.rows * s.cols > 0x7fffffff) return sg::fail("matrix %d: bad shape %lld x %lld", i, (long long)s.rows, (long long)s.cols);
@@ -808,10 +1032,11 @@ int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
         M.m = (int)std::min(s.rows, s.cols); M.n = (int)std::max(s.rows, s.cols);
         M.mp = round_up(M.m, pad); M.np = round_up(M.n, pad);
 
-        const int nt = L->small ? 0 : M.mp / BT, tri = nt * (nt + 1) / 2;      // symmetric products: tiles on or above the diagonal
-        L->pre_g[EPI_GRAM][i + 1] = L->pre_g[EPI_GRAM][i] + tri;
-        L->pre_g[EPI_POLY][i + 1] = L->pre_g[EPI_POLY][i] + tri;
-        L->pre_g[EPI_APPLY][i + 1] = L->pre_g[EPI_APPLY][i] + nt * (M.np / BT);
+        for (int e = 0; e < 3; e++) {
+            const int size = L->fine[e] ? NT64 : BT, nt = M.mp / size;
+            // symmetric products: tiles on or above the diagonal
+            L->pre_g[e][i + 1] = L->pre_g[e][i] + (e == EPI_APPLY ? nt * (M.np / size) : nt * (nt + 1) / 2);
+        }
         L->pre_t[i + 1] = L->pre_t[i] + (M.mp / 64) * (M.np / 64);
     }
     int64_t ttiles = 0;
@@ -823,8 +1048,12 @@ int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
         // offsets for now; turned into pointers once the workspace base is known
         M.Y = (bf16_t*)take(2 * (size_t)M.mp * M.np);
         M.Y2 = (bf16_t*)take(2 * (size_t)M.mp * M.np);
-        M.G = M.H = nullptr;
+        M.G = M.H = M.T = M.T2 = nullptr;
         if (L->small) continue;
+        if (L->fine[EPI_APPLY]) {
+            M.T = (bf16_t*)take(2 * (size_t)M.mp * M.np);
+            M.T2 = (bf16_t*)take(2 * (size_t)M.mp * M.np);
+        }
         M.G = (bf16_t*)take(2 * (size_t)M.mp * M.mp);
         M.H = (bf16_t*)take(2 * (size_t)M.mp * M.mp);
     }
@@ -862,6 +1091,7 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
     for (auto& M : L.mats) {
         M.Y = (bf16_t*)(ws + (size_t)M.Y); M.Y2 = (bf16_t*)(ws + (size_t)M.Y2);
         M.G = (bf16_t*)(ws + (size_t)M.G); M.H = (bf16_t*)(ws + (size_t)M.H);
+        if (M.T) { M.T = (bf16_t*)(ws + (size_t)M.T); M.T2 = (bf16_t*)(ws + (size_t)M.T2); }
     }
     // per-call tables: through kernel arguments (no host-to-device copy, nothing blocks the host), records and tile prefixes
     // one after the other
@@ -894,13 +1124,17 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
             SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_nt<EPI_GRAM>), hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS_BYTES));
             SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_nt<EPI_POLY>), hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS_BYTES));
             SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_nt<EPI_APPLY>), hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS_BYTES));
+            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_64<EPI_GRAM>), hipFuncAttributeMaxDynamicSharedMemorySize, KS_LDS_BYTES));
+            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_64<EPI_POLY>), hipFuncAttributeMaxDynamicSharedMemorySize, KS_LDS_BYTES));
+            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_64<EPI_APPLY>), hipFuncAttributeMaxDynamicSharedMemorySize, KS_LDS_BYTES));
             SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_newton_schulz), hipFuncAttributeMaxDynamicSharedMemorySize, NS_LDS_BYTES));
             raised[dev] = true;
         }
     }
 
     hipLaunchKernelGGL(k_momentum, dim3(B.ttiles), dim3(256), 0, st, B, momentum);
-    if (!L.small || ns_steps == 0) hipLaunchKernelGGL(k_norm, dim3(P), dim3(256), 0, st, B);
+    // k_newton_schulz and k_gemm_64 add the norm up themselves
+    if (ns_steps == 0 || (!L.small && !(L.fine[EPI_GRAM] && L.fine[EPI_APPLY]))) hipLaunchKernelGGL(k_norm, dim3(P), dim3(256), 0, st, B);
     SG_LAUNCH_CHECK("muon prologue");
     if (L.small && ns_steps > 0) {
         size_t lds = 0;
@@ -909,10 +1143,17 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
         SG_LAUNCH_CHECK("k_newton_schulz");
     }
     for (int it = 0; it < (L.small ? 0 : ns_steps); it++) {
-        const int sel = it & 1, last = it == 0 ? 2 : 0;     // iter_flags
-        hipLaunchKernelGGL(k_gemm_nt<EPI_GRAM>, dim3(B.gtiles[EPI_GRAM]), dim3(GTHREADS), GEMM_LDS_BYTES, st, B, sel, last);
-        hipLaunchKernelGGL(k_gemm_nt<EPI_POLY>, dim3(B.gtiles[EPI_POLY]), dim3(GTHREADS), GEMM_LDS_BYTES, st, B, sel, last);
-        hipLaunchKernelGGL(k_gemm_nt<EPI_APPLY>, dim3(B.gtiles[EPI_APPLY]), dim3(GTHREADS), GEMM_LDS_BYTES, st, B, sel, last);
+        const int sel = it & 1, flags = (it == 0 ? 2 : 0) | (it + 1 == ns_steps ? 4 : 0);     // iter_flags
+        for (int e = 0; e < 3; e++) {
+            const dim3 grid(B.gtiles[e]);
+            if (L.fine[e]) {
+                auto* const k = e == EPI_GRAM ? k_gemm_64<EPI_GRAM> : e == EPI_POLY ? k_gemm_64<EPI_POLY> : k_gemm_64<EPI_APPLY>;
+                hipLaunchKernelGGL(k, grid, dim3(KS_THREADS), KS_LDS_BYTES, st, B, sel, flags);
+            } else {
+                auto* const k = e == EPI_GRAM ? k_gemm_nt<EPI_GRAM> : e == EPI_POLY ? k_gemm_nt<EPI_POLY> : k_gemm_nt<EPI_APPLY>;
+                hipLaunchKernelGGL(k, grid, dim3(GTHREADS), GEMM_LDS_BYTES, st, B, sel, flags);
+            }
+        }
         SG_LAUNCH_CHECK("muon newton-schulz");
     }
     hipLaunchKernelGGL(k_update, dim3(B.ttiles), dim3(256), 0, st, B, lr, 1.0f - lr * wd, ns_steps & 1, ns_steps == 0 ? 1 : 0);
