@@ -573,6 +573,26 @@ size_t sg_muon_workspace_bytes(int num_matrices, const SgMuonMatrix* mats);
 int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, float lr, float wd, int ns_steps,
                  void* workspace, size_t workspace_bytes, void* stream);
 
+/* Expert recycling event (mamba3_peer_metanet.py:437-491): the rows of the
+ * dead experts (ascending) in the four expert tensors become the row of expert
+ * `top` + 0.01 N(0,1), the given key rows 0.02 N(0,1).  Draw d, counted from 0
+ * at the generator's `offset` (a multiple of 4), is the framework generator's
+ * d-th normal draw of up to 65536 values; dead expert k takes draws draw[k] ..
+ * draw[k] + 3.  All tensors fp32 and contiguous on the stream's device; the
+ * arrays are host memory, read before the call returns.  Workspace: 16 bytes
+ * per key row and 8 per dead expert, 16-byte aligned. */
+typedef struct {
+    float* tensors[4];
+    int row[4];                    /* values per expert */
+    int num_experts, num_dead, num_keys, top;
+    const int *dead, *draw;        /* [num_dead] */
+    float* const* key_rows;        /* [num_keys] */
+    const int *key_lengths, *key_draws;
+    unsigned long long seed, offset;
+} SgRecycle;
+
+int sg_recycle_experts(const SgRecycle* r, void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -671,6 +671,75 @@ void recycle_draws(const std::vector<torch::Tensor>& noise, const std::vector<to
     }
 }
 
+// The same event for float32 parameters on the GPU: all draws in two launches.  False (nothing changed) where that is not
+// what the tensors are, or where a row is so long that its draw is not a block of the generator.
+bool recycle_experts(const std::vector<torch::Tensor>& experts, const std::vector<torch::Tensor>& keys_a, const std::vector<torch::Tensor>& keys_b,
+                     const std::vector<int64_t>& dead, const std::vector<bool>& row_dead, const std::vector<bool>& col_dead, int64_t pk,
+                     int64_t num_experts, int64_t top) {
+    constexpr int64_t MAX_ROW = 65536;         // 256 values per CU
+    const torch::Tensor& first = experts.at(0);
+    if (experts.size() != 4) return false;
+    for (const auto* list : {&experts, &keys_a, &keys_b})
+        for (const torch::Tensor& t : *list)
+            if (!t.is_cuda() || t.device() != first.device() || t.scalar_type() != at::kFloat || !t.is_contiguous() || t.dim() < 1 || t.numel() == 0 ||
+                t.numel() / t.size(0) > MAX_ROW)
+                return false;
+    for (const torch::Tensor& t : experts)
+        if (t.size(0) != num_experts) return false;
+    for (const auto* list : {&keys_a, &keys_b})
+        for (const torch::Tensor& t : *list)
+            if (t.size(0) < pk) return false;
+    c10::DeviceGuard device(first.device());
+    std::vector<int> index, draw, key_lengths, key_draws;
+    std::vector<float*> key_rows;
+    int draws = 0;
+    auto redraw = [&](const std::vector<torch::Tensor>& keys, int64_t row, bool stays) {
+        for (const torch::Tensor& k : keys) {
+            if (stays) {
+                const int64_t n = k.numel() / k.size(0);
+                key_rows.push_back(k.data_ptr<float>() + row * n);
+                key_lengths.push_back((int)n);
+                key_draws.push_back(draws);
+            }
+            draws++;
+        }
+    };
+    for (const int64_t i : dead) {
+        const int64_t a = i / pk, b = i % pk;
+        index.push_back((int)i);
+        draw.push_back(draws);
+        draws += 4;
+        if (row_dead.at(a)) redraw(keys_a, a, i == std::min(num_experts, (a + 1) * pk) - 1);
+        if (col_dead.at(b)) redraw(keys_b, b, i + pk >= num_experts);
+    }
+    at::Generator gen = at::globalContext().defaultGenerator(first.device());
+    SgRecycle r = {};
+    {
+        std::lock_guard<std::mutex> lock(gen.mutex());
+        r.seed = gen.current_seed();
+        r.offset = gen.get_offset();
+        if (r.offset % 4 != 0) return false;
+        gen.set_offset(r.offset + 4 * (uint64_t)draws);
+    }
+    for (int k = 0; k < 4; k++) {
+        r.tensors[k] = experts[k].data_ptr<float>();
+        r.row[k] = (int)(experts[k].numel() / num_experts);
+    }
+    r.num_experts = (int)num_experts;
+    r.num_dead = (int)index.size();
+    r.num_keys = (int)key_rows.size();
+    r.top = (int)top;
+    r.dead = index.data();
+    r.draw = draw.data();
+    r.key_rows = key_rows.data();
+    r.key_lengths = key_lengths.data();
+    r.key_draws = key_draws.data();
+    const int64_t bytes = 16 * (int64_t)key_rows.size() + 8 * (int64_t)index.size();
+    at::Tensor ws = at::empty({bytes}, first.options().dtype(at::kByte));
+    check_status(sg_recycle_experts(&r, ws.data_ptr(), (size_t)bytes, current_stream(first)), "recycle_experts");
+    return true;
+}
+
 }  // namespace
 
 void bind_group_steps(pybind11::module_& m) {
@@ -689,4 +758,5 @@ void bind_group_steps(pybind11::module_& m) {
     m.def("supergrok2_bilevel_finish", &supergrok2_bilevel_finish);
     m.def("add_flat_grads", &add_flat_grads);
     m.def("recycle_draws", &recycle_draws);
+    m.def("recycle_experts", &recycle_experts);
 }

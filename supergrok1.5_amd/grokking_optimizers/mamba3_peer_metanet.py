@@ -254,9 +254,13 @@ class Mamba3PEERMetaNet(nn.Module):
         flags, where = dead.tolist(), dead.nonzero(as_tuple=True)[0]
         indices = where.tolist()
         tensors = [getattr(self, name).data for name in ("expert_W1", "expert_b1", "expert_W2", "expert_b2")]
+        keys_A, keys_B = [k.data for k in self.product_keys_A], [k.data for k in self.product_keys_B]
+        rows_dead, cols_dead = [all(flags[a * pk:(a + 1) * pk]) for a in range(pk)], [all(flags[b:E:pk]) for b in range(pk)]
+        if _ops.recycle_experts(tensors, keys_A, keys_B, indices, rows_dead, cols_dead, pk, E, top):
+            self.expert_counts.zero_()
+            return True
         noise = [torch.empty((len(indices),) + tuple(t.shape[1:]), dtype=t.dtype, device=t.device) for t in tensors]
-        _ops.recycle_draws(noise, [k.data for k in self.product_keys_A], [k.data for k in self.product_keys_B], indices,
-                           [all(flags[a * pk:(a + 1) * pk]) for a in range(pk)], [all(flags[b:E:pk]) for b in range(pk)], pk, E)
+        _ops.recycle_draws(noise, keys_A, keys_B, indices, rows_dead, cols_dead, pk, E)
         where = where.to(self.expert_counts.device)
         for t, z in zip(tensors, noise):
             rows = t[top] + 0.01 * z
