@@ -195,12 +195,18 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
         from grokking_optimizers import _bilevel
         self._ensure_state()
         named = list(model.named_parameters())
-        saved = {n: p.grad for n, p in named if p.grad is not None}
+        # copies: a backward pass may leave its gradients in memory that the next one writes again (captured graphs, bucket
+        # views, a function that returns one buffer every time), and the validation pass below is one
+        with torch.no_grad():
+            have = {n: p.grad for n, p in named if p.grad is not None}
+            saved = {n: torch.empty_like(g) for n, g in have.items()}
+            if have:
+                torch._foreach_copy_(list(saved.values()), list(have.values()))
         picked = [(n, p, self._param_to_idx[id(p)]) for n, p in named
                   if n in saved and id(p) in self._param_to_idx and saved[n].numel() > 0]
         if not picked:
             return 0.0
-        grads = [saved[n].detach() for n, _, _ in picked]
+        grads = [saved[n] for n, _, _ in picked]
         state = [[kept[i] for _, _, i in picked] for kept in (self._flat_sharpness, self._flat_gru_states, self._flat_mamba_fwd_states,
                                                               self._flat_mamba_bwd_states)]
         # sort and scan need the training gradients only: the GPU has them to do while the validation pass is being enqueued
