@@ -49,16 +49,14 @@ class NeuralGrok(Optimizer):
         self._device_weights = {}
 
     def _weights_on(self, dev):
-        """The amplifier's four tensors on `dev`.  An amplifier that lives elsewhere is copied again when its weights
-        have changed (in-place updates count up a tensor's version, a new extraction makes new tensors)."""
+        """The amplifier's four tensors on `dev`, as they are now.  One that lives on the CPU (where it is made) is copied when
+        its values have changed; one on another GPU is copied for every step, as comparing would mean waiting for it."""
         weights = self._cached_meta_weights
         if weights[0].device == dev:
             return weights
-        key = tuple((id(w), w._version) for w in weights)
-        held = self._device_weights.get(dev)
-        if held is None or held[0] != key:
-            held = self._device_weights[dev] = (key, tuple(w.to(dev) for w in weights))
-        return held[1]
+        if dev.type != "cuda" or weights[0].is_cuda:
+            return tuple(w.to(dev) for w in weights)
+        return _ops.amplifier_on(weights, self._device_weights, dev)
 
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)

@@ -215,3 +215,32 @@ def test_supergrok15_sam_and_bilevel_steps():
     opt.step(train_loss=1.0, val_loss=1.2, train_acc=0.5)
     metrics = opt.step_full(m, x, y, vx, vy, crit)
     assert isinstance(metrics, dict) and opt.get_global_step() == 2
+
+
+@pytest.mark.parametrize("write", ["data", "numpy", "in place"])
+def test_neuralgrok_sees_every_write_to_a_cpu_amplifier(write):
+    """The amplifier is made on the CPU; a step uses its values of that moment, however they were written."""
+    from grokking_optimizers import NeuralGrok
+
+    def run(changed):
+        m = _model(4)
+        torch.manual_seed(6)
+        opt = NeuralGrok(m.parameters(), lr=1e-3, num_layers=2, hidden_dim=16)
+        for t in range(3):
+            x, y = _batch(t)
+            m.zero_grad()
+            nn.CrossEntropyLoss()(m(x), y).backward()
+            w = opt.amplifier.net[0].weight
+            if t == 2 and changed == "data":
+                w.data.mul_(3.0)
+            elif t == 2 and changed == "numpy":
+                w.detach().numpy()[:] *= 3.0
+            elif t == 2:
+                with torch.no_grad():
+                    w.mul_(3.0)
+                if changed == "marked":
+                    opt.mark_amplifier_dirty()
+            opt.step()
+        return list(m.parameters())
+    for a, b in zip(run("marked"), run(write)):
+        assert torch.equal(a, b)
