@@ -6,7 +6,7 @@
 // cub::DeviceSegmentedRadixSort::SortPairs call (:1860-1879).  Non-negative
 // floats order like their bit patterns, so the keys are sorted as uint32.
 //
-// Four passes of 8 bits over tiles of 8192 keys (512 lanes x 16), or of 2048 where every tensor is small.  Per pass:
+// Four passes of 8 bits over tiles of 8192 keys (512 lanes x 16), or of 2048 where the call is small.  Per pass:
 //   hist     per-tile digit counts -> spine[segment][digit][tile]  (first pass: counted while the keys are made)
 //   scan     exclusive prefix over the whole spine (2 small kernels).  Because
 //            the spine is laid out segment-major, the global prefix of entry

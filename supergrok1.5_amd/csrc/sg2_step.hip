@@ -125,11 +125,16 @@ __global__ __launch_bounds__(256) void k_pad_weights(PadArgs a) {
     }
 }
 
-// Keys per sort tile.  A scatter of 8192 keys is 16 rounds in series per wave whatever the call's size; tensors of at
-// most 65 536 elements take tiles of 2048 (the 14-tensor set: 212 workgroups instead of 57, 6 us per pass instead of 11), at
-// which they have no more than SELF_SCAN_TILES.  Tensors of one large tile each are sorted in LDS by one launch.
-inline int sort_tile_for(int64_t widest) {
-    return widest > SORT_TILE && widest <= (int64_t)SELF_SCAN_TILES * SORT_TILE_SMALL ? SORT_TILE_SMALL : SORT_TILE;
+// Keys per sort tile.  A scatter of 8192 keys is 16 rounds in series per wave whatever the call's size; where every tensor
+// has at most 65 536 elements, and so no more than SELF_SCAN_TILES tiles of 2048, and the call has fewer elements than
+// make a large tile for each of the 256 CUs, it takes the small ones (the 14-tensor set: 212 workgroups instead of 57, 6 us per
+// pass instead of 11).  Beyond that the small tiles no longer fill idle CUs, scatter shorter runs and read more counts: step
+// times with 2048 / 8192 keys are 226 / 246 us for 14 tensors of 30 000, 359 / 369 for 16 of 60 000, 650 / 663 for 100 of
+// 20 000, but 760 / 751 for 256 of 9000, 833 / 812 for 48 of 60 000 and 5.86 / 5.55 ms for 400 of 60 000.
+// Tensors of one large tile each are sorted in LDS by one launch.
+inline int sort_tile_for(int64_t widest, int64_t total) {
+    return widest > SORT_TILE && widest <= (int64_t)SELF_SCAN_TILES * SORT_TILE_SMALL && total < (int64_t)256 * SORT_TILE ? SORT_TILE_SMALL
+                                                                                                                       : SORT_TILE;
 }
 // Elements per workgroup of the norm reduction: as the other steps' tiles (many short ones for small calls).
 inline int norm_tile_for(int64_t total) { return total >= (8 << 20) ? 4096 : (total >= (1 << 20) ? 1024 : 256); }
@@ -145,7 +150,7 @@ int make_layout(int geo, int P, Numels numels, int chunk_len, Layout* L, bool bi
         total += n;
         widest = n > widest ? n : widest;
     }
-    L->sort_tile = sort_tile_for(widest);
+    L->sort_tile = sort_tile_for(widest, total);
     L->sort_widest = (int)((widest + L->sort_tile - 1) / L->sort_tile);
     L->norm_tile = norm_tile_for(total);
     for (int i = 0; i < P; i++) {

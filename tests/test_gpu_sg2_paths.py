@@ -1,5 +1,5 @@
 """The v2 step at the edges of its sort and clip dispatch: tensor sizes on both sides of what one LDS sort holds, of the
-small sort tile and of what a scatter workgroup adds up itself; and the clipping step of the class (factor applied as
+small sort tile (by the widest tensor and by the total) and of what a scatter workgroup adds up itself; and the clipping step of the class (factor applied as
 the gradients are read, fp32 sharpness beside 16-bit gradients) against clipped copies through the list functions."""
 import pytest
 import torch
@@ -10,7 +10,8 @@ from sg2_harness import Sg2Case, per_tensor_scalars, shared_scalars
 pytestmark = pytest.mark.gpu
 
 SIZES = {"one tile each": [8192, 1, 512, 513, 2048], "one above": [8193, 2047, 2049], "most small tiles": [65536, 70],
-         "one above that": [65537, 3], "most tiles of a self scan": [262144, 9], "one above that too": [262145, 8191]}
+         "one above that": [65537, 3], "most tiles of a self scan": [262144, 9], "one above that too": [262145, 8191],
+         "one below a large tile per CU": [65536] * 31 + [65535], "a large tile per CU": [65536] * 32}
 
 
 @pytest.mark.parametrize("sizes", list(SIZES), ids=lambda s: s.replace(" ", "_"))
