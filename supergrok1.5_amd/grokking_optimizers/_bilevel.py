@@ -227,6 +227,13 @@ def elem_parameters(mn):
     return out + [mn.expert_W1, mn.expert_b1, mn.expert_W2, mn.expert_b2]
 
 
+# Elements up to which SuperGrok2.bilevel_step starts the pass before the validation pass, which then runs with the pass's
+# workspace held: 281 bytes per element, 9.4 GB here, 3 % of the card.  The start hides host work only (behind a validation
+# pass of 200 launches, started before / after it: 2.44 / 2.67 ms for 0.42 M elements, 6.0 / 7.1 for 3 M, 35.3 / 36.8 for
+# 25 M), while a large model may need the memory for its activations.
+EARLY_ELEMENTS = 1 << 25
+
+
 def begin_pass(mn, grads, sharps, gru_states, mamba_fwd, mamba_bwd, exact_sharpness=False):
     """The part of accumulate_meta_gradients that needs no cotangents (sort and scan: sg2_bilevel_pass_begin), enqueued on
     the current stream: what its `begun` takes, or None for nets and tensors that the pass is not built for."""

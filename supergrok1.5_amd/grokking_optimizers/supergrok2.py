@@ -209,8 +209,11 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
         grads = [saved[n] for n, _, _ in picked]
         state = [[kept[i] for _, _, i in picked] for kept in (self._flat_sharpness, self._flat_gru_states, self._flat_mamba_fwd_states,
                                                               self._flat_mamba_bwd_states)]
-        # sort and scan need the training gradients only: the GPU has them to do while the validation pass is being enqueued
-        begun = _bilevel.begin_pass(self.meta_net, grads, *state, exact_sharpness=True)
+        # sort and scan need the training gradients only: the GPU has them to do while the validation pass is being enqueued,
+        # except where their workspace would take much of the memory that the validation pass may need
+        begun = None
+        if sum(g.numel() for g in grads) <= _bilevel.EARLY_ELEMENTS:
+            begun = _bilevel.begin_pass(self.meta_net, grads, *state, exact_sharpness=True)
         for _, p in named:
             p.grad = None              # the training gradients step aside, whatever zero_grad would do to them
         model.zero_grad()

@@ -71,6 +71,20 @@ def test_training_gradients_reach_the_pass_and_stay(static, monkeypatch):
         assert all(torch.equal(a, b) for a, b in zip(seen[name], ref.sets[k])), name
 
 
+@pytest.mark.parametrize("over,order", [(0, ["begin", "network", "finish"]), (1, ["network", "finish"])])
+def test_a_large_pass_takes_its_workspace_after_the_validation_pass(over, order, monkeypatch):
+    """Up to EARLY_ELEMENTS the sort and scan are enqueued first; beyond, the pass begins inside the accumulation, when the
+    validation pass has given its activations back."""
+    calls = []
+    forward = _Network.forward
+    monkeypatch.setattr(_Network, "forward", lambda self, which: calls.append("network") or forward(self, which))
+    monkeypatch.setattr(_bilevel, "EARLY_ELEMENTS", sum(torch.Size(s).numel() for s in SHAPES) - over)
+    monkeypatch.setattr(_bilevel, "begin_pass", lambda *a, **kw: calls.append("begin"))
+    monkeypatch.setattr(_bilevel, "accumulate_meta_gradients", lambda *a, **kw: calls.append("finish"))
+    _bilevel_step("cpu", False)
+    assert calls == ["network"] + order               # the first one is the training pass
+
+
 @pytest.mark.gpu
 def test_static_gradient_buffers_give_the_same_meta_gradients():
     a, b = (_bilevel_step("cuda", static).meta_net for static in (False, True))
