@@ -124,7 +124,7 @@ def test_chunked_scan_matches_sequential(n, chunk):
 
 
 def test_windowed_summaries_match_full_chunks():
-    """Chunk summaries built backwards in blocks of 64/128 steps, stopping once the 2x2 part is below 2^-100, give
+    """Chunk summaries built backwards in blocks of 64/128 steps, stopping once the 2x2 part is below 2^-64, give
     the sequential result to rounding -- for strongly contracting weights (the first block suffices), for poles that
     need several blocks (the reference's initialisation A = -1..-16 with a large dt: |A_bar| close to 1 again), and
     for weights that barely contract (the walk reaches the chunk start: the exact summary, re-associated)."""
@@ -156,6 +156,35 @@ def test_windowed_summaries_match_full_chunks():
     plain, dplain = _run_oracle(Wslow, st, g, s, sc, 32, 256)
     win, dwin = _run_oracle(Wslow, st, g, s, sc, 32, 256, window=256)
     assert np.array_equal(dplain["ctx"], dwin["ctx"]) and np.array_equal(plain["mamba_fwd"], win["mamba_fwd"])
+
+
+@pytest.mark.parametrize("skip", [True, False])
+@pytest.mark.parametrize("before", [72, 104, 136, 168, 200])
+def test_a_forgotten_state_does_not_show_where_the_drive_falls(before, skip):
+    """The case in which a state multiplied by less than 2^-64 could show: no constant drive (input_proj without bias), and
+    the reverse scan goes from gradients near 1 to gradients near 1e-8, whose drive is 2^-53 of it, `before` steps ahead of a
+    chunk's start, on both sides of where the summary walk ends (about 120 steps back).  The fp32 contexts with windowed
+    summaries are no further from float64 than the sequential fp32 recurrence, entry by entry relative to the entry, also where
+    the context is the scan's output alone (D = 0: no skip).  (A bound of 2^-40 fails here.  Where the drive falls so far that
+    2^-64 would show in the state, C and the gate have fallen with it and the context is below the smallest normal number.)"""
+    n, chunk = 1024, 256
+    W = weights_np()
+    W[1][:] = 0.0
+    if not skip:
+        W[8][:] = W[17][:] = 0.0
+    rng = np.random.RandomState(3)
+    g = ((rng.rand(n) * 0.5 + 0.5) * np.sign(rng.randn(n))).astype(np.float32)
+    g[rng.permutation(n)[:n - (2 * chunk - before)]] *= np.float32(1e-8)
+    st = random_state_np(n, 11)
+    for k in ("mamba_fwd", "mamba_bwd"):
+        st[k][:] = 0.0
+    zero = np.zeros_like(g)
+    ref = _run_oracle(W, st, g, zero, default_scalars(), 64, 0)[1]["ctx"]
+    worst = []
+    for kw in (dict(chunk_len=0), dict(chunk_len=chunk, window=64)):
+        got = _run_oracle(W, st, g, zero, default_scalars(), 32, **kw)[1]["ctx"].astype(np.float64)
+        worst.append(float((np.abs(got - ref) / np.maximum(np.abs(ref), 1e-37)).max()))
+    assert worst[1] <= 1.01 * worst[0] and worst[0] < 1e-3, worst
 
 
 def test_contracted_summary_forgets_a_finite_state_and_keeps_a_non_finite_one():
