@@ -12,6 +12,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <vector>
 
 #include "ops_common.hpp"
@@ -715,24 +717,82 @@ void recycle_draws(const std::vector<torch::Tensor>& noise, const std::vector<to
     }
 }
 
+constexpr int64_t RECYCLE_MAX_ROW = 65536;         // 256 values per CU
+
+// Whether k_redraw_keys' draws are the framework's: the layout of a draw (how far it moves the generator's offset, which words
+// of which counter an element takes) is no documented interface and may change with the framework or the device.  Rows of one
+// value, of an odd length and of the largest one are drawn both ways from a generator of their own, once per device (a
+// property of the two, not of any object); where they differ recycling takes recycle_draws.
+bool draws_agree(const std::vector<torch::Tensor>& ours, const std::vector<torch::Tensor>& theirs) {
+    for (size_t k = 0; k < ours.size(); k++) {
+        const torch::Tensor d = (ours[k] - theirs[k]).abs().max();
+        if (!(d.item<float>() < 1e-5f)) return false;       // deviations of 0.02: another layout is off by as much, another rounding of log, root and sine by 1e-6
+    }
+    return true;
+}
+bool generator_is_known(const torch::Device& device) {
+    static std::mutex mutex;
+    static std::map<int, bool> known;
+    std::lock_guard<std::mutex> lock(mutex);
+    const auto it = known.find(device.index());
+    if (it != known.end()) return it->second;
+    at::NoGradGuard guard;
+    c10::DeviceGuard on(device);
+    at::Generator shared = at::globalContext().defaultGenerator(device);
+    at::Generator gen = [&] {
+        std::lock_guard<std::mutex> held(shared.mutex());
+        return shared.clone();
+    }();
+    gen.set_current_seed(0x9E3779B97F4A7C15ull);
+    gen.set_offset(12);
+    const auto opt = torch::TensorOptions().device(device).dtype(torch::kFloat32);
+    std::vector<torch::Tensor> ours, theirs;
+    std::vector<float*> rows;
+    std::vector<int> lengths, draws;
+    for (const int64_t n : {(int64_t)1, (int64_t)301, RECYCLE_MAX_ROW}) {
+        lengths.push_back((int)n);
+        draws.push_back((int)draws.size());
+        ours.push_back(torch::empty({n}, opt));
+        rows.push_back(ours.back().data_ptr<float>());
+        theirs.push_back(torch::empty({n}, opt).normal_(0.0, 1.0, gen).mul_(0.02));
+    }
+    bool same = gen.get_offset() == 12 + 4 * lengths.size();
+    if (same) {
+        SgRecycle r = {};
+        r.num_experts = 1;
+        r.num_keys = (int)rows.size();
+        r.key_rows = rows.data();
+        r.key_lengths = lengths.data();
+        r.key_draws = draws.data();
+        r.seed = gen.current_seed();
+        r.offset = 12;
+        at::Tensor ws = at::empty({16 * (int64_t)rows.size()}, opt.dtype(at::kByte));
+        check_status(sg_recycle_experts(&r, ws.data_ptr(), (size_t)ws.numel(), current_stream(ws)), "recycle_experts");
+        same = draws_agree(ours, theirs);
+    }
+    known[device.index()] = same;
+    return same;
+}
+
 // The same event for float32 parameters on the GPU: all draws in two launches.  False (nothing changed) where that is not
-// what the tensors are, or where a row is so long that its draw is not a block of the generator.
+// what the tensors are, where a row is so long that its draw is not a block of the generator, or where the generator draws
+// otherwise than the kernels.
 bool recycle_experts(const std::vector<torch::Tensor>& experts, const std::vector<torch::Tensor>& keys_a, const std::vector<torch::Tensor>& keys_b,
                      const std::vector<int64_t>& dead, const std::vector<bool>& row_dead, const std::vector<bool>& col_dead, int64_t pk,
                      int64_t num_experts, int64_t top) {
-    constexpr int64_t MAX_ROW = 65536;         // 256 values per CU
     const torch::Tensor& first = experts.at(0);
     if (experts.size() != 4) return false;
     for (const auto* list : {&experts, &keys_a, &keys_b})
         for (const torch::Tensor& t : *list)
             if (!t.is_cuda() || t.device() != first.device() || t.scalar_type() != at::kFloat || !t.is_contiguous() || t.dim() < 1 || t.numel() == 0 ||
-                t.numel() / t.size(0) > MAX_ROW)
+                t.numel() / t.size(0) > RECYCLE_MAX_ROW)
                 return false;
     for (const torch::Tensor& t : experts)
         if (t.size(0) != num_experts) return false;
     for (const auto* list : {&keys_a, &keys_b})
         for (const torch::Tensor& t : *list)
             if (t.size(0) < pk) return false;
+    if (!generator_is_known(first.device())) return false;
     c10::DeviceGuard device(first.device());
     std::vector<int> index, draw, key_lengths, key_draws;
     std::vector<float*> key_rows;
@@ -804,4 +864,5 @@ void bind_group_steps(pybind11::module_& m) {
     m.def("add_flat_grads", &add_flat_grads);
     m.def("recycle_draws", &recycle_draws);
     m.def("recycle_experts", &recycle_experts);
+    m.def("draws_agree", &draws_agree);
 }

@@ -3,9 +3,11 @@
 // A few hundred draws of a few values each: as library calls they are a launch apiece, 3.5 ms of host time in an event with
 // 144 dead experts (35 us a step at one event in 100 steps, a third of the step of a small model).  Here they are two launches.
 //
-// The draws are those of the framework's device generator, to rounding: Philox4x32-10 (Salmon et al., "Parallel random
-// numbers: as easy as 1, 2, 3", 2011) with the generator's seed as key, counter = (offset / 4, element), and Box-Muller on
-// the first two words.  A draw of up to 256 values per CU moves the generator's offset by 4.
+// The draws are those of the framework's device generator (torch's normal_ on the GPU), to rounding: Philox4x32-10 (Salmon
+// et al., "Parallel random numbers: as easy as 1, 2, 3", 2011) with the generator's seed as key, counter = (offset / 4,
+// element), and Box-Muller (1958) on the first two words.  A draw of up to 256 values per CU moves the generator's offset by
+// 4.  Which words and counters a draw takes is observed, not documented: the caller compares both once per device
+// (generator_is_known in ops_group.cpp) and leaves these kernels where they differ.
 #include "sg_common.hpp"
 
 #include <cstring>
