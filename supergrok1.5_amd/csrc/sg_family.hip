@@ -49,6 +49,10 @@ __global__ __launch_bounds__(THREADS) void k_grokadamw(BT B, float clip_norm, fl
 // launch reduce the gradient norm); an element finds its interval by a search of the thresholds in LDS and evaluates
 // one fma.  Evaluating the units one by one is 3 vector instructions and LDS operands for each of 128 units: 332 us
 // for 25 M elements against 140 us for the step's memory traffic.
+// Error: A and B are rounded once, so the amplifier is within 2^-24 (|A g| + |B| + |A g + B|).  Close to a far threshold the
+// first two cancel and a unit-by-unit sum, which rounds only what is left of them, can be closer there; over module-made
+// weights (128 units) and gradients of deviation 1e-3, 1 and 1000 the largest error against float64 is 6e-9, 4e-8 and 4e-5, unit
+// by unit 9e-8, 2e-7 and 2e-4.
 constexpr int AMP_SLOTS = 511;         // thresholds, padded with +inf to 2^k - 1 (at most MAX_HIDDEN = 256 real ones)
 struct AmpTable {
     float t[AMP_SLOTS + 1];
@@ -642,7 +646,7 @@ int sg11_fused_step(int num_tensors, const SgFamilyTensor* tensors, const Sg15Ne
         launch_tensor_sums<3>(G, st);
         hipLaunchKernelGGL(k_sg11_adam<BT>, dim3(B.tiles), dim3(THREADS), 0, st, G, beta2, eps, 1.0f - lr * wd, lamb, ramp, gate_temperature,
                            smart);
-        SG_LAUNCH_CHECK("k_sg11");
+        SG_LAUNCH_CHECK("k_sg11_adam");
         return 0;
     });
 }

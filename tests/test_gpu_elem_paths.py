@@ -1,5 +1,5 @@
 """The elementwise kernels at the edges of their dispatch: amplifier tables of every width class with units that have no
-threshold, gradients on both sides of the meta-net polynomial's reach, tensor counts on both sides of what travels
+threshold and its rounding far from zero, gradients on both sides of the meta-net polynomial's reach, tensor counts on both sides of what travels
 as kernel arguments, and pointers that do not allow four elements per access."""
 import numpy as np
 import pytest
@@ -56,6 +56,24 @@ def test_amplifier_table(H, shift):
     _ops().neuralgrok_fused_step(got["p"], got["g"], got["ea"], got["easq"], [3, 3], *W, sc[0], sc[1], H, *sc[2:])
     fo.neuralgrok_step(want["p"], want["g"], want["ea"], want["easq"], [3, 3], w1, b1, w2, b2, *sc)
     _check({k: got[k] for k in ("p", "g", "ea", "easq")}, want, H)
+
+
+@pytest.mark.parametrize("spread", [1e-3, 1.0, 300.0])
+def test_amplifier_table_stays_within_its_rounding(spread):
+    """The line A g + B of an interval against float64, for gradients up to and far beyond the thresholds: A and B are rounded
+    once (2^-24 each), the fused multiply-add and the product with g once more."""
+    r, H = np.random.RandomState(5), 128
+    w1, b1, w2 = (r.uniform(-1, 1, s).astype(np.float32) for s in ((H, 1), (H,), (1, H)))
+    g = (r.randn(40_000) * spread).astype(np.float32)
+    got = {k: _dev([x]) for k, x in dict(p=np.zeros_like(g), g=g, ea=np.zeros_like(g), easq=np.zeros_like(g)).items()}
+    W = [torch.from_numpy(x).to(DEV) for x in (w1, b1, w2, np.float32([0.0]))]
+    _ops().neuralgrok_fused_step(got["p"], got["g"], got["ea"], got["easq"], [3], *W, 1.0, 0.0, H, 0.0, 0.98, 1e-3, 1.0, 1e-8, 0.0)      # beta1 = 0: exp_avg is the amplified gradient
+    x, w1, b1, w2 = (a.astype(np.float64).reshape(-1) for a in (g, w1, b1, w2))
+    active = w1[:, None] * x + b1[:, None] > 0
+    A, B = ((active * (w2 * c)[:, None]).sum(0) for c in (w1, b1))
+    value = A * x + B
+    err = np.abs(got["ea"][0].cpu().numpy() / x - value)
+    assert (err <= 2.0 ** -24 * 1.01 * (np.abs(A * x) + np.abs(B) + 2 * np.abs(value)) + 1e-30).all(), float(err.max())
 
 
 @pytest.mark.parametrize("H", [1, 32, 256])
