@@ -506,7 +506,7 @@ def secondary_configs(dev, steps=20, warmup=3):
                            ("bilevel_pass_shared14", "bilevel"), ("bilevel_pass_scale50", "bilevel50"), ("grokadamw_scale50", "grokadamw"), ("neuralgrok_scale50", "neuralgrok"),
                            ("prodigy_scale50", "prodigy"), ("lion_scale50", "lion"), ("supergrok11_scale50", "sg11")):
         W = build_step(workload, _ops, dev)
-        n_steps, n_warm = (5, 1) if workload == "bilevel50" else (steps, warmup)       # 0.15 s a pass
+        n_steps, n_warm = (5, 1) if workload == "bilevel50" else (steps, warmup)       # 0.04 s a pass
         for _ in range(n_warm):
             W["step"]()
         torch.cuda.synchronize()

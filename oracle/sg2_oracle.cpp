@@ -699,7 +699,7 @@ int step_tensor(const Dims& d, const float* const* W, int64_t chunk_len, int64_t
             x[t * dm + k] = O::fma((R)W[W_IN_W][2 * k + 1], sv, (R)W[W_IN_W][2 * k] * gv) + (R)W[W_IN_B][k];
     }
 
-    /* length of a summary's first block, from the weights alone (the kernels' k_compose does the same) */
+    /* length of a summary's first block, from the weights alone (the kernels' compose_block does the same) */
     int64_t first_block = 0;
     {
         int largest = 0, any_zero = 0;

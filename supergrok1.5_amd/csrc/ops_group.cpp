@@ -647,6 +647,8 @@ py::object supergrok2_bilevel_finish(BilevelPass& pass, py::list cots, float res
     }
     const auto opt = torch::TensorOptions().device(pass.ws.device()).dtype(torch::kFloat32);
     torch::Tensor norms;
+    // (tensor by tensor with the framework's own reduction, as v.norm() forms them: the sums of a fresh meta-net's experts can
+    // nearly cancel, and the first step of an optimizer that divides by their size shows the last bits of the cotangents)
     if (normalise) {
         norms = torch::empty({(int64_t)v.size()}, opt);
         for (size_t i = 0; i < v.size(); i++) {

@@ -5,9 +5,9 @@
 // Stands in for the scan part of launch_mamba3_peer_backward[_batched]
 // (csrc/supergrok2_mamba_peer_backward_kernels.cu:2512-3624 of the reference, called from
 // grokking_optimizers/supergrok2.py:516-1330).  The forward pass is the production scan itself
-// (sg2_bilevel_forward: sort + summaries + prefix + replay, carried states untouched), which additionally keeps
-// the state entering every 32nd step; the per-element part of the meta-net (GRU, soft top-4 PEER routing,
-// experts) is differentiated by torch autograd on the caller's side.
+// (sort + summaries + prefix + replay, carried states untouched), which additionally keeps the state entering every
+// HT_STEP-th step; the per-element part of the meta-net (GRU, soft top-4 PEER routing, experts) is differentiated by
+// sg2_bilevel_elem.hip (from torch operations for routing sizes that kernel is not built for).
 //
 // The adjoint state lambda obeys a linear recurrence over the scan steps in reverse.  Its transfer map contracts like
 // the forward recurrence's, so it is not handed from chunk to chunk: k_adjoint gives every wave a range of steps of equal

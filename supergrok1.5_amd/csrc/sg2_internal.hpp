@@ -122,7 +122,7 @@ struct Plan {
     uint32_t* keys[2];
     int32_t* vals[2];              // element index within the tensor | sign bit of the gradient in bit 31
     float* ssorted;                // [total] sharpness gathered into sorted order
-    uint32_t* spine;               // [256 * sort_tiles] per-tile digit counts, layout [segment][digit][tile]
+    uint32_t* spine;               // [256 * sort_tiles] per-tile digit counts, layout [segment][digit][tile], or [segment][tile][digit] in calls without scan kernels
     uint32_t* blocksums;
     float* summaries;              // [2][wchunks][6][THREADS]
     float* hstart;                 // [2][chunks][2][THREADS]
@@ -133,7 +133,7 @@ struct Plan {
     float* adj_lam;                // bilevel: [2][chunks][128][2] adjoint state arriving at the end of every chunk
     float* adj_blk;                // bilevel: [2][SG2_BWD_STRIDE] sums of adj_part's rows
     float* adj_part;               // bilevel: [2][ADJ_GROUPS][SG2_BWD_STRIDE] per-workgroup gradient sums
-    int* contracted;               // [3] bilevel pass: every unit threshold of the experts is 0 (set by k_tables, cleared by k_expert_tables); [0] set by k_compose (1 while every carried state of the call is finite), cleared by any summary whose 2x2 part is not exactly zero; [1] steps of a summary's first block (k_compose); [2] k_compose: some carried state is not finite
+    int* contracted;               // [0] set by compose_block (1 while every carried state of the call is finite), cleared by any summary whose 2x2 part is not exactly zero; [1] steps of a summary's first block (compose_block); [2] compose_block: some carried state is not finite; [3] bilevel pass: every unit threshold of the experts is 0 (set by k_tables, cleared by k_expert_tables)
     int* state_bad;                // [P] set by k_tables: a carried Mamba state of the tensor holds a non-finite entry
     int* sharp_nonzero;            // [P] uploaded as 0; set by k_keys when some sharpness entry of the tensor is not 0
     float* ctx;                    // [2][total][d_model]

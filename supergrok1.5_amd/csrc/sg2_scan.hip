@@ -22,11 +22,11 @@
 //                  state part only and a norm bound instead of M.
 //   k_chunk_prefix start state of each chunk: summaries applied in order to
 //                  the carried state of the tensor.
-//   k_scan<true>   every chunk replayed from its start state: y = h.C, gate,
-//                  D skip, out_proj, and the 8-float context written straight
-//                  to the element's original position (the "unsort").  The
-//                  last chunk stores the new carried state.
-//   compose_block  (sg2_compose_block.hpp) ran beside the sort's first kernel: the input of a timestep is two numbers (g, s)
+//   k_replay       every chunk replayed from its start state: y = h.C, gate,
+//   (k_scan<true>  D skip, out_proj, and the 8-float context written straight
+//   for the large  to the element's original position (the "unsort").  The
+//   geometry)      last chunk stores the new carried state.
+//   compose_block  (sg2_compose_block.hpp) runs beside the sort's first kernel: the input of a timestep is two numbers (g, s)
 //                  and every projection of the block is linear in their 8-float
 //                  input projection, so input_proj, in_proj, dt_proj, B_proj and
 //                  C_proj are folded into 5 x d_inner coefficient triples per
@@ -54,8 +54,8 @@
 // Where the inputs are small (the usual case: sg2_taylor_ok, sg2_poly_ok in sg2_compose.h) the step size and the gate
 // of a tile come from cubic Taylor polynomials around their zero-input arguments, and A_bar, sin and cos of a block
 // from per-lane polynomials in dt - dt0; the forms above serve the remaining tiles and blocks.
-// For the bilevel pass k_scan<true, true> also stores the state entering every
-// 32nd step (Plan::htile), which the adjoint kernels restart from.
+// For the bilevel pass k_replay<G, true> also stores the state entering every
+// HT_STEP-th step (Plan::htile), which the adjoint kernels restart from.
 #include <type_traits>
 #include "sg2_internal.hpp"
 #include "sg2_pair_sums.hpp"

@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256) void k_tables(TableChunk c) {
     if (blockIdx.x > 0) {
         // A tensor whose carried state is not finite (a diverged run) must come out non-finite as a whole, as it does in
         // the reference, which multiplies every chunk's start state through: the scan only lets contracted summaries
-        // forget what came before them while every carried state of the call is finite (k_compose reads these flags).
+        // forget what came before them while every carried state of the call is finite (compose_block reads these flags).
         const int k = blockIdx.x - 1;
         const TensorDev& t = c.rec[k];
         bool bad = false;
@@ -440,7 +440,7 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
     if (!workspace || workspace_bytes < L.bytes)
         return sg::fail("workspace too small: need %zu bytes, got %zu", L.bytes, workspace_bytes);
     if (((uintptr_t)workspace & 255u) != 0) return sg::fail("workspace must be 256-byte aligned");
-    // ---- per-tensor records and the four prefix tables: written by k_tables from kernel arguments, UPLOAD_RECS
+    // ---- per-tensor records and the five prefix tables: written by k_tables from kernel arguments, UPLOAD_RECS
     // tensors per launch (no host-to-device copy: nothing here blocks the host or depends on the lifetime of host
     // memory, and the call can be recorded into a graph)
     unsigned char* ws = static_cast<unsigned char*>(workspace);

@@ -11,9 +11,10 @@ lambda_eff = lamb*ramp*gate, progressive wd) and the same 51-argument
 expert recycling every `recycle_interval` steps.
 
 Differences, all on the host side:
-  * the per-tensor norm clip is applied with device-side scale factors
-    (torch._foreach_norm) instead of two host syncs per tensor; a gradient whose
-    norm is below the threshold is multiplied by exactly 1.0;
+  * the per-tensor norm clip is a factor that the step's kernels apply as they
+    read a gradient (norms reduced by the step itself) instead of two host syncs
+    per tensor; a gradient whose norm is below the threshold is multiplied by
+    exactly 1.0;
   * non-finite gradient entries are zeroed inside the kernel (the reference
     does it both on the host and in the kernel);
   * after a recycling event the cached weight tensors are rebuilt, so re-drawn

@@ -64,7 +64,7 @@ def test_multi_chunk_small_chunks():
 
 def test_windowed_summaries_accept_and_fall_back():
     """Window 64 on chunks of 256: the first block is accepted with the N(0,0.1) weights; with barely contracting
-    poles (A_log = -12) no block passes the 2^-100 test and the walk covers the whole chunk."""
+    poles (A_log = -12) no block passes the 2^-64 test and the walk covers the whole chunk."""
     from grokking_optimizers import _cabi
     shapes = [(3000,), (64, 65), (700,)]
     assert _cabi.lib().sg2_set_chunk_len(256) == 0 and _cabi.lib().sg2_set_scan_window(64) == 0
@@ -97,7 +97,7 @@ def test_module_initialised_weights_over_several_chunks(seed):
 
 def test_adaptive_window_needs_several_blocks():
     """A_log = log(1..16) with dt about 1.7: |A_bar| of the fast poles is close to 1 again, a 64-step block does not
-    contract to 2^-100 and the summary walk has to go back several blocks (device and checker must stop at the same
+    contract to 2^-64 and the summary walk has to go back several blocks (device and checker must stop at the same
     block: the results are bit-identical or the comparison of the contexts fails)."""
     from grokking_optimizers import _cabi
     shapes = [(3000,), (64, 65)]

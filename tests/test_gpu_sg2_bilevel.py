@@ -98,7 +98,7 @@ def test_small_tensors_with_sharpness_and_carried_states():
 
 
 def test_ragged_tile_ends():
-    """Lengths that end 1..7 steps after a multiple of 32 or 64 (the forward pass keeps a state every 32 steps, and the
+    """Lengths that end 1..7 steps after a multiple of 32 or 64 (the forward pass keeps a state every 16 steps, and the
     last steps of a tensor run through its scalar tail loop)."""
     _case([(99,), (33,), (97,), (39,), (64 + 32,), (32,), (31,), (64 + 39,)], seed=15, sharp=True, state_std=0.3)
 
@@ -121,7 +121,7 @@ def test_barely_contracting_poles_walk_the_whole_chunk():
 
 def test_slow_poles_need_several_summary_blocks():
     """A_log = -2 (A = -0.135, the slowest pole of the optimizer's own initialisation is -1): with blocks of 64 steps
-    the 2x2 part falls below 2^-100 only after several of them, so the block walk of both summary kernels composes
+    the 2x2 part falls below 2^-64 (2^-100 in the adjoint summaries) only after several of them, so the block walk of both summary kernels composes
     maps (chunk length 1024, window 64)."""
     _case([(5000,), (2100,)], seed=17, sharp=True, state_std=0.3, chunk_len=1024, a_log=-2.0, window=64)
 
