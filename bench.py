@@ -22,7 +22,7 @@ BYTES_PER_ELEMENT = 72          # algorithmic HBM bytes per element per step (fp
 HBM_PEAK_GBS = 8000.0
 SIMDS = 1024
 REPLAY_WAVES_PER_SIMD = 2        # k_replay: eight one-wave workgroups per compute unit (19.8 KB of LDS each)
-STAGE_KERNEL_PREFIX = {"scan_output": "k_replay<", "scan_summary": "k_scan<false, false>", "elementwise": "k_elem<"}
+STAGE_KERNEL_PREFIX = {"scan_output": "k_replay<", "scan_summary": "k_scan<default, false>", "elementwise": "k_elem<"}
 
 
 def profile_figures():
