@@ -239,19 +239,19 @@ bool adamw_group_step(py::handle params, py::handle state, double lr, double bet
     return true;
 }
 
-// The amplifier's four tensors on `device`, for an amplifier that lives on the CPU: one packed copy per device and stream,
-// made again whenever the values differ from those it was made from (a comparison of a few hundred floats takes 0.1 us, a
-// copy 20 us; version counters do not see writes through .data or a NumPy view).  A copy is only ever used on the stream it
-// was made on, so that replacing it frees it in that stream's order.
+// The amplifier's four tensors on `device`, for an amplifier that lives on the CPU: one packed copy per device, made again
+// whenever the values differ from those it was made from (a comparison of a few hundred floats takes 0.1 us, a copy 20 us;
+// version counters do not see writes through .data or a NumPy view).  The copy is complete before it is handed out, and a
+// stream other than the one it was made on is recorded with it, so that replacing it does not free it under that
+// stream's kernels; a graph that captures its address keeps it for good.
 py::tuple amplifier_on(const std::vector<torch::Tensor>& weights, py::dict held, const torch::Device& device) {
-    constexpr size_t MAX_COPIES = 16;
     int64_t total = 0;
     for (const torch::Tensor& w : weights) {
         TORCH_CHECK(w.device().is_cpu() && w.scalar_type() == torch::kFloat32 && w.is_contiguous(), "amplifier weights must be contiguous float32 on the CPU");
         total += w.numel();
     }
     const auto stream = c10::hip::getCurrentHIPStream(device.index());
-    const py::tuple key = py::make_tuple(stream.device_index(), (uintptr_t)stream.stream());
+    const py::int_ key(stream.device_index()), made_on((uintptr_t)stream.stream());
     if (held.contains(key)) {
         const py::tuple entry = held[key];
         const torch::Tensor made_from = entry[0].cast<torch::Tensor>();
@@ -261,7 +261,16 @@ py::tuple amplifier_on(const std::vector<torch::Tensor>& weights, py::dict held,
             same = same && std::memcmp(made_from.data_ptr<float>() + o, w.data_ptr<float>(), sizeof(float) * (size_t)w.numel()) == 0;
             o += w.numel();
         }
-        if (same) return entry[1].cast<py::tuple>();
+        if (same) {
+            if (!py::object(entry[3]).equal(made_on))
+                entry[1].cast<torch::Tensor>().record_stream(c10::Stream(c10::Stream::UNSAFE, device, stream.id()));
+            hipStreamCaptureStatus status = hipStreamCaptureStatusNone;      // (the null stream cannot capture)
+            if (stream.stream() != nullptr && hipStreamIsCapturing(stream.stream(), &status) == hipSuccess && status != hipStreamCaptureStatusNone) {
+                if (!held.contains("captured")) held["captured"] = py::list();
+                held["captured"].cast<py::list>().append(entry[1]);
+            }
+            return entry[2].cast<py::tuple>();
+        }
     }
     at::NoGradGuard guard;
     torch::Tensor host = torch::empty({total}, torch::kFloat32);
@@ -277,8 +286,7 @@ py::tuple amplifier_on(const std::vector<torch::Tensor>& weights, py::dict held,
         parts[k] = py::cast(flat.narrow(0, o, weights[k].numel()).view(weights[k].sizes()));
         o += weights[k].numel();
     }
-    if (held.size() >= MAX_COPIES) held.clear();
-    held[key] = py::make_tuple(host, parts);
+    held[key] = py::make_tuple(host, flat, parts, made_on);
     return parts;
 }
 

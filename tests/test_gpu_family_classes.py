@@ -244,3 +244,47 @@ def test_neuralgrok_sees_every_write_to_a_cpu_amplifier(write):
         return list(m.parameters())
     for a, b in zip(run("marked"), run(write)):
         assert torch.equal(a, b)
+
+
+def test_neuralgrok_step_with_a_cpu_amplifier_in_a_graph():
+    """One eager step, then the second step captured (on a stream of its own) and replayed: as two eager steps; and other
+    values of the amplifier in between reach an eager step without disturbing a later replay."""
+    from grokking_optimizers import NeuralGrok
+
+    def make():
+        m = _model(4)
+        torch.manual_seed(6)
+        opt = NeuralGrok(m.parameters(), lr=1e-3, num_layers=2, hidden_dim=16)
+        x, y = _batch(0)
+        nn.CrossEntropyLoss()(m(x), y).backward()
+        grads = [p.grad.clone() for p in m.parameters()]
+
+        def refill():          # the step clips the gradients where they lie
+            for p, g in zip(m.parameters(), grads):
+                p.grad.copy_(g)
+        opt.step()
+        refill()
+        return m, opt, refill
+    m, opt, refill = make()
+    opt.step()
+    want = [p.detach().clone() for p in m.parameters()]
+    m, opt, refill = make()
+    start = [p.detach().clone() for p in m.parameters()]
+    state = {p: {k: v.clone() for k, v in opt.state[p].items() if torch.is_tensor(v)} for p in m.parameters()}
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        opt.step()
+    for again in range(3):
+        with torch.no_grad():
+            if again == 2:                       # an eager step with other values makes another copy
+                opt.amplifier.net[0].weight.mul_(2.0)
+                opt.step()
+                torch.zeros(4096, device=DEV).fill_(float("nan"))
+            for p, v in zip(m.parameters(), start):
+                p.copy_(v)
+                for k, b in state[p].items():
+                    opt.state[p][k].copy_(b)
+            refill()
+        graph.replay()
+        for a, b in zip(m.parameters(), want):
+            assert torch.equal(a, b), again
