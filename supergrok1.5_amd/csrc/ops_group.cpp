@@ -674,6 +674,16 @@ py::object supergrok2_bilevel_finish(BilevelPass& pass, py::list cots, float res
     return py::make_tuple(want_smart ? py::cast(smart) : py::object(py::none()), elem, scan);
 }
 
+// Copies of gradients (their strides kept), in one batched copy.
+std::vector<torch::Tensor> copies_of(const std::vector<torch::Tensor>& grads) {
+    at::NoGradGuard guard;
+    std::vector<torch::Tensor> out;
+    out.reserve(grads.size());
+    for (const torch::Tensor& g : grads) out.push_back(at::empty_like(g));
+    if (!out.empty()) at::_foreach_copy_(out, grads);
+    return out;
+}
+
 // p.grad (+)= its slice of `flat`, parameter after parameter; one without a gradient gets a view of the flat tensor.
 void add_flat_grads(const std::vector<torch::Tensor>& params, const torch::Tensor& flat) {
     at::NoGradGuard guard;
@@ -871,6 +881,7 @@ void bind_group_steps(pybind11::module_& m) {
     py::class_<BilevelPass>(m, "BilevelPass");
     m.def("supergrok2_bilevel_begin", &supergrok2_bilevel_begin);
     m.def("supergrok2_bilevel_finish", &supergrok2_bilevel_finish);
+    m.def("copies_of", &copies_of);
     m.def("add_flat_grads", &add_flat_grads);
     m.def("recycle_draws", &recycle_draws);
     m.def("recycle_experts", &recycle_experts);

@@ -198,11 +198,8 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
         named = list(model.named_parameters())
         # copies: a backward pass may leave its gradients in memory that the next one writes again (captured graphs, bucket
         # views, a function that returns one buffer every time), and the validation pass below is one
-        with torch.no_grad():
-            have = {n: p.grad for n, p in named if p.grad is not None}
-            saved = {n: torch.empty_like(g) for n, g in have.items()}
-            if have:
-                torch._foreach_copy_(list(saved.values()), list(have.values()))
+        have = [(n, p.grad) for n, p in named if p.grad is not None]
+        saved = dict(zip([n for n, _ in have], _ops.copies_of([g for _, g in have])))
         picked = [(n, p, self._param_to_idx[id(p)]) for n, p in named
                   if n in saved and id(p) in self._param_to_idx and saved[n].numel() > 0]
         if not picked:
