@@ -417,8 +417,11 @@ int sg2_bilevel_elem_ex(const SgDims* dims, const Sg2Weights* weights, int64_t t
  *   elem_grads_out         as grads_out of sg2_bilevel_elem, the expert tensors at the caller's own expert_hidden
  *                          (1364 + 144 * (3 * expert_hidden + 1) floats)
  *   scan_grads_out [SG2_SCAN_GRAD_FLOATS]
+ * Between the two calls gradients, sharpness, states and weights keep their values: the second reads them again (where a
+ * backward pass in between may write into the gradients' memory, hand over copies).
  * Built for d_model 8, d_state 16, d_inner 16, gru_hidden 4, 4 heads, 12 keys, 144 experts of width <= 16.  Contexts and
- * their gradients travel between the three parts in the workspace. */
+ * their gradients travel between the three parts in the workspace, 281 bytes per element, which is held from the first
+ * call to the end of the second. */
 size_t sg2_bilevel_pass_workspace_bytes(const SgDims* dims, int num_tensors, const int64_t* numels);
 int sg2_bilevel_pass_begin(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, void* workspace,
                            size_t workspace_bytes, void* stream);

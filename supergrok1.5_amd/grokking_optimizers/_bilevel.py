@@ -236,7 +236,8 @@ EARLY_ELEMENTS = 1 << 25
 
 def begin_pass(mn, grads, sharps, gru_states, mamba_fwd, mamba_bwd, exact_sharpness=False):
     """The part of accumulate_meta_gradients that needs no cotangents (sort and scan: sg2_bilevel_pass_begin), enqueued on
-    the current stream: what its `begun` takes, or None for nets and tensors that the pass is not built for."""
+    the current stream: what its `begun` takes, or None for nets and tensors that the pass is not built for.  The tensors and the weights have to
+    keep their values until then: a backward pass in between may write into .grad, so hand over copies."""
     if not (_pass_fits(mn) and all(m is not None for m in mamba_fwd) and all(m is not None for m in mamba_bwd)):
         return None
     return _ops.supergrok2_bilevel_begin(grads, sharps, gru_states, mamba_fwd, mamba_bwd, mn.flat_weights(), exact_sharpness,
