@@ -86,7 +86,8 @@ __device__ __forceinline__ void compose_block(const Plan& pl, int threads) {
     __syncthreads();
     // How many steps the first block of a chunk summary should cover: what the slowest pair of either direction needs
     // to contract at the step size a zero input gives (sg2_contraction_steps, sg2_first_block_steps).
-    // For sg2_poly_ok: the largest -A/2 and the largest |rotation frequency| of each direction.
+    // For sg2_poly_ok: the largest rate at which a pair's A_bar follows its step size (sg2_abar_rate) and the largest
+    // |rotation frequency| of each direction.
     for (int t = tid; t < 2 * ROWS * G::HP; t += threads) {
         const int d = t / (ROWS * G::HP), j = t / G::HP % ROWS, p = t % G::HP;
         const float* alog = pl.W.w[d ? W_B_ALOG : W_F_ALOG] + j * G::DS;
@@ -94,7 +95,7 @@ __device__ __forceinline__ void compose_block(const Plan& pl, int threads) {
         const int n = sg2_contraction_steps(s_dt0[d][j], a_e, a_o);
         if (n == 0) atomicOr(&s_zero, 1);
         atomicMax(&s_largest, n);
-        atomicMax(&s_amax[d], sg_f2i(sg_max(a_e, a_o)));
+        atomicMax(&s_amax[d], sg_f2i(sg_max(sg2_abar_rate(s_dt0[d][j], a_e), sg2_abar_rate(s_dt0[d][j], a_o))));
         atomicMax(&s_fmax[d], sg_f2i(sg_abs(pl.W.w[d ? W_B_ROPE : W_F_ROPE][j * G::HP + p])));
     }
     __syncthreads();
