@@ -187,6 +187,20 @@ SG_HD void sg2_pair_products(float dt0, float nhA_e, float nhA_o, float f, float
     sg2_prod_poly(po, qs, k + 9);
 }
 
+/* What eight steps multiply the 2x2 part of a pair by at most while |dt - dt0| < d_max: rotations preserve length, so a
+ * step shrinks it by max(|A_bar_e|, |A_bar_o|), and |A_bar(dt) - A_bar(dt0)| <= 2 r x / (1 - x) with x = a r |dt - dt0|
+ * (at most 2^-7.5 / 2.3 where the products are in use, d_max = 1 / (416 (a r)_max + 184 f_max): 2.1 covers the quotient). */
+SG_HD float sg2_abar_bound(float dt0, float nhA, float d_max) {
+    const float r = sg_rcp_pos(sg_fma(dt0, nhA, 1.0f));
+    return sg_abs(sg_fma(2.0f, r, -1.0f)) + (2.1f * d_max) * ((nhA * r) * r);
+}
+SG_HD float sg2_shrink8(float dt0, float nhA_e, float nhA_o, float d_max) {
+    float m = sg_max(sg2_abar_bound(dt0, nhA_e, d_max), sg2_abar_bound(dt0, nhA_o, d_max));
+    m = m * m;
+    m = m * m;
+    return m * m;
+}
+
 /* value of a composed output for one element */
 SG_HD float sg2_comp_eval(const float* c, float g, float s) { return sg_fma(c[0], g, sg_fma(c[1], s, c[2])); }
 

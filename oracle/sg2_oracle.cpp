@@ -62,7 +62,8 @@
  * Before that walk a windowed summary makes one cheaper attempt: a single block whose length comes from the weights
  * alone (the steps the slowest RoPE pair needs to contract below 2^-64 at the step size of a zero input, plus a
  * margin: sg2_first_block_steps in include/sg2_compose.h), walked with the state part only, while the 2x2 part is
- * bounded by the running product of max(|A_bar_e|, |A_bar_o|) (rotations preserve length).  If the bound is below
+ * bounded by the running product of max(|A_bar_e|, |A_bar_o|) (rotations preserve length), or of its bound over eight steps
+ * (sg2_shrink8) in tiles that take the products of the replay.  If the bound is below
  * 2^-64 in every (j,p) the summary is (0, b) with that block's b; otherwise the walk above starts from scratch.
  * Step size and gate of a 64-step tile (fp32 policy, as the kernels): when every timestep of the tile has
  * cmax_g |g| + cmax_s |s| < 2^-5 (cmax: the largest |c_g|, |c_s| of the composed dt and gate rows of the
@@ -259,6 +260,8 @@ struct DirW {
      * (sg2_pair_products), and the factors of their limit */
     std::vector<float> lane_prod;
     float kprod[2];
+    /* what eight steps on the products shrink a (column, pair)'s 2x2 part by at least (sg2_shrink8) */
+    std::vector<float> shrink8;
 };
 
 template <class O>
@@ -331,12 +334,15 @@ struct TileCoef {
     std::vector<char> prod_block;
 };
 enum { ORC_TILE = 64, ORC_BLOCK = 8, ORC_WAVE = 64 };
+/* general walk of a summary, its first attempt (state part only), output pass */
+enum Pass { PASS_SUMMARY, PASS_LITE, PASS_OUTPUT };
 
 template <class O>
 void tile_coefficients(const Dims& d, const DirW<O>& w, const std::vector<typename O::R>& A, const typename O::R* x,
-                       const float* gs, int64_t N, bool reverse, int64_t u0, int cnt, bool need_zc, TileCoef<O>& tc) {
+                       const float* gs, int64_t N, bool reverse, int64_t u0, int cnt, Pass pass, TileCoef<O>& tc) {
     typedef typename O::R R;
     const int dm = d.d_model, di = d.d_inner, ds = d.d_state, hp = ds / 2, lanes = di * hp;
+    const bool need_zc = pass == PASS_OUTPUT;
     tc.sp.resize(ORC_TILE);
     tc.ae.resize((size_t)ORC_TILE * lanes);
     tc.ao.resize((size_t)ORC_TILE * lanes);
@@ -357,35 +363,39 @@ void tile_coefficients(const Dims& d, const DirW<O>& w, const std::vector<typena
                           &tc.cs[(size_t)k * lanes + j * hp + p]);
     }
     /* blocks of 8 steps whose timesteps all pass sg2_poly_ok take A_bar, sin and cos from the lane polynomials (summary
-     * pass) or, with the tighter limit of the output pass (need_zc), the four products of the update */
+     * pass) or, with the tighter limit of the output pass, the four products of the update.  A tile on Taylor step sizes
+     * whose timesteps all pass the limit of the products takes them in every block: in the output pass also in the partial
+     * one at the end of a tensor, in the first attempt of a summary (which otherwise goes by the summary's limits) where
+     * it consists of whole blocks. */
     std::vector<char> poly_block(ORC_TILE / ORC_BLOCK, 0);
     tc.prod_block.assign(ORC_TILE / ORC_BLOCK, 0);
     if (sizeof(R) == 4) {
-        const float* lim = need_zc ? w.kprod : w.kpoly;
-        /* (the device knows before its projections whether the whole 64-step tile qualifies) */
-        bool whole_tile_poly = taylor && cnt == ORC_TILE;
-        for (int k = 0; k < cnt && whole_tile_poly; k++) {
+        bool whole = taylor && pass != PASS_SUMMARY && (pass == PASS_OUTPUT || cnt % ORC_BLOCK == 0);
+        for (int k = 0; k < cnt && whole; k++) {
             const int64_t u = u0 + k, t = reverse ? (N - 1 - u) : u;
-            whole_tile_poly = sg2_poly_ok(lim[0], lim[1], gs[2 * t], gs[2 * t + 1]) != 0;
+            whole = sg2_poly_ok(w.kprod[0], w.kprod[1], gs[2 * t], gs[2 * t + 1]) != 0;
         }
-        for (int b0 = 0; b0 + ORC_BLOCK <= cnt; b0 += ORC_BLOCK) {
+        const bool products = need_zc || whole;
+        const float* lim = products ? w.kprod : w.kpoly;
+        for (int b0 = 0; b0 + (whole ? 0 : ORC_BLOCK - 1) < cnt; b0 += ORC_BLOCK) {
+            const int len = std::min((int)ORC_BLOCK, cnt - b0);
             bool ok = true;
-            for (int q = 0; q < ORC_BLOCK && ok; q++) {
+            for (int q = 0; q < len && ok; q++) {
                 const int64_t u = u0 + b0 + q, t = reverse ? (N - 1 - u) : u;
                 ok = sg2_poly_ok(lim[0], lim[1], gs[2 * t], gs[2 * t + 1]) != 0;
             }
             poly_block[b0 / ORC_BLOCK] = ok;
             if (!ok) continue;
-            if (need_zc) {
+            if (products) {
                 tc.prod_block[b0 / ORC_BLOCK] = 1;
-                /* the linear parts alone: a whole tile on Taylor step sizes and products, and this block's inputs
-                 * SG2_PROD_LINEAR_FACTOR times further inside the limit */
-                bool linear = whole_tile_poly;
-                for (int q = 0; q < ORC_BLOCK && linear; q++) {
+                /* the linear parts alone: such a tile, and this block's (whole) inputs SG2_PROD_LINEAR_FACTOR times further
+                 * inside the limit */
+                bool linear = whole && len == ORC_BLOCK;
+                for (int q = 0; q < len && linear; q++) {
                     const int64_t u = u0 + b0 + q, t = reverse ? (N - 1 - u) : u;
                     linear = sg2_poly_ok(SG2_PROD_LINEAR_FACTOR * lim[0], SG2_PROD_LINEAR_FACTOR * lim[1], gs[2 * t], gs[2 * t + 1]) != 0;
                 }
-                for (int q = 0; q < ORC_BLOCK; q++)
+                for (int q = 0; q < len; q++)
                     for (int l = 0; l < lanes; l++) {
                         const float* k = &w.lane_prod[(size_t)l * 12];
                         const float dd = (float)tc.sp[b0 + q].dt[l / hp] - w.tay[((size_t)0 * w.comp_rows + l / hp) * 4];
@@ -463,7 +473,7 @@ void tile_coefficients(const Dims& d, const DirW<O>& w, const std::vector<typena
             }
         }
     }
-    for (; k0 < cnt; k0++)
+    for (; k0 < cnt && !poly_block[k0 / ORC_BLOCK]; k0++)
         for (int j = 0; j < di; j++)
             for (int p = 0; p < hp; p++)
                 O::abar_pair(tc.sp[k0].dt[j], A[j * ds + 2 * p], A[j * ds + 2 * p + 1], &tc.ae[(size_t)k0 * lanes + j * hp + p],
@@ -510,7 +520,7 @@ void scan_dir(const Dims& d, const DirW<O>& w, const typename O::R* x, const flo
             }
             for (int64_t tile0 = u1 - first_block; tile0 < u1; tile0 += ORC_TILE) {
                 const int cnt = (int)std::min<int64_t>(ORC_TILE, u1 - tile0);
-                tile_coefficients<O>(d, w, A, x, gs, N, reverse, tile0, cnt, false, tc);
+                tile_coefficients<O>(d, w, A, x, gs, N, reverse, tile0, cnt, PASS_LITE, tc);
                 for (int k = 0; k < cnt; k++) {
                     const StepProj<O>& sp = tc.sp[k];
                     for (int j = 0; j < di; j++) {
@@ -520,9 +530,15 @@ void scan_dir(const Dims& d, const DirW<O>& w, const typename O::R* x, const flo
                             const R ae = tc.ae[li], ao = tc.ao[li], sn = tc.sn[li], cs = tc.cs[li];
                             const R ux = dt * xb, be = ux * sp.B[2 * p], bo = ux * sp.B[2 * p + 1];
                             R* m = &sm[(j * hp + p) * 6];
+                            const R ve = m[4], vo = m[5];
+                            if (tc.prod_block[k / ORC_BLOCK]) {      /* ae = P1, sn = N2, ao = P3, cs = P4 */
+                                m[4] = O::fma(ae, ve, O::fma(sn, vo, be));
+                                m[5] = O::fma(ao, vo, O::fma(cs, ve, bo));
+                                if (k % ORC_BLOCK == ORC_BLOCK - 1) bound[j * hp + p] = bound[j * hp + p] * (R)w.shrink8[j * hp + p];
+                                continue;
+                            }
                             const R abs_e = ae < 0 ? -ae : ae, abs_o = ao < 0 ? -ao : ao;
                             bound[j * hp + p] = bound[j * hp + p] * (abs_e > abs_o ? abs_e : abs_o);
-                            const R ve = m[4], vo = m[5];
                             const R re = O::fma(ve, cs, -(vo * sn));
                             const R ro = O::fma(vo, cs, ve * sn);
                             m[4] = O::fma(ae, re, be);
@@ -542,7 +558,7 @@ void scan_dir(const Dims& d, const DirW<O>& w, const typename O::R* x, const flo
             }
             for (int64_t tile0 = blk_first; tile0 < blk_end; tile0 += ORC_TILE) {
                 const int cnt = (int)std::min<int64_t>(ORC_TILE, blk_end - tile0);
-                tile_coefficients<O>(d, w, A, x, gs, N, reverse, tile0, cnt, false, tc);
+                tile_coefficients<O>(d, w, A, x, gs, N, reverse, tile0, cnt, PASS_SUMMARY, tc);
                 for (int k = 0; k < cnt; k++) {
                     const StepProj<O>& sp = tc.sp[k];
                     for (int j = 0; j < di; j++) {
@@ -618,7 +634,7 @@ void scan_dir(const Dims& d, const DirW<O>& w, const typename O::R* x, const flo
         const int64_t u_end = std::min<int64_t>((c + 1) * chunk_len, N);
         for (int64_t tile0 = c * chunk_len; tile0 < u_end; tile0 += ORC_TILE) {
             const int cnt = (int)std::min<int64_t>(ORC_TILE, u_end - tile0);
-            tile_coefficients<O>(d, w, A, x, gs, N, reverse, tile0, cnt, true, tc);
+            tile_coefficients<O>(d, w, A, x, gs, N, reverse, tile0, cnt, PASS_OUTPUT, tc);
             for (int k = 0; k < cnt; k++) {
                 const int64_t u = tile0 + k, t = reverse ? (N - 1 - u) : u;
                 const StepProj<O>& sp = tc.sp[k];
@@ -767,7 +783,13 @@ int step_tensor(const Dims& d, const float* const* W, int64_t chunk_len, int64_t
             const float kp = sg2_limit_factor(sg_max(128.0f * amax, 256.0f * fmax), slope);
             w.kpoly[0] = kp * cdt[0];
             w.kpoly[1] = kp * cdt[1];
-            const float kq = sg2_limit_factor(sg_fma(416.0f, amax, 184.0f * fmax), slope);
+            const float kprod = sg_fma(416.0f, amax, 184.0f * fmax);
+            const float kq = sg2_limit_factor(kprod, slope);
+            w.shrink8.assign((size_t)di * hp, 0.0f);
+            for (int j = 0; j < di; j++)
+                for (int p = 0; p < hp; p++)
+                    w.shrink8[(size_t)j * hp + p] = sg2_shrink8(w.tay[((size_t)0 * w.comp_rows + j) * 4], -0.5f * -sg_exp(w.A_log[j * ds + 2 * p]),
+                                                                -0.5f * -sg_exp(w.A_log[j * ds + 2 * p + 1]), 1.0f / kprod);
             w.kprod[0] = kq * cdt[0];
             w.kprod[1] = kq * cdt[1];
         }

@@ -816,7 +816,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 }
 
 // ---- the gradients with the gradient of the input projection, chunk by chunk: one 128-lane workgroup per (chunk,
-// direction), lane (j,p) owning column j and RoPE pair p as in k_scan
+// direction), lane (j,p) owning column j and RoPE pair p
 __global__ __launch_bounds__(SCAN_THREADS) void k_bilevel_backward(Plan pl, AdjIO io) {
     constexpr bool DX = true;
     extern __shared__ __attribute__((aligned(16))) float lds[];

@@ -112,7 +112,9 @@ __device__ __forceinline__ void compose_block(const Plan& pl, int threads) {
             cmax[4 + 2 * k] = kp * sg_i2f(s_cdt[k][0]);
             cmax[5 + 2 * k] = kp * sg_i2f(s_cdt[k][1]);
             // ... and for the products of the output pass (sg2_pair_products)
-            const float kq = sg2_limit_factor(sg_fma(416.0f, sg_i2f(s_amax[k]), 184.0f * sg_i2f(s_fmax[k])), slope);
+            const float kprod = sg_fma(416.0f, sg_i2f(s_amax[k]), 184.0f * sg_i2f(s_fmax[k]));
+            const float kq = sg2_limit_factor(kprod, slope);
+            cmax[16 + k] = 1.0f / kprod;                // how far dt can be from dt0 there (sg2_shrink8)
             cmax[8 + 2 * k] = kq * sg_i2f(s_cdt[k][0]);
             cmax[9 + 2 * k] = kq * sg_i2f(s_cdt[k][1]);
             // ... and for the polynomials of the adjoint (sg2_bilevel.hip)

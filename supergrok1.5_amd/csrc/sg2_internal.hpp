@@ -118,7 +118,7 @@ struct Plan {
                                    // entries of the kernel geometry beyond them read as 0 and are not stored)
     SgDims dims;                   // the caller's dimensions (what k_elem_any indexes the per-element weights with)
     int chunk_len;
-    int window;                    // summary window (0: whole chunk), see k_scan<false>
+    int window;                    // summary window (0: whole chunk), see k_summary
     uint32_t* keys[2];
     int32_t* vals[2];              // element index within the tensor | sign bit of the gradient in bit 31
     float* ssorted;                // [total] sharpness gathered into sorted order

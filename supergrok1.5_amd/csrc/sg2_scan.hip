@@ -8,10 +8,9 @@
 //
 // The sorted sequence of a tensor is cut into chunks of chunk_len timesteps
 // (scan order: t ascending for the forward direction, descending for the
-// backward one).  One workgroup of d_inner * d_state/2 lanes (128 for the default
-// geometry, 512 for the large one) owns one chunk; lane (j,p) owns column j and
-// RoPE pair p, i.e. the two states h[j][2p], h[j][2p+1].
-//   k_scan<false>  every chunk but the last of a tensor: 2x2 affine summary
+// backward one).  One workgroup owns one chunk: one wave for the default geometry, four for
+// the large one; a lane owns one RoPE pair p of two columns j, i.e. the states h[j][2p], h[j][2p+1] of both.
+//   k_summary      every chunk but the last of a tensor: 2x2 affine summary
 //                  (M,b) of the chunk, accumulated from the identity.  The
 //                  recurrence contracts (|A_bar| < 1), so the chunk is walked
 //                  backwards in blocks of `window` steps and the walk stops as
@@ -23,9 +22,9 @@
 //   k_chunk_prefix start state of each chunk: summaries applied in order to
 //                  the carried state of the tensor.
 //   k_replay       every chunk replayed from its start state: y = h.C, gate,
-//   (k_scan<true>  D skip, out_proj, and the 8-float context written straight
-//   for the large  to the element's original position (the "unsort").  The
-//   geometry)      last chunk stores the new carried state.
+//   (k_replay_wide D skip, out_proj, and the 8-float (16-float) context written
+//   for the large  straight to the element's original position (the "unsort").
+//   geometry)      The last chunk stores the new carried state.
 //   compose_block  (sg2_compose_block.hpp) runs beside the sort's first kernel: the input of a timestep is two numbers (g, s)
 //                  and every projection of the block is linear in their 8-float
 //                  input projection, so input_proj, in_proj, dt_proj, B_proj and
@@ -53,7 +52,9 @@
 // and the CPU checker makes the same one).
 // Where the inputs are small (the usual case: sg2_taylor_ok, sg2_poly_ok in sg2_compose.h) the step size and the gate
 // of a tile come from cubic Taylor polynomials around their zero-input arguments, and A_bar, sin and cos of a block
-// from per-lane polynomials in dt - dt0; the forms above serve the remaining tiles and blocks.
+// from per-lane polynomials in dt - dt0; the forms above serve the remaining tiles and blocks.  The ragged tile at the end
+// of a tensor takes the polynomials like any other (its missing steps are zero inputs whose effect on the state is taken
+// back): single steps with their own divisions were 10 % of a step whose tensors are all below 256 elements.
 // For the bilevel pass k_replay<G, true> also stores the state entering every
 // HT_STEP-th step (Plan::htile), which the adjoint kernels restart from.
 #include <type_traits>
@@ -73,16 +74,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int UB = SG2_SCAN_UB;           // timesteps per unrolled block of the recurrence
 static_assert(UB % 4 == 0 && SCAN_TT % UB == 0 && SCAN_TT == 64, "blocks are fetched 4 timesteps per LDS read; one ballot covers a tile");
 static_assert(HT_STEP % UB == 0 && SCAN_TT % HT_STEP == 0, "kept states fall on block borders");
-// Three waves per SIMD (168 VGPRs) is where the default geometry's kernels stop gaining from occupancy; keep the
-// register allocation from drifting just past that boundary.  The large geometry's workgroup is two waves per SIMD by itself,
-// and at 128 VGPRs (two workgroups per CU) the recurrence spills: one workgroup per CU, up to 256 VGPRs.
-#ifndef SG2_SCAN_WAVES
-#define SG2_SCAN_WAVES 3
-#endif
-template <class G>
-constexpr int scan_waves() { return G::PARTS == 2 ? SG2_SCAN_WAVES : 2; }
-#define SG2_SCAN_ATTR __attribute__((amdgpu_waves_per_eu(scan_waves<G>(), scan_waves<G>())))
-
 template <int HP>
 __device__ __forceinline__ float pair_tree_max(float f) {
     f = sg_max(f, dpp_quad_swap1(f));
@@ -90,116 +81,6 @@ __device__ __forceinline__ float pair_tree_max(float f) {
     f = sg_max(f, dpp_half_mirror(f));
     if (HP == 16) f = sg_max(f, dpp_row_mirror(f));
     return f;
-}
-
-// Projections of one timestep from the element's (g, s).  Each wave of the workgroup produces its
-// share (rows PART*n/PARTS ...) of dt / dt*x-branch / B (/ D*x-branch / C / gate).  PART is a template parameter so that every row
-// index is a compile-time constant; a caller with many waves passes PART = 0 and array pointers moved to its wave's first row.  The coefficient triple of an output row sits in the four padding floats of the
-// LDS row it produces (staged once per workgroup, see stage_coefficients): one 16-byte broadcast read per output,
-// no scalar loads in the loop (a scalar load can only be waited for with lgkmcnt(0), which also drains the LDS queue).
-// Returns bit 0: every rotation angle of this timestep, over this half's columns, is small enough for
-// sg_sincos_small; bit 1: small enough for sg_sincos_tiny (fmax: per column, the largest |rope frequency| of its 8 pairs; dt >= 0 and
-// rounding is monotone, so dt*fmax < limit is the same statement as |dt*freq| < limit for all pairs).
-// TAYLOR: every timestep of the tile has passed sg2_taylor_ok: step size and gate come from their cubic Taylor
-// polynomials.  Those cost no LDS of their own in the output pass (the workgroup's LDS is what limits it to six per CU):
-// the step-size polynomial of column j sits in the padding of row j of s_dx, and the gate polynomial of column j
-// is spread over the fourth padding floats of rows j of s_dt, s_B, s_C and s_gate, which this wave reads anyway
-// (d_inner = d_state: the wave's columns and its rows of B and C carry the same indices).  The summary pass has
-// no s_dx and keeps the step-size polynomials in s_tay.
-// DSTORE (with TAYLOR, whole tiles whose blocks all run on the lane polynomials): the step-size row receives dt - dt0,
-// which is all those blocks want to know (one subtraction per column here instead of one per pair in the recurrence),
-// and nobody asks for the angle flags.
-template <class G, bool OUT, int PART, bool HAS_S, bool TAYLOR, bool DSTORE = false>
-__device__ __forceinline__ int project_tile(float g, float s, int tu, float* s_dt, float* s_ux, float* s_dx, float* s_B,
-                                             float* s_C, float* s_gate, const float* s_fmax, const float* s_tay) {
-    static_assert(G::DI == G::DS, "the gate polynomials ride on the rows of B and C");
-    auto delta = [&](const f32x4 t) { return HAS_S ? sg_fma(t[0], g, t[1] * s) : t[0] * g; };
-    auto poly = [&](const f32x4 t, float d) { return sg_fma(sg_fma(sg_fma(t[3], d, t[2]), d, t[1]), d, t[0]); };
-    // HAS_S is false for a tensor whose sharpness is all zero: fma(c_s, 0, c_0) is c_0 itself, so the term is skipped
-    auto eval = [&](const f32x4 t) { return sg_fma(t[0], g, HAS_S ? sg_fma(t[1], s, t[2]) : t[2]); };
-    auto coef = [&](const float* arr, int row) { return *reinterpret_cast<const f32x4*>(arr + row * LDS_STRIDE + SCAN_TT); };
-    constexpr int NR = G::DI / G::PARTS;        // this wave's columns = its rows of B and C
-    float gp0[NR], gp1[NR], gp2[NR];            // first three coefficients of the gate polynomials, picked up on the way
-    bool small = true, tiny = true;
-#pragma unroll
-    for (int q = 0; q < NR; q++) {
-        const int jj = PART * NR + q;
-        const f32x4 cd = coef(s_dt, jj);
-        gp0[q] = cd[3];
-        float dtv, dt0 = 0.0f;
-        if (TAYLOR) {
-            const f32x4 tp = OUT ? coef(s_dx, jj) : *reinterpret_cast<const f32x4*>(s_tay + jj * 4);
-            dtv = poly(tp, delta(cd));
-            dt0 = tp[0];
-        } else {
-            dtv = sg_softplus(eval(cd));
-        }
-        if (!DSTORE) {
-            const float amax = dtv * s_fmax[jj];
-            small = small && (amax < SG_SINCOS_SMALL_LIMIT);
-            tiny = tiny && (amax < SG_SINCOS_TINY_LIMIT);
-        }
-        const f32x4 cx = coef(s_ux, jj);              // x-branch coefficients; [3] = D of this column
-        const float xbv = eval(cx);
-        s_dt[jj * LDS_STRIDE + tu] = DSTORE ? dtv - dt0 : dtv;
-        s_ux[jj * LDS_STRIDE + tu] = dtv * xbv;
-        if (OUT) s_dx[jj * LDS_STRIDE + tu] = cx[3] * xbv;
-    }
-#pragma unroll
-    for (int q = 0; q < NR; q++) {
-        const int ss = PART * NR + q;
-        const f32x4 cb = coef(s_B, ss);
-        gp1[q] = cb[3];
-        s_B[ss * LDS_STRIDE + tu] = eval(cb);
-        if (OUT) {
-            const f32x4 cc = coef(s_C, ss);
-            gp2[q] = cc[3];
-            s_C[ss * LDS_STRIDE + tu] = eval(cc);
-        }
-    }
-    if (OUT) {
-        // the gates of this wave's columns share one reciprocal (sg_silu_block)
-        static_assert(NR <= 8, "sg_silu_block takes at most 8 values");
-        float zv[NR], gv[NR];
-        if (TAYLOR) {
-#pragma unroll
-            for (int q = 0; q < NR; q++) {
-                const f32x4 cz = coef(s_gate, PART * NR + q);
-                gv[q] = poly(f32x4{gp0[q], gp1[q], gp2[q], cz[3]}, delta(cz));
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < NR; q++) zv[q] = eval(coef(s_gate, PART * NR + q));
-            sg_silu_block(NR, zv, gv);
-        }
-#pragma unroll
-        for (int q = 0; q < NR; q++) s_gate[(PART * NR + q) * LDS_STRIDE + tu] = gv[q];
-    }
-    return (small ? 1 : 0) | (tiny ? 2 : 0);
-}
-
-// Once per workgroup: the composed coefficient triples of this direction (and D) into the padding of the LDS rows.
-// tay: this direction's Taylor polynomials, [step size | gate][row][4] (see project_tile for where they go).
-template <class G, bool OUT>
-__device__ __forceinline__ void stage_coefficients(const float* __restrict__ comp, const float* __restrict__ tay, const float* __restrict__ Dw,
-                                                   int tid, float* s_dt, float* s_ux, float* s_dx, float* s_B, float* s_C, float* s_gate,
-                                                   float* s_tay) {
-    static_assert(SG2_COMP_GROUPS * G::ROWS <= G::THREADS && G::ROWS == G::DI, "one thread per (group, row)");
-    if (tid < SG2_COMP_GROUPS * G::ROWS) {
-        const int group = tid / G::ROWS, row = tid % G::ROWS;
-        float* arr = group == SG2_COMP_XB ? s_ux : group == SG2_COMP_DT ? s_dt : group == SG2_COMP_B ? s_B : group == SG2_COMP_C ? s_C : s_gate;
-        if (OUT || (group != SG2_COMP_C && group != SG2_COMP_Z)) {
-            const float* t = comp + (group * G::ROWS + row) * 3;
-            // fourth float: D next to the x-branch triple; coefficient 0, 1, 2, 3 of the row's gate polynomial next to dt, B, C, z
-            const float* gp = tay + (G::ROWS + row) * 4;
-            const float w = group == SG2_COMP_XB ? Dw[row] : !OUT ? 0.0f : group == SG2_COMP_DT ? gp[0] : group == SG2_COMP_B ? gp[1] : group == SG2_COMP_C ? gp[2] : gp[3];
-            *reinterpret_cast<f32x4*>(arr + row * LDS_STRIDE + SCAN_TT) = f32x4{t[0], t[1], t[2], w};
-        }
-        if (group == SG2_COMP_DT) {
-            const float* dp = tay + row * 4;
-            *reinterpret_cast<f32x4*>(OUT ? s_dx + row * LDS_STRIDE + SCAN_TT : s_tay + row * 4) = f32x4{dp[0], dp[1], dp[2], dp[3]};
-        }
-    }
 }
 
 // scan state of one lane: OUT -> (he,ho) only; summary -> also the two columns of M
@@ -242,9 +123,7 @@ __device__ __forceinline__ void step_update(LaneState& S, float ae, float ao, fl
 // (sg_abar_block_*) unless some lane of the wave has a product of denominators too large for it.
 // ANGLE: 0 full sin/cos, 1 sg_sincos_small (bit-identical to 0), 2 sg_sincos_tiny_dt (its own values, polynomials in dt),
 // 3: every timestep of the block has passed sg2_poly_ok: A_bar, sin and cos from the lane's polynomials in dt - dt0.
-// DGIVEN (ANGLE 3 only): dt[] holds dt - dt0 already (project_tile's DSTORE).  LINEAR (output pass, ANGLE 3): the
-// inputs are small enough for the linear parts of the products.
-template <int HP, bool OUT, int ANGLE, bool LITE = false, bool DGIVEN = false, bool LINEAR = false>
+template <int HP, bool OUT, int ANGLE, bool LITE = false>
 __device__ __forceinline__ void block_steps(LaneState& S, const float (&dt)[UB], const float (&ux)[UB], const float (&Be)[UB],
                                             const float (&Bo)[UB], const float (&Ce)[UB], const float (&Co)[UB], float hAe,
                                             float hAo, float freq, const LanePoly<OUT>& LP, float (&y)[UB]) {
@@ -253,16 +132,16 @@ __device__ __forceinline__ void block_steps(LaneState& S, const float (&dt)[UB],
         // the four products of the update as quadratics: ae = P1, sn = N2, ao = P3, cs = P4 (see the update below)
 #pragma unroll
         for (int u = 0; u < UB; u++) {
-            const float d = DGIVEN ? dt[u] : dt[u] - LP.dt0;
-            ae[u] = LINEAR ? sg2_poly1(LP.k, d) : sg2_poly2(LP.k, d);
-            sn[u] = LINEAR ? sg2_poly1(LP.k + 3, d) : sg2_poly2(LP.k + 3, d);
-            ao[u] = LINEAR ? sg2_poly1(LP.k + 6, d) : sg2_poly2(LP.k + 6, d);
-            cs[u] = LINEAR ? sg2_poly1(LP.k + 9, d) : sg2_poly2(LP.k + 9, d);
+            const float d = dt[u] - LP.dt0;
+            ae[u] = sg2_poly2(LP.k, d);
+            sn[u] = sg2_poly2(LP.k + 3, d);
+            ao[u] = sg2_poly2(LP.k + 6, d);
+            cs[u] = sg2_poly2(LP.k + 9, d);
         }
     } else if constexpr (ANGLE == 3) {
 #pragma unroll
         for (int u = 0; u < UB; u++) {
-            const float d = DGIVEN ? dt[u] : dt[u] - LP.dt0;
+            const float d = dt[u] - LP.dt0;
             ae[u] = sg2_poly3(LP.pe, d);
             ao[u] = sg2_poly3(LP.po, d);
             sn[u] = sg2_poly2(LP.qs, d);
@@ -305,366 +184,47 @@ __device__ __forceinline__ void block_steps(LaneState& S, const float (&dt)[UB],
     }
 }
 
-template <class G, bool OUT>
-__global__ __launch_bounds__(G::THREADS) SG2_SCAN_ATTR void k_scan(Plan pl) {
-    constexpr int DM = G::DM, DS = G::DS, DI = G::DI, HP = G::HP, SCAN_THREADS = G::THREADS, PARTS = G::PARTS;
-    __shared__ __attribute__((aligned(16))) float s_dt[DI * LDS_STRIDE];
-    __shared__ __attribute__((aligned(16))) float s_ux[DI * LDS_STRIDE];       // dt * x-branch
-    __shared__ __attribute__((aligned(16))) float s_B[DS * LDS_STRIDE];
-    __shared__ __attribute__((aligned(16))) float s_C[OUT ? DS * LDS_STRIDE : 1];
-    __shared__ __attribute__((aligned(16))) float s_gate[OUT ? DI * LDS_STRIDE : 1];
-    __shared__ __attribute__((aligned(16))) float s_dx[OUT ? DI * LDS_STRIDE : 1];   // D * x-branch (skip term)
-    // y of column j goes where dt of column j was: both are touched only by the 8 lanes of column j, in program order
-    float* const s_y = s_dt;
-    __shared__ float s_fmax[DI];
-    __shared__ __attribute__((aligned(16))) float s_tay[OUT ? 4 : DI * 4];   // summary pass: Taylor polynomials of the step size (the output pass keeps its own in row padding)
-    __shared__ __attribute__((aligned(16))) float s_wout[OUT ? DM * DI : 4];      // out_proj of this direction
-    __shared__ unsigned long long s_large[PARTS];      // per wave's share of the columns: bit t set = timestep t of the tile needs the full sin/cos
-    __shared__ unsigned long long s_nottiny[PARTS];    // ... bit t set = timestep t is not eligible for sg_sincos_tiny
+// How the waves of a chunk share its recurrences: a lane owns one RoPE pair of two columns, so a chunk takes
+// THREADS / 128 waves (one for the default geometry, four for the large one), wave w the columns CPW w .. CPW w + CPW - 1:
+// lane (jl, p) = (lane / HP, lane % HP) pair p of columns CPW w + jl and CPW w + CPH + jl.
+template <class G>
+struct Split {
+    static constexpr int WAVES = G::THREADS / 128;
+    static constexpr int CPW = G::DI / WAVES;       // columns (and rows of B and C) of a wave
+    static constexpr int CPH = CPW / 2;             // ... of one of a lane's two columns over the lanes
+    static constexpr int SPL = CPW;                 // row owners: lane (row r, part q) takes SPL consecutive timesteps of row r
+    static_assert(CPH * G::HP == 64 && G::DI == G::DS && SPL * (64 / CPW) == SCAN_TT && SPL % 4 == 0, "64 lanes: CPH columns x HP pairs, CPW rows x parts");
+};
+// Where row r of B or C lies: the even rows first.  The lanes of a wave read rows 2 p and 2 p + 1 of all pairs p; with 16 pairs
+// the even rows in their own order would start 8 banks apart and meet on half of them.
+template <class G>
+__device__ __forceinline__ int bc_slot(int r) { return (r & 1) * G::HP + (r >> 1); }
 
-    const int per_dir = OUT ? pl.chunks : pl.wchunks;
-    const int dir = (int)blockIdx.x >= per_dir ? 1 : 0;
-    const int cidx = (int)blockIdx.x - dir * per_dir;
-    const sg::cint_p prefix = sg::as_const(OUT ? pl.chunk_prefix : pl.wchunk_prefix);
-    const sg::Seg seg = sg::find_seg(prefix, pl.P, cidx);
-    const int ti = seg.i;
-    const int c = cidx - seg.first;                        // chunk within the tensor
-    const TensorDev& T = pl.tensors[ti];
-    const int N = T.numel, off = T.off;
-    const int u0 = c * pl.chunk_len;                       // first scan step of the chunk
-    const int u1 = min(u0 + pl.chunk_len, N);
-    const uint32_t* __restrict__ skey = pl.keys[0] + off;      // sorted |g| bits
-    const int32_t* __restrict__ sval = pl.vals[0] + off;       // element index | sign of g
-    const float* __restrict__ ssrt = pl.ssorted + off;          // sharpness in sorted order
-    const bool has_s = __builtin_amdgcn_readfirstlane(pl.sharp_nonzero[ti]) != 0;
-
-    const int tid = threadIdx.x;
-    const int tu = tid & (SCAN_TT - 1);                                   // projection role: timestep of the tile
-    const int half = __builtin_amdgcn_readfirstlane(tid >> 6);           // projection role: which share of the outputs (the wave)
-    const int j = tid / HP, p = tid % HP;                                 // scan role
-
-    // -A/2 with A = -exp(A_log): the two poles of this lane's pair
-    // (formed again from the weights wherever a block or a ragged end needs them: the usual blocks run on the lane
-    // polynomials below, and three registers held for the exceptions would spill)
-    auto pole_e = [&]() { return -0.5f * -sg_exp(pl.W.w[dir ? W_B_ALOG : W_F_ALOG][j * DS + 2 * p]); };
-    auto pole_o = [&]() { return -0.5f * -sg_exp(pl.W.w[dir ? W_B_ALOG : W_F_ALOG][j * DS + 2 * p + 1]); };
-    auto rope_f = [&]() { return pl.W.w[dir ? W_B_ROPE : W_F_ROPE][j * HP + p]; };
-    // this lane's pair as polynomials in dt - dt0, dt0 = the step size of its column for a zero input
-    LanePoly<OUT> LP;
-    LP.dt0 = pl.comp[2 * SG2_COMP_GROUPS * G::ROWS * 3 + dir * 2 * G::ROWS * 4 + j * 4];
-    if constexpr (OUT) {
-        sg2_pair_products(LP.dt0, pole_e(), pole_o(), rope_f(), LP.k);
-    } else {
-        sg2_abar_poly(LP.dt0, pole_e(), LP.pe);
-        sg2_abar_poly(LP.dt0, pole_o(), LP.po);
-        sg2_sincos_poly(LP.dt0, rope_f(), LP.qs, LP.qc);
-    }
-
-    {   // largest |frequency| of each column's pairs
-        const float f = pair_tree_max<HP>(sg_abs(rope_f()));
-        if (p == 0) s_fmax[j] = f;
-        stage_coefficients<G, OUT>(pl.comp + dir * (SG2_COMP_GROUPS * G::ROWS * 3), pl.comp + 2 * SG2_COMP_GROUPS * G::ROWS * 3 + dir * 2 * G::ROWS * 4,
-                                   pl.W.w[dir ? W_B_D : W_F_D], tid, s_dt, s_ux, s_dx, s_B, s_C, s_gate, s_tay);
-        static_assert(DM * DI == SCAN_THREADS, "one out_proj entry per thread");
-        if (OUT) s_wout[tid] = pl.W.w[dir ? W_B_OUT : W_F_OUT][tid];
-        __syncthreads();
-    }
-    // largest |c_g|, |c_s| over this direction's step-size and gate rows: what decides whether a tile may use the polynomials
-    const float cmax_g = sg::as_const(pl.comp)[2 * SG2_COMP_GROUPS * G::ROWS * 3 + 2 * 2 * G::ROWS * 4 + 2 * dir];
-    const float cmax_s = sg::as_const(pl.comp)[2 * SG2_COMP_GROUPS * G::ROWS * 3 + 2 * 2 * G::ROWS * 4 + 2 * dir + 1];
-    // ... and whether a block of the recurrence may use the lane polynomials (sg2_poly_ok)
-    // (the output pass with the tighter limit of its products)
-    const float kpoly_g = sg::as_const(pl.comp)[2 * SG2_COMP_GROUPS * G::ROWS * 3 + 2 * 2 * G::ROWS * 4 + (OUT ? 8 : 4) + 2 * dir];
-    const float kpoly_s = sg::as_const(pl.comp)[2 * SG2_COMP_GROUPS * G::ROWS * 3 + 2 * 2 * G::ROWS * 4 + (OUT ? 8 : 4) + 2 * dir + 1];
-
-    LaneState S = {0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 1.0f};
-    bool fully_contracted = false;      // summary pass: the walk stopped because the 2x2 part had contracted
-    if (OUT) {
-        // When every summary of this call has an exactly zero 2x2 part, a chunk's start state is the offset of the
-        // summary before it, whatever came earlier: k_chunk_prefix has then only placed the carried states (chunk 0).
-        if (c > 0 && __builtin_amdgcn_readfirstlane(*pl.contracted) != 0) {
-            const float* sm = pl.summaries + (size_t)(dir * pl.wchunks + pl.wchunk_prefix[ti] + c - 1) * 6 * SCAN_THREADS;
-            S.he = sm[4 * SCAN_THREADS + tid];
-            S.ho = sm[5 * SCAN_THREADS + tid];
-        } else if (T.nchunks == 1) {       // nothing before it: the carried state itself (no other workgroup writes it)
-            const float* st = dir ? T.mbwd : T.mfwd;
-            if (j < pl.st_di && 2 * p < pl.st_ds) {
-                S.he = st[j * pl.st_ds + 2 * p];
-                S.ho = st[j * pl.st_ds + 2 * p + 1];
-            }
-        } else {
-            const float* hs = pl.hstart + ((size_t)(dir * pl.chunks + cidx) * 2) * SCAN_THREADS;
-            S.he = hs[tid];
-            S.ho = hs[SCAN_THREADS + tid];
-        }
-    }
-
-    // Summary pass: the chunk is walked backwards in blocks of `window` steps.  Each block is summarised from the
-    // identity and the summary of everything after it (`late`) is applied on top; as soon as the 2x2 part of the
-    // running summary has contracted below 2^-64 the steps before the block cannot matter and the walk stops.
-    int blk_end = u1;
-    int blk_first = u0;
-    if (!OUT && pl.window > 0 && pl.window < pl.chunk_len) blk_first = max(u0, u1 - pl.window);
-    // First attempt: ONE block of as many steps as compose_block expects the slowest pair to need, walked with the state
-    // part only (LITE) and a bound on the 2x2 part in its place.  If the bound is below 2^-64 in every lane the summary
-    // is (0, b) as below; if not, the walk starts over in its general form.
-    bool lite = false;
-    if (!OUT && blk_first > u0) {
-        const int first_block = __builtin_amdgcn_readfirstlane(pl.contracted[1]);
-        if (first_block > 0 && u1 - first_block > u0) {
-            lite = true;
-            blk_first = u1 - first_block;
-        }
-    }
-    LaneState late = {0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 1.0f};
-    bool have_late = false;
-    // inputs of one tile (sorted |g| bits, payload, sorted sharpness) for this lane's timestep; zero beyond the block
-    uint32_t nx_key = 0;
-    int32_t nx_val = 0;
-    float nx_sh = 0.0f;
-    auto load_inputs = [&](int tile0) {
-        const int u = tile0 + tu;
-        if (u < blk_end) {
-            const int t = dir ? (N - 1 - u) : u;
-            nx_key = skey[t];
-            nx_val = sval[t];
-            nx_sh = has_s ? ssrt[t] : 0.0f;      // an all-zero tensor has no sorted copy of its sharpness (uniform branch)
-        }
-    };
-    for (;;) {
-    load_inputs(blk_first);
-    for (int tile0 = blk_first; tile0 < blk_end; tile0 += SCAN_TT) {
-        const int cnt = min(SCAN_TT, blk_end - tile0);
-        // ---------------- phase A: projections of SCAN_TT timesteps -> LDS
-        // this tile's inputs were requested one tile ago (or just before the loop); request the next tile's now
-        const uint32_t kbits = nx_key;
-        const int32_t v = nx_val;
-        const float shv = nx_sh;
-        const bool valid = tile0 + tu < blk_end;
-        if (tile0 + SCAN_TT < blk_end) load_inputs(tile0 + SCAN_TT);
-        int orig = v & 0x7fffffff;
-        orig = ((unsigned)orig < (unsigned)N) ? orig : 0;   // never index outside the tensor
-        const float g = valid ? sg_i2f((int32_t)kbits | (v & (int32_t)0x80000000)) : 0.0f;
-        const float sh = valid ? shv : 0.0f;
-        int angle_t;
-        bool dgiven = false;     // whole tile on the lane polynomials: phase A leaves dt - dt0 in place of dt
-        // bit t set = timestep t of the tile may not use the lane polynomials (the same mask in every wave: the same 64 timesteps)
-        const unsigned long long notpoly = __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kpoly_g, kpoly_s, g, sh));
-        // ... may not use the linear parts alone (output pass)
-        const unsigned long long notlin =
-            OUT ? __builtin_amdgcn_ballot_w64(!sg2_poly_ok(SG2_PROD_LINEAR_FACTOR * kpoly_g, SG2_PROD_LINEAR_FACTOR * kpoly_s, g, sh)) : ~0ull;
-        {
-            // the same 64 timesteps in every wave of the workgroup: the same decision without talking to one another
-            const bool tay = __builtin_amdgcn_ballot_w64(!sg2_taylor_ok(cmax_g, cmax_s, g, sh)) == 0;
-            dgiven = tay && notpoly == 0 && cnt == SCAN_TT;
-            // PARTS == 2: the wave's share is a template parameter; more waves: one copy of the code, the arrays moved to this wave's first row
-            const int rj = (PARTS == 2) ? 0 : half * (DI / PARTS) * LDS_STRIDE, rs = (PARTS == 2) ? 0 : half * (DS / PARTS) * LDS_STRIDE;
-            const int rt = (PARTS == 2 || OUT) ? 0 : half * (DI / PARTS) * 4;
-            auto run = [&](auto part_c, auto has_s_c, auto tay_c) {
-                if (decltype(tay_c)::value && dgiven)
-                    return project_tile<G, OUT, decltype(part_c)::value, decltype(has_s_c)::value, true, true>(
-                        g, sh, tu, s_dt + rj, s_ux + rj, s_dx + (OUT ? rj : 0), s_B + rs, s_C + (OUT ? rs : 0), s_gate + (OUT ? rj : 0),
-                        s_fmax + ((PARTS == 2) ? 0 : half * (DI / PARTS)), s_tay + rt);
-                return project_tile<G, OUT, decltype(part_c)::value, decltype(has_s_c)::value, decltype(tay_c)::value>(
-                    g, sh, tu, s_dt + rj, s_ux + rj, s_dx + (OUT ? rj : 0), s_B + rs, s_C + (OUT ? rs : 0), s_gate + (OUT ? rj : 0),
-                    s_fmax + ((PARTS == 2) ? 0 : half * (DI / PARTS)), s_tay + rt);
-            };
-            auto with_part = [&](auto has_s_c, auto tay_c) {
-                if (PARTS == 2 && half == 1) return run(std::integral_constant<int, (PARTS == 2) ? 1 : 0>{}, has_s_c, tay_c);
-                return run(std::integral_constant<int, 0>{}, has_s_c, tay_c);
-            };
-            if (tay) angle_t = has_s ? with_part(std::true_type{}, std::true_type{}) : with_part(std::false_type{}, std::true_type{});
-            else angle_t = has_s ? with_part(std::true_type{}, std::false_type{}) : with_part(std::false_type{}, std::false_type{});
-        }
-        {   // wave w projects the dt of columns w*64/HP .. (w+1)*64/HP-1, which are the columns it owns in the recurrence
-            const unsigned long long large = __builtin_amdgcn_ballot_w64(!(angle_t & 1));
-            const unsigned long long nottiny = __builtin_amdgcn_ballot_w64(!(angle_t & 2));
-            if (tu == 0) { s_large[half] = large; s_nottiny[half] = nottiny; }
-        }
-        __syncthreads();
-        // wave-uniform masks into scalar registers: the per-block tests below are then scalar instructions
-        auto uniform64 = [](unsigned long long v) {
-            const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v);
-            const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32));
-            return ((unsigned long long)hi << 32) | lo;
-        };
-        const unsigned long long large = uniform64(s_large[half]), nottiny = uniform64(s_nottiny[half]);
-
-        // ---------------- phase B: the recurrence over the tile, lane = (j,p)
-        const float* __restrict__ r_dt = s_dt + j * LDS_STRIDE;
-        const float* __restrict__ r_ux = s_ux + j * LDS_STRIDE;
-        const float* __restrict__ r_Be = s_B + (2 * p) * LDS_STRIDE;
-        const float* __restrict__ r_Bo = s_B + (2 * p + 1) * LDS_STRIDE;
-        const float* __restrict__ r_Ce = s_C + (OUT ? (2 * p) * LDS_STRIDE : 0);
-        const float* __restrict__ r_Co = s_C + (OUT ? (2 * p + 1) * LDS_STRIDE : 0);
-        int k0 = 0;
-        for (; k0 + UB <= cnt; k0 += UB) {
-            float dt[UB], xv[UB], Be[UB], Bo[UB], Ce[UB], Co[UB], y[UB];
-#pragma unroll
-            for (int q = 0; q < UB; q += 4) {
-                const f32x4 a = *reinterpret_cast<const f32x4*>(r_dt + k0 + q), b = *reinterpret_cast<const f32x4*>(r_ux + k0 + q);
-                const f32x4 c = *reinterpret_cast<const f32x4*>(r_Be + k0 + q), d = *reinterpret_cast<const f32x4*>(r_Bo + k0 + q);
-#pragma unroll
-                for (int e = 0; e < 4; e++) { dt[q + e] = a[e]; xv[q + e] = b[e]; Be[q + e] = c[e]; Bo[q + e] = d[e]; Ce[q + e] = 0.0f; Co[q + e] = 0.0f; }
-                if (OUT) {
-                    const f32x4 f = *reinterpret_cast<const f32x4*>(r_Ce + k0 + q), g = *reinterpret_cast<const f32x4*>(r_Co + k0 + q);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) { Ce[q + e] = f[e]; Co[q + e] = g[e]; }
-                }
-            }
-            const unsigned long long blk = ((1ull << UB) - 1) << k0;
-            auto steps = [&](auto lite_c) {
-                constexpr bool LT = decltype(lite_c)::value;
-                if (OUT && dgiven && (notlin & blk) == 0)
-                    block_steps<HP, OUT, 3, LT, true, true>(S, dt, xv, Be, Bo, Ce, Co, 0.0f, 0.0f, 0.0f, LP, y);
-                else if (dgiven)
-                    block_steps<HP, OUT, 3, LT, true>(S, dt, xv, Be, Bo, Ce, Co, 0.0f, 0.0f, 0.0f, LP, y);
-                else if ((notpoly & blk) == 0)
-                    block_steps<HP, OUT, 3, LT>(S, dt, xv, Be, Bo, Ce, Co, 0.0f, 0.0f, 0.0f, LP, y);
-                else if ((nottiny & blk) == 0)
-                    block_steps<HP, OUT, 2, LT>(S, dt, xv, Be, Bo, Ce, Co, pole_e(), pole_o(), rope_f(), LP, y);
-                else if ((large & blk) == 0)
-                    block_steps<HP, OUT, 1, LT>(S, dt, xv, Be, Bo, Ce, Co, pole_e(), pole_o(), rope_f(), LP, y);
-                else
-                    block_steps<HP, OUT, 0, LT>(S, dt, xv, Be, Bo, Ce, Co, pole_e(), pole_o(), rope_f(), LP, y);
-            };
-            if (!OUT && lite) steps(std::true_type{});
-            else steps(std::false_type{});
-            if (OUT && (p & 3) == 0) {       // the first lane of every bank holds the totals of its bank's steps (block_pair_sums)
-                if constexpr (HP == 8)
-                    *reinterpret_cast<f32x4*>(&s_y[j * LDS_STRIDE + k0 + 4 * (p >> 2)]) = f32x4{y[0], y[1], y[2], y[3]};
-                else
-                    *reinterpret_cast<float2*>(&s_y[j * LDS_STRIDE + k0 + 2 * (p >> 2)]) = make_float2(y[0], y[1]);
-            }
-        }
-        for (; k0 < cnt; k0++) {       // ragged end of the last tile of a tensor
-            const float dt = r_dt[k0], ux = r_ux[k0];
-            float ae, ao, sn, cs;
-            sg_abar_pair(dt, pole_e(), pole_o(), &ae, &ao);
-            sg_sincos(dt * rope_f(), &sn, &cs);
-            if (!OUT && lite) step_update<OUT, true>(S, ae, ao, sn, cs, ux * r_Be[k0], ux * r_Bo[k0]);
-            else step_update<OUT>(S, ae, ao, sn, cs, ux * r_Be[k0], ux * r_Bo[k0]);
-            if (OUT) {
-                const float y = pair_tree_sum<HP>(sg_fma(S.ho, r_Co[k0], S.he * r_Ce[k0]));
-                if (p == 0) s_y[j * LDS_STRIDE + k0] = y;
-            }
-        }
-        __syncthreads();
-
-        // ---------------- phase C: gate, D skip, out_proj, scatter to element order
-        if (OUT) {
-            float o[DI];
-#pragma unroll
-            for (int jj = 0; jj < DI; jj++)
-                o[jj] = sg_fma(s_y[jj * LDS_STRIDE + tu], s_gate[jj * LDS_STRIDE + tu], s_dx[jj * LDS_STRIDE + tu]);
-            constexpr int CPP = DM / PARTS;     // context entries this wave produces per timestep
-            float cx[CPP];
-#pragma unroll
-            for (int q = 0; q < CPP; q++) {
-                // row CPP * half + q of out_proj: the same address for every lane of the wave (broadcast reads)
-                const float* wr = s_wout + (half * CPP + q) * DI;
-                float a = 0.0f;
-#pragma unroll
-                for (int m = 0; m < DI; m += 4) {
-                    const f32x4 w4 = *reinterpret_cast<const f32x4*>(wr + m);
-                    a = sg_fma(w4[0], o[m], a);
-                    a = sg_fma(w4[1], o[m + 1], a);
-                    a = sg_fma(w4[2], o[m + 2], a);
-                    a = sg_fma(w4[3], o[m + 3], a);
-                }
-                cx[q] = a;
-            }
-            if (valid) {
-                float* dst = pl.ctx + ((size_t)dir * pl.total + off + orig) * DM + half * CPP;
-                static_assert(CPP == 4 || CPP == 2, "one vector store per lane");
-                if constexpr (CPP == 4)
-                    *reinterpret_cast<float4*>(dst) = make_float4(cx[0], cx[1], cx[2], cx[3]);
-                else
-                    *reinterpret_cast<float2*>(dst) = make_float2(cx[0], cx[1]);
-            }
-            __syncthreads();
-        }
-    }
-    if (OUT) break;
-    if (lite) {          // c0e holds the bound (a NaN counts as "not contracted")
-        if (!__syncthreads_or(!(S.c0e < SG2_FORGOTTEN))) {
-            S.c0e = S.c0o = S.c1e = S.c1o = 0.0f;
-            fully_contracted = true;
-            break;
-        }
-        lite = false;    // the general walk, from the end of the chunk
-        blk_first = max(u0, u1 - pl.window);
-        S = {0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 1.0f};
-        continue;
-    }
-    if (have_late) {     // S covers [blk_first, blk_end), late covers [blk_end, u1): the summary of both is late o S
-        const LaneState E = S;
-        S.c0e = sg_fma(late.c0e, E.c0e, late.c1e * E.c0o);
-        S.c0o = sg_fma(late.c0o, E.c0e, late.c1o * E.c0o);
-        S.c1e = sg_fma(late.c0e, E.c1e, late.c1e * E.c1o);
-        S.c1o = sg_fma(late.c0o, E.c1e, late.c1o * E.c1o);
-        S.he = sg_fma(late.c0e, E.he, sg_fma(late.c1e, E.ho, late.he));
-        S.ho = sg_fma(late.c0o, E.he, sg_fma(late.c1o, E.ho, late.ho));
-    }
-    if (blk_first == u0) break;       // the whole chunk is covered
-    {   // has the running summary contracted?  (a NaN counts as "no")
-        const float mx = sg_max(sg_max(sg_abs(S.c0e), sg_abs(S.c0o)), sg_max(sg_abs(S.c1e), sg_abs(S.c1o)));
-        if (!__syncthreads_or(!(mx < SG2_FORGOTTEN))) {
-            S.c0e = S.c0o = S.c1e = S.c1o = 0.0f;
-            fully_contracted = true;
-            break;
-        }
-    }
-    late = S;
-    have_late = true;
-    blk_end = blk_first;
-    blk_first = max(u0, blk_first - pl.window);
-    S = {0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 1.0f};
-    }
-
-    if (OUT) {
-        if (u1 == N) {   // last chunk in scan order: new carried state of the tensor
-            float* st = dir ? T.mbwd : T.mfwd;
-            if (j < pl.st_di && 2 * p < pl.st_ds) {
-                st[j * pl.st_ds + 2 * p] = S.he;
-                st[j * pl.st_ds + 2 * p + 1] = S.ho;
-            }
-        }
-    } else {
-        float* sm = pl.summaries + (size_t)(dir * pl.wchunks + cidx) * 6 * SCAN_THREADS;
-        sm[0 * SCAN_THREADS + tid] = S.c0e;   // M = [c0e c1e; c0o c1o]
-        sm[1 * SCAN_THREADS + tid] = S.c0o;
-        sm[2 * SCAN_THREADS + tid] = S.c1e;
-        sm[3 * SCAN_THREADS + tid] = S.c1o;
-        sm[4 * SCAN_THREADS + tid] = S.he;
-        sm[5 * SCAN_THREADS + tid] = S.ho;
-        if (!fully_contracted && tid == 0) *pl.contracted = 0;      // plain store: every writer stores the same value
-    }
-}
-
-// Projections of one timestep for the one-wave replay, for a tile that does not run on the polynomials throughout
-// (project_rows covers the usual tile): the lane computes every row of every group for its timestep (what the two
-// waves of k_scan each do half of through project_tile, with the same expressions in the same order).  Step size,
-// dt * x-branch, B and C go to LDS for the recurrence; the skip terms D * x-branch stay in the lane's registers,
-// because the lane that forms them is the one that uses them after the recurrence, and for the same reason the gates
-// are not formed here at all (gates_all, after the recurrence).
+// Projections of one timestep, for a tile that does not run on the polynomials throughout (row owners form the usual tile):
+// the lane computes its wave's rows of every group for its timestep.  Step size, dt * x-branch, B and C go to LDS for
+// the recurrence; the skip terms D * x-branch stay in the lane's registers, because the lane that forms them is the one
+// that uses them after the recurrence, and for the same reason the gates are not formed here at all (gates_of).
 // coef: [group][row] composed triple + one more float (D next to the x-branch triple); tay: [step size | gate][row][4].
-// angle[h]: bit 0 / 1 = every rotation angle of columns 8 h .. 8 h + 7 at this timestep is small / tiny.
-template <class G, bool HAS_S, bool TAYLOR>
-__device__ __forceinline__ void project_all(float g, float s, int tu, const float* s_coef, const float* s_tay, const float* s_fmax, float* s_dt,
-                                            float* s_ux, float* s_B, float* s_C, float (&dxv)[G::DI], int (&angle)[2]) {
-    constexpr int DI = G::DI, DS = G::DS;
+// c0: first column of the wave.  angle[h]: bit 0 / 1 = every rotation angle of columns c0 + CPH h .. + CPH - 1 at this timestep is
+// small enough for sg_sincos_small / sg_sincos_tiny (fmax: per column, the largest |rope frequency| of its pairs; dt >= 0
+// and rounding is monotone, so dt*fmax < limit is the same statement as |dt*freq| < limit for all pairs).
+// TAYLOR: every timestep of the tile has passed sg2_taylor_ok: step size and gate come from their cubic Taylor polynomials.
+// HAS_S is false for a tensor whose sharpness is all zero: fma(c_s, 0, c_0) is c_0 itself, so the term is skipped.
+// SLOTTED: rows of B and C at bc_slot.
+template <class G, bool OUT, bool SLOTTED, bool HAS_S, bool TAYLOR>
+__device__ __forceinline__ void project_steps(float g, float s, int tu, int c0, const float* s_coef, const float* s_tay, const float* s_fmax, float* s_dt,
+                                              float* s_ux, float* s_B, float* s_C, float (&dxv)[Split<G>::CPW], int (&angle)[2]) {
+    constexpr int DI = G::DI, CPW = Split<G>::CPW, CPH = Split<G>::CPH;
     auto delta = [&](const f32x4 t) { return HAS_S ? sg_fma(t[0], g, t[1] * s) : t[0] * g; };
     auto poly = [&](const f32x4 t, float d) { return sg_fma(sg_fma(sg_fma(t[3], d, t[2]), d, t[1]), d, t[0]); };
     auto eval = [&](const f32x4 t) { return sg_fma(t[0], g, HAS_S ? sg_fma(t[1], s, t[2]) : t[2]); };
     auto coef = [&](int group, int row) { return *reinterpret_cast<const f32x4*>(s_coef + (group * DI + row) * 4); };
-    static_assert(DI == 16 && DS == 16, "two halves of eight columns");
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         bool small = true, tiny = true;
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const int jj = 8 * h + q;
+        for (int q = 0; q < CPH; q++) {
+            const int jj = c0 + CPH * h + q;
             const f32x4 cd = coef(SG2_COMP_DT, jj);
             const float dtv = TAYLOR ? poly(*reinterpret_cast<const f32x4*>(s_tay + jj * 4), delta(cd)) : sg_softplus(eval(cd));
             const float amax = dtv * s_fmax[jj];
@@ -674,37 +234,39 @@ __device__ __forceinline__ void project_all(float g, float s, int tu, const floa
             const float xbv = eval(cx);
             s_dt[jj * LDS_STRIDE + tu] = dtv;
             s_ux[jj * LDS_STRIDE + tu] = dtv * xbv;
-            dxv[jj] = cx[3] * xbv;
+            if (OUT) dxv[CPH * h + q] = cx[3] * xbv;
         }
         angle[h] = (small ? 1 : 0) | (tiny ? 2 : 0);
     }
 #pragma unroll
-    for (int ss = 0; ss < DS; ss++) {
-        s_B[ss * LDS_STRIDE + tu] = eval(coef(SG2_COMP_B, ss));
-        s_C[ss * LDS_STRIDE + tu] = eval(coef(SG2_COMP_C, ss));
+    for (int q = 0; q < CPW; q++) {
+        const int ss = c0 + q, at = SLOTTED ? bc_slot<G>(ss) : ss;
+        s_B[at * LDS_STRIDE + tu] = eval(coef(SG2_COMP_B, ss));
+        if (OUT) s_C[at * LDS_STRIDE + tu] = eval(coef(SG2_COMP_C, ss));
     }
 }
-// The 16 gates silu(z) of one timestep: Taylor polynomials for a tile that qualifies, else eight at a time on one shared
-// reciprocal (columns 0-7, 8-15: the groups the two-wave kernel and the checker form).
+// The gates silu(z) of the wave's columns at one timestep: Taylor polynomials for a tile that qualifies, else one column of
+// every lane at a time (CPH of them) on one shared reciprocal, the groups the checker forms.
 template <class G, bool HAS_S, bool TAYLOR>
-__device__ __forceinline__ void gates_all(float g, float s, const float* s_coef, const float* s_tay, float (&gv)[G::DI]) {
-    constexpr int DI = G::DI;
+__device__ __forceinline__ void gates_of(float g, float s, int c0, const float* s_coef, const float* s_tay, float (&gv)[Split<G>::CPW]) {
+    constexpr int DI = G::DI, CPH = Split<G>::CPH;
     auto delta = [&](const f32x4 t) { return HAS_S ? sg_fma(t[0], g, t[1] * s) : t[0] * g; };
     auto poly = [&](const f32x4 t, float d) { return sg_fma(sg_fma(sg_fma(t[3], d, t[2]), d, t[1]), d, t[0]); };
     auto eval = [&](const f32x4 t) { return sg_fma(t[0], g, HAS_S ? sg_fma(t[1], s, t[2]) : t[2]); };
     auto coef = [&](int row) { return *reinterpret_cast<const f32x4*>(s_coef + (SG2_COMP_Z * DI + row) * 4); };
     if (TAYLOR) {
 #pragma unroll
-        for (int jj = 0; jj < DI; jj++) gv[jj] = poly(*reinterpret_cast<const f32x4*>(s_tay + (DI + jj) * 4), delta(coef(jj)));
+        for (int q = 0; q < 2 * CPH; q++) gv[q] = poly(*reinterpret_cast<const f32x4*>(s_tay + (DI + c0 + q) * 4), delta(coef(c0 + q)));
     } else {
+        static_assert(CPH <= 8, "sg_silu_block takes at most 8 values");
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            float zv[8], out[8];
+            float zv[CPH], out[CPH];
 #pragma unroll
-            for (int q = 0; q < 8; q++) zv[q] = eval(coef(8 * h + q));
-            sg_silu_block(8, zv, out);
+            for (int q = 0; q < CPH; q++) zv[q] = eval(coef(c0 + CPH * h + q));
+            sg_silu_block(CPH, zv, out);
 #pragma unroll
-            for (int q = 0; q < 8; q++) gv[8 * h + q] = out[q];
+            for (int q = 0; q < CPH; q++) gv[CPH * h + q] = out[q];
         }
     }
 }
@@ -716,7 +278,7 @@ __device__ __forceinline__ void gates_all(float g, float s, const float* s_coef,
 // 16-byte LDS reads per tile and lane instead of one per (timestep, row), the 64 (g, s) of the tile travel through the
 // four padding floats of the rows of s_B / s_C, and the results leave as 16-byte LDS writes: the same arithmetic as
 // the timestep-per-lane form with a fifth of its LDS instructions.  Every value is formed by the expressions of
-// project_all (Taylor form) on the same operands, so it is the same float; the step-size row receives dt - dt0, which
+// project_steps (Taylor form) on the same operands, so it is the same float; the step-size row receives dt - dt0, which
 // is what the lane polynomials of the recurrence take.
 // dxk: this lane's 16 skips D * x-branch of (column cj, timestep 16 cq + k), kept for gate_rows.
 template <class G, bool HAS_S>
@@ -796,12 +358,15 @@ __device__ __forceinline__ void gate_rows(int tid, const float* s_coef, const fl
     }
 }
 
-// UB steps of both columns of a lane on the lane polynomials, dt - dt0 given (what block_steps<HP, true, 3, false, true,
-// LINEAR> does for one column), written as one straight-line block so that the two independent recurrences interleave.
-template <int HP, bool LINEAR>
+// UB steps of both columns of a lane on the products, dt - dt0 given (what block_steps<HP, true, 3> does for one column
+// with dt), written as one straight-line block so that the two independent recurrences interleave.
+// OUT false (summary): the states alone.  PARTIAL: the steps from `rem` on lie beyond the end of the tensor; they are
+// computed (on projections of zero inputs) and their effect on the state is taken back.
+template <int HP, bool LINEAR, bool OUT, bool PARTIAL>
 __device__ __forceinline__ void block_steps_pair(LaneState (&S)[2], const float (&dt)[2][UB], const float (&ux)[2][UB], const float (&Be)[UB],
                                                  const float (&Bo)[UB], const float (&Ce)[UB], const float (&Co)[UB], const LanePoly<true> (&LP)[2],
-                                                 float (&y)[2][UB]) {
+                                                 int rem, float (&y)[2][UB]) {
+    float keep[4];
 #pragma unroll
     for (int u = 0; u < UB; u++) {
 #pragma unroll
@@ -815,28 +380,37 @@ __device__ __forceinline__ void block_steps_pair(LaneState (&S)[2], const float 
             const float he = sg_fma(p1, S[h].he, sg_fma(n2, S[h].ho, be));      // P1 he + N2 ho + b_e
             S[h].ho = sg_fma(p3, S[h].ho, sg_fma(p4, S[h].he, bo));            // P3 ho + P4 he + b_o
             S[h].he = he;
-            y[h][u] = sg_fma(S[h].ho, Co[u], S[h].he * Ce[u]);
+            if (OUT) y[h][u] = sg_fma(S[h].ho, Co[u], S[h].he * Ce[u]);
+        }
+        if (PARTIAL && u == rem - 1) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) { keep[2 * h] = S[h].he; keep[2 * h + 1] = S[h].ho; }
         }
     }
-    block_pair_sums<HP>(y[0]);
-    block_pair_sums<HP>(y[1]);
+    if (PARTIAL) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) { S[h].he = keep[2 * h]; S[h].ho = keep[2 * h + 1]; }
+    }
+    if (OUT) {
+        block_pair_sums<HP>(y[0]);
+        block_pair_sums<HP>(y[1]);
+    }
 }
 
-// The replay of the default geometry (what k_scan<G, true> computes, value for value) as ONE wave per chunk: lane
-// (jl, p) owns RoPE pair p of the two columns jl and jl + 8.  The 16 lanes that need the same B / C entries of a
-// timestep are then 8, and each entry a lane fetches from LDS feeds two recurrences: a third less LDS traffic per
-// step -- the pass was bound by the LDS queue and the vector ALU together, and the B / C fetches alone were a fifth of
+// The replay of the default geometry as ONE wave per chunk: lane (jl, p) owns RoPE pair p of the two columns jl and
+// jl + 8.  The lanes that need the same B / C entries of a timestep are then 8, and each entry a lane fetches from LDS
+// feeds two recurrences: a third less LDS traffic per step than with a column per lane of two waves -- the pass was bound
+// by the LDS queue and the vector ALU together, and the B / C fetches alone were a fifth of
 // its time.  A single wave also needs no workgroup barrier between the phases of a tile (its LDS accesses execute in
-// program order), forms the 16 gated outputs of a timestep once instead of once per wave, and holds all eight context
+// program order), forms the 16 gated outputs of a timestep once, and holds all eight context
 // entries of its timestep: the two 16-byte stores of an element are adjacent in one lane and leave as one 32-byte
-// write.  Column jl + 8 h plays the part of wave h of the two-wave kernel throughout (its half of the projections, its
-// angle masks, its ballots over the same 64 (column, pair) lanes), so every decision and every value is the one the
-// checker makes for the two-wave form.
+// write.  Columns jl + 8 h of all lanes form a group that decides together (angle masks, the shared reciprocals, gates eight
+// at a time), as in the checker.
 // A tile has three lane roles.  Recurrence (phase B): lane (jl, p) as above.  Timestep: lane t loads the inputs of
 // timestep t, votes on the form the tile takes, and at the end multiplies its 16 gated outputs by out_proj and stores
 // its element's row.  Row owner (the usual tile, on the polynomials throughout): lane (column, quarter of the tile)
 // forms that column's projections before the recurrence and gates its outputs after it (project_rows, gate_rows);
-// other tiles keep the timestep-per-lane projections (project_all, gates_all).
+// other tiles keep the timestep-per-lane projections (project_steps, gates_of).
 // KEEP (bilevel pass): also store the state entering every HT_STEP-th step for the adjoint kernels, and the gated outputs
 // where they are asked for.  (5.9 ms for 25 M elements; 7.1 as a variant of the two-wave kernel.)
 template <class G, bool KEEP>
@@ -974,7 +548,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         const unsigned long long notlin =
             __builtin_amdgcn_ballot_w64(!sg2_poly_ok(SG2_PROD_LINEAR_FACTOR * kpoly_g, SG2_PROD_LINEAR_FACTOR * kpoly_s, g, sh));
         const bool tay = __builtin_amdgcn_ballot_w64(!sg2_taylor_ok(cmax_g, cmax_s, g, sh)) == 0;
-        const bool dgiven = tay && notpoly == 0 && cnt == SCAN_TT;
+        const bool dgiven = tay && notpoly == 0;       // (steps beyond the end of the tensor carry zero inputs and qualify)
         unsigned long long large[2] = {0, 0}, nottiny[2] = {0, 0};
         float dxv[DI];           // D * x-branch, kept for phase C: of this lane's timestep, or (dgiven) of its column's 16 timesteps
         if (dgiven) {
@@ -984,7 +558,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             int angle[2];
             auto run = [&](auto has_s_c, auto tay_c) {
                 constexpr bool HS = decltype(has_s_c)::value, TY = decltype(tay_c)::value;
-                project_all<G, HS, TY>(g, sh, tu, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, angle);
+                project_steps<G, true, false, HS, TY>(g, sh, tu, 0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, angle);
             };
             if (tay) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
             else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
@@ -1012,7 +586,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         const float* __restrict__ r_Co = s_C + (2 * p + 1) * LDS_STRIDE;
         int k0 = 0;
         if (dgiven) {
-            // a whole tile on the lane polynomials (the usual case): both columns in one instruction stream
+            // a tile on the products throughout (the usual case): both columns in one instruction stream
             float Be[UB], Bo[UB], Ce[UB], Co[UB], dt[2][UB], xv[2][UB];
             auto fetch = [&](int kb, float (&tBe)[UB], float (&tBo)[UB], float (&tCe)[UB], float (&tCo)[UB], float (&tdt)[2][UB], float (&tux)[2][UB]) {
 #pragma unroll
@@ -1034,15 +608,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                                const float (&tdt)[2][UB], const float (&tux)[2][UB]) {
                 float y[2][UB];
                 const unsigned long long blk = ((1ull << UB) - 1) << kb;
-                if ((notlin & blk) == 0) block_steps_pair<HP, true>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, y);
-                else block_steps_pair<HP, false>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, y);
+                if (kb + UB > cnt) block_steps_pair<HP, false, true, true>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, cnt - kb, y);      // the tensor's last block
+                else if ((notlin & blk) == 0) block_steps_pair<HP, true, true, false>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, UB, y);
+                else block_steps_pair<HP, false, true, false>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, UB, y);
                 if ((p & 3) == 0) {      // the first lane of every bank holds the totals of its bank's steps (block_pair_sums)
                     *reinterpret_cast<f32x4*>(&s_y[jl * LDS_STRIDE + kb + 4 * (p >> 2)]) = f32x4{y[0][0], y[0][1], y[0][2], y[0][3]};
                     *reinterpret_cast<f32x4*>(&s_y[(jl + 8) * LDS_STRIDE + kb + 4 * (p >> 2)]) = f32x4{y[1][0], y[1][1], y[1][2], y[1][3]};
                 }
             };
 #pragma unroll 1
-            for (; k0 < SCAN_TT; k0 += UB) {
+            for (; k0 < cnt; k0 += UB) {
                 if (KEEP && k0 % HT_STEP == 0) keep_state(tile0 + k0);
                 fetch(k0, Be, Bo, Ce, Co, dt, xv);
                 compute(k0, Be, Bo, Ce, Co, dt, xv);
@@ -1069,11 +644,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
                     for (int e = 0; e < 4; e++) { dt[q + e] = a4[e]; xv[q + e] = b4[e]; }
                 }
-                if (dgiven && (notlin & blk) == 0)
-                    block_steps<HP, OUT, 3, false, true, true>(S[h], dt, xv, Be, Bo, Ce, Co, 0.0f, 0.0f, 0.0f, LP[h], y);
-                else if (dgiven)
-                    block_steps<HP, OUT, 3, false, true>(S[h], dt, xv, Be, Bo, Ce, Co, 0.0f, 0.0f, 0.0f, LP[h], y);
-                else if ((notpoly & blk) == 0)
+                if ((notpoly & blk) == 0)
                     block_steps<HP, OUT, 3, false>(S[h], dt, xv, Be, Bo, Ce, Co, 0.0f, 0.0f, 0.0f, LP[h], y);
                 else if ((nottiny[h] & blk) == 0)
                     block_steps<HP, OUT, 2, false>(S[h], dt, xv, Be, Bo, Ce, Co, pole_e(h), pole_o(h), rope_f(h), LP[h], y);
@@ -1111,8 +682,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
                 for (int jj = 0; jj < DI; jj++) o[jj] = s_y[jj * LDS_STRIDE + tu];
             } else {
-                if (tay) { if (has_s) gates_all<G, true, true>(g, sh, s_coef, s_tay, o); else gates_all<G, false, true>(g, sh, s_coef, s_tay, o); }
-                else { if (has_s) gates_all<G, true, false>(g, sh, s_coef, s_tay, o); else gates_all<G, false, false>(g, sh, s_coef, s_tay, o); }
+                if (tay) { if (has_s) gates_of<G, true, true>(g, sh, 0, s_coef, s_tay, o); else gates_of<G, false, true>(g, sh, 0, s_coef, s_tay, o); }
+                else { if (has_s) gates_of<G, true, false>(g, sh, 0, s_coef, s_tay, o); else gates_of<G, false, false>(g, sh, 0, s_coef, s_tay, o); }
 #pragma unroll
                 for (int jj = 0; jj < DI; jj++) o[jj] = sg_fma(s_y[jj * LDS_STRIDE + tu], o[jj], dxv[jj]);
             }
@@ -1159,6 +730,613 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                 st[j * pl.st_ds + 2 * p + 1] = S[h].ho;
             }
         }
+    }
+}
+
+// Which chunk a workgroup of a scan launch owns (per_dir chunks of each direction, found through `prefix`).
+struct ChunkOf {
+    int dir, cidx, ti, c, N, off, u0, u1;
+    bool has_s;
+};
+__device__ __forceinline__ ChunkOf chunk_of(const Plan& pl, const int* chunk_prefix, int per_dir) {
+    ChunkOf k;
+    k.dir = (int)blockIdx.x >= per_dir ? 1 : 0;
+    k.cidx = (int)blockIdx.x - k.dir * per_dir;
+    const sg::cint_p prefix = sg::as_const(chunk_prefix);
+    const sg::Seg seg = sg::find_seg(prefix, pl.P, k.cidx);
+    k.ti = seg.i;
+    k.c = k.cidx - seg.first;
+    k.N = pl.tensors[k.ti].numel;
+    k.off = pl.tensors[k.ti].off;
+    k.u0 = k.c * pl.chunk_len;
+    k.u1 = min(k.u0 + pl.chunk_len, k.N);
+    k.has_s = __builtin_amdgcn_readfirstlane(pl.sharp_nonzero[k.ti]) != 0;
+    return k;
+}
+
+// The projections of a tile that runs on the products throughout, formed by lanes that own rows: lane (row r, part q) of
+// wave w forms column CPW w + r (dt - dt0, dt * x-branch, D * x-branch) and row CPW w + r of B (and C) for timesteps SPL q ..
+// SPL q + SPL - 1.  s_in: the tile's 64 g and 64 s, the wave's own copy.  Values and reasons as in project_rows.
+template <class G, bool OUT, bool HAS_S>
+__device__ __forceinline__ void project_own_rows(const float* s_in, int lane, int c0, const float* s_coef, const float* s_tay, float* s_dt, float* s_ux,
+                                                 float* s_B, float* s_C, float (&dxk)[Split<G>::SPL]) {
+    constexpr int DI = G::DI, CPW = Split<G>::CPW, SPL = Split<G>::SPL;
+    auto delta = [&](const f32x4 t, float gg, float ss) { return HAS_S ? sg_fma(t[0], gg, t[1] * ss) : t[0] * gg; };
+    auto poly = [&](const f32x4 t, float d) { return sg_fma(sg_fma(sg_fma(t[3], d, t[2]), d, t[1]), d, t[0]); };
+    auto eval = [&](const f32x4 t, float gg, float ss) { return sg_fma(t[0], gg, HAS_S ? sg_fma(t[1], ss, t[2]) : t[2]); };
+    const int row = c0 + lane % CPW, t0 = SPL * (lane / CPW);
+    auto coef = [&](int group) { return *reinterpret_cast<const f32x4*>(s_coef + (group * DI + row) * 4); };
+    const f32x4 cd = coef(SG2_COMP_DT), cx = coef(SG2_COMP_XB), cb = coef(SG2_COMP_B), cc = OUT ? coef(SG2_COMP_C) : cb;
+    const f32x4 tp = *reinterpret_cast<const f32x4*>(s_tay + row * 4);
+    float* const r_dt = s_dt + row * LDS_STRIDE + t0;
+    float* const r_ux = s_ux + row * LDS_STRIDE + t0;
+    float* const r_B = s_B + bc_slot<G>(row) * LDS_STRIDE + t0;
+    float* const r_C = OUT ? s_C + bc_slot<G>(row) * LDS_STRIDE + t0 : nullptr;
+#pragma unroll
+    for (int i = 0; i < SPL / 4; i++) {
+        const f32x4 g4 = *reinterpret_cast<const f32x4*>(s_in + t0 + 4 * i);
+        const f32x4 s4 = HAS_S ? *reinterpret_cast<const f32x4*>(s_in + SCAN_TT + t0 + 4 * i) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        f32x4 d4, u4, b4, k4;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float dtv = poly(tp, delta(cd, g4[e], s4[e]));
+            const float xbv = eval(cx, g4[e], s4[e]);
+            d4[e] = dtv - tp[0];
+            u4[e] = dtv * xbv;
+            if (OUT) dxk[4 * i + e] = cx[3] * xbv;
+            b4[e] = eval(cb, g4[e], s4[e]);
+            if (OUT) k4[e] = eval(cc, g4[e], s4[e]);
+        }
+        *reinterpret_cast<f32x4*>(r_dt + 4 * i) = d4;
+        *reinterpret_cast<f32x4*>(r_ux + 4 * i) = u4;
+        *reinterpret_cast<f32x4*>(r_B + 4 * i) = b4;
+        if (OUT) *reinterpret_cast<f32x4*>(r_C + 4 * i) = k4;
+    }
+}
+
+// The tables a workgroup of the scan reads from LDS: composed triples (D beside the x-branch's), Taylor polynomials, the
+// largest |rope frequency| of each column.
+template <class G>
+__device__ __forceinline__ void stage_tables(const Plan& pl, int dir, int tid, int threads, float* s_coef, float* s_tay, float* s_fmax) {
+    constexpr int DI = G::DI, HP = G::HP;
+    const float* comp = pl.comp + dir * (SG2_COMP_GROUPS * G::ROWS * 3);
+    const float* tay = pl.comp + 2 * SG2_COMP_GROUPS * G::ROWS * 3 + dir * 2 * G::ROWS * 4;
+    const float* Dw = pl.W.w[dir ? W_B_D : W_F_D];
+    const float* rope = pl.W.w[dir ? W_B_ROPE : W_F_ROPE];
+    for (int i = tid; i < SG2_COMP_GROUPS * DI; i += threads) {
+        const float* t = comp + i * 3;
+        *reinterpret_cast<f32x4*>(s_coef + i * 4) = f32x4{t[0], t[1], t[2], i / DI == SG2_COMP_XB ? Dw[i % DI] : 0.0f};
+    }
+    for (int i = tid; i < 2 * DI * 4; i += threads) s_tay[i] = tay[i];
+    if (tid < DI) {
+        float m = 0.0f;
+#pragma unroll
+        for (int p = 0; p < HP; p++) m = sg_max(m, sg_abs(rope[tid * HP + p]));
+        s_fmax[tid] = m;
+    }
+}
+
+// ---- chunk summaries
+// Bound by the vector ALU like the replay, and laid out like it: a lane owns one pair of two columns, a wave CPW columns and
+// as many rows of B, which feed both columns of a lane.  The first attempt walks the states alone on the products of
+// the output pass: ten instructions per step, column and pair on their linear parts, 14 on the quadratics, where the separate
+// A_bar, sin, cos and the bound on the 2x2 part took 22.  The bound needs nothing per step there: while a tile
+// qualifies, |dt - dt0| is below pl.comp's limit, so a pair's part shrinks at least by sg2_abar_bound in every step.
+// 28 us on 0.42 M elements, 82 us on 3.1 M, 141 us on 25 M, 167 us on 0.42 M with the large geometry; with one column per lane,
+// two or eight waves per chunk and the separate factors 46, 115, 212 and 254 us.
+template <class G>
+__global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_summary(Plan pl) {
+    constexpr int DS = G::DS, DI = G::DI, HP = G::HP, LANES = G::THREADS, WAVES = Split<G>::WAVES, CPW = Split<G>::CPW, CPH = Split<G>::CPH;
+    __shared__ __attribute__((aligned(16))) float s_dt[DI * LDS_STRIDE];
+    __shared__ __attribute__((aligned(16))) float s_ux[DI * LDS_STRIDE];       // dt * x-branch
+    __shared__ __attribute__((aligned(16))) float s_B[DS * LDS_STRIDE];
+    __shared__ __attribute__((aligned(16))) float s_in_all[WAVES * 2 * SCAN_TT];
+    __shared__ __attribute__((aligned(16))) float s_coef[SG2_COMP_GROUPS * DI * 4];
+    __shared__ __attribute__((aligned(16))) float s_tay[2 * DI * 4];
+    __shared__ float s_fmax[DI];
+
+    const ChunkOf K = chunk_of(pl, pl.wchunk_prefix, pl.wchunks);
+    const int dir = K.dir, N = K.N, u0 = K.u0, u1 = K.u1;
+    const bool has_s = K.has_s;
+    const uint32_t* __restrict__ skey = pl.keys[0] + K.off;      // sorted |g| bits
+    const int32_t* __restrict__ sval = pl.vals[0] + K.off;       // element index | sign of g
+    const float* __restrict__ ssrt = pl.ssorted + K.off;          // sharpness in sorted order
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c0 = CPW * wave, jl = lane / HP, p = lane % HP;       // scan role: pair p of columns c0 + jl and c0 + CPH + jl
+    const int tu = lane;                                            // projection role: timestep of the tile
+    float* const s_in = s_in_all + wave * 2 * SCAN_TT;
+    const float* alog = pl.W.w[dir ? W_B_ALOG : W_F_ALOG];
+    const float* rope = pl.W.w[dir ? W_B_ROPE : W_F_ROPE];
+    const float* tay = pl.comp + 2 * SG2_COMP_GROUPS * G::ROWS * 3 + dir * 2 * G::ROWS * 4;
+    auto col = [&](int h) { return c0 + jl + CPH * h; };
+    // -A/2 with A = -exp(A_log): the two poles of a pair (formed again where an exceptional block needs them)
+    auto pole_e = [&](int h) { return -0.5f * -sg_exp(alog[col(h) * DS + 2 * p]); };
+    auto pole_o = [&](int h) { return -0.5f * -sg_exp(alog[col(h) * DS + 2 * p + 1]); };
+    auto rope_f = [&](int h) { return rope[col(h) * HP + p]; };
+    const sg::cfloat_p lim = sg::as_const(pl.comp) + 2 * SG2_COMP_GROUPS * G::ROWS * 3 + 2 * 2 * G::ROWS * 4;
+    const float cmax_g = lim[2 * dir], cmax_s = lim[2 * dir + 1];              // what decides whether a tile may use the Taylor polynomials
+    const float kpoly_g = lim[4 + 2 * dir], kpoly_s = lim[5 + 2 * dir];        // ... a block the lane polynomials (sg2_poly_ok)
+    const float kprod_g = lim[8 + 2 * dir], kprod_s = lim[9 + 2 * dir];        // ... a tile of the first attempt the products
+    LanePoly<true> LP[2];
+    float shrink[2];            // what eight steps on the products multiply a pair's 2x2 part by at most
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        LP[h].dt0 = tay[col(h) * 4];
+        const float ae = pole_e(h), ao = pole_o(h);
+        sg2_pair_products(LP[h].dt0, ae, ao, rope_f(h), LP[h].k);
+        shrink[h] = sg2_shrink8(LP[h].dt0, ae, ao, lim[16 + dir]);
+    }
+    stage_tables<G>(pl, dir, tid, 64 * WAVES, s_coef, s_tay, s_fmax);
+    __syncthreads();
+
+    const LaneState identity = {0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 1.0f};
+    LaneState S[2] = {identity, identity}, late[2] = {identity, identity};
+    bool fully_contracted = false;      // the walk stopped because the 2x2 part had contracted
+    bool have_late = false;
+    // The chunk is walked backwards in blocks of `window` steps.  Each block is summarised from the identity and the
+    // summary of everything after it (`late`) is applied on top; as soon as the 2x2 part of the running summary has
+    // contracted below 2^-64 the steps before the block cannot matter and the walk stops.
+    int blk_end = u1;
+    int blk_first = u0;
+    if (pl.window > 0 && pl.window < pl.chunk_len) blk_first = max(u0, u1 - pl.window);
+    // First attempt: ONE block of as many steps as compose_block expects the slowest pair to need, walked with the state
+    // part only (LITE) and a bound on the 2x2 part in its place.  If the bound is below 2^-64 in every lane the summary
+    // is (0, b) as below; if not, the walk starts over in its general form.
+    bool lite = false;
+    if (blk_first > u0) {
+        const int first_block = __builtin_amdgcn_readfirstlane(pl.contracted[1]);
+        if (first_block > 0 && u1 - first_block > u0) {
+            lite = true;
+            blk_first = u1 - first_block;
+        }
+    }
+    // inputs of one tile (sorted |g| bits, payload, sorted sharpness) for this lane's timestep; zero beyond the block
+    uint32_t nx_key = 0;
+    int32_t nx_val = 0;
+    float nx_sh = 0.0f;
+    auto load_inputs = [&](int tile0) {
+        const int u = tile0 + tu;
+        if (u < blk_end) {
+            const int t = dir ? (N - 1 - u) : u;
+            nx_key = skey[t];
+            nx_val = sval[t];
+            nx_sh = has_s ? ssrt[t] : 0.0f;      // an all-zero tensor has no sorted copy of its sharpness (uniform branch)
+        }
+    };
+    const float* const r_Be = s_B + p * LDS_STRIDE;
+    const float* const r_Bo = s_B + (HP + p) * LDS_STRIDE;
+    auto fetch4 = [&](const float* r, float (&out)[UB], int k0) {
+#pragma unroll
+        for (int q = 0; q < UB; q += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(r + k0 + q);
+#pragma unroll
+            for (int e = 0; e < 4; e++) out[q + e] = v[e];
+        }
+    };
+    // the steps from blk_first to blk_end
+    auto walk = [&](auto lite_c) {
+        constexpr bool LITE = decltype(lite_c)::value;
+        load_inputs(blk_first);
+        for (int tile0 = blk_first; tile0 < blk_end; tile0 += SCAN_TT) {
+            const int cnt = min(SCAN_TT, blk_end - tile0);
+            const bool valid = tile0 + tu < blk_end;
+            // this tile's inputs were requested one tile ago (or just before the loop); request the next tile's now
+            const float g = valid ? sg_i2f((int32_t)nx_key | (nx_val & (int32_t)0x80000000)) : 0.0f;
+            const float sh = valid ? nx_sh : 0.0f;
+            if (tile0 + SCAN_TT < blk_end) load_inputs(tile0 + SCAN_TT);
+            // the same 64 timesteps in every wave of the workgroup: the same decisions without talking to one another
+            const bool ty = __builtin_amdgcn_ballot_w64(!sg2_taylor_ok(cmax_g, cmax_s, g, sh)) == 0;
+            const bool fast = LITE && ty && cnt % UB == 0 && __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kprod_g, kprod_s, g, sh)) == 0;
+            unsigned long long notpoly = 0, large[2] = {0, 0}, nottiny[2] = {0, 0};
+            float unused[CPW];
+            if (fast) {
+                s_in[tu] = g;
+                if (has_s) s_in[SCAN_TT + tu] = sh;
+                __builtin_amdgcn_wave_barrier();      // one wave's LDS accesses execute in program order
+                if (has_s) project_own_rows<G, false, true>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, nullptr, unused);
+                else project_own_rows<G, false, false>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, nullptr, unused);
+            } else {
+                int angle[2];
+                auto run = [&](auto has_s_c, auto tay_c) {
+                    project_steps<G, false, true, decltype(has_s_c)::value, decltype(tay_c)::value>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B,
+                                                                                                   nullptr, unused, angle);
+                };
+                if (ty) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
+                else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
+                notpoly = __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kpoly_g, kpoly_s, g, sh));
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    large[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 1));
+                    nottiny[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 2));
+                }
+            }
+            __syncthreads();
+            if (fast) {
+                const unsigned long long notlin =
+                    __builtin_amdgcn_ballot_w64(!sg2_poly_ok(SG2_PROD_LINEAR_FACTOR * kprod_g, SG2_PROD_LINEAR_FACTOR * kprod_s, g, sh));
+#pragma unroll 1
+                for (int k0 = 0; k0 < cnt; k0 += UB) {
+                    float dt[2][UB], ux[2][UB], Be[UB], Bo[UB], y[2][UB];
+                    fetch4(r_Be, Be, k0);
+                    fetch4(r_Bo, Bo, k0);
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        fetch4(s_dt + col(h) * LDS_STRIDE, dt[h], k0);
+                        fetch4(s_ux + col(h) * LDS_STRIDE, ux[h], k0);
+                    }
+                    const unsigned long long blk = ((1ull << UB) - 1) << k0;
+                    if ((notlin & blk) == 0) block_steps_pair<HP, true, false, false>(S, dt, ux, Be, Bo, Be, Bo, LP, UB, y);
+                    else block_steps_pair<HP, false, false, false>(S, dt, ux, Be, Bo, Be, Bo, LP, UB, y);
+#pragma unroll
+                    for (int h = 0; h < 2; h++) S[h].c0e = S[h].c0e * shrink[h];
+                }
+            } else {
+                // exceptional: one column after the other, the forms of its blocks chosen one by one
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    LanePoly<false> GP;
+                    const float ae0 = pole_e(h), ao0 = pole_o(h), f0 = rope_f(h);
+                    GP.dt0 = tay[col(h) * 4];
+                    sg2_abar_poly(GP.dt0, ae0, GP.pe);
+                    sg2_abar_poly(GP.dt0, ao0, GP.po);
+                    sg2_sincos_poly(GP.dt0, f0, GP.qs, GP.qc);
+                    LaneState T = S[h];
+                    const unsigned long long lg = large[h], nt = nottiny[h];
+                    const float* r_dt = s_dt + col(h) * LDS_STRIDE;
+                    const float* r_ux = s_ux + col(h) * LDS_STRIDE;
+                    int k0 = 0;
+                    for (; k0 + UB <= cnt; k0 += UB) {
+                        float dt[UB], ux[UB], Be[UB], Bo[UB], y[UB];
+                        fetch4(r_Be, Be, k0);
+                        fetch4(r_Bo, Bo, k0);
+                        fetch4(r_dt, dt, k0);
+                        fetch4(r_ux, ux, k0);
+                        const unsigned long long blk = ((1ull << UB) - 1) << k0;
+                        if ((notpoly & blk) == 0) block_steps<HP, false, 3, LITE>(T, dt, ux, Be, Bo, Be, Bo, 0.0f, 0.0f, 0.0f, GP, y);
+                        else if ((nt & blk) == 0) block_steps<HP, false, 2, LITE>(T, dt, ux, Be, Bo, Be, Bo, ae0, ao0, f0, GP, y);
+                        else if ((lg & blk) == 0) block_steps<HP, false, 1, LITE>(T, dt, ux, Be, Bo, Be, Bo, ae0, ao0, f0, GP, y);
+                        else block_steps<HP, false, 0, LITE>(T, dt, ux, Be, Bo, Be, Bo, ae0, ao0, f0, GP, y);
+                    }
+                    for (; k0 < cnt; k0++) {
+                        float ae, ao, sn, cs;
+                        sg_abar_pair(r_dt[k0], ae0, ao0, &ae, &ao);
+                        sg_sincos(r_dt[k0] * f0, &sn, &cs);
+                        step_update<false, LITE>(T, ae, ao, sn, cs, r_ux[k0] * r_Be[k0], r_ux[k0] * r_Bo[k0]);
+                    }
+                    S[h] = T;
+                }
+            }
+            __syncthreads();
+        }
+    };
+    if (lite) {
+        walk(std::true_type{});      // c0e holds the bound (a NaN counts as "not contracted")
+        fully_contracted = !__syncthreads_or(!(S[0].c0e < SG2_FORGOTTEN) || !(S[1].c0e < SG2_FORGOTTEN));
+        if (!fully_contracted) {     // the general walk, from the end of the chunk
+            blk_first = max(u0, u1 - pl.window);
+            S[0] = identity;
+            S[1] = identity;
+        }
+    }
+    while (!fully_contracted) {
+        walk(std::false_type{});
+        bool open = false;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (have_late) {     // S covers [blk_first, blk_end), late covers [blk_end, u1): the summary of both is late o S
+                const LaneState E = S[h], &L = late[h];
+                S[h].c0e = sg_fma(L.c0e, E.c0e, L.c1e * E.c0o);
+                S[h].c0o = sg_fma(L.c0o, E.c0e, L.c1o * E.c0o);
+                S[h].c1e = sg_fma(L.c0e, E.c1e, L.c1e * E.c1o);
+                S[h].c1o = sg_fma(L.c0o, E.c1e, L.c1o * E.c1o);
+                S[h].he = sg_fma(L.c0e, E.he, sg_fma(L.c1e, E.ho, L.he));
+                S[h].ho = sg_fma(L.c0o, E.he, sg_fma(L.c1o, E.ho, L.ho));
+            }
+            // has the running summary contracted?  (a NaN counts as "no")
+            const float mx = sg_max(sg_max(sg_abs(S[h].c0e), sg_abs(S[h].c0o)), sg_max(sg_abs(S[h].c1e), sg_abs(S[h].c1o)));
+            open = open || !(mx < SG2_FORGOTTEN);
+        }
+        if (blk_first == u0) break;       // the whole chunk is covered
+        fully_contracted = !__syncthreads_or(open);
+        if (fully_contracted) break;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            late[h] = S[h];
+            S[h] = identity;
+        }
+        have_late = true;
+        blk_end = blk_first;
+        blk_first = max(u0, blk_first - pl.window);
+    }
+    if (fully_contracted) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) S[h].c0e = S[h].c0o = S[h].c1e = S[h].c1o = 0.0f;
+    }
+    float* sm = pl.summaries + (size_t)(dir * pl.wchunks + K.cidx) * 6 * LANES;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int at = 128 * wave + 64 * h + lane;       // (column, pair) in the order of the columns
+        sm[0 * LANES + at] = S[h].c0e;   // M = [c0e c1e; c0o c1o]
+        sm[1 * LANES + at] = S[h].c0o;
+        sm[2 * LANES + at] = S[h].c1e;
+        sm[3 * LANES + at] = S[h].c1o;
+        sm[4 * LANES + at] = S[h].he;
+        sm[5 * LANES + at] = S[h].ho;
+    }
+    if (!fully_contracted && tid == 0) *pl.contracted = 0;      // plain store: every writer stores the same value
+}
+
+// ---- the replay of the large geometry: four waves per chunk, each k_replay's wave over eight of the 32 columns
+// A wave forms its own columns and its eighth of the rows of B and C, walks its columns and gates them; what the waves share is
+// B and C, and the outputs that out_proj sums over all columns.  So a tile has two barriers (B and C stand; the gated
+// outputs stand), the row s_dt / s_y alternates between two buffers, and two workgroups (98 KB of LDS, 256 registers a
+// lane) share a compute unit to work across them.  Each B / C entry a lane fetches feeds two recurrences, and a
+// context leaves as 64 contiguous bytes: wave w multiplies timesteps 16 w .. 16 w + 15 by all of out_proj (4x4x1
+// matrix instructions, block (timestep quad, four rows): the fmaf chain over the columns, bit for bit).
+// 300 us on 0.42 M elements; as
+// one 512-lane workgroup per compute unit with a column per lane and a barrier after every phase 409 us.
+template <class G>
+__global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_replay_wide(Plan pl) {
+    constexpr int DM = G::DM, DS = G::DS, DI = G::DI, HP = G::HP, LANES = G::THREADS, WAVES = Split<G>::WAVES, CPW = Split<G>::CPW, CPH = Split<G>::CPH;
+    constexpr int SPL = Split<G>::SPL, WSTRIDE = DI + 4;        // out_proj rows: 16 lanes read 16 rows at once
+    static_assert(WAVES == 4 && DM == 16 && SCAN_TT / WAVES == 16, "out_proj roles");
+    __shared__ __attribute__((aligned(16))) float s_dty[2][DI * LDS_STRIDE];    // dt (dt - dt0) of a column, then its y, then its gated output
+    __shared__ __attribute__((aligned(16))) float s_ux[DI * LDS_STRIDE];
+    __shared__ __attribute__((aligned(16))) float s_B[DS * LDS_STRIDE];
+    __shared__ __attribute__((aligned(16))) float s_C[DS * LDS_STRIDE];
+    __shared__ __attribute__((aligned(16))) float s_in_all[WAVES * 2 * SCAN_TT];
+    __shared__ __attribute__((aligned(16))) float s_coef[SG2_COMP_GROUPS * DI * 4];
+    __shared__ __attribute__((aligned(16))) float s_tay[2 * DI * 4];
+    __shared__ __attribute__((aligned(16))) float s_wout[DM * WSTRIDE];
+    __shared__ float s_fmax[DI];
+
+    const ChunkOf K = chunk_of(pl, pl.chunk_prefix, pl.chunks);
+    const int dir = K.dir, N = K.N, off = K.off, u0 = K.u0, u1 = K.u1, c = K.c;
+    const bool has_s = K.has_s;
+    const TensorDev& T = pl.tensors[K.ti];
+    const uint32_t* __restrict__ skey = pl.keys[0] + off;
+    const int32_t* __restrict__ sval = pl.vals[0] + off;
+    const float* __restrict__ ssrt = pl.ssorted + off;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c0 = CPW * wave, jl = lane / HP, p = lane % HP;
+    const int tu = lane;
+    float* const s_in = s_in_all + wave * 2 * SCAN_TT;
+    const float* alog = pl.W.w[dir ? W_B_ALOG : W_F_ALOG];
+    const float* rope = pl.W.w[dir ? W_B_ROPE : W_F_ROPE];
+    auto col = [&](int h) { return c0 + jl + CPH * h; };
+    auto pole_e = [&](int h) { return -0.5f * -sg_exp(alog[col(h) * DS + 2 * p]); };
+    auto pole_o = [&](int h) { return -0.5f * -sg_exp(alog[col(h) * DS + 2 * p + 1]); };
+    auto rope_f = [&](int h) { return rope[col(h) * HP + p]; };
+    LanePoly<true> LP[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        LP[h].dt0 = pl.comp[2 * SG2_COMP_GROUPS * G::ROWS * 3 + dir * 2 * G::ROWS * 4 + col(h) * 4];
+        sg2_pair_products(LP[h].dt0, pole_e(h), pole_o(h), rope_f(h), LP[h].k);
+    }
+    stage_tables<G>(pl, dir, tid, 64 * WAVES, s_coef, s_tay, s_fmax);
+    for (int i = tid; i < DM * DI; i += 64 * WAVES) s_wout[i / DI * WSTRIDE + i % DI] = pl.W.w[dir ? W_B_OUT : W_F_OUT][i];
+    __syncthreads();
+    const sg::cfloat_p lim = sg::as_const(pl.comp) + 2 * SG2_COMP_GROUPS * G::ROWS * 3 + 2 * 2 * G::ROWS * 4;
+    const float cmax_g = lim[2 * dir], cmax_s = lim[2 * dir + 1];
+    const float kpoly_g = lim[8 + 2 * dir], kpoly_s = lim[8 + 2 * dir + 1];
+
+    LaneState S[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        S[h] = {0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 1.0f};
+        const int at = 128 * wave + 64 * h + lane;
+        if (c > 0 && __builtin_amdgcn_readfirstlane(*pl.contracted) != 0) {
+            const float* sm = pl.summaries + (size_t)(dir * pl.wchunks + pl.wchunk_prefix[K.ti] + c - 1) * 6 * LANES;
+            S[h].he = sm[4 * LANES + at];
+            S[h].ho = sm[5 * LANES + at];
+        } else if (T.nchunks == 1) {       // nothing before it: the carried state itself (no other workgroup writes it)
+            const float* st = dir ? T.mbwd : T.mfwd;
+            if (col(h) < pl.st_di && 2 * p < pl.st_ds) {
+                S[h].he = st[col(h) * pl.st_ds + 2 * p];
+                S[h].ho = st[col(h) * pl.st_ds + 2 * p + 1];
+            }
+        } else {
+            const float* hs = pl.hstart + ((size_t)(dir * pl.chunks + K.cidx) * 2) * LANES;
+            S[h].he = hs[at];
+            S[h].ho = hs[LANES + at];
+        }
+    }
+    uint32_t nx_key = 0;
+    int32_t nx_val = 0;
+    float nx_sh = 0.0f;
+    auto load_inputs = [&](int tile0) {
+        const int u = tile0 + tu;
+        if (u < u1) {
+            const int t = dir ? (N - 1 - u) : u;
+            nx_key = skey[t];
+            nx_val = sval[t];
+            nx_sh = has_s ? ssrt[t] : 0.0f;
+        }
+    };
+    load_inputs(u0);
+    // a context leaves one tile late, after the next tile's inputs have arrived (see k_replay)
+    f32x4 held = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4* held_dst = nullptr;
+    const float* const r_Be = s_B + p * LDS_STRIDE;
+    const float* const r_Bo = s_B + (HP + p) * LDS_STRIDE;
+    const float* const r_Ce = s_C + p * LDS_STRIDE;
+    const float* const r_Co = s_C + (HP + p) * LDS_STRIDE;
+    auto fetch4 = [&](const float* r, float (&out)[UB], int k0) {
+#pragma unroll
+        for (int q = 0; q < UB; q += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(r + k0 + q);
+#pragma unroll
+            for (int e = 0; e < 4; e++) out[q + e] = v[e];
+        }
+    };
+    int buffer = 0;
+    for (int tile0 = u0; tile0 < u1; tile0 += SCAN_TT, buffer ^= 1) {
+        float* const s_dt = s_dty[buffer];      // read by other waves until the tile after the next begins: two barriers lie between
+        const int cnt = min(SCAN_TT, u1 - tile0);
+        const uint32_t kbits = nx_key;
+        const int32_t v = nx_val;
+        const float shv = nx_sh;
+        const bool valid = tile0 + tu < u1;
+        asm volatile("" : : "v"(kbits), "v"(v), "v"(shv) : "memory");      // the wait for this tile's inputs goes here, before the store
+        if (held_dst != nullptr) *held_dst = held;
+        if (tile0 + SCAN_TT < u1) load_inputs(tile0 + SCAN_TT);
+        int orig = v & 0x7fffffff;
+        orig = valid && (unsigned)orig < (unsigned)N ? orig : 0;   // never index outside the tensor
+        const float g = valid ? sg_i2f((int32_t)kbits | (v & (int32_t)0x80000000)) : 0.0f;
+        const float sh = valid ? shv : 0.0f;
+        const unsigned long long notpoly = __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kpoly_g, kpoly_s, g, sh));
+        const bool ty = __builtin_amdgcn_ballot_w64(!sg2_taylor_ok(cmax_g, cmax_s, g, sh)) == 0;
+        const bool fast = ty && notpoly == 0;
+        unsigned long long large[2] = {0, 0}, nottiny[2] = {0, 0};
+        float dx[CPW];           // D * x-branch: of this lane's column for its SPL timesteps (fast), or of its timestep for the wave's columns
+        if (fast) {
+            s_in[tu] = g;
+            if (has_s) s_in[SCAN_TT + tu] = sh;
+            __builtin_amdgcn_wave_barrier();
+            if (has_s) project_own_rows<G, true, true>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, s_C, dx);
+            else project_own_rows<G, true, false>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, s_C, dx);
+        } else {
+            int angle[2];
+            auto run = [&](auto has_s_c, auto tay_c) {
+                project_steps<G, true, true, decltype(has_s_c)::value, decltype(tay_c)::value>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dx, angle);
+            };
+            if (ty) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
+            else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                large[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 1));
+                nottiny[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 2));
+            }
+        }
+        __syncthreads();
+
+        // the recurrences of this lane's two columns; lanes whose p is a multiple of four hold two steps' totals each
+        if (fast) {
+            const unsigned long long notlin =
+                __builtin_amdgcn_ballot_w64(!sg2_poly_ok(SG2_PROD_LINEAR_FACTOR * kpoly_g, SG2_PROD_LINEAR_FACTOR * kpoly_s, g, sh));
+#pragma unroll 1
+            for (int k0 = 0; k0 < cnt; k0 += UB) {
+                float dt[2][UB], ux[2][UB], Be[UB], Bo[UB], Ce[UB], Co[UB], y[2][UB];
+                fetch4(r_Be, Be, k0);
+                fetch4(r_Bo, Bo, k0);
+                fetch4(r_Ce, Ce, k0);
+                fetch4(r_Co, Co, k0);
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    fetch4(s_dt + col(h) * LDS_STRIDE, dt[h], k0);
+                    fetch4(s_ux + col(h) * LDS_STRIDE, ux[h], k0);
+                }
+                const unsigned long long blk = ((1ull << UB) - 1) << k0;
+                if (k0 + UB > cnt) block_steps_pair<HP, false, true, true>(S, dt, ux, Be, Bo, Ce, Co, LP, cnt - k0, y);
+                else if ((notlin & blk) == 0) block_steps_pair<HP, true, true, false>(S, dt, ux, Be, Bo, Ce, Co, LP, UB, y);
+                else block_steps_pair<HP, false, true, false>(S, dt, ux, Be, Bo, Ce, Co, LP, UB, y);
+                if ((p & 3) == 0) {
+#pragma unroll
+                    for (int h = 0; h < 2; h++) *reinterpret_cast<float2*>(&s_dt[col(h) * LDS_STRIDE + k0 + 2 * (p >> 2)]) = make_float2(y[h][0], y[h][1]);
+                }
+            }
+        } else {
+            int k0 = 0;
+            for (; k0 + UB <= cnt; k0 += UB) {
+                float Be[UB], Bo[UB], Ce[UB], Co[UB];
+                fetch4(r_Be, Be, k0);
+                fetch4(r_Bo, Bo, k0);
+                fetch4(r_Ce, Ce, k0);
+                fetch4(r_Co, Co, k0);
+                const unsigned long long blk = ((1ull << UB) - 1) << k0;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    float dt[UB], ux[UB], y[UB];
+                    fetch4(s_dt + col(h) * LDS_STRIDE, dt, k0);
+                    fetch4(s_ux + col(h) * LDS_STRIDE, ux, k0);
+                    if ((notpoly & blk) == 0)
+                        block_steps<HP, true, 3>(S[h], dt, ux, Be, Bo, Ce, Co, 0.0f, 0.0f, 0.0f, LP[h], y);
+                    else if ((nottiny[h] & blk) == 0)
+                        block_steps<HP, true, 2>(S[h], dt, ux, Be, Bo, Ce, Co, pole_e(h), pole_o(h), rope_f(h), LP[h], y);
+                    else if ((large[h] & blk) == 0)
+                        block_steps<HP, true, 1>(S[h], dt, ux, Be, Bo, Ce, Co, pole_e(h), pole_o(h), rope_f(h), LP[h], y);
+                    else
+                        block_steps<HP, true, 0>(S[h], dt, ux, Be, Bo, Ce, Co, pole_e(h), pole_o(h), rope_f(h), LP[h], y);
+                    if ((p & 3) == 0)
+                        *reinterpret_cast<float2*>(&s_dt[col(h) * LDS_STRIDE + k0 + 2 * (p >> 2)]) = make_float2(y[0], y[1]);
+                }
+            }
+            for (; k0 < cnt; k0++) {       // ragged end of the last tile of a tensor
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const float dt = s_dt[col(h) * LDS_STRIDE + k0], ux = s_ux[col(h) * LDS_STRIDE + k0];
+                    float ae, ao, sn, cs;
+                    sg_abar_pair(dt, pole_e(h), pole_o(h), &ae, &ao);
+                    sg_sincos(dt * rope_f(h), &sn, &cs);
+                    step_update<true>(S[h], ae, ao, sn, cs, ux * r_Be[k0], ux * r_Bo[k0]);
+                    const float y = pair_tree_sum<HP>(sg_fma(S[h].ho, r_Co[k0], S[h].he * r_Ce[k0]));
+                    if (p == 0) s_dt[col(h) * LDS_STRIDE + k0] = y;
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();        // a wave gates its own columns: its LDS accesses execute in program order
+
+        // gate and D skip, in place
+        if (fast) {
+            const int row = c0 + lane % CPW, t0 = SPL * (lane / CPW);
+            const f32x4 cz = *reinterpret_cast<const f32x4*>(s_coef + (SG2_COMP_Z * DI + row) * 4);
+            const f32x4 tz = *reinterpret_cast<const f32x4*>(s_tay + (DI + row) * 4);
+            auto gate = [&](auto has_s_c) {
+                constexpr bool HS = decltype(has_s_c)::value;
+#pragma unroll
+                for (int i = 0; i < SPL / 4; i++) {
+                    const f32x4 g4 = *reinterpret_cast<const f32x4*>(s_in + t0 + 4 * i);
+                    const f32x4 s4 = HS ? *reinterpret_cast<const f32x4*>(s_in + SCAN_TT + t0 + 4 * i) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    f32x4 y4 = *reinterpret_cast<const f32x4*>(s_dt + row * LDS_STRIDE + t0 + 4 * i);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float d = HS ? sg_fma(cz[0], g4[e], cz[1] * s4[e]) : cz[0] * g4[e];
+                        y4[e] = sg_fma(y4[e], sg_fma(sg_fma(sg_fma(tz[3], d, tz[2]), d, tz[1]), d, tz[0]), dx[4 * i + e]);
+                    }
+                    *reinterpret_cast<f32x4*>(s_dt + row * LDS_STRIDE + t0 + 4 * i) = y4;
+                }
+            };
+            if (has_s) gate(std::true_type{});
+            else gate(std::false_type{});
+        } else {
+            float gv[CPW];
+            if (ty) { if (has_s) gates_of<G, true, true>(g, sh, c0, s_coef, s_tay, gv); else gates_of<G, false, true>(g, sh, c0, s_coef, s_tay, gv); }
+            else { if (has_s) gates_of<G, true, false>(g, sh, c0, s_coef, s_tay, gv); else gates_of<G, false, false>(g, sh, c0, s_coef, s_tay, gv); }
+#pragma unroll
+            for (int q = 0; q < CPW; q++) s_dt[(c0 + q) * LDS_STRIDE + tu] = sg_fma(s_dt[(c0 + q) * LDS_STRIDE + tu], gv[q], dx[q]);
+        }
+        __syncthreads();
+
+        // out_proj of timesteps 16 wave .. + 15: block b of the matrix instruction is timestep quad b / 4 and rows 4 (b % 4) .. + 3
+        {
+            const int n = lane & 3, rows4 = (lane >> 2) & 3, t = 16 * wave + 4 * (lane >> 4) + n;
+            const float* w = s_wout + (4 * rows4 + n) * WSTRIDE;      // A operand: row lane % 4 of the block's four
+            const float* o = s_dt + t;                                // B operand: the lane's timestep
+            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int m = 0; m < DI; m += 4) {
+                const f32x4 w4 = *reinterpret_cast<const f32x4*>(w + m);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(w4[e], o[(m + e) * LDS_STRIDE], acc, 0, 0, 0);
+            }
+            const int at = __shfl(orig, t, 64);
+            held_dst = tile0 + t < u1 ? reinterpret_cast<f32x4*>(pl.ctx + ((size_t)dir * pl.total + off + at) * DM + 4 * rows4) : nullptr;
+            held = acc;
+        }
+    }
+    if (held_dst != nullptr) *held_dst = held;
+    if (u1 == N) {   // last chunk in scan order: new carried state of the tensor
+        float* st = dir ? T.mbwd : T.mfwd;
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (col(h) < pl.st_di && 2 * p < pl.st_ds) {
+                st[col(h) * pl.st_ds + 2 * p] = S[h].he;
+                st[col(h) * pl.st_ds + 2 * p + 1] = S[h].ho;
+            }
     }
 }
 
@@ -1239,8 +1417,8 @@ __global__ __launch_bounds__(1024) void k_chunk_prefix(Plan pl) {
 template <class G>
 int launch_scan_geo(const Plan& pl, hipStream_t st) {
     if (pl.wchunks > 0) {
-        hipLaunchKernelGGL((k_scan<G, false>), dim3(2 * pl.wchunks), dim3(G::THREADS), 0, st, pl);
-        SG_LAUNCH_CHECK("k_scan<summary>");
+        hipLaunchKernelGGL(k_summary<G>, dim3(2 * pl.wchunks), dim3(64 * Split<G>::WAVES), 0, st, pl);
+        SG_LAUNCH_CHECK("k_summary");
     }
     prof_mark(2, st);
     if (pl.wchunks > 0) {      // (tensors of one chunk start from their carried state without it)
@@ -1254,8 +1432,8 @@ int launch_scan_geo(const Plan& pl, hipStream_t st) {
         else hipLaunchKernelGGL((k_replay<G, false>), dim3(2 * pl.chunks), dim3(64), 0, st, pl);
         SG_LAUNCH_CHECK("k_replay");
     } else {
-        hipLaunchKernelGGL((k_scan<G, true>), dim3(2 * pl.chunks), dim3(G::THREADS), 0, st, pl);
-        SG_LAUNCH_CHECK("k_scan<out>");
+        hipLaunchKernelGGL(k_replay_wide<G>, dim3(2 * pl.chunks), dim3(64 * Split<G>::WAVES), 0, st, pl);
+        SG_LAUNCH_CHECK("k_replay_wide");
     }
     prof_mark(4, st);
     return 0;

@@ -177,7 +177,7 @@ int make_layout(int geo, int P, Numels numels, int chunk_len, Layout* L, bool bi
     L->off_blocksums = take(4 * (size_t)(L->nb + 1));
     L->off_summ = take(4 * 2 * (size_t)wch * 6 * gi.threads);
     L->off_hstart = take(4 * 2 * (size_t)ch * 2 * gi.threads);
-    L->off_comp = take(4 * (2 * 5 * (size_t)gi.rows * 3 + 2 * 2 * (size_t)gi.rows * 4 + 16));      // composed triples, Taylor polynomials, coefficient maxima and polynomial limits
+    L->off_comp = take(4 * (2 * 5 * (size_t)gi.rows * 3 + 2 * 2 * (size_t)gi.rows * 4 + 18));      // composed triples, Taylor polynomials, coefficient maxima and polynomial limits
     L->off_norm = take(8 * (size_t)nt);
     L->off_gscale = take(4 * (size_t)P);
     L->off_flags = take(4 * (2 * (size_t)P + 4));    // apart from the tensor records: it is written while those are being read
