@@ -242,14 +242,17 @@ class Mamba3PEERMetaNet(nn.Module):
         then per dead expert (ascending index) W1, b1, W2, b2 noise, then key A redraws per head, then
         key B redraws per head -- the sequence of the reference (mamba3_peer_metanet.py:453-488)."""
         from grokking_optimizers import _ops
-        total = self.expert_counts.sum().item()
+        # the kernels count in 32 bits: from 2^31 on (22 steps of 25 M elements) an entry reads as negative, which the draw
+        # below answers with an assertion on the device; taken modulo 2^32 it is a count again
+        counts = self.expert_counts.long() & 0xFFFFFFFF
+        total = counts.sum().item()
         if total == 0:
             return False
-        dead = ((self.expert_counts.float() / total) < self.recycle_threshold).cpu()
+        dead = ((counts.float() / total) < self.recycle_threshold).cpu()
         if not dead.any():
             self.expert_counts.zero_()
             return False
-        top = torch.multinomial(self.expert_counts.float(), 1).item()
+        top = torch.multinomial(counts.float(), 1).item()
         pk, E = self.pk_dim, self.num_experts
         flags, where = dead.tolist(), dead.nonzero(as_tuple=True)[0]
         indices = where.tolist()
