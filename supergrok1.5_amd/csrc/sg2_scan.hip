@@ -548,7 +548,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         const unsigned long long notlin =
             __builtin_amdgcn_ballot_w64(!sg2_poly_ok(SG2_PROD_LINEAR_FACTOR * kpoly_g, SG2_PROD_LINEAR_FACTOR * kpoly_s, g, sh));
         const bool tay = __builtin_amdgcn_ballot_w64(!sg2_taylor_ok(cmax_g, cmax_s, g, sh)) == 0;
-        const bool dgiven = tay && notpoly == 0;       // (steps beyond the end of the tensor carry zero inputs and qualify)
+        const bool dgiven = tay && notpoly == 0 && (!KEEP || cnt == SCAN_TT);       // (steps beyond the end of the tensor carry zero inputs and qualify)
         unsigned long long large[2] = {0, 0}, nottiny[2] = {0, 0};
         float dxv[DI];           // D * x-branch, kept for phase C: of this lane's timestep, or (dgiven) of its column's 16 timesteps
         if (dgiven) {
@@ -822,6 +822,7 @@ __device__ __forceinline__ void stage_tables(const Plan& pl, int dir, int tid, i
 // the output pass: ten instructions per step, column and pair on their linear parts, 14 on the quadratics, where the separate
 // A_bar, sin, cos and the bound on the 2x2 part took 22.  The bound needs nothing per step there: while a tile
 // qualifies, |dt - dt0| is below pl.comp's limit, so a pair's part shrinks at least by sg2_abar_bound in every step.
+// (The bilevel pass keeps the separate factors: compose_block says why.)
 // 28 us on 0.42 M elements, 82 us on 3.1 M, 141 us on 25 M, 167 us on 0.42 M with the large geometry; with one column per lane,
 // two or eight waves per chunk and the separate factors 46, 115, 212 and 254 us.
 template <class G>
@@ -928,7 +929,7 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
             if (tile0 + SCAN_TT < blk_end) load_inputs(tile0 + SCAN_TT);
             // the same 64 timesteps in every wave of the workgroup: the same decisions without talking to one another
             const bool ty = __builtin_amdgcn_ballot_w64(!sg2_taylor_ok(cmax_g, cmax_s, g, sh)) == 0;
-            const bool fast = LITE && ty && cnt % UB == 0 && __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kprod_g, kprod_s, g, sh)) == 0;
+            const bool fast = LITE && pl.htile == nullptr && ty && cnt % UB == 0 && __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kprod_g, kprod_s, g, sh)) == 0;
             unsigned long long notpoly = 0, large[2] = {0, 0}, nottiny[2] = {0, 0};
             float unused[CPW];
             if (fast) {
