@@ -8,6 +8,7 @@
 // Stands behind supergrok2_mamba_peer_batched_step (csrc/ops.cpp:815-877 of
 // the reference) in place of launch_mamba3_peer_batched_step
 // (csrc/supergrok2_mamba_peer_kernels.cu:1754-2117).
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -54,6 +55,36 @@ int auto_chunk_len(int P, Numels numels) {
 int effective_chunk_len(int P, Numels numels) {
     const int set = g_chunk_len.load();
     return set > 0 ? set : auto_chunk_len(P, numels);
+}
+
+// The chunk length of sg2_clipped_step.  512 while the chip holds all
+// chunks of 512 at once (`slots` workgroups: two waves per SIMD).  Beyond that the chunks run in rounds, and a round takes as
+// long as a chunk whether it is full or not; so does its share of the summaries, which walk `tail` steps whatever the
+// chunk's length (what the module's weights need, at the summary's cost per step).  Of the lengths that just fill
+// 1, 2, 3 ... rounds, a multiple of 128 up to 4096, the one with the least of both is taken.  Against chunks of 4096 / 2048 /
+// 1024 / 512 by the amount of work: 0.42 M elements at the large geometry 557 -> 467 us (1792 for 512), 3 M there 2.69 -> 2.47 ms
+// (3968 for 1024), 1.2 M at the default one 468 -> 430 us (1280 for 512), 3.1 M 963 -> 877 us (3200 for 1024).
+int fitted_chunk_len(int geo, int P, Numels numels) {
+    const int set = g_chunk_len.load();
+    if (set > 0) return set;
+    constexpr int STEP = 128, SHORTEST = 512, LONGEST = 4096;
+    const int64_t slots = geo == GEO_LARGE ? 512 : 2048, tail = geo == GEO_LARGE ? 288 : 128;
+    auto chunks = [&](int64_t L) {
+        int64_t n = 0;
+        for (int i = 0; i < P; i++) n += 2 * ((numels[i] + L - 1) / L);
+        return n;
+    };
+    if (chunks(SHORTEST) <= slots) return SHORTEST;
+    int64_t total = 0;
+    for (int i = 0; i < P; i++) total += numels[i];
+    const int64_t fewest = std::max<int64_t>(1, (chunks(LONGEST) + slots - 1) / slots);
+    int64_t best = LONGEST, best_cost = fewest * (LONGEST + tail);
+    for (int64_t rounds = fewest; rounds < fewest + 4; rounds++) {
+        int64_t L = std::max<int64_t>(SHORTEST, (2 * total / (rounds * slots) + STEP - 1) / STEP * STEP);      // no shorter one can do
+        while (L < LONGEST && chunks(L) > rounds * slots) L += STEP;
+        if (L < LONGEST && rounds * (L + tail) < best_cost) { best = L; best_cost = rounds * (L + tail); }
+    }
+    return (int)best;
 }
 
 // ---- optional per-stage timing with HIP events on the step's stream
@@ -394,8 +425,11 @@ size_t sg2_workspace_bytes(const SgDims* dims, int num_tensors, const int64_t* n
     const int geo = sg2::geo_of(dims);
     if (geo < 0 || num_tensors < 0 || (num_tensors > 0 && !numels)) return 0;
     sg2::Layout L;
-    if (sg2::make_layout(geo, num_tensors, sg2::Numels{numels, nullptr}, sg2::effective_chunk_len(num_tensors, sg2::Numels{numels, nullptr}), &L)) return 0;
-    return L.bytes;
+    const sg2::Numels n = {numels, nullptr};
+    if (sg2::make_layout(geo, num_tensors, n, sg2::effective_chunk_len(num_tensors, n), &L)) return 0;
+    const size_t bytes = L.bytes;
+    if (sg2::make_layout(geo, num_tensors, n, sg2::fitted_chunk_len(geo, num_tensors, n), &L)) return 0;      // sg2_clipped_step
+    return bytes > L.bytes ? bytes : L.bytes;
 }
 
 }  // extern "C"
@@ -559,6 +593,8 @@ int run_step(const SgDims* dims, const Sg2Weights* weights, int num_tensors, con
     Layout L;
     int chunk_override = 0, window_override = -1;
     if (options && num_tensors > 0 && tensors && resolve_options(options, num_tensors, Numels{nullptr, tensors}, &chunk_override, &window_override)) return 1;
+    if (clip_norm > 0.0f && num_tensors > 0 && tensors && geo_of(dims) >= 0)
+        chunk_override = fitted_chunk_len(geo_of(dims), num_tensors, Numels{nullptr, tensors});
     if (build_plan(dims, weights, num_tensors, tensors, scalars, workspace, workspace_bytes, true, false, false, st, &pl, &L, chunk_override,
                    window_override))
         return 1;
