@@ -108,6 +108,7 @@ struct Plan {
     int elem_tiles, sort_tiles, chunks, wchunks, norm_tiles;
     int sort_tile;                 // SORT_TILE or SORT_TILE_SMALL
     int sort_widest;               // sort tiles of the largest tensor
+    bool half_grads;               // every tensor's gradient is of a 16-bit type: two sort passes instead of four
     int norm_tile;
     double* norm_partials;         // [norm_tiles] sums of squares
     float* gscale;                 // [P] factor of each tensor's gradients in a clipping call (written by the sort's first kernel); NULL otherwise

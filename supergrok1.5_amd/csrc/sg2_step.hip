@@ -458,6 +458,7 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
     const int P = num_tensors;
 
     const Numels numels = {nullptr, tensors};
+    pl.half_grads = true;
     for (int i = 0; i < P; i++) {
         const Sg2Tensor& t = tensors[i];
         if (t.numel > 0) {
@@ -465,6 +466,7 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
             if (full_step && (!t.param || !t.exp_avg || !t.exp_avg_sq || !t.mu || !t.gru_state)) return sg::fail("tensor %d: NULL pointer", i);
             const int dtype = t.dtype & ~(SG_SHARP_F32 | SG_SHARP_EXACT);
             if (dtype != SG_F32 && dtype != SG_F16 && dtype != SG_BF16) return sg::fail("tensor %d: bad dtype %d", i, t.dtype);
+            pl.half_grads = pl.half_grads && dtype != SG_F32;
             if (full_step && ((uintptr_t)t.gru_state & 15u) != 0) return sg::fail("tensor %d: gru_state must be 16-byte aligned", i);
         }
     }
