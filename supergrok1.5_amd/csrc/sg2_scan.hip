@@ -8,8 +8,9 @@
 //
 // The sorted sequence of a tensor is cut into chunks of chunk_len timesteps
 // (scan order: t ascending for the forward direction, descending for the
-// backward one).  One workgroup owns one chunk: one wave for the default geometry, four for
-// the large one; a lane owns one RoPE pair p of two columns j, i.e. the states h[j][2p], h[j][2p+1] of both.
+// backward one).  One workgroup owns one chunk: one wave for the default geometry, four for the
+// large one; a lane owns one RoPE pair p of two columns j, i.e. the states h[j][2p], h[j][2p+1] of both.  (Calls that do
+// not fill the chip that way: twice the waves, one column per lane.)
 //   k_summary      every chunk but the last of a tensor: 2x2 affine summary
 //                  (M,b) of the chunk, accumulated from the identity.  The
 //                  recurrence contracts (|A_bar| < 1), so the chunk is walked
@@ -22,9 +23,10 @@
 //   k_chunk_prefix start state of each chunk: summaries applied in order to
 //                  the carried state of the tensor.
 //   k_replay       every chunk replayed from its start state: y = h.C, gate,
-//   (k_replay_wide D skip, out_proj, and the 8-float (16-float) context written
+//   (k_replay_cols D skip, out_proj, and the 8-float (16-float) context written
 //   for the large  straight to the element's original position (the "unsort").
-//   geometry)      The last chunk stores the new carried state.
+//   geometry and   The last chunk stores the new carried state.
+//   small calls)
 //   compose_block  (sg2_compose_block.hpp) runs beside the sort's first kernel: the input of a timestep is two numbers (g, s)
 //                  and every projection of the block is linear in their 8-float
 //                  input projection, so input_proj, in_proj, dt_proj, B_proj and
@@ -184,14 +186,14 @@ __device__ __forceinline__ void block_steps(LaneState& S, const float (&dt)[UB],
     }
 }
 
-// How the waves of a chunk share its recurrences: a lane owns one RoPE pair of two columns, so a chunk takes
-// THREADS / 128 waves (one for the default geometry, four for the large one), wave w the columns CPW w .. CPW w + CPW - 1:
-// lane (jl, p) = (lane / HP, lane % HP) pair p of columns CPW w + jl and CPW w + CPH + jl.
-template <class G>
+// How the waves of a chunk share its recurrences: a lane owns one RoPE pair of CL columns (two, or one where the call has
+// too few chunks to fill the chip with waves of two), so a chunk takes THREADS / (64 CL) waves, wave w the columns
+// CPW w .. CPW w + CPW - 1: lane (jl, p) = (lane / HP, lane % HP) pair p of columns CPW w + jl (and CPW w + CPH + jl).
+template <class G, int CL>
 struct Split {
-    static constexpr int WAVES = G::THREADS / 128;
+    static constexpr int WAVES = G::THREADS / (64 * CL);
     static constexpr int CPW = G::DI / WAVES;       // columns (and rows of B and C) of a wave
-    static constexpr int CPH = CPW / 2;             // ... of one of a lane's two columns over the lanes
+    static constexpr int CPH = CPW / CL;            // ... of one of a lane's columns over the lanes
     static constexpr int SPL = CPW;                 // row owners: lane (row r, part q) takes SPL consecutive timesteps of row r
     static_assert(CPH * G::HP == 64 && G::DI == G::DS && SPL * (64 / CPW) == SCAN_TT && SPL % 4 == 0, "64 lanes: CPH columns x HP pairs, CPW rows x parts");
 };
@@ -211,16 +213,16 @@ __device__ __forceinline__ int bc_slot(int r) { return (r & 1) * G::HP + (r >> 1
 // TAYLOR: every timestep of the tile has passed sg2_taylor_ok: step size and gate come from their cubic Taylor polynomials.
 // HAS_S is false for a tensor whose sharpness is all zero: fma(c_s, 0, c_0) is c_0 itself, so the term is skipped.
 // SLOTTED: rows of B and C at bc_slot.
-template <class G, bool OUT, bool SLOTTED, bool HAS_S, bool TAYLOR>
+template <class G, int CL, bool OUT, bool SLOTTED, bool HAS_S, bool TAYLOR>
 __device__ __forceinline__ void project_steps(float g, float s, int tu, int c0, const float* s_coef, const float* s_tay, const float* s_fmax, float* s_dt,
-                                              float* s_ux, float* s_B, float* s_C, float (&dxv)[Split<G>::CPW], int (&angle)[2]) {
-    constexpr int DI = G::DI, CPW = Split<G>::CPW, CPH = Split<G>::CPH;
+                                              float* s_ux, float* s_B, float* s_C, float (&dxv)[Split<G, CL>::CPW], int (&angle)[CL]) {
+    constexpr int DI = G::DI, CPW = Split<G, CL>::CPW, CPH = Split<G, CL>::CPH;
     auto delta = [&](const f32x4 t) { return HAS_S ? sg_fma(t[0], g, t[1] * s) : t[0] * g; };
     auto poly = [&](const f32x4 t, float d) { return sg_fma(sg_fma(sg_fma(t[3], d, t[2]), d, t[1]), d, t[0]); };
     auto eval = [&](const f32x4 t) { return sg_fma(t[0], g, HAS_S ? sg_fma(t[1], s, t[2]) : t[2]); };
     auto coef = [&](int group, int row) { return *reinterpret_cast<const f32x4*>(s_coef + (group * DI + row) * 4); };
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
+    for (int h = 0; h < CL; h++) {
         bool small = true, tiny = true;
 #pragma unroll
         for (int q = 0; q < CPH; q++) {
@@ -247,20 +249,20 @@ __device__ __forceinline__ void project_steps(float g, float s, int tu, int c0, 
 }
 // The gates silu(z) of the wave's columns at one timestep: Taylor polynomials for a tile that qualifies, else one column of
 // every lane at a time (CPH of them) on one shared reciprocal, the groups the checker forms.
-template <class G, bool HAS_S, bool TAYLOR>
-__device__ __forceinline__ void gates_of(float g, float s, int c0, const float* s_coef, const float* s_tay, float (&gv)[Split<G>::CPW]) {
-    constexpr int DI = G::DI, CPH = Split<G>::CPH;
+template <class G, int CL, bool HAS_S, bool TAYLOR>
+__device__ __forceinline__ void gates_of(float g, float s, int c0, const float* s_coef, const float* s_tay, float (&gv)[Split<G, CL>::CPW]) {
+    constexpr int DI = G::DI, CPH = Split<G, CL>::CPH;
     auto delta = [&](const f32x4 t) { return HAS_S ? sg_fma(t[0], g, t[1] * s) : t[0] * g; };
     auto poly = [&](const f32x4 t, float d) { return sg_fma(sg_fma(sg_fma(t[3], d, t[2]), d, t[1]), d, t[0]); };
     auto eval = [&](const f32x4 t) { return sg_fma(t[0], g, HAS_S ? sg_fma(t[1], s, t[2]) : t[2]); };
     auto coef = [&](int row) { return *reinterpret_cast<const f32x4*>(s_coef + (SG2_COMP_Z * DI + row) * 4); };
     if (TAYLOR) {
 #pragma unroll
-        for (int q = 0; q < 2 * CPH; q++) gv[q] = poly(*reinterpret_cast<const f32x4*>(s_tay + (DI + c0 + q) * 4), delta(coef(c0 + q)));
+        for (int q = 0; q < CL * CPH; q++) gv[q] = poly(*reinterpret_cast<const f32x4*>(s_tay + (DI + c0 + q) * 4), delta(coef(c0 + q)));
     } else {
         static_assert(CPH <= 8, "sg_silu_block takes at most 8 values");
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
+        for (int h = 0; h < CL; h++) {
             float zv[CPH], out[CPH];
 #pragma unroll
             for (int q = 0; q < CPH; q++) zv[q] = eval(coef(c0 + CPH * h + q));
@@ -358,19 +360,19 @@ __device__ __forceinline__ void gate_rows(int tid, const float* s_coef, const fl
     }
 }
 
-// UB steps of both columns of a lane on the products, dt - dt0 given (what block_steps<HP, true, 3> does for one column
-// with dt), written as one straight-line block so that the two independent recurrences interleave.
+// UB steps of all columns of a lane on the products, dt - dt0 given (what block_steps<HP, true, 3> does for one column
+// with dt), written as one straight-line block so that two independent recurrences interleave.
 // OUT false (summary): the states alone.  PARTIAL: the steps from `rem` on lie beyond the end of the tensor; they are
 // computed (on projections of zero inputs) and their effect on the state is taken back.
-template <int HP, bool LINEAR, bool OUT, bool PARTIAL>
-__device__ __forceinline__ void block_steps_pair(LaneState (&S)[2], const float (&dt)[2][UB], const float (&ux)[2][UB], const float (&Be)[UB],
-                                                 const float (&Bo)[UB], const float (&Ce)[UB], const float (&Co)[UB], const LanePoly<true> (&LP)[2],
-                                                 int rem, float (&y)[2][UB]) {
-    float keep[4];
+template <int HP, bool LINEAR, bool OUT, bool PARTIAL, int CL>
+__device__ __forceinline__ void block_steps_cols(LaneState (&S)[CL], const float (&dt)[CL][UB], const float (&ux)[CL][UB], const float (&Be)[UB],
+                                                 const float (&Bo)[UB], const float (&Ce)[UB], const float (&Co)[UB], const LanePoly<true> (&LP)[CL],
+                                                 int rem, float (&y)[CL][UB]) {
+    float keep[2 * CL];
 #pragma unroll
     for (int u = 0; u < UB; u++) {
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
+        for (int h = 0; h < CL; h++) {
             const float d = dt[h][u];
             const float p1 = LINEAR ? sg2_poly1(LP[h].k, d) : sg2_poly2(LP[h].k, d);
             const float n2 = LINEAR ? sg2_poly1(LP[h].k + 3, d) : sg2_poly2(LP[h].k + 3, d);
@@ -384,16 +386,16 @@ __device__ __forceinline__ void block_steps_pair(LaneState (&S)[2], const float 
         }
         if (PARTIAL && u == rem - 1) {
 #pragma unroll
-            for (int h = 0; h < 2; h++) { keep[2 * h] = S[h].he; keep[2 * h + 1] = S[h].ho; }
+            for (int h = 0; h < CL; h++) { keep[2 * h] = S[h].he; keep[2 * h + 1] = S[h].ho; }
         }
     }
     if (PARTIAL) {
 #pragma unroll
-        for (int h = 0; h < 2; h++) { S[h].he = keep[2 * h]; S[h].ho = keep[2 * h + 1]; }
+        for (int h = 0; h < CL; h++) { S[h].he = keep[2 * h]; S[h].ho = keep[2 * h + 1]; }
     }
     if (OUT) {
-        block_pair_sums<HP>(y[0]);
-        block_pair_sums<HP>(y[1]);
+#pragma unroll
+        for (int h = 0; h < CL; h++) block_pair_sums<HP>(y[h]);
     }
 }
 
@@ -558,7 +560,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             int angle[2];
             auto run = [&](auto has_s_c, auto tay_c) {
                 constexpr bool HS = decltype(has_s_c)::value, TY = decltype(tay_c)::value;
-                project_steps<G, true, false, HS, TY>(g, sh, tu, 0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, angle);
+                project_steps<G, 2, true, false, HS, TY>(g, sh, tu, 0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, angle);
             };
             if (tay) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
             else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
@@ -608,9 +610,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                                const float (&tdt)[2][UB], const float (&tux)[2][UB]) {
                 float y[2][UB];
                 const unsigned long long blk = ((1ull << UB) - 1) << kb;
-                if (kb + UB > cnt) block_steps_pair<HP, false, true, true>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, cnt - kb, y);      // the tensor's last block
-                else if ((notlin & blk) == 0) block_steps_pair<HP, true, true, false>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, UB, y);
-                else block_steps_pair<HP, false, true, false>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, UB, y);
+                if (kb + UB > cnt) block_steps_cols<HP, false, true, true>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, cnt - kb, y);      // the tensor's last block
+                else if ((notlin & blk) == 0) block_steps_cols<HP, true, true, false>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, UB, y);
+                else block_steps_cols<HP, false, true, false>(S, tdt, tux, tBe, tBo, tCe, tCo, LP, UB, y);
                 if ((p & 3) == 0) {      // the first lane of every bank holds the totals of its bank's steps (block_pair_sums)
                     *reinterpret_cast<f32x4*>(&s_y[jl * LDS_STRIDE + kb + 4 * (p >> 2)]) = f32x4{y[0][0], y[0][1], y[0][2], y[0][3]};
                     *reinterpret_cast<f32x4*>(&s_y[(jl + 8) * LDS_STRIDE + kb + 4 * (p >> 2)]) = f32x4{y[1][0], y[1][1], y[1][2], y[1][3]};
@@ -682,8 +684,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
                 for (int jj = 0; jj < DI; jj++) o[jj] = s_y[jj * LDS_STRIDE + tu];
             } else {
-                if (tay) { if (has_s) gates_of<G, true, true>(g, sh, 0, s_coef, s_tay, o); else gates_of<G, false, true>(g, sh, 0, s_coef, s_tay, o); }
-                else { if (has_s) gates_of<G, true, false>(g, sh, 0, s_coef, s_tay, o); else gates_of<G, false, false>(g, sh, 0, s_coef, s_tay, o); }
+                if (tay) { if (has_s) gates_of<G, 2, true, true>(g, sh, 0, s_coef, s_tay, o); else gates_of<G, 2, false, true>(g, sh, 0, s_coef, s_tay, o); }
+                else { if (has_s) gates_of<G, 2, true, false>(g, sh, 0, s_coef, s_tay, o); else gates_of<G, 2, false, false>(g, sh, 0, s_coef, s_tay, o); }
 #pragma unroll
                 for (int jj = 0; jj < DI; jj++) o[jj] = sg_fma(s_y[jj * LDS_STRIDE + tu], o[jj], dxv[jj]);
             }
@@ -757,10 +759,10 @@ __device__ __forceinline__ ChunkOf chunk_of(const Plan& pl, const int* chunk_pre
 // The projections of a tile that runs on the products throughout, formed by lanes that own rows: lane (row r, part q) of
 // wave w forms column CPW w + r (dt - dt0, dt * x-branch, D * x-branch) and row CPW w + r of B (and C) for timesteps SPL q ..
 // SPL q + SPL - 1.  s_in: the tile's 64 g and 64 s, the wave's own copy.  Values and reasons as in project_rows.
-template <class G, bool OUT, bool HAS_S>
+template <class G, int CL, bool OUT, bool HAS_S>
 __device__ __forceinline__ void project_own_rows(const float* s_in, int lane, int c0, const float* s_coef, const float* s_tay, float* s_dt, float* s_ux,
-                                                 float* s_B, float* s_C, float (&dxk)[Split<G>::SPL]) {
-    constexpr int DI = G::DI, CPW = Split<G>::CPW, SPL = Split<G>::SPL;
+                                                 float* s_B, float* s_C, float (&dxk)[Split<G, CL>::SPL]) {
+    constexpr int DI = G::DI, CPW = Split<G, CL>::CPW, SPL = Split<G, CL>::SPL;
     auto delta = [&](const f32x4 t, float gg, float ss) { return HAS_S ? sg_fma(t[0], gg, t[1] * ss) : t[0] * gg; };
     auto poly = [&](const f32x4 t, float d) { return sg_fma(sg_fma(sg_fma(t[3], d, t[2]), d, t[1]), d, t[0]); };
     auto eval = [&](const f32x4 t, float gg, float ss) { return sg_fma(t[0], gg, HAS_S ? sg_fma(t[1], ss, t[2]) : t[2]); };
@@ -816,6 +818,13 @@ __device__ __forceinline__ void stage_tables(const Plan& pl, int dir, int tid, i
     }
 }
 
+// What block_pair_sums leaves in the first lane of every bank: the totals of its bank's steps.
+template <int HP>
+__device__ __forceinline__ void store_sums(float* row, int p, const float (&y)[UB]) {
+    if constexpr (HP == 8) *reinterpret_cast<f32x4*>(row + 4 * (p >> 2)) = f32x4{y[0], y[1], y[2], y[3]};
+    else *reinterpret_cast<float2*>(row + 2 * (p >> 2)) = make_float2(y[0], y[1]);
+}
+
 // ---- chunk summaries
 // Bound by the vector ALU like the replay, and laid out like it: a lane owns one pair of two columns, a wave CPW columns and
 // as many rows of B, which feed both columns of a lane.  The first attempt walks the states alone on the products of
@@ -825,9 +834,9 @@ __device__ __forceinline__ void stage_tables(const Plan& pl, int dir, int tid, i
 // (The bilevel pass keeps the separate factors: compose_block says why.)
 // 28 us on 0.42 M elements, 82 us on 3.1 M, 141 us on 25 M, 167 us on 0.42 M with the large geometry; with one column per lane,
 // two or eight waves per chunk and the separate factors 46, 115, 212 and 254 us.
-template <class G>
-__global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_summary(Plan pl) {
-    constexpr int DS = G::DS, DI = G::DI, HP = G::HP, LANES = G::THREADS, WAVES = Split<G>::WAVES, CPW = Split<G>::CPW, CPH = Split<G>::CPH;
+template <class G, int CL>
+__global__ __launch_bounds__((64 * Split<G, CL>::WAVES)) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_summary(Plan pl) {
+    constexpr int DS = G::DS, DI = G::DI, HP = G::HP, LANES = G::THREADS, WAVES = Split<G, CL>::WAVES, CPW = Split<G, CL>::CPW, CPH = Split<G, CL>::CPH;
     __shared__ __attribute__((aligned(16))) float s_dt[DI * LDS_STRIDE];
     __shared__ __attribute__((aligned(16))) float s_ux[DI * LDS_STRIDE];       // dt * x-branch
     __shared__ __attribute__((aligned(16))) float s_B[DS * LDS_STRIDE];
@@ -860,10 +869,10 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
     const float cmax_g = lim[2 * dir], cmax_s = lim[2 * dir + 1];              // what decides whether a tile may use the Taylor polynomials
     const float kpoly_g = lim[4 + 2 * dir], kpoly_s = lim[5 + 2 * dir];        // ... a block the lane polynomials (sg2_poly_ok)
     const float kprod_g = lim[8 + 2 * dir], kprod_s = lim[9 + 2 * dir];        // ... a tile of the first attempt the products
-    LanePoly<true> LP[2];
-    float shrink[2];            // what eight steps on the products multiply a pair's 2x2 part by at most
+    LanePoly<true> LP[CL];
+    float shrink[CL];            // what eight steps on the products multiply a pair's 2x2 part by at most
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
+    for (int h = 0; h < CL; h++) {
         LP[h].dt0 = tay[col(h) * 4];
         const float ae = pole_e(h), ao = pole_o(h);
         sg2_pair_products(LP[h].dt0, ae, ao, rope_f(h), LP[h].k);
@@ -873,7 +882,9 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
     __syncthreads();
 
     const LaneState identity = {0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 1.0f};
-    LaneState S[2] = {identity, identity}, late[2] = {identity, identity};
+    LaneState S[CL], late[CL];
+#pragma unroll
+    for (int h = 0; h < CL; h++) S[h] = late[h] = identity;
     bool fully_contracted = false;      // the walk stopped because the 2x2 part had contracted
     bool have_late = false;
     // The chunk is walked backwards in blocks of `window` steps.  Each block is summarised from the identity and the
@@ -930,25 +941,25 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
             // the same 64 timesteps in every wave of the workgroup: the same decisions without talking to one another
             const bool ty = __builtin_amdgcn_ballot_w64(!sg2_taylor_ok(cmax_g, cmax_s, g, sh)) == 0;
             const bool fast = LITE && pl.htile == nullptr && ty && cnt % UB == 0 && __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kprod_g, kprod_s, g, sh)) == 0;
-            unsigned long long notpoly = 0, large[2] = {0, 0}, nottiny[2] = {0, 0};
+            unsigned long long notpoly = 0, large[CL] = {}, nottiny[CL] = {};
             float unused[CPW];
             if (fast) {
                 s_in[tu] = g;
                 if (has_s) s_in[SCAN_TT + tu] = sh;
                 __builtin_amdgcn_wave_barrier();      // one wave's LDS accesses execute in program order
-                if (has_s) project_own_rows<G, false, true>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, nullptr, unused);
-                else project_own_rows<G, false, false>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, nullptr, unused);
+                if (has_s) project_own_rows<G, CL, false, true>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, nullptr, unused);
+                else project_own_rows<G, CL, false, false>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, nullptr, unused);
             } else {
-                int angle[2];
+                int angle[CL];
                 auto run = [&](auto has_s_c, auto tay_c) {
-                    project_steps<G, false, true, decltype(has_s_c)::value, decltype(tay_c)::value>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B,
+                    project_steps<G, CL, false, true, decltype(has_s_c)::value, decltype(tay_c)::value>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B,
                                                                                                    nullptr, unused, angle);
                 };
                 if (ty) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
                 else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
                 notpoly = __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kpoly_g, kpoly_s, g, sh));
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
+                for (int h = 0; h < CL; h++) {
                     large[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 1));
                     nottiny[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 2));
                 }
@@ -959,24 +970,24 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
                     __builtin_amdgcn_ballot_w64(!sg2_poly_ok(SG2_PROD_LINEAR_FACTOR * kprod_g, SG2_PROD_LINEAR_FACTOR * kprod_s, g, sh));
 #pragma unroll 1
                 for (int k0 = 0; k0 < cnt; k0 += UB) {
-                    float dt[2][UB], ux[2][UB], Be[UB], Bo[UB], y[2][UB];
+                    float dt[CL][UB], ux[CL][UB], Be[UB], Bo[UB], y[CL][UB];
                     fetch4(r_Be, Be, k0);
                     fetch4(r_Bo, Bo, k0);
 #pragma unroll
-                    for (int h = 0; h < 2; h++) {
+                    for (int h = 0; h < CL; h++) {
                         fetch4(s_dt + col(h) * LDS_STRIDE, dt[h], k0);
                         fetch4(s_ux + col(h) * LDS_STRIDE, ux[h], k0);
                     }
                     const unsigned long long blk = ((1ull << UB) - 1) << k0;
-                    if ((notlin & blk) == 0) block_steps_pair<HP, true, false, false>(S, dt, ux, Be, Bo, Be, Bo, LP, UB, y);
-                    else block_steps_pair<HP, false, false, false>(S, dt, ux, Be, Bo, Be, Bo, LP, UB, y);
+                    if ((notlin & blk) == 0) block_steps_cols<HP, true, false, false>(S, dt, ux, Be, Bo, Be, Bo, LP, UB, y);
+                    else block_steps_cols<HP, false, false, false>(S, dt, ux, Be, Bo, Be, Bo, LP, UB, y);
 #pragma unroll
-                    for (int h = 0; h < 2; h++) S[h].c0e = S[h].c0e * shrink[h];
+                    for (int h = 0; h < CL; h++) S[h].c0e = S[h].c0e * shrink[h];
                 }
             } else {
                 // exceptional: one column after the other, the forms of its blocks chosen one by one
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
+                for (int h = 0; h < CL; h++) {
                     LanePoly<false> GP;
                     const float ae0 = pole_e(h), ao0 = pole_o(h), f0 = rope_f(h);
                     GP.dt0 = tay[col(h) * 4];
@@ -1014,18 +1025,21 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
     };
     if (lite) {
         walk(std::true_type{});      // c0e holds the bound (a NaN counts as "not contracted")
-        fully_contracted = !__syncthreads_or(!(S[0].c0e < SG2_FORGOTTEN) || !(S[1].c0e < SG2_FORGOTTEN));
+        bool open = false;
+#pragma unroll
+        for (int h = 0; h < CL; h++) open = open || !(S[h].c0e < SG2_FORGOTTEN);
+        fully_contracted = !__syncthreads_or(open);
         if (!fully_contracted) {     // the general walk, from the end of the chunk
             blk_first = max(u0, u1 - pl.window);
-            S[0] = identity;
-            S[1] = identity;
+#pragma unroll
+            for (int h = 0; h < CL; h++) S[h] = identity;
         }
     }
     while (!fully_contracted) {
         walk(std::false_type{});
         bool open = false;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
+        for (int h = 0; h < CL; h++) {
             if (have_late) {     // S covers [blk_first, blk_end), late covers [blk_end, u1): the summary of both is late o S
                 const LaneState E = S[h], &L = late[h];
                 S[h].c0e = sg_fma(L.c0e, E.c0e, L.c1e * E.c0o);
@@ -1043,7 +1057,7 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
         fully_contracted = !__syncthreads_or(open);
         if (fully_contracted) break;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
+        for (int h = 0; h < CL; h++) {
             late[h] = S[h];
             S[h] = identity;
         }
@@ -1053,12 +1067,12 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
     }
     if (fully_contracted) {
 #pragma unroll
-        for (int h = 0; h < 2; h++) S[h].c0e = S[h].c0o = S[h].c1e = S[h].c1o = 0.0f;
+        for (int h = 0; h < CL; h++) S[h].c0e = S[h].c0o = S[h].c1e = S[h].c1o = 0.0f;
     }
     float* sm = pl.summaries + (size_t)(dir * pl.wchunks + K.cidx) * 6 * LANES;
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int at = 128 * wave + 64 * h + lane;       // (column, pair) in the order of the columns
+    for (int h = 0; h < CL; h++) {
+        const int at = 64 * (CL * wave + h) + lane;       // (column, pair) in the order of the columns
         sm[0 * LANES + at] = S[h].c0e;   // M = [c0e c1e; c0o c1o]
         sm[1 * LANES + at] = S[h].c0o;
         sm[2 * LANES + at] = S[h].c1e;
@@ -1069,20 +1083,21 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
     if (!fully_contracted && tid == 0) *pl.contracted = 0;      // plain store: every writer stores the same value
 }
 
-// ---- the replay of the large geometry: four waves per chunk, each k_replay's wave over eight of the 32 columns
-// A wave forms its own columns and its eighth of the rows of B and C, walks its columns and gates them; what the waves share is
+// ---- the replay with several waves per chunk: the large geometry (four, two columns per lane) and small calls (one column
+// per lane: two for the default geometry, eight for the large one)
+// A wave forms its own columns and as many rows of B and C, walks its columns and gates them; what the waves share is
 // B and C, and the outputs that out_proj sums over all columns.  So a tile has two barriers (B and C stand; the gated
-// outputs stand), the row s_dt / s_y alternates between two buffers, and two workgroups (98 KB of LDS, 256 registers a
-// lane) share a compute unit to work across them.  Each B / C entry a lane fetches feeds two recurrences, and a
-// context leaves as 64 contiguous bytes: wave w multiplies timesteps 16 w .. 16 w + 15 by all of out_proj (4x4x1
+// outputs stand), the rows s_dt / s_y alternate between two buffers, and two workgroups of the large geometry (103 KB of LDS,
+// 246 registers a lane) share a compute unit to work across them.  Each B / C entry a lane fetches feeds CL recurrences, and
+// a context leaves as contiguous bytes: a wave multiplies 64 / WAVES timesteps by all of out_proj (4x4x1
 // matrix instructions, block (timestep quad, four rows): the fmaf chain over the columns, bit for bit).
-// 300 us on 0.42 M elements; as
-// one 512-lane workgroup per compute unit with a column per lane and a barrier after every phase 409 us.
-template <class G>
-__global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_replay_wide(Plan pl) {
-    constexpr int DM = G::DM, DS = G::DS, DI = G::DI, HP = G::HP, LANES = G::THREADS, WAVES = Split<G>::WAVES, CPW = Split<G>::CPW, CPH = Split<G>::CPH;
-    constexpr int SPL = Split<G>::SPL, WSTRIDE = DI + 4;        // out_proj rows: 16 lanes read 16 rows at once
-    static_assert(WAVES == 4 && DM == 16 && SCAN_TT / WAVES == 16, "out_proj roles");
+// Large geometry, 0.42 M elements: 300 us; as one 512-lane workgroup per compute unit with a column per lane, a barrier
+// after every phase and 8-byte pieces of the contexts 409 us.
+template <class G, int CL>
+__global__ __launch_bounds__((64 * Split<G, CL>::WAVES)) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_replay_cols(Plan pl) {
+    constexpr int DM = G::DM, DS = G::DS, DI = G::DI, HP = G::HP, LANES = G::THREADS, WAVES = Split<G, CL>::WAVES, CPW = Split<G, CL>::CPW, CPH = Split<G, CL>::CPH;
+    constexpr int SPL = Split<G, CL>::SPL, WSTRIDE = DI + 4;        // out_proj rows: 16 lanes read 16 rows at once
+    static_assert((SCAN_TT / WAVES) % 4 == 0 && 4 * (SCAN_TT / WAVES) * (DM / 4) <= 4 * 64, "out_proj roles");
     __shared__ __attribute__((aligned(16))) float s_dty[2][DI * LDS_STRIDE];    // dt (dt - dt0) of a column, then its y, then its gated output
     __shared__ __attribute__((aligned(16))) float s_ux[DI * LDS_STRIDE];
     __shared__ __attribute__((aligned(16))) float s_B[DS * LDS_STRIDE];
@@ -1112,9 +1127,9 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
     auto pole_e = [&](int h) { return -0.5f * -sg_exp(alog[col(h) * DS + 2 * p]); };
     auto pole_o = [&](int h) { return -0.5f * -sg_exp(alog[col(h) * DS + 2 * p + 1]); };
     auto rope_f = [&](int h) { return rope[col(h) * HP + p]; };
-    LanePoly<true> LP[2];
+    LanePoly<true> LP[CL];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
+    for (int h = 0; h < CL; h++) {
         LP[h].dt0 = pl.comp[2 * SG2_COMP_GROUPS * G::ROWS * 3 + dir * 2 * G::ROWS * 4 + col(h) * 4];
         sg2_pair_products(LP[h].dt0, pole_e(h), pole_o(h), rope_f(h), LP[h].k);
     }
@@ -1125,11 +1140,11 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
     const float cmax_g = lim[2 * dir], cmax_s = lim[2 * dir + 1];
     const float kpoly_g = lim[8 + 2 * dir], kpoly_s = lim[8 + 2 * dir + 1];
 
-    LaneState S[2];
+    LaneState S[CL];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
+    for (int h = 0; h < CL; h++) {
         S[h] = {0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 1.0f};
-        const int at = 128 * wave + 64 * h + lane;
+        const int at = 64 * (CL * wave + h) + lane;
         if (c > 0 && __builtin_amdgcn_readfirstlane(*pl.contracted) != 0) {
             const float* sm = pl.summaries + (size_t)(dir * pl.wchunks + pl.wchunk_prefix[K.ti] + c - 1) * 6 * LANES;
             S[h].he = sm[4 * LANES + at];
@@ -1192,23 +1207,23 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
         const unsigned long long notpoly = __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kpoly_g, kpoly_s, g, sh));
         const bool ty = __builtin_amdgcn_ballot_w64(!sg2_taylor_ok(cmax_g, cmax_s, g, sh)) == 0;
         const bool fast = ty && notpoly == 0;
-        unsigned long long large[2] = {0, 0}, nottiny[2] = {0, 0};
+        unsigned long long large[CL] = {}, nottiny[CL] = {};
         float dx[CPW];           // D * x-branch: of this lane's column for its SPL timesteps (fast), or of its timestep for the wave's columns
         if (fast) {
             s_in[tu] = g;
             if (has_s) s_in[SCAN_TT + tu] = sh;
             __builtin_amdgcn_wave_barrier();
-            if (has_s) project_own_rows<G, true, true>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, s_C, dx);
-            else project_own_rows<G, true, false>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, s_C, dx);
+            if (has_s) project_own_rows<G, CL, true, true>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, s_C, dx);
+            else project_own_rows<G, CL, true, false>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, s_C, dx);
         } else {
-            int angle[2];
+            int angle[CL];
             auto run = [&](auto has_s_c, auto tay_c) {
-                project_steps<G, true, true, decltype(has_s_c)::value, decltype(tay_c)::value>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dx, angle);
+                project_steps<G, CL, true, true, decltype(has_s_c)::value, decltype(tay_c)::value>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dx, angle);
             };
             if (ty) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
             else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
+            for (int h = 0; h < CL; h++) {
                 large[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 1));
                 nottiny[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 2));
             }
@@ -1221,23 +1236,23 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
                 __builtin_amdgcn_ballot_w64(!sg2_poly_ok(SG2_PROD_LINEAR_FACTOR * kpoly_g, SG2_PROD_LINEAR_FACTOR * kpoly_s, g, sh));
 #pragma unroll 1
             for (int k0 = 0; k0 < cnt; k0 += UB) {
-                float dt[2][UB], ux[2][UB], Be[UB], Bo[UB], Ce[UB], Co[UB], y[2][UB];
+                float dt[CL][UB], ux[CL][UB], Be[UB], Bo[UB], Ce[UB], Co[UB], y[CL][UB];
                 fetch4(r_Be, Be, k0);
                 fetch4(r_Bo, Bo, k0);
                 fetch4(r_Ce, Ce, k0);
                 fetch4(r_Co, Co, k0);
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
+                for (int h = 0; h < CL; h++) {
                     fetch4(s_dt + col(h) * LDS_STRIDE, dt[h], k0);
                     fetch4(s_ux + col(h) * LDS_STRIDE, ux[h], k0);
                 }
                 const unsigned long long blk = ((1ull << UB) - 1) << k0;
-                if (k0 + UB > cnt) block_steps_pair<HP, false, true, true>(S, dt, ux, Be, Bo, Ce, Co, LP, cnt - k0, y);
-                else if ((notlin & blk) == 0) block_steps_pair<HP, true, true, false>(S, dt, ux, Be, Bo, Ce, Co, LP, UB, y);
-                else block_steps_pair<HP, false, true, false>(S, dt, ux, Be, Bo, Ce, Co, LP, UB, y);
+                if (k0 + UB > cnt) block_steps_cols<HP, false, true, true>(S, dt, ux, Be, Bo, Ce, Co, LP, cnt - k0, y);
+                else if ((notlin & blk) == 0) block_steps_cols<HP, true, true, false>(S, dt, ux, Be, Bo, Ce, Co, LP, UB, y);
+                else block_steps_cols<HP, false, true, false>(S, dt, ux, Be, Bo, Ce, Co, LP, UB, y);
                 if ((p & 3) == 0) {
 #pragma unroll
-                    for (int h = 0; h < 2; h++) *reinterpret_cast<float2*>(&s_dt[col(h) * LDS_STRIDE + k0 + 2 * (p >> 2)]) = make_float2(y[h][0], y[h][1]);
+                    for (int h = 0; h < CL; h++) store_sums<HP>(s_dt + col(h) * LDS_STRIDE + k0, p, y[h]);
                 }
             }
         } else {
@@ -1250,7 +1265,7 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
                 fetch4(r_Co, Co, k0);
                 const unsigned long long blk = ((1ull << UB) - 1) << k0;
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
+                for (int h = 0; h < CL; h++) {
                     float dt[UB], ux[UB], y[UB];
                     fetch4(s_dt + col(h) * LDS_STRIDE, dt, k0);
                     fetch4(s_ux + col(h) * LDS_STRIDE, ux, k0);
@@ -1262,13 +1277,12 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
                         block_steps<HP, true, 1>(S[h], dt, ux, Be, Bo, Ce, Co, pole_e(h), pole_o(h), rope_f(h), LP[h], y);
                     else
                         block_steps<HP, true, 0>(S[h], dt, ux, Be, Bo, Ce, Co, pole_e(h), pole_o(h), rope_f(h), LP[h], y);
-                    if ((p & 3) == 0)
-                        *reinterpret_cast<float2*>(&s_dt[col(h) * LDS_STRIDE + k0 + 2 * (p >> 2)]) = make_float2(y[0], y[1]);
+                    if ((p & 3) == 0) store_sums<HP>(s_dt + col(h) * LDS_STRIDE + k0, p, y);
                 }
             }
             for (; k0 < cnt; k0++) {       // ragged end of the last tile of a tensor
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
+                for (int h = 0; h < CL; h++) {
                     const float dt = s_dt[col(h) * LDS_STRIDE + k0], ux = s_ux[col(h) * LDS_STRIDE + k0];
                     float ae, ao, sn, cs;
                     sg_abar_pair(dt, pole_e(h), pole_o(h), &ae, &ao);
@@ -1305,16 +1319,17 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
             else gate(std::false_type{});
         } else {
             float gv[CPW];
-            if (ty) { if (has_s) gates_of<G, true, true>(g, sh, c0, s_coef, s_tay, gv); else gates_of<G, false, true>(g, sh, c0, s_coef, s_tay, gv); }
-            else { if (has_s) gates_of<G, true, false>(g, sh, c0, s_coef, s_tay, gv); else gates_of<G, false, false>(g, sh, c0, s_coef, s_tay, gv); }
+            if (ty) { if (has_s) gates_of<G, CL, true, true>(g, sh, c0, s_coef, s_tay, gv); else gates_of<G, CL, false, true>(g, sh, c0, s_coef, s_tay, gv); }
+            else { if (has_s) gates_of<G, CL, true, false>(g, sh, c0, s_coef, s_tay, gv); else gates_of<G, CL, false, false>(g, sh, c0, s_coef, s_tay, gv); }
 #pragma unroll
             for (int q = 0; q < CPW; q++) s_dt[(c0 + q) * LDS_STRIDE + tu] = sg_fma(s_dt[(c0 + q) * LDS_STRIDE + tu], gv[q], dx[q]);
         }
         __syncthreads();
 
-        // out_proj of timesteps 16 wave .. + 15: block b of the matrix instruction is timestep quad b / 4 and rows 4 (b % 4) .. + 3
+        // out_proj of the wave's SCAN_TT / WAVES timesteps: a block of the matrix instruction is four timesteps by four rows
         {
-            const int n = lane & 3, rows4 = (lane >> 2) & 3, t = 16 * wave + 4 * (lane >> 4) + n;
+            constexpr int GROUPS = DM / 4, TW = SCAN_TT / WAVES;
+            const int n = lane & 3, rows4 = (lane >> 2) % GROUPS, quad = (lane >> 2) / GROUPS, t = (TW * wave + 4 * quad + n) & (SCAN_TT - 1);
             const float* w = s_wout + (4 * rows4 + n) * WSTRIDE;      // A operand: row lane % 4 of the block's four
             const float* o = s_dt + t;                                // B operand: the lane's timestep
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1325,7 +1340,8 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
                 for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(w4[e], o[(m + e) * LDS_STRIDE], acc, 0, 0, 0);
             }
             const int at = __shfl(orig, t, 64);
-            held_dst = tile0 + t < u1 ? reinterpret_cast<f32x4*>(pl.ctx + ((size_t)dir * pl.total + off + at) * DM + 4 * rows4) : nullptr;
+            const bool mine = 4 * quad < TW && tile0 + t < u1;       // (eight waves have twice the lanes that the timesteps need)
+            held_dst = mine ? reinterpret_cast<f32x4*>(pl.ctx + ((size_t)dir * pl.total + off + at) * DM + 4 * rows4) : nullptr;
             held = acc;
         }
     }
@@ -1333,7 +1349,7 @@ __global__ __launch_bounds__(64 * Split<G>::WAVES) __attribute__((amdgpu_waves_p
     if (u1 == N) {   // last chunk in scan order: new carried state of the tensor
         float* st = dir ? T.mbwd : T.mfwd;
 #pragma unroll
-        for (int h = 0; h < 2; h++)
+        for (int h = 0; h < CL; h++)
             if (col(h) < pl.st_di && 2 * p < pl.st_ds) {
                 st[col(h) * pl.st_ds + 2 * p] = S[h].he;
                 st[col(h) * pl.st_ds + 2 * p + 1] = S[h].ho;
@@ -1415,10 +1431,26 @@ __global__ __launch_bounds__(1024) void k_chunk_prefix(Plan pl) {
     }
 }
 
+template <class G, int CL>
+void launch_summary(const Plan& pl, hipStream_t st) {
+    hipLaunchKernelGGL((k_summary<G, CL>), dim3(2 * pl.wchunks), dim3(64 * Split<G, CL>::WAVES), 0, st, pl);
+}
+template <class G, int CL>
+void launch_replay_cols(const Plan& pl, hipStream_t st) {
+    hipLaunchKernelGGL((k_replay_cols<G, CL>), dim3(2 * pl.chunks), dim3(64 * Split<G, CL>::WAVES), 0, st, pl);
+}
+
 template <class G>
 int launch_scan_geo(const Plan& pl, hipStream_t st) {
+    // One column per lane while all waves of the call are then resident at once (two per SIMD): a chunk's steps are a serial
+    // chain, and a wave alone on its SIMD takes as long for one column's instructions as two waves for theirs.  Replay and
+    // summaries of 30 000 elements 151 -> 121 us a step (large geometry 182 -> 157), of 200 000 217 -> 194; past the line
+    // 300 000 elements 236 -> 243 us, 120 000 at the large geometry 265 -> 284.
+    constexpr int RESIDENT = 2 * 4 * 256;
+    const auto single = [](int chunks) { return 2 * chunks * Split<G, 1>::WAVES <= RESIDENT; };
     if (pl.wchunks > 0) {
-        hipLaunchKernelGGL(k_summary<G>, dim3(2 * pl.wchunks), dim3(64 * Split<G>::WAVES), 0, st, pl);
+        if (single(pl.wchunks)) launch_summary<G, 1>(pl, st);
+        else launch_summary<G, 2>(pl, st);
         SG_LAUNCH_CHECK("k_summary");
     }
     prof_mark(2, st);
@@ -1427,15 +1459,17 @@ int launch_scan_geo(const Plan& pl, hipStream_t st) {
         SG_LAUNCH_CHECK("k_chunk_prefix");
     }
     prof_mark(3, st);
-    if (pl.htile != nullptr && G::PARTS != 2) return sg::fail("the bilevel pass is built for the default meta-net dimensions only");
-    if constexpr (G::PARTS == 2) {          // one wave per chunk, two columns per lane
+    constexpr bool DEFAULT = G::THREADS == 128;
+    if (pl.htile != nullptr && !DEFAULT) return sg::fail("the bilevel pass is built for the default meta-net dimensions only");
+    if (pl.htile == nullptr && single(pl.chunks)) {
+        launch_replay_cols<G, 1>(pl, st);
+    } else if constexpr (DEFAULT) {          // one wave per chunk, two columns per lane
         if (pl.htile != nullptr) hipLaunchKernelGGL((k_replay<G, true>), dim3(2 * pl.chunks), dim3(64), 0, st, pl);
         else hipLaunchKernelGGL((k_replay<G, false>), dim3(2 * pl.chunks), dim3(64), 0, st, pl);
-        SG_LAUNCH_CHECK("k_replay");
     } else {
-        hipLaunchKernelGGL(k_replay_wide<G>, dim3(2 * pl.chunks), dim3(64 * Split<G>::WAVES), 0, st, pl);
-        SG_LAUNCH_CHECK("k_replay_wide");
+        launch_replay_cols<G, 2>(pl, st);
     }
+    SG_LAUNCH_CHECK("k_replay");
     prof_mark(4, st);
     return 0;
 }

@@ -19,7 +19,18 @@ SHAPES = [(1,), (7,), (8,), (9,), (63,), (64,), (65,), (71,), (127,), (512,), (5
 @pytest.mark.parametrize("std", [1e-4, 3e-3, 0.05, 2.0])
 @pytest.mark.parametrize("dims", [None, LARGE], ids=["default", "large"])
 def test_bit_identical_to_the_checker(dims, std, sharp):
-    case = Sg2Case(SHAPES, seed=4, random_state=True, dims=dims)
+    _compare(SHAPES, dims, std, sharp)
+
+
+@pytest.mark.parametrize("std", [1e-3, 0.3])
+@pytest.mark.parametrize("dims,more", [(None, [(13000,)] * 24), (LARGE, [(5003,)] * 16)], ids=["default", "large"])
+def test_bit_identical_with_chunks_that_fill_the_chip(dims, more, std):
+    """Enough chunks for two columns per lane (the sets above take one)."""
+    _compare(SHAPES + more, dims, std, True)
+
+
+def _compare(shapes, dims, std, sharp):
+    case = Sg2Case(shapes, seed=4, random_state=True, dims=dims)
     for t in (1, 2):
         grads = wl.make_grads(case.shapes, seed=20 + t, std=std)
         sharps = [g.abs() * 0.5 for g in wl.make_grads(case.shapes, seed=520 + t, std=std)] if sharp else [torch.zeros_like(g) for g in grads]
