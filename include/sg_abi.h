@@ -98,7 +98,7 @@ const char* sg_last_error(void);
 /* Length (timesteps) of the scan chunks a tensor's sorted sequence is cut
  * into; a multiple of 64.  0 (the default) lets each call choose 4096, 2048,
  * 1024 or 512 from the amount of work; sg2_chunk_len_for tells what a call with
- * these tensor sizes will use.  sg2_clipped_step chooses, between 512 and 4096,
+ * these tensor sizes will use.  sg2_clipped_step chooses, between 256 and 4096,
  * the length whose chunks fill the chip in whole rounds.  Affects results only by re-association of the chunk products. */
 int sg2_set_chunk_len(int chunk_len);
 int sg2_get_chunk_len(void);

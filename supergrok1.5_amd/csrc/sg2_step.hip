@@ -57,7 +57,10 @@ int effective_chunk_len(int P, Numels numels) {
     return set > 0 ? set : auto_chunk_len(P, numels);
 }
 
-// The chunk length of sg2_clipped_step.  512 while the chip holds all
+// The chunk length of sg2_clipped_step.  256 for small calls at the default geometry, while the chip has a SIMD for each of
+// their waves (one column per lane, so two a chunk): the replay is then half as long, and so is what the summaries of the
+// module's weights need (184 to 240 steps) less than a chunk (30 000 elements 121 -> 105 us a step, 600 in one tensor
+// 82 -> 67; with every pole slowed by e, whose summaries need more, 125 -> 140, by e^2 171 -> 141).  512 while the chip holds all
 // chunks of 512 at once (`slots` workgroups: two waves per SIMD).  Beyond that the chunks run in rounds, and a round takes as
 // long as a chunk whether it is full or not; so does its share of the summaries, which walk `tail` steps whatever the
 // chunk's length (what the module's weights need, at the summary's cost per step).  Of the lengths that just fill
@@ -74,7 +77,11 @@ int fitted_chunk_len(int geo, int P, Numels numels) {
         for (int i = 0; i < P; i++) n += 2 * ((numels[i] + L - 1) / L);
         return n;
     };
-    if (chunks(SHORTEST) <= slots) return SHORTEST;
+    if (chunks(SHORTEST) <= slots) {
+        int64_t widest = 0;
+        for (int i = 0; i < P; i++) widest = std::max(widest, numels[i]);
+        return geo == GEO_DEFAULT && widest > SHORTEST && 2 * chunks(SHORTEST / 2) <= 1024 ? SHORTEST / 2 : SHORTEST;
+    }
     int64_t total = 0;
     for (int i = 0; i < P; i++) total += numels[i];
     const int64_t fewest = std::max<int64_t>(1, (chunks(LONGEST) + slots - 1) / slots);
