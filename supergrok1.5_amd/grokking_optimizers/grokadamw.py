@@ -11,7 +11,7 @@ import torch
 from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import check_hyper, gather, run_closure
+from grokking_optimizers._common import check_hyper, gather, observed_step, run_closure
 
 
 class GrokAdamW(Optimizer):
@@ -24,6 +24,7 @@ class GrokAdamW(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay, alpha=alpha, lamb=lamb,
                                       gamma=gamma, decay=decay, grad_clip=grad_clip))
 
+    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         for group in self.param_groups:

@@ -14,6 +14,7 @@ from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
 from grokking_optimizers._adamw_helper import adamw_step
+from grokking_optimizers._common import observed_step
 
 
 class Grokfast(Optimizer):
@@ -34,6 +35,7 @@ class Grokfast(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay,
                                       grokfast_alpha=grokfast_alpha, grokfast_lamb=grokfast_lamb))
 
+    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = None
         if closure is not None:

@@ -10,7 +10,7 @@ import torch
 from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import check_hyper, run_closure
+from grokking_optimizers._common import check_hyper, observed_step, run_closure
 
 
 class Lion(Optimizer):
@@ -19,6 +19,7 @@ class Lion(Optimizer):
         check_hyper(lr, None, betas)
         super().__init__(params, dict(lr=lr, betas=betas, weight_decay=weight_decay))
 
+    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         for group in self.param_groups:

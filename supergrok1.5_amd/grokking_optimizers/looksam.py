@@ -15,7 +15,7 @@ from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
 from grokking_optimizers._adamw_helper import adamw_step
-from grokking_optimizers._common import check_hyper, gather, run_closure
+from grokking_optimizers._common import check_hyper, gather, observed_step, run_closure
 
 
 class LookSAM(Optimizer):
@@ -31,6 +31,7 @@ class LookSAM(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay, rho=rho, k=k, alpha=alpha))
         self._global_step: int = 0
 
+    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         self._global_step += 1

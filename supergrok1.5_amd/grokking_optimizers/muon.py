@@ -9,7 +9,7 @@ from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
 from grokking_optimizers._adamw_helper import adamw_step
-from grokking_optimizers._common import check_ranges
+from grokking_optimizers._common import check_ranges, observed_step
 
 
 class Muon(Optimizer):
@@ -33,6 +33,7 @@ class Muon(Optimizer):
         super().__init__(groups, dict(lr=lr, momentum=momentum, weight_decay=weight_decay, ns_steps=ns_steps,
                                       group_type="muon"))
 
+    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = None
         if closure is not None:

@@ -13,7 +13,7 @@ import torch.nn as nn
 from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import check_hyper, gather, run_closure
+from grokking_optimizers._common import check_hyper, gather, observed_step, run_closure
 
 
 class _Amplifier(nn.Module):
@@ -58,6 +58,7 @@ class NeuralGrok(Optimizer):
             return tuple(w.to(dev) for w in weights)
         return _ops.amplifier_on(weights, self._device_weights, dev)
 
+    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         if self._meta_weights_dirty or self._cached_meta_weights is None:

@@ -11,7 +11,7 @@ import torch
 from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import check_hyper, gather, run_closure
+from grokking_optimizers._common import check_hyper, gather, observed_step, run_closure
 
 
 class Prodigy(Optimizer):
@@ -21,6 +21,7 @@ class Prodigy(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay))
         self._d_lr: float = 1e-6
 
+    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
 

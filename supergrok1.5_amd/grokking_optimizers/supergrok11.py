@@ -17,6 +17,7 @@ import torch.nn as nn
 from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
+from grokking_optimizers._common import observed_step
 from grokking_optimizers._meta_training import MetaTraining
 from grokking_optimizers._schedule import GrokSchedule
 from grokking_optimizers.supergrok15 import SharpnessMetaNet
@@ -72,6 +73,7 @@ class SuperGrok11(MetaTraining, Optimizer):
         """999999 (off) below sam_enable_threshold, else 1: the training loop decides the actual frequency."""
         return 999999 if self._cached_train_acc < self.sam_enable_threshold else 1
 
+    @observed_step
     def step(self, closure=None, train_loss=None, val_loss=None, train_acc=None):
         loss = None
         if closure is not None:

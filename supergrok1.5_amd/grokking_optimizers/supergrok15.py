@@ -15,6 +15,7 @@ import torch.nn as nn
 from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
+from grokking_optimizers._common import observed_step
 from grokking_optimizers._meta_training import MetaTraining, ScheduledTraining
 from grokking_optimizers._schedule import GrokSchedule
 
@@ -99,6 +100,7 @@ class SuperGrok15(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
             self._flat_sharpness.append(mk())
         self._state_initialized = True
 
+    @observed_step
     def step(self, closure=None, train_loss=None, val_loss=None, train_acc=None):
         loss = None
         if closure is not None:

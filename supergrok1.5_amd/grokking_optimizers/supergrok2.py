@@ -32,6 +32,7 @@ import torch.nn as nn
 from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
+from grokking_optimizers._common import observed_step
 from grokking_optimizers._meta_training import MetaTraining, ScheduledTraining
 from grokking_optimizers._schedule import GrokSchedule
 from grokking_optimizers.mamba3_peer_metanet import Mamba3PEERMetaNet
@@ -108,6 +109,7 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
         three launches for all tensors, norms reduced on the device, no host syncs."""
         return _ops.supergrok2_clip_grads([g.contiguous() for g in grads], float(self.gradient_clipping))
 
+    @observed_step
     def step(self, closure=None, train_loss=None, val_loss=None, train_acc=None):
         loss = None
         if closure is not None:
