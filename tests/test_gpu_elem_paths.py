@@ -76,6 +76,32 @@ def test_amplifier_table_stays_within_its_rounding(spread):
     assert (err <= 2.0 ** -24 * 1.01 * (np.abs(A * x) + np.abs(B) + 2 * np.abs(value)) + 1e-30).all(), float(err.max())
 
 
+@pytest.mark.parametrize("H", [63, 64, 65, 128, 129, 193, 256])
+def test_amplifier_table_across_waves(H):
+    """Widths at which the running sums cross a wave, with equal thresholds, thresholds that overflow to either infinity and units
+    that do not look at the gradient, against float64: the line's rounding as above, and each of H float64 additions 2^-53."""
+    r = np.random.RandomState(H)
+    w1, b1, w2 = (r.uniform(-1, 1, s).astype(np.float32) for s in ((H, 1), (H,), (1, H)))
+    w1[1::6], b1[1::6] = 0.5, -0.25                    # all at 0.5, rising
+    w1[2::6], b1[2::6] = -0.5, 0.25                    # all at 0.5, falling
+    w1[3::12], b1[3::12] = 1e-39, 0.75                 # -inf
+    w1[9::12], b1[9::12] = -1e-39, 0.75                # +inf, always active
+    w1[4::6] = 0.0
+    g = np.concatenate([r.randn(20_000), np.float32([0.5, -0.5, 3e38, -3e38, 1e-30])]).astype(np.float32)
+    got = {k: _dev([x]) for k, x in dict(p=np.zeros_like(g), g=g, ea=np.zeros_like(g), easq=np.zeros_like(g)).items()}
+    W = [torch.from_numpy(x).to(DEV) for x in (w1, b1, w2, np.float32([0.0]))]
+    _ops().neuralgrok_fused_step(got["p"], got["g"], got["ea"], got["easq"], [3], *W, 1.0, 0.0, H, 0.0, 0.98, 1e-3, 1.0, 1e-8, 0.0)
+    x, w1, b1, w2 = (a.astype(np.float64).reshape(-1) for a in (g, w1, b1, w2))
+    active = w1[:, None] * x + b1[:, None] > 0
+    A, B = ((active * (w2 * c)[:, None]).sum(0) for c in (w1, b1))
+    sA, sB = ((active * np.abs(w2 * c)[:, None]).sum(0) for c in (w1, b1))
+    value = A * x + B
+    sel = np.abs(x) < 1e4                              # the product with g overflows for the largest
+    err = np.abs(got["ea"][0].cpu().numpy() / x - value)
+    bound = 2.0 ** -24 * 1.01 * (np.abs(A * x) + np.abs(B) + 2 * np.abs(value)) + H * 2.0 ** -53 * (sA * np.abs(x) + sB) + 1e-30
+    assert (err <= bound)[sel].all(), float((err / bound)[sel].max())
+
+
 @pytest.mark.parametrize("H", [1, 32, 256])
 @pytest.mark.parametrize("gstd", [1e-3, 0.03, 1.0])
 def test_meta_net_polynomial(H, gstd):
