@@ -744,156 +744,266 @@ __global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, int y_sel, int
 }
 
 // ---- all iterations of one matrix in one workgroup: Y [mp x np] (mp 64 or 128) and G, then H in its place, stay in LDS.
-// Eight waves.  G and G G: 32x32 tiles, one row of tiles to a pair of waves; apply: strips of 32 columns, whose Y' replaces
+// Eight waves.  G and G G: 32x32 tiles, those left of the diagonal mirrored; apply: strips of 32 columns, whose Y' replaces
 // their Y (a strip is read by its own wave only).  Same roundings as the GEMM path: G, H and Y are bf16 between the
 // products, the first step carries 1/norm^2 and 1/norm.
-// Rows lie 16-byte chunk by chunk, chunk c of row r at c ^ swizzle(r): consecutive rows' chunks fall on different banks.
-// Bound by LDS operand fetches (1.25 to 1.5 per MFMA) and the barriers between the products: 50 us for five iterations of
-// 128 x 512, the largest, where fifteen launches of k_gemm_nt took 180.
+// Rows lie 16-byte chunk by chunk, chunk c of row r at c ^ ns_swizzle(r): a quarter wave's 16-byte reads of a chunk of
+// consecutive rows and the transposing reads of four rows of four chunks both meet every bank once (with the row's low bits
+// as they are, the transposing read took 8 cycles instead of 2.5).
+// One CU per matrix.  Of an iteration of 128 x 512, the largest, about 15 400 cycles: matrix cores 7900, and the ends of
+// three dependent products (operands on their way, conversion, LDS writes at 64 bytes a cycle, a barrier each).
+// 41 us for five; 50 before the products' operand addresses were kept in registers, the reads dealt between the matrix
+// instructions and half of the symmetric products left out; 180 as fifteen launches of k_gemm_nt.
 constexpr int NS_THREADS = 512;
 constexpr int NS_Y_ELEMS = 128 * 512;          // Y: 128 KB ...
 constexpr int NS_LDS_BYTES = 2 * (NS_Y_ELEMS + 128 * 128);      // ... and G: 32 KB, all of a CU's 160 KB
 inline bool fits_lds(int mp, int np) { return mp <= 128 && mp * np <= NS_Y_ELEMS; }
-__device__ __forceinline__ int ns_swizzle(int row, int width) { return (width & 64) ? (row >> 1) & 7 : row & 15; }
+// of a row, its low bits dealt to the bits of a chunk's place; linear over exclusive or
+__device__ __forceinline__ constexpr int ns_swizzle(int row, bool odd) { return odd ? ((row & 2) << 1) | ((row >> 2) & 3) : ((row & 3) << 2) | ((row >> 2) & 3); }
 
 template <int MT>       // mp / 32
-__device__ __forceinline__ void newton_schulz(const Mat& M, float inv, int steps, bf16_t* __restrict__ sY, bf16_t* __restrict__ sG) {
-    constexpr int mp = 32 * MT, TPW = MT == 4 ? 2 : 1;       // tiles of a row of tiles per wave
-    const int np = M.np, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int r32 = lane & 31, kh = lane >> 5;
-    {
-        const int chunks = np / 8;
-        const u32x4* __restrict__ src = reinterpret_cast<const u32x4*>(M.Y);
-        for (int i = tid; i < mp * chunks; i += NS_THREADS) {
-            const int r = i / chunks, c = i % chunks;
-            *reinterpret_cast<u32x4*>(sY + (size_t)r * np + (c ^ ns_swizzle(r, np)) * 8) = *(gvec_p)(src + i);
+__device__ __forceinline__ void newton_schulz(const Mat& M, float inv, int steps, bf16_t* __restrict__ smem) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(3))) unsigned char* lds_t;
+    typedef __attribute__((address_space(3))) bf16x8* lds_op;
+    typedef __attribute__((address_space(3))) u32x4* lds_vec;
+    typedef __attribute__((address_space(3))) bf16_t* lds_b16;
+    constexpr int mp = 32 * MT, WAVES = NS_THREADS / 64, GROW = 2 * mp, BATCH = 16;
+    const int np = M.np, row = 2 * np, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const bool odd = np & 64;
+    const lds_t Y = (lds_t)smem, G = Y + mp * row;
+    // sixteen bytes of every chunk in order, a batch of them on their way at once
+    const int chunks = np / 8, dr = NS_THREADS / chunks, dc = NS_THREADS % chunks;
+    auto stream = [&](auto move) {
+        int r = tid / chunks, c = tid % chunks;
+        for (int i = tid; i < mp * chunks; i += BATCH * NS_THREADS) {
+            int at[BATCH];
+#pragma unroll
+            for (int u = 0; u < BATCH; u++) {
+                at[u] = r * row + ((c ^ ns_swizzle(r, odd)) << 4);
+                r += dr;
+                c += dc;
+                if (c >= chunks) { c -= chunks; r++; }
+            }
+            move(i, at, min(BATCH, (mp * chunks - i + NS_THREADS - 1) / NS_THREADS));
         }
+    };
+    {
+        const u32x4* __restrict__ src = reinterpret_cast<const u32x4*>(M.Y);
+        stream([&](int i, const int (&at)[BATCH], int n) {
+            u32x4 v[BATCH];
+#pragma unroll
+            for (int u = 0; u < BATCH; u++) if (u < n) v[u] = *(gvec_p)(src + i + u * NS_THREADS);
+#pragma unroll
+            for (int u = 0; u < BATCH; u++) if (u < n) *(lds_vec)(Y + at[u]) = v[u];
+        });
     }
     __syncthreads();
-    // eight consecutive k of row r of a [rows x width] array
-    auto chunk = [](const bf16_t* s, int width, int r, int c) {
-        return *reinterpret_cast<const bf16x8*>(s + (size_t)r * width + (c ^ ns_swizzle(r, width)) * 8);
-    };
-    // four consecutive columns c .. c + 3 (c a multiple of 4) of row r
-    auto at = [](int width, int r, int c) { return (size_t)r * width + (((c >> 3) ^ ns_swizzle(r, width)) << 3) + (c & 4); };
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    const bool active = wave < MT * MT / TPW;
-    const int rt = active ? wave / (MT / TPW) : 0, ct = active ? (wave % (MT / TPW)) * TPW : 0;
+    // S S^T is symmetric: the tiles on and right of the diagonal, dealt so that the waves of a SIMD (w and w + 4) have at most
+    // three; each reads the rows of its row of tiles rt and, with a tile off the diagonal, those of ct.
+    const bool on = MT == 4 ? wave < 2 || wave == 4 || wave == 5 : wave < 2, off = MT == 4 ? wave != 4 && wave != 5 : wave == 2;
+    const int rt = MT == 4 ? (wave < 2 ? 2 * wave : wave == 4 ? 1 : wave == 5 ? 3 : wave & 1) : wave & 1;
+    const int ct = MT == 4 ? (wave < 2 ? 2 * wave + 1 : wave < 4 ? 2 : 3) : 1;
+#pragma unroll 1
     for (int it = 0; it < steps; it++) {
-        const float g_scale = it == 0 ? inv * inv : 1.0f, y_scale = it == 0 ? inv : 1.0f;
-        f32x16 acc[TPW];
-        // the wave's tiles of S S^T, S [mp x width]
-        auto gram = [&](const bf16_t* s, int width) {
+        int ln = lane;                       // keeps the address arithmetic in its phase: hoisted out of the loop it spills
+        asm volatile("" : "+v"(ln));
+        const int r32 = ln & 31, kh = ln >> 5;
+        // a tile's 32 columns of a row, four of every eight in this lane (4 kh ..) and four in the lane 32 away: two exchanges give
+        // each lane a whole chunk
+        auto put_row = [&](lds_t at, u32x2 v, u32x2 w) {
+            const auto x = __builtin_amdgcn_permlane32_swap(v[0], w[0], false, false);
+            const auto y = __builtin_amdgcn_permlane32_swap(v[1], w[1], false, false);
+            *(lds_vec)at = u32x4{x[0], y[0], x[1], y[1]};
+        };
+        f32x16 acc[2];                       // of the tile on the diagonal and of the one off it
+        u32x2 g[2][4];                       // the same as bf16: four times four consecutive columns of a lane's row
+        // the wave's tiles of S S^T, S [mp x width], in steps of 16 columns: four at a time, the next four on their way
+        auto gram = [&](auto diag, auto side, lds_t s, int width, bool wodd) {
+            constexpr bool D = decltype(diag)::value, O = decltype(side)::value;
+            const int nk = width / 16;       // a multiple of four
+            const int sw = ns_swizzle(r32, wodd) ^ kh, to_b = 64 * (ct - rt) * width;
+            lds_t at[2][4];                  // of an even and an odd four: eight chunks on is a flipped bit or, with odd rows, 128 bytes
 #pragma unroll
-            for (int j = 0; j < TPW; j++)
+            for (int u = 0; u < 4; u++) {
+                at[0][u] = s + (32 * rt + r32) * 2 * width + ((sw ^ (2 * u)) << 4);
+                at[1][u] = s + (32 * rt + r32) * 2 * width + (wodd ? ((sw ^ (2 * u)) << 4) + 128 : (sw ^ (2 * u) ^ 8) << 4);
+            }
+            bf16x8 a[2][4], b[2][4];
+            auto fetch = [&](auto set, int k) {          // k: of the even four
+                constexpr int S = decltype(set)::value;
 #pragma unroll
-                for (int e = 0; e < 16; e++) acc[j][e] = 0.0f;
-            // two k steps at a time (width is a multiple of 64), the operands of the next two on their way
-            const int nk = width / 16;
-            bf16x8 a[2], b[2][TPW];
-            auto fetch = [&](int k) {
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    a[u] = chunk(s, width, 32 * rt + r32, 2 * (k + u) + kh);
-#pragma unroll
-                    for (int j = 0; j < TPW; j++) b[u][j] = chunk(s, width, 32 * (ct + j) + r32, 2 * (k + u) + kh);
+                for (int u = 0; u < 4; u++) {
+                    const lds_t p = at[S][u] + 32 * k;
+                    a[S][u] = *(lds_op)p;
+                    if (O) b[S][u] = *(lds_op)(p + to_b);
                 }
             };
-            fetch(0);
-#pragma unroll 1
-            for (int k = 0; k < nk; k += 2) {
-                bf16x8 a0[2], b0[2][TPW];
+            auto multiply = [&](auto set) {
+                constexpr int S = decltype(set)::value;
 #pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    a0[u] = a[u];
-#pragma unroll
-                    for (int j = 0; j < TPW; j++) b0[u][j] = b[u][j];
+                for (int u = 0; u < 4; u++) {
+                    if (D) acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[S][u], a[S][u], acc[0], 0, 0, 0);
+                    if (O) acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[S][u], a[S][u], acc[1], 0, 0, 0);
                 }
-                fetch(min(k + 2, nk - 2));
+                // the reads between the products
 #pragma unroll
-                for (int u = 0; u < 2; u++)
+                for (int u = 0; u < 4; u++) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, O ? 2 : 1, 0);
+                }
+                if (D && O) __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            using Z0 = std::integral_constant<int, 0>;
+            using Z1 = std::integral_constant<int, 1>;
+            fetch(Z0{}, 0);
+#pragma unroll 1
+            for (int k = 0; k + 8 <= nk; k += 8) {       // (without branches around the reads: they would be waited for at once)
+                fetch(Z1{}, k);
+                multiply(Z0{});
+                fetch(Z0{}, k + 8 < nk ? k + 8 : k);     // (after the last an operand that nobody uses)
+                multiply(Z1{});
+            }
+            if (nk & 4) multiply(Z0{});
+        };
+        // a tile and, off the diagonal, its mirror image
+        auto put = [&](auto side) {
+            constexpr int J = decltype(side)::value;
+            const int col = J ? ct : rt, sw = ns_swizzle(r32, mp & 64) ^ kh;
+            const lds_t at = G + (32 * rt + r32) * GROW;
 #pragma unroll
-                    for (int j = 0; j < TPW; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b0[u][j], a0[u], acc[j], 0, 0, 0);
+            for (int q = 0; q < 4; q += 2) put_row(at + ((sw ^ (4 * col + q)) << 4), g[J][q], g[J][q + 1]);
+            if (J) {
+                const lds_t mirror = G + (32 * col + 4 * kh) * GROW + 2 * (r32 & 7);
+                const int place = (4 * rt + (r32 >> 3)) ^ ns_swizzle(4 * kh, mp & 64);
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        *(lds_b16)(mirror + ((place ^ ns_swizzle((8 * q + e) & 15, mp & 64)) << 4) + (8 * q + e) * GROW) = (bf16_t)(g[J][q][e >> 1] >> (16 * (e & 1)));
             }
         };
-        // (the operands change places, so that a lane holds, of its row of the result, four times four consecutive columns)
-        auto put = [&](auto value) {
+        using T = std::true_type;
+        using F = std::false_type;
+#pragma unroll 1
+        for (int phase = 0; phase < 2; phase++) {
+            const lds_t s = phase ? G : Y;               // G is symmetric
+            const int width = phase ? mp : np;
 #pragma unroll
-            for (int j = 0; j < TPW; j++)
+            for (int j = 0; j < 2; j++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int c = 32 * (ct + j) + 8 * q + 4 * kh;
-                    u32x2* p = reinterpret_cast<u32x2*>(sG + at(mp, 32 * rt + r32, c));
-                    *p = value(j, q, c, p);
+                for (int e = 0; e < 16; e++) acc[j][e] = 0.0f;
+            if (on && off) gram(T{}, T{}, s, width, width & 64);
+            else if (on) gram(T{}, F{}, s, width, width & 64);
+            else if (off) gram(F{}, T{}, s, width, width & 64);
+            if (phase == 0) {
+                const float scale = it == 0 ? inv * inv : 1.0f;
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    if (j ? !off : !on) continue;
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        g[j][q] = u32x2{bf16r2(acc[j][4 * q] * scale, acc[j][4 * q + 1] * scale), bf16r2(acc[j][4 * q + 2] * scale, acc[j][4 * q + 3] * scale)};
                 }
-        };
-        if (active) {
-            gram(sY, np);
-            put([&](int j, int q, int, const u32x2*) {
-                return u32x2{bf16r2(acc[j][4 * q] * g_scale, acc[j][4 * q + 1] * g_scale), bf16r2(acc[j][4 * q + 2] * g_scale, acc[j][4 * q + 3] * g_scale)};
-            });
+            } else {                                     // H = a I + b G + c G G in place of G
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    if (j ? !off : !on) continue;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const u32x2 w = g[j][q];
+                        float v[4];
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const float x = sg_i2f((int32_t)((e & 1) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16)));
+                            v[e] = sg_fma(NS_C, acc[j][4 * q + e], NS_B * x) + (j == 0 && r32 == 8 * q + 4 * kh + e ? NS_A : 0.0f);
+                        }
+                        g[j][q] = u32x2{bf16r2(v[0], v[1]), bf16r2(v[2], v[3])};
+                    }
+                }
+                __syncthreads();
+            }
+            if (on) put(std::integral_constant<int, 0>{});
+            if (off) put(std::integral_constant<int, 1>{});
+            __syncthreads();
         }
-        __syncthreads();
-        if (active) gram(sG, mp);            // G is symmetric
-        __syncthreads();
-        if (active)
-            put([&](int j, int q, int c, const u32x2* p) {       // H = a I + b G + c G G in place of G
-                const u32x2 w = *p;
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float x = sg_i2f((int32_t)((e & 1) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16)));
-                    v[e] = sg_fma(NS_C, acc[j][4 * q + e], NS_B * x) + (32 * rt + r32 == c + e ? NS_A : 0.0f);
-                }
-                return u32x2{bf16r2(v[0], v[1]), bf16r2(v[2], v[3])};
-            });
-        __syncthreads();
-        // transposing read (see k_gemm_nt): lane -> k row 8 (lane / 32) + (lane % 16) / 4, columns 16 ((lane / 16) % 2) + 4 (lane % 4)
-        for (int strip = wave; strip < np / 32; strip += NS_THREADS / 64) {
+        // Y' = H Y by strips of 32 columns
+        for (int strip = wave; strip < np / 32; strip += WAVES) {
             f32x16 y[MT];
 #pragma unroll
             for (int i = 0; i < MT; i++)
 #pragma unroll
                 for (int e = 0; e < 16; e++) y[i][e] = 0.0f;
-            const int col = 32 * strip + 16 * ((lane >> 4) & 1) + 4 * (lane & 3), row0 = 8 * kh + ((lane & 15) >> 2);
-#pragma unroll 2
-            for (int k = 0; k < mp / 16; k++) {
-                const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_p)(sY + at(np, 16 * k + row0, col)));
-                const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_p)(sY + at(np, 16 * k + row0 + 4, col)));
-                const bf16x8 b = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            // transposing read (see k_gemm_nt): lane -> k row 8 (lane / 32) + (lane % 16) / 4, columns 16 ((lane / 16) % 2) + 4 (lane % 4)
+            const int c0 = 4 * strip + 2 * ((ln >> 4) & 1) + ((ln & 3) >> 1), k0 = 8 * kh + ((ln & 15) >> 2);
+            const lds_t t0 = Y + k0 * row + ((c0 ^ ns_swizzle(k0, odd)) << 4) + 8 * (ln & 1);
+            const lds_t t4 = Y + (k0 + 4) * row + ((c0 ^ ns_swizzle(k0 + 4, odd)) << 4) + 8 * (ln & 1);
+            const int hat = (ns_swizzle(r32, mp & 64) ^ kh) << 4;
+            const lds_t hr = G + r32 * GROW;
+            bf16x8 b[2], h[2][MT];
+            auto fetch = [&](int k) {
+                const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_p)(t0 + 16 * k * row));
+                const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_p)(t4 + 16 * k * row));
+                b[k & 1] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-                for (int i = 0; i < MT; i++)
-                    y[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, chunk(sG, mp, 32 * i + r32, 2 * k + kh), y[i], 0, 0, 0);
+                for (int i = 0; i < MT; i++) h[k & 1][i] = *(lds_op)(hr + (hat ^ (32 * k)) + 32 * i * GROW);
+            };
+            fetch(0);
+#pragma unroll
+            for (int k = 0; k < mp / 16; k++) {
+                if (k + 1 < mp / 16) fetch(k + 1);
+#pragma unroll
+                for (int i = 0; i < MT; i++) y[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[k & 1], h[k & 1][i], y[i], 0, 0, 0);
+                if (k + 1 < mp / 16) {
+#pragma unroll
+                    for (int i = 0; i < MT; i++) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
             __builtin_amdgcn_wave_barrier();
+            if (it == 0)
 #pragma unroll
-            for (int i = 0; i < MT; i++)
+                for (int i = 0; i < MT; i++)
 #pragma unroll
-                for (int q = 0; q < 4; q++)
-                    *reinterpret_cast<u32x2*>(sY + at(np, 32 * i + r32, 32 * strip + 8 * q + 4 * kh)) =
-                        u32x2{bf16r2(y[i][4 * q] * y_scale, y[i][4 * q + 1] * y_scale), bf16r2(y[i][4 * q + 2] * y_scale, y[i][4 * q + 3] * y_scale)};
+                    for (int e = 0; e < 16; e++) y[i][e] *= inv;
+            const int sw = ns_swizzle(r32, odd) ^ kh;
+#pragma unroll
+            for (int q = 0; q < 4; q += 2) {
+                lds_t at = Y + r32 * row + ((sw ^ (4 * strip + q)) << 4);
+#pragma unroll
+                for (int i = 0; i < MT; i++, at += 32 * row)
+                    put_row(at, u32x2{bf16r2(y[i][4 * q], y[i][4 * q + 1]), bf16r2(y[i][4 * q + 2], y[i][4 * q + 3])},
+                            u32x2{bf16r2(y[i][4 * q + 4], y[i][4 * q + 5]), bf16r2(y[i][4 * q + 6], y[i][4 * q + 7])});
+            }
         }
         __syncthreads();
     }
-    const int chunks = np / 8;
     u32x4* dst = reinterpret_cast<u32x4*>(steps & 1 ? M.Y2 : M.Y);
-    for (int i = tid; i < mp * chunks; i += NS_THREADS) {
-        const int r = i / chunks, c = i % chunks;
-        *(gvec_w)(dst + i) = *reinterpret_cast<const u32x4*>(sY + (size_t)r * np + (c ^ ns_swizzle(r, np)) * 8);
-    }
+    stream([&](int i, const int (&at)[BATCH], int n) {
+        u32x4 v[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) if (u < n) v[u] = *(lds_vec)(Y + at[u]);
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) if (u < n) *(gvec_w)(dst + i + u * NS_THREADS) = v[u];
+    });
 }
 
 __global__ __launch_bounds__(NS_THREADS) void k_newton_schulz(Batch B, int steps) {
     extern __shared__ __attribute__((aligned(16))) bf16_t smem[];
     const int mi = blockIdx.x;
     const Mat& M = B.mats[mi];
-    // the norm, from the momentum kernel's tiles (a matrix has at most 16 of them)
+    // the norm, from the momentum kernel's tiles (a matrix has at most 16 of them): all read at once, then added in order
+    const int t0 = B.ttile_prefix[mi], nt = B.ttile_prefix[mi + 1] - t0;
+    const double mine = (int)(threadIdx.x & 63) < nt ? B.partials[t0 + (threadIdx.x & 63)] : 0.0;
     double part = 0.0;
-    for (int k = B.ttile_prefix[mi]; k < B.ttile_prefix[mi + 1]; k++) part += B.partials[k];
+    for (int k = 0; k < nt; k++) part += __shfl(mine, k);
     const float inv = 1.0f / ((float)sqrt(part) + 1e-7f);
-    bf16_t* const sG = smem + M.mp * M.np;
-    if (M.mp == 128) newton_schulz<4>(M, inv, steps, smem, sG);
-    else newton_schulz<2>(M, inv, steps, smem, sG);
+    if (M.mp == 128) newton_schulz<4>(M, inv, steps, smem);
+    else newton_schulz<2>(M, inv, steps, smem);
 }
 
 // p = (p - 0.2*lr*X) * (1 - lr*wd).  X lies in the wide orientation; one 64x64 tile of the parameter's own
