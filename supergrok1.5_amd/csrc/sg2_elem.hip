@@ -52,15 +52,22 @@ template <class G>
 constexpr int elem_waves() { return G::DM == 8 ? 4 : 2; }
 // FWD: the net's forward alone (sg2_meta_forward) -- smart gradient and new GRU state of every element go to the packed
 // arrays fwd_smart / fwd_gru, nothing of the optimizer state is read or written.
-template <class G, int EH, bool DBG, bool FWD = false>
+// HEADS: small calls.  The four waves of a workgroup share 64 elements and evaluate one head each, so that an element's
+// serial chain holds one head instead of four; wave 0 goes on with the sum, in the order of the heads as ever.
+template <class G, int EH, bool DBG, bool FWD = false, bool HEADS = false>
 __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(elem_waves<G>(), elem_waves<G>()))) void k_elem(Plan pl, int32_t* __restrict__ expert_counts,
                                                        int32_t* __restrict__ dbg_eidx, float* __restrict__ fwd_smart,
                                                        float* __restrict__ fwd_gru, int split) {
     constexpr int DM = G::DM, GRL = G::GRL, PIN = G::PIN, EXP_STRIDE = exp_stride<EH>();
+    static_assert(!HEADS || ELEM_THREADS == 64 * NH, "a wave per head");
+    constexpr int STEP = HEADS ? 64 : ELEM_THREADS;      // elements a workgroup works on at once
     static_assert(EH % 4 == 0, "expert records are read 16 bytes at a time");
     __shared__ float s_exp[NE * EXP_STRIDE];
     __shared__ float s_b2[NE];
     __shared__ int s_cnt[NE];
+    __shared__ float s_head[HEADS ? 2 : 1][HEADS ? NH : 1][HEADS ? 64 : 1];
+    const int own = HEADS ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, member = threadIdx.x & (STEP - 1);
+    int turn = 0;
 
     warm_scalar_cache<G>(pl);
     {
@@ -104,7 +111,7 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
     const sg::cfloat_p KA0 = sg::as_const(pl.W.w[W_KEYS_A]);
     const sg::cfloat_p KB0 = sg::as_const(pl.W.w[W_KEYS_B]);
 
-    // split: parts that a tile is cut into (1 or ELEM_TILE / ELEM_THREADS, see elem_grid)
+    // split: parts that a tile is cut into (1 or ELEM_TILE / STEP, see elem_grid)
     for (int part = blockIdx.x; part < pl.elem_tiles * split; part += gridDim.x) {
         const int tile = split == 1 ? part : part / split, len = split == 1 ? ELEM_TILE : ELEM_TILE / split;
         const sg::Seg seg = sg::find_seg(sg::as_const(pl.elem_tile_prefix), pl.P, tile);
@@ -120,9 +127,9 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
 
         // every lane runs every iteration (the matrix instructions ignore the execution mask); lanes past the end
         // of the tile recompute its last element and store nothing
-        for (int k0 = 0; k0 < cnt; k0 += ELEM_THREADS) {
-            const bool live = k0 + (int)threadIdx.x < cnt;
-            const int i = start + min(k0 + (int)threadIdx.x, cnt - 1);
+        for (int k0 = 0; k0 < cnt; k0 += STEP) {
+            const bool live = k0 + member < cnt;
+            const int i = start + min(k0 + member, cnt - 1);
             // the weights are re-read (scalar loads, cache hits) for every element instead of being hoisted
             const int zo = sg::opaque_zero();
             const sg::cfloat_p Wz = Wz0 + zo, bz = bz0 + zo, Wr = Wr0 + zo, br = br0 + zo, Wh = Wh0 + zo, bh = bh0 + zo;
@@ -144,7 +151,7 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
             }
             // the optimizer state is requested now, so that its latency passes under the meta-net's arithmetic
             float mu = 0.0f, ea = 0.0f, easq = 0.0f, pv = 0.0f;
-            if (!FWD) {
+            if (!FWD && own == 0) {
                 mu = sg::gptr(T.mu)[i]; ea = sg::gptr(T.ea)[i]; easq = sg::gptr(T.easq)[i];
                 pv = sg::load_elem(T.param, dtype, i);
             }
@@ -189,7 +196,7 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
             sg_tanh_block(GH, pre_c, cand);
 #pragma unroll
             for (int j = 0; j < GH; j++) hnew[j] = sg_fma(zg[j], cand[j], (1.0f - zg[j]) * hold[j]);
-            if (live) {
+            if (!HEADS && live) {
                 if (FWD) ((SG_GLOBAL vf4*)fwd_gru)[(size_t)T.off + i] = vf4{hnew[0], hnew[1], hnew[2], hnew[3]};
                 else ((SG_GLOBAL vf4*)T.gru)[i] = vf4{hnew[0], hnew[1], hnew[2], hnew[3]};
             }
@@ -222,6 +229,7 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
             float total = 0.0f;
 #pragma unroll
             for (int hh = 0; hh < NH; hh++) {
+                if (HEADS && hh != own) continue;
                 const float* query = qall + hh * DM;
                 int best[2];
 #pragma unroll
@@ -259,6 +267,16 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
                     z = sg_max(sg_fma(w1.w, g, b1.w), 0.0f); ho = sg_fma(w2.w, z, ho);
                 }
                 total = total + ho;
+            }
+            if (HEADS) {
+                s_head[turn][own][member] = total;       // 0 + the head
+                __syncthreads();                         // (every wave has read the GRU state)
+                if (own != 0) { turn ^= 1; continue; }
+                total = 0.0f;
+#pragma unroll
+                for (int hh = 0; hh < NH; hh++) total = total + s_head[turn][hh][member];
+                turn ^= 1;
+                if (live) ((SG_GLOBAL vf4*)T.gru)[i] = vf4{hnew[0], hnew[1], hnew[2], hnew[3]};
             }
             const float smart = g + (rescale * total) / (float)NH;
             if (FWD) {
@@ -488,13 +506,23 @@ __global__ __launch_bounds__(ELEM_THREADS) void k_elem_any(Plan pl, int ctx_stri
 
 }  // namespace
 
+// A wave per head while that takes at most one workgroup per compute unit.  Beyond, the element's chain is shorter still, but
+// every 64 elements pay for an LDS fill of 28 KB that otherwise serves 256: steps over 1000 elements in 3 tensors 65.9 -> 64.2 us,
+// 5000 in 4 84.0 -> 82.6, 8 small tensors 46.4 -> 43.9, but 15 000 in 6 (about 300 parts) 101.5 -> 102.5, 0.42 M 212 -> 274.
+constexpr int HEADS_PARTS = 256;
+inline bool by_heads(const Plan& pl) { return pl.elem_kind != ELEM_ANY && pl.elem_tiles * (ELEM_TILE / 64) <= HEADS_PARTS; }
+
 // Workgroups of the per-element kernel, and the parts its tiles are cut into.  Large calls: about five workgroups per
 // resident slot (768 at three per CU): measured 1.38 / 1.35 / 1.33 / 1.33 / 1.37 ms with 768 / 2048 / 4096 / 8192 / 16384
 // workgroups on 24 424 tiles (fewer leave the chip unevenly loaded at the end, more pay the LDS fill too often).  Calls of
 // at most 1024 tiles would leave most of the chip idle while some workgroups run four rounds of 256 elements: they take
 // rounds as units, spread evenly over at most 1024 resident workgroups.
-int elem_grid(const Plan& pl, int* split) {
+int elem_grid(const Plan& pl, bool heads, int* split) {
     *split = 1;
+    if (heads && by_heads(pl)) {
+        *split = ELEM_TILE / 64;
+        return pl.elem_tiles * *split;
+    }
     if (pl.elem_tiles > 1024 || pl.elem_kind == ELEM_ANY) return pl.elem_tiles < 4096 ? pl.elem_tiles : 4096;
     *split = ELEM_TILE / ELEM_THREADS;
     const int parts = pl.elem_tiles * *split, rounds = (parts + 1023) / 1024;
@@ -504,7 +532,7 @@ int elem_grid(const Plan& pl, int* split) {
 int launch_elem_forward(const Plan& pl, int32_t* expert_counts, float* smart_out, float* gru_out, hipStream_t st) {
     if (pl.total == 0) return 0;
     int split;
-    const int grid = elem_grid(pl, &split);
+    const int grid = elem_grid(pl, false, &split);
     int32_t* const no_dbg = nullptr;
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(ELEM_THREADS), 0, st, pl, expert_counts, no_dbg, smart_out, gru_out, split); };
     if (pl.elem_kind == ELEM_ANY)
@@ -519,7 +547,7 @@ int launch_elem_forward(const Plan& pl, int32_t* expert_counts, float* smart_out
 int launch_elem(const Plan& pl, int32_t* expert_counts, int32_t* dbg_expert_idx, hipStream_t st) {
     if (pl.total == 0) return 0;
     int split;
-    const int grid = elem_grid(pl, &split);
+    const int grid = elem_grid(pl, dbg_expert_idx == nullptr, &split);
     float* const none = nullptr;
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(ELEM_THREADS), 0, st, pl, expert_counts, dbg_expert_idx, none, none, split); };
     if (pl.elem_kind == ELEM_ANY) {
@@ -528,12 +556,16 @@ int launch_elem(const Plan& pl, int32_t* expert_counts, int32_t* dbg_expert_idx,
         else hipLaunchKernelGGL(k_elem_any<false>, dim3(grid), dim3(ELEM_THREADS), 0, st, pl, stride, expert_counts, dbg_expert_idx, none, none);
     } else if (pl.geo == GEO_LARGE) {
         if (dbg_expert_idx) go(k_elem<GeoLarge, 16, true>);
+        else if (by_heads(pl)) go(k_elem<GeoLarge, 16, false, false, true>);
         else go(k_elem<GeoLarge, 16, false>);
     } else if (pl.elem_kind == ELEM_FAST4) {
         if (dbg_expert_idx) go(k_elem<GeoDefault, 4, true>);
+        else if (by_heads(pl)) go(k_elem<GeoDefault, 4, false, false, true>);
         else go(k_elem<GeoDefault, 4, false>);
     } else if (dbg_expert_idx) {
         go(k_elem<GeoDefault, 16, true>);
+    } else if (by_heads(pl)) {
+        go(k_elem<GeoDefault, 16, false, false, true>);
     } else {
         go(k_elem<GeoDefault, 16, false>);
     }
