@@ -29,8 +29,12 @@
 //     threshold of an expert, the lane that holds that expert's sums adds them to the interval's bin (a row of this
 //     workgroup in memory) and starts again.  In element order x stays next to zero.  The exceptions - elements in
 //     another interval of one of their experts - look the interval up in the tables and move their (w, w g) to its bin
-//     with atomics, one expert per lane at a time (four at a time cost more registers than they saved time).  (With all of a trained net's exceptions taken by LDS atomics, in
-//     element order, they were half of the pass.)
+//     with atomics.  They are the largest of a tensor and come together, sixteen a lane and head, so a head's exceptions
+//     are dealt to all lanes of the wave.  (A lane going through its own one by one waited twice for
+//     memory each time: in a call of 0.42 M elements the wave with the most, 340 a head, took 330 us, 150 being the
+//     median, and the launch 370; now 310.  Two jobs a lane
+//     at a time took 280 there, but the registers they need are missed by every tile: 1.3 % of a pass over 25 M.  With all of a trained net's exceptions taken by LDS atomics, in element
+//     order, they were half of the pass.)
 //     (An element exactly on a threshold counts the unit as inactive on both sides; forward value and gradient use
 //     the same interval, so they stay consistent.)
 //   * GRU and query matrices: d (x) x, 16 x 16 x 4 steps over 27 columns of x;
@@ -44,7 +48,7 @@
 // Bound by the vector ALU (about 5000 instructions per wave and tile, two thirds of them the fixed multiply-adds of the
 // net and its derivative).  Measured on 25 M elements with module-initialised experts after some meta steps: 8.4 ms, 47 ms
 // as one lane per element of a 256-lane workgroup that summed the outer products lane by lane from LDS; on 0.42 M elements
-// 0.33 ms instead of 1.1.  (The net's products as 4 x 4 x 1 matrix instructions with the weights in LDS or in memory took as
+// 0.31 ms instead of 1.1.  (The net's products as 4 x 4 x 1 matrix instructions with the weights in LDS or in memory took as
 // long, with the bins in LDS longer on large calls: registers are what there is least of.)
 #include "sg2_internal.hpp"
 
@@ -64,9 +68,10 @@ constexpr int XW = 27;
 constexpr int CW = 25;                  // routing weights of a head: first sub-key[12], second sub-key[12], g
 constexpr int C_ROWS = 80;              // 64 elements, those of either sign padded to whole pairs of steps
 constexpr int KW = 33;                  // d score of a head: first[12], second[12], query[8]
+constexpr int EW = 13;                  // of a head's picks whose interval is another one: weights [4][4], indexes (two words), g, d loss / d head; then up to 1024 jobs
 constexpr int DW = 17;                  // d query of two heads [16], or d pre_z[4], d pre_r[4], d pre_h[4] of the GRU
 constexpr int R_FLOATS = 64 * KW;
-static_assert(C_ROWS * CW <= R_FLOATS && XW % 2 == 1 && CW % 2 == 1 && KW % 2 == 1 && DW % 2 == 1, "odd strides: lane-consecutive rows hit all banks");
+static_assert(C_ROWS * CW <= R_FLOATS && 64 * EW + 64 * TOPK * TOPK <= R_FLOATS && EW % 2 == 1 && XW % 2 == 1 && CW % 2 == 1 && KW % 2 == 1 && DW % 2 == 1, "odd strides: lane-consecutive rows hit all banks");
 constexpr int WAVE_FLOATS = 64 * XW + R_FLOATS + 2 * NE * 4;       // ... and the lines (A, B, low border, high border) of every expert at +x and -x
 constexpr int KEY_FLOATS = 2 * NH * PK * (DM / 2);
 constexpr int BE_LDS_BYTES = 4 * (KEY_FLOATS + BE_WAVES * WAVE_FLOATS);
@@ -522,30 +527,62 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                 }
             }
             if (!valid) other = 0u;
-            while (__builtin_amdgcn_ballot_w64(other != 0u) != 0) {
-                if (other != 0u) {
-                    const int pick = __builtin_ctz(other), ia = pick / TOPK, ib = pick % TOPK;
-                    other &= other - 1u;
-                    // (selects keep idx and wgt in registers: a dynamic index would send them to scratch)
-                    const int ea = ia == 0 ? idx[0][0] : ia == 1 ? idx[0][1] : ia == 2 ? idx[0][2] : idx[0][3];
-                    const int eb = ib == 0 ? idx[1][0] : ib == 1 ? idx[1][1] : ib == 2 ? idx[1][2] : idx[1][3];
-                    const float wa = ia == 0 ? wgt[0][0] : ia == 1 ? wgt[0][1] : ia == 2 ? wgt[0][2] : wgt[0][3];
-                    const float wb = ib == 0 ? wgt[1][0] : ib == 1 ? wgt[1][1] : ib == 2 ? wgt[1][2] : wgt[1][3];
-                    const int e = ea * PK + eb;
+            if (__builtin_amdgcn_ballot_w64(other != 0u) != 0) {
+                // some lanes have all sixteen of them (the largest elements of a tensor), others none: they are dealt to all lanes
+                float* const mine = s_r + lane * EW;
+                int ia4 = 0, ib4 = 0;
+#pragma unroll
+                for (int k = 0; k < TOPK; k++) {
+                    ia4 |= idx[0][k] << (8 * k); ib4 |= idx[1][k] << (8 * k);
+                    mine[k] = wgt[0][k]; mine[TOPK + k] = wgt[1][k];
+                }
+                mine[2 * TOPK] = __int_as_float(ia4); mine[2 * TOPK + 1] = __int_as_float(ib4);
+                mine[2 * TOPK + 2] = g; mine[2 * TOPK + 3] = kk;
+                float* const jobs = s_r + 64 * EW;           // (lane, pick) of each, then its output in the same place
+                const int picks = __popc(other);
+                int rank = 0, all = 0;                       // picks of the lanes below, of all
+#pragma unroll
+                for (int b = 0; b < 5; b++) {
+                    const unsigned long long has = __builtin_amdgcn_ballot_w64((picks >> b) & 1);
+                    rank += (int)__builtin_amdgcn_mbcnt_hi((unsigned)(has >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)has, 0u)) << b;
+                    all += __popcll(has) << b;
+                }
+#pragma unroll
+                for (int ia = 0; ia < TOPK; ia++)
+                    if (__builtin_amdgcn_ballot_w64((other >> (TOPK * ia)) & 15u) != 0)
+#pragma unroll
+                        for (int p = TOPK * ia; p < TOPK * ia + TOPK; p++)
+                            if ((other >> p) & 1u) jobs[rank + __popc(other & ((1u << p) - 1u))] = __int_as_float(16 * lane + p);
+                wave_sync();
+#pragma unroll 1
+                for (int n = lane; n < all; n += 64) {
+                    const int job = __float_as_int(jobs[n]), ia = (job >> 2) & 3, ib = job & 3;
+                    const float* row = s_r + (job >> 4) * EW;
+                    const int e = ((__float_as_int(row[2 * TOPK]) >> (8 * ia)) & 255) * PK + ((__float_as_int(row[2 * TOPK + 1]) >> (8 * ib)) & 255);
+                    const float wa = row[ia], wb = row[TOPK + ib], eg = row[2 * TOPK + 2];
                     const Thresholds th(ths, e);
-                    const int k = th.below(g), kr = th.below(reference(x_held, side != 0));
+                    const int k = th.below(eg), kr = th.below(reference(x_held, !(eg > 0.0f)));
                     const float2 ab = reinterpret_cast<const float2*>(lines)[e * NBIN + k];
-                    const float out = sg_fma(ab.x, g, ab.y);
-                    const float pa = wb * out, pb = wa * out;
-                    ra[0] += ia == 0 ? pa : 0.0f; ra[1] += ia == 1 ? pa : 0.0f; ra[2] += ia == 2 ? pa : 0.0f; ra[3] += ia == 3 ? pa : 0.0f;
-                    rb[0] += ib == 0 ? pb : 0.0f; rb[1] += ib == 1 ? pb : 0.0f; rb[2] += ib == 2 ? pb : 0.0f; rb[3] += ib == 3 ? pb : 0.0f;
-                    const float w = (kk * wa) * wb;
+                    jobs[n] = sg_fma(ab.x, eg, ab.y);
+                    const float w = (row[2 * TOPK + 3] * wa) * wb;
                     float* b = bins + 2 * e * NBIN;
                     bin_add(b + 2 * k, w);
-                    bin_add(b + 2 * k + 1, w * g);
+                    bin_add(b + 2 * k + 1, w * eg);
                     bin_add(b + 2 * kr, -w);
-                    bin_add(b + 2 * kr + 1, -(w * g));
+                    bin_add(b + 2 * kr + 1, -(w * eg));
                 }
+                wave_sync();
+#pragma unroll
+                for (int ia = 0; ia < TOPK; ia++)
+                    if (__builtin_amdgcn_ballot_w64((other >> (TOPK * ia)) & 15u) != 0)
+#pragma unroll
+                        for (int ib = 0; ib < TOPK; ib++) {
+                            const int p = TOPK * ia + ib;
+                            const float out = (other >> p) & 1u ? jobs[rank + __popc(other & ((1u << p) - 1u))] : 0.0f;
+                            ra[ia] += wgt[1][ib] * out;
+                            rb[ib] += wgt[0][ia] * out;
+                        }
+                wave_sync();
             }
             float head_out = 0.0f;
 #pragma unroll
