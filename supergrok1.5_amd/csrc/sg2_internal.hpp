@@ -58,8 +58,8 @@ constexpr int PIN = GeoDefault::PIN;
 
 constexpr int ELEM_TILE = 1024;        // elements per tile of the elementwise kernels
 constexpr int SORT_TILE = 8192;        // keys per radix-sort tile (16 per thread) ...
-constexpr int SORT_TILE_SMALL = 2048;  // ... and where every tensor is small (4 per thread): see sort_tile_for
-constexpr int SELF_SCAN_TILES = 32;    // tiles of a segment up to which a scatter block adds up the digit counts of its segment itself
+constexpr int SORT_TILE_SMALL = 2048;  // ... and in small calls (4 per thread): see sort_tile_for
+constexpr int SELF_SCAN_TILES = 32;    // large tiles of a segment up to which a scatter block adds up the digit counts of its segment itself (small ones: always)
 constexpr int SCAN_TT = 64;            // timesteps projected per LDS tile
 constexpr int SCAN_THREADS = GeoDefault::THREADS;
 constexpr int SCAN_BLOCK_ITEMS = 2048; // entries per block of the spine scan

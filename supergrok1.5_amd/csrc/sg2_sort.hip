@@ -6,6 +6,7 @@
 // cub::DeviceSegmentedRadixSort::SortPairs call (:1860-1879).  Non-negative
 // floats order like their bit patterns, so the keys are sorted as uint32.
 //
+// Small calls sort runs of 4096 keys in LDS and merge a tensor's runs (k_sort_runs, k_merge_runs); the others:
 // Four passes of 8 bits (two where all gradients are 16-bit, see key_bits) over tiles of 8192 keys (512 lanes x 16), or of
 // 2048 where the call is small.  Per pass:
 //   hist     per-tile digit counts -> spine[segment][digit][tile]  (first pass: counted while the keys are made)
@@ -14,13 +15,13 @@
 //            (seg, d, tile) is exactly: keys in earlier segments + keys of this
 //            segment with a smaller digit + keys with digit d in earlier tiles
 //            = destination of the first such key of this tile.
-//            Calls whose tensors have few tiles each have no scan: a scatter
-//            workgroup adds up the counts of its own segment itself.
+//            Calls whose tensors have few tiles each, and small calls, have no scan: a
+//            scatter workgroup adds up the counts of its own segment itself.
 //   scatter  stable rank inside the tile (each wave owns a contiguous quarter
 //            of the tile; match-any ballots give the rank among equal digits)
 //            and write to destination; the last pass of a small call also takes
 //            the sharpness along into sorted order (large ones: a kernel of its own).
-// Calls whose tensors all fit one tile are sorted by one launch, a workgroup per
+// Calls whose tensors all fit one tile (see sort_tile_for) are sorted by one launch, a workgroup per
 // tensor that keeps its keys in LDS for all passes.
 #include <type_traits>
 
@@ -351,7 +352,7 @@ __device__ __forceinline__ void digit_starts(RankLds& L) {
 // FIRST: the pass over digit 0 takes its keys and payloads from the tensor's gradients (element order) instead of
 // the key / payload arrays, which nothing has written yet.  LAST (small calls): the sharpness of an element goes with it.  SELF: the
 // spine holds plain counts: digit d of the tile starts after the segment's keys of smaller digits and those of digit d in
-// earlier tiles, added up here (at most SELF_SCAN_TILES counts per digit, two lanes a digit); a scan kernel between the
+// earlier tiles, added up here (a count per digit and tile of the segment, at most 256 of them, two lanes a digit); a scan kernel between the
 // counting and the scatter of each pass costs a small call 5 us and another gap.
 template <int TILE, bool FIRST, bool LAST, bool SELF, bool HALF>
 __global__ __launch_bounds__(SORT_THREADS) void k_scatter(Plan pl, int src, int shift) {
@@ -471,6 +472,36 @@ __global__ __launch_bounds__(SORT_THREADS) void k_scatter(Plan pl, int src, int 
     else body(std::false_type{});
 }
 
+// All passes over n keys in LDS, by the whole workgroup after a barrier; ends with one.  ROUNDS rounds of 64 keys per wave cover them.
+template <int ROUNDS, bool HALF>
+__device__ __forceinline__ void sort_in_lds(RankLds& L, uint32_t* skey, int32_t* sval, int n, KeyBits bits) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t key[ROUNDS], rank[ROUNDS];
+    int32_t val[ROUNDS];
+    auto at = [&](int r) { return (w * ROUNDS + r) * 64 + lane; };
+    for (int shift = 0; shift < (HALF ? 16 : 32); shift += 8) {
+        for (int k = threadIdx.x; k < WAVES * 256; k += SORT_THREADS) (&L.cnt[0][0])[k] = 0;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) {
+            key[r] = at(r) < n ? skey[at(r)] : 0u;
+            val[r] = at(r) < n ? sval[at(r)] : 0;
+        }
+        __syncthreads();
+        rank_keys<HALF>(L, key, rank, bits, shift, [&](int r) { return at(r) < n; });
+        __syncthreads();
+        digit_starts(L);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++)
+            if (at(r) < n) {
+                const uint32_t lp = L.cnt[w][(order_of<HALF>(key[r], bits) >> shift) & 255u] + rank[r];
+                skey[lp] = key[r];
+                sval[lp] = val[r];
+            }
+        __syncthreads();
+    }
+}
+
 // ---- every tensor fits one tile: keys, four passes and the sharpness in one launch ----------------------------------
 // Workgroup 0 derives the scan's coefficients; workgroup 1 + i sorts tensor i.  The keys stay in LDS between the passes:
 // the launches of the general sort (12 for 8 tensors of at most 255 elements, 48 us) carry next to no work there.
@@ -484,7 +515,7 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort_tile(Plan pl) {
     __shared__ RankLds L;
     __shared__ uint32_t skey[SORT_TILE];
     __shared__ int32_t sval[SORT_TILE];
-    const int seg = (int)blockIdx.x - 1, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int seg = (int)blockIdx.x - 1;
     const TensorDev& T = pl.tensors[seg];
     const int n = T.numel, dtype = T.dtype;
     if (n == 0) return;
@@ -498,41 +529,13 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort_tile(Plan pl) {
     }
     note_sharpness(pl, seg, nz);
     const bool gather = __syncthreads_or(nz);
-    // rounds per wave, so that the waves' parts cover the tensor: 1, 2, 4, 8 or 16
-    auto passes = [&](auto rounds_c, auto half_c) {
-        constexpr int ROUNDS = decltype(rounds_c)::value;
-        constexpr bool HALF = decltype(half_c)::value;
-        const KeyBits bits = key_bits<HALF>(dtype);
-        uint32_t key[ROUNDS], rank[ROUNDS];
-        int32_t val[ROUNDS];
-        auto at = [&](int r) { return (w * ROUNDS + r) * 64 + lane; };
-        for (int shift = 0; shift < (HALF ? 16 : 32); shift += 8) {
-            for (int k = threadIdx.x; k < WAVES * 256; k += SORT_THREADS) (&L.cnt[0][0])[k] = 0;
-#pragma unroll
-            for (int r = 0; r < ROUNDS; r++) {
-                key[r] = at(r) < n ? skey[at(r)] : 0u;
-                val[r] = at(r) < n ? sval[at(r)] : 0;
-            }
-            __syncthreads();
-            rank_keys<HALF>(L, key, rank, bits, shift, [&](int r) { return at(r) < n; });
-            __syncthreads();
-            digit_starts(L);
-            __syncthreads();
-#pragma unroll
-            for (int r = 0; r < ROUNDS; r++)
-                if (at(r) < n) {
-                    const uint32_t lp = L.cnt[w][(order_of<HALF>(key[r], bits) >> shift) & 255u] + rank[r];
-                    skey[lp] = key[r];
-                    sval[lp] = val[r];
-                }
-            __syncthreads();
-        }
-    };
     const int rounds = (n + SORT_THREADS - 1) / SORT_THREADS;
     auto with = [&](auto half_c) {
-        if (rounds <= 1) passes(std::integral_constant<int, 1>{}, half_c);
-        else if (rounds <= 4) passes(std::integral_constant<int, 4>{}, half_c);
-        else passes(std::integral_constant<int, ITEMS>{}, half_c);
+        constexpr bool HALF = decltype(half_c)::value;
+        const KeyBits bits = key_bits<HALF>(dtype);
+        if (rounds <= 1) sort_in_lds<1, HALF>(L, skey, sval, n, bits);
+        else if (rounds <= 4) sort_in_lds<4, HALF>(L, skey, sval, n, bits);
+        else sort_in_lds<ITEMS, HALF>(L, skey, sval, n, bits);
     };
     if (dtype == SG_F32) with(std::false_type{});
     else with(std::true_type{});
@@ -542,6 +545,139 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort_tile(Plan pl) {
         pl.vals[0][T.off + i] = v;
         if (gather) pl.ssorted[T.off + i] = sharp_of(T, v & 0x7fffffff);
     }
+}
+
+// ---- small calls: runs of RUN keys sorted by themselves, then all runs of a tensor merged at once --------------------------
+// Two launches instead of the eight of the radix passes, which are bound by their latency and the gaps between them in
+// such calls (14 tensors of 0.42 M elements: 57 us and as much again for 15 000).  A key's place in the tensor is its
+// place in its own run plus, for every other run, the number of that run's keys before it: smaller ones, and equal ones
+// where the run lies earlier (stable, as the passes are).  The runs pass through LDS two at a time while the next two are on
+// their way, and a workgroup looks its 2048 keys up by halving steps.
+// Bound by the vector ALU (three instructions a step, 13 steps a key and run) where a tensor has many runs: runs of 4096
+// instead of 2048 halve that and add 6 us of sorting.  0.42 M elements: 21 + 26 us; steps 215 -> 203 us, 15 000 elements in 6
+// tensors 102 -> 81, 30 000 in 5 105 -> 88, one tensor of 60 000 113 -> 103.
+constexpr int RUN_TILES = 2, RUN = RUN_TILES * SORT_TILE_SMALL;
+template <class G, bool HALF>
+__global__ __launch_bounds__(SORT_THREADS) void k_sort_runs(Plan pl) {
+    if (blockIdx.x == 0) {
+        compose_block<G>(pl, SORT_THREADS);
+        return;
+    }
+    constexpr int ITEMS = RUN / SORT_THREADS;
+    __shared__ RankLds L;
+    __shared__ uint32_t skey[RUN];
+    __shared__ int32_t sval[RUN];
+    const TileRef tr = tile_ref<true>(pl, (int)blockIdx.x - 1);
+    if (tr.tile % RUN_TILES != 0) return;
+    const TensorDev& T = pl.tensors[tr.seg];
+    const int start = tr.base - T.off, dtype = T.dtype, cnt = min(RUN, T.numel - start);
+    float g[ITEMS];
+    bool nz = false;
+    // everything is requested before the clip factor is waited for
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const int k = r * SORT_THREADS + (int)threadIdx.x;
+        g[r] = k < cnt ? sg::load_elem(T.grad, dtype, start + k) : 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const int k = r * SORT_THREADS + (int)threadIdx.x;
+        if (k < cnt) nz = nz || sharp_rounded(T, start + k) != 0.0f;
+    }
+    const float gs = clip_factor(pl, tr.seg, tr.tile == 0);
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const int k = r * SORT_THREADS + (int)threadIdx.x;
+        const float v = clipped(g[r], gs, dtype);
+        if (k < cnt) {
+            skey[k] = key_of(v);
+            sval[k] = payload_of(v, start + k);
+        }
+    }
+    note_sharpness(pl, tr.seg, nz);              // (its barrier covers the keys)
+    sort_in_lds<ITEMS, HALF>(L, skey, sval, cnt, key_bits<HALF>(dtype));
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const int k = r * SORT_THREADS + (int)threadIdx.x;
+        if (k < cnt) {
+            pl.keys[1][tr.base + k] = skey[k];
+            pl.vals[1][tr.base + k] = sval[k];
+        }
+    }
+}
+
+template <bool HALF>
+__global__ __launch_bounds__(SORT_THREADS) void k_merge_runs(Plan pl) {
+    constexpr int ITEMS = SORT_TILE_SMALL / SORT_THREADS, PARTS = RUN / SORT_THREADS, GROUP = 2;
+    static_assert((RUN & (RUN - 1)) == 0, "binary search by halving steps");
+    __shared__ uint32_t run[2][GROUP][RUN];
+    // a tensor's tiles next to each other on an XCD: their keys fall between each other, into the same lines of its L2
+    const int nb = gridDim.x, tile = nb % 8 == 0 ? ((int)blockIdx.x % 8) * (nb / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
+    const TileRef tr = tile_ref<true>(pl, tile);
+    const TensorDev& T = pl.tensors[tr.seg];
+    const KeyBits bits = key_bits<HALF>(T.dtype);
+    uint32_t key[ITEMS], at[ITEMS], place[ITEMS], next[GROUP][PARTS];
+    int32_t val[ITEMS];
+    const int mine = tr.tile / RUN_TILES, others = (tr.tiles - 1) / RUN_TILES;
+    auto other = [&](int j) { return j < mine ? j : j + 1; };      // the j-th of the other runs
+    auto request = [&](int j0) {
+#pragma unroll
+        for (int u = 0; u < GROUP; u++) {
+            const int first = other(j0 + u) * RUN, n = j0 + u < others ? T.numel - first : 0;
+#pragma unroll
+            for (int r = 0; r < PARTS; r++) {
+                const int k = r * SORT_THREADS + (int)threadIdx.x;
+                next[u][r] = k < n ? order_of<HALF>(pl.keys[1][tr.seg_off + first + k], bits) : 0xffffffffu;       // (beyond every key)
+            }
+        }
+    };
+    request(0);
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const int k = r * SORT_THREADS + (int)threadIdx.x;
+        key[r] = k < tr.cnt ? pl.keys[1][tr.base + k] : 0u;
+        val[r] = k < tr.cnt ? pl.vals[1][tr.base + k] : 0;
+        at[r] = order_of<HALF>(key[r], bits);
+        place[r] = (uint32_t)(tr.seg_off + (tr.tile % RUN_TILES) * SORT_TILE_SMALL + k);      // in its own run
+    }
+    int turn = 0;
+    for (int j = 0; j < others; j += GROUP, turn ^= 1) {
+#pragma unroll
+        for (int u = 0; u < GROUP; u++)
+#pragma unroll
+            for (int r = 0; r < PARTS; r++) run[turn][u][r * SORT_THREADS + (int)threadIdx.x] = next[u][r];
+        __syncthreads();                             // (a wave is at most one group ahead: the other buffer)
+        if (j + GROUP < others) request(j + GROUP);
+        // (pointers instead of indexes: the halving steps fit the reads' offsets)
+        typedef const __attribute__((address_space(3))) uint32_t* lds_keys;
+        lds_keys from[GROUP][ITEMS];
+        uint32_t limit[GROUP][ITEMS];
+#pragma unroll
+        for (int u = 0; u < GROUP; u++)
+#pragma unroll
+            for (int r = 0; r < ITEMS; r++) {
+                from[u][r] = (lds_keys)run[turn][u];
+                limit[u][r] = at[r] + (j + u < mine ? 1u : 0u);
+            }
+#pragma unroll
+        for (int step = RUN / 2; step > 0; step >>= 1)
+#pragma unroll
+            for (int u = 0; u < GROUP; u++)
+#pragma unroll
+                for (int r = 0; r < ITEMS; r++) from[u][r] += from[u][r][step - 1] < limit[u][r] ? step : 0;
+#pragma unroll
+        for (int u = 0; u < GROUP; u++)
+#pragma unroll
+            for (int r = 0; r < ITEMS; r++) place[r] += (uint32_t)(from[u][r] - (lds_keys)run[turn][u]) + (*from[u][r] < limit[u][r] ? 1u : 0u);
+    }
+    const bool gather = pl.sharp_nonzero[tr.seg] != 0;       // all-zero sharpness: no sorted copy is made, every reader tests the same flag
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++)
+        if (r * SORT_THREADS + (int)threadIdx.x < tr.cnt) {
+            pl.keys[0][place[r]] = key[r];
+            pl.vals[0][place[r]] = val[r];
+            if (gather) pl.ssorted[place[r]] = sharp_of(T, val[r] & 0x7fffffff);
+        }
 }
 
 // Sharpness into sorted order for large calls (one random read per element, once, instead of one per scan pass and
@@ -604,9 +740,24 @@ int launch_passes(const Plan& pl, hipStream_t st) {
     return 0;
 }
 
+// Tiles of the largest tensor up to which runs are merged.  The merge's work grows with the square of a tensor's length and the
+// passes' with the length; 16-bit gradients have two passes only.  Step times with passes / runs over small tiles: four fp32
+// tensors of 20 000 133 / 116 us, one of 60 000 112 / 103, of 80 000 132 / 132, of 130 000 148 / 155, sixteen of 60 000
+// 337 / 325, thirty 514 / 517 (hence the product); bfloat16, one of 8000 85 / 76, four of 20 000 111 / 114, one of 60 000 92 / 116.
+constexpr int MERGE_TILES = 40, MERGE_WORK = 20000, HALF_MERGE_TILES = 4;
+inline bool merges(const Plan& pl, bool half) {
+    return pl.sort_widest <= (half ? HALF_MERGE_TILES : MERGE_TILES) && (int64_t)pl.sort_tiles * pl.sort_widest <= MERGE_WORK;
+}
 template <class G, bool HALF>
 int launch_sort_geo(const Plan& pl, hipStream_t st) {
-    if (pl.sort_tile == SORT_TILE_SMALL) return launch_passes<G, SORT_TILE_SMALL, true, HALF>(pl, st);
+    if (pl.sort_tile == SORT_TILE_SMALL) {
+        if (!merges(pl, HALF)) return launch_passes<G, SORT_TILE_SMALL, true, HALF>(pl, st);
+        hipLaunchKernelGGL((k_sort_runs<G, HALF>), dim3(1 + pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl);
+        SG_LAUNCH_CHECK("k_sort_runs");
+        hipLaunchKernelGGL(k_merge_runs<HALF>, dim3(pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl);
+        SG_LAUNCH_CHECK("k_merge_runs");
+        return 0;
+    }
     if (pl.sort_widest <= 1) {
         hipLaunchKernelGGL(k_sort_tile<G>, dim3(1 + pl.P), dim3(SORT_THREADS), 0, st, pl);
         SG_LAUNCH_CHECK("k_sort_tile");

@@ -163,16 +163,17 @@ __global__ __launch_bounds__(256) void k_pad_weights(PadArgs a) {
     }
 }
 
-// Keys per sort tile.  A scatter of 8192 keys is 16 rounds in series per wave whatever the call's size; where every tensor
-// has at most 65 536 elements, and so no more than SELF_SCAN_TILES tiles of 2048, and the call has fewer elements than
-// make a large tile for each of the 256 CUs, it takes the small ones (the 14-tensor set: 212 workgroups instead of 57, 6 us per
-// pass instead of 11).  Beyond that the small tiles no longer fill idle CUs, scatter shorter runs and read more counts: step
-// times with 2048 / 8192 keys are 226 / 246 us for 14 tensors of 30 000, 359 / 369 for 16 of 60 000, 650 / 663 for 100 of
-// 20 000, but 760 / 751 for 256 of 9000, 833 / 812 for 48 of 60 000 and 5.86 / 5.55 ms for 400 of 60 000.
-// Tensors of one large tile each are sorted in LDS by one launch.
+// Keys per sort tile.  A scatter of 8192 keys is 16 rounds in series per wave whatever the call's size.  Calls of fewer
+// elements than make a large tile for every fourth CU take the small ones, and so do those whose tensors have at most
+// 65 536 elements each up to a large tile for every CU; with the small ones come the merged runs (see launch_sort_geo).
+// Step times with large / small tiles: one tensor of 200 000 180 / 164 us, of 500 000 261 / 251, two of 200 000 237 / 223,
+// one of 200 000 bfloat16 160 / 136; 16 of 60 000 336 / 320 us and 33 of 60 000 567 / 563, but 12 of 100 000 402 / 418, 256
+// of 9000 751 / 760 and 400 of 60 000 5.55 / 5.86 ms: then the small tiles fill no idle CUs and scatter shorter runs.
+// Tensors of at most one small tile each are sorted in LDS by one launch (of at most a large one, in calls that take
+// those: beside small tiles, 8000 elements in one workgroup are 93 us of a step and 79 in runs).
 inline int sort_tile_for(int64_t widest, int64_t total) {
-    return widest > SORT_TILE && widest <= (int64_t)SELF_SCAN_TILES * SORT_TILE_SMALL && total < (int64_t)256 * SORT_TILE ? SORT_TILE_SMALL
-                                                                                                                       : SORT_TILE;
+    const bool small = total < (int64_t)64 * SORT_TILE || (widest <= 32 * SORT_TILE_SMALL && total < (int64_t)256 * SORT_TILE);
+    return small && widest > SORT_TILE_SMALL ? SORT_TILE_SMALL : SORT_TILE;
 }
 // Elements per workgroup of the norm reduction: as the other steps' tiles (many short ones for small calls).
 inline int norm_tile_for(int64_t total) { return total >= (8 << 20) ? 4096 : (total >= (1 << 20) ? 1024 : 256); }
