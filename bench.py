@@ -22,7 +22,7 @@ BYTES_PER_ELEMENT = 72          # algorithmic HBM bytes per element per step (fp
 HBM_PEAK_GBS = 8000.0
 SIMDS = 1024
 REPLAY_WAVES_PER_SIMD = 2        # k_replay: eight one-wave workgroups per compute unit (19.8 KB of LDS each)
-STAGE_KERNEL_PREFIX = {"scan_output": "k_replay<", "scan_summary": "k_scan<default, false>", "elementwise": "k_elem<"}
+STAGE_KERNEL_PREFIX = {"scan_output": "k_replay<", "scan_summary": "k_summary<default", "elementwise": "k_elem<"}
 
 
 def profile_figures():
@@ -675,8 +675,8 @@ def main():
     ms_per_step = 1e3 * elapsed / args.steps
     value = total * args.steps / elapsed
     dom = max(stage_avg, key=stage_avg.get)
-    kernel_of = {"sort": "k_keys + 4 x (k_hist, k_spine_*, k_scatter)", "scan_summary": "k_scan<false>",
-                 "chunk_prefix": "k_chunk_prefix", "scan_output": "k_replay", "elementwise": "k_elem<false>"}
+    kernel_of = {"sort": "k_keys + 4 x (k_hist, k_spine_*, k_scatter)", "scan_summary": "k_summary",
+                 "chunk_prefix": "k_chunk_prefix", "scan_output": "k_replay", "elementwise": "k_elem"}
     achieved = BYTES_PER_ELEMENT * total / (stage_avg[dom] * 1e-3) / 1e9
     default_workload = (args.workload, args.weights, args.geometry, args.sharpness) == ("scale50", "bench", "default", False)
     prof = profile_figures() if default_workload else {"traffic": {}, "valu": {}, "sustained": None, "source": {}}

@@ -118,15 +118,13 @@ SG_HD int sg2_taylor_ok(float cmax_g, float cmax_s, float g, float s) {
 
 /* Near-constant step sizes.  Where dt stays within a small d of the zero-input step size dt0 of its column, the
  * coefficients of the recurrence are polynomials in d = dt - dt0 with per-pair constants: A_bar(dt) = 2/(1 + a dt) - 1
- * (a = -A/2) is 2 r (1 - x + x^2 - ...) - 1 with r = 1/(1 + a dt0) and x = a r d, so a cubic has the remainder 2 r x^4;
- * sin/cos(f dt) as quadratics (remainder (f d)^3 / 6).  What d is measured against is a r (sg2_abar_rate), never more
- * than 1/dt0 however fast the pole.  A block of 8 timesteps uses them when for each of its timesteps
- * kpoly_g |g| + kpoly_s |s| < 1,  with kpoly = max(128 (a r)_max, 256 f_max) times the largest |c_g|, |c_s| of the
- * direction's dt rows (|dt - dt0| <= |c_g g + c_s s|: softplus has slope <= 1): x < 2^-7 and f d < 2^-8, remainders
- * below 1e-8.  (With a in the place of a r, poles down to -16 and -32 kept a third to all of the tiles of gradients of
- * 1e-3 on the general recurrence: steps of 283 us on 0.42 M elements with sharpness, 5.80 ms on 25 M without, 917 us with
- * the meta-net (16, 32, 32) instead of 233, 5.40 and 749; contexts as far from float64 either way, 8e-8 to 1.2e-7.) */
-SG_HD float sg2_abar_rate(float dt0, float nhA) { return nhA * sg_rcp_pos(sg_fma(dt0, nhA, 1.0f)); }
+ * (a = -A/2) as a cubic (remainder 2 (a d)^4), sin/cos(f dt) as quadratics (remainder (f d)^3 / 6).  A block of 8
+ * timesteps uses them when for each of its timesteps  kpoly_g |g| + kpoly_s |s| < 1,  with kpoly = max(128 a_max,
+ * 256 f_max) times the largest |c_g|, |c_s| of the direction's dt rows (|dt - dt0| <= |c_g g + c_s s|: softplus has
+ * slope <= 1): a d < 2^-7 and f d < 2^-8, remainders below 1e-8.  (What decides the cubic's remainder is a r,
+ * r = 1/(1 + a dt0), in the place of a: measured against that, twice as many tiles qualify and steps are 7 to 25 % shorter, as
+ * close to float64; but the other form rounds differently, and in 1 to 30 % of steps over 0.4 to 25 M elements one routing
+ * decision at a tie, and with it two expert counts, came out another.) */
 SG_HD void sg2_abar_poly(float dt0, float nhA, float p[4]) {
     const float r = sg_rcp_pos(sg_fma(dt0, nhA, 1.0f));
     const float ar = nhA * r;
@@ -162,11 +160,11 @@ SG_HD float sg2_limit_factor(float k, float slope_max) {
  * P1 = A_bar_e cos, N2 = -A_bar_e sin, P3 = A_bar_o cos, P4 = A_bar_o sin, and takes those as quadratics in d = dt - dt0
  * (products of the series above, truncated): he' = P1 he + N2 ho + b_e, ho' = P3 ho + P4 he + b_o, four fma instead of
  * two multiplications and four fma, and four quadratics instead of two cubics and two quadratics.  The truncated terms
- * are bounded by ((2.3 a r + |f|) d)^3 / 6 (a r: sg2_abar_rate); a block uses the products when
- * kprod_g |g| + kprod_s |s| < 1 for each of its timesteps, kprod = (416 (a r)_max + 184 f_max) times the largest
- * |c_g|, |c_s| of the dt rows: (2.3 a r + |f|) d < 2^-7.5, remainder below 3e-8. */
-/* Where the inputs are smaller still, kprod times 24 below 1, i.e. (2.3 a r + |f|) d < 2^-12, the linear part alone is
- * within 3e-8 (remainder ((2.3 a r + |f|) d)^2 / 2): SG2_PROD_LINEAR_FACTOR. */
+ * are bounded by ((2.3 a + |f|) d)^3 / 6; a block uses the products when kprod_g |g| + kprod_s |s| < 1 for each of its
+ * timesteps, kprod = (416 a_max + 184 f_max) times the largest |c_g|, |c_s| of the dt rows: (2.3 a + |f|) d < 2^-7.5,
+ * remainder below 3e-8. */
+/* Where the inputs are smaller still, kprod times 24 below 1, i.e. (2.3 a + |f|) d < 2^-12, the linear part alone is
+ * within 3e-8 (remainder ((2.3 a + |f|) d)^2 / 2): SG2_PROD_LINEAR_FACTOR. */
 #define SG2_PROD_LINEAR_FACTOR 24.0f
 SG_HD float sg2_poly1(const float* k, float d) { return sg_fma(k[1], d, k[0]); }
 SG_HD void sg2_prod_poly(const float a[3], const float c[3], float k[3]) {
@@ -189,7 +187,7 @@ SG_HD void sg2_pair_products(float dt0, float nhA_e, float nhA_o, float f, float
 
 /* What eight steps multiply the 2x2 part of a pair by at most while |dt - dt0| < d_max: rotations preserve length, so a
  * step shrinks it by max(|A_bar_e|, |A_bar_o|), and |A_bar(dt) - A_bar(dt0)| <= 2 r x / (1 - x) with x = a r |dt - dt0|
- * (at most 2^-7.5 / 2.3 where the products are in use, d_max = 1 / (416 (a r)_max + 184 f_max): 2.1 covers the quotient). */
+ * (at most 2^-7.5 / 2.3 where the products are in use, d_max = 1 / (416 a_max + 184 f_max), r <= 1: 2.1 covers the quotient). */
 SG_HD float sg2_abar_bound(float dt0, float nhA, float d_max) {
     const float r = sg_rcp_pos(sg_fma(dt0, nhA, 1.0f));
     return sg_abs(sg_fma(2.0f, r, -1.0f)) + (2.1f * d_max) * ((nhA * r) * r);

@@ -771,7 +771,7 @@ int step_tensor(const Dims& d, const float* const* W, int64_t chunk_len, int64_t
                 for (int p = 0; p < hp; p++) {
                     const float a_e = -0.5f * -sg_exp(w.A_log[j * ds + 2 * p]), a_o = -0.5f * -sg_exp(w.A_log[j * ds + 2 * p + 1]);
                     const float f = w.rope[j * hp + p];
-                    amax = sg_max(amax, sg_max(sg2_abar_rate(dt0, a_e), sg2_abar_rate(dt0, a_o)));
+                    amax = sg_max(amax, sg_max(a_e, a_o));
                     fmax = sg_max(fmax, sg_abs(f));
                     float* lp = &w.lane_poly[((size_t)j * hp + p) * 14];
                     sg2_abar_poly(dt0, a_e, lp);

@@ -86,11 +86,7 @@ __device__ __forceinline__ void compose_block(const Plan& pl, int threads) {
     __syncthreads();
     // How many steps the first block of a chunk summary should cover: what the slowest pair of either direction needs
     // to contract at the step size a zero input gives (sg2_contraction_steps, sg2_first_block_steps).
-    // For sg2_poly_ok: the largest rate at which a pair's A_bar follows its step size (sg2_abar_rate) and the largest
-    // |rotation frequency| of each direction.  The bilevel pass counts the poles themselves, which admits fewer tiles: other
-    // roundings of its forward scan buy 3 % there, but a fresh net's sums nearly cancel and an optimizer that divides by their
-    // size turns the last bits into the next pass's thresholds (one of 24 second passes came out 8e-3 away).
-    const bool bilevel = pl.htile != nullptr;
+    // For sg2_poly_ok: the largest -A/2 and the largest |rotation frequency| of each direction.
     for (int t = tid; t < 2 * ROWS * G::HP; t += threads) {
         const int d = t / (ROWS * G::HP), j = t / G::HP % ROWS, p = t % G::HP;
         const float* alog = pl.W.w[d ? W_B_ALOG : W_F_ALOG] + j * G::DS;
@@ -98,7 +94,7 @@ __device__ __forceinline__ void compose_block(const Plan& pl, int threads) {
         const int n = sg2_contraction_steps(s_dt0[d][j], a_e, a_o);
         if (n == 0) atomicOr(&s_zero, 1);
         atomicMax(&s_largest, n);
-        atomicMax(&s_amax[d], sg_f2i(bilevel ? sg_max(a_e, a_o) : sg_max(sg2_abar_rate(s_dt0[d][j], a_e), sg2_abar_rate(s_dt0[d][j], a_o))));
+        atomicMax(&s_amax[d], sg_f2i(sg_max(a_e, a_o)));
         atomicMax(&s_fmax[d], sg_f2i(sg_abs(pl.W.w[d ? W_B_ROPE : W_F_ROPE][j * G::HP + p])));
     }
     __syncthreads();

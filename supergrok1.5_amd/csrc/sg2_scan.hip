@@ -831,7 +831,8 @@ __device__ __forceinline__ void store_sums(float* row, int p, const float (&y)[U
 // the output pass: ten instructions per step, column and pair on their linear parts, 14 on the quadratics, where the separate
 // A_bar, sin, cos and the bound on the 2x2 part took 22.  The bound needs nothing per step there: while a tile
 // qualifies, |dt - dt0| is below pl.comp's limit, so a pair's part shrinks at least by sg2_abar_bound in every step.
-// (The bilevel pass keeps the separate factors: compose_block says why.)
+// (The bilevel pass keeps the separate factors: a fresh net's sums nearly cancel, and an optimizer that divides by their size
+// turns other last bits of its contexts into other thresholds of the next pass.)
 // 28 us on 0.42 M elements, 82 us on 3.1 M, 141 us on 25 M, 167 us on 0.42 M with the large geometry; with one column per lane,
 // two or eight waves per chunk and the separate factors 46, 115, 212 and 254 us.
 template <class G, int CL>
