@@ -452,9 +452,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const int jl = tid >> 3, p = tid & 7;    // scan role: pair p of columns jl and jl + 8
     const float* alog = pl.W.w[dir ? W_B_ALOG : W_F_ALOG];
     const float* rope = pl.W.w[dir ? W_B_ROPE : W_F_ROPE];
-    auto pole_e = [&](int h) { return -0.5f * -sg_exp(alog[(jl + 8 * h) * DS + 2 * p]); };
-    auto pole_o = [&](int h) { return -0.5f * -sg_exp(alog[(jl + 8 * h) * DS + 2 * p + 1]); };
-    auto rope_f = [&](int h) { return rope[(jl + 8 * h) * HP + p]; };
+    // -A/2 with A = -exp(A_log) of the two poles of a pair, and its frequency, in registers (256 now): with module-made poles about half
+    // of the blocks of ordinary gradients take a form that needs them, and forming them again in each, two loads and two
+    // exponentials, cost 7 to 10 % of a step (3.1 M bf16 1135 -> 1026 us, 0.42 M 267 -> 250, wide geometry 625 -> 576).
+    float poles[2][3];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        poles[h][0] = -0.5f * -sg_exp(alog[(jl + 8 * h) * DS + 2 * p]);
+        poles[h][1] = -0.5f * -sg_exp(alog[(jl + 8 * h) * DS + 2 * p + 1]);
+        poles[h][2] = rope[(jl + 8 * h) * HP + p];
+        asm("" : "+v"(poles[h][0]), "+v"(poles[h][1]), "+v"(poles[h][2]));       // (keeps the compiler from forming them where they are used)
+    }
+    auto pole_e = [&](int h) { return poles[h][0]; };
+    auto pole_o = [&](int h) { return poles[h][1]; };
+    auto rope_f = [&](int h) { return poles[h][2]; };
     LanePoly<true> LP[2];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -862,10 +873,18 @@ __global__ __launch_bounds__((64 * Split<G, CL>::WAVES)) __attribute__((amdgpu_w
     const float* rope = pl.W.w[dir ? W_B_ROPE : W_F_ROPE];
     const float* tay = pl.comp + 2 * SG2_COMP_GROUPS * G::ROWS * 3 + dir * 2 * G::ROWS * 4;
     auto col = [&](int h) { return c0 + jl + CPH * h; };
-    // -A/2 with A = -exp(A_log): the two poles of a pair (formed again where an exceptional block needs them)
-    auto pole_e = [&](int h) { return -0.5f * -sg_exp(alog[col(h) * DS + 2 * p]); };
-    auto pole_o = [&](int h) { return -0.5f * -sg_exp(alog[col(h) * DS + 2 * p + 1]); };
-    auto rope_f = [&](int h) { return rope[col(h) * HP + p]; };
+    // -A/2 with A = -exp(A_log): the two poles of a pair, and its frequency (see k_replay)
+    float poles[CL][3];
+#pragma unroll
+    for (int h = 0; h < CL; h++) {
+        poles[h][0] = -0.5f * -sg_exp(alog[col(h) * DS + 2 * p]);
+        poles[h][1] = -0.5f * -sg_exp(alog[col(h) * DS + 2 * p + 1]);
+        poles[h][2] = rope[col(h) * HP + p];
+        asm("" : "+v"(poles[h][0]), "+v"(poles[h][1]), "+v"(poles[h][2]));       // (keeps the compiler from forming them where they are used)
+    }
+    auto pole_e = [&](int h) { return poles[h][0]; };
+    auto pole_o = [&](int h) { return poles[h][1]; };
+    auto rope_f = [&](int h) { return poles[h][2]; };
     const sg::cfloat_p lim = sg::as_const(pl.comp) + 2 * SG2_COMP_GROUPS * G::ROWS * 3 + 2 * 2 * G::ROWS * 4;
     const float cmax_g = lim[2 * dir], cmax_s = lim[2 * dir + 1];              // what decides whether a tile may use the Taylor polynomials
     const float kpoly_g = lim[4 + 2 * dir], kpoly_s = lim[5 + 2 * dir];        // ... a block the lane polynomials (sg2_poly_ok)
@@ -1125,9 +1144,17 @@ __global__ __launch_bounds__((64 * Split<G, CL>::WAVES)) __attribute__((amdgpu_w
     const float* alog = pl.W.w[dir ? W_B_ALOG : W_F_ALOG];
     const float* rope = pl.W.w[dir ? W_B_ROPE : W_F_ROPE];
     auto col = [&](int h) { return c0 + jl + CPH * h; };
-    auto pole_e = [&](int h) { return -0.5f * -sg_exp(alog[col(h) * DS + 2 * p]); };
-    auto pole_o = [&](int h) { return -0.5f * -sg_exp(alog[col(h) * DS + 2 * p + 1]); };
-    auto rope_f = [&](int h) { return rope[col(h) * HP + p]; };
+    float poles[CL][3];
+#pragma unroll
+    for (int h = 0; h < CL; h++) {
+        poles[h][0] = -0.5f * -sg_exp(alog[col(h) * DS + 2 * p]);
+        poles[h][1] = -0.5f * -sg_exp(alog[col(h) * DS + 2 * p + 1]);
+        poles[h][2] = rope[col(h) * HP + p];
+        asm("" : "+v"(poles[h][0]), "+v"(poles[h][1]), "+v"(poles[h][2]));       // (keeps the compiler from forming them where they are used)
+    }
+    auto pole_e = [&](int h) { return poles[h][0]; };
+    auto pole_o = [&](int h) { return poles[h][1]; };
+    auto rope_f = [&](int h) { return poles[h][2]; };
     LanePoly<true> LP[CL];
 #pragma unroll
     for (int h = 0; h < CL; h++) {
