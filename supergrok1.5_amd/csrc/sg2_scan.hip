@@ -283,9 +283,13 @@ __device__ __forceinline__ void gates_of(float g, float s, int c0, const float* 
 // project_steps (Taylor form) on the same operands, so it is the same float; the step-size row receives dt - dt0, which
 // is what the lane polynomials of the recurrence take.
 // dxk: this lane's 16 skips D * x-branch of (column cj, timestep 16 cq + k), kept for gate_rows.
-template <class G, bool HAS_S>
-__device__ __forceinline__ void project_rows(float g, float s, int tid, const float* s_coef, const float* s_tay, float* s_dt, float* s_ux,
-                                             float* s_B, float* s_C, float (&dxk)[G::DI]) {
+// DELTA false, for a tile whose steps are inside the Taylor range but not all on the polynomials (with timesteps per lane there, 3.1 M
+// bf16 elements took 1026 us a step for 1001, 25 M 5595 for 5468): the step-size row receives dt itself,
+// and angle the lane's verdict on the two blocks of its timesteps (bits 0 / 1: every angle of its column small enough for
+// sg_sincos_small / sg_sincos_tiny in the first, bits 2 / 3 in the second; see project_steps).
+template <class G, bool HAS_S, bool DELTA>
+__device__ __forceinline__ void project_rows(float g, float s, int tid, const float* s_coef, const float* s_tay, const float* s_fmax, float* s_dt,
+                                             float* s_ux, float* s_B, float* s_C, float (&dxk)[G::DI], int& angle) {
     constexpr int DI = G::DI, DS = G::DS;
     static_assert(DI == 16 && DS == 16 && SCAN_TT == 64 && LDS_STRIDE == SCAN_TT + 4, "64 lanes: 16 columns x 4 quarters, 32 rows x 2 halves");
     auto delta = [&](const f32x4 t, float gg, float ss) { return HAS_S ? sg_fma(t[0], gg, t[1] * ss) : t[0] * gg; };
@@ -305,6 +309,8 @@ __device__ __forceinline__ void project_rows(float g, float s, int tid, const fl
         const f32x4 tp = *reinterpret_cast<const f32x4*>(s_tay + cj * 4);
         float* const r_dt = s_dt + cj * LDS_STRIDE + 16 * cq;
         float* const r_ux = s_ux + cj * LDS_STRIDE + 16 * cq;
+        const float fmax = DELTA ? 0.0f : s_fmax[cj];
+        bool small[2] = {true, true}, tiny[2] = {true, true};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             f32x4 g4, s4, d4, u4;
@@ -313,13 +319,18 @@ __device__ __forceinline__ void project_rows(float g, float s, int tid, const fl
             for (int e = 0; e < 4; e++) {
                 const float dtv = poly(tp, delta(cd, g4[e], s4[e]));
                 const float xbv = eval(cx, g4[e], s4[e]);
-                d4[e] = dtv - tp[0];
+                d4[e] = DELTA ? dtv - tp[0] : dtv;
                 u4[e] = dtv * xbv;
                 dxk[4 * i + e] = cx[3] * xbv;
+                if (!DELTA) {
+                    small[i / 2] = small[i / 2] && (dtv * fmax < SG_SINCOS_SMALL_LIMIT);
+                    tiny[i / 2] = tiny[i / 2] && (dtv * fmax < SG_SINCOS_TINY_LIMIT);
+                }
             }
             *reinterpret_cast<f32x4*>(r_dt + 4 * i) = d4;
             *reinterpret_cast<f32x4*>(r_ux + 4 * i) = u4;
         }
+        if (!DELTA) angle = (small[0] ? 1 : 0) | (tiny[0] ? 2 : 0) | (small[1] ? 4 : 0) | (tiny[1] ? 8 : 0);
     }
     {
         const int br = tid & 31, bh = tid >> 5;
@@ -565,16 +576,30 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         unsigned long long large[2] = {0, 0}, nottiny[2] = {0, 0};
         float dxv[DI];           // D * x-branch, kept for phase C: of this lane's timestep, or (dgiven) of its column's 16 timesteps
         if (dgiven) {
-            if (has_s) project_rows<G, true>(g, sh, tid, s_coef, s_tay, s_dt, s_ux, s_B, s_C, dxv);
-            else project_rows<G, false>(g, sh, tid, s_coef, s_tay, s_dt, s_ux, s_B, s_C, dxv);
+            int none;
+            if (has_s) project_rows<G, true, true>(g, sh, tid, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, none);
+            else project_rows<G, false, true>(g, sh, tid, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, none);
+        } else if (tay) {
+            int angle;
+            if (has_s) project_rows<G, true, false>(g, sh, tid, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, angle);
+            else project_rows<G, false, false>(g, sh, tid, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, angle);
+            // blocks 2 q and 2 q + 1 are in the hands of lanes 16 q .. 16 q + 15, a column each
+#pragma unroll
+            for (int odd = 0; odd < 2; odd++) {
+                const unsigned long long l = __builtin_amdgcn_ballot_w64(!(angle & (odd ? 4 : 1))), n = __builtin_amdgcn_ballot_w64(!(angle & (odd ? 8 : 2)));
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const unsigned long long blk = 255ull << (16 * q + 8 * odd);
+                        if ((l >> (16 * q + 8 * h)) & 255u) large[h] |= blk;
+                        if ((n >> (16 * q + 8 * h)) & 255u) nottiny[h] |= blk;
+                    }
+            }
         } else {
             int angle[2];
-            auto run = [&](auto has_s_c, auto tay_c) {
-                constexpr bool HS = decltype(has_s_c)::value, TY = decltype(tay_c)::value;
-                project_steps<G, 2, true, false, HS, TY>(g, sh, tu, 0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, angle);
-            };
-            if (tay) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
-            else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
+            if (has_s) project_steps<G, 2, true, false, true, false>(g, sh, tu, 0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, angle);
+            else project_steps<G, 2, true, false, false, false>(g, sh, tu, 0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dxv, angle);
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 large[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 1));
@@ -688,15 +713,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         // ---------------- phase C: gate, D skip, out_proj, scatter to element order (one 32-byte row per lane)
         {
             float o[DI];
-            if (dgiven) {        // the row owners gate their 16 outputs in place, then every timestep collects its 16 columns
+            if (tay) {           // the row owners gate their 16 outputs in place, then every timestep collects its 16 columns
                 if (has_s) gate_rows<G, true>(tid, s_coef, s_tay, s_B, s_C, s_y, dxv);
                 else gate_rows<G, false>(tid, s_coef, s_tay, s_B, s_C, s_y, dxv);
                 __syncthreads();
 #pragma unroll
                 for (int jj = 0; jj < DI; jj++) o[jj] = s_y[jj * LDS_STRIDE + tu];
             } else {
-                if (tay) { if (has_s) gates_of<G, 2, true, true>(g, sh, 0, s_coef, s_tay, o); else gates_of<G, 2, false, true>(g, sh, 0, s_coef, s_tay, o); }
-                else { if (has_s) gates_of<G, 2, true, false>(g, sh, 0, s_coef, s_tay, o); else gates_of<G, 2, false, false>(g, sh, 0, s_coef, s_tay, o); }
+                if (has_s) gates_of<G, 2, true, false>(g, sh, 0, s_coef, s_tay, o);
+                else gates_of<G, 2, false, false>(g, sh, 0, s_coef, s_tay, o);
 #pragma unroll
                 for (int jj = 0; jj < DI; jj++) o[jj] = sg_fma(s_y[jj * LDS_STRIDE + tu], o[jj], dxv[jj]);
             }
