@@ -31,7 +31,7 @@ typedef float vf32 __attribute__((ext_vector_type(32)));
 // One word of every 64 bytes of the weights that come in through the scalar cache, all requested at once: cold, each of
 // the loads between an element's products waits for the memory by itself, some forty times in a row.  With the expert
 // records' loads all in flight before the first of them is stored, the launch over 8 small tensors takes 10.4 us, 12.1
-// without, and a step of the wide geometry over 0.42 M elements 458 us for 471.
+// without, and a step of the wide geometry over 0.42 M elements 13 us less.
 template <class G>
 __device__ __forceinline__ void warm_scalar_cache(const Plan& pl) {
     uint32_t x = 0;
@@ -507,8 +507,8 @@ __global__ __launch_bounds__(ELEM_THREADS) void k_elem_any(Plan pl, int ctx_stri
 }  // namespace
 
 // A wave per head while that takes at most one workgroup per compute unit.  Beyond, the element's chain is shorter still, but
-// every 64 elements pay for an LDS fill of 28 KB that otherwise serves 256: steps over 1000 elements in 3 tensors 65.9 -> 64.2 us,
-// 5000 in 4 84.0 -> 82.6, 8 small tensors 46.4 -> 43.9, but 15 000 in 6 (about 300 parts) 101.5 -> 102.5, 0.42 M 212 -> 274.
+// every 64 elements pay for an LDS fill of 28 KB that otherwise serves 256: 8 small tensors -2.5 us a step, 1000 elements in 3
+// tensors -1.7, 5000 in 4 -1.4, but 15 000 in 6 (about 300 parts) +1, 0.42 M +62.
 constexpr int HEADS_PARTS = 256;
 inline bool by_heads(const Plan& pl) { return pl.elem_kind != ELEM_ANY && pl.elem_tiles * (ELEM_TILE / 64) <= HEADS_PARTS; }
 

@@ -1497,8 +1497,8 @@ template <class G>
 int launch_scan_geo(const Plan& pl, hipStream_t st) {
     // One column per lane while all waves of the call are then resident at once (two per SIMD): a chunk's steps are a serial
     // chain, and a wave alone on its SIMD takes as long for one column's instructions as two waves for theirs.  Replay and
-    // summaries of 30 000 elements 151 -> 121 us a step (large geometry 182 -> 157), of 200 000 217 -> 194; past the line
-    // 300 000 elements 236 -> 243 us, 120 000 at the large geometry 265 -> 284.
+    // summaries of 30 000 elements 137 -> 102 us a step (large geometry 222 -> 160), of 200 000 229 -> 183; past the line
+    // two columns are ahead, by 3 % at 300 000 elements, by 7 % at 120 000 of the large geometry.
     constexpr int RESIDENT = 2 * 4 * 256;
     const auto single = [](int chunks) { return 2 * chunks * Split<G, 1>::WAVES <= RESIDENT; };
     if (pl.wchunks > 0) {

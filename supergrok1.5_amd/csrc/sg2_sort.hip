@@ -75,7 +75,7 @@ __device__ __forceinline__ int32_t payload_of(float g, int index) { return index
 // where one workgroup sorts it) of such gradients only takes two passes: bfloat16 is the upper half of the key; a float16
 // that is not zero has its ten mantissa bits at 13 .. 22 and an exponent field from 103 (subnormals) to 142, so the key >> 13
 // less 102 << 10 fits 16 bits and orders like the key.  Arrays, payloads and whatever is read from them stay as they are.
-// (3.1 M bfloat16 elements: the step 877 -> 812 us, two scatters of 17, two counts of 9 and four scans of 5 us less.)
+// (3.1 M bfloat16 elements: 65 us less, two scatters of 17, two counts of 9 and four scans of 5 us less.)
 struct KeyBits {
     int shift, bias;
 };
@@ -554,8 +554,8 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort_tile(Plan pl) {
 // where the run lies earlier (stable, as the passes are).  The runs pass through LDS two at a time while the next two are on
 // their way, and a workgroup looks its 2048 keys up by halving steps.
 // Bound by the vector ALU (three instructions a step, 13 steps a key and run) where a tensor has many runs: runs of 4096
-// instead of 2048 halve that and add 6 us of sorting.  0.42 M elements: 21 + 26 us; steps 215 -> 203 us, 15 000 elements in 6
-// tensors 102 -> 81, 30 000 in 5 105 -> 88, one tensor of 60 000 113 -> 103.
+// instead of 2048 halve that and add 6 us of sorting.  0.42 M elements: 21 + 26 us for 57; 15 000 elements in 6 tensors and
+// 30 000 in 5 take 21 and 17 us less, one tensor of 60 000 10.
 constexpr int RUN_TILES = 2, RUN = RUN_TILES * SORT_TILE_SMALL;
 template <class G, bool HALF>
 __global__ __launch_bounds__(SORT_THREADS) void k_sort_runs(Plan pl) {
@@ -741,9 +741,9 @@ int launch_passes(const Plan& pl, hipStream_t st) {
 }
 
 // Tiles of the largest tensor up to which runs are merged.  The merge's work grows with the square of a tensor's length and the
-// passes' with the length; 16-bit gradients have two passes only.  Step times with passes / runs over small tiles: four fp32
-// tensors of 20 000 133 / 116 us, one of 60 000 112 / 103, of 80 000 132 / 132, of 130 000 148 / 155, sixteen of 60 000
-// 337 / 325, thirty 514 / 517 (hence the product); bfloat16, one of 8000 85 / 76, four of 20 000 111 / 114, one of 60 000 92 / 116.
+// passes' with the length; 16-bit gradients have two passes only.  What runs change against passes over small tiles: four
+// fp32 tensors of 20 000 -17 us, one of 60 000 -9, of 80 000 0, of 130 000 +7, sixteen of 60 000 -12, thirty +3 (hence the
+// product); bfloat16, one of 8000 -9, four of 20 000 +3, one of 60 000 +24.
 constexpr int MERGE_TILES = 40, MERGE_WORK = 20000, HALF_MERGE_TILES = 4;
 inline bool merges(const Plan& pl, bool half) {
     return pl.sort_widest <= (half ? HALF_MERGE_TILES : MERGE_TILES) && (int64_t)pl.sort_tiles * pl.sort_widest <= MERGE_WORK;

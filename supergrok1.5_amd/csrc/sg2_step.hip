@@ -57,39 +57,42 @@ int effective_chunk_len(int P, Numels numels) {
     return set > 0 ? set : auto_chunk_len(P, numels);
 }
 
-// The chunk length of sg2_clipped_step.  256 for small calls at the default geometry, while the chip has a SIMD for each of
-// their waves (one column per lane, so two a chunk): the replay is then half as long, and so is what the summaries of the
-// module's weights need (184 to 240 steps) less than a chunk (30 000 elements 121 -> 105 us a step, 600 in one tensor
-// 82 -> 67; with every pole slowed by e, whose summaries need more, 125 -> 140, by e^2 171 -> 141).  512 while the chip holds all
-// chunks of 512 at once (`slots` workgroups: two waves per SIMD).  Beyond that the chunks run in rounds, and a round takes as
-// long as a chunk whether it is full or not; so does its share of the summaries, which walk `tail` steps whatever the
-// chunk's length (what the module's weights need, at the summary's cost per step).  Of the lengths that just fill
-// 1, 2, 3 ... rounds, a multiple of 128 up to 4096, the one with the least of both is taken.  Against chunks of 4096 / 2048 /
-// 1024 / 512 by the amount of work: 0.42 M elements at the large geometry 557 -> 467 us (1792 for 512), 3 M there 2.69 -> 2.47 ms
-// (3968 for 1024), 1.2 M at the default one 468 -> 430 us (1280 for 512), 3.1 M 963 -> 877 us (3200 for 1024).
+// The chunk length of sg2_clipped_step.
+// Default geometry: 256 for small calls, while the chip has a SIMD for each of their waves (one column per lane, so two a
+// chunk): the replay is then half as long, and so is what the summaries of the module's weights need (184 to 240 steps) less
+// than a chunk (30 000 elements 127 -> 102 us a step, 600 in one tensor 86 -> 72; with every pole slowed by e, whose summaries
+// need more, 125 -> 140, by e^2 171 -> 141).  Otherwise by the amount of work, as in sg2_batched_step: a tensor's last
+// chunks, its largest gradients, take slower forms, and short chunks spread them (chunks that fill the chip in whole rounds
+// as below: 3.1 M bf16 elements 930 -> 998 us, 0.42 M and 1.2 M the same).
+// Large geometry: 512 while the chip holds all chunks of 512 at once (`SLOTS` workgroups).  Beyond that the chunks run in
+// rounds, and a round takes as long as a chunk whether it is full or not; so does its share of the summaries, which walk
+// `TAIL` steps whatever the chunk's length (what the module's weights need, at the summary's cost per step).  Of the lengths
+// that just fill 1, 2, 3 ... rounds, a multiple of 128 up to 4096, the one with the least of both is taken: 0.42 M elements
+// 731 -> 573 us (1792 for 512), 3 M 3.45 -> 3.10 ms (3968 for 1024).
 int fitted_chunk_len(int geo, int P, Numels numels) {
     const int set = g_chunk_len.load();
     if (set > 0) return set;
     constexpr int STEP = 128, SHORTEST = 512, LONGEST = 4096;
-    const int64_t slots = geo == GEO_LARGE ? 512 : 2048, tail = geo == GEO_LARGE ? 288 : 128;
+    constexpr int64_t SLOTS = 512, TAIL = 288;
     auto chunks = [&](int64_t L) {
         int64_t n = 0;
         for (int i = 0; i < P; i++) n += 2 * ((numels[i] + L - 1) / L);
         return n;
     };
-    if (chunks(SHORTEST) <= slots) {
+    if (geo == GEO_DEFAULT) {
         int64_t widest = 0;
         for (int i = 0; i < P; i++) widest = std::max(widest, numels[i]);
-        return geo == GEO_DEFAULT && widest > SHORTEST && 2 * chunks(SHORTEST / 2) <= 1024 ? SHORTEST / 2 : SHORTEST;
+        return widest > SHORTEST && 2 * chunks(SHORTEST / 2) <= 1024 ? SHORTEST / 2 : auto_chunk_len(P, numels);
     }
+    if (chunks(SHORTEST) <= SLOTS) return SHORTEST;
     int64_t total = 0;
     for (int i = 0; i < P; i++) total += numels[i];
-    const int64_t fewest = std::max<int64_t>(1, (chunks(LONGEST) + slots - 1) / slots);
-    int64_t best = LONGEST, best_cost = fewest * (LONGEST + tail);
+    const int64_t fewest = std::max<int64_t>(1, (chunks(LONGEST) + SLOTS - 1) / SLOTS);
+    int64_t best = LONGEST, best_cost = fewest * (LONGEST + TAIL);
     for (int64_t rounds = fewest; rounds < fewest + 4; rounds++) {
-        int64_t L = std::max<int64_t>(SHORTEST, (2 * total / (rounds * slots) + STEP - 1) / STEP * STEP);      // no shorter one can do
-        while (L < LONGEST && chunks(L) > rounds * slots) L += STEP;
-        if (L < LONGEST && rounds * (L + tail) < best_cost) { best = L; best_cost = rounds * (L + tail); }
+        int64_t L = std::max<int64_t>(SHORTEST, (2 * total / (rounds * SLOTS) + STEP - 1) / STEP * STEP);      // no shorter one can do
+        while (L < LONGEST && chunks(L) > rounds * SLOTS) L += STEP;
+        if (L < LONGEST && rounds * (L + TAIL) < best_cost) { best = L; best_cost = rounds * (L + TAIL); }
     }
     return (int)best;
 }
@@ -166,11 +169,11 @@ __global__ __launch_bounds__(256) void k_pad_weights(PadArgs a) {
 // Keys per sort tile.  A scatter of 8192 keys is 16 rounds in series per wave whatever the call's size.  Calls of fewer
 // elements than make a large tile for every fourth CU take the small ones, and so do those whose tensors have at most
 // 65 536 elements each up to a large tile for every CU; with the small ones come the merged runs (see launch_sort_geo).
-// Step times with large / small tiles: one tensor of 200 000 180 / 164 us, of 500 000 261 / 251, two of 200 000 237 / 223,
-// one of 200 000 bfloat16 160 / 136; 16 of 60 000 336 / 320 us and 33 of 60 000 567 / 563, but 12 of 100 000 402 / 418, 256
-// of 9000 751 / 760 and 400 of 60 000 5.55 / 5.86 ms: then the small tiles fill no idle CUs and scatter shorter runs.
+// What small tiles change in a step: one tensor of 200 000 elements -16 us, of 500 000 -10, two of 200 000 -14, one of 200 000
+// bfloat16 -24, 16 of 60 000 -16 and 33 of 60 000 -4, but 12 of 100 000 +16, 256 of 9000 +9 and 400 of 60 000 +310: then
+// they fill no idle CUs and scatter shorter runs.
 // Tensors of at most one small tile each are sorted in LDS by one launch (of at most a large one, in calls that take
-// those: beside small tiles, 8000 elements in one workgroup are 93 us of a step and 79 in runs).
+// those: beside small tiles, 8000 elements take 14 us more in one workgroup than in runs).
 inline int sort_tile_for(int64_t widest, int64_t total) {
     const bool small = total < (int64_t)64 * SORT_TILE || (widest <= 32 * SORT_TILE_SMALL && total < (int64_t)256 * SORT_TILE);
     return small && widest > SORT_TILE_SMALL ? SORT_TILE_SMALL : SORT_TILE;
