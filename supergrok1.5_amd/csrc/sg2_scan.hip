@@ -795,9 +795,12 @@ __device__ __forceinline__ ChunkOf chunk_of(const Plan& pl, const int* chunk_pre
 // The projections of a tile that runs on the products throughout, formed by lanes that own rows: lane (row r, part q) of
 // wave w forms column CPW w + r (dt - dt0, dt * x-branch, D * x-branch) and row CPW w + r of B (and C) for timesteps SPL q ..
 // SPL q + SPL - 1.  s_in: the tile's 64 g and 64 s, the wave's own copy.  Values and reasons as in project_rows.
-template <class G, int CL, bool OUT, bool HAS_S>
-__device__ __forceinline__ void project_own_rows(const float* s_in, int lane, int c0, const float* s_coef, const float* s_tay, float* s_dt, float* s_ux,
-                                                 float* s_B, float* s_C, float (&dxk)[Split<G, CL>::SPL]) {
+// DELTA false: as there (0.42 M elements 247.5 -> 242 us a step, 3.1 M bf16 932 -> 919, 30 000 102 -> 100); large / nottiny[h] receive the blocks of 8 timesteps in which an angle of columns c0 + CPH h ..
+// c0 + CPH h + CPH - 1 is too large for sg_sincos_small / sg_sincos_tiny.
+template <class G, int CL, bool OUT, bool HAS_S, bool DELTA>
+__device__ __forceinline__ void project_own_rows(const float* s_in, int lane, int c0, const float* s_coef, const float* s_tay, const float* s_fmax,
+                                                 float* s_dt, float* s_ux, float* s_B, float* s_C, float (&dxk)[Split<G, CL>::SPL],
+                                                 unsigned long long (&large)[CL], unsigned long long (&nottiny)[CL]) {
     constexpr int DI = G::DI, CPW = Split<G, CL>::CPW, SPL = Split<G, CL>::SPL;
     auto delta = [&](const f32x4 t, float gg, float ss) { return HAS_S ? sg_fma(t[0], gg, t[1] * ss) : t[0] * gg; };
     auto poly = [&](const f32x4 t, float d) { return sg_fma(sg_fma(sg_fma(t[3], d, t[2]), d, t[1]), d, t[0]); };
@@ -810,6 +813,10 @@ __device__ __forceinline__ void project_own_rows(const float* s_in, int lane, in
     float* const r_ux = s_ux + row * LDS_STRIDE + t0;
     float* const r_B = s_B + bc_slot<G>(row) * LDS_STRIDE + t0;
     float* const r_C = OUT ? s_C + bc_slot<G>(row) * LDS_STRIDE + t0 : nullptr;
+    constexpr int NB = SPL > UB ? SPL / UB : 1;              // blocks that a lane has timesteps of
+    static_assert(UB == 8 && (SPL == 4 || SPL % 8 == 0), "a lane has half a block or whole ones");
+    const float fmax = DELTA ? 0.0f : s_fmax[row];
+    bool is_large[NB] = {}, not_tiny[NB] = {};
 #pragma unroll
     for (int i = 0; i < SPL / 4; i++) {
         const f32x4 g4 = *reinterpret_cast<const f32x4*>(s_in + t0 + 4 * i);
@@ -819,7 +826,11 @@ __device__ __forceinline__ void project_own_rows(const float* s_in, int lane, in
         for (int e = 0; e < 4; e++) {
             const float dtv = poly(tp, delta(cd, g4[e], s4[e]));
             const float xbv = eval(cx, g4[e], s4[e]);
-            d4[e] = dtv - tp[0];
+            d4[e] = DELTA ? dtv - tp[0] : dtv;
+            if (!DELTA) {
+                is_large[i * 4 / UB] = is_large[i * 4 / UB] || !(dtv * fmax < SG_SINCOS_SMALL_LIMIT);
+                not_tiny[i * 4 / UB] = not_tiny[i * 4 / UB] || !(dtv * fmax < SG_SINCOS_TINY_LIMIT);
+            }
             u4[e] = dtv * xbv;
             if (OUT) dxk[4 * i + e] = cx[3] * xbv;
             b4[e] = eval(cb, g4[e], s4[e]);
@@ -829,6 +840,22 @@ __device__ __forceinline__ void project_own_rows(const float* s_in, int lane, in
         *reinterpret_cast<f32x4*>(r_ux + 4 * i) = u4;
         *reinterpret_cast<f32x4*>(r_B + 4 * i) = b4;
         if (OUT) *reinterpret_cast<f32x4*>(r_C + 4 * i) = k4;
+    }
+    if (!DELTA) {
+        constexpr int CPH = Split<G, CL>::CPH;
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            const unsigned long long l = __builtin_amdgcn_ballot_w64(is_large[k]), n = __builtin_amdgcn_ballot_w64(not_tiny[k]);
+#pragma unroll
+            for (int q = 0; q < 64 / CPW; q++)
+#pragma unroll
+                for (int h = 0; h < CL; h++) {
+                    const int at = CPW * q + CPH * h;
+                    const unsigned long long blk = 255ull << (SPL * q / UB * UB + UB * k);
+                    if ((l >> at) & ((1u << CPH) - 1)) large[h] |= blk;
+                    if ((n >> at) & ((1u << CPH) - 1)) nottiny[h] |= blk;
+                }
+        }
     }
 }
 
@@ -988,21 +1015,21 @@ __global__ __launch_bounds__((64 * Split<G, CL>::WAVES)) __attribute__((amdgpu_w
             const bool fast = LITE && pl.htile == nullptr && ty && cnt % UB == 0 && __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kprod_g, kprod_s, g, sh)) == 0;
             unsigned long long notpoly = 0, large[CL] = {}, nottiny[CL] = {};
             float unused[CPW];
-            if (fast) {
+            if (!fast) notpoly = __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kpoly_g, kpoly_s, g, sh));
+            if (ty) {
                 s_in[tu] = g;
                 if (has_s) s_in[SCAN_TT + tu] = sh;
                 __builtin_amdgcn_wave_barrier();      // one wave's LDS accesses execute in program order
-                if (has_s) project_own_rows<G, CL, false, true>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, nullptr, unused);
-                else project_own_rows<G, CL, false, false>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, nullptr, unused);
+                auto run = [&](auto has_s_c, auto delta_c) {
+                    project_own_rows<G, CL, false, decltype(has_s_c)::value, decltype(delta_c)::value>(s_in, lane, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B,
+                                                                                                       nullptr, unused, large, nottiny);
+                };
+                if (fast) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
+                else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
             } else {
                 int angle[CL];
-                auto run = [&](auto has_s_c, auto tay_c) {
-                    project_steps<G, CL, false, true, decltype(has_s_c)::value, decltype(tay_c)::value>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B,
-                                                                                                   nullptr, unused, angle);
-                };
-                if (ty) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
-                else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
-                notpoly = __builtin_amdgcn_ballot_w64(!sg2_poly_ok(kpoly_g, kpoly_s, g, sh));
+                if (has_s) project_steps<G, CL, false, true, true, false>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, nullptr, unused, angle);
+                else project_steps<G, CL, false, true, false, false>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, nullptr, unused, angle);
 #pragma unroll
                 for (int h = 0; h < CL; h++) {
                     large[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 1));
@@ -1261,20 +1288,20 @@ __global__ __launch_bounds__((64 * Split<G, CL>::WAVES)) __attribute__((amdgpu_w
         const bool ty = __builtin_amdgcn_ballot_w64(!sg2_taylor_ok(cmax_g, cmax_s, g, sh)) == 0;
         const bool fast = ty && notpoly == 0;
         unsigned long long large[CL] = {}, nottiny[CL] = {};
-        float dx[CPW];           // D * x-branch: of this lane's column for its SPL timesteps (fast), or of its timestep for the wave's columns
-        if (fast) {
+        float dx[CPW];           // D * x-branch: of this lane's column for its SPL timesteps (ty), or of its timestep for the wave's columns
+        if (ty) {
             s_in[tu] = g;
             if (has_s) s_in[SCAN_TT + tu] = sh;
             __builtin_amdgcn_wave_barrier();
-            if (has_s) project_own_rows<G, CL, true, true>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, s_C, dx);
-            else project_own_rows<G, CL, true, false>(s_in, lane, c0, s_coef, s_tay, s_dt, s_ux, s_B, s_C, dx);
+            auto run = [&](auto has_s_c, auto delta_c) {
+                project_own_rows<G, CL, true, decltype(has_s_c)::value, decltype(delta_c)::value>(s_in, lane, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dx, large, nottiny);
+            };
+            if (fast) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
+            else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
         } else {
             int angle[CL];
-            auto run = [&](auto has_s_c, auto tay_c) {
-                project_steps<G, CL, true, true, decltype(has_s_c)::value, decltype(tay_c)::value>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dx, angle);
-            };
-            if (ty) { if (has_s) run(std::true_type{}, std::true_type{}); else run(std::false_type{}, std::true_type{}); }
-            else { if (has_s) run(std::true_type{}, std::false_type{}); else run(std::false_type{}, std::false_type{}); }
+            if (has_s) project_steps<G, CL, true, true, true, false>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dx, angle);
+            else project_steps<G, CL, true, true, false, false>(g, sh, tu, c0, s_coef, s_tay, s_fmax, s_dt, s_ux, s_B, s_C, dx, angle);
 #pragma unroll
             for (int h = 0; h < CL; h++) {
                 large[h] = __builtin_amdgcn_ballot_w64(!(angle[h] & 1));
@@ -1349,7 +1376,7 @@ __global__ __launch_bounds__((64 * Split<G, CL>::WAVES)) __attribute__((amdgpu_w
         __builtin_amdgcn_wave_barrier();        // a wave gates its own columns: its LDS accesses execute in program order
 
         // gate and D skip, in place
-        if (fast) {
+        if (ty) {
             const int row = c0 + lane % CPW, t0 = SPL * (lane / CPW);
             const f32x4 cz = *reinterpret_cast<const f32x4*>(s_coef + (SG2_COMP_Z * DI + row) * 4);
             const f32x4 tz = *reinterpret_cast<const f32x4*>(s_tay + (DI + row) * 4);
@@ -1372,8 +1399,8 @@ __global__ __launch_bounds__((64 * Split<G, CL>::WAVES)) __attribute__((amdgpu_w
             else gate(std::false_type{});
         } else {
             float gv[CPW];
-            if (ty) { if (has_s) gates_of<G, CL, true, true>(g, sh, c0, s_coef, s_tay, gv); else gates_of<G, CL, false, true>(g, sh, c0, s_coef, s_tay, gv); }
-            else { if (has_s) gates_of<G, CL, true, false>(g, sh, c0, s_coef, s_tay, gv); else gates_of<G, CL, false, false>(g, sh, c0, s_coef, s_tay, gv); }
+            if (has_s) gates_of<G, CL, true, false>(g, sh, c0, s_coef, s_tay, gv);
+            else gates_of<G, CL, false, false>(g, sh, c0, s_coef, s_tay, gv);
 #pragma unroll
             for (int q = 0; q < CPW; q++) s_dt[(c0 + q) * LDS_STRIDE + tu] = sg_fma(s_dt[(c0 + q) * LDS_STRIDE + tu], gv[q], dx[q]);
         }
