@@ -768,13 +768,15 @@ __device__ __forceinline__ void newton_schulz(const Mat& M, float inv, int steps
     typedef __attribute__((address_space(3))) bf16x8* lds_op;
     typedef __attribute__((address_space(3))) u32x4* lds_vec;
     typedef __attribute__((address_space(3))) bf16_t* lds_b16;
-    constexpr int mp = 32 * MT, WAVES = NS_THREADS / 64, GROW = 2 * mp, BATCH = 16;
+    constexpr int mp = 32 * MT, WAVES = NS_THREADS / 64, GROW = 2 * mp;
     const int np = M.np, row = 2 * np, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bool odd = np & 64;
     const lds_t Y = (lds_t)smem, G = Y + mp * row;
-    // sixteen bytes of every chunk in order, a batch of them on their way at once
+    // sixteen bytes of every chunk in order, a batch of them on their way at once (few for a small matrix: 54 x 112 has two a lane)
     const int chunks = np / 8, dr = NS_THREADS / chunks, dc = NS_THREADS % chunks;
-    auto stream = [&](auto move) {
+    const bool few = mp * chunks <= 4 * NS_THREADS;
+    auto stream = [&](auto batch, auto move) {
+        constexpr int BATCH = decltype(batch)::value;
         int r = tid / chunks, c = tid % chunks;
         for (int i = tid; i < mp * chunks; i += BATCH * NS_THREADS) {
             int at[BATCH];
@@ -790,20 +792,24 @@ __device__ __forceinline__ void newton_schulz(const Mat& M, float inv, int steps
     };
     {
         const u32x4* __restrict__ src = reinterpret_cast<const u32x4*>(M.Y);
-        stream([&](int i, const int (&at)[BATCH], int n) {
+        auto load = [&](int i, const auto& at, int n) {
+            constexpr int BATCH = std::extent_v<std::remove_reference_t<decltype(at)>>;
             u32x4 v[BATCH];
 #pragma unroll
             for (int u = 0; u < BATCH; u++) if (u < n) v[u] = *(gvec_p)(src + i + u * NS_THREADS);
 #pragma unroll
             for (int u = 0; u < BATCH; u++) if (u < n) *(lds_vec)(Y + at[u]) = v[u];
-        });
+        };
+        if (few) stream(std::integral_constant<int, 4>{}, load);
+        else stream(std::integral_constant<int, 16>{}, load);
     }
     __syncthreads();
     // S S^T is symmetric: the tiles on and right of the diagonal, dealt so that the waves of a SIMD (w and w + 4) have at most
-    // three; each reads the rows of its row of tiles rt and, with a tile off the diagonal, those of ct.
-    const bool on = MT == 4 ? wave < 2 || wave == 4 || wave == 5 : wave < 2, off = MT == 4 ? wave != 4 && wave != 5 : wave == 2;
+    // three; each reads the rows of its row of tiles rt and, with a tile off the diagonal, those of ct.  (Of two rows of tiles all
+    // four are formed, a wave each: mirroring is longer than the product there.)
+    const bool on = MT == 4 ? wave < 2 || wave == 4 || wave == 5 : wave < 2, off = MT == 4 ? wave != 4 && wave != 5 : wave == 2 || wave == 3;
     const int rt = MT == 4 ? (wave < 2 ? 2 * wave : wave == 4 ? 1 : wave == 5 ? 3 : wave & 1) : wave & 1;
-    const int ct = MT == 4 ? (wave < 2 ? 2 * wave + 1 : wave < 4 ? 2 : 3) : 1;
+    const int ct = MT == 4 ? (wave < 2 ? 2 * wave + 1 : wave < 4 ? 2 : 3) : 1 - rt;
 #pragma unroll 1
     for (int it = 0; it < steps; it++) {
         int ln = lane;                       // keeps the address arithmetic in its phase: hoisted out of the loop it spills
@@ -874,7 +880,7 @@ __device__ __forceinline__ void newton_schulz(const Mat& M, float inv, int steps
             const lds_t at = G + (32 * rt + r32) * GROW;
 #pragma unroll
             for (int q = 0; q < 4; q += 2) put_row(at + ((sw ^ (4 * col + q)) << 4), g[J][q], g[J][q + 1]);
-            if (J) {
+            if (J && MT == 4) {
                 const lds_t mirror = G + (32 * col + 4 * kh) * GROW + 2 * (r32 & 7);
                 const int place = (4 * rt + (r32 >> 3)) ^ ns_swizzle(4 * kh, mp & 64);
 #pragma unroll
@@ -983,13 +989,16 @@ __device__ __forceinline__ void newton_schulz(const Mat& M, float inv, int steps
         __syncthreads();
     }
     u32x4* dst = reinterpret_cast<u32x4*>(steps & 1 ? M.Y2 : M.Y);
-    stream([&](int i, const int (&at)[BATCH], int n) {
+    auto store = [&](int i, const auto& at, int n) {
+        constexpr int BATCH = std::extent_v<std::remove_reference_t<decltype(at)>>;
         u32x4 v[BATCH];
 #pragma unroll
         for (int u = 0; u < BATCH; u++) if (u < n) v[u] = *(lds_vec)(Y + at[u]);
 #pragma unroll
         for (int u = 0; u < BATCH; u++) if (u < n) *(gvec_w)(dst + i + u * NS_THREADS) = v[u];
-    });
+    };
+    if (few) stream(std::integral_constant<int, 4>{}, store);
+    else stream(std::integral_constant<int, 16>{}, store);
 }
 
 __global__ __launch_bounds__(NS_THREADS) void k_newton_schulz(Batch B, int steps) {
