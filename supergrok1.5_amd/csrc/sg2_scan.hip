@@ -896,7 +896,7 @@ __device__ __forceinline__ void store_sums(float* row, int p, const float (&y)[U
 // qualifies, |dt - dt0| is below pl.comp's limit, so a pair's part shrinks at least by sg2_abar_bound in every step.
 // (The bilevel pass keeps the separate factors: a fresh net's sums nearly cancel, and an optimizer that divides by their size
 // turns other last bits of its contexts into other thresholds of the next pass.)
-// 44 us on 0.42 M elements, 110 us on 3.1 M, 89 us on 25 M whose tiles qualify, 80 us on 0.42 M with the large geometry; with one
+// 39 us on 0.42 M elements, 100 us on 3.1 M, 89 us on 25 M whose tiles qualify, 79 us on 0.42 M with the large geometry; with one
 // column per lane of 128 or 512 and the separate factors throughout 46, 113, 141 and 255 us.
 template <class G, int CL>
 __global__ __launch_bounds__((64 * Split<G, CL>::WAVES)) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_summary(Plan pl) {
