@@ -7,6 +7,10 @@
 // A call that meets anything but the ordinary case (state not created yet, a
 // step counter that is no int) changes nothing and returns False; the class then
 // takes its Python path, which creates the state and calls the list functions.
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/record_function.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/autograd/profiler.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
@@ -864,9 +868,17 @@ bool recycle_experts(const std::vector<torch::Tensor>& experts, const std::vecto
     return true;
 }
 
+// Whether a profiler record around a call could be seen: by a running profiler, by callbacks that an observer has added
+// without one (execution traces, itt and nvtx ranges), or as an operator by a dispatch or function mode of this thread.
+bool calls_are_observed() {
+    return at::hasCallbacks() || torch::autograd::profiler::profilerEnabled() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+           at::impl::torch_function_mode_enabled();
+}
+
 }  // namespace
 
 void bind_group_steps(pybind11::module_& m) {
+    m.def("calls_are_observed", &calls_are_observed);
     m.def("grokfast_group_step", &grokfast_group_step);
     m.def("lion_group_step", &lion_group_step);
     m.def("grokadamw_group_step", &grokadamw_group_step);

@@ -8,13 +8,12 @@ of `_ops.grokadamw_fused_step` per parameter group.
 from typing import Iterable, Optional, Tuple
 
 import torch
-from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import check_hyper, gather, observed_step, run_closure
+from grokking_optimizers._common import FusedOptimizer, check_hyper, gather, run_closure
 
 
-class GrokAdamW(Optimizer):
+class GrokAdamW(FusedOptimizer):
     def __init__(self, params: Iterable, lr: float = 1e-3, betas: Tuple[float, float] = (0.9, 0.98), eps: float = 1e-8,
                  weight_decay: float = 1.0, alpha: float = 0.98, lamb: float = 5.0, gamma: float = 0.1, decay: float = 0.1,
                  grad_clip: float = 1.0) -> None:
@@ -24,7 +23,6 @@ class GrokAdamW(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay, alpha=alpha, lamb=lamb,
                                       gamma=gamma, decay=decay, grad_clip=grad_clip))
 
-    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         for group in self.param_groups:

@@ -10,14 +10,13 @@ reference's two-phase sequence (`_ops.grokfast_fused_step`, then AdamW).
 from typing import Iterable, Optional, Tuple
 
 import torch
-from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
 from grokking_optimizers._adamw_helper import adamw_step
-from grokking_optimizers._common import observed_step
+from grokking_optimizers._common import FusedOptimizer
 
 
-class Grokfast(Optimizer):
+class Grokfast(FusedOptimizer):
     def __init__(self, params: Iterable, lr: float = 1e-3, betas: Tuple[float, float] = (0.9, 0.98),
                  eps: float = 1e-8, weight_decay: float = 1.0, grokfast_alpha: float = 0.98,
                  grokfast_lamb: float = 2.0, fused: bool = True) -> None:
@@ -35,7 +34,6 @@ class Grokfast(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay,
                                       grokfast_alpha=grokfast_alpha, grokfast_lamb=grokfast_lamb))
 
-    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = None
         if closure is not None:

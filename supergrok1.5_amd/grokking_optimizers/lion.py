@@ -7,19 +7,17 @@ counter.  One call of `_ops.lion_fused_step` per parameter group.
 from typing import Iterable, Optional, Tuple
 
 import torch
-from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import check_hyper, observed_step, run_closure
+from grokking_optimizers._common import FusedOptimizer, check_hyper, run_closure
 
 
-class Lion(Optimizer):
+class Lion(FusedOptimizer):
     def __init__(self, params: Iterable, lr: float = 1e-4, betas: Tuple[float, float] = (0.9, 0.99),
                  weight_decay: float = 3.0) -> None:
         check_hyper(lr, None, betas)
         super().__init__(params, dict(lr=lr, betas=betas, weight_decay=weight_decay))
 
-    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         for group in self.param_groups:

@@ -11,14 +11,13 @@ and adds alpha*|g|*v to the gradient.  The four tensor passes run through
 from typing import Callable, Iterable, Optional, Tuple
 
 import torch
-from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
 from grokking_optimizers._adamw_helper import adamw_step
-from grokking_optimizers._common import check_hyper, gather, observed_step, run_closure
+from grokking_optimizers._common import FusedOptimizer, check_hyper, gather, run_closure
 
 
-class LookSAM(Optimizer):
+class LookSAM(FusedOptimizer):
     _BUFFERS = ("exp_avg", "exp_avg_sq", "sam_direction")
 
     def __init__(self, params: Iterable, lr: float = 1e-3, betas: Tuple[float, float] = (0.9, 0.98), eps: float = 1e-8,
@@ -31,7 +30,6 @@ class LookSAM(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay, rho=rho, k=k, alpha=alpha))
         self._global_step: int = 0
 
-    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         self._global_step += 1

@@ -5,14 +5,13 @@ for the rest.  Drop-in for the reference class (grokking_optimizers/muon.py):
 from typing import Iterable, Optional, Tuple
 
 import torch
-from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
 from grokking_optimizers._adamw_helper import adamw_step
-from grokking_optimizers._common import check_ranges, observed_step
+from grokking_optimizers._common import FusedOptimizer, check_ranges
 
 
-class Muon(Optimizer):
+class Muon(FusedOptimizer):
     """Args (as the reference, muon.py:45-56 there): params_2d, params_1d=None, lr=0.02,
     momentum=0.95, weight_decay=1.0, adamw_lr=1e-3, adamw_betas=(0.9, 0.98),
     adamw_eps=1e-8, ns_steps=5.  Group 0 holds the 2-D parameters (Muon),
@@ -33,7 +32,6 @@ class Muon(Optimizer):
         super().__init__(groups, dict(lr=lr, momentum=momentum, weight_decay=weight_decay, ns_steps=ns_steps,
                                       group_type="muon"))
 
-    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = None
         if closure is not None:

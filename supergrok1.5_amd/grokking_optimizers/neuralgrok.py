@@ -10,10 +10,9 @@ from typing import Iterable, List, Optional, Tuple
 
 import torch
 import torch.nn as nn
-from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import check_hyper, gather, observed_step, run_closure
+from grokking_optimizers._common import FusedOptimizer, check_hyper, gather, run_closure
 
 
 class _Amplifier(nn.Module):
@@ -36,7 +35,7 @@ class _Amplifier(nn.Module):
         return tuple(t.detach().float().contiguous() for t in (first.weight, first.bias, last.weight, last.bias))
 
 
-class NeuralGrok(Optimizer):
+class NeuralGrok(FusedOptimizer):
     def __init__(self, params: Iterable, lr: float = 1e-3, betas: Tuple[float, float] = (0.9, 0.98), eps: float = 1e-8,
                  weight_decay: float = 1.0, alpha: float = 10.0, beta: float = 4.0, num_layers: int = 3, hidden_dim: int = 128,
                  inner_steps: int = 1, grad_clip: float = 1.0) -> None:
@@ -58,7 +57,6 @@ class NeuralGrok(Optimizer):
             return tuple(w.to(dev) for w in weights)
         return _ops.amplifier_on(weights, self._device_weights, dev)
 
-    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
         if self._meta_weights_dirty or self._cached_meta_weights is None:

@@ -8,20 +8,18 @@ constructor arguments and defaults, state `step`, `exp_avg`, `exp_avg_sq`, `s`
 from typing import Iterable, Optional, Tuple
 
 import torch
-from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import check_hyper, gather, observed_step, run_closure
+from grokking_optimizers._common import FusedOptimizer, check_hyper, gather, run_closure
 
 
-class Prodigy(Optimizer):
+class Prodigy(FusedOptimizer):
     def __init__(self, params: Iterable, lr: float = 1.0, betas: Tuple[float, float] = (0.9, 0.999), eps: float = 1e-8,
                  weight_decay: float = 1.0) -> None:
         check_hyper(lr, eps, betas)
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay))
         self._d_lr: float = 1e-6
 
-    @observed_step
     def step(self, closure=None) -> Optional[float]:
         loss = run_closure(closure)
 

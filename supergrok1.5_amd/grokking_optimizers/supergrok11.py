@@ -14,16 +14,15 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import observed_step
+from grokking_optimizers._common import FusedOptimizer
 from grokking_optimizers._meta_training import MetaTraining
 from grokking_optimizers._schedule import GrokSchedule
 from grokking_optimizers.supergrok15 import SharpnessMetaNet
 
 
-class SuperGrok11(MetaTraining, Optimizer):
+class SuperGrok11(MetaTraining, FusedOptimizer):
     def __init__(self, params, lr: float = 1e-3, betas: tuple = (0.9, 0.999), eps: float = 1e-8, weight_decay: float = 1.0,
                  alpha_init: float = 0.98, lamb: float = 5.0, gamma: float = 0.1, gamma_alpha: float = 0.0, kappa: float = 0.1,
                  warmup_steps: int = 100, warmup_ramp: int = 100, gradient_clipping: float = 1.0,
@@ -73,7 +72,6 @@ class SuperGrok11(MetaTraining, Optimizer):
         """999999 (off) below sam_enable_threshold, else 1: the training loop decides the actual frequency."""
         return 999999 if self._cached_train_acc < self.sam_enable_threshold else 1
 
-    @observed_step
     def step(self, closure=None, train_loss=None, val_loss=None, train_acc=None):
         loss = None
         if closure is not None:

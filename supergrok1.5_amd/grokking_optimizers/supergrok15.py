@@ -12,10 +12,9 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import observed_step
+from grokking_optimizers._common import FusedOptimizer
 from grokking_optimizers._meta_training import MetaTraining, ScheduledTraining
 from grokking_optimizers._schedule import GrokSchedule
 
@@ -46,7 +45,7 @@ class SharpnessMetaNet(nn.Module):
                 self.rescale.data.item())
 
 
-class SuperGrok15(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
+class SuperGrok15(GrokSchedule, MetaTraining, ScheduledTraining, FusedOptimizer):
     def __init__(self, params, lr: float = 1e-3, betas: tuple = (0.9, 0.999), eps: float = 1e-8,
                  weight_decay: float = 1.0, alpha_init: float = 0.98, lamb: float = 2.0, gamma: float = 0.1,
                  gamma_alpha: float = 0.0, kappa: float = 0.1, warmup_steps: int = 100, warmup_ramp: int = 100,
@@ -57,7 +56,7 @@ class SuperGrok15(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
                  bilevel_freq_max: int = 30, bilevel_scale: float = 20.0, bilevel_thresh: float = 0.9,
                  wd_ramp: float = 4.0, wd_scale: float = 20.0, wd_thresh: float = 0.9,
                  sam_enable_threshold: float = 0.0):
-        Optimizer.__init__(self, params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay))
+        FusedOptimizer.__init__(self, params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay))
         # None: whatever `_ops.supergrok15_set_gelu_mode` last selected for the process ("erf" unless changed); "erf" / "sigmoid":
         # this instance's own form (the reference's CPU path / its GPU kernel), whatever other instances use
         self.gelu_mode = None
@@ -100,7 +99,6 @@ class SuperGrok15(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
             self._flat_sharpness.append(mk())
         self._state_initialized = True
 
-    @observed_step
     def step(self, closure=None, train_loss=None, val_loss=None, train_acc=None):
         loss = None
         if closure is not None:

@@ -29,16 +29,15 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-from torch.optim import Optimizer
 
 from grokking_optimizers import _ops
-from grokking_optimizers._common import observed_step
+from grokking_optimizers._common import FusedOptimizer
 from grokking_optimizers._meta_training import MetaTraining, ScheduledTraining
 from grokking_optimizers._schedule import GrokSchedule
 from grokking_optimizers.mamba3_peer_metanet import Mamba3PEERMetaNet
 
 
-class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
+class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, FusedOptimizer):
     def __init__(self, params, lr: float = 1e-3, betas: tuple = (0.9, 0.999), eps: float = 1e-8,
                  weight_decay: float = 1.0, alpha_init: float = 0.98, lamb: float = 2.0, gamma: float = 0.1,
                  gamma_alpha: float = 0.0, kappa: float = 0.1, warmup_steps: int = 100, warmup_ramp: int = 100,
@@ -51,7 +50,7 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
                  sam_thresh: float = 0.85, bilevel_freq_min: int = 5, bilevel_freq_max: int = 30,
                  bilevel_scale: float = 20.0, bilevel_thresh: float = 0.9, wd_ramp: float = 4.0, wd_scale: float = 20.0,
                  wd_thresh: float = 0.9, sam_enable_threshold: float = 0.0, bilevel_checkpoint_interval: int = 1):
-        Optimizer.__init__(self, params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay))
+        FusedOptimizer.__init__(self, params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay))
         for k, v in dict(alpha_init=alpha_init, sam_enable_threshold=sam_enable_threshold, lamb=lamb, gamma=gamma,
                          gamma_alpha=gamma_alpha, kappa=kappa, warmup_steps=warmup_steps,
                          warmup_ramp=max(1, warmup_ramp), gradient_clipping=gradient_clipping,
@@ -109,7 +108,6 @@ class SuperGrok2(GrokSchedule, MetaTraining, ScheduledTraining, Optimizer):
         three launches for all tensors, norms reduced on the device, no host syncs."""
         return _ops.supergrok2_clip_grads([g.contiguous() for g in grads], float(self.gradient_clipping))
 
-    @observed_step
     def step(self, closure=None, train_loss=None, val_loss=None, train_acc=None):
         loss = None
         if closure is not None:
