@@ -423,6 +423,11 @@ int sg2_chunk_len_for(int num_tensors, const int64_t* numels) {
     if (num_tensors < 0 || (num_tensors > 0 && !numels)) return 0;
     return sg2::effective_chunk_len(num_tensors, sg2::Numels{numels, nullptr});
 }
+int sg2_clipped_chunk_len_for(const SgDims* dims, int num_tensors, const int64_t* numels) {
+    const int geo = sg2::geo_of(dims);
+    if (geo < 0 || num_tensors < 0 || (num_tensors > 0 && !numels)) return 0;
+    return sg2::fitted_chunk_len(geo, num_tensors, sg2::Numels{numels, nullptr});
+}
 
 int sg2_set_scan_window(int window) {
     if (window < 0) window = SG2_DEFAULT_SCAN_WINDOW;

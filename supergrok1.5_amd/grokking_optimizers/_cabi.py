@@ -51,7 +51,7 @@ class Sg2Debug(C.Structure):
     _fields_ = [("perm", C.c_void_p), ("expert_idx", C.c_void_p), ("ctx", C.c_void_p)]
 
 
-EXPORTS = ("sg_last_error", "sg2_set_chunk_len", "sg2_get_chunk_len", "sg2_set_scan_window", "sg2_get_scan_window", "sg2_chunk_len_for", "sg2_workspace_bytes", "sg2_batched_step",
+EXPORTS = ("sg_last_error", "sg2_set_chunk_len", "sg2_get_chunk_len", "sg2_set_scan_window", "sg2_get_scan_window", "sg2_chunk_len_for", "sg2_clipped_chunk_len_for", "sg2_workspace_bytes", "sg2_batched_step",
            "sg2_profile_enable", "sg2_profile_read")
 SG2_PROF_STAGES = ("sort", "scan_summary", "chunk_prefix", "scan_output", "elementwise")
 
@@ -130,9 +130,19 @@ def make_dims(dims=None):
 
 
 def chunk_len_for(numels):
-    """Scan chunk length a call with these tensor sizes uses (the configured one, or the automatic choice)."""
+    """Scan chunk length a call of sg2_batched_step with these tensor sizes uses (the configured one, or the automatic choice)."""
     arr = (C.c_int64 * len(numels))(*numels)
     return lib().sg2_chunk_len_for(len(numels), arr)
+
+
+def clipped_chunk_len_for(numels, dims=None):
+    """The same for sg2_clipped_step, which SuperGrok2.step calls."""
+    arr = (C.c_int64 * len(numels))(*numels)
+    d = make_dims(dims)
+    n = lib().sg2_clipped_chunk_len_for(C.byref(d), len(numels), arr)
+    if n == 0:
+        raise RuntimeError(last_error())
+    return n
 
 
 def workspace_bytes(numels, dims=None, options=None):

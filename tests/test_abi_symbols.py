@@ -4,6 +4,8 @@ import ctypes
 import os
 import re
 
+import pytest
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
@@ -29,6 +31,7 @@ def test_library_exports_every_declared_symbol():
 
 def test_host_side_validation_without_gpu():
     from grokking_optimizers import _cabi
+    from workloads import DEFAULT_DIMS
     assert _cabi.workspace_bytes([0, 0]) >= 0
     n = _cabi.workspace_bytes([1000, 5000])
     assert n > 8 * 6000 * 4
@@ -37,6 +40,15 @@ def test_host_side_validation_without_gpu():
     assert lib.sg2_set_chunk_len(256) == 0 and lib.sg2_get_chunk_len() == 256
     assert lib.sg2_set_chunk_len(0) == 0 and lib.sg2_get_chunk_len() == 0
     assert _cabi.chunk_len_for([1000, 5000]) == 512 and _cabi.chunk_len_for([4 << 20] * 8) == 4096 and _cabi.chunk_len_for([1 << 20] * 3) == 1024
+    # the clipped step's own choice; a pinned length serves both
+    large = dict(DEFAULT_DIMS, d_model=16, d_state=32, d_inner=32)
+    assert _cabi.clipped_chunk_len_for([5000, 300]) == 256 and _cabi.clipped_chunk_len_for([512] * 9) == 512
+    assert _cabi.clipped_chunk_len_for([4 << 20] * 8) == 4096 and _cabi.clipped_chunk_len_for([1 << 20] * 3) == 1024
+    assert _cabi.clipped_chunk_len_for([131072], large) == 512 and _cabi.clipped_chunk_len_for([131073], large) == 640
+    for d in (None, large):
+        assert lib.sg2_set_chunk_len(320) == 0 and _cabi.clipped_chunk_len_for([5000, 300], d) == 320 and lib.sg2_set_chunk_len(0) == 0
+    with pytest.raises(RuntimeError, match="MAX_D_MODEL"):
+        _cabi.clipped_chunk_len_for([5000], dict(DEFAULT_DIMS, d_model=18))
     assert lib.sg2_set_scan_window(100) != 0 and lib.sg2_set_scan_window(128) == 0 and lib.sg2_get_scan_window() == 128
     assert lib.sg2_set_scan_window(-1) == 0 and lib.sg2_get_scan_window() == 64
 

@@ -40,7 +40,7 @@ def test_config3_v2_fifty_steps_with_recycling_on_the_14_tensor_set():
         ref.append(dict(param=p.numpy().reshape(-1).copy(), exp_avg=np.zeros(n, np.float32), exp_avg_sq=np.zeros(n, np.float32),
                         mu=np.zeros(n, np.float32), gru=np.zeros((n, 4), np.float32), mamba_fwd=np.zeros((16, 16), np.float32),
                         mamba_bwd=np.zeros((16, 16), np.float32)))
-    chunk_len = _cabi.chunk_len_for([wl.numel(s) for s in shapes])
+    chunk_len = _cabi.clipped_chunk_len_for([wl.numel(s) for s in shapes])
     window = _cabi.lib().sg2_get_scan_window()
     sig = lambda s, v, th: 1.0 / (1.0 + math.exp(-s * (v - th)))
     counts = np.zeros(144, np.int32)

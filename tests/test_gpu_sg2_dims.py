@@ -81,7 +81,7 @@ def test_class_steps_at_these_dims(kw):
         ref.append(dict(param=p.numpy().reshape(-1).copy(), exp_avg=np.zeros(n, np.float32), exp_avg_sq=np.zeros(n, np.float32),
                         mu=np.zeros(n, np.float32), gru=np.zeros((n, dims["gru_hidden"]), np.float32),
                         mamba_fwd=np.zeros((DI, DS), np.float32), mamba_bwd=np.zeros((DI, DS), np.float32)))
-    chunk_len = _cabi.chunk_len_for([wl.numel(s) for s in shapes])
+    chunk_len = _cabi.clipped_chunk_len_for([wl.numel(s) for s in shapes], dims)
     window = _cabi.lib().sg2_get_scan_window()
     f32 = lambda v: float(np.float32(v))
     sig = lambda s, v, th: 1.0 / (1.0 + math.exp(-s * (v - th)))

@@ -90,7 +90,7 @@ def test_optimizer_class_with_large_meta_net():
     ref = [dict(param=p.numpy().reshape(-1).copy(), exp_avg=np.zeros(p.numel(), np.float32), exp_avg_sq=np.zeros(p.numel(), np.float32),
                 mu=np.zeros(p.numel(), np.float32), gru=np.zeros((p.numel(), 4), np.float32), mamba_fwd=np.zeros((32, 32), np.float32),
                 mamba_bwd=np.zeros((32, 32), np.float32)) for p in p0]
-    chunk_len = _cabi.chunk_len_for([wl.numel(s) for s in shapes])
+    chunk_len = _cabi.clipped_chunk_len_for([wl.numel(s) for s in shapes], LARGE)
     window = _cabi.lib().sg2_get_scan_window()
     W = [w.detach().cpu().numpy() for w in mn.flat_weights()]
     for t in range(1, 4):
