@@ -100,10 +100,10 @@ const char* sg_last_error(void);
  * sg2_batched_step takes 4096, 2048, 1024 or 512 by the amount of work;
  * sg2_chunk_len_for tells what a call with these tensor sizes will use.
  * sg2_clipped_step, which sg2_clipped_chunk_len_for answers for (0 where the
- * dimensions are refused), takes the same and 256 in small calls while the
- * scan block fits (8, 16, 16); for larger blocks a multiple of 128 from 512 to
- * 4096 whose chunks fill the chip in whole rounds.  Affects results only by
- * re-association of the chunk products. */
+ * dimensions are refused), takes the same and 256 in small calls of tensors up
+ * to 8192 elements while the scan block fits (8, 16, 16); for larger blocks a
+ * multiple of 128 from 512 to 4096 whose chunks fill the chip in whole rounds.
+ * Affects results only by re-association of the chunk products. */
 int sg2_set_chunk_len(int chunk_len);
 int sg2_get_chunk_len(void);
 int sg2_chunk_len_for(int num_tensors, const int64_t* numels);

@@ -59,16 +59,22 @@ int effective_chunk_len(int P, Numels numels) {
 
 // The chunk length of sg2_clipped_step.
 // Default geometry: 256 for small calls, while the chip has a SIMD for each of their waves (one column per lane, so two a
-// chunk): the replay is then half as long, and so is what the summaries of the module's weights need (184 to 240 steps) less
-// than a chunk (30 000 elements 127 -> 102 us a step, 600 in one tensor 86 -> 72; with every pole slowed by e, whose summaries
-// need more, 125 -> 140, by e^2 171 -> 141).  Otherwise by the amount of work, as in sg2_batched_step: a tensor's last
+// chunk): the replay is then half as long.  So are the summaries, while the poles contract within a chunk; where they need
+// more (the module's weights 184 to 240 steps, weights in training more or less) every start state comes from the one
+// before it in k_chunk_prefix, a chain as long as the widest tensor has chunks.  Hence only tensors of at most 32 chunks,
+// which that kernel takes in one batch.  A step with 256 and 512, every pole slowed by e^0 / e^1.2 / e^2: one tensor of
+// 2000 elements 66 : 83 / 81 : 89 / 81 : 120 us, of 8192 81 : 97 / 98 : 100 / 98 : 135, seven of 8192 90 : 102 / 107 : 106 / 108 : 140;
+// beyond, one of 16 384 87 : 104 / 110 : 104 / 110 : 142, and 60 000 in four by e^0 / e / e^2 109 : 128 / 158 : 116 / 157 : 171.
+// Otherwise by the amount of work, as in sg2_batched_step: a tensor's last
 // chunks, its largest gradients, take slower forms, and short chunks spread them (chunks that fill the chip in whole rounds
 // as below: 3.1 M bf16 elements 930 -> 998 us, 0.42 M and 1.2 M the same).
 // Large geometry: 512 while the chip holds all chunks of 512 at once (`SLOTS` workgroups).  Beyond that the chunks run in
 // rounds, and a round takes as long as a chunk whether it is full or not; so does its share of the summaries, which walk
 // `TAIL` steps whatever the chunk's length (what the module's weights need, at the summary's cost per step).  Of the lengths
 // that just fill 1, 2, 3 ... rounds, a multiple of 128 up to 4096, the one with the least of both is taken: 0.42 M elements
-// 731 -> 573 us (1792 for 512), 3 M 3.45 -> 3.10 ms (3968 for 1024).
+// 731 -> 573 us (1792 for 512), 3 M 3.45 -> 3.10 ms (3968 for 1024).  With every pole slowed by e^0.5, e and e^2 the same
+// choices stand: 0.42 M 537, 532, 468 us (512: 590, 537, 808), 1.2 M 1.24, 1.14, 1.12 ms (1024: 1.19, 1.13, 1.25), 3 M 2.66,
+// 2.51, 2.43 ms (1024: 2.63, 2.50, 2.81).
 int fitted_chunk_len(int geo, int P, Numels numels) {
     const int set = g_chunk_len.load();
     if (set > 0) return set;
@@ -82,7 +88,8 @@ int fitted_chunk_len(int geo, int P, Numels numels) {
     if (geo == GEO_DEFAULT) {
         int64_t widest = 0;
         for (int i = 0; i < P; i++) widest = std::max(widest, numels[i]);
-        return widest > SHORTEST && 2 * chunks(SHORTEST / 2) <= 1024 ? SHORTEST / 2 : auto_chunk_len(P, numels);
+        const bool small = widest > SHORTEST && widest <= 32 * (SHORTEST / 2) && 2 * chunks(SHORTEST / 2) <= 1024;
+        return small ? SHORTEST / 2 : auto_chunk_len(P, numels);
     }
     if (chunks(SHORTEST) <= SLOTS) return SHORTEST;
     int64_t total = 0;

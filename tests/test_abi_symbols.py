@@ -42,7 +42,9 @@ def test_host_side_validation_without_gpu():
     assert _cabi.chunk_len_for([1000, 5000]) == 512 and _cabi.chunk_len_for([4 << 20] * 8) == 4096 and _cabi.chunk_len_for([1 << 20] * 3) == 1024
     # the clipped step's own choice; a pinned length serves both
     large = dict(DEFAULT_DIMS, d_model=16, d_state=32, d_inner=32)
-    assert _cabi.clipped_chunk_len_for([5000, 300]) == 256 and _cabi.clipped_chunk_len_for([512] * 9) == 512
+    # (256 only where a tensor's start states come in one batch, should the poles not contract within a chunk)
+    for sizes, expected in (([512] * 9, 512), ([513], 256), ([5000, 300], 256), ([8192] * 8, 256), ([8193], 512), ([8192] * 9, 512), ([2000] * 30, 256)):
+        assert _cabi.clipped_chunk_len_for(sizes) == expected, sizes
     assert _cabi.clipped_chunk_len_for([4 << 20] * 8) == 4096 and _cabi.clipped_chunk_len_for([1 << 20] * 3) == 1024
     assert _cabi.clipped_chunk_len_for([131072], large) == 512 and _cabi.clipped_chunk_len_for([131073], large) == 640
     for d in (None, large):

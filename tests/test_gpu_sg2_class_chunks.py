@@ -17,7 +17,7 @@ LARGE = dict(wl.DEFAULT_DIMS, d_model=16, d_state=32, d_inner=32)
 STATE = dict(exp_avg="_flat_exp_avgs", exp_avg_sq="_flat_exp_avg_sqs", mu="_flat_mus", gru="_flat_gru_states",
              mamba_fwd="_flat_mamba_fwd_states", mamba_bwd="_flat_mamba_bwd_states")
 # dimensions, tensor sizes, the length that the class takes there
-CALLS = {"small": (None, [3000, 700, 513, 40], 256), "as the batched step": (None, [70001, 512, 5], 512),
+CALLS = {"small": (None, [3000, 700, 513, 40], 256), "largest small": (None, [8192, 8191, 257], 256), "just beyond": (None, [8193, 700], 512), "as the batched step": (None, [70001, 512, 5], 512),
          "large, all at once": (LARGE, [20000, 9000, 513, 77], 512), "large, just beyond": (LARGE, [131073, 300], 640),
          "large, transformer": (LARGE, [wl.numel(s) for s in wl.shared14_shapes()], 1792),
          "large, one long round": (LARGE, [63400] * 15 + [63488], 3968)}
