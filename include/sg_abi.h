@@ -109,6 +109,18 @@ int sg2_get_chunk_len(void);
 int sg2_chunk_len_for(int num_tensors, const int64_t* numels);
 int sg2_clipped_chunk_len_for(const SgDims* dims, int num_tensors, const int64_t* numels);
 
+/* The form of the sort that a call with these tensor sizes takes (all_16bit:
+ * every gradient is float16 or bfloat16), -1 for sizes it refuses.  The order
+ * is the same in all of them. */
+enum {
+    SG2_SORT_TENSORS = 0,        /* one workgroup per tensor, all passes in LDS */
+    SG2_SORT_RUNS = 1,           /* runs of 4096 keys in LDS, then merged */
+    SG2_SORT_SMALL_PASSES = 2,   /* radix passes over tiles of 2048 keys */
+    SG2_SORT_PASSES = 3,         /* ... of 8192 */
+    SG2_SORT_SCANNED_PASSES = 4  /* ... with the digit counts scanned by kernels of their own */
+};
+int sg2_sort_form_for(int num_tensors, const int64_t* numels, int all_16bit);
+
 /* Summary window of the scan (timesteps, a multiple of 64; 0 disables, a
  * negative value restores the default, SG2_DEFAULT_SCAN_WINDOW).  The recurrence contracts, so a
  * chunk summary is built backwards in blocks of `window` steps and the walk

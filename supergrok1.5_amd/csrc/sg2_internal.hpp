@@ -163,6 +163,7 @@ __device__ __forceinline__ float sharp_of(const TensorDev& T, int64_t i) { retur
 
 int launch_norm(const Plan& pl, hipStream_t st);
 int launch_sort(const Plan& pl, int32_t* dbg_perm, hipStream_t st);
+int sort_form(int sort_tile, int sort_tiles, int sort_widest, bool half);      // SG2_SORT_*
 int launch_scan(const Plan& pl, hipStream_t st);
 // bilevel path: the forward scan keeps the state entering every HT_STEP-th step of a tensor; index of scan step u
 // (a multiple of HT_STEP) of tensor ti (element offset off) in that array, and the array's length

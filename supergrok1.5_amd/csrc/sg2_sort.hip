@@ -740,34 +740,40 @@ int launch_passes(const Plan& pl, hipStream_t st) {
     return 0;
 }
 
+template <class G, bool HALF>
+int launch_sort_geo(const Plan& pl, hipStream_t st) {
+    switch (sort_form(pl.sort_tile, pl.sort_tiles, pl.sort_widest, HALF)) {
+        case SG2_SORT_RUNS:
+            hipLaunchKernelGGL((k_sort_runs<G, HALF>), dim3(1 + pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl);
+            SG_LAUNCH_CHECK("k_sort_runs");
+            hipLaunchKernelGGL(k_merge_runs<HALF>, dim3(pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl);
+            SG_LAUNCH_CHECK("k_merge_runs");
+            return 0;
+        case SG2_SORT_TENSORS:
+            hipLaunchKernelGGL(k_sort_tile<G>, dim3(1 + pl.P), dim3(SORT_THREADS), 0, st, pl);
+            SG_LAUNCH_CHECK("k_sort_tile");
+            return 0;
+        case SG2_SORT_SMALL_PASSES: return launch_passes<G, SORT_TILE_SMALL, true, HALF>(pl, st);
+        case SG2_SORT_PASSES: return launch_passes<G, SORT_TILE, true, HALF>(pl, st);
+        default: return launch_passes<G, SORT_TILE, false, HALF>(pl, st);
+    }
+}
+
+}  // namespace
+
 // Tiles of the largest tensor up to which runs are merged.  The merge's work grows with the square of a tensor's length and the
 // passes' with the length; 16-bit gradients have two passes only.  What runs change against passes over small tiles: four
 // fp32 tensors of 20 000 -17 us, one of 60 000 -9, of 80 000 0, of 130 000 +7, sixteen of 60 000 -12, thirty +3 (hence the
 // product); bfloat16, one of 8000 -9, four of 20 000 +3, one of 60 000 +24.
 constexpr int MERGE_TILES = 40, MERGE_WORK = 20000, HALF_MERGE_TILES = 4;
-inline bool merges(const Plan& pl, bool half) {
-    return pl.sort_widest <= (half ? HALF_MERGE_TILES : MERGE_TILES) && (int64_t)pl.sort_tiles * pl.sort_widest <= MERGE_WORK;
-}
-template <class G, bool HALF>
-int launch_sort_geo(const Plan& pl, hipStream_t st) {
-    if (pl.sort_tile == SORT_TILE_SMALL) {
-        if (!merges(pl, HALF)) return launch_passes<G, SORT_TILE_SMALL, true, HALF>(pl, st);
-        hipLaunchKernelGGL((k_sort_runs<G, HALF>), dim3(1 + pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl);
-        SG_LAUNCH_CHECK("k_sort_runs");
-        hipLaunchKernelGGL(k_merge_runs<HALF>, dim3(pl.sort_tiles), dim3(SORT_THREADS), 0, st, pl);
-        SG_LAUNCH_CHECK("k_merge_runs");
-        return 0;
+int sort_form(int sort_tile, int sort_tiles, int sort_widest, bool half) {
+    if (sort_tile == SORT_TILE_SMALL) {
+        const bool merges = sort_widest <= (half ? HALF_MERGE_TILES : MERGE_TILES) && (int64_t)sort_tiles * sort_widest <= MERGE_WORK;
+        return merges ? SG2_SORT_RUNS : SG2_SORT_SMALL_PASSES;
     }
-    if (pl.sort_widest <= 1) {
-        hipLaunchKernelGGL(k_sort_tile<G>, dim3(1 + pl.P), dim3(SORT_THREADS), 0, st, pl);
-        SG_LAUNCH_CHECK("k_sort_tile");
-        return 0;
-    }
-    if (pl.sort_widest <= SELF_SCAN_TILES) return launch_passes<G, SORT_TILE, true, HALF>(pl, st);
-    return launch_passes<G, SORT_TILE, false, HALF>(pl, st);
+    if (sort_widest <= 1) return SG2_SORT_TENSORS;
+    return sort_widest <= SELF_SCAN_TILES ? SG2_SORT_PASSES : SG2_SORT_SCANNED_PASSES;
 }
-
-}  // namespace
 
 int launch_sort(const Plan& pl, int32_t* dbg_perm, hipStream_t st) {
     if (pl.total == 0) return 0;

@@ -435,6 +435,12 @@ int sg2_clipped_chunk_len_for(const SgDims* dims, int num_tensors, const int64_t
     if (geo < 0 || num_tensors < 0 || (num_tensors > 0 && !numels)) return 0;
     return sg2::fitted_chunk_len(geo, num_tensors, sg2::Numels{numels, nullptr});
 }
+int sg2_sort_form_for(int num_tensors, const int64_t* numels, int all_16bit) {
+    if (num_tensors < 0 || (num_tensors > 0 && !numels)) return -1;
+    sg2::Layout L;
+    if (sg2::make_layout(sg2::GEO_DEFAULT, num_tensors, sg2::Numels{numels, nullptr}, 512, &L)) return -1;
+    return sg2::sort_form(L.sort_tile, L.sort_tiles, L.sort_widest, all_16bit != 0);
+}
 
 int sg2_set_scan_window(int window) {
     if (window < 0) window = SG2_DEFAULT_SCAN_WINDOW;

@@ -51,7 +51,7 @@ class Sg2Debug(C.Structure):
     _fields_ = [("perm", C.c_void_p), ("expert_idx", C.c_void_p), ("ctx", C.c_void_p)]
 
 
-EXPORTS = ("sg_last_error", "sg2_set_chunk_len", "sg2_get_chunk_len", "sg2_set_scan_window", "sg2_get_scan_window", "sg2_chunk_len_for", "sg2_clipped_chunk_len_for", "sg2_workspace_bytes", "sg2_batched_step",
+EXPORTS = ("sg_last_error", "sg2_set_chunk_len", "sg2_get_chunk_len", "sg2_set_scan_window", "sg2_get_scan_window", "sg2_chunk_len_for", "sg2_clipped_chunk_len_for", "sg2_sort_form_for", "sg2_workspace_bytes", "sg2_batched_step",
            "sg2_profile_enable", "sg2_profile_read")
 SG2_PROF_STAGES = ("sort", "scan_summary", "chunk_prefix", "scan_output", "elementwise")
 
@@ -143,6 +143,18 @@ def clipped_chunk_len_for(numels, dims=None):
     if n == 0:
         raise RuntimeError(last_error())
     return n
+
+
+SORT_FORMS = ("tensors", "runs", "small passes", "passes", "scanned passes")
+
+
+def sort_form_for(numels, all_16bit=False):
+    """The form of the sort (one of SORT_FORMS) that a call with these tensor sizes takes."""
+    arr = (C.c_int64 * len(numels))(*numels)
+    n = lib().sg2_sort_form_for(len(numels), arr, 1 if all_16bit else 0)
+    if n < 0:
+        raise RuntimeError(last_error())
+    return SORT_FORMS[n]
 
 
 def workspace_bytes(numels, dims=None, options=None):

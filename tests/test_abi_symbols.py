@@ -51,6 +51,8 @@ def test_host_side_validation_without_gpu():
         assert lib.sg2_set_chunk_len(320) == 0 and _cabi.clipped_chunk_len_for([5000, 300], d) == 320 and lib.sg2_set_chunk_len(0) == 0
     with pytest.raises(RuntimeError, match="MAX_D_MODEL"):
         _cabi.clipped_chunk_len_for([5000], dict(DEFAULT_DIMS, d_model=18))
+    with pytest.raises(RuntimeError, match="negative numel"):
+        _cabi.sort_form_for([-1])
     assert lib.sg2_set_scan_window(100) != 0 and lib.sg2_set_scan_window(128) == 0 and lib.sg2_get_scan_window() == 128
     assert lib.sg2_set_scan_window(-1) == 0 and lib.sg2_get_scan_window() == 64
 

@@ -1,5 +1,6 @@
 """The v2 step at the edges of its sort and clip dispatch: tensor sizes on both sides of what one LDS sort holds, of the
-small sort tile (by the widest tensor and by the total) and of what a scatter workgroup adds up itself; and the clipping step of the class (factor applied as
+small sort tile (by the widest tensor and by the total), of what is merged from runs, and of what a scatter workgroup adds up itself - each
+in the form of the sort that it is there for, as the library reports it; and the clipping step of the class (factor applied as
 the gradients are read, fp32 sharpness beside 16-bit gradients) against clipped copies through the list functions."""
 import pytest
 import torch
@@ -9,15 +10,25 @@ from sg2_harness import Sg2Case, per_tensor_scalars, shared_scalars
 
 pytestmark = pytest.mark.gpu
 
-SIZES = {"one tile each": [8192, 1, 512, 513, 2048], "one above": [8193, 2047, 2049], "most small tiles": [65536, 70],
-         "one above that": [65537, 3], "most tiles of a self scan": [262144, 9], "one above that too": [262145, 8191],
-         "one below a large tile per CU": [65536] * 31 + [65535], "a large tile per CU": [65536] * 32}
+# name: (tensor sizes, form of the sort)
+SIZES = {"a workgroup each": ([2048, 1, 512, 513, 2047, 65], "tensors"), "one above": ([2049, 2048, 1, 512], "runs"),
+         "a large tile at most": ([8192, 1, 512, 513, 2048], "runs"), "one above a large tile": ([8193, 2047, 2049], "runs"),
+         "most merged by work": ([65536] * 19 + [17 * 2048], "runs"), "one above the work": ([65536] * 19 + [17 * 2048, 1], "small passes"),
+         "32 small tiles": ([65536, 70], "runs"), "one above 32": ([65537, 3], "runs"),
+         "128 small tiles": ([262144, 9], "small passes"), "one above 128": ([262145, 8191], "small passes"),
+         "one below a large tile for every fourth CU": ([262144, 262143], "small passes"), "a large tile for every fourth CU": ([262144, 262144], "passes"),
+         "narrow beyond that": ([65536] * 9, "runs"), "not narrow": ([65537] + [65536] * 8, "passes"),
+         "most tiles of a self scan": ([262144, 9, 262144], "passes"), "one above that": ([262145, 262144, 8191], "scanned passes"),
+         "one below a large tile per CU": ([65536] * 31 + [65535], "small passes"), "a large tile per CU": ([65536] * 32, "passes"),
+         "a large tile each": ([8192, 8191, 2049, 4097, 513] + [8192] * 255, "tensors")}
 
 
 @pytest.mark.parametrize("sizes", list(SIZES), ids=lambda s: s.replace(" ", "_"))
 @pytest.mark.parametrize("sharpness", [False, True])
 def test_sort_paths(sizes, sharpness):
-    shapes = [(n,) for n in SIZES[sizes]]
+    from grokking_optimizers import _cabi
+    assert _cabi.sort_form_for(SIZES[sizes][0]) == SIZES[sizes][1]
+    shapes = [(n,) for n in SIZES[sizes][0]]
     case = Sg2Case(shapes, seed=3, random_state=True)
     grads = wl.make_grads(shapes, seed=4, tail_frac=0.01)
     grads[0][::7] = 0.0                                   # runs of equal keys

@@ -1,5 +1,5 @@
 """The two-pass sort of calls whose gradients are all 16-bit: the permutation against a stable argsort of the magnitudes, over
-every form of the sort (one tile per tensor, small tiles, large tiles with and without scan kernels) and the whole range of
+every form of the sort (a workgroup per tensor, merged runs, small tiles, large tiles with and without scan kernels) and the whole range of
 the types (subnormals, zeros of either sign, the largest values, non-finite entries, ties)."""
 import numpy as np
 import pytest
@@ -10,8 +10,14 @@ from sg2_harness import Sg2Case, per_tensor_scalars, shared_scalars
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = {"tile": [(1,), (511,), (513,), (2049,), (8192,)], "small": [(8193,), (2048,), (4097,), (5,)],
-          "large": [(70001,), (2200000 // 16,), (250000,), (1900000 // 8,)] * 4, "scan": [(300001,), (8191,), (16384,)]}
+# name: (shapes, form of the sort where all gradients are 16-bit, form where some are fp32)
+SHAPES = {"tensors": ([(1,), (511,), (513,), (2048,), (2047,)], "tensors", "tensors"),
+          "large_tensors": ([(8192,), (8191,), (4097,), (2049,), (513,)] + [(8192,)] * 255, "tensors", "tensors"),
+          "runs": ([(1,), (511,), (513,), (2049,), (8192,)], "runs", "runs"),
+          "small": ([(8193,), (2048,), (4097,), (5,)], "small passes", "runs"),
+          "small_wide": ([(300001,), (8191,), (16384,)], "small passes", "small passes"),
+          "large": ([(70001,), (2200000 // 16,), (250000,), (1900000 // 8,)] * 4, "passes", "passes"),
+          "scan": ([(300001,), (8191,), (250000,)], "scanned passes", "scanned passes")}
 
 
 def _values(n, dtype, seed):
@@ -29,7 +35,9 @@ def _values(n, dtype, seed):
 @pytest.mark.parametrize("form", sorted(SHAPES))
 @pytest.mark.parametrize("types", ["bf16", "fp16", "both", "with_fp32"])
 def test_permutation(form, types):
-    shapes = SHAPES[form]
+    from grokking_optimizers import _cabi
+    shapes, of_16bit, of_mixed = SHAPES[form]
+    assert _cabi.sort_form_for([wl.numel(s) for s in shapes], types != "with_fp32") == (of_mixed if types == "with_fp32" else of_16bit)
     of = {"bf16": [torch.bfloat16], "fp16": [torch.float16], "both": [torch.float16, torch.bfloat16],
           "with_fp32": [torch.bfloat16, torch.float32, torch.float16]}[types]
     dtypes = [of[i % len(of)] for i in range(len(shapes))]

@@ -9,8 +9,11 @@ from sg2_harness import Sg2Case, per_tensor_scalars, shared_scalars
 
 pytestmark = pytest.mark.gpu
 
+# (both sides of the limits on the work are in test_gpu_sg2_paths.py)
 SHAPES = {"one run": [(2049,), (1,), (4095,), (4096,), (2048,)], "two": [(4097,), (6145,), (8192,), (3,)], "more": [(8193,), (12288,), (12289,), (40000,)],
           "most": [(81920,), (5,), (65537,)], "passes": [(81921,), (2500,)], "beyond": [(300000,), (230000,), (2049,)]}
+FORMS = {"passes": "small passes", "beyond": "scanned passes"}       # the others are merged
+WIDE = ("more", "most", "passes")                                    # ... as fp32 only: 16-bit tensors above 8192 elements are not
 VALUES = ["random", "ties", "equal", "ascending", "descending", "not finite"]
 
 
@@ -33,6 +36,10 @@ def _values(kind, n, r):
 @pytest.mark.parametrize("form", sorted(SHAPES))
 @pytest.mark.parametrize("kind", VALUES)
 def test_permutation(form, kind):
+    from grokking_optimizers import _cabi
+    sizes = [wl.numel(s) for s in SHAPES[form]]
+    assert _cabi.sort_form_for(sizes) == FORMS.get(form, "runs")
+    assert _cabi.sort_form_for(sizes, True) == ("small passes" if form in WIDE else FORMS.get(form, "runs"))
     for dtype in ([torch.float32, torch.bfloat16] if kind in ("random", "ties") else [torch.float32]):
         shapes, r = SHAPES[form], np.random.RandomState(len(form) + len(kind))
         case = Sg2Case(shapes, dtypes=[dtype] * len(shapes), seed=1)
