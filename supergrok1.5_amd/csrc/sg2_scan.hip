@@ -284,7 +284,7 @@ __device__ __forceinline__ void gates_of(float g, float s, int c0, const float* 
 // is what the lane polynomials of the recurrence take.
 // dxk: this lane's 16 skips D * x-branch of (column cj, timestep 16 cq + k), kept for gate_rows.
 // DELTA false, for a tile whose steps are inside the Taylor range but not all on the polynomials (with timesteps per lane there, 3.1 M
-// bf16 elements took 1026 us a step for 1001, 25 M 5595 for 5468): the step-size row receives dt itself,
+// bf16 elements took 1020 us a step for 991, 0.42 M 248 for 243, 25 M the same): the step-size row receives dt itself,
 // and angle the lane's verdict on the two blocks of its timesteps (bits 0 / 1: every angle of its column small enough for
 // sg_sincos_small / sg_sincos_tiny in the first, bits 2 / 3 in the second; see project_steps).
 template <class G, bool HAS_S, bool DELTA>
@@ -465,7 +465,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const float* rope = pl.W.w[dir ? W_B_ROPE : W_F_ROPE];
     // -A/2 with A = -exp(A_log) of the two poles of a pair, and its frequency, in registers (256 now): with module-made poles about half
     // of the blocks of ordinary gradients take a form that needs them, and forming them again in each, two loads and two
-    // exponentials, cost 7 to 10 % of a step (3.1 M bf16 1135 -> 1026 us, 0.42 M 267 -> 250, wide geometry 625 -> 576).
+    // exponentials, cost 6 to 10 % of a step (3.1 M bf16 1112 -> 1020 us, 0.42 M 263 -> 248, wide geometry 628 -> 566; 25 M the same).
     float poles[2][3];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
