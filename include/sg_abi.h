@@ -581,12 +581,20 @@ typedef struct SgMuonMatrix {
 
 size_t sg_muon_workspace_bytes(int num_matrices, const SgMuonMatrix* mats);
 
+/* How many times a call with these matrices (their sizes and types are read)
+ * and iterations forms the Gram matrix from the iterate and applies polynomials
+ * to it: ns_steps, or less where several iterations share both, tracking the
+ * Gram matrix in between (half precision in the place of bf16).  -1 for what
+ * sg_muon_step refuses. */
+int sg_muon_stages_for(int num_matrices, const SgMuonMatrix* mats, int ns_steps);
+
 /* Muon step for all matrices: buf = momentum*buf + g; X = buf/(||buf||_F+1e-7)
  * with the norm reduced on the device; ns_steps quintic Newton-Schulz
  * iterations X <- aX + b(XX^T)X + c(XX^T)^2 X with (a,b,c) = (3.4445, -4.7750,
- * 2.0315); p = (p - 0.2*lr*X) * (1 - lr*wd).  The iterations run as bf16 MFMA
+ * 2.0315); p = (p - 0.2*lr*X) * (1 - lr*wd).  The iterations run as 16-bit MFMA
  * GEMMs with fp32 accumulation, on the Gram matrix of the smaller dimension
- * (X^T X for tall matrices; the same product re-associated).  Replaces the
+ * (X^T X for tall matrices; the same product re-associated), up to three
+ * iterations on one Gram matrix (sg_muon_stages_for).  Replaces the
  * body of muon_fused_step (csrc/ops.cpp:663-746: ATen norm + host sync,
  * three torch::mm per iteration, muon_ns_combine_kernel and
  * muon_update_kernel, csrc/muon_kernels.cu:37-72). */

@@ -1,5 +1,5 @@
 // Muon step: momentum (which also leaves the bf16 work copy), Frobenius norm (folded into the first iteration), quintic Newton-Schulz
-// orthogonalisation as bf16 MFMA GEMMs with fp32 accumulation, parameter
+// orthogonalisation as 16-bit MFMA GEMMs with fp32 accumulation, parameter
 // update.  Replaces the body of muon_fused_step (csrc/ops.cpp:663-746 of the
 // reference: ATen norm + one host sync, three torch::mm per iteration,
 // muon_ns_combine_kernel / muon_update_kernel of csrc/muon_kernels.cu:37-72).
@@ -12,6 +12,16 @@
 // a Y in the epilogue, the error of either form is set by the rounding of G)
 // (for a tall parameter X this is X^T X and X (bG + cG^2): the reference's
 // X X^T form re-associated, 6 m^2 n instead of 6 n^2 m flops per iteration).
+// Forming G from Y costs as much as n / m small products, the apply step as much as 2 n / m.  The polynomials of one iterate
+// commute, so several iterations share both (a stage): with G tracked instead of formed again,
+//     P = a I + b G + c G G        Q <- P Q        G <- P G P, as S = P G and S P
+// and Y <- Q Y at the stage's end.  Five iterations are two stages, of two and three: 2 (n/m + 2 n/m) + 14 small products where
+// one stage an iteration takes 5 (n/m + 2 n/m) + 5.  A tracked G drifts from Y Y^T by its roundings, which small singular
+// values feel (they grow by a = 3.4 an iteration, those of G by its square): not more than three iterations a stage, and
+// everything but the momentum itself and what multiplies it in half precision, eight times finer than bf16 (numbers stay
+// below 1.3 resp. 41, scales in F16_SCALE).  Distance from float64 over Gaussian, low-rank, power-law and badly scaled
+// matrices: 0.3-0.9 of that of five stages in bf16 (1024 x 4096 Gaussian 3.0e-3 against 6.9e-3).  All five in one stage would
+// be 0.107 against 0.017 on a power law.  24 bf16 matrices of 1024 x 4096: 2181 -> 1642 us a step.
 // The Gram and polynomial products are "NT" GEMMs (both operands K-contiguous).
 // The apply step is (on 256x256 tiles) an "NN" one: its B operand is Y itself, whose K axis is
 // the slow one.  Its tiles are staged in LDS as they lie in memory
@@ -49,9 +59,14 @@
 namespace sgmu {
 namespace {
 
-typedef uint16_t bf16_t;
+typedef uint16_t bf16_t;           // sixteen bits of either type: what a buffer holds is known where it is used
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+enum { T_BF16 = 0, T_F16 = 1 };
+// Half-precision iterates and Gram matrices are held times 2^14: the largest singular value stays below 1.3 throughout, so no
+// entry can overflow, and full precision reaches down to 4e-9.  (Powers of two: the factors round nothing.)
+constexpr float F16_SCALE = 16384.0f, F16_UNSCALE = 1.0f / 16384.0f;
 
 constexpr int BT = 256;            // GEMM tile (M and N)
 // Waves of a workgroup along N (2 along M).  Eight waves of 128 x 64 (two per SIMD, 128 accumulators each) measured
@@ -67,7 +82,8 @@ struct Mat {
     void* param;
     const void* grad;
     float* buf;
-    bf16_t *Y, *Y2, *G, *H;       // [mp x np] twice (an iteration reads one and writes the other), [mp x mp], [mp x mp]
+    bf16_t *Y, *Y2;                // [mp x np] twice (an apply step reads one and writes the other)
+    bf16_t* W[5];                  // [mp x mp]: Gram matrices, polynomials and their products
     bf16_t *T, *T2;                // the transposes of Y and Y2 [np x mp], or NULL (kept for k_gemm_64's apply step)
     int rows, cols, dtype;
     int m, n, mp, np;              // min / max dim and their padded sizes
@@ -228,7 +244,13 @@ __global__ __launch_bounds__(256) void k_norm(Batch B) {
 // Per 16-wide k step a wave fetches 4+4 16-byte operands from LDS for 16 MFMAs.
 // The Gram and polynomial products are symmetric: only tiles on or above the diagonal are
 // computed, each off-diagonal tile is also stored transposed.
-enum { EPI_GRAM = 0, EPI_POLY = 1, EPI_APPLY = 2 };
+// EPI_MUL is a plain product of two commuting symmetric matrices, as symmetric as they are.
+enum { EPI_GRAM = 0, EPI_POLY = 1, EPI_APPLY = 2, EPI_MUL = 3 };
+constexpr int shape_of(int epi) { return epi == EPI_MUL ? EPI_POLY : epi; }      // whose tiles and tables it takes
+// Which of Mat::W a launch reads and writes: W[c] = A(a) B(b); c2 >= 0: the second half of the grid forms W[c2] = W[a2] W[b2]
+struct Ops {
+    int a, b, c, a2, b2, c2;
+};
 // explicit global address space: a generic (flat) load would count against the LDS wait counter as well
 typedef const __attribute__((address_space(1))) u32x4* gvec_p;
 typedef __attribute__((address_space(1))) u32x4* gvec_w;
@@ -238,6 +260,38 @@ __device__ __forceinline__ uint32_t bf16r2(float lo, float hi) {
     typedef __attribute__((ext_vector_type(2))) float f32x2;
     typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){lo, hi}, bf16x2));
+}
+
+template <int T>
+__device__ __forceinline__ uint32_t round2(float lo, float hi) {
+    if (T == T_BF16) return bf16r2(lo, hi);
+    typedef __attribute__((ext_vector_type(2))) float f32x2;
+    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){lo, hi}, f16x2));
+}
+// entry k of two packed ones
+template <int T>
+__device__ __forceinline__ float widen(uint32_t w, int k) {
+    if (T == T_BF16) return sg_i2f((int32_t)((k & 1) ? (w & 0xffff0000u) : (w << 16)));
+    return __half2float(__ushort_as_half((uint16_t)((k & 1) ? (w >> 16) : (w & 0xffffu))));
+}
+template <int T>
+__device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
+    if (T == T_BF16) return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+// what a product is multiplied by besides the norm: the scales of half-precision operands and results (above)
+template <int EPI, int IN, int OUT>
+constexpr float epi_factor() {
+    if (EPI == EPI_GRAM) return (IN == T_F16 ? F16_UNSCALE * F16_UNSCALE : 1.0f) * (OUT == T_F16 ? F16_SCALE : 1.0f);
+    if (EPI == EPI_APPLY) return (IN == T_F16 ? F16_UNSCALE : 1.0f) * (OUT == T_F16 ? F16_SCALE : 1.0f);
+    return 1.0f;
+}
+// b G + c G G (+ a on the diagonal) from a product of G, as it is held, and an entry of it
+template <int T>
+__device__ __forceinline__ float polynomial(float gg, float g) {
+    if (T == T_BF16) return sg_fma(NS_C, gg, NS_B * g);
+    return sg_fma(NS_C * F16_UNSCALE * F16_UNSCALE, gg, NS_B * F16_UNSCALE * g);
 }
 
 // The R operand reads of the next k step are dealt over the first eight of a phase's M MFMAs (R/8 after each, one more
@@ -257,8 +311,9 @@ typedef __attribute__((address_space(3))) i16x4* lds_i16x4_p;
 
 // y_sel: which of the two Y buffers holds the current iterate
 // iter_flags: bit 1 = first iteration (Y still carries the factor norm: see k_momentum)
-template <int EPI>
-__global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int iter_flags) {
+// IN, OUT: what the operands and the result are held in
+template <int EPI, int IN, int OUT>
+__global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, Ops ops, int y_sel, int iter_flags) {
     constexpr bool BKN = EPI == EPI_APPLY;             // B operand stored [K x N]
     constexpr int TM = BT / 64, TN = WCOLS / 32;       // MFMA tiles per wave in each direction (4 x 4 or 4 x 2)
     constexpr int LPT = 16 / GWAVES;                  // loads per wave, tile and operand (a tile is 16 blocks of 1 KB)
@@ -271,7 +326,8 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int i
     if (nblk % 8 == 0) lb = (blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / GWN, wn = wave % GWN;
-    const sg::cint_p prefix = sg::as_const(Bt.gtile_prefix[EPI]);
+    const sg::cint_p prefix = sg::as_const(Bt.gtile_prefix[shape_of(EPI)]);
+    if (EPI == EPI_MUL && ops.c2 >= 0 && lb >= nblk / 2) { lb -= nblk / 2; ops.a = ops.a2; ops.b = ops.b2; ops.c = ops.c2; }
     const int mi = sg::upper_seg(prefix, Bt.P, lb);
     const Mat& Mt = Bt.mats[mi];
     int tile = lb - prefix[mi];
@@ -280,7 +336,7 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int i
     bf16_t *C, *CT;         // CT: where the transposed tile goes (the symmetric products mirror into C itself)
     int K, lda, ldb, ldc, ldct, tm, tn;
     if (EPI == EPI_APPLY) {
-        A = Mt.H; B = y_sel ? Mt.Y2 : Mt.Y; C = y_sel ? Mt.Y : Mt.Y2; K = Mt.mp; lda = Mt.mp; ldb = ldc = Mt.np;
+        A = Mt.W[ops.a]; B = y_sel ? Mt.Y2 : Mt.Y; C = y_sel ? Mt.Y : Mt.Y2; K = Mt.mp; lda = Mt.mp; ldb = ldc = Mt.np;
         CT = C; ldct = ldc;      // unused: the apply step never mirrors
         // bands of 8 tile columns: 32 tiles that run together span 4 x 8 tiles instead of 2 x 16,
         // which halves the panel bytes they pull into L2
@@ -294,8 +350,9 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int i
             tn = tile % ntn;
         }
     } else {
-        if (EPI == EPI_GRAM) { A = y_sel ? Mt.Y2 : Mt.Y; B = A; C = Mt.G; K = Mt.np; lda = ldb = Mt.np; ldc = Mt.mp; }
-        else { A = Mt.G; B = Mt.G; C = Mt.H; K = Mt.mp; lda = ldb = ldc = Mt.mp; }
+        C = Mt.W[ops.c];
+        if (EPI == EPI_GRAM) { A = y_sel ? Mt.Y2 : Mt.Y; B = A; K = Mt.np; lda = ldb = Mt.np; ldc = Mt.mp; }
+        else { A = Mt.W[ops.a]; B = Mt.W[ops.b]; K = Mt.mp; lda = ldb = ldc = Mt.mp; }
         CT = C; ldct = ldc;
         const int nt = Mt.mp / BT;      // upper-triangular enumeration: row tm holds nt - tm tiles
         tm = 0;
@@ -389,11 +446,11 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int i
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[s][i], bv[s][j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < TN; j++) acc[i][j] = mfma<IN>(av[s][i], bv[s][j], acc[i][j]);
     };
 
     const int nk = K / BKD;      // a multiple of 8: K is a multiple of 256
-    const bf16_t* aux = Mt.G;
+    const bf16_t* aux = EPI == EPI_POLY ? Mt.W[ops.a] : nullptr;
     const int gcol0 = tn * BT + wn * WCOLS;
     // the auxiliary operand of the polynomial's epilogue (G):
     // 16 bytes per lane and 8-column chunk of a 32-row block of this wave's tile.  The first two blocks are requested during
@@ -451,7 +508,7 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int i
             }
 #pragma unroll
             for (int m = MPG * g; m < MPG * (g + 1); m++)
-                acc[m / TN][m % TN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[1][m / TN], bv[1][m % TN], acc[m / TN][m % TN], 0, 0, 0);
+                acc[m / TN][m % TN] = mfma<IN>(av[1][m / TN], bv[1][m % TN], acc[m / TN][m % TN]);
             __builtin_amdgcn_sched_barrier(0);
             if (DMA && g < 2 * LPT) dma_one(kt + 4, g);
             __builtin_amdgcn_sched_barrier(0);
@@ -488,7 +545,8 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int i
     const float inv = Bt.inv_norm[mi];
     const bool diag_wave = EPI == EPI_POLY && tm == tn && wn / (GWN / 2) == wm;     // this wave's block meets the diagonal
     const bool first = (iter_flags & 2) != 0;
-    const float first_scale = first ? (EPI == EPI_GRAM ? inv * inv : (EPI == EPI_APPLY ? inv : 1.0f)) : 1.0f;
+    constexpr float factor = epi_factor<EPI, IN, OUT>();
+    const float scale = first ? (EPI == EPI_GRAM ? inv * inv : inv) * factor : factor;
 #pragma unroll
     for (int i = 0; i < TM; i++) {
         const int grow0 = tm * BT + wm * (BT / 2) + i * 32;
@@ -507,9 +565,7 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int i
             if (EPI == EPI_POLY) {
 #pragma unroll
                 for (int k = 0; k < 8; k++) {
-                    const uint32_t w = ax[i & 1][c][k >> 1];
-                    const float x = sg_i2f((int32_t)((k & 1) ? (w & 0xffff0000u) : (w << 16)));
-                    v[k] = sg_fma(NS_C, v[k], NS_B * x);
+                    v[k] = polynomial<IN>(v[k], widen<IN>(ax[i & 1][c][k >> 1], k));
                 }
                 if (diag_wave) {        // H + a I: the apply step is then the single product (H + a I) Y
                     const int dk = (wm * (BT / 2) + i * 32 + row) - (wn * WCOLS + c8 * 8);
@@ -517,15 +573,15 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, int y_sel, int i
                     for (int k = 0; k < 8; k++) v[k] += (dk == k) ? NS_A : 0.0f;
                 }
             }
-            if (EPI != EPI_POLY && first) {      // uniform over the grid
+            if ((EPI == EPI_GRAM || EPI == EPI_APPLY) && (first || factor != 1.0f)) {      // uniform over the grid
 #pragma unroll
-                for (int k = 0; k < 8; k++) v[k] *= first_scale;
+                for (int k = 0; k < 8; k++) v[k] *= scale;
             }
             u32x4 out;
 #pragma unroll
-            for (int k = 0; k < 4; k++) out[k] = bf16r2(v[2 * k], v[2 * k + 1]);
+            for (int k = 0; k < 4; k++) out[k] = round2<OUT>(v[2 * k], v[2 * k + 1]);
             *(gvec_w)(C + (size_t)(grow0 + row) * ldc + gcol0 + c8 * 8) = out;
-            if (mirror) {   // rounded values (as bf16 bit patterns) back into the staged block
+            if (mirror) {   // rounded values (as bit patterns) back into the staged block
                 u32x4 b0 = {out[0] & 0xffffu, out[0] >> 16, out[1] & 0xffffu, out[1] >> 16};
                 u32x4 b1 = {out[2] & 0xffffu, out[2] >> 16, out[3] & 0xffffu, out[3] >> 16};
                 reinterpret_cast<u32x4*>(src)[0] = b0;
@@ -570,8 +626,8 @@ constexpr int KS_STAGE = 2 * NT64 * 32 * 2, KS_WAVE = 2 * KS_STAGE;             
 static_assert(KS_WAVES * KS_WAVE <= KS_LDS_BYTES, "the waves' stages fit where their partial tiles go");
 
 // y_sel: as for k_gemm_nt; iter_flags: bit 1 = first iteration, bit 2 = last (no product reads T any more)
-template <int EPI>
-__global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, int y_sel, int iter_flags) {
+template <int EPI, int IN, int OUT>
+__global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, Ops ops, int y_sel, int iter_flags) {
     constexpr int W = KS_WAVES;
     extern __shared__ __attribute__((aligned(16))) float part[];
     __shared__ double sm[W];
@@ -579,7 +635,8 @@ __global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, int y_sel, int
     int lb = blockIdx.x;
     if (nblk % 8 == 0) lb = (blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8;      // XCD-contiguous, as in k_gemm_nt
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const sg::cint_p prefix = sg::as_const(Bt.gtile_prefix[EPI]);
+    const sg::cint_p prefix = sg::as_const(Bt.gtile_prefix[shape_of(EPI)]);
+    if (EPI == EPI_MUL && ops.c2 >= 0 && lb >= nblk / 2) { lb -= nblk / 2; ops.a = ops.a2; ops.b = ops.b2; ops.c = ops.c2; }
     const int mi = sg::upper_seg(prefix, Bt.P, lb);
     const Mat& Mt = Bt.mats[mi];
     int tile = lb - prefix[mi];
@@ -589,14 +646,15 @@ __global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, int y_sel, int
     bf16_t *C, *CT;         // CT: where the transposed tile goes (NULL: nowhere)
     int K, ldc, ldct, tm, tn;
     if (EPI == EPI_APPLY) {
-        A = Mt.H; B = y_sel ? Mt.T2 : Mt.T; C = y_sel ? Mt.Y : Mt.Y2; K = Mt.mp; ldc = Mt.np;
+        A = Mt.W[ops.a]; B = y_sel ? Mt.T2 : Mt.T; C = y_sel ? Mt.Y : Mt.Y2; K = Mt.mp; ldc = Mt.np;
         CT = last ? nullptr : (y_sel ? Mt.T : Mt.T2); ldct = Mt.mp;
         const int ntm = Mt.mp / NT64;
         tm = tile % ntm;
         tn = tile / ntm;
     } else {
-        if (EPI == EPI_GRAM) { A = B = y_sel ? Mt.Y2 : Mt.Y; C = Mt.G; K = Mt.np; }
-        else { A = B = Mt.G; C = Mt.H; K = Mt.mp; }
+        C = Mt.W[ops.c];
+        if (EPI == EPI_GRAM) { A = B = y_sel ? Mt.Y2 : Mt.Y; K = Mt.np; }
+        else { A = Mt.W[ops.a]; B = Mt.W[ops.b]; K = Mt.mp; }
         ldc = ldct = Mt.mp;
         const int nt = Mt.mp / NT64;
         tm = 0;
@@ -643,7 +701,7 @@ __global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, int y_sel, int
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[u][j], a[u][i], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < 2; j++) acc[i][j] = mfma<IN>(b[u][j], a[u][i], acc[i][j]);
     };
     const int nk = K / 32;
     int c = wave, s = 0;
@@ -670,11 +728,12 @@ __global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, int y_sel, int
     u32x4 g[NR];
     if (EPI == EPI_POLY) {
 #pragma unroll
-        for (int h = 0; h < NR; h++) g[h] = *(gvec_p)(Mt.G + (size_t)(tm * NT64 + row0 + 8 * W * h) * ldc + tn * NT64 + 8 * c8);
+        for (int h = 0; h < NR; h++) g[h] = *(gvec_p)(A + (size_t)(tm * NT64 + row0 + 8 * W * h) * ldc + tn * NT64 + 8 * c8);
     }
     // first iteration: Y is the unnormalised momentum, see k_momentum; the norm is added up from its tiles here
-    float scale = 1.0f;
-    if (EPI != EPI_POLY && first) {
+    constexpr float factor = epi_factor<EPI, IN, OUT>();
+    float scale = factor;
+    if ((EPI == EPI_GRAM || EPI == EPI_APPLY) && first) {
         double sq = 0.0;
         for (int k = Bt.ttile_prefix[mi] + tid; k < Bt.ttile_prefix[mi + 1]; k += 64 * W) sq += Bt.partials[k];
 #pragma unroll
@@ -693,10 +752,10 @@ __global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, int y_sel, int
                         f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
     }
     __syncthreads();
-    if (EPI != EPI_POLY && first) {
+    if ((EPI == EPI_GRAM || EPI == EPI_APPLY) && first) {
         const double tot = (sm[0] + sm[1]) + (sm[2] + sm[3]);
         const float inv = 1.0f / ((float)sqrt(tot) + 1e-7f);
-        scale = EPI == EPI_GRAM ? inv * inv : inv;
+        scale = (EPI == EPI_GRAM ? inv * inv : inv) * factor;
     }
     u32x4 out[NR];
 #pragma unroll
@@ -714,15 +773,14 @@ __global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, int y_sel, int
         if (EPI == EPI_POLY) {
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                const float x = sg_i2f((int32_t)((k & 1) ? (g[h][k >> 1] & 0xffff0000u) : (g[h][k >> 1] << 16)));
-                v[k] = sg_fma(NS_C, v[k], NS_B * x) + (tm == tn && row == 8 * c8 + k ? NS_A : 0.0f);
+                v[k] = polynomial<IN>(v[k], widen<IN>(g[h][k >> 1], k)) + (tm == tn && row == 8 * c8 + k ? NS_A : 0.0f);
             }
-        } else if (first) {
+        } else if (EPI != EPI_MUL && (first || factor != 1.0f)) {
 #pragma unroll
             for (int k = 0; k < 8; k++) v[k] *= scale;
         }
 #pragma unroll
-        for (int k = 0; k < 4; k++) out[h][k] = bf16r2(v[2 * k], v[2 * k + 1]);
+        for (int k = 0; k < 4; k++) out[h][k] = round2<OUT>(v[2 * k], v[2 * k + 1]);
         *(gvec_w)(C + (size_t)(tm * NT64 + row) * ldc + tn * NT64 + 8 * c8) = out[h];
     }
     if (CT) {       // uniform over the workgroup
@@ -1017,8 +1075,8 @@ __global__ __launch_bounds__(NS_THREADS) void k_newton_schulz(Batch B, int steps
 
 // p = (p - 0.2*lr*X) * (1 - lr*wd).  X lies in the wide orientation; one 64x64 tile of the parameter's own
 // orientation per workgroup (the grid of k_momentum), a tall parameter's tile of X is transposed through LDS.
-// scale_inv: no iteration ran, X is still the unnormalised momentum
-__global__ __launch_bounds__(256) void k_update(Batch B, float lr, float decay, int y_sel, int scale_inv) {
+// scale_inv: no iteration ran, X is still the unnormalised momentum; type: what X is held in
+__global__ __launch_bounds__(256) void k_update(Batch B, float lr, float decay, int y_sel, int scale_inv, int type) {
     __shared__ bf16_t t[64][66];
     const int mi = sg::upper_seg(B.ttile_prefix, B.P, blockIdx.x);
     const Mat& M = B.mats[mi];
@@ -1031,7 +1089,8 @@ __global__ __launch_bounds__(256) void k_update(Batch B, float lr, float decay, 
     const float max_dim = (float)max(M.rows, M.cols);
     const float scale_factor = 0.2f * sqrtf(max_dim);
     const float neg_lr_scale = -lr * scale_factor / sqrtf(max_dim);
-    const float xs = scale_inv ? B.inv_norm[mi] : 1.0f;
+    const float xs = scale_inv ? B.inv_norm[mi] : type == T_F16 ? F16_UNSCALE : 1.0f;
+    const int dtype = type == T_F16 ? SG_F16 : SG_BF16;
     const bool full = tr0 + 64 <= M.rows && tc0 + 64 <= M.cols && M.vec8;
     const int lr_ = threadIdx.x >> 2, c0 = (threadIdx.x & 3) * 16;
     if (!M.wide) {
@@ -1052,11 +1111,11 @@ __global__ __launch_bounds__(256) void k_update(Batch B, float lr, float decay, 
         const size_t at = (size_t)(tr0 + lr_) * M.cols + tc0 + c0;
         float o[16], p[16];
         if (M.wide) {
-            load8(X, SG_BF16, (size_t)(tr0 + lr_) * M.np + tc0 + c0, o);
-            load8(X, SG_BF16, (size_t)(tr0 + lr_) * M.np + tc0 + c0 + 8, o + 8);
+            load8(X, dtype, (size_t)(tr0 + lr_) * M.np + tc0 + c0, o);
+            load8(X, dtype, (size_t)(tr0 + lr_) * M.np + tc0 + c0 + 8, o + 8);
         } else {
 #pragma unroll
-            for (int e = 0; e < 16; e++) o[e] = sg::bf16_bits_to_f(t[c0 + e][lr_]);
+            for (int e = 0; e < 16; e++) o[e] = type == T_F16 ? widen<T_F16>(t[c0 + e][lr_], 0) : sg::bf16_bits_to_f(t[c0 + e][lr_]);
         }
         load8(M.param, M.dtype, at, p);
         load8(M.param, M.dtype, at + 8, p + 8);
@@ -1073,7 +1132,8 @@ __global__ __launch_bounds__(256) void k_update(Batch B, float lr, float decay, 
     for (int k = threadIdx.x; k < 64 * 64; k += 256) {
         const int r = tr0 + (k >> 6), c = tc0 + (k & 63);
         if (r >= M.rows || c >= M.cols) continue;
-        float o = sg::bf16_bits_to_f(M.wide ? X[(size_t)r * M.np + c] : t[k & 63][k >> 6]) * xs;
+        const bf16_t x = M.wide ? X[(size_t)r * M.np + c] : t[k & 63][k >> 6];
+        float o = (type == T_F16 ? widen<T_F16>(x, 0) : sg::bf16_bits_to_f(x)) * xs;
         if (M.dtype == SG_F16) o = __half2float(__float2half_rn(o));
         const int64_t i = (int64_t)r * M.cols + c;
         const float p = sg::load_elem(M.param, M.dtype, i);
@@ -1088,6 +1148,7 @@ struct Layout {
     std::vector<Mat> mats;
     bool small;                    // every matrix fits k_newton_schulz
     bool fine[3];                  // products that go to k_gemm_64
+    double time[3];                // and what choose_tiles expects each to take
     std::vector<int> pre_g[3], pre_t;
     size_t off_mats, off_pre, off_partials, off_inv, bytes;
 };
@@ -1097,7 +1158,7 @@ struct Layout {
 // longer of the chain of one tile (0.003 K) and what all tiles take together (3 ns and 14 ps per k each).  Over 18 sets from
 // 1 x 200 x 800 to 6 x 1024 x 4096 the choice so made was within 8 % of the best.
 // fine_pad: what the matrices would be padded to for k_gemm_64 (64, or 256 where another product keeps its large tiles)
-void choose_tiles(int P, const SgMuonMatrix* in, int fine_pad, bool fine[3]) {
+void choose_tiles(int P, const SgMuonMatrix* in, int fine_pad, bool fine[3], double time[3]) {
     double tiles[3] = {}, each[3] = {}, chain[3] = {}, k_max[3] = {};
     for (int i = 0; i < P; i++) {
         const double m = (double)std::min(in[i].rows, in[i].cols), n = (double)std::max(in[i].rows, in[i].cols);
@@ -1114,8 +1175,11 @@ void choose_tiles(int P, const SgMuonMatrix* in, int fine_pad, bool fine[3]) {
             chain[e] = std::max(chain[e], 0.003 * k);
         }
     }
-    for (int e = 0; e < 3; e++)
-        fine[e] = 5.0 + std::max(chain[e], each[e]) < std::ceil(tiles[e] / 256.0) * (7.0 + 0.0165 * k_max[e]);
+    for (int e = 0; e < 3; e++) {
+        const double small = 5.0 + std::max(chain[e], each[e]), large = std::ceil(tiles[e] / 256.0) * (7.0 + 0.0165 * k_max[e]);
+        fine[e] = small < large;
+        time[e] = std::min(small, large);
+    }
 }
 
 int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
@@ -1136,8 +1200,8 @@ int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
         L->small = L->small && m > 0 && m <= 128 && n <= NS_Y_ELEMS && fits_lds(round_up((int)m, 64), round_up((int)n, 64));
     }
     auto all_fine = [&] { return L->fine[EPI_GRAM] && L->fine[EPI_POLY] && L->fine[EPI_APPLY]; };
-    choose_tiles(P, in, NT64, L->fine);
-    if (!all_fine()) choose_tiles(P, in, BT, L->fine);
+    choose_tiles(P, in, NT64, L->fine, L->time);
+    if (!all_fine()) choose_tiles(P, in, BT, L->fine, L->time);
     const int pad = L->small || all_fine() ? 64 : BT;
     for (int i = 0; i < P; i++) {
         const SgMuonMatrix& s = in[i];
@@ -1167,17 +1231,46 @@ int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
         // offsets for now; turned into pointers once the workspace base is known
         M.Y = (bf16_t*)take(2 * (size_t)M.mp * M.np);
         M.Y2 = (bf16_t*)take(2 * (size_t)M.mp * M.np);
-        M.G = M.H = M.T = M.T2 = nullptr;
+        M.T = M.T2 = nullptr;
+        for (auto& w : M.W) w = nullptr;
         if (L->small) continue;
         if (L->fine[EPI_APPLY]) {
             M.T = (bf16_t*)take(2 * (size_t)M.mp * M.np);
             M.T2 = (bf16_t*)take(2 * (size_t)M.mp * M.np);
         }
-        M.G = (bf16_t*)take(2 * (size_t)M.mp * M.mp);
-        M.H = (bf16_t*)take(2 * (size_t)M.mp * M.mp);
+        for (auto& w : M.W) w = (bf16_t*)take(2 * (size_t)M.mp * M.mp);
     }
     L->bytes = o;
     return 0;
+}
+
+// The products, on tiles of either size.
+struct Product {
+    int epi, in, out;
+    void (*k256)(Batch, Ops, int, int);
+    void (*k64)(Batch, Ops, int, int);
+};
+#define SG_PRODUCT(E, I, O) {E, I, O, k_gemm_nt<E, I, O>, k_gemm_64<E, I, O>}
+const Product products[] = {
+    SG_PRODUCT(EPI_GRAM, T_BF16, T_BF16),  SG_PRODUCT(EPI_POLY, T_BF16, T_BF16),  SG_PRODUCT(EPI_APPLY, T_BF16, T_BF16),
+    SG_PRODUCT(EPI_GRAM, T_BF16, T_F16),   SG_PRODUCT(EPI_GRAM, T_F16, T_F16),    SG_PRODUCT(EPI_POLY, T_F16, T_F16),
+    SG_PRODUCT(EPI_MUL, T_F16, T_F16),     SG_PRODUCT(EPI_MUL, T_F16, T_BF16),
+    SG_PRODUCT(EPI_APPLY, T_BF16, T_F16),  SG_PRODUCT(EPI_APPLY, T_F16, T_F16),
+};
+#undef SG_PRODUCT
+
+// In how many stages the iterations run (see the head of the file): at most three iterations a stage, or one a stage (the Gram
+// matrix from Y every time, in bf16), which near squares and in calls that wait for launches more than for products is
+// faster.  By what choose_tiles expects; over 22 sets the measured ratio tracked / each lay between -0.11 and +0.18 of the
+// expected one (the small products of a full chip take longer than their fit), so it has to be below 0.95.  Five iterations,
+// each / tracked: 24 of 1024 x 1024 834 / 995 us (expected 1.00), 2 of 1000 x 1500 250 / 257 (0.99), 16 of 512 x 2048 404 / 388
+// (0.93), 12 of 300 x 1200 234 / 202 (0.93), 1 of 1024 x 4096 284 / 237 (0.80), 1 of 100 x 4000 162 / 129 (0.86).
+int count_stages(const Layout& L, int ns_steps) {
+    if (L.small) return ns_steps;
+    const int stages = (ns_steps + 2) / 3;
+    const double ends = L.time[EPI_GRAM] + L.time[EPI_APPLY], poly = L.time[EPI_POLY];
+    const double tracked = stages * ends + (4 * ns_steps - 3 * stages) * poly, each = ns_steps * (ends + poly);
+    return tracked < 0.95 * each ? stages : ns_steps;
 }
 
 }  // namespace
@@ -1190,6 +1283,13 @@ size_t sg_muon_workspace_bytes(int num_matrices, const SgMuonMatrix* mats) {
     sgmu::Layout L;
     if (sgmu::make_layout(num_matrices, mats, &L)) return 0;
     return L.bytes;
+}
+
+int sg_muon_stages_for(int num_matrices, const SgMuonMatrix* mats, int ns_steps) {
+    sgmu::Layout L;
+    if (num_matrices <= 0 || ns_steps < 0 || !mats) return sg::fail("no matrices, or ns_steps below 0"), -1;
+    if (sgmu::make_layout(num_matrices, mats, &L)) return -1;
+    return sgmu::count_stages(L, ns_steps);
 }
 
 int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, float lr, float wd, int ns_steps, void* workspace,
@@ -1209,7 +1309,7 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
     const int P = L.P;
     for (auto& M : L.mats) {
         M.Y = (bf16_t*)(ws + (size_t)M.Y); M.Y2 = (bf16_t*)(ws + (size_t)M.Y2);
-        M.G = (bf16_t*)(ws + (size_t)M.G); M.H = (bf16_t*)(ws + (size_t)M.H);
+        for (auto& w : M.W) w = (bf16_t*)(ws + (size_t)w);
         if (M.T) { M.T = (bf16_t*)(ws + (size_t)M.T); M.T2 = (bf16_t*)(ws + (size_t)M.T2); }
     }
     // per-call tables: through kernel arguments (no host-to-device copy, nothing blocks the host), records and tile prefixes
@@ -1239,13 +1339,10 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
         SG_HIP_CHECK(hipGetDevice(&dev));
         if (dev < 0 || dev >= 64) return sg::fail("device index %d out of range", dev);
         if (!raised[dev]) {
-
-            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_nt<EPI_GRAM>), hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS_BYTES));
-            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_nt<EPI_POLY>), hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS_BYTES));
-            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_nt<EPI_APPLY>), hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS_BYTES));
-            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_64<EPI_GRAM>), hipFuncAttributeMaxDynamicSharedMemorySize, KS_LDS_BYTES));
-            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_64<EPI_POLY>), hipFuncAttributeMaxDynamicSharedMemorySize, KS_LDS_BYTES));
-            SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_64<EPI_APPLY>), hipFuncAttributeMaxDynamicSharedMemorySize, KS_LDS_BYTES));
+            for (const Product& p : products)
+                for (int fine = 0; fine < 2; fine++)
+                    SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(fine ? p.k64 : p.k256), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     fine ? KS_LDS_BYTES : GEMM_LDS_BYTES));
             SG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_newton_schulz), hipFuncAttributeMaxDynamicSharedMemorySize, NS_LDS_BYTES));
             raised[dev] = true;
         }
@@ -1261,21 +1358,51 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
         hipLaunchKernelGGL(k_newton_schulz, dim3(P), dim3(NS_THREADS), lds, st, B, ns_steps);
         SG_LAUNCH_CHECK("k_newton_schulz");
     }
-    for (int it = 0; it < (L.small ? 0 : ns_steps); it++) {
-        const int sel = it & 1, flags = (it == 0 ? 2 : 0) | (it + 1 == ns_steps ? 4 : 0);     // iter_flags
-        for (int e = 0; e < 3; e++) {
-            const dim3 grid(B.gtiles[e]);
-            if (L.fine[e]) {
-                auto* const k = e == EPI_GRAM ? k_gemm_64<EPI_GRAM> : e == EPI_POLY ? k_gemm_64<EPI_POLY> : k_gemm_64<EPI_APPLY>;
-                hipLaunchKernelGGL(k, grid, dim3(KS_THREADS), KS_LDS_BYTES, st, B, sel, flags);
-            } else {
-                auto* const k = e == EPI_GRAM ? k_gemm_nt<EPI_GRAM> : e == EPI_POLY ? k_gemm_nt<EPI_POLY> : k_gemm_nt<EPI_APPLY>;
-                hipLaunchKernelGGL(k, grid, dim3(GTHREADS), GEMM_LDS_BYTES, st, B, sel, flags);
+    auto launch = [&](int epi, int in, int out, Ops ops, int sel, int flags) {
+        const int e = shape_of(epi);
+        const dim3 grid(B.gtiles[e] * (ops.c2 >= 0 ? 2 : 1));
+        for (const Product& p : products) {
+            if (p.epi != epi || p.in != in || p.out != out) continue;
+            if (L.fine[e]) hipLaunchKernelGGL(p.k64, grid, dim3(KS_THREADS), KS_LDS_BYTES, st, B, ops, sel, flags);
+            else hipLaunchKernelGGL(p.k256, grid, dim3(GTHREADS), GEMM_LDS_BYTES, st, B, ops, sel, flags);
+        }
+    };
+    const int stages = count_stages(L, ns_steps);
+    const bool tracked = stages < ns_steps;
+    for (int j = 0, left = ns_steps; !L.small && j < stages; j++) {
+        const int n = left / (stages - j);               // iterations of this stage: the later ones take one more where they differ
+        left -= n;
+        const int sel = j & 1, flags = (j == 0 ? 2 : 0) | (j + 1 == stages ? 4 : 0);     // iter_flags
+        if (!tracked) {
+            launch(EPI_GRAM, T_BF16, T_BF16, Ops{0, 0, 0, 0, 0, -1}, sel, flags);
+            launch(EPI_POLY, T_BF16, T_BF16, Ops{0, 0, 1, 0, 0, -1}, sel, flags);
+            launch(EPI_APPLY, T_BF16, T_BF16, Ops{1, 0, 0, 0, 0, -1}, sel, flags);
+        } else {
+            // W[0] the Gram matrix, W[q] the product of the polynomials so far; the other three hold what a step forms
+            const int in = j == 0 ? T_BF16 : T_F16;      // the last product of a stage becomes what Y is held in
+            launch(EPI_GRAM, in, T_F16, Ops{0, 0, 0, 0, 0, -1}, sel, flags);
+            int q = -1, free[4] = {1, 2, 3, 4};
+            for (int k = 0; k < n; k++) {
+                // P = a I + b G + c G^2, then S = P G and Q <- P Q together, then G <- S P
+                const int p = free[0], s = free[1], to = free[2];
+                launch(EPI_POLY, T_F16, T_F16, Ops{0, 0, p, 0, 0, -1}, sel, flags);
+                if (k + 1 < n) {
+                    launch(EPI_MUL, T_F16, T_F16, k == 0 ? Ops{p, 0, s, 0, 0, -1} : Ops{p, 0, s, p, q, to}, sel, flags);
+                    launch(EPI_MUL, T_F16, T_F16, Ops{s, p, 0, 0, 0, -1}, sel, flags);
+                } else if (k > 0) {
+                    launch(EPI_MUL, T_F16, in, Ops{p, q, to, 0, 0, -1}, sel, flags);
+                }
+                if (k == 0) {
+                    q = p; free[0] = 4;                  // of 1..4
+                } else {
+                    std::swap(q, free[2]);
+                }
             }
+            launch(EPI_APPLY, in, T_F16, Ops{q, 0, 0, 0, 0, -1}, sel, flags);
         }
         SG_LAUNCH_CHECK("muon newton-schulz");
     }
-    hipLaunchKernelGGL(k_update, dim3(B.ttiles), dim3(256), 0, st, B, lr, 1.0f - lr * wd, ns_steps & 1, ns_steps == 0 ? 1 : 0);
+    hipLaunchKernelGGL(k_update, dim3(B.ttiles), dim3(256), 0, st, B, lr, 1.0f - lr * wd, stages & 1, ns_steps == 0 ? 1 : 0, tracked ? T_F16 : T_BF16);
     SG_LAUNCH_CHECK("k_update");
     return 0;
 }

@@ -47,6 +47,11 @@ class Sg2Options(C.Structure):
     _fields_ = [("chunk_len", C.c_int32), ("scan_window", C.c_int32)]
 
 
+class SgMuonMatrix(C.Structure):
+    _fields_ = [("param", C.c_void_p), ("grad", C.c_void_p), ("buf", C.c_void_p), ("rows", C.c_int64), ("cols", C.c_int64),
+                ("dtype", C.c_int32)]
+
+
 class Sg2Debug(C.Structure):
     _fields_ = [("perm", C.c_void_p), ("expert_idx", C.c_void_p), ("ctx", C.c_void_p)]
 
@@ -155,6 +160,15 @@ def sort_form_for(numels, all_16bit=False):
     if n < 0:
         raise RuntimeError(last_error())
     return SORT_FORMS[n]
+
+
+def muon_stages_for(shapes, ns_steps=5):
+    """How many Gram matrices a Muon step of these fp32 matrices forms from its iterates."""
+    arr = (SgMuonMatrix * len(shapes))(*[SgMuonMatrix(None, None, None, r, c, 0) for r, c in shapes])
+    n = lib().sg_muon_stages_for(len(shapes), arr, ns_steps)
+    if n < 0:
+        raise RuntimeError(last_error())
+    return n
 
 
 def workspace_bytes(numels, dims=None, options=None):

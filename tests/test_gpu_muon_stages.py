@@ -1,0 +1,84 @@
+"""Muon calls whose iterations share Gram matrices (the tracked one in half precision, products of polynomials, two products in
+one launch), on tiles of either size and at both sides of the rule that chooses them, against the fp32 restatement and, for
+spectra that a tracked Gram matrix feels most, against float64."""
+import pytest
+import torch
+
+from grokking_optimizers import _cabi
+from oracle import muon_oracle
+from test_gpu_muon import _ops, _run_case
+
+pytestmark = pytest.mark.gpu
+
+SETS = {
+    "fine": [(64, 3000)] * 3,                                      # 64x64 tiles for all products
+    "ragged": [(100, 4000), (3999, 97), (1, 5)],                   # padding, tall beside wide, a matrix of one row
+    "mixed": [(700, 4096), (1500, 260), (512, 2050)],              # 256x256 tiles for the apply step
+    "large": [(257, 2048)] * 24 + [(2049, 255)] * 24,              # ... for all of them, more than one round of tiles
+}
+
+
+@pytest.mark.parametrize("ns", [2, 3, 4, 5, 6, 7])
+def test_iterations_of_a_stage(ns):
+    stages = {2: 1, 3: 1, 4: 2, 5: 2, 6: 2, 7: 3}
+    assert _cabi.muon_stages_for(SETS["ragged"], ns) == stages[ns]
+    _compare(SETS["ragged"], ns)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shapes", SETS.values(), ids=SETS.keys())
+def test_tiles(shapes, dtype):
+    assert _cabi.muon_stages_for(shapes) == 2
+    _run_case(shapes, dtype, 1, seed=11, ns=3 if dtype != torch.float32 or len(shapes) > 4 else 5)
+
+
+def _compare(shapes, ns, make=None, bound=2e-2):
+    """The update itself (a parameter of zero, lr 5) against the float64 iteration, in the 2-norm."""
+    gen = torch.Generator().manual_seed(ns)
+    bufs = [make(s, gen) if make else torch.randn(*s, generator=gen) * 1e-3 for s in shapes]
+    params = [torch.zeros(s, device="cuda") for s in shapes]
+    grads = [b.cuda() for b in bufs]
+    _ops().muon_fused_step(params, grads, [torch.zeros_like(p) for p in params], 0.95, 5.0, 0.0, ns)
+    for b, p in zip(bufs, params):
+        x = b.double().numpy()
+        x = muon_oracle.newton_schulz((x if x.shape[0] <= x.shape[1] else x.T) / (b.double().norm().item() + 1e-7), ns, x.dtype.type)
+        got = -p.cpu().double()
+        d = (got if b.shape[0] <= b.shape[1] else got.T) - torch.from_numpy(x)
+        assert d.norm() <= bound * torch.from_numpy(x).norm(), (tuple(b.shape), (d.norm() / torch.from_numpy(x).norm()).item())
+
+
+def _power_law(shape, gen):
+    r = min(shape)
+    u, v = (torch.linalg.qr(torch.randn(n, r, dtype=torch.float64, generator=gen))[0] for n in shape)
+    return ((u / torch.arange(1, r + 1)) @ v.T).float()
+
+
+def _scaled_rows(shape, gen):
+    return torch.randn(*shape, generator=gen) * 10 ** (-4 * torch.rand(shape[0], 1, generator=gen))
+
+
+# The first rounding, of the momentum to bf16 (2^-9 at most of every entry, 1.7e-3 in the 2-norm), is an error spread over all
+# directions; relative to a singular value of 1/r of the largest it is larger by that much and grows with it, so a power law's
+# smallest directions carry several times the relative error of rows of one scale.  The bounds are twice what the iteration
+# with a Gram matrix formed every time, in bf16, shows (0.014 and 0.011 here); a missing factor or product shows as 0.1 and more.
+@pytest.mark.parametrize("make, bound", [(_power_law, 0.03), (_scaled_rows, 0.02)], ids=["power_law", "rows"])
+def test_spectra(make, bound):
+    _compare([(64, 3000), (100, 4000)], 5, make, bound)
+    _compare([(3000, 64)], 5, make, bound)
+
+
+def test_rule():
+    assert _cabi.muon_stages_for([(1024, 1024)] * 24) == 5 and _cabi.muon_stages_for([(1024, 4096)] * 24) == 2
+    assert _cabi.muon_stages_for([(200, 800)]) == 5 and _cabi.muon_stages_for([(100, 4000)]) == 2
+    assert [_cabi.muon_stages_for([(1024, 4096)], ns) for ns in (0, 1)] == [0, 1]
+
+
+def test_not_finite_and_zero():
+    """A gradient that is not finite makes the whole parameter so, as in the reference; zeros stay zeros."""
+    shapes = [(64, 3000), (64, 3000), (64, 3000)]
+    grads = [torch.randn(s, device="cuda") * 1e-3 for s in shapes]
+    grads[0][3, 5] = float("nan")
+    grads[1].zero_()
+    params = [torch.ones(s, device="cuda") for s in shapes]
+    _ops().muon_fused_step(params, grads, [torch.zeros(s, device="cuda") for s in shapes], 0.95, 0.02, 0.0, 5)
+    assert bool(torch.isnan(params[0]).all()) and bool((params[1] == 1).all()) and bool(torch.isfinite(params[2]).all())
