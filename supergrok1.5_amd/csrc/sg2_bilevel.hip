@@ -285,8 +285,9 @@ constexpr int AB = 4;                   // steps per block
 constexpr int FLUSH_TILES = 64;         // tiles between two writes of the sums
 constexpr int ADJ_STRIDE = 4 * DI + 4;  // per step: (dt, dt - dt0, dt * x-branch, d y) of the 16 columns; later (d x-branch, d dt, d z, out)
 constexpr int BC_STRIDE = 4 * HP + 4;   // per step: (B even, B odd, C even, C odd) of the 8 pairs
-constexpr int SUM_STRIDE = AT + 4;      // per column: sums over the pairs of every step
-constexpr int IN_STRIDE = 17;           // per step: g, s, 1, d ctx[8]
+constexpr int SUM_STRIDE = AT + 4;      // per input: its values at the steps
+constexpr int BLK_STRIDE = 64 * 4 + 4;  // per block of steps (the four blocks' reads of a column's step fall on different banks)
+constexpr int IN_STRIDE = 13;           // per step: g, s, 1, d ctx[8]
 typedef float adj_f32x4 __attribute__((ext_vector_type(4)));
 
 // sigmoid and the derivative of SiLU as cubics around c (as sg2_softplus_taylor, sg2_silu_taylor)
@@ -307,17 +308,26 @@ __device__ __forceinline__ void dsilu_taylor(float c, float t[4]) {
 }
 __device__ __forceinline__ float cubic(const adj_f32x4 t, float d) { return sg_fma(sg_fma(sg_fma(t[3], d, t[2]), d, t[1]), d, t[0]); }
 
+// Bound by the vector ALU: about 2500 instructions a tile of 16 steps at 4.1 clocks each and SIMD (two waves), of 20 600 clocks a
+// tile blocks 12 900, states at their starts 2950, part 3 2700, projections 1650.  So that nothing of the tile loop spills at 256
+// registers, what only part 3 needs lies in LDS (matrix accumulators; the pair sums where the states of their block were) and
+// addresses are formed where they are used: a reload, or the spill of a prefetched value, waits for every load before it, and
+// that was four memory latencies a tile.  25 M elements: the pass 33.6 -> 31.2 ms; 0.42 M: 1267 -> 1227 us.
 template <bool SCAN_GRADS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adjoint(Plan pl, AdjIO io) {      // SCAN_GRADS: the gradient of the gated outputs comes in instead of that of the contexts
     static_assert(AT == 16 && DI == 16 && DS == 16 && HP == 8 && DM == 8 && AB == 4, "lane roles");
     __shared__ __attribute__((aligned(16))) float s_a[AT * ADJ_STRIDE];
     __shared__ __attribute__((aligned(16))) float s_b[AT * BC_STRIDE];
-    __shared__ __attribute__((aligned(16))) float s_y[DI * SUM_STRIDE], s_q[DI * SUM_STRIDE], s_d[DI * SUM_STRIDE];     // y, d / d (dt * x-branch), d dt but for that
-    __shared__ __attribute__((aligned(16))) float s_in[AT * IN_STRIDE], s_gt[4 * SUM_STRIDE];      // inputs per step; g, s, 1 per row
-    __shared__ __attribute__((aligned(16))) float s_h[(AT / AB) * 64 * 4];        // the lanes' states at the starts of the blocks
+    __shared__ __attribute__((aligned(16))) float s_in[AT * IN_STRIDE + 4], s_gt[4 * SUM_STRIDE];      // inputs per step; g, s, 1 per row
+    // per block of steps the lanes' states at its start; once these are read, the sums over the pairs of its steps: y,
+    // d / d (dt * x-branch), d dt but for that, [16 columns][4 steps] each
+    __shared__ __attribute__((aligned(16))) float s_h[(AT / AB) * BLK_STRIDE];
+    // sums of part 3 (rows x (g, s, 1, d ctx): d x-branch, d dt, d z, out), a lane's matrix accumulators
+    __shared__ __attribute__((aligned(16))) float s_acc[4 * 64 * 4];
     __shared__ __attribute__((aligned(16))) float s_k[2 * 64 * 4];                // gate and d out of the lanes' steps and rows, for part 3
     __shared__ __attribute__((aligned(16))) float s_coef[SG2_COMP_GROUPS * DI * 4];   // composed triples, D beside the x-branch's
     __shared__ __attribute__((aligned(16))) float s_tay[4 * DI * 4];              // dt, its derivative, gate, its derivative
+    // (together 20 432 bytes: eight workgroups share a CU's 160 KB)
 
     const int lane = threadIdx.x, dir = blockIdx.y;
     const int st = lane & 15, rg = lane >> 4;
@@ -344,7 +354,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             dsilu_taylor(comp[(SG2_COMP_Z * DI + lane) * 3 + 2], t);
             *reinterpret_cast<adj_f32x4*>(s_tay + (3 * DI + lane) * 4) = adj_f32x4{t[0], t[1], t[2], t[3]};
         }
-        for (int i = lane; i < AT * IN_STRIDE; i += 64) s_in[i] = 0.0f;
+        for (int i = lane; i < AT * IN_STRIDE + 4; i += 64) s_in[i] = 0.0f;
         for (int i = lane; i < 4 * SUM_STRIDE; i += 64) s_gt[i] = 0.0f;
         __syncthreads();
     }
@@ -370,7 +380,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const adj_f32x4 zero4 = adj_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     float al_e[2] = {0.0f, 0.0f}, al_o[2] = {0.0f, 0.0f}, rope[2] = {0.0f, 0.0f};
     adj_f32x4 aBe = zero4, aBo = zero4, aCe = zero4, aCo = zero4;
-    adj_f32x4 a16[4] = {zero4, zero4, zero4, zero4};     // rows x (g, s, 1, d ctx): d x-branch, d dt, d z, out
+    adj_f32x4* const acc16 = reinterpret_cast<adj_f32x4*>(s_acc) + lane;
+#pragma unroll
+    for (int q = 0; q < 4; q++) acc16[64 * q] = zero4;
     float accD[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 
     // this wave's sums -> its row of the partials buffer, every FLUSH_TILES tiles: one chain of additions over all of a
@@ -385,6 +397,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         float* const g_rope = g_alog + DI * DS;
         float* const g_D = g_rope + DI * HP;
         float* const g_wout = g_D + DI;
+        adj_f32x4 a16[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) { a16[q] = acc16[64 * q]; acc16[64 * q] = zero4; }
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int j = jl + 8 * h;
@@ -422,7 +437,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         }
         aBe = aBo = aCe = aCo = zero4;
 #pragma unroll
-        for (int q = 0; q < 4; q++) { a16[q] = zero4; accD[q] = 0.0f; }
+        for (int q = 0; q < 4; q++) accD[q] = 0.0f;
         unflushed = 0;
     };
 
@@ -438,23 +453,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     struct Inputs { uint32_t key; int32_t val; float s, d0, d1; adj_f32x4 ds, h; };
     auto request = [&](int u0, bool with_state) {
         Inputs in = {0, 0, 0.0f, 0.0f, 0.0f, zero4, zero4};
-        const int u = u0 + st;
-        if (u < N) {
-            const int t = dir ? N - 1 - u : u;
-            in.key = pl.keys[0][off + t];
-            in.val = pl.vals[0][off + t];
-            if (has_s) in.s = pl.ssorted[off + t];
-            if (SCAN_GRADS) {
-                in.ds = *reinterpret_cast<const adj_f32x4*>(dscan + (size_t)u * DI + 4 * rg);
-            } else {
-                const int at = in_order ? t : min(in.val & 0x7fffffff, N - 1);
-                in.d0 = dctx[(size_t)at * DM + rg];
-                in.d1 = dctx[(size_t)at * DM + 4 + rg];
+        // (opaque: a lane's addresses, formed ahead of the loop, would spill, and their reload waits for every load before it)
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int st = ln & 15, rg = ln >> 4, u = min(u0 + st, N - 1);      // (steps past the end: unpack and project leave them out)
+        const int t = dir ? N - 1 - u : u;
+        in.key = pl.keys[0][off + t];
+        in.val = pl.vals[0][off + t];
+        if (has_s) in.s = pl.ssorted[off + t];
+        if (SCAN_GRADS) {
+            in.ds = *reinterpret_cast<const adj_f32x4*>(dscan + (size_t)u * DI + 4 * rg);
+        } else {
+            int at = t;
+            if (!in_order) {      // (kept a branch: a choice would wait for the index here)
+                asm volatile("");
+                at = min(in.val & 0x7fffffff, N - 1);
             }
+            in.d0 = dctx[(size_t)at * DM + rg];
+            in.d1 = dctx[(size_t)at * DM + 4 + rg];
         }
         if (with_state) {
             const float* ht = pl.htile + ((size_t)dir * htile_count(pl.total, pl.P) + htile_index(off, ti, u0)) * 2 * SCAN_THREADS;
-            in.h = adj_f32x4{ht[lane], ht[SCAN_THREADS + lane], ht[64 + lane], ht[SCAN_THREADS + 64 + lane]};
+            in.h = adj_f32x4{ht[ln], ht[SCAN_THREADS + ln], ht[64 + ln], ht[SCAN_THREADS + 64 + ln]};
         }
         return in;
     };
@@ -628,13 +648,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                                 hh[2 * h + 1] = sg_fma(ao, ro, a[2] * bc[1]);
                             }
                         }
-                        sh[(k0 / AB + 1) * 64] = hh;
+                        sh[(k0 / AB + 1) * (BLK_STRIDE / 4)] = hh;
                     }
                 }
                 // ---- the blocks, last first (a ragged tile: its steps past the end leave lambda alone and add nothing, their
                 // dt, x-branch and d y being 0)
                 Step o = step_at(AT - AB);
-                adj_f32x4 h_next = sh[(AT / AB - 1) * 64];
+                adj_f32x4 h_next = sh[(AT / AB - 1) * (BLK_STRIDE / 4)];
 #pragma unroll 1
                 for (int k0 = AT - AB; k0 >= 0; k0 -= AB) {
                     const adj_f32x4 h0 = h_next;
@@ -664,13 +684,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                     const adj_f32x4 gt = *reinterpret_cast<const adj_f32x4*>(s_gt + (lane & 3) * SUM_STRIDE + k0);
                     fetched_here();
                     block_pair_sums<HP>(y);
+                    // lanes p = 0 hold the sums of column jl, p = 4 those of column jl + 8 (the block's state has been read)
+                    adj_f32x4* const sums = reinterpret_cast<adj_f32x4*>(s_h + k0 / AB * BLK_STRIDE) + jl + 2 * p;
+                    if ((p & 3) == 0) sums[0] = adj_f32x4{y[0], y[1], y[2], y[3]};
                     float q[8], dd[8];
 #pragma unroll
                     for (int u = AB - 1; u >= 0; u--) {
                         float tBe = 0.0f, tBo = 0.0f, tCe = 0.0f, tCo = 0.0f;
                         const Step now = o;
                         o = step_at(max(u > 0 ? k0 + u - 1 : k0 - AB, 0));
-                        if (u == 0) h_next = sh[max(k0 / AB - 1, 0) * 64];
+                        if (u == 0) h_next = sh[max(k0 / AB - 1, 0) * (BLK_STRIDE / 4)];
                         fetched_here();
                         const adj_f32x4 bc = now.bc;
 #pragma unroll
@@ -706,20 +729,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                     }
                     block_pair_sums<HP>(q);
                     block_pair_sums<HP>(dd);
-                    if ((p & 3) == 0) {      // lanes p = 0 hold the sums of column jl, p = 4 those of column jl + 8
-                        const int at = (jl + 2 * p) * SUM_STRIDE + k0;
-                        *reinterpret_cast<adj_f32x4*>(s_y + at) = adj_f32x4{y[0], y[1], y[2], y[3]};
-                        *reinterpret_cast<adj_f32x4*>(s_q + at) = adj_f32x4{q[0], q[1], q[2], q[3]};
-                        *reinterpret_cast<adj_f32x4*>(s_d + at) = adj_f32x4{dd[0], dd[1], dd[2], dd[3]};
+                    if ((p & 3) == 0) {
+                        sums[DI] = adj_f32x4{q[0], q[1], q[2], q[3]};
+                        sums[2 * DI] = adj_f32x4{dd[0], dd[1], dd[2], dd[3]};
                     }
                 }
                 __syncthreads();
                 // ---- 3
-                const adj_f32x4 gate = reinterpret_cast<adj_f32x4*>(s_k)[lane], dout = reinterpret_cast<adj_f32x4*>(s_k)[64 + lane];
+                int ln = lane;         // (opaque, as in request)
+                asm volatile("" : "+v"(ln));
+                const int st = ln & 15, rg = ln >> 4;
+                const float* const sums = s_h + (st >> 2) * BLK_STRIDE + (st & 3);
+                const adj_f32x4 gate = reinterpret_cast<adj_f32x4*>(s_k)[ln], dout = reinterpret_cast<adj_f32x4*>(s_k)[64 + ln];
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
                     const int row = 4 * rg + v;
-                    const float yv = s_y[row * SUM_STRIDE + st], qb = s_q[row * SUM_STRIDE + st], ddr = s_d[row * SUM_STRIDE + st];
+                    const float yv = sums[AB * row], qb = sums[AB * (DI + row)], ddr = sums[AB * (2 * DI + row)];
                     const float dt = s_a[st * ADJ_STRIDE + 4 * row];
                     const adj_f32x4 cd = *reinterpret_cast<const adj_f32x4*>(s_coef + (SG2_COMP_DT * DI + row) * 4);
                     const adj_f32x4 cz = *reinterpret_cast<const adj_f32x4*>(s_coef + (SG2_COMP_Z * DI + row) * 4);
@@ -745,6 +770,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                     *reinterpret_cast<adj_f32x4*>(s_a + st * ADJ_STRIDE + 4 * row) = out;
                 }
                 __syncthreads();
+                adj_f32x4 a16[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) a16[q] = acc16[64 * q];
 #pragma unroll
                 for (int t = 0; t < AT / 4; t++) {
                     const adj_f32x4 d = *reinterpret_cast<const adj_f32x4*>(s_a + (4 * t + rg) * ADJ_STRIDE + 4 * st);      // step 4 t + rg, row st
@@ -752,6 +780,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
                     for (int q4 = 0; q4 < 4; q4++) a16[q4] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[q4], in16, a16[q4], 0, 0, 0);
                 }
+#pragma unroll
+                for (int q = 0; q < 4; q++) acc16[64 * q] = a16[q];
                 __syncthreads();
             };
             if (fast) walk(std::true_type{});
@@ -763,8 +793,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     auto set_tensor = [&](int i) {
         ti = i;
         const TensorDev& T = pl.tensors[i];
-        N = T.numel;
-        off = T.off;
+        N = __builtin_amdgcn_readfirstlane(T.numel);
+        off = __builtin_amdgcn_readfirstlane(T.off);
         has_s = __builtin_amdgcn_readfirstlane(pl.sharp_nonzero[i]) != 0;
         dctx = io.d_ctx ? io.d_ctx + ((size_t)dir * pl.total + off) * DM : nullptr;
         dscan = io.d_scan[dir] ? io.d_scan[dir] + (size_t)off * DI : nullptr;
