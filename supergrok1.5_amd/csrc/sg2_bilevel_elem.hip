@@ -31,8 +31,7 @@
 //     another interval of one of their experts - look the interval up in the tables and move their (w, w g) to its bin
 //     with atomics.  They are the largest of a tensor and come together, sixteen a lane and head, so a head's exceptions
 //     are dealt to all lanes of the wave.  (A lane going through its own one by one waited twice for
-//     memory each time: in a call of 0.42 M elements the wave with the most, 340 a head, took 330 us, 150 being the
-//     median, and the launch 370; now 310.  Two jobs a lane
+//     memory each time: 370 us instead of 310 in a call of 0.42 M elements whose small tensors lay with few waves.  Two jobs a lane
 //     at a time took 280 there, but the registers they need are missed by every tile: 1.3 % of a pass over 25 M.  With all of a trained net's exceptions taken by LDS atomics, in element
 //     order, they were half of the pass.)
 //     (An element exactly on a threshold counts the unit as inactive on both sides; forward value and gradient use
@@ -46,9 +45,12 @@
 // reference's atomicAdd).
 //
 // Bound by the vector ALU (about 5000 instructions per wave and tile, two thirds of them the fixed multiply-adds of the
-// net and its derivative).  Measured on 25 M elements with module-initialised experts after some meta steps: 8.4 ms, 47 ms
-// as one lane per element of a 256-lane workgroup that summed the outer products lane by lane from LDS; on 0.42 M elements
-// 0.31 ms instead of 1.1.  (The net's products as 4 x 4 x 1 matrix instructions with the weights in LDS or in memory took as
+// net and its derivative; a tile takes 84 000 clocks beside the other wave of its SIMD, of which the experts' 64 lines 8500,
+// the sums of routing weights 17 000, scores and best four 13 000).  Measured on 25 M elements with module-initialised experts
+// after some meta steps: 7.8 ms (9.2 with the experts' lines read pick by pick, the matrix instructions' operands not ahead of
+// them, and a tile's indexes not before the tile), 47 ms as one lane per element of a 256-lane workgroup that summed the
+// outer products lane by lane from LDS; on 0.42 M elements 0.23 ms, 0.29 before those and with a small tensor's tiles side by
+// side, 1.1 at first.  (The net's products as 4 x 4 x 1 matrix instructions with the weights in LDS or in memory took as
 // long, with the bins in LDS longer on large calls: registers are what there is least of.)
 #include "sg2_internal.hpp"
 
@@ -263,7 +265,7 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 
     for (int i = tid; i < N_BINS; i += BE_THREADS) bins[i] = 0.0f;
     for (int i = tid; i < KEY_FLOATS; i += BE_THREADS) s_keys[i] = i < KEY_FLOATS / 2 ? a.W.w[W_KEYS_A][i] : a.W.w[W_KEYS_B][i - KEY_FLOATS / 2];
-    for (int i = lane; i < 64 * XW + R_FLOATS; i += 64) s_x[i] = 0.0f;     // rows are read whole: no NaN may lie in what was never written
+    for (int i = lane; i < (64 * XW + R_FLOATS) / 4; i += 64) reinterpret_cast<be_f32x4*>(s_x)[i] = be_f32x4{0.0f, 0.0f, 0.0f, 0.0f};     // rows are read whole: no NaN may lie in what was never written
     __syncthreads();
 
     const sg::cfloat_p Wz = sg::as_const(a.W.w[W_GRU_WZ]), bz = sg::as_const(a.W.w[W_GRU_BZ]);
@@ -282,22 +284,46 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     const int kb = (lane >> 2) % 12, kb6 = kb % 6;
     const int key_a = (kb / 6) * KW + kb6 * 4 + (lane & 3), key_b = (kb / 6) * KW + 24 + (kb6 / 3) * 4 + (lane & 3);
 
+    // sums over the tile's elements of (rows of d, DW floats each) (x) (rows of x), four elements a step, operands two steps ahead
+    auto outer_sums = [&](be_f32x4 (&acc)[2]) {
+        const float* d = s_r + lk * DW + li;
+        const float* x = s_x + lk * XW + li;
+        float dv[2][2], x0[2][2], x1[2][2];
+        auto fetch = [&](int t0, int q) {
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                dv[q][t] = d[4 * (t0 + t) * DW];
+                x0[q][t] = x[4 * (t0 + t) * XW];
+                x1[q][t] = x[4 * (t0 + t) * XW + 16];
+            }
+            asm volatile("" ::: "memory");
+        };
+        auto sum = [&](int q) {
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(dv[q][t], x0[q][t], acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(dv[q][t], x1[q][t], acc[1], 0, 0, 0);
+            }
+        };
+        fetch(0, 0);
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            if (q < 7) fetch(2 * q + 2, (q + 1) & 1);
+            sum(q & 1);
+        }
+    };
+
     // the four experts whose sums this lane holds in cen: first index 4 lk + v, second index li
     const bool owner = lane < 48 && li < PK;
     float x_held = -1.0f;                                 // reference magnitude of the lines in s_tab (< 0: none yet)
     auto reference = [](float x, int neg) { return neg ? -x : __builtin_fmaxf(x, 1.40129846e-45f); };      // (+0 stands for the interval just above zero)
     auto line_at = [&](const Thresholds& th, int e, float r) {       // the expert's line at r and the borders of its interval
         const float2 ab = reinterpret_cast<const float2*>(lines)[e * NBIN + th.below(r)];
-        return make_float4(ab.x, ab.y, th.low(r), th.high(r));
+        const float high = th.high(r);
+        return make_float4(ab.x, ab.y, th.low(r), high == high ? high : -__builtin_inff());      // (a NaN border holds nothing: minima would drop it)
     };
     auto move_reference = [&](float x) {
-        if (x_held < 0.0f) {
-#pragma unroll 1
-            for (int t = lane; t < 2 * NE; t += 64) {
-                const int neg = t >= NE ? 1 : 0, e = t - neg * NE;
-                s_tab[t] = line_at(Thresholds(ths, e), e, reference(x, neg));
-            }
-        } else if (!FLAT) {
+        if (!FLAT) {
             unsigned stale = 0u;             // bit 2 v + neg: x lies in another interval of expert v on that side
             if (owner) {
 #pragma unroll
@@ -331,10 +357,35 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
         x_held = x;
         wave_sync();
     };
+    // the first lines of a wave, everything requested at once
+    auto first_reference = [&](float x) {
+        constexpr int ROUNDS = (2 * NE + 63) / 64;
+        float4 line[ROUNDS];
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) {
+            const int t = min(r * 64 + lane, 2 * NE - 1), neg = t >= NE ? 1 : 0, e = t - neg * NE;
+            line[r] = line_at(Thresholds(ths, e), e, reference(x, neg));
+        }
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++)
+            if (r * 64 + lane < 2 * NE) s_tab[r * 64 + lane] = line[r];
+        x_held = x;
+        wave_sync();
+    };
 
     const int ntiles = FLAT ? (a.total + 63) / 64 : pl.elem_tiles * (ELEM_TILE / 64);
     const int nwaves = (int)gridDim.x * BE_WAVES, wv = (int)blockIdx.x * BE_WAVES + wave;
     int tile0 = (int)((int64_t)ntiles * wv / nwaves), tile1 = (int)((int64_t)ntiles * (wv + 1) / nwaves), step = 1;
+    if ((int)gridDim.x == BE_MAX_GROUPS && ntiles < 16 * nwaves) {
+        // Few tiles a wave: two waves share a SIMD, in the order of dispatch wv and wv + nwaves / 2, so an equal part is dealt to
+        // every such pair and halved between its waves.  (Dealt wave by wave, both had one tile more than the others or neither:
+        // 0.42 M elements are 3.2 tiles a wave, and the launch, 233 us, waited for a SIMD with eight; 226 now.  Where a wave
+        // has many the odd tile is nothing, and neighbours on one SIMD cost: 25 M elements, 191 a wave, 7.8 ms -> 8.7.)
+        const int half = nwaves / 2, pair = wv % half, second = wv / half;
+        const int p0 = (int)((int64_t)ntiles * pair / half), p1 = (int)((int64_t)ntiles * (pair + 1) / half), mid = p0 + (p1 - p0 + 1) / 2;
+        tile0 = second ? mid : p0;
+        tile1 = second ? p1 : mid;
+    }
     const bool plain = !FLAT && !sorted_rows(pl);
     if (plain) {
         static_assert(PLAIN_TILE == 64 * BE_WAVES, "a tile of 64 per wave");
@@ -345,6 +396,35 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     const float kscale = a.rescale / (float)NH;
     sg::Seg seg = {-1, 0, 0};
     float cot_norm = 0.0f;
+    // The tensor at a tile index, the tile's first element there and how many it holds; 0 where the index has no tile.  A tensor's
+    // last ELEM_TILE elements are 16 indexes whatever there is of them, their tiles spread evenly over these: the tiles of a
+    // small tensor, whose elements are mostly exceptions (99 of them two or three times a tile's usual time), then fall to
+    // waves with little else.
+    auto place = [&](int tile, int& start) {
+        constexpr int PER = ELEM_TILE / 64;
+        const int et = tile / PER, at = tile % PER;
+        if (et >= seg.end) {
+            seg = sg::find_seg(sg::as_const(pl.elem_tile_prefix), pl.P, et);
+            cot_norm = a.norms ? a.norms[seg.i] : 0.0f;
+        }
+        const int first = (et - seg.first) * ELEM_TILE, left = pl.tensors[seg.i].numel - first, tiles = min(PER, (left + 63) / 64);
+        const int here = at * tiles / PER;
+        start = first + here * 64;
+        return at > 0 && (at - 1) * tiles / PER == here ? 0 : left - here * 64;
+    };
+    if (FLAT || plain) {
+        if (tile0 < tile1) first_reference(0.0f);
+    } else {
+        for (int start; tile0 < tile1; tile0++) {
+            const int cnt = place(tile0, start);
+            if (cnt <= 0) continue;
+            first_reference(sg_i2f((int32_t)pl.keys[0][pl.tensors[seg.i].off + start + min(cnt - 1, 32)]));
+            break;
+        }
+    }
+    int32_t next_val = 0;                 // of the lane's element in the next tile, requested a tile ahead (the gathers wait for it)
+    uint32_t next_key = 0u;
+    bool have_next = false;
     for (int tile = tile0; tile < tile1; tile += step) {
         // every lane runs the element code (the wave works on whole tiles): lanes past the end redo the last element with a
         // zero cotangent, which zeroes everything they add, and store nothing
@@ -358,7 +438,6 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             at = out_at = valid ? tile * 64 + lane : a.total - 1;
             g = a.g[at]; s = a.s[at]; cot = valid ? a.cot[at] : 0.0f;
             h4 = reinterpret_cast<const float4*>(a.gru)[at];
-            if (x_held < 0.0f) move_reference(0.0f);
         } else if (plain) {
             valid = tile * 64 + lane < a.total;
             at = out_at = valid ? tile * 64 + lane : a.total - 1;
@@ -377,21 +456,16 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             cot = valid ? cot : 0.0f;
             const be_f32x4 hv = ((const SG_GLOBAL be_f32x4*)T.gru)[orig];
             h4 = make_float4(hv[0], hv[1], hv[2], hv[3]);
-            if (x_held < 0.0f) move_reference(0.0f);
         } else {
-            const int et = tile / (ELEM_TILE / 64);
-            if (et >= seg.end) {
-                seg = sg::find_seg(sg::as_const(pl.elem_tile_prefix), pl.P, et);
-                cot_norm = a.norms ? a.norms[seg.i] : 0.0f;
-            }
+            int start;
+            const int cnt = place(tile, start);
+            if (cnt <= 0) continue;
             const TensorDev& T = pl.tensors[seg.i];
-            const int start = (et - seg.first) * ELEM_TILE + (tile % (ELEM_TILE / 64)) * 64;
-            const int cnt = T.numel - start;
-            if (cnt <= 0) continue;          // an empty rest of a tensor's last tile
             valid = lane < cnt;
             at = T.off + start + (valid ? lane : cnt - 1);
-            const int32_t val = pl.vals[0][at];
-            const uint32_t key = pl.keys[0][at];
+            int32_t val = next_val;
+            uint32_t key = next_key;
+            if (!have_next) { val = pl.vals[0][at]; key = pl.keys[0][at]; }
             const int orig = min(val & 0x7fffffff, T.numel - 1);
             out_at = T.off + orig;
             // the sort's values, except where it put 0 for an entry that is not finite: those stay what they are
@@ -407,6 +481,12 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             cot = valid ? cot : 0.0f;
             const be_f32x4 hv = ((const SG_GLOBAL be_f32x4*)T.gru)[orig];
             h4 = make_float4(hv[0], hv[1], hv[2], hv[3]);
+            have_next = cnt > 64 && tile + 1 < tile1;
+            if (have_next) {
+                const int then = T.off + start + 64 + min(lane, cnt - 65);
+                next_val = pl.vals[0][then];
+                next_key = pl.keys[0][then];
+            }
             move_reference(__shfl(sg_abs(g), min(cnt - 1, 32), 64));
         }
         float* const xrow = s_x + lane * XW;
@@ -511,19 +591,42 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             }
             wave_sync();
             // ---- experts: the line of each at this element's side of zero, where its interval holds g
+            // (The sixteen records of a lane are requested four at a time, whole and one row ahead of their use, and the borders are
+            // compared together: chosen pick by pick, they became sixteen branches with two waits for LDS each.)
             float ra[TOPK] = {0.f, 0.f, 0.f, 0.f}, rb[TOPK] = {0.f, 0.f, 0.f, 0.f};
             unsigned other = 0u;                     // picks whose interval is another one
+            {
+                const be_f32x4* const ta = reinterpret_cast<const be_f32x4*>(s_tab) + side;
+                be_f32x4 t[2][TOPK];
+                auto fetch = [&](int ia) {
+                    const be_f32x4* const row = ta + idx[0][ia] * PK;
 #pragma unroll
-            for (int ia = 0; ia < TOPK; ia++) {
-                const float4* ta = s_tab + side + idx[0][ia] * PK;
+                    for (int ib = 0; ib < TOPK; ib++) t[ia & 1][ib] = row[idx[1][ib]];
+                };
+                fetch(0);
 #pragma unroll
-                for (int ib = 0; ib < TOPK; ib++) {
-                    const float4 t = ta[idx[1][ib]];
-                    const bool in = t.z < g && g <= t.w;
-                    const float out = in ? sg_fma(t.x, g, t.y) : 0.0f;
-                    other |= in ? 0u : 1u << (ia * TOPK + ib);
-                    ra[ia] = sg_fma(wgt[1][ib], out, ra[ia]);
-                    rb[ib] = sg_fma(wgt[0][ia], out, rb[ib]);
+                for (int ia = 0; ia < TOPK; ia++) {
+                    if (ia + 1 < TOPK) fetch(ia + 1);
+                    be_f32x4 (&u)[TOPK] = t[ia & 1];
+                    asm volatile("" : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]));
+                    float out[TOPK];
+#pragma unroll
+                    for (int ib = 0; ib < TOPK; ib++) out[ib] = sg_fma(u[ib][0], g, u[ib][1]);
+                    const float low = __builtin_fmaxf(__builtin_fmaxf(u[0][2], u[1][2]), __builtin_fmaxf(u[2][2], u[3][2]));
+                    const float high = __builtin_fminf(__builtin_fminf(u[0][3], u[1][3]), __builtin_fminf(u[2][3], u[3][3]));
+                    if (__builtin_amdgcn_ballot_w64(!(low < g && g <= high)) != 0) {
+#pragma unroll
+                        for (int ib = 0; ib < TOPK; ib++) {
+                            const bool in = u[ib][2] < g && g <= u[ib][3];
+                            out[ib] = in ? out[ib] : 0.0f;
+                            other |= in ? 0u : 1u << (ia * TOPK + ib);
+                        }
+                    }
+#pragma unroll
+                    for (int ib = 0; ib < TOPK; ib++) {
+                        ra[ia] = sg_fma(wgt[1][ib], out[ib], ra[ia]);
+                        rb[ib] = sg_fma(wgt[0][ia], out[ib], rb[ib]);
+                    }
                 }
             }
             if (!valid) other = 0u;
@@ -683,10 +786,24 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
                 for (int dd = 0; dd < DM; dd++) krow[2 * PK + dd] = query[dd];
                 wave_sync();
+                // (operands eight steps ahead of the instructions that take them)
                 auto key_sums = [&](be_f32x4& acc) {
-#pragma unroll 8
-                    for (int t = 0; t < 32; t++)
-                        acc = __builtin_amdgcn_mfma_f32_4x4x1f32(s_r[2 * t * KW + key_a], s_r[2 * t * KW + key_b], acc, 0, 0, 0);
+                    float ka[2][8], kv[2][8];
+                    auto fetch = [&](int t0, int q) {
+#pragma unroll
+                        for (int t = 0; t < 8; t++) { ka[q][t] = s_r[2 * (t0 + t) * KW + key_a]; kv[q][t] = s_r[2 * (t0 + t) * KW + key_b]; }
+                        asm volatile("" ::: "memory");
+                    };
+                    auto sum = [&](int q) {
+#pragma unroll
+                        for (int t = 0; t < 8; t++) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(ka[q][t], kv[q][t], acc, 0, 0, 0);
+                    };
+                    fetch(0, 0);
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        if (q < 3) fetch(8 * q + 8, (q + 1) & 1);
+                        sum(q & 1);
+                    }
                 };
                 if (hh == 0) key_sums(kacc[0]);
                 else if (hh == 1) key_sums(kacc[1]);
@@ -703,17 +820,8 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
                 for (int dd = 0; dd < DM; dd++) { drow[dd] = dq_even[dd]; drow[DM + dd] = dq[dd]; }
                 wave_sync();
-                auto query_sums = [&](be_f32x4 (&acc)[2]) {
-#pragma unroll 4
-                    for (int t = 0; t < 16; t++) {
-                        const float av = s_r[(4 * t + lk) * DW + li];
-                        const float* xr = s_x + (4 * t + lk) * XW + li;
-                        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, xr[0], acc[0], 0, 0, 0);
-                        acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, xr[16], acc[1], 0, 0, 0);
-                    }
-                };
-                if (hh == 1) query_sums(qacc[0]);
-                else query_sums(qacc[1]);
+                if (hh == 1) outer_sums(qacc[0]);
+                else outer_sums(qacc[1]);
                 wave_sync();
             }
         }
@@ -758,13 +866,7 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
             for (int j = 0; j < GH; j++) { drow[j] = dpz[j]; drow[GH + j] = dpr[j]; drow[2 * GH + j] = dph[j]; xrow[X_HN + j] = rg[j] * h[j]; }
             wave_sync();
-#pragma unroll 4
-            for (int t = 0; t < 16; t++) {
-                const float av = s_r[(4 * t + lk) * DW + li];
-                const float* xr = s_x + (4 * t + lk) * XW + li;
-                gacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, xr[0], gacc[0], 0, 0, 0);
-                gacc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, xr[16], gacc[1], 0, 0, 0);
-            }
+            outer_sums(gacc);
             wave_sync();
         }
     }

@@ -10,12 +10,14 @@ from grokking_optimizers.mamba3_peer_metanet import Mamba3PEERMetaNet
 
 pytestmark = pytest.mark.gpu
 
-SIZES = {"tiles": [1, 63, 64, 65, 1023, 1024, 1025], "one_element": [1], "many": [7] * 70 + [200_003]}
+# "rests": every number of tiles that a tensor's last 1024 elements can hold
+SIZES = {"rests": [64 * k - 31 for k in range(1, 17)] + [1024 + 64 * 3], "tiles": [1, 63, 64, 65, 1023, 1024, 1025], "one_element": [1], "many": [7] * 70 + [200_003]}
 
 
 @pytest.mark.parametrize("validation", [False, True])
 @pytest.mark.parametrize("sizes,dtype,eh,theta,sharp", [
     ("tiles", torch.float32, 16, 0.0, "none"), ("tiles", torch.bfloat16, 4, 1e-3, "some"), ("one_element", torch.float32, 16, 1e-3, "some"),
+    ("rests", torch.float32, 16, 1e-3, "some"),
     ("many", torch.float32, 16, 1e-3, "nan"), ("many", torch.float16, 16, 1.0, "none")])
 def test_pass_equals_separate_calls(sizes, dtype, eh, theta, sharp, validation, monkeypatch):
     torch.manual_seed(3)
