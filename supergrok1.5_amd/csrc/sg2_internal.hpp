@@ -102,15 +102,14 @@ struct Plan {
     const int* sort_tile_prefix;   // [P+1] tiles of SORT_TILE keys
     const int* chunk_prefix;       // [P+1] scan chunks
     const int* wchunk_prefix;      // [P+1] scan chunks that need a summary (all but the last of a tensor)
-    const int* norm_tile_prefix;   // [P+1] tiles of norm_tile elements (clipping calls)
+    const int* norm_tile_prefix;   // [P+1] norm tiles (clipping calls)
     int P;
     int total;                     // sum of numel
-    int elem_tiles, sort_tiles, chunks, wchunks, norm_tiles;
+    int elem_tiles, sort_tiles, chunks, wchunks;
     int sort_tile;                 // SORT_TILE or SORT_TILE_SMALL
     int sort_widest;               // sort tiles of the largest tensor
     bool half_grads;               // every tensor's gradient is of a 16-bit type: two sort passes instead of four
-    int norm_tile;
-    double* norm_partials;         // [norm_tiles] sums of squares
+    double* norm_partials;         // sums of squares of the norm tiles (written by k_tables)
     float* gscale;                 // [P] factor of each tensor's gradients in a clipping call (written by the sort's first kernel); NULL otherwise
     float max_norm;
     int geo;                       // GEO_*: which instantiation of the scan / elementwise kernels runs
@@ -161,7 +160,6 @@ __device__ __forceinline__ float sharp_value(const TensorDev& T, float v) { retu
 __device__ __forceinline__ float sharp_rounded(const TensorDev& T, int64_t i) { const float v = sharp_raw(T, i); return T.sharp32 == 1 ? sg::round_to(T.dtype, v) : v; }      // not finite stays so
 __device__ __forceinline__ float sharp_of(const TensorDev& T, int64_t i) { return sharp_value(T, sharp_raw(T, i)); }
 
-int launch_norm(const Plan& pl, hipStream_t st);
 int launch_sort(const Plan& pl, int32_t* dbg_perm, hipStream_t st);
 int sort_form(int sort_tile, int sort_tiles, int sort_widest, bool half);      // SG2_SORT_*
 int launch_scan(const Plan& pl, hipStream_t st);

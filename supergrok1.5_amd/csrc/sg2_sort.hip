@@ -98,7 +98,7 @@ __device__ __forceinline__ void note_sharpness(const Plan& pl, int seg, bool nz)
     }
 }
 
-// Factor of the tensor's gradients in a clipping call: the workgroup adds up the tensor's norm tiles (k_norm) itself, in
+// Factor of the tensor's gradients in a clipping call: the workgroup adds up the tensor's norm tiles (k_tables) itself, in
 // the order of a 256-lane reduction; `keep` stores it for the later kernels.
 __device__ __forceinline__ float clip_factor(const Plan& pl, int ti, bool keep) {
     if (!pl.gscale) return 1.0f;

@@ -114,7 +114,7 @@ struct Prof {
 
 constexpr int PREFIXES = 5;     // prefix tables: tiles of the elementwise kernels, sort tiles, scan chunks, chunks with a summary, norm tiles
 struct Layout {
-    int P, total, elem_tiles, sort_tiles, chunks, wchunks, nb, sort_tile, sort_widest, norm_tile, norm_tiles;
+    int P, total, elem_tiles, sort_tiles, chunks, wchunks, nb, sort_tile, sort_widest, norm_tile;
     size_t off_norm, off_gscale, off_tables, off_keys[2], off_vals[2], off_ssorted, off_spine, off_blocksums, off_summ, off_hstart, off_comp, off_flags, off_padw, off_ctx, off_htile, off_adj_summ, off_adj_lam, off_adj_part, off_adj_blk, off_dctx, off_elem, bytes;
     size_t tables_bytes;
 };
@@ -213,7 +213,7 @@ int make_layout(int geo, int P, Numels numels, int chunk_len, Layout* L, bool bi
     }
     if (total > 0x7ffffff0) return sg::fail("total element count %lld exceeds the 2^31 indexing limit", (long long)total);
     L->P = P; L->total = (int)total; L->elem_tiles = (int)et; L->sort_tiles = (int)stl;
-    L->chunks = (int)ch; L->wchunks = (int)wch; L->norm_tiles = (int)nt;
+    L->chunks = (int)ch; L->wchunks = (int)wch;
     L->nb = (int)((256 * stl + SCAN_BLOCK_ITEMS - 1) / SCAN_BLOCK_ITEMS);
     size_t o = 0;
     auto take = [&](size_t bytes) { size_t r = o; o = sg::align_up(o + bytes, 256); return r; };
@@ -255,11 +255,47 @@ struct TableChunk {
     int* flags;                    // per-tensor "sharpness is not all zero" flags to clear, or NULL to keep them
     int* state_bad;                // with flags: per tensor, 1 when one of its carried Mamba states holds a non-finite entry
     int i0, cnt, P, state_floats;  // state_floats: d_inner * d_state of the caller's states
+    double* norm_partials;         // clipping calls: sum of squares per norm tile, else NULL
+    int norm_tile, norm_first;     // elements of a norm tile; the first tile of tensor i0
 };
 static_assert(sizeof(TableChunk) <= 3700, "kernel arguments stay well below 4 KB");
 
-// Workgroup 0 writes the records and tables; workgroup 1 + k looks at the carried states of tensor i0 + k.
+// Clipping calls (supergrok2.py:316-321 of the reference): sums of squares of every tensor's gradient, one per
+// tile; the sort's first kernel adds them up (clip_factor) and every kernel applies the factor to a gradient as it reads
+// it.  HBM bound (one read of the gradients); writing clipped copies and reading those instead cost a second pass (38 us
+// for 25 M elements) and three launches.  (The tile that finishes a tensor could add them up here, but an atomic counter
+// with release order per workgroup took 38 us where the plain stores take 5: each one writes back its L2.)
+// It needs nothing but the records, which are kernel arguments here: as a launch of its own after k_tables it was 3 to 5 us of
+// every small step (8 tensors below 256 elements 48.4 -> 45.6 us, 0.42 M elements 243 -> 241).
+__device__ __forceinline__ void norm_tile(const TableChunk& c, int tile) {
+    __shared__ double sm[4];
+    // the tensor: the last entries of the prefix table that are not above the tile are those before it
+    const int lane = threadIdx.x & 63, end = lane < c.cnt ? c.pre[PREFIXES - 1][lane] : 0x7fffffff;
+    const int i = __popcll(__ballot(end <= tile)), first = i > 0 ? __builtin_amdgcn_readlane(end, i - 1) : c.norm_first;
+    const TensorDev& T = c.rec[i];
+    const int start = (tile - first) * c.norm_tile, cnt = min(c.norm_tile, T.numel - start);
+    float acc = 0.0f;
+    for (int k0 = 0; k0 < cnt; k0 += 8 * 256) {       // eight loads on their way at a time, added in order
+        float g[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const int k = k0 + r * 256 + (int)threadIdx.x;
+            g[r] = k < cnt ? sg::load_elem(T.grad, T.dtype, start + k) : 0.0f;
+        }
+#pragma unroll
+        for (int r = 0; r < 8; r++) acc = sg_fma(g[r], g[r], acc);
+    }
+    const double sum = sg::block_sum((double)acc, sm);
+    if (threadIdx.x == 0) c.norm_partials[tile] = sum;
+}
+
+// Workgroup 0 writes the records and tables; workgroup 1 + k looks at the carried states of tensor i0 + k; those after them
+// (clipping calls) take a norm tile of the gradients each.
 __global__ __launch_bounds__(256) void k_tables(TableChunk c) {
+    if ((int)blockIdx.x > c.cnt) {
+        norm_tile(c, c.norm_first + (int)blockIdx.x - 1 - c.cnt);
+        return;
+    }
     if (blockIdx.x > 0) {
         // A tensor whose carried state is not finite (a diverged run) must come out non-finite as a whole, as it does in
         // the reference, which multiplies every chunk's start state through: the scan only lets contracted summaries
@@ -288,39 +324,7 @@ __global__ __launch_bounds__(256) void k_tables(TableChunk c) {
     if (c.flags != nullptr && c.i0 == 0 && threadIdx.x == 0) c.flags[c.P + 3] = 1;
 }
 
-// Pre-pass of a clipping call (supergrok2.py:316-321 of the reference): sums of squares of every tensor's gradient, one per
-// tile; the sort's first kernel adds them up (clip_factor) and every kernel applies the factor to a gradient as it reads
-// it.  HBM bound (one read of the gradients); writing clipped copies and reading those instead cost a second pass (38 us
-// for 25 M elements) and three launches.  (The tile that finishes a tensor could add them up here, but an atomic counter
-// with release order per workgroup took 38 us where the plain stores take 5: each one writes back its L2.)
-__global__ __launch_bounds__(256) void k_norm(Plan pl) {
-    __shared__ double sm[4];
-    const int tile = blockIdx.x;
-    const sg::Seg seg = sg::find_seg(sg::as_const(pl.norm_tile_prefix), pl.P, tile);
-    const TensorDev& T = pl.tensors[seg.i];
-    const int start = (tile - seg.first) * pl.norm_tile, cnt = min(pl.norm_tile, T.numel - start);
-    float acc = 0.0f;
-    for (int k0 = 0; k0 < cnt; k0 += 8 * 256) {       // eight loads on their way at a time, added in order
-        float g[8];
-#pragma unroll
-        for (int r = 0; r < 8; r++) {
-            const int k = k0 + r * 256 + (int)threadIdx.x;
-            g[r] = k < cnt ? sg::load_elem(T.grad, T.dtype, start + k) : 0.0f;
-        }
-#pragma unroll
-        for (int r = 0; r < 8; r++) acc = sg_fma(g[r], g[r], acc);
-    }
-    const double sum = sg::block_sum((double)acc, sm);
-    if (threadIdx.x == 0) pl.norm_partials[tile] = sum;
-}
-
 }  // namespace
-
-int launch_norm(const Plan& pl, hipStream_t st) {
-    hipLaunchKernelGGL(k_norm, dim3(pl.norm_tiles), dim3(256), 0, st, pl);
-    SG_LAUNCH_CHECK("k_norm");
-    return 0;
-}
 
 int geo_of(const SgDims* d) {
     if (!d) return sg::fail("dims is NULL"), -1;
@@ -466,10 +470,10 @@ size_t sg2_workspace_bytes(const SgDims* dims, int num_tensors, const int64_t* n
 namespace sg2 {
 // Validates the call, lays out the workspace, uploads the per-tensor records and fills the Plan.  full_step:
 // the optimizer-state pointers of every tensor are required; otherwise only grad, sharpness and the two Mamba
-// states (bilevel forward/backward).  Returns 0 with pl->total == 0 when there is nothing to do.
+// states (bilevel forward/backward).  clips: the norms of the gradients are taken beside the upload.  Returns 0 with pl->total == 0 when there is nothing to do.
 int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, const Sg2Tensor* tensors, const Sg2Scalars* scalars,
                void* workspace, size_t workspace_bytes, bool full_step, bool bilevel, bool keep_flags, hipStream_t st, Plan* plp, Layout* Lp,
-               int chunk_override = 0, int window_override = -1, bool whole_pass = false) {
+               int chunk_override = 0, int window_override = -1, bool whole_pass = false, bool clips = false) {
     Plan& pl = *plp;
     Layout& L = *Lp;
     pl.total = 0;
@@ -520,6 +524,9 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
             c.state_bad = reinterpret_cast<int*>(ws + L.off_flags) + P + 4;
             c.state_floats = dims->d_inner * dims->d_state;
             c.i0 = i0; c.cnt = P - i0 < UPLOAD_RECS ? P - i0 : UPLOAD_RECS; c.P = P;
+            c.norm_partials = clips ? reinterpret_cast<double*>(ws + L.off_norm) : nullptr;
+            c.norm_tile = L.norm_tile;
+            c.norm_first = run[PREFIXES - 1];
             for (int k = 0; k < c.cnt; k++) {
                 const Sg2Tensor& t = tensors[i0 + k];
                 const int n = (int)t.numel;
@@ -541,7 +548,8 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
                 run[4] += (int)(((int64_t)n + L.norm_tile - 1) / L.norm_tile);
                 for (int q = 0; q < PREFIXES; q++) c.pre[q][k] = run[q];
             }
-            hipLaunchKernelGGL(k_tables, dim3(d_flags ? 1 + c.cnt : 1), dim3(256), 0, st, c);
+            if (clips && !d_flags) return sg::fail("internal: a clipping call keeps no flags");
+            hipLaunchKernelGGL(k_tables, dim3((d_flags ? 1 + c.cnt : 1) + (clips ? run[PREFIXES - 1] - c.norm_first : 0)), dim3(256), 0, st, c);
             SG_LAUNCH_CHECK("k_tables");
         }
     }
@@ -554,7 +562,6 @@ int build_plan(const SgDims* dims, const Sg2Weights* weights, int num_tensors, c
     pl.wchunk_prefix = dpre + 3 * (P + 1);
     pl.norm_tile_prefix = dpre + 4 * (P + 1);
     pl.sort_tile = L.sort_tile; pl.sort_widest = L.sort_widest;
-    pl.norm_tile = L.norm_tile; pl.norm_tiles = L.norm_tiles;
     pl.norm_partials = reinterpret_cast<double*>(ws + L.off_norm);
     pl.gscale = nullptr;
     pl.max_norm = 0.0f;
@@ -627,14 +634,13 @@ int run_step(const SgDims* dims, const Sg2Weights* weights, int num_tensors, con
     if (clip_norm > 0.0f && num_tensors > 0 && tensors && geo_of(dims) >= 0)
         chunk_override = fitted_chunk_len(geo_of(dims), num_tensors, Numels{nullptr, tensors});
     if (build_plan(dims, weights, num_tensors, tensors, scalars, workspace, workspace_bytes, true, false, false, st, &pl, &L, chunk_override,
-                   window_override))
+                   window_override, false, clip_norm > 0.0f))
         return 1;
     if (pl.total == 0) return 0;
     prof_mark(0, st);
     if (clip_norm > 0.0f) {
         pl.gscale = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + L.off_gscale);
         pl.max_norm = clip_norm;
-        if (launch_norm(pl, st)) return 1;
     }
     if (launch_sort(pl, debug ? debug->perm : nullptr, st)) return 1;
     prof_mark(1, st);

@@ -141,3 +141,24 @@ def test_class_clip_matches_formula():
     want = fo.sg2_clip([x.float().cpu().numpy() for x in h], 0.5)
     for a, b in zip(got, want):
         assert a.dtype == torch.bfloat16 and np.allclose(a.float().cpu().numpy(), b, rtol=2 ** -7, atol=0)
+
+
+@pytest.mark.parametrize("sizes", [[0, 1, 255, 256, 257, 0, 513], [300] * 24, [511 + k % 3 for k in range(25)], [0] * 24 + [260] * 25 + [1]],
+                         ids=["tile_edges", "one_upload", "one_more", "uploads_of_nothing"])
+def test_norms_of_every_upload(sizes):
+    """Each tensor is clipped by its own norm, wherever its record travels: mu is linear in the clipped gradient.  Factors of
+    either side are within two roundings of the same number, a clipped gradient within one more."""
+    from grokking_optimizers import SuperGrok2
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    grads = [torch.randn(n, generator=gen, device="cuda") * 0.5 * (1 + k) for k, n in enumerate(sizes)]
+    mus = []
+    for clip, given in ((0.5, grads), (1e30, [g * min(1.0, 0.5 / (float(g.double().norm()) + 1e-12)) for g in grads])):
+        params = [torch.nn.Parameter(torch.zeros(n, device="cuda")) for n in sizes]
+        torch.manual_seed(2)
+        opt = SuperGrok2(params, gradient_clipping=clip)
+        for p, g in zip(params, given):
+            p.grad = g.clone()
+        opt.step()
+        mus.append(opt._flat_mus)
+    for a, b in zip(*mus):
+        torch.testing.assert_close(a, b, rtol=1e-6, atol=0)
