@@ -277,8 +277,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_adj_prefix(Plan pl, bool use_f
 // around the constant of their row (sg2_taylor_ok), A_bar as a cubic, sin and cos as quadratics in d = dt - dt0 (remainders
 // below 5e-8 while a d < 1/80, f d < 1/256; limits from compose_block).  Other tiles, and the ragged last one of a tensor, take the functions
 // themselves.
-// Bound by the vector ALU: 160 instructions per step (for its 256 states), 78 % of the time one is issued.  18.9 ms on 25 M
-// elements, 0.40 ms on 0.42 M; 53.5 and 1.14 as one 128-lane workgroup per chunk with one wave per SIMD, the exact functions
+// Bound by the vector ALU: 156 instructions per step (for its 256 states).  15.5 ms on 25 M
+// elements, 0.33 ms on 0.42 M; 53.5 and 1.14 as one 128-lane workgroup per chunk with one wave per SIMD, the exact functions
 // at every step and all states of a tile in LDS.
 constexpr int AT = HT_STEP;             // steps per tile
 constexpr int AB = 4;                   // steps per block
@@ -312,7 +312,7 @@ __device__ __forceinline__ float cubic(const adj_f32x4 t, float d) { return sg_f
 // tile blocks 12 900, states at their starts 2950, part 3 2700, projections 1650.  So that nothing of the tile loop spills at 256
 // registers, what only part 3 needs lies in LDS (matrix accumulators; the pair sums where the states of their block were) and
 // addresses are formed where they are used: a reload, or the spill of a prefetched value, waits for every load before it, and
-// that was four memory latencies a tile.  25 M elements: the pass 33.6 -> 31.2 ms; 0.42 M: 1267 -> 1227 us.
+// that was four memory latencies a tile (25 M elements 18.4 -> 16.2 ms).
 template <bool SCAN_GRADS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adjoint(Plan pl, AdjIO io) {      // SCAN_GRADS: the gradient of the gated outputs comes in instead of that of the contexts
     static_assert(AT == 16 && DI == 16 && DS == 16 && HP == 8 && DM == 8 && AB == 4, "lane roles");
@@ -708,9 +708,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                             tBe = sg_fma(l_e, ux, tBe);
                             tBo = sg_fma(l_o, ux, tBo);
                             q[4 * h + u] = sg_fma(l_e, bc[0], l_o * bc[1]);
-                            // A_bar = 2/(1 + a dt) - 1: dA_bar/d dt = -a/2 (A_bar + 1)^2
-                            const float ve = ae[h][u] + 1.0f, vo = ao[h][u] + 1.0f;
-                            const float te = (l_e * re[h][u]) * (ve * ve), to = (l_o * ro[h][u]) * (vo * vo);
+                            // A_bar = 2/(1 + a dt) - 1: dA_bar/d dt = -a/2 (A_bar + 1)^2 (x + x A_bar, twice, each one rounding)
+                            const float xe = l_e * re[h][u], xo = l_o * ro[h][u];
+                            const float we = sg_fma(xe, ae[h][u], xe), wo = sg_fma(xo, ao[h][u], xo);
+                            const float te = sg_fma(we, ae[h][u], we), to = sg_fma(wo, ao[h][u], wo);
                             al_e[h] = sg_fma(te, dt, al_e[h]);
                             al_o[h] = sg_fma(to, dt, al_o[h]);
                             // lambda for the previous step; d theta = d ro * re - d re * ro
