@@ -47,7 +47,7 @@
 // Bound by the vector ALU (about 5000 instructions per wave and tile, two thirds of them the fixed multiply-adds of the
 // net and its derivative; a tile takes 84 000 clocks beside the other wave of its SIMD, of which the experts' 64 lines 8500,
 // the sums of routing weights 17 000, scores and best four 13 000).  Measured on 25 M elements with module-initialised experts
-// after some meta steps: 7.8 ms (9.2 with the experts' lines read pick by pick, the matrix instructions' operands not ahead of
+// after some meta steps: 7.65 ms (9.2 with the experts' lines read pick by pick, the matrix instructions' operands not ahead of
 // them, and a tile's indexes not before the tile), 47 ms as one lane per element of a 256-lane workgroup that summed the
 // outer products lane by lane from LDS; on 0.42 M elements 0.23 ms, 0.29 before those and with a small tensor's tiles side by
 // side, 1.1 at first.  (The net's products as 4 x 4 x 1 matrix instructions with the weights in LDS or in memory took as
@@ -85,6 +85,7 @@ constexpr int N_BINS = NE * NBIN * 2;                              // sums of w 
 constexpr int ROW_FLOATS = (N_BINS + N_DENSE + 31) / 32 * 32;      // a workgroup's row: bins, then the dense sums
 constexpr int TABLE_FLOATS = NE * EH + NE * NBIN * 2;              // thresholds ascending [NE][EH], lines [NE][NBIN][2]
 static_assert(TABLE_FLOATS % 32 == 0 && N_DENSE + 3 * NE * EH + NE == SG2_ELEM_GRAD_FLOATS, "gradient layout, aligned rows");
+constexpr int AHEAD = 4;                 // rows of a head's weights requested ahead of the one in use (all eight: a tenth of the instructions moved spilled ones; two: 1 % behind)
 constexpr int BE_MAX_GROUPS = 512;       // two resident workgroups on each of the 256 CUs: one round, every wave walks the same number of tiles (+-1)
 
 // (row of d, column of x) whose product sums make up GRU gradient entry o, in the order
@@ -174,6 +175,13 @@ __device__ __forceinline__ void wave_sync() {
 // (the row belongs to this workgroup alone: workgroup scope lets the add run in the L2 next to it)
 __device__ __forceinline__ void bin_add(float* p, float v) { __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 
+// A zero in a scalar register that stands only once v does: weights read at it are requested after v, so that those of one
+// row are not all held, and spilled into vector-register lanes, while another's are used.
+__device__ __forceinline__ int zero_after(float& v) {
+    int z = 0;
+    asm volatile("" : "+s"(z), "+v"(v));
+    return z;
+}
 // The thresholds of an expert, read together.
 struct Thresholds {
     float t[EH];
@@ -562,7 +570,7 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             float query[DM];
 #pragma unroll
             for (int dd = 0; dd < DM; dd++) {
-                const sg::cfloat_p qr = Wq + (hh * DM + dd) * PIN + zo_q;
+                const sg::cfloat_p qr = Wq + (hh * DM + dd) * PIN + (dd < AHEAD ? zo_q : zero_after(query[dd - AHEAD]));
                 float v = 0.0f;
 #pragma unroll
                 for (int q = 0; q < GH; q++) v = sg_fma(qr[q], hn[q], v);
@@ -578,7 +586,7 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             float wgt[2][TOPK];
 #pragma unroll
             for (int hf = 0; hf < 2; hf++) {
-                const sg::cfloat_p keys = (hf ? KB : KA) + hh * PK * (DM / 2) + zo_q;
+                const sg::cfloat_p keys = (hf ? KB : KA) + hh * PK * (DM / 2) + zero_after(query[hf ? DM - 1 : DM - AHEAD]);
                 float sc[PK];
 #pragma unroll
                 for (int q = 0; q < PK; q++) {
@@ -765,7 +773,7 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             const int zo_rb = sg::opaque_zero();
 #pragma unroll
             for (int dd = 0; dd < DM; dd++) {
-                const sg::cfloat_p qr = Wq + (hh * DM + dd) * PIN + zo_rb;
+                const sg::cfloat_p qr = Wq + (hh * DM + dd) * PIN + (dd < AHEAD ? zo_rb : zero_after(dhn[GH - 1]));
 #pragma unroll
                 for (int q = 0; q < GH; q++) dhn[q] = sg_fma(qr[q], dq[dd], dhn[q]);
 #pragma unroll
