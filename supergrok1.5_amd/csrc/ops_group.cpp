@@ -706,6 +706,39 @@ void add_flat_grads(const std::vector<torch::Tensor>& params, const torch::Tenso
     TORCH_CHECK(o == flat.numel(), "add_flat_grads: parameters and gradients do not match");
 }
 
+// The meta-net's 33 weights from its parameters: detached, fp32, contiguous; an entry that is a list of tensors (one per head)
+// becomes their stack, the experts' get their two or one dimensions.  Empty where an entry is neither.
+std::vector<torch::Tensor> meta_weights(py::list entries, int64_t num_experts) {
+    at::NoGradGuard guard;
+    auto plain = [](const at::Tensor& t) {
+        at::Tensor d = t.detach();
+        if (d.scalar_type() != torch::kFloat32) d = d.to(torch::kFloat32);
+        return d.is_contiguous() ? d : d.contiguous();
+    };
+    const Py_ssize_t n = PyList_GET_SIZE(entries.ptr());
+    std::vector<torch::Tensor> out;
+    out.reserve(n);
+    for (Py_ssize_t i = 0; i < n; i++) {
+        PyObject* o = PyList_GET_ITEM(entries.ptr(), i);
+        if (const at::Tensor* t = as_tensor(o)) {
+            out.push_back(plain(*t));
+            continue;
+        }
+        std::vector<at::Tensor> parts;
+        for (Py_ssize_t k = 0; PyList_Check(o) && k < PyList_GET_SIZE(o); k++) {
+            const at::Tensor* t = as_tensor(PyList_GET_ITEM(o, k));
+            if (!t) return {};
+            parts.push_back(t->scalar_type() == torch::kFloat32 ? *t : t->to(torch::kFloat32));
+        }
+        if (parts.empty()) return {};
+        out.push_back(at::stack(parts));
+    }
+    if (n != SG2_NUM_WEIGHTS) return {};
+    for (int k : {29, 31}) out[k] = out[k].reshape({num_experts, -1});
+    out[32] = out[32].reshape({-1});
+    return out;
+}
+
 // The random draws of an expert recycling event, in the order of the reference's loop
 // (grokking_optimizers/mamba3_peer_metanet.py:453-488): per dead expert one N(0,1) draw for each of the four expert
 // tensors into its row of `noise`, then a redraw of its key A row if every expert of that row is dead, then of its key B
@@ -895,6 +928,7 @@ void bind_group_steps(pybind11::module_& m) {
     m.def("supergrok2_bilevel_finish", &supergrok2_bilevel_finish);
     m.def("copies_of", &copies_of);
     m.def("add_flat_grads", &add_flat_grads);
+    m.def("meta_weights", &meta_weights);
     m.def("recycle_draws", &recycle_draws);
     m.def("recycle_experts", &recycle_experts);
     m.def("draws_agree", &draws_agree);

@@ -24,6 +24,18 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 
+def _parameter(module, name):
+    """module.<name>, past the module's attribute lookup where it is a plain parameter."""
+    p = module._parameters.get(name)
+    return getattr(module, name) if p is None else p
+
+
+def _entries(params):
+    """The entries of a ParameterList, past its index lookups where they are plain parameters."""
+    held = list(params._parameters.values())
+    return held if len(held) == len(params) else list(params)
+
+
 class Mamba3ScanBlock(nn.Module):
     def __init__(self, d_model: int = 8, d_state: int = 16, expand: int = 2):
         super().__init__()
@@ -201,6 +213,13 @@ class Mamba3PEERMetaNet(nn.Module):
 
     def flat_weights(self):
         """The 33 tensors in the argument order of _ops.supergrok2_mamba_peer_batched_step."""
+        fwd, bwd = self.mamba_fwd, self.mamba_bwd
+        if type(self).get_weights is Mamba3PEERMetaNet.get_weights and type(fwd).export is type(bwd).export is Mamba3ScanBlock.export:
+            # without the dictionary and the calls and lookups per tensor (91 -> 38 us of every bilevel pass and of the first step after one)
+            from grokking_optimizers import _ops
+            out = _ops.meta_weights(self._weight_entries(), self.num_experts)
+            if out:
+                return out
         w = self.get_weights()
         out = [w["input_proj_W"], w["input_proj_b"]]
         for tag in ("fwd", "bwd"):
@@ -211,6 +230,22 @@ class Mamba3PEERMetaNet(nn.Module):
         E = self.num_experts
         out += [w["expert_W1"].reshape(E, -1), w["expert_b1"], w["expert_W2"].reshape(E, -1), w["expert_b2"].reshape(-1)]
         return out
+
+    def _weight_entries(self):
+        """The parameters behind flat_weights, in its order; the per-head ones as lists."""
+        lin = self.input_proj
+        out = [_parameter(lin, "weight"), _parameter(lin, "bias")]
+        for blk in (self.mamba_fwd, self.mamba_bwd):
+            mods = blk._modules
+            dt = mods["dt_proj"]
+            out += [_parameter(mods["in_proj"], "weight"), _parameter(dt, "weight"), _parameter(dt, "bias"), _parameter(mods["B_proj"], "weight"),
+                    _parameter(mods["C_proj"], "weight"), _parameter(blk, "A_log"), _parameter(blk, "D"), _parameter(blk, "rope_freq"),
+                    _parameter(mods["out_proj"], "weight")]
+        mods = self.gru._modules
+        for lin in (mods["W_z"], mods["W_r"], mods["W_h"]):
+            out += [_parameter(lin, "weight"), _parameter(lin, "bias")]
+        out += [[_parameter(q, "weight") for q in self.peer_queries], _entries(self.product_keys_A), _entries(self.product_keys_B)]
+        return out + [_parameter(self, "expert_W1"), _parameter(self, "expert_b1"), _parameter(self, "expert_W2"), _parameter(self, "expert_b2")]
 
     @torch.no_grad()
     def load_flat_weights(self, weights):

@@ -3,6 +3,7 @@ add up to the sizes the C ABI declares, and the header's layout comments name th
 import re
 import os
 
+import pytest
 import torch
 
 from grokking_optimizers import Mamba3PEERMetaNet, _bilevel, _cabi
@@ -94,3 +95,32 @@ def test_reference_names_for_the_device_bilevel_path():
     mn = Mamba3PEERMetaNet()
     assert mn.has_cuda_bilevel is False                # parameters on the CPU: no device kernels can serve it
     assert callable(mn.forward_for_bilevel_cuda)
+
+
+@pytest.mark.parametrize("kw", [{}, dict(d_model=4, d_state=8, gru_hidden=2, num_peer_heads=1, num_experts=25, expert_hidden=3)])
+@pytest.mark.parametrize("change", ["none", "half", "parametrized", "other_list", "strided"])
+def test_flat_weights_are_the_exported_ones(kw, change):
+    """The direct walk over the parameters against the one through get_weights, bit for bit."""
+    class ThroughGetWeights(Mamba3PEERMetaNet):
+        def get_weights(self):
+            return super().get_weights()
+    torch.manual_seed(1)
+    nets = [cls(**kw) for cls in (Mamba3PEERMetaNet, ThroughGetWeights)]
+    nets[1].load_state_dict(nets[0].state_dict())
+    for mn in nets:
+        if change == "half":
+            mn.half()
+        if change == "parametrized":
+            torch.manual_seed(2)
+            torch.nn.utils.parametrizations.orthogonal(mn.gru.W_z)
+        if change == "other_list":
+            mn.product_keys_A = torch.nn.ParameterList([torch.nn.Parameter(2 * k.detach()) for k in mn.product_keys_A])
+        if change == "strided":
+            w = mn.mamba_fwd.in_proj.weight
+            mn.mamba_fwd.in_proj.weight = torch.nn.Parameter(w.detach().t().contiguous().t())
+    if change == "parametrized":
+        nets[1].load_state_dict(nets[0].state_dict())
+    a, b = (mn.flat_weights() for mn in nets)
+    assert len(a) == len(b) == 33
+    for x, y in zip(a, b):
+        assert x.shape == y.shape and x.dtype == torch.float32 and x.is_contiguous() and not x.requires_grad and torch.equal(x, y)
