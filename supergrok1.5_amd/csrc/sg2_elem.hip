@@ -10,11 +10,13 @@
 // elements; the tile index is mapped to (tensor, offset) by a binary search
 // over a P+1 entry prefix table.  The 144 expert MLPs live in LDS (records of
 // 48 floats padded to 52 so that random per-lane experts spread over the
-// banks); GRU and key weights are wave-uniform and come in through scalar
-// loads (constant address space); the query projection is a chain of fp32
-// matrix instructions.  expert_counts is accumulated in an LDS histogram and flushed
+// banks); the net's dense products are chains of fp32 matrix instructions
+// (step4).  expert_counts is accumulated in an LDS histogram and flushed
 // once per workgroup (the reference issues one global atomic per element and
 // head).
+#include <type_traits>
+#include <utility>
+
 #include "sg2_internal.hpp"
 
 namespace sg2 {
@@ -26,28 +28,26 @@ constexpr int ELEM_THREADS = 256;
 template <int EHW>
 constexpr int exp_stride() { return EHW == 16 ? 52 : 3 * EHW; }
 typedef float vf4 __attribute__((ext_vector_type(4)));
-typedef float vf32 __attribute__((ext_vector_type(32)));
 
-// One word of every 64 bytes of the weights that come in through the scalar cache, all requested at once: cold, each of
-// the loads between an element's products waits for the memory by itself, some forty times in a row.  With the expert
-// records' loads all in flight before the first of them is stored, the launch over 8 small tensors takes 10.4 us, 12.1
-// without, and a step of the wide geometry over 0.42 M elements 13 us less.
-template <class G>
-__device__ __forceinline__ void warm_scalar_cache(const Plan& pl) {
-    uint32_t x = 0;
-    auto touch = [&](int which, int floats) {
-        const sg::cint_p p = (sg::cint_p)sg::as_const(pl.W.w[which]);
-#pragma unroll
-        for (int i = 0; i < floats; i += 16) x |= (uint32_t)p[i];
-        x |= (uint32_t)p[floats - 1];
-    };
-    touch(W_GRU_WZ, GH * G::GRL); touch(W_GRU_WR, GH * G::GRL); touch(W_GRU_WH, GH * G::GRL);
-    touch(W_KEYS_A, NH * PK * (G::DM / 2)); touch(W_KEYS_B, NH * PK * (G::DM / 2));
-    asm volatile("" : : "s"(x));
-}
+// The net's small matrix-vector products (GRU, queries, key scores) run on the matrix pipe.  v_mfma_f32_4x4x1_16b is one fused
+// multiply-add per output and step, so a chain of them is the fmaf chain of the scalar form, bit for bit, in the same
+// order.  Its 16 blocks are 4 elements each: lane l brings its own element's input and gets its own element's four outputs.
+// The other operand of a step, four rows' weights, is the same for all blocks: the instruction broadcasts it from any one
+// block, so a register holds 16 steps' weights (block n % 16 of register n / 16: step n) and a whole net of the default
+// geometry takes 22.  As multiply-adds with scalar operands, GRU and scores were 650 of 1550 vector instructions an element and wave
+// with some forty scalar loads between them; the queries, as 32x32x1 products whose outputs had to be exchanged between
+// lanes, are as fast in large calls, but a wave that evaluates one head needs only its quarter of them now.  The launch:
+// 8 tensors below 256 elements 8.6 -> 6.6 us, 0.42 M elements 38.5 -> 34.6 (wide geometry 71 -> 61), 3.1 M bfloat16
+// 174 -> 171, 25 M 1.21 -> 1.20 ms (there the part's power sets the rate: 4.65 ns a product and SIMD, 1.3 to 1.9 a multiply-add).
+template <int N>
+__device__ __forceinline__ vf4 step4(const float* w, float x, vf4 acc) { return __builtin_amdgcn_mfma_f32_4x4x1f32(w[N / 16], x, acc, 4, N % 16, 0); }
+template <class F, int... I>
+__device__ __forceinline__ void each_of(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F>
+__device__ __forceinline__ void each(F f) { each_of(f, std::make_integer_sequence<int, N>{}); }
 
 // Four waves per SIMD for the default geometry: told so, the compiler keeps the matrix results in ordinary registers
-// (115 of them, no accumulation registers to copy out of) instead of settling for three waves at 112 + 32.
+// instead of settling for three waves with accumulation registers to copy out of.
 template <class G>
 constexpr int elem_waves() { return G::DM == 8 ? 4 : 2; }
 // FWD: the net's forward alone (sg2_meta_forward) -- smart gradient and new GRU state of every element go to the packed
@@ -65,11 +65,18 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
     __shared__ float s_exp[NE * EXP_STRIDE];
     __shared__ float s_b2[NE];
     __shared__ int s_cnt[NE];
+    // Weights of the products, four rows a block (see step4): GRU [z, r, h][input], queries [4 rows][input], keys [head][half][4 keys]
+    // [dimension]; of the wave's own head only where it evaluates one.  Keys stay in registers, the others come from LDS, four
+    // registers to a read.
+    constexpr int HEADS_HERE = HEADS ? 1 : NH, HALF = DM / 2, KEY_GROUPS = PK / 4, Q_GROUPS = HEADS_HERE * DM / 4;
+    static_assert(GH == 4 && PK % 4 == 0 && HALF % 4 == 0, "rows in groups of four");
+    constexpr int N_GRU = 3 * GRL, N_QUERY = Q_GROUPS * PIN, N_KEYS = HEADS_HERE * 2 * KEY_GROUPS * HALF;
+    constexpr int R_GRU = (N_GRU + 63) / 64 * 4, R_QUERY = (N_QUERY + 63) / 64 * 4, R_KEYS = (N_KEYS + 15) / 16;
+    __shared__ __attribute__((aligned(16))) float s_w[(R_GRU + (HEADS ? NH : 1) * R_QUERY) * 64];
     __shared__ float s_head[HEADS ? 2 : 1][HEADS ? NH : 1][HEADS ? 64 : 1];
     const int own = HEADS ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, member = threadIdx.x & (STEP - 1);
     int turn = 0;
 
-    warm_scalar_cache<G>(pl);
     {
         const float* __restrict__ W[3] = {pl.W.w[W_EXP_W1], pl.W.w[W_EXP_B1], pl.W.w[W_EXP_W2]};
         constexpr int ROUNDS = (NE * EH + ELEM_THREADS - 1) / ELEM_THREADS;
@@ -89,27 +96,38 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
             for (int m = 0; m < 3; m++) s_exp[at + m * EH] = v[m][r];
         }
     }
+    float w_keys[R_KEYS];
+    {
+        const int lane = threadIdx.x & 63, row = lane & 3, block = lane >> 2;
+        constexpr int WAVES = ELEM_THREADS / 64, QUERIES = (HEADS ? NH : 1) * R_QUERY;
+        auto put = [&](int r, float v) { s_w[(r / 4) * 256 + lane * 4 + r % 4] = v; };
+#pragma unroll
+        for (int r0 = 0; r0 < R_GRU; r0 += WAVES) {
+            const int r = r0 + (int)(threadIdx.x >> 6), n = min(16 * r + block, N_GRU - 1), m = n / GRL;
+            put(r, (m == 0 ? pl.W.w[W_GRU_WZ] : m == 1 ? pl.W.w[W_GRU_WR] : pl.W.w[W_GRU_WH])[row * GRL + n % GRL]);
+        }
+#pragma unroll
+        for (int r0 = 0; r0 < QUERIES; r0 += WAVES) {
+            const int r = r0 + (int)(threadIdx.x >> 6), n = min(16 * (r % R_QUERY) + block, N_QUERY - 1);
+            put(R_GRU + r, pl.W.w[W_PEER_Q][(r / R_QUERY * DM + 4 * (n / PIN) + row) * PIN + n % PIN]);
+        }
+#pragma unroll
+        for (int r = 0; r < R_KEYS; r++) {
+            const int n = min(16 * r + block, N_KEYS - 1), at = n / HALF, hh = own + at / (2 * KEY_GROUPS);
+            w_keys[r] = (at / KEY_GROUPS % 2 ? pl.W.w[W_KEYS_B] : pl.W.w[W_KEYS_A])[(hh * PK + 4 * (at % KEY_GROUPS) + row) * HALF + n % HALF];
+        }
+    }
     __syncthreads();
+    auto weights = [&](int first, auto& w) {
+#pragma unroll
+        for (int r = 0; r < (int)(sizeof(w) / 16); r++) {
+            const vf4 v = *reinterpret_cast<const vf4*>(s_w + (first / 4 + r) * 256 + (threadIdx.x & 63) * 4);
+#pragma unroll
+            for (int q = 0; q < 4; q++) w[4 * r + q] = v[q];
+        }
+    };
 
-    const sg::cfloat_p Wz0 = sg::as_const(pl.W.w[W_GRU_WZ]);
-    const sg::cfloat_p bz0 = sg::as_const(pl.W.w[W_GRU_BZ]);
-    const sg::cfloat_p Wr0 = sg::as_const(pl.W.w[W_GRU_WR]);
-    const sg::cfloat_p br0 = sg::as_const(pl.W.w[W_GRU_BR]);
-    const sg::cfloat_p Wh0 = sg::as_const(pl.W.w[W_GRU_WH]);
-    const sg::cfloat_p bh0 = sg::as_const(pl.W.w[W_GRU_BH]);
-    // The query projection runs on the matrix pipe: v_mfma_f32_32x32x1_2b is one fused multiply-add per output and
-    // step, so a chain of them is the fmaf chain of the scalar form, bit for bit, in the same order.  Lane l supplies
-    // row l % 32 of each 32-row slice of the query matrix (held in registers for the whole kernel) and its own
-    // element's inputs; the outputs come back split over lanes l and l ^ 32 and are exchanged below.
-    constexpr int NQM = NH * DM / 32;
-    static_assert(NH * DM % 32 == 0 && 32 % DM == 0, "query rows are handled in slices of 32");
-    float aq[NQM][PIN];
-#pragma unroll
-    for (int m = 0; m < NQM; m++)
-#pragma unroll
-        for (int q = 0; q < PIN; q++) aq[m][q] = pl.W.w[W_PEER_Q][(m * 32 + (threadIdx.x & 31)) * PIN + q];
-    const sg::cfloat_p KA0 = sg::as_const(pl.W.w[W_KEYS_A]);
-    const sg::cfloat_p KB0 = sg::as_const(pl.W.w[W_KEYS_B]);
+    const sg::cfloat_p bz0 = sg::as_const(pl.W.w[W_GRU_BZ]), br0 = sg::as_const(pl.W.w[W_GRU_BR]), bh0 = sg::as_const(pl.W.w[W_GRU_BH]);
 
     // split: parts that a tile is cut into (1 or ELEM_TILE / STEP, see elem_grid)
     for (int part = blockIdx.x; part < pl.elem_tiles * split; part += gridDim.x) {
@@ -130,10 +148,6 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
         for (int k0 = 0; k0 < cnt; k0 += STEP) {
             const bool live = k0 + member < cnt;
             const int i = start + min(k0 + member, cnt - 1);
-            // the weights are re-read (scalar loads, cache hits) for every element instead of being hoisted
-            const int zo = sg::opaque_zero();
-            const sg::cfloat_p Wz = Wz0 + zo, bz = bz0 + zo, Wr = Wr0 + zo, br = br0 + zo, Wh = Wh0 + zo, bh = bh0 + zo;
-            const sg::cfloat_p KA = KA0 + zo, KB = KB0 + zo;
             const float g_raw = sg::load_elem(T.grad, dtype, i);        // clipped below, when the loads behind it are on their way
             float s = has_s ? sharp_raw(T, i) : 0.0f;
             float cf[DM], cb[DM], hold[GH];
@@ -161,38 +175,31 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
             // ---- GRU: chain order = bias, g, s, fwd ctx, bwd ctx, h
             float zg[GH], rg[GH], hnew[GH];
             float pre_g[2 * GH], gate[2 * GH], pre_c[GH], cand[GH];      // gates and candidates share one reciprocal each
+            float x[GRL];
+            x[0] = g; x[1] = s;
 #pragma unroll
-            for (int j = 0; j < GH; j++) {
-                const sg::cfloat_p wz = Wz + j * GRL;
-                const sg::cfloat_p wr = Wr + j * GRL;
-                float vz = bz[j], vr = br[j];
-                vz = sg_fma(wz[0], g, vz); vz = sg_fma(wz[1], s, vz);
-                vr = sg_fma(wr[0], g, vr); vr = sg_fma(wr[1], s, vr);
+            for (int q = 0; q < DM; q++) { x[2 + q] = cf[q]; x[2 + DM + q] = cb[q]; }
 #pragma unroll
-                for (int q = 0; q < DM; q++) { vz = sg_fma(wz[2 + q], cf[q], vz); vr = sg_fma(wr[2 + q], cf[q], vr); }
+            for (int q = 0; q < GH; q++) x[2 + 2 * DM + q] = hold[q];
+            // (re-read for every element, cache hits: hoisted they would take twelve registers)
+            const int zo = sg::opaque_zero();
+            const sg::cfloat_p bz = bz0 + zo, br = br0 + zo, bh = bh0 + zo;
+            float w_gru[R_GRU], w_query[R_QUERY];
+            weights(zo, w_gru);
+            vf4 az = {bz[0], bz[1], bz[2], bz[3]}, ar = {br[0], br[1], br[2], br[3]}, ah = {bh[0], bh[1], bh[2], bh[3]};
+            each<GRL>([&](auto c) {
+                az = step4<c>(w_gru, x[c], az);
+                ar = step4<GRL + c>(w_gru, x[c], ar);
+                if (c < GRL - GH) ah = step4<2 * GRL + c>(w_gru, x[c], ah);
+            });
 #pragma unroll
-                for (int q = 0; q < DM; q++) { vz = sg_fma(wz[2 + DM + q], cb[q], vz); vr = sg_fma(wr[2 + DM + q], cb[q], vr); }
-#pragma unroll
-                for (int q = 0; q < GH; q++) { vz = sg_fma(wz[2 + 2 * DM + q], hold[q], vz); vr = sg_fma(wr[2 + 2 * DM + q], hold[q], vr); }
-                pre_g[j] = vz;
-                pre_g[GH + j] = vr;
-            }
+            for (int j = 0; j < GH; j++) { pre_g[j] = az[j]; pre_g[GH + j] = ar[j]; }
             sg_sigmoid_block(2 * GH, pre_g, gate);
 #pragma unroll
             for (int j = 0; j < GH; j++) { zg[j] = gate[j]; rg[j] = gate[GH + j]; }
+            each<GH>([&](auto q) { ah = step4<2 * GRL + GRL - GH + q>(w_gru, rg[q] * hold[q], ah); });
 #pragma unroll
-            for (int j = 0; j < GH; j++) {
-                const sg::cfloat_p wh = Wh + j * GRL;
-                float v = bh[j];
-                v = sg_fma(wh[0], g, v); v = sg_fma(wh[1], s, v);
-#pragma unroll
-                for (int q = 0; q < DM; q++) v = sg_fma(wh[2 + q], cf[q], v);
-#pragma unroll
-                for (int q = 0; q < DM; q++) v = sg_fma(wh[2 + DM + q], cb[q], v);
-#pragma unroll
-                for (int q = 0; q < GH; q++) v = sg_fma(wh[2 + 2 * DM + q], rg[q] * hold[q], v);
-                pre_c[j] = v;
-            }
+            for (int j = 0; j < GH; j++) pre_c[j] = ah[j];
             sg_tanh_block(GH, pre_c, cand);
 #pragma unroll
             for (int j = 0; j < GH; j++) hnew[j] = sg_fma(zg[j], cand[j], (1.0f - zg[j]) * hold[j]);
@@ -202,61 +209,26 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
             }
 
             // ---- PEER queries: chain order = h, fwd ctx, bwd ctx, g, s
-            float qall[NH * DM];
+            float xq[PIN];
 #pragma unroll
-            for (int m = 0; m < NQM; m++) {
-                vf32 acc = {};
-                int c = 0;
+            for (int q = 0; q < GH; q++) xq[q] = hnew[q];
 #pragma unroll
-                for (int q = 0; q < GH; q++, c++) acc = __builtin_amdgcn_mfma_f32_32x32x1f32(aq[m][c], hnew[q], acc, 0, 0, 0);
-#pragma unroll
-                for (int q = 0; q < DM; q++, c++) acc = __builtin_amdgcn_mfma_f32_32x32x1f32(aq[m][c], cf[q], acc, 0, 0, 0);
-#pragma unroll
-                for (int q = 0; q < DM; q++, c++) acc = __builtin_amdgcn_mfma_f32_32x32x1f32(aq[m][c], cb[q], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x1f32(aq[m][c], g, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x1f32(aq[m][c + 1], s, acc, 0, 0, 0);
-                // register r of block b holds row 8 (r / 4) + 4 (lane / 32) + r % 4 of element 32 b + lane % 32:
-                // exchanging the upper half of block 0 with the lower half of block 1 gives each lane its own element
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const auto pr = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[r]), __float_as_uint(acc[16 + r]), false, false);
-                    qall[m * 32 + 8 * (r / 4) + r % 4] = __uint_as_float(pr[0]);
-                    qall[m * 32 + 8 * (r / 4) + 4 + r % 4] = __uint_as_float(pr[1]);
-                }
-            }
+            for (int q = 0; q < DM; q++) { xq[GH + q] = cf[q]; xq[GH + DM + q] = cb[q]; }
+            xq[GH + 2 * DM] = g; xq[GH + 2 * DM + 1] = s;
+            weights(R_GRU + own * R_QUERY + zo, w_query);
+            vf4 query[Q_GROUPS];
+            each<Q_GROUPS>([&](auto m) { query[m] = vf4{0.0f, 0.0f, 0.0f, 0.0f}; });
+            each<PIN>([&](auto c) { each<Q_GROUPS>([&](auto m) { query[m] = step4<m * PIN + c>(w_query, xq[c], query[m]); }); });
 
             // ---- PEER routing + expert MLP
-            float total = 0.0f;
-#pragma unroll
-            for (int hh = 0; hh < NH; hh++) {
-                if (HEADS && hh != own) continue;
-                const float* query = qall + hh * DM;
-                int best[2];
-#pragma unroll
-                for (int hf = 0; hf < 2; hf++) {
-                    const sg::cfloat_p keys = (hf ? KB : KA) + hh * PK * (DM / 2);
-                    // the first of the largest scores: the maximum, then the lowest index that has it.  (A running comparison
-                    // takes two selects per key, each waiting two clocks for the comparison before it.)
-                    float dot[PK], bs = -1e30f;
-#pragma unroll
-                    for (int q = 0; q < PK; q++) {
-                        dot[q] = 0.0f;
-#pragma unroll
-                        for (int dd = 0; dd < DM / 2; dd++) dot[q] = sg_fma(query[hf * (DM / 2) + dd], keys[q * (DM / 2) + dd], dot[q]);
-                        bs = __builtin_fmaxf(bs, dot[q]);
-                    }
-                    int bi = 0;
-#pragma unroll
-                    for (int q = PK - 1; q > 0; q--) bi = dot[q] == bs ? q : bi;
-                    best[hf] = dot[0] == bs ? 0 : bi;
-                }
-                int e = best[0] * PK + best[1];
-                if (e >= NE) e = NE - 1;
-                if (live) atomicAdd(&s_cnt[e], 1);
-                if (DBG && live) dbg_eidx[((size_t)T.off + i) * NH + hh] = e;
-
-                const float4* rec = reinterpret_cast<const float4*>(s_exp + e * EXP_STRIDE);
-                float ho = s_b2[e];
+            // (an expert's record is requested before the next head's scores and evaluated after them)
+            // Waves that route go before waves in the products above: those are long runs of matrix instructions that need no
+            // other wave's time to hide anything, these wait for LDS.  (25 M elements 1.23 -> 1.20 ms; the other way round 1.22,
+            // both parts ahead of the update below 1.24.)
+            __builtin_amdgcn_s_setprio(1);
+            float total = 0.0f, ho = 0.0f;
+            float4 rec[3 * (EH / 4)];
+            auto evaluate = [&]() {
 #pragma unroll
                 for (int q4 = 0; q4 < EH / 4; q4++) {
                     const float4 w1 = rec[q4], b1 = rec[EH / 4 + q4], w2 = rec[2 * (EH / 4) + q4];
@@ -267,7 +239,40 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
                     z = sg_max(sg_fma(w1.w, g, b1.w), 0.0f); ho = sg_fma(w2.w, z, ho);
                 }
                 total = total + ho;
-            }
+                asm volatile("" : "+v"(total));       // before the next record is requested, or registers spill
+            };
+            each<HEADS_HERE>([&](auto head) {
+                vf4 score[2][KEY_GROUPS];
+                each<2>([&](auto hf) { each<KEY_GROUPS>([&](auto t) { score[hf][t] = vf4{0.0f, 0.0f, 0.0f, 0.0f}; }); });
+                each<HALF>([&](auto dd) {
+                    each<2>([&](auto hf) {
+                        constexpr int row = head * DM + hf * HALF + dd;
+                        each<KEY_GROUPS>([&](auto t) { score[hf][t] = step4<((head * 2 + hf) * KEY_GROUPS + t) * HALF + dd>(w_keys, query[row / 4][row % 4], score[hf][t]); });
+                    });
+                });
+                int best[2];
+#pragma unroll
+                for (int hf = 0; hf < 2; hf++) {
+                    // the first of the largest scores: the maximum, then the lowest index that has it.  (A running comparison
+                    // takes two selects per key, each waiting two clocks for the comparison before it.)
+                    float bs = -1e30f;
+#pragma unroll
+                    for (int q = 0; q < PK; q++) bs = __builtin_fmaxf(bs, score[hf][q / 4][q % 4]);
+                    int bi = 0;
+#pragma unroll
+                    for (int q = PK - 1; q > 0; q--) bi = score[hf][q / 4][q % 4] == bs ? q : bi;
+                    best[hf] = score[hf][0][0] == bs ? 0 : bi;
+                }
+                int e = best[0] * PK + best[1];
+                if (e >= NE) e = NE - 1;
+                if (live) atomicAdd(&s_cnt[e], 1);
+                if (DBG && live) dbg_eidx[((size_t)T.off + i) * NH + own + head] = e;
+                if (head > 0) evaluate();
+                ho = s_b2[e];
+#pragma unroll
+                for (int q = 0; q < 3 * (EH / 4); q++) rec[q] = reinterpret_cast<const float4*>(s_exp + e * EXP_STRIDE)[q];
+            });
+            evaluate();
             if (HEADS) {
                 s_head[turn][own][member] = total;       // 0 + the head
                 __syncthreads();                         // (every wave has read the GRU state)
@@ -278,6 +283,7 @@ __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(el
                 turn ^= 1;
                 if (live) ((SG_GLOBAL vf4*)T.gru)[i] = vf4{hnew[0], hnew[1], hnew[2], hnew[3]};
             }
+            __builtin_amdgcn_s_setprio(0);
             const float smart = g + (rescale * total) / (float)NH;
             if (FWD) {
                 if (live) sg::gptr(fwd_smart)[(size_t)T.off + i] = smart;
@@ -477,6 +483,7 @@ __global__ __launch_bounds__(ELEM_THREADS) void k_elem_any(Plan pl, int ctx_stri
                 }
                 total = total + ho;
             }
+            __builtin_amdgcn_s_setprio(0);
             const float smart = g + (rescale * total) / (float)H;
             if (fwd_smart != nullptr) {
                 sg::gptr(fwd_smart)[(size_t)T.off + i] = smart;
