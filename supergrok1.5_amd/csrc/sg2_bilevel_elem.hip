@@ -44,14 +44,18 @@
 // filled by atomics of four waves, so the last bits of the expert gradients can differ from run to run (as with the
 // reference's atomicAdd).
 //
-// Bound by the vector ALU (about 5000 instructions per wave and tile, two thirds of them the fixed multiply-adds of the
-// net and its derivative; a tile takes 84 000 clocks beside the other wave of its SIMD, of which the experts' 64 lines 8500,
-// the sums of routing weights 17 000, scores and best four 13 000).  Measured on 25 M elements with module-initialised experts
-// after some meta steps: 7.65 ms (9.2 with the experts' lines read pick by pick, the matrix instructions' operands not ahead of
-// them, and a tile's indexes not before the tile), 47 ms as one lane per element of a 256-lane workgroup that summed the
-// outer products lane by lane from LDS; on 0.42 M elements 0.23 ms, 0.29 before those and with a small tensor's tiles side by
-// side, 1.1 at first.  (The net's products as 4 x 4 x 1 matrix instructions with the weights in LDS or in memory took as
-// long, with the bins in LDS longer on large calls: registers are what there is least of.)
+// The net's products and their transposes are chains of 4 x 4 x 1 matrix instructions (product4), the same multiply-adds in the
+// same order as scalar code: 550 of them for 2200 multiply-adds with scalar operands, whose loads were waited for in some
+// hundred places and spilled into vector-register lanes.  A head's nine registers of weights are requested a phase ahead.
+// (7.65 -> 7.2 ms, 0.227 -> 0.218.)
+// Bound by the vector ALU and the waits between its phases (about 3000 vector and 900 matrix instructions per wave and tile;
+// a tile takes 80 000 clocks beside the other wave of its SIMD, of which the experts' 64 lines 8500, the sums of routing
+// weights 17 000).  Measured on 25 M elements with module-initialised experts
+// after some meta steps: 7.2 ms (9.2 with the experts' lines read pick by pick, the sums' operands not ahead of
+// them, a tile's indexes not before the tile and the products in scalar form), 47 ms as one lane per element of a 256-lane workgroup that summed the
+// outer products lane by lane from LDS; on 0.42 M elements 0.22 ms, 0.29 before those and with a small tensor's tiles side by
+// side, 1.1 at first.  (Products with their weights spread over all lanes' registers, from LDS or memory, took as
+// long as the scalar form, with the bins in LDS longer on large calls: registers are what there is least of.)
 #include "sg2_internal.hpp"
 
 namespace sg2 {
@@ -85,7 +89,6 @@ constexpr int N_BINS = NE * NBIN * 2;                              // sums of w 
 constexpr int ROW_FLOATS = (N_BINS + N_DENSE + 31) / 32 * 32;      // a workgroup's row: bins, then the dense sums
 constexpr int TABLE_FLOATS = NE * EH + NE * NBIN * 2;              // thresholds ascending [NE][EH], lines [NE][NBIN][2]
 static_assert(TABLE_FLOATS % 32 == 0 && N_DENSE + 3 * NE * EH + NE == SG2_ELEM_GRAD_FLOATS, "gradient layout, aligned rows");
-constexpr int AHEAD = 4;                 // rows of a head's weights requested ahead of the one in use (all eight: a tenth of the instructions moved spilled ones; two: 1 % behind)
 constexpr int BE_MAX_GROUPS = 512;       // two resident workgroups on each of the 256 CUs: one round, every wave walks the same number of tiles (+-1)
 
 // (row of d, column of x) whose product sums make up GRU gradient entry o, in the order
@@ -175,13 +178,6 @@ __device__ __forceinline__ void wave_sync() {
 // (the row belongs to this workgroup alone: workgroup scope lets the add run in the L2 next to it)
 __device__ __forceinline__ void bin_add(float* p, float v) { __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 
-// A zero in a scalar register that stands only once v does: weights read at it are requested after v, so that those of one
-// row are not all held, and spilled into vector-register lanes, while another's are used.
-__device__ __forceinline__ int zero_after(float& v) {
-    int z = 0;
-    asm volatile("" : "+s"(z), "+v"(v));
-    return z;
-}
 // The thresholds of an expert, read together.
 struct Thresholds {
     float t[EH];
@@ -276,11 +272,7 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     for (int i = lane; i < (64 * XW + R_FLOATS) / 4; i += 64) reinterpret_cast<be_f32x4*>(s_x)[i] = be_f32x4{0.0f, 0.0f, 0.0f, 0.0f};     // rows are read whole: no NaN may lie in what was never written
     __syncthreads();
 
-    const sg::cfloat_p Wz = sg::as_const(a.W.w[W_GRU_WZ]), bz = sg::as_const(a.W.w[W_GRU_BZ]);
-    const sg::cfloat_p Wr = sg::as_const(a.W.w[W_GRU_WR]), br = sg::as_const(a.W.w[W_GRU_BR]);
-    const sg::cfloat_p Wh = sg::as_const(a.W.w[W_GRU_WH]), bh = sg::as_const(a.W.w[W_GRU_BH]);
-    const sg::cfloat_p Wq = sg::as_const(a.W.w[W_PEER_Q]);
-    const sg::cfloat_p KA = sg::as_const(a.W.w[W_KEYS_A]), KB = sg::as_const(a.W.w[W_KEYS_B]);
+    const sg::cfloat_p bz = sg::as_const(a.W.w[W_GRU_BZ]), br = sg::as_const(a.W.w[W_GRU_BR]), bh = sg::as_const(a.W.w[W_GRU_BH]);
 
     const int li = lane & 15, lk = lane >> 4;             // operand roles of the 16 x 16 x 4 instructions: row / column, element of the step
     // accumulators.  Register v of a 16 x 16 one: row 4 (lane / 16) + v, column lane % 16; of a 4 x 4 x 16 one: block lane / 4, row v, column lane % 4
@@ -514,39 +506,47 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             cf[0] = a0.x; cf[1] = a0.y; cf[2] = a0.z; cf[3] = a0.w; cf[4] = a1.x; cf[5] = a1.y; cf[6] = a1.z; cf[7] = a1.w;
             cb[0] = b0.x; cb[1] = b0.y; cb[2] = b0.z; cb[3] = b0.w; cb[4] = b1.x; cb[5] = b1.y; cb[6] = b1.z; cb[7] = b1.w;
         }
-        // (a zero the compiler cannot see through where the wave-uniform weights are used keeps their scalar loads there;
-        //  held across the whole element they are spilled into vector-register lanes and read back, 3000 instructions)
-        const int zo_gf = sg::opaque_zero();
+        // Weights of the products (product4), requested where they are used: lane 4 block + row holds row `row` of four.  (The lane
+        // is opaque to the compiler, or they would be held, and spilled, from one tile to the next.)
+        auto opaque_lane = [&]() { int ln = lane; asm volatile("" : "+v"(ln)); return ln; };
+        // of a head's products: inputs 0 .. 7, 8 .. 15, 14 .. 21 of the query's two halves; the keys' entries
+        struct HeadWeights { float w[3], k[2]; };
+        auto head_weights = [&](int hh) {
+            const int ln = opaque_lane(), row = ln & 3, block = ln >> 2;
+            const float* const wq = a.W.w[W_PEER_Q] + hh * DM * PIN + (4 * (block >> 3) + row) * PIN + (block & 7);
+            const int at_k = hh * PK * (DM / 2) + (4 * min(block >> 2, PK / 4 - 1) + row) * (DM / 2) + (block & 3);
+            return HeadWeights{{wq[0], wq[8], wq[14]}, {a.W.w[W_KEYS_A][at_k], a.W.w[W_KEYS_B][at_k]}};
+        };
+        HeadWeights ahead;
         // ---- GRU forward
         float zg[GH], rg[GH], cand[GH], hn[GH];
         {
+            const int ln = opaque_lane(), at_w = (ln & 3) * GRL + (ln >> 2);
+            float wz[2], wr[2], wh[2];       // inputs 0 .. 15 and 6 .. 21
+#pragma unroll
+            for (int r = 0; r < 2; r++) { wz[r] = a.W.w[W_GRU_WZ][at_w + 6 * r]; wr[r] = a.W.w[W_GRU_WR][at_w + 6 * r]; wh[r] = a.W.w[W_GRU_WH][at_w + 6 * r]; }
+            float x[GRL];
+            x[0] = g; x[1] = s;
+#pragma unroll
+            for (int q = 0; q < DM; q++) { x[2 + q] = cf[q]; x[2 + DM + q] = cb[q]; }
+#pragma unroll
+            for (int q = 0; q < GH; q++) x[2 + 2 * DM + q] = h[q];
+            static_assert(GRL == 22 && GH == 4, "two registers of sixteen inputs");
+            const int zo = sg::opaque_zero();
+            be_f32x4 vz = {bz[zo], bz[zo + 1], bz[zo + 2], bz[zo + 3]}, vr = {br[zo], br[zo + 1], br[zo + 2], br[zo + 3]}, vh = {bh[zo], bh[zo + 1], bh[zo + 2], bh[zo + 3]};
+            each<GRL>([&](auto c) {
+                constexpr int R = c < 16 ? 0 : 1, B = c - 6 * R;
+                vz = product4<B>(wz[R], x[c], vz);
+                vr = product4<B>(wr[R], x[c], vr);
+                if constexpr (c < GRL - GH) vh = product4<B>(wh[R], x[c], vh);
+            });
+#pragma unroll
+            for (int j = 0; j < GH; j++) { zg[j] = sg_sigmoid(vz[j]); rg[j] = sg_sigmoid(vr[j]); }
+            ahead = head_weights(0);
+            each<GH>([&](auto q) { vh = product4<GRL - GH + q - 6>(wh[1], rg[q] * h[q], vh); });
 #pragma unroll
             for (int j = 0; j < GH; j++) {
-                const sg::cfloat_p wz = Wz + j * GRL + zo_gf, wr = Wr + j * GRL + zo_gf;
-                float vz = bz[j], vr = br[j];
-                vz = sg_fma(wz[0], g, vz); vz = sg_fma(wz[1], s, vz);
-                vr = sg_fma(wr[0], g, vr); vr = sg_fma(wr[1], s, vr);
-#pragma unroll
-                for (int q = 0; q < DM; q++) { vz = sg_fma(wz[2 + q], cf[q], vz); vr = sg_fma(wr[2 + q], cf[q], vr); }
-#pragma unroll
-                for (int q = 0; q < DM; q++) { vz = sg_fma(wz[2 + DM + q], cb[q], vz); vr = sg_fma(wr[2 + DM + q], cb[q], vr); }
-#pragma unroll
-                for (int q = 0; q < GH; q++) { vz = sg_fma(wz[2 + 2 * DM + q], h[q], vz); vr = sg_fma(wr[2 + 2 * DM + q], h[q], vr); }
-                zg[j] = sg_sigmoid(vz);
-                rg[j] = sg_sigmoid(vr);
-            }
-#pragma unroll
-            for (int j = 0; j < GH; j++) {
-                const sg::cfloat_p wh = Wh + j * GRL + zo_gf;
-                float v = bh[j];
-                v = sg_fma(wh[0], g, v); v = sg_fma(wh[1], s, v);
-#pragma unroll
-                for (int q = 0; q < DM; q++) v = sg_fma(wh[2 + q], cf[q], v);
-#pragma unroll
-                for (int q = 0; q < DM; q++) v = sg_fma(wh[2 + DM + q], cb[q], v);
-#pragma unroll
-                for (int q = 0; q < GH; q++) v = sg_fma(wh[2 + 2 * DM + q], rg[q] * h[q], v);
-                cand[j] = sg_tanh(v);
+                cand[j] = sg_tanh(vh[j]);
                 hn[j] = sg_fma(zg[j], cand[j], (1.0f - zg[j]) * h[j]);
             }
         }
@@ -559,43 +559,53 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 
         // ---- heads: forward, then at once the head's backward
         float total = 0.0f;
-        float dhn[GH] = {0.f, 0.f, 0.f, 0.f}, dcf[DM], dcb[DM], dq_even[DM];
+        // d loss / d h_new and the contexts, [0] and four at a time in [1] .. [4]
+        be_f32x4 dx[1 + 2 * DM / 4];
+        float dq_even[DM];
 #pragma unroll
-        for (int q = 0; q < DM; q++) { dcf[q] = 0.0f; dcb[q] = 0.0f; dq_even[q] = 0.0f; }
+        for (int q = 0; q < 1 + 2 * DM / 4; q++) dx[q] = be_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int q = 0; q < DM; q++) dq_even[q] = 0.0f;
         const float kk = cot * kscale;                 // d loss / d head output
         const int side = g > 0.0f ? 0 : NE;
 #pragma unroll 1
         for (int hh = 0; hh < NH; hh++) {
-            const int zo_q = sg::opaque_zero();
             float query[DM];
-#pragma unroll
-            for (int dd = 0; dd < DM; dd++) {
-                const sg::cfloat_p qr = Wq + (hh * DM + dd) * PIN + (dd < AHEAD ? zo_q : zero_after(query[dd - AHEAD]));
-                float v = 0.0f;
-#pragma unroll
-                for (int q = 0; q < GH; q++) v = sg_fma(qr[q], hn[q], v);
-#pragma unroll
-                for (int q = 0; q < DM; q++) v = sg_fma(qr[GH + q], cf[q], v);
-#pragma unroll
-                for (int q = 0; q < DM; q++) v = sg_fma(qr[GH + DM + q], cb[q], v);
-                v = sg_fma(qr[GH + 2 * DM], g, v);
-                v = sg_fma(qr[GH + 2 * DM + 1], s, v);
-                query[dd] = v;
-            }
             int idx[2][TOPK];
             float wgt[2][TOPK];
+            {
+                const float (&w)[3] = ahead.w;
+                const float (&wk)[2] = ahead.k;
+                static_assert(PIN == 22 && DM == 8 && PK == 12, "blocks of the weights' registers");
+                float x[PIN];
 #pragma unroll
-            for (int hf = 0; hf < 2; hf++) {
-                const sg::cfloat_p keys = (hf ? KB : KA) + hh * PK * (DM / 2) + zero_after(query[hf ? DM - 1 : DM - AHEAD]);
-                float sc[PK];
+                for (int q = 0; q < GH; q++) x[q] = hn[q];
 #pragma unroll
-                for (int q = 0; q < PK; q++) {
-                    float dot = 0.0f;
+                for (int q = 0; q < DM; q++) { x[GH + q] = cf[q]; x[GH + DM + q] = cb[q]; }
+                x[GH + 2 * DM] = g; x[GH + 2 * DM + 1] = s;
+                be_f32x4 q4[2] = {be_f32x4{0.0f, 0.0f, 0.0f, 0.0f}, be_f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+                each<PIN>([&](auto c) {
+                    constexpr int R = c / 8, B = R < 2 ? c % 8 : c - 14;
+                    q4[0] = product4<B>(w[R], x[c], q4[0]);
+                    q4[1] = product4<8 + B>(w[R], x[c], q4[1]);
+                });
 #pragma unroll
-                    for (int dd = 0; dd < DM / 2; dd++) dot = sg_fma(query[hf * (DM / 2) + dd], keys[q * (DM / 2) + dd], dot);
-                    sc[q] = dot;
+                for (int dd = 0; dd < DM; dd++) query[dd] = q4[dd / 4][dd % 4];
+                be_f32x4 sc4[2][PK / 4];
+#pragma unroll
+                for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+                    for (int t = 0; t < PK / 4; t++) sc4[hf][t] = be_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                each<DM / 2>([&](auto dd) {
+                    each<2>([&](auto hf) { each<PK / 4>([&](auto t) { sc4[hf][t] = product4<4 * t + dd>(wk[hf], q4[hf][int(dd)], sc4[hf][t]); }); });
+                });
+#pragma unroll
+                for (int hf = 0; hf < 2; hf++) {
+                    float sc[PK];
+#pragma unroll
+                    for (int q = 0; q < PK; q++) sc[q] = sc4[hf][q / 4][q % 4];
+                    best_four(sc, s_r + lane * CW + hf * PK, idx[hf], wgt[hf]);
                 }
-                best_four(sc, s_r + lane * CW + hf * PK, idx[hf], wgt[hf]);
             }
             wave_sync();
             // ---- experts: the line of each at this element's side of zero, where its interval holds g
@@ -699,6 +709,13 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
             for (int ia = 0; ia < TOPK; ia++) head_out = sg_fma(wgt[0][ia], ra[ia], head_out);
             total += head_out;
+            float w_back[4];       // of the query's derivative, two of its entries each
+            {
+                const int ln = opaque_lane(), row = ln & 3, block = ln >> 2;
+                const float* const wq = a.W.w[W_PEER_Q] + hh * DM * PIN + (block >> 3) * PIN + 4 * min(block & 7, 4) + row;
+#pragma unroll
+                for (int r = 0; r < 4; r++) w_back[r] = wq[2 * r * PIN];
+            }
             // ---- sums of the routing weights over this tile's elements, four a step
             {
                 float* const crow = s_r + slot * CW;
@@ -770,16 +787,8 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                 }
                 dq[4 * hf] = d0; dq[4 * hf + 1] = d1; dq[4 * hf + 2] = d2; dq[4 * hf + 3] = d3;
             }
-            const int zo_rb = sg::opaque_zero();
-#pragma unroll
-            for (int dd = 0; dd < DM; dd++) {
-                const sg::cfloat_p qr = Wq + (hh * DM + dd) * PIN + (dd < AHEAD ? zo_rb : zero_after(dhn[GH - 1]));
-#pragma unroll
-                for (int q = 0; q < GH; q++) dhn[q] = sg_fma(qr[q], dq[dd], dhn[q]);
-#pragma unroll
-                for (int q = 0; q < DM; q++) dcf[q] = sg_fma(qr[GH + q], dq[dd], dcf[q]);
-#pragma unroll
-                for (int q = 0; q < DM; q++) dcb[q] = sg_fma(qr[GH + DM + q], dq[dd], dcb[q]);
+            {
+                each<DM>([&](auto dd) { each<5>([&](auto q) { dx[q] = product4<8 * (dd % 2) + q>(w_back[dd / 2], dq[dd], dx[q]); }); });
             }
             // ---- product-key gradients, d score (x) query half, two elements a step
             {
@@ -813,6 +822,7 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                         sum(q & 1);
                     }
                 };
+                if (hh + 1 < NH) ahead = head_weights(hh + 1);
                 if (hh == 0) key_sums(kacc[0]);
                 else if (hh == 1) key_sums(kacc[1]);
                 else if (hh == 2) key_sums(kacc[2]);
@@ -835,38 +845,34 @@ __global__ __launch_bounds__(BE_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
         }
         if (valid && a.smart != nullptr) a.smart[out_at] = sg_fma(a.rescale, total / (float)NH, g);
 
-        const int zo_gb = sg::opaque_zero();
         // ---- GRU backward
-        float dpz[GH], dpr[GH], dph[GH], drh[GH] = {0.f, 0.f, 0.f, 0.f};
+        float dpz[GH], dpr[GH], dph[GH];
 #pragma unroll
         for (int j = 0; j < GH; j++) {
-            dpz[j] = (dhn[j] * (cand[j] - h[j])) * (zg[j] * (1.0f - zg[j]));
-            dph[j] = (dhn[j] * zg[j]) * (1.0f - cand[j] * cand[j]);
+            dpz[j] = (dx[0][j] * (cand[j] - h[j])) * (zg[j] * (1.0f - zg[j]));
+            dph[j] = (dx[0][j] * zg[j]) * (1.0f - cand[j] * cand[j]);
         }
+        {
+            const int ln = opaque_lane(), row = ln & 3, block = ln >> 2, at_w = (block >> 2) * GRL + 2 + 4 * (block & 3) + row;
+            const float wz = a.W.w[W_GRU_WZ][at_w], wr = a.W.w[W_GRU_WR][at_w], wh = a.W.w[W_GRU_WH][at_w];
+            const float wh_h = a.W.w[W_GRU_WH][(block & 3) * GRL + 2 + 2 * DM + row];
+            be_f32x4 drh = {0.0f, 0.0f, 0.0f, 0.0f};
+            each<GH>([&](auto j) {
+                each<4>([&](auto q) { dx[1 + q] = product4<4 * j + q>(wh, dph[j], dx[1 + q]); });
+                drh = product4<j>(wh_h, dph[j], drh);
+            });
 #pragma unroll
-        for (int j = 0; j < GH; j++) {
-            const sg::cfloat_p wh = Wh + j * GRL + zo_gb;
-#pragma unroll
-            for (int q = 0; q < DM; q++) { dcf[q] = sg_fma(wh[2 + q], dph[j], dcf[q]); dcb[q] = sg_fma(wh[2 + DM + q], dph[j], dcb[q]); }
-#pragma unroll
-            for (int q = 0; q < GH; q++) drh[q] = sg_fma(wh[2 + 2 * DM + q], dph[j], drh[q]);
-        }
-#pragma unroll
-        for (int j = 0; j < GH; j++) dpr[j] = (drh[j] * h[j]) * (rg[j] * (1.0f - rg[j]));
-#pragma unroll
-        for (int j = 0; j < GH; j++) {
-            const sg::cfloat_p wz = Wz + j * GRL + zo_gb, wr = Wr + j * GRL + zo_gb;
-#pragma unroll
-            for (int q = 0; q < DM; q++) {
-                dcf[q] = sg_fma(wz[2 + q], dpz[j], dcf[q]); dcf[q] = sg_fma(wr[2 + q], dpr[j], dcf[q]);
-                dcb[q] = sg_fma(wz[2 + DM + q], dpz[j], dcb[q]); dcb[q] = sg_fma(wr[2 + DM + q], dpr[j], dcb[q]);
-            }
+            for (int j = 0; j < GH; j++) dpr[j] = (drh[j] * h[j]) * (rg[j] * (1.0f - rg[j]));
+            each<GH>([&](auto j) {
+                each<4>([&](auto q) { dx[1 + q] = product4<4 * j + q>(wz, dpz[j], dx[1 + q]); });
+                each<4>([&](auto q) { dx[1 + q] = product4<4 * j + q>(wr, dpr[j], dx[1 + q]); });
+            });
         }
         if (valid) {
             float4* of = reinterpret_cast<float4*>(a.d_ctx + (size_t)at * DM);
             float4* ob = reinterpret_cast<float4*>(a.d_ctx + ((size_t)a.total + at) * DM);
-            of[0] = make_float4(dcf[0], dcf[1], dcf[2], dcf[3]); of[1] = make_float4(dcf[4], dcf[5], dcf[6], dcf[7]);
-            ob[0] = make_float4(dcb[0], dcb[1], dcb[2], dcb[3]); ob[1] = make_float4(dcb[4], dcb[5], dcb[6], dcb[7]);
+            of[0] = make_float4(dx[1][0], dx[1][1], dx[1][2], dx[1][3]); of[1] = make_float4(dx[2][0], dx[2][1], dx[2][2], dx[2][3]);
+            ob[0] = make_float4(dx[3][0], dx[3][1], dx[3][2], dx[3][3]); ob[1] = make_float4(dx[4][0], dx[4][1], dx[4][2], dx[4][3]);
         }
         // ---- GRU gradients
         {

@@ -14,9 +14,6 @@
 // (step4).  expert_counts is accumulated in an LDS histogram and flushed
 // once per workgroup (the reference issues one global atomic per element and
 // head).
-#include <type_traits>
-#include <utility>
-
 #include "sg2_internal.hpp"
 
 namespace sg2 {
@@ -27,24 +24,17 @@ constexpr int ELEM_THREADS = 256;
 // experts spread over the banks)
 template <int EHW>
 constexpr int exp_stride() { return EHW == 16 ? 52 : 3 * EHW; }
-typedef float vf4 __attribute__((ext_vector_type(4)));
+typedef outputs4 vf4;
 
-// The net's small matrix-vector products (GRU, queries, key scores) run on the matrix pipe.  v_mfma_f32_4x4x1_16b is one fused
-// multiply-add per output and step, so a chain of them is the fmaf chain of the scalar form, bit for bit, in the same
-// order.  Its 16 blocks are 4 elements each: lane l brings its own element's input and gets its own element's four outputs.
-// The other operand of a step, four rows' weights, is the same for all blocks: the instruction broadcasts it from any one
-// block, so a register holds 16 steps' weights (block n % 16 of register n / 16: step n) and a whole net of the default
+// The net's small matrix-vector products (GRU, queries, key scores) run on the matrix pipe (product4): step n's weights are
+// block n % 16 of register n / 16, and a whole net of the default
 // geometry takes 22.  As multiply-adds with scalar operands, GRU and scores were 650 of 1550 vector instructions an element and wave
 // with some forty scalar loads between them; the queries, as 32x32x1 products whose outputs had to be exchanged between
 // lanes, are as fast in large calls, but a wave that evaluates one head needs only its quarter of them now.  The launch:
 // 8 tensors below 256 elements 8.6 -> 6.6 us, 0.42 M elements 38.5 -> 34.6 (wide geometry 71 -> 61), 3.1 M bfloat16
 // 174 -> 171, 25 M 1.21 -> 1.20 ms (there the part's power sets the rate: 4.65 ns a product and SIMD, 1.3 to 1.9 a multiply-add).
 template <int N>
-__device__ __forceinline__ vf4 step4(const float* w, float x, vf4 acc) { return __builtin_amdgcn_mfma_f32_4x4x1f32(w[N / 16], x, acc, 4, N % 16, 0); }
-template <class F, int... I>
-__device__ __forceinline__ void each_of(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
-template <int N, class F>
-__device__ __forceinline__ void each(F f) { each_of(f, std::make_integer_sequence<int, N>{}); }
+__device__ __forceinline__ vf4 step4(const float* w, float x, vf4 acc) { return product4<N % 16>(w[N / 16], x, acc); }
 
 // Four waves per SIMD for the default geometry: told so, the compiler keeps the matrix results in ordinary registers
 // instead of settling for three waves with accumulation registers to copy out of.

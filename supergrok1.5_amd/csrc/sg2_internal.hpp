@@ -1,6 +1,9 @@
 // Internal layout shared by the SuperGrok v2 translation units.
 #pragma once
 
+#include <type_traits>
+#include <utility>
+
 #include "sg_common.hpp"
 
 namespace sg2 {
@@ -141,6 +144,20 @@ struct Plan {
     float decay, beta2, eps, rescale;
     Sg2Weights W;
 };
+
+// A step of four matrix-vector products on the matrix pipe.  v_mfma_f32_4x4x1_16b is one fused multiply-add per output and
+// step, so a chain of them is the fmaf chain of the scalar form, bit for bit, in the same order.  Its 16 blocks are 4
+// elements each: lane l brings its own element's input x and gets its own element's four outputs.  The other operand, four
+// rows' weights, is the same for all blocks: the instruction broadcasts it from block BLOCK (lane 4 BLOCK + i: row i), so a
+// register holds 16 steps' weights.
+typedef float outputs4 __attribute__((ext_vector_type(4)));
+template <int BLOCK>
+__device__ __forceinline__ outputs4 product4(float w, float x, outputs4 acc) { return __builtin_amdgcn_mfma_f32_4x4x1f32(w, x, acc, 4, BLOCK, 0); }
+// f(0), ..., f(N - 1) with the index as a constant
+template <class F, int... I>
+__device__ __forceinline__ void each_of(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F>
+__device__ __forceinline__ void each(F f) { each_of(f, std::make_integer_sequence<int, N>{}); }
 
 // records a profiling event (no-op unless profiling is enabled)
 void prof_mark(int idx, hipStream_t st);
