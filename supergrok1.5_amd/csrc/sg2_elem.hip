@@ -504,8 +504,9 @@ __global__ __launch_bounds__(ELEM_THREADS) void k_elem_any(Plan pl, int ctx_stri
 }  // namespace
 
 // A wave per head while that takes at most one workgroup per compute unit.  Beyond, the element's chain is shorter still, but
-// every 64 elements pay for an LDS fill of 28 KB that otherwise serves 256: 8 small tensors -2.5 us a step, 1000 elements in 3
-// tensors -1.7, 5000 in 4 -1.4, but 15 000 in 6 (about 300 parts) +1, 0.42 M +62.
+// every 64 elements pay for an LDS fill of 36 KB that otherwise serves 256: 8 small tensors -2.1 us a step, 1000 elements in 3
+// tensors -2, 5000 in 4 -2; taken up to twice as many parts, 15 000 in 6 (about 300) no difference, 28 000 in 5 +1.6.  (0.42 M: +62
+// with the scalar form.)
 constexpr int HEADS_PARTS = 256;
 inline bool by_heads(const Plan& pl) { return pl.elem_kind != ELEM_ANY && pl.elem_tiles * (ELEM_TILE / 64) <= HEADS_PARTS; }
 
