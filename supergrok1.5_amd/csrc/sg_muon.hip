@@ -64,9 +64,12 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 enum { T_BF16 = 0, T_F16 = 1 };
-// Half-precision iterates and Gram matrices are held times 2^14: the largest singular value stays below 1.3 throughout, so no
-// entry can overflow, and full precision reaches down to 4e-9.  (Powers of two: the factors round nothing.)
-constexpr float F16_SCALE = 16384.0f, F16_UNSCALE = 1.0f / 16384.0f;
+// Half-precision iterates and Gram matrices (and S) are held times 2^14: the largest singular value stays below 1.3 throughout,
+// so no entry can overflow, and full precision reaches down to 4e-9.  Polynomials and their products, below 41, are held times
+// 2^10: a row far below the others meets them only in entries as small as it is, and at a scale of one rows 1e-5 and 1e-6 times
+// as large as the others of 700 x 2800 came out 4 and 40 % off after five iterations (now 0.4 %; 0.6 % at 1e-7).  (Powers of two:
+// the factors round nothing.)
+constexpr float F16_SCALE = 16384.0f, F16_UNSCALE = 1.0f / 16384.0f, POLY_SCALE = 1024.0f, POLY_UNSCALE = 1.0f / 1024.0f;
 
 constexpr int BT = 256;            // GEMM tile (M and N)
 // Waves of a workgroup along N (2 along M).  Eight waves of 128 x 64 (two per SIMD, 128 accumulators each) measured
@@ -284,15 +287,18 @@ __device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
 template <int EPI, int IN, int OUT>
 constexpr float epi_factor() {
     if (EPI == EPI_GRAM) return (IN == T_F16 ? F16_UNSCALE * F16_UNSCALE : 1.0f) * (OUT == T_F16 ? F16_SCALE : 1.0f);
-    if (EPI == EPI_APPLY) return (IN == T_F16 ? F16_UNSCALE : 1.0f) * (OUT == T_F16 ? F16_SCALE : 1.0f);
+    if (EPI == EPI_APPLY) return IN == T_F16 ? POLY_UNSCALE : OUT == T_F16 ? F16_SCALE : 1.0f;
+    if (EPI == EPI_MUL) return OUT == T_F16 ? POLY_UNSCALE : POLY_UNSCALE * POLY_UNSCALE;       // one factor is a polynomial, both are where the result is one in bf16
     return 1.0f;
 }
-// b G + c G G (+ a on the diagonal) from a product of G, as it is held, and an entry of it
+// b G + c G G from a product of G and an entry of it, and the a of the diagonal, as the operands and the result are held
 template <int T>
 __device__ __forceinline__ float polynomial(float gg, float g) {
     if (T == T_BF16) return sg_fma(NS_C, gg, NS_B * g);
-    return sg_fma(NS_C * F16_UNSCALE * F16_UNSCALE, gg, NS_B * F16_UNSCALE * g);
+    return sg_fma(NS_C * F16_UNSCALE * F16_UNSCALE * POLY_SCALE, gg, NS_B * F16_UNSCALE * POLY_SCALE * g);
 }
+template <int T>
+constexpr float diagonal() { return T == T_BF16 ? NS_A : NS_A * POLY_SCALE; }
 
 // The R operand reads of the next k step are dealt over the first eight of a phase's M MFMAs (R/8 after each, one more
 // after the first R%8), the other MFMAs follow on their own
@@ -544,7 +550,7 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, Ops ops, int y_s
     // first iteration: Y is the unnormalised momentum, so its Gram matrix carries 1/norm^2 and the applied Y 1/norm
     const float inv = Bt.inv_norm[mi];
     const bool diag_wave = EPI == EPI_POLY && tm == tn && wn / (GWN / 2) == wm;     // this wave's block meets the diagonal
-    const bool first = (iter_flags & 2) != 0;
+    const bool first = (EPI == EPI_GRAM || EPI == EPI_APPLY) && (iter_flags & 2) != 0;       // (only they read Y)
     constexpr float factor = epi_factor<EPI, IN, OUT>();
     const float scale = first ? (EPI == EPI_GRAM ? inv * inv : inv) * factor : factor;
 #pragma unroll
@@ -570,10 +576,10 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, Ops ops, int y_s
                 if (diag_wave) {        // H + a I: the apply step is then the single product (H + a I) Y
                     const int dk = (wm * (BT / 2) + i * 32 + row) - (wn * WCOLS + c8 * 8);
 #pragma unroll
-                    for (int k = 0; k < 8; k++) v[k] += (dk == k) ? NS_A : 0.0f;
+                    for (int k = 0; k < 8; k++) v[k] += (dk == k) ? diagonal<IN>() : 0.0f;
                 }
             }
-            if ((EPI == EPI_GRAM || EPI == EPI_APPLY) && (first || factor != 1.0f)) {      // uniform over the grid
+            if (EPI != EPI_POLY && (first || factor != 1.0f)) {      // uniform over the grid
 #pragma unroll
                 for (int k = 0; k < 8; k++) v[k] *= scale;
             }
@@ -773,9 +779,9 @@ __global__ __launch_bounds__(KS_THREADS) void k_gemm_64(Batch Bt, Ops ops, int y
         if (EPI == EPI_POLY) {
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                v[k] = polynomial<IN>(v[k], widen<IN>(g[h][k >> 1], k)) + (tm == tn && row == 8 * c8 + k ? NS_A : 0.0f);
+                v[k] = polynomial<IN>(v[k], widen<IN>(g[h][k >> 1], k)) + (tm == tn && row == 8 * c8 + k ? diagonal<IN>() : 0.0f);
             }
-        } else if (EPI != EPI_MUL && (first || factor != 1.0f)) {
+        } else if (first || factor != 1.0f) {
 #pragma unroll
             for (int k = 0; k < 8; k++) v[k] *= scale;
         }
