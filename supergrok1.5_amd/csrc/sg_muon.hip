@@ -1154,7 +1154,7 @@ struct Layout {
     std::vector<Mat> mats;
     bool small;                    // every matrix fits k_newton_schulz
     bool fine[3];                  // products that go to k_gemm_64
-    double time[3];                // and what choose_tiles expects each to take
+    double time[3];                // and what count_stages takes each to cost, in microseconds
     std::vector<int> pre_g[3], pre_t;
     size_t off_mats, off_pre, off_partials, off_inv, bytes;
 };
@@ -1164,8 +1164,10 @@ struct Layout {
 // longer of the chain of one tile (0.003 K) and what all tiles take together (3 ns and 14 ps per k each).  Over 18 sets from
 // 1 x 200 x 800 to 6 x 1024 x 4096 the choice so made was within 8 % of the best.
 // fine_pad: what the matrices would be padded to for k_gemm_64 (64, or 256 where another product keeps its large tiles)
+// time: what the chosen form costs one of many products in a row.  Rounds that fill the chip are held at the rate that the part's
+// power allows, 1.1 PFLOP/s (a tile's K at 0.12 ns; 24 of 1024 x 1024 take 43 to 55 us for the symmetric products, the fit 24).
 void choose_tiles(int P, const SgMuonMatrix* in, int fine_pad, bool fine[3], double time[3]) {
-    double tiles[3] = {}, each[3] = {}, chain[3] = {}, k_max[3] = {};
+    double tiles[3] = {}, each[3] = {}, chain[3] = {}, k_max[3] = {}, work[3] = {};
     for (int i = 0; i < P; i++) {
         const double m = (double)std::min(in[i].rows, in[i].cols), n = (double)std::max(in[i].rows, in[i].cols);
         auto up = [](double x, int a) { return std::ceil(x / a) * a; };
@@ -1174,17 +1176,20 @@ void choose_tiles(int P, const SgMuonMatrix* in, int fine_pad, bool fine[3], dou
                 const double tm = up(m, pad) / size, tn = up(n, pad) / size;
                 return e == EPI_APPLY ? tm * tn : tm * (tm + 1) / 2;
             };
+            const double k256 = up(e == EPI_GRAM ? n : m, BT);
             tiles[e] += count(BT, BT);
-            k_max[e] = std::max(k_max[e], up(e == EPI_GRAM ? n : m, BT));
+            work[e] += count(BT, BT) * k256;
+            k_max[e] = std::max(k_max[e], k256);
             const double k = up(e == EPI_GRAM ? n : m, fine_pad);
             each[e] += count(fine_pad, NT64) * (0.003 + 14e-6 * k);
             chain[e] = std::max(chain[e], 0.003 * k);
         }
     }
     for (int e = 0; e < 3; e++) {
-        const double small = 5.0 + std::max(chain[e], each[e]), large = std::ceil(tiles[e] / 256.0) * (7.0 + 0.0165 * k_max[e]);
+        const double rounds = std::ceil(tiles[e] / 256.0);
+        const double small = 5.0 + std::max(chain[e], each[e]), large = rounds * (7.0 + 0.0165 * k_max[e]);
         fine[e] = small < large;
-        time[e] = std::min(small, large);
+        time[e] = fine[e] ? small : std::max(large, 12.0 * rounds + 1.2e-4 * work[e]);
     }
 }
 
@@ -1267,16 +1272,20 @@ const Product products[] = {
 
 // In how many stages the iterations run (see the head of the file): at most three iterations a stage, or one a stage (the Gram
 // matrix from Y every time, in bf16), which near squares and in calls that wait for launches more than for products is
-// faster.  By what choose_tiles expects; over 22 sets the measured ratio tracked / each lay between -0.11 and +0.18 of the
-// expected one (the small products of a full chip take longer than their fit), so it has to be below 0.95.  Five iterations,
-// each / tracked: 24 of 1024 x 1024 834 / 995 us (expected 1.00), 2 of 1000 x 1500 250 / 257 (0.99), 16 of 512 x 2048 404 / 388
-// (0.93), 12 of 300 x 1200 234 / 202 (0.93), 1 of 1024 x 4096 284 / 237 (0.80), 1 of 100 x 4000 162 / 129 (0.86).
+// faster.  By the products' costs.  Over 80 sets of 1 to 60 matrices with sides of 130 to 8192, ratios of 1 to 30 and 2 to 7
+// iterations, the measured ratio tracked / each was 0.89-1.07 of the expected one where all products take 64x64 tiles, 1.0-1.24
+// where some do and 1.07-1.20 where none does, hence three lines.  They keep out what would be slower for it (tracked is at most
+// 0.99 of each where they choose it), and with that some calls that would be up to 10 % faster.  Five iterations, each /
+// tracked, expected: 24 of 1024 x 1024 822 / 933 us (1.05), 12 of 1536 x 1920 1434 / 1513 (0.91), 24 of 768 x 1152 670 / 694
+// (0.92), 12 of 1536 x 2304 1538 / 1563 (0.88), 24 of 1024 x 2048 1262 / 1169 (0.81), 24 of 1024 x 4096 2243 / 1683 (0.63); 16 of
+// 512 x 2048 367 / 341 (0.82), 6 of 1024 x 2048 465 / 463 (0.94); 12 of 300 x 1200 234 / 200 (0.93), 1 of 200 x 800 116 / 119 (1.13).
 int count_stages(const Layout& L, int ns_steps) {
     if (L.small) return ns_steps;
     const int stages = (ns_steps + 2) / 3;
     const double ends = L.time[EPI_GRAM] + L.time[EPI_APPLY], poly = L.time[EPI_POLY];
-    const double tracked = stages * ends + (4 * ns_steps - 3 * stages) * poly, each = ns_steps * (ends + poly);
-    return tracked < 0.95 * each ? stages : ns_steps;
+    const double tracked = stages * ends + (4.0 * ns_steps - 3.0 * stages) * poly, each = ns_steps * (ends + poly);
+    const int fine = L.fine[EPI_GRAM] + L.fine[EPI_POLY] + L.fine[EPI_APPLY];
+    return tracked < (fine == 3 ? 0.95 : fine > 0 ? 0.9 : 0.86) * each ? stages : ns_steps;
 }
 
 }  // namespace
