@@ -86,7 +86,7 @@ struct Mat {
     const void* grad;
     float* buf;
     bf16_t *Y, *Y2;                // [mp x np] twice (an apply step reads one and writes the other)
-    bf16_t* W[5];                  // [mp x mp]: Gram matrices, polynomials and their products
+    bf16_t* W[5];                  // [mp x mp]: Gram matrices, polynomials and their products (the last three only where iterations can share them)
     bf16_t *T, *T2;                // the transposes of Y and Y2 [np x mp], or NULL (kept for k_gemm_64's apply step)
     int rows, cols, dtype;
     int m, n, mp, np;              // min / max dim and their padded sizes
@@ -1153,6 +1153,7 @@ struct Layout {
     int P;
     std::vector<Mat> mats;
     bool small;                    // every matrix fits k_newton_schulz
+    bool may_share;                // some number of iterations runs in fewer stages than iterations
     bool fine[3];                  // products that go to k_gemm_64
     double time[3];                // and what count_stages takes each to cost, in microseconds
     std::vector<int> pre_g[3], pre_t;
@@ -1193,6 +1194,24 @@ void choose_tiles(int P, const SgMuonMatrix* in, int fine_pad, bool fine[3], dou
     }
 }
 
+// In how many stages the iterations run (see the head of the file): at most three iterations a stage, or one a stage (the Gram
+// matrix from Y every time, in bf16), which near squares and in calls that wait for launches more than for products is
+// faster.  By the products' costs.  Over 80 sets of 1 to 60 matrices with sides of 130 to 8192, ratios of 1 to 30 and 2 to 7
+// iterations, the measured ratio tracked / each was 0.89-1.07 of the expected one where all products take 64x64 tiles, 1.0-1.24
+// where some do and 1.07-1.20 where none does, hence three lines.  They keep out what would be slower for it (tracked is at most
+// 0.99 of each where they choose it), and with that some calls that would be up to 10 % faster.  Five iterations, each /
+// tracked, expected: 24 of 1024 x 1024 822 / 933 us (1.05), 12 of 1536 x 1920 1434 / 1513 (0.91), 24 of 768 x 1152 670 / 694
+// (0.92), 12 of 1536 x 2304 1538 / 1563 (0.88), 24 of 1024 x 2048 1262 / 1169 (0.81), 24 of 1024 x 4096 2243 / 1683 (0.63); 16 of
+// 512 x 2048 367 / 341 (0.82), 6 of 1024 x 2048 465 / 463 (0.94); 12 of 300 x 1200 234 / 200 (0.93), 1 of 200 x 800 116 / 119 (1.13).
+int count_stages(const Layout& L, int ns_steps) {
+    if (!L.may_share) return ns_steps;
+    const int stages = (ns_steps + 2) / 3;
+    const double ends = L.time[EPI_GRAM] + L.time[EPI_APPLY], poly = L.time[EPI_POLY];
+    const double tracked = stages * ends + (4.0 * ns_steps - 3.0 * stages) * poly, each = ns_steps * (ends + poly);
+    const int fine = L.fine[EPI_GRAM] + L.fine[EPI_POLY] + L.fine[EPI_APPLY];
+    return tracked < (fine == 3 ? 0.95 : fine > 0 ? 0.9 : 0.86) * each ? stages : ns_steps;
+}
+
 int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
     L->P = P;
     L->mats.resize(P);
@@ -1214,6 +1233,9 @@ int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
     choose_tiles(P, in, NT64, L->fine, L->time);
     if (!all_fine()) choose_tiles(P, in, BT, L->fine, L->time);
     const int pad = L->small || all_fine() ? 64 : BT;
+    // (sharing costs least, beside one Gram matrix an iteration, where every stage has its three iterations)
+    L->may_share = !L->small;
+    L->may_share = count_stages(*L, 3) < 3;
     for (int i = 0; i < P; i++) {
         const SgMuonMatrix& s = in[i];
         if (s.rows <= 0 || s.cols <= 0 || s.rows * s.cols > 0x7fffffff) return sg::fail("matrix %d: bad shape %lld x %lld", i, (long long)s.rows, (long long)s.cols);
@@ -1249,7 +1271,7 @@ int make_layout(int P, const SgMuonMatrix* in, Layout* L) {
             M.T = (bf16_t*)take(2 * (size_t)M.mp * M.np);
             M.T2 = (bf16_t*)take(2 * (size_t)M.mp * M.np);
         }
-        for (auto& w : M.W) w = (bf16_t*)take(2 * (size_t)M.mp * M.mp);
+        for (int k = 0; k < (L->may_share ? 5 : 2); k++) M.W[k] = (bf16_t*)take(2 * (size_t)M.mp * M.mp);
     }
     L->bytes = o;
     return 0;
@@ -1269,24 +1291,6 @@ const Product products[] = {
     SG_PRODUCT(EPI_APPLY, T_BF16, T_F16),  SG_PRODUCT(EPI_APPLY, T_F16, T_F16),
 };
 #undef SG_PRODUCT
-
-// In how many stages the iterations run (see the head of the file): at most three iterations a stage, or one a stage (the Gram
-// matrix from Y every time, in bf16), which near squares and in calls that wait for launches more than for products is
-// faster.  By the products' costs.  Over 80 sets of 1 to 60 matrices with sides of 130 to 8192, ratios of 1 to 30 and 2 to 7
-// iterations, the measured ratio tracked / each was 0.89-1.07 of the expected one where all products take 64x64 tiles, 1.0-1.24
-// where some do and 1.07-1.20 where none does, hence three lines.  They keep out what would be slower for it (tracked is at most
-// 0.99 of each where they choose it), and with that some calls that would be up to 10 % faster.  Five iterations, each /
-// tracked, expected: 24 of 1024 x 1024 822 / 933 us (1.05), 12 of 1536 x 1920 1434 / 1513 (0.91), 24 of 768 x 1152 670 / 694
-// (0.92), 12 of 1536 x 2304 1538 / 1563 (0.88), 24 of 1024 x 2048 1262 / 1169 (0.81), 24 of 1024 x 4096 2243 / 1683 (0.63); 16 of
-// 512 x 2048 367 / 341 (0.82), 6 of 1024 x 2048 465 / 463 (0.94); 12 of 300 x 1200 234 / 200 (0.93), 1 of 200 x 800 116 / 119 (1.13).
-int count_stages(const Layout& L, int ns_steps) {
-    if (L.small) return ns_steps;
-    const int stages = (ns_steps + 2) / 3;
-    const double ends = L.time[EPI_GRAM] + L.time[EPI_APPLY], poly = L.time[EPI_POLY];
-    const double tracked = stages * ends + (4.0 * ns_steps - 3.0 * stages) * poly, each = ns_steps * (ends + poly);
-    const int fine = L.fine[EPI_GRAM] + L.fine[EPI_POLY] + L.fine[EPI_APPLY];
-    return tracked < (fine == 3 ? 0.95 : fine > 0 ? 0.9 : 0.86) * each ? stages : ns_steps;
-}
 
 }  // namespace
 }  // namespace sgmu
@@ -1324,7 +1328,7 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
     const int P = L.P;
     for (auto& M : L.mats) {
         M.Y = (bf16_t*)(ws + (size_t)M.Y); M.Y2 = (bf16_t*)(ws + (size_t)M.Y2);
-        for (auto& w : M.W) w = (bf16_t*)(ws + (size_t)w);
+        for (auto& w : M.W) if (w) w = (bf16_t*)(ws + (size_t)w);
         if (M.T) { M.T = (bf16_t*)(ws + (size_t)M.T); M.T2 = (bf16_t*)(ws + (size_t)M.T2); }
     }
     // per-call tables: through kernel arguments (no host-to-device copy, nothing blocks the host), records and tile prefixes

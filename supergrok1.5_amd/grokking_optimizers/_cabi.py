@@ -88,6 +88,7 @@ def lib():
         L.sg2_batched_step_static.restype = C.c_int
         L.sg2_batched_step_static.argtypes = [C.POINTER(SgDims), C.POINTER(Sg2Weights), C.c_int, C.POINTER(Sg2Tensor),
                                               C.POINTER(Sg2Scalars), C.c_void_p, C.POINTER(Sg2Debug), C.c_void_p]
+        L.sg_muon_workspace_bytes.restype = C.c_size_t
         L.sg2_bilevel_workspace_bytes.restype = C.c_size_t
         L.sg2_bilevel_workspace_bytes.argtypes = [C.POINTER(SgDims), C.c_int, C.POINTER(C.c_int64)]
         L.sg2_bilevel_forward.restype = C.c_int
@@ -162,13 +163,20 @@ def sort_form_for(numels, all_16bit=False):
     return SORT_FORMS[n]
 
 
+def _muon_matrices(shapes):
+    return (SgMuonMatrix * len(shapes))(*[SgMuonMatrix(None, None, None, r, c, 0) for r, c in shapes])
+
+
 def muon_stages_for(shapes, ns_steps=5):
     """How many Gram matrices a Muon step of these fp32 matrices forms from its iterates."""
-    arr = (SgMuonMatrix * len(shapes))(*[SgMuonMatrix(None, None, None, r, c, 0) for r, c in shapes])
-    n = lib().sg_muon_stages_for(len(shapes), arr, ns_steps)
+    n = lib().sg_muon_stages_for(len(shapes), _muon_matrices(shapes), ns_steps)
     if n < 0:
         raise RuntimeError(last_error())
     return n
+
+
+def muon_workspace_bytes(shapes):
+    return lib().sg_muon_workspace_bytes(len(shapes), _muon_matrices(shapes))
 
 
 def workspace_bytes(numels, dims=None, options=None):
