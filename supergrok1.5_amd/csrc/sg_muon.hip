@@ -1377,14 +1377,14 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
         hipLaunchKernelGGL(k_newton_schulz, dim3(P), dim3(NS_THREADS), lds, st, B, ns_steps);
         SG_LAUNCH_CHECK("k_newton_schulz");
     }
+    bool missing = false;
     auto launch = [&](int epi, int in, int out, Ops ops, int sel, int flags) {
         const int e = shape_of(epi);
         const dim3 grid(B.gtiles[e] * (ops.c2 >= 0 ? 2 : 1));
-        for (const Product& p : products) {
-            if (p.epi != epi || p.in != in || p.out != out) continue;
-            if (L.fine[e]) hipLaunchKernelGGL(p.k64, grid, dim3(KS_THREADS), KS_LDS_BYTES, st, B, ops, sel, flags);
-            else hipLaunchKernelGGL(p.k256, grid, dim3(GTHREADS), GEMM_LDS_BYTES, st, B, ops, sel, flags);
-        }
+        const Product* p = std::find_if(std::begin(products), std::end(products), [&](const Product& q) { return q.epi == epi && q.in == in && q.out == out; });
+        if (p == std::end(products)) missing = true;
+        else if (L.fine[e]) hipLaunchKernelGGL(p->k64, grid, dim3(KS_THREADS), KS_LDS_BYTES, st, B, ops, sel, flags);
+        else hipLaunchKernelGGL(p->k256, grid, dim3(GTHREADS), GEMM_LDS_BYTES, st, B, ops, sel, flags);
     };
     const int stages = count_stages(L, ns_steps);
     const bool tracked = stages < ns_steps;
@@ -1420,6 +1420,7 @@ int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, flo
             launch(EPI_APPLY, in, T_F16, Ops{q, 0, 0, 0, 0, -1}, sel, flags);
         }
         SG_LAUNCH_CHECK("muon newton-schulz");
+        if (missing) return sg::fail("internal: a product of these types has no kernel");
     }
     hipLaunchKernelGGL(k_update, dim3(B.ttiles), dim3(256), 0, st, B, lr, 1.0f - lr * wd, stages & 1, ns_steps == 0 ? 1 : 0, tracked ? T_F16 : T_BF16);
     SG_LAUNCH_CHECK("k_update");
