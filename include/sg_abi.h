@@ -588,6 +588,12 @@ size_t sg_muon_workspace_bytes(int num_matrices, const SgMuonMatrix* mats);
  * sg_muon_step refuses. */
 int sg_muon_stages_for(int num_matrices, const SgMuonMatrix* mats, int ns_steps);
 
+/* The side of the output tiles (64 or 256) that a call with these matrices
+ * takes for its Gram matrices, the products of their size and the apply steps;
+ * all 0 where every matrix stays in one workgroup's LDS.  Nonzero for what
+ * sg_muon_step refuses. */
+int sg_muon_tiles_for(int num_matrices, const SgMuonMatrix* mats, int tiles[3]);
+
 /* Muon step for all matrices: buf = momentum*buf + g; X = buf/(||buf||_F+1e-7)
  * with the norm reduced on the device; ns_steps quintic Newton-Schulz
  * iterations X <- aX + b(XX^T)X + c(XX^T)^2 X with (a,b,c) = (3.4445, -4.7750,

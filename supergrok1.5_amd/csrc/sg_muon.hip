@@ -1311,6 +1311,14 @@ int sg_muon_stages_for(int num_matrices, const SgMuonMatrix* mats, int ns_steps)
     return sgmu::count_stages(L, ns_steps);
 }
 
+int sg_muon_tiles_for(int num_matrices, const SgMuonMatrix* mats, int tiles[3]) {
+    sgmu::Layout L;
+    if (num_matrices <= 0 || !mats || !tiles) return sg::fail("no matrices, or nowhere to write");
+    if (sgmu::make_layout(num_matrices, mats, &L)) return 1;
+    for (int e = 0; e < 3; e++) tiles[e] = L.small ? 0 : L.fine[e] ? sgmu::NT64 : sgmu::BT;
+    return 0;
+}
+
 int sg_muon_step(int num_matrices, const SgMuonMatrix* mats, float momentum, float lr, float wd, int ns_steps, void* workspace,
                  size_t workspace_bytes, void* stream) {
     using namespace sgmu;

@@ -175,6 +175,14 @@ def muon_stages_for(shapes, ns_steps=5):
     return n
 
 
+def muon_tiles_for(shapes):
+    """The sides of the output tiles of its Gram matrices, the products of their size and the apply steps (0: no tiles)."""
+    out = (C.c_int * 3)()
+    if lib().sg_muon_tiles_for(len(shapes), _muon_matrices(shapes), out):
+        raise RuntimeError(last_error())
+    return tuple(out)
+
+
 def muon_workspace_bytes(shapes):
     return lib().sg_muon_workspace_bytes(len(shapes), _muon_matrices(shapes))
 
