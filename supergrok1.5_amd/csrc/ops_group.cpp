@@ -706,27 +706,27 @@ void add_flat_grads(const std::vector<torch::Tensor>& params, const torch::Tenso
     TORCH_CHECK(o == flat.numel(), "add_flat_grads: parameters and gradients do not match");
 }
 
-// The meta-net's 33 weights from its parameters: detached, fp32, contiguous; an entry that is a list of tensors (one per head)
-// becomes their stack, the experts' get their two or one dimensions.  Empty where an entry is neither.
-std::vector<torch::Tensor> meta_weights(py::list entries, int64_t num_experts) {
+// The meta-net's 33 weights from its parameters: detached, fp32, contiguous; an entry that is a list of them (one per head)
+// becomes their stack, the experts' get their two or one dimensions.  Empty where an entry is neither: `kind` is the class of a
+// parameter, and what derives from it may see more than a tensor's own operations.
+std::vector<torch::Tensor> meta_weights(py::list entries, py::object kind, int64_t num_experts) {
     at::NoGradGuard guard;
-    auto plain = [](const at::Tensor& t) {
-        at::Tensor d = t.detach();
-        if (d.scalar_type() != torch::kFloat32) d = d.to(torch::kFloat32);
-        return d.is_contiguous() ? d : d.contiguous();
-    };
+    c10::AutoFwGradMode no_tangents(false);       // what is stacked below is not detached by itself
+    auto parameter = [&](PyObject* o) { return o && (PyObject*)Py_TYPE(o) == kind.ptr() ? as_tensor(o) : nullptr; };
     const Py_ssize_t n = PyList_GET_SIZE(entries.ptr());
     std::vector<torch::Tensor> out;
     out.reserve(n);
     for (Py_ssize_t i = 0; i < n; i++) {
         PyObject* o = PyList_GET_ITEM(entries.ptr(), i);
-        if (const at::Tensor* t = as_tensor(o)) {
-            out.push_back(plain(*t));
+        if (const at::Tensor* t = parameter(o)) {
+            at::Tensor d = t->detach();
+            if (d.scalar_type() != torch::kFloat32) d = d.to(torch::kFloat32);
+            out.push_back(d.is_contiguous() ? d : d.contiguous());
             continue;
         }
         std::vector<at::Tensor> parts;
         for (Py_ssize_t k = 0; PyList_Check(o) && k < PyList_GET_SIZE(o); k++) {
-            const at::Tensor* t = as_tensor(PyList_GET_ITEM(o, k));
+            const at::Tensor* t = parameter(PyList_GET_ITEM(o, k));
             if (!t) return {};
             parts.push_back(t->scalar_type() == torch::kFloat32 ? *t : t->to(torch::kFloat32));
         }

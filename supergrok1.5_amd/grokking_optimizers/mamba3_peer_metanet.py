@@ -18,22 +18,28 @@ The sub-modules' own forwards (Mamba3ScanBlock on an arbitrary sequence,
 MiniGRU) are plain torch operations for callers that use them on their own.
 """
 import math
+import operator
 
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
 
-def _parameter(module, name):
-    """module.<name>, past the module's attribute lookup where it is a plain parameter."""
-    p = module._parameters.get(name)
-    return getattr(module, name) if p is None else p
+def _plain(kind, table, *names):
+    """A function of a module: what module.<name> gives for the names, past the attribute lookup, from the module's own table
+    (its parameters or modules).  It raises KeyError where the module is more than a `kind` or holds something else there."""
+    entries = operator.itemgetter(*names) if len(names) > 1 else lambda held, name=names[0]: (held[name],)
+
+    def get(module):
+        own = module.__dict__
+        if type(module) is not kind or not own.keys().isdisjoint(names):
+            raise KeyError(names)
+        return entries(own[table])
+    return get
 
 
-def _entries(params):
-    """The entries of a ParameterList, past its index lookups where they are plain parameters."""
-    held = list(params._parameters.values())
-    return held if len(held) == len(params) else list(params)
+_weight = _plain(nn.Linear, "_parameters", "weight")
+_weight_and_bias = _plain(nn.Linear, "_parameters", "weight", "bias")
 
 
 class Mamba3ScanBlock(nn.Module):
@@ -213,11 +219,13 @@ class Mamba3PEERMetaNet(nn.Module):
 
     def flat_weights(self):
         """The 33 tensors in the argument order of _ops.supergrok2_mamba_peer_batched_step."""
-        fwd, bwd = self.mamba_fwd, self.mamba_bwd
-        if type(self).get_weights is Mamba3PEERMetaNet.get_weights and type(fwd).export is type(bwd).export is Mamba3ScanBlock.export:
-            # without the dictionary and the calls and lookups per tensor (91 -> 38 us of every bilevel pass and of the first step after one)
+        if type(self).get_weights is Mamba3PEERMetaNet.get_weights and "get_weights" not in self.__dict__ and not torch._C._len_torch_function_stack():
+            # without the dictionary and the calls and lookups per tensor (80 -> 33 us of every bilevel pass and of the first step after one)
             from grokking_optimizers import _ops
-            out = _ops.meta_weights(self._weight_entries(), self.num_experts)
+            try:
+                out = _ops.meta_weights(self._weight_entries(), nn.Parameter, self.num_experts)
+            except KeyError:
+                out = []
             if out:
                 return out
         w = self.get_weights()
@@ -232,20 +240,25 @@ class Mamba3PEERMetaNet(nn.Module):
         return out
 
     def _weight_entries(self):
-        """The parameters behind flat_weights, in its order; the per-head ones as lists."""
-        lin = self.input_proj
-        out = [_parameter(lin, "weight"), _parameter(lin, "bias")]
-        for blk in (self.mamba_fwd, self.mamba_bwd):
-            mods = blk._modules
-            dt = mods["dt_proj"]
-            out += [_parameter(mods["in_proj"], "weight"), _parameter(dt, "weight"), _parameter(dt, "bias"), _parameter(mods["B_proj"], "weight"),
-                    _parameter(mods["C_proj"], "weight"), _parameter(blk, "A_log"), _parameter(blk, "D"), _parameter(blk, "rope_freq"),
-                    _parameter(mods["out_proj"], "weight")]
-        mods = self.gru._modules
-        for lin in (mods["W_z"], mods["W_r"], mods["W_h"]):
-            out += [_parameter(lin, "weight"), _parameter(lin, "bias")]
-        out += [[_parameter(q, "weight") for q in self.peer_queries], _entries(self.product_keys_A), _entries(self.product_keys_B)]
-        return out + [_parameter(self, "expert_W1"), _parameter(self, "expert_b1"), _parameter(self, "expert_W2"), _parameter(self, "expert_b2")]
+        """The parameters behind flat_weights, in its order; the per-head ones as lists.  KeyError where a layer is not the one
+        made above (get_weights knows what to make of it)."""
+        input_proj, mamba_fwd, mamba_bwd, gru, queries, keys_A, keys_B = (
+            _modules_of_net(self) if type(self) is Mamba3PEERMetaNet else
+            (self.input_proj, self.mamba_fwd, self.mamba_bwd, self.gru, self.peer_queries, self.product_keys_A, self.product_keys_B))
+        out = [*_weight_and_bias(input_proj)]
+        for blk in (mamba_fwd, mamba_bwd):
+            if "export" in blk.__dict__:
+                raise KeyError("export")
+            in_proj, dt, B, C, out_proj = _modules_of_block(blk)
+            out += (*_weight(in_proj), *_weight_and_bias(dt), *_weight(B), *_weight(C), *_parameters_of_block(blk), *_weight(out_proj))
+        for lin in _modules_of_gru(gru):
+            out += _weight_and_bias(lin)
+        out.append([_weight(q)[0] for q in queries])
+        for keys in (keys_A, keys_B):
+            n = len(keys)
+            out.append([*_plain(nn.ParameterList, "_parameters", *map(str, range(n)))(keys)] if n else [])
+        out += _parameters_of_net(self) if type(self) is Mamba3PEERMetaNet else (self.expert_W1, self.expert_b1, self.expert_W2, self.expert_b2)
+        return out
 
     @torch.no_grad()
     def load_flat_weights(self, weights):
@@ -308,3 +321,10 @@ class Mamba3PEERMetaNet(nn.Module):
             t[where] = rows
         self.expert_counts.zero_()
         return True
+
+
+_modules_of_net = _plain(Mamba3PEERMetaNet, "_modules", "input_proj", "mamba_fwd", "mamba_bwd", "gru", "peer_queries", "product_keys_A", "product_keys_B")
+_parameters_of_net = _plain(Mamba3PEERMetaNet, "_parameters", "expert_W1", "expert_b1", "expert_W2", "expert_b2")
+_modules_of_block = _plain(Mamba3ScanBlock, "_modules", "in_proj", "dt_proj", "B_proj", "C_proj", "out_proj")
+_parameters_of_block = _plain(Mamba3ScanBlock, "_parameters", "A_log", "D", "rope_freq")
+_modules_of_gru = _plain(MiniGRU, "_modules", "W_z", "W_r", "W_h")

@@ -124,3 +124,72 @@ def test_flat_weights_are_the_exported_ones(kw, change):
     assert len(a) == len(b) == 33
     for x, y in zip(a, b):
         assert x.shape == y.shape and x.dtype == torch.float32 and x.is_contiguous() and not x.requires_grad and torch.equal(x, y)
+
+
+def _repruned(mn):
+    """Pruning an entry of the key list and making it permanent registers the parameter anew, behind the others."""
+    from torch.nn.utils import prune
+    prune.l1_unstructured(mn.product_keys_A, "0", amount=3)
+    prune.remove(mn.product_keys_A, "0")
+
+
+def _own_get_weights(mn):
+    exported = mn.get_weights
+    mn.get_weights = lambda: dict(exported(), expert_b1=exported()["expert_b1"] + 1)
+
+
+def _own_export(mn):
+    exported = mn.mamba_bwd.export
+    mn.mamba_bwd.export = lambda: [2 * t for t in exported()]
+
+
+def _own_layers(mn):
+    class Tied(torch.nn.Linear):
+        @property
+        def weight(self):
+            return 0.5 * self._parameters["weight"]
+
+    class Gate(torch.nn.Module):                        # a cell whose layers are not registered under the reference's names
+        def __init__(self, cell):
+            super().__init__()
+            self.layers = torch.nn.ModuleList([cell.W_z, cell.W_r, cell.W_h])
+            self.hidden_dim = cell.hidden_dim
+
+        W_z = property(lambda self: self.layers[0])
+        W_r = property(lambda self: self.layers[1])
+        W_h = property(lambda self: self.layers[2])
+
+    mn.input_proj.__class__ = Tied
+    mn.gru = Gate(mn.gru)
+
+
+def _shadowed(mn):
+    object.__setattr__(mn.mamba_fwd.dt_proj, "weight", 3 * mn.mamba_fwd.dt_proj._parameters["weight"].detach())
+
+
+@pytest.mark.parametrize("change", [_repruned, _own_get_weights, _own_export, _own_layers, _shadowed])
+def test_flat_weights_see_what_get_weights_sees(change):
+    """Parameters registered in another order, methods and layers that an object brings itself."""
+    class ThroughGetWeights(Mamba3PEERMetaNet):
+        def get_weights(self):
+            return super().get_weights()
+    nets = [cls() for cls in (Mamba3PEERMetaNet, ThroughGetWeights)]
+    nets[1].load_state_dict(nets[0].state_dict())
+    for mn in nets:
+        change(mn)
+    for x, y in zip(*(mn.flat_weights() for mn in nets)):
+        assert torch.equal(x, y)
+
+
+def test_flat_weights_carry_no_tangents():
+    """Forward-mode duals are left behind, as by detach()."""
+    import torch.autograd.forward_ad as fwd_ad
+    mn = Mamba3PEERMetaNet()
+    with fwd_ad.dual_level():
+        for name in ("product_keys_B", "peer_queries"):
+            at = getattr(mn, name)[0]
+            owner, key = (at, "weight") if name == "peer_queries" else (mn.product_keys_B, "0")
+            p = owner._parameters.pop(key)
+            object.__setattr__(owner, key, fwd_ad.make_dual(p.detach(), torch.ones_like(p)))
+        for w in mn.flat_weights():
+            assert fwd_ad.unpack_dual(w).tangent is None
