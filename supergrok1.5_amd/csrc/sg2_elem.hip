@@ -473,7 +473,6 @@ __global__ __launch_bounds__(ELEM_THREADS) void k_elem_any(Plan pl, int ctx_stri
                 }
                 total = total + ho;
             }
-            __builtin_amdgcn_s_setprio(0);
             const float smart = g + (rescale * total) / (float)H;
             if (fwd_smart != nullptr) {
                 sg::gptr(fwd_smart)[(size_t)T.off + i] = smart;
