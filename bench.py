@@ -161,10 +161,7 @@ def build_step(workload, ops, dev, limit=None):
         bufs = [torch.zeros(s, device=dev) for s in shapes]
         W.update(step=lambda: ops.muon_fused_step(params, grads, bufs, 0.95, 0.02, 1.0, 5),
                  units=5 * sum(6 * min(s) ** 2 * max(s) for s in shapes), unit="FLOP/s",       # 6 min^2 max per NS iteration
-                 # what the kernels execute: the five iterations share two Gram matrices and two apply steps and form 14 products of
-                 # the Gram matrices' size; the symmetric ones launch only the 256 x 256 tiles on or above the diagonal
-                 executed=sum(2 * 256 * 256 * ((-(-min(s) // 256)) * (-(-min(s) // 256) + 1) // 2) * (2 * (-(-max(s) // 256)) * 256 + 14 * (-(-min(s) // 256)) * 256)
-                              + 2 * 2 * ((-(-min(s) // 256)) * 256) ** 2 * ((-(-max(s) // 256)) * 256) for s in shapes),
+                 executed=muon_executed(shapes, 5),
                  name="Muon step, %d x [1024,4096] + %d x [4096,1024], 5 Newton-Schulz iterations" % (len(shapes) // 2, len(shapes) // 2),
                  dtype="bf16", bound="mfma", peak=2500.0)
         return W
@@ -454,9 +451,24 @@ def v2_variants(shapes, st, grad_sets, D, dev, steps=8, warmup=2):
     return out
 
 
+def muon_executed(shapes, ns):
+    """Operations of the products that a Muon step launches: Gram matrices and apply steps once a stage, products of the Gram
+    matrices' size in between; the symmetric ones on the tiles on or above the diagonal only."""
+    from grokking_optimizers import _cabi
+    stages, tiles = _cabi.muon_stages_for(shapes, ns), _cabi.muon_tiles_for(shapes)
+    pad = max(tiles)
+    squares = ns if stages == ns else 4 * ns - 3 * stages
+    total = 0
+    for s in shapes:
+        m, n = (-(-d // pad) * pad for d in sorted(s))
+        upper = lambda t: t * t * (m // t) * (m // t + 1) // 2
+        total += 2 * (stages * (upper(tiles[0]) * n + m * m * n) + squares * upper(tiles[1]) * m)
+    return total
+
+
 def muon_precision(dev):
-    """One wide and one tall matrix of the Muon workload: this library's step (bf16 Newton-Schulz on the Gram matrix of
-    the smaller side, fp32 accumulation) against the reference's arithmetic (fp32 iteration on X X^T, csrc/ops.cpp:704-727
+    """One wide and one tall of the Muon workload's 24 matrices, stepped together as in the timed call: this library's step
+    (Newton-Schulz on Gram matrices of the smaller side in 16 bits, fp32 accumulation) against the reference's arithmetic (fp32 iteration on X X^T, csrc/ops.cpp:704-727
     of the reference) restated with torch fp32 products on the device.  Fraction of updated bf16 parameters that differ
     from the fp32-iteration result rounded to bf16 by more than one bf16 spacing, the fraction that round differently at
     all, and the largest deviation in units of the largest entry of the update (one bf16 spacing of a parameter of size
@@ -468,12 +480,13 @@ def muon_precision(dev):
     prev = torch.backends.cuda.matmul.allow_tf32
     torch.backends.cuda.matmul.allow_tf32 = False
     try:
-        for name, shape in (("wide_1024x4096", (1024, 4096)), ("tall_4096x1024", (4096, 1024))):
-            p = (torch.randn(*shape, generator=gen) * 0.02).to(torch.bfloat16).to(dev)
-            g = (torch.randn(*shape, generator=gen) * 1e-3).to(torch.bfloat16).to(dev)
-            buf = torch.zeros(shape, device=dev)
-            p_new = p.clone()
-            _ops.muon_fused_step([p_new], [g], [buf], 0.95, 0.02, 1.0, 5)
+        shapes = [(1024, 4096)] * 12 + [(4096, 1024)] * 12
+        ps = [(torch.randn(*s, generator=gen) * 0.02).to(torch.bfloat16).to(dev) for s in shapes]
+        gs = [(torch.randn(*s, generator=gen) * 1e-3).to(torch.bfloat16).to(dev) for s in shapes]
+        news = [p.clone() for p in ps]
+        _ops.muon_fused_step(news, gs, [torch.zeros(s, device=dev) for s in shapes], 0.95, 0.02, 1.0, 5)
+        for name, at in (("wide_1024x4096", 0), ("tall_4096x1024", 23)):
+            shape, p, g, p_new = shapes[at], ps[at], gs[at], news[at]
             X = g.float()
             X = X / (X.norm() + 1e-7)
             if shape[0] > shape[1]:
