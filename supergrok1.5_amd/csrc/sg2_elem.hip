@@ -27,12 +27,12 @@ constexpr int exp_stride() { return EHW == 16 ? 52 : 3 * EHW; }
 typedef outputs4 vf4;
 
 // The net's small matrix-vector products (GRU, queries, key scores) run on the matrix pipe (product4): step n's weights are
-// block n % 16 of register n / 16, and a whole net of the default
-// geometry takes 22.  As multiply-adds with scalar operands, GRU and scores were 650 of 1550 vector instructions an element and wave
-// with some forty scalar loads between them; the queries, as 32x32x1 products whose outputs had to be exchanged between
-// lanes, are as fast in large calls, but a wave that evaluates one head needs only its quarter of them now.  The launch:
-// 8 tensors below 256 elements 8.6 -> 6.6 us, 0.42 M elements 38.5 -> 34.6 (wide geometry 71 -> 61), 3.1 M bfloat16
-// 174 -> 171, 25 M 1.21 -> 1.20 ms (there the part's power sets the rate: 4.65 ns a product and SIMD, 1.3 to 1.9 a multiply-add).
+// block n % 16 of register n / 16, and a whole net of the default geometry takes 22.  As multiply-adds with scalar operands,
+// GRU and scores were 650 of 1550 vector instructions an element and wave, with some forty scalar loads between them; the
+// queries, as 32x32x1 products whose outputs had to be exchanged between lanes, are as fast in large calls, but a wave that
+// evaluates one head needs only its quarter of them now.  The launch: 8 tensors below 256 elements 8.6 -> 6.6 us, 0.42 M
+// elements 38.5 -> 34.6 (wide geometry 71 -> 61), 3.1 M bfloat16 174 -> 171, 25 M 1.21 -> 1.20 ms (there the part's power sets
+// the rate: 4.65 ns a product and SIMD, 1.3 to 1.9 a multiply-add).
 template <int N>
 __device__ __forceinline__ vf4 step4(const float* w, float x, vf4 acc) { return product4<N % 16>(w[N / 16], x, acc); }
 

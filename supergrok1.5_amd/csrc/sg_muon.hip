@@ -19,9 +19,11 @@
 // one stage an iteration takes 5 (n/m + 2 n/m) + 5.  A tracked G drifts from Y Y^T by its roundings, which small singular
 // values feel (they grow by a = 3.4 an iteration, those of G by its square): not more than three iterations a stage, and
 // everything but the momentum itself and what multiplies it in half precision, eight times finer than bf16 (numbers stay
-// below 1.3 resp. 41, scales in F16_SCALE).  Distance from float64 over Gaussian, low-rank, power-law and badly scaled
-// matrices: 0.3-0.9 of that of five stages in bf16 (1024 x 4096 Gaussian 3.0e-3 against 6.9e-3).  All five in one stage would
-// be 0.107 against 0.017 on a power law.  24 bf16 matrices of 1024 x 4096: 2181 -> 1642 us a step.
+// below 1.3 resp. 41, scales in F16_SCALE).  Distance from float64 over Gaussian, low-rank, power-law, sparse and row-scaled
+// matrices: 0.24-0.98 of that of five stages in bf16 (1024 x 4096 Gaussian 3.0e-3 against 6.9e-3).  Columns (of the wide
+// orientation) spread over six decades and more are the exception: there the drift of the second stage is 0.011 to 0.018
+// where bf16 is at 0.0095 (three iterations before two would be 0.006, but 6.4e-3 on a Gaussian).  All five in one stage
+// would be 0.107 against 0.017 on a power law.  24 bf16 matrices of 1024 x 4096: 2178 -> 1622 us a step.
 // The Gram and polynomial products are "NT" GEMMs (both operands K-contiguous).
 // The apply step is (on 256x256 tiles) an "NN" one: its B operand is Y itself, whose K axis is
 // the slow one.  Its tiles are staged in LDS as they lie in memory
@@ -622,8 +624,8 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_nt(Batch Bt, Ops ops, int y_s
 // three products have both operands K-contiguous.
 // Bound by latency for few tiles (the operands come through memory, where other XCDs wrote them: 5 to 8 us a product, of
 // which 4 are the launch), for many by what a CU gets from L2 (32 flop per byte: 0.6 PFLOP/s).
-// Step over bf16 matrices, with k_gemm_nt alone and with choose_tiles between the two: 1 of 200 x 800 232 -> 112 us,
-// 24 of 64 x 3000 493 -> 180, 1 of 1024 x 1024 410 -> 147, 2 of 1024 x 4096 691 -> 365, 24 of 512 x 2048 642 -> 498.
+// Step over bf16 matrices, with k_gemm_nt alone and with choose_tiles between the two: 1 of 200 x 800 235 -> 116 us,
+// 24 of 64 x 3000 368 -> 148, 1 of 1024 x 1024 413 -> 155, 2 of 1024 x 4096 621 -> 323, 24 of 512 x 2048 558 -> 457.
 constexpr int NT64 = 64;
 constexpr int KS_WAVES = 4, KS_THREADS = 64 * KS_WAVES;
 constexpr int KS_ROW = NT64 + 4;                                                // floats per row of a partial tile
